@@ -409,9 +409,10 @@ int mrl_scale_rows_note(void* x, int dtype, int64_t n_rows, int64_t vocab, int64
  * torch.nn.Linear weight), both dense and 16-byte aligned; hidden_dim % 64 == 0.  labels
  * [n_tokens] I32 / I64.  Outputs as mrl_vocab_logprob_fwd (entropy, lse nullable).  workspace:
  * mrl_lmhead_workspace_bytes(n_tokens, vocab) bytes of device memory, 16-byte aligned, holding
- * the per-vocabulary-group partial statistics (MRL_LMHEAD_GROUPS x n_tokens x 16 bytes).
+ * partial statistics of the vocabulary, 12 bytes per token and leaf of up to 3 x 256 entries (2.4 KB
+ * per token at 152 064 entries; more than 65 536 tokens are taken in slices of as many, so about
+ * 190 MiB at most).  A token's result does not depend on the other tokens of the call.
  */
-#define MRL_LMHEAD_GROUPS 8
 int64_t mrl_lmhead_workspace_bytes(int64_t n_tokens, int64_t vocab);
 int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
                            int64_t hidden_dim, const void* labels, int labels_dtype,
@@ -446,7 +447,7 @@ int mrl_lmhead_logprob_bwd(const void* hidden, const void* weight, const void* d
 /* mrl_lmhead_logprob_fwd for callers that cannot allocate device memory or pass a workspace (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in
  * the reference.  Same arguments, kernels and results as mrl_lmhead_logprob_fwd, but the partial
- * statistics live in a static device array of the library (8 MiB per GPU that runs it, looked up
+ * statistics live in a static device array of the library (64 MiB per GPU that runs it, looked up
  * once per device with hipGetSymbolAddress and held until the process ends), so at most
  * mrl_lmhead_static_max_tokens() = 65536 tokens per call: more is rejected with
  * MRL_ERR_UNSUPPORTED (slice the tokens).  Calls nothing that allocates or frees.  Every call on a

@@ -8,12 +8,12 @@
 // wavefront per SIMD with a 128 x 128 sub-tile of v_mfma_f32_16x16x32_bf16 blocks, operands straight
 // from global memory into two LDS stages) with the vocabulary as the MFMA's M and the tokens as its
 // N: in the 16x16 result layout a lane then owns ONE token column of each block and 4 vocabulary
-// rows, so the softmax statistics of a token accumulate inside a lane; only the four lane quarters
-// and the two vocabulary wavefronts have to be combined once, at the very end.  A workgroup owns
-// 256 tokens and walks the 256-row vocabulary tiles of its vocabulary group; the groups (8, dealt so
-// that the workgroups of one XCD share hidden blocks and weight tiles in its L2) leave per-group
-// partial statistics that a small second kernel merges, together with the label logit (one fp32 dot
-// product per token).
+// rows, so the softmax statistics of a token accumulate inside a lane.  The vocabulary is cut into leaves
+// of a few tiles (VocabLeaves) that follow from the vocabulary alone; every leaf leaves its own partial
+// statistics per token, and a second kernel merges them in a fixed order, together with the label
+// logit (one fp32 dot product per token).  So a token's result does not depend on which other tokens
+// share the call, whatever the work distribution is: units of 256 tokens by a group of leaves, as many
+// groups as fill the chip (pick_groups), walked by one persistent workgroup per CU.
 #include <stdlib.h>
 
 #include <atomic>
@@ -26,59 +26,140 @@
 // one copy per GPU that runs it, held until the process ends.  In host code this name is only a
 // handle for hipGetSymbolAddress; kernels get the address that call returns.
 #define MRL_LMHEAD_STATIC_MAX_TOKENS 65536
-static __device__ __align__(256) float scratch[(size_t)MRL_LMHEAD_GROUPS * MRL_LMHEAD_STATIC_MAX_TOKENS * 4];
+#define MRL_LMHEAD_STATIC_BYTES (64 << 20)
+static __device__ __align__(256) float scratch[MRL_LMHEAD_STATIC_BYTES / sizeof(float)];
 
 namespace {
 
 using namespace mrl_vocab;
 
-// The tiles of one workgroup: the vocabulary tiles of its group against its block of tokens.  The
-// tile loop runs over the flattened (vocabulary tile, k-step) sequence, so the first loads of the
-// next tile are in flight during the statistics of the current one.
-struct VocabGroupTiles {
-    int tile_begin, n_tiles, token_tile;
-    __device__ __forceinline__ void coords(int j, int& tm, int& tn) const {
-        tm = tile_begin + j;
-        tn = token_tile;
+// The leaves of a vocabulary: 1 to 3 tiles of 256 rows, more where that would make more than kMaxLeaves of
+// them.  A call with few tokens can be spread over no more workgroups than there are leaves (162 tokens x
+// 95 920 entries: 187 us with leaves of 2 tiles, 240 us with 3), but a leaf costs its statistics' last
+// reduction (19 202 x 148 784 at 1088 hidden: 5.30 ms with 2, 5.20 ms with 3) and 12 bytes per token.
+constexpr int kMaxLeaves = 256;
+struct VocabLeaves {
+    int n_tiles, tiles_per_leaf, n;
+    __host__ __device__ explicit VocabLeaves(int64_t vocab) {
+        n_tiles = (int)((vocab + mrl_tile::BM - 1) / mrl_tile::BM);
+        tiles_per_leaf = (n_tiles + kMaxLeaves - 1) / kMaxLeaves;
+        const int least = n_tiles <= 128 ? 1 : (n_tiles <= 384 ? 2 : 3);
+        if (tiles_per_leaf < least) tiles_per_leaf = least;
+        n = (n_tiles + tiles_per_leaf - 1) / tiles_per_leaf;
+    }
+    __host__ __device__ int begin_tile(int leaf) const {
+        const int t = leaf * tiles_per_leaf;
+        return t < n_tiles ? t : n_tiles;
     }
 };
 
+// Tokens of one launch: bounds the partial statistics (12 bytes per token and leaf) to about 190 MiB.
+constexpr int64_t kMaxSlice = 65536;
+constexpr int kUnitsPerRound = 256;             // one workgroup per CU
+constexpr int kMaxRounds = 64;                  // units a workgroup may take
+
+// The tiles of one workgroup: the tiles of its first unit, then of its second, ...  The tile loop runs
+// over the flattened (unit, vocabulary tile, k-step) sequence, so the first loads of the next tile are in
+// flight during the statistics of the current one, also across units.
+//
+// Workgroups are dealt round-robin to the 8 XCDs; the 32 of an XCD take consecutive units in each round.
+// Units are numbered so that these 32 are 4 token tiles x 8 groups: those that stream the same hidden
+// block and those that stream the same weight tiles run side by side and share them in the XCD's L2; and
+// so that the 8 XCDs hold 32 token tiles x the SAME 8 groups, so that a weight tile comes from HBM once
+// for all of them (numbering all groups of 4 token tiles first: 2 % slower at 8 and more groups).
+struct UnitInfo {
+    int start;                                  // flattened number of the unit's first tile
+    int tm, tn;                                 // its first vocabulary tile, its token tile
+};
+struct UnitTiles {
+    const UnitInfo* units;                      // LDS, n_units + 1 entries (the last: start = n_tiles)
+    int n_tiles;
+    __device__ __forceinline__ void coords(int j, int& tm, int& tn) const {
+        int r = 0;
+        while (j >= units[r + 1].start) ++r;
+        tm = __builtin_amdgcn_readfirstlane(units[r].tm - units[r].start) + j;
+        tn = __builtin_amdgcn_readfirstlane(units[r].tn);
+    }
+};
+
+// partial: [leaf][m, s, u][token of the slice]
 __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
-    const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, int64_t n_tokens, int vocab, int hdim,
-    int n_groups, int tiles_per_group, float k_scale, float* __restrict__ partial) {
+    const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, int n_tokens, int vocab, int hdim,
+    int n_groups, float k_scale, float* __restrict__ partial) {
     using namespace mrl_tile;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ Stats comb[2][kBlocks][16];       // [token wavefront][token block][lane % 16]
+    __shared__ Stats comb[2][kThreads];          // [vocabulary wavefront][token]: a finished leaf
+    __shared__ UnitInfo units[kMaxRounds + 1];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wv = wave >> 1, wt = wave & 1;
-    // Workgroups are dealt round-robin to the 8 XCDs and one round of 256 fills the chip.  The 32
-    // workgroups that share an XCD (and its L2) in a round are 4 token tiles x 8 vocabulary groups:
-    // the 8 that stream the same hidden block and the 4 that stream the same weight tiles run side
-    // by side, so most of both streams hits in L2 (with one vocabulary group per XCD every
-    // workgroup re-read its own hidden block from beyond the L2 for each vocabulary tile).
-    const int xcd = blockIdx.x & 7, slot = (blockIdx.x >> 3) & 31, round = blockIdx.x >> 8;
-    const int group = slot & 7;
-    const int64_t ttile = (int64_t)(round * 8 + xcd) * 4 + (slot >> 3);
-    const int64_t t0 = ttile * BN;
-    if (t0 >= n_tokens) return;                 // padding of the last round
-    const int n_vtiles = (vocab + BM - 1) / BM;
-    VocabGroupTiles seq;
-    seq.tile_begin = group * tiles_per_group;
-    seq.n_tiles = max(0, min(seq.tile_begin + tiles_per_group, n_vtiles) - seq.tile_begin);
-    seq.token_tile = (int)ttile;
+    const VocabLeaves leaves(vocab);
+    UnitTiles seq = {units, 0};
+    {
+        const int n_ttiles = (n_tokens + BN - 1) / BN;
+        int r = 0;
+        for (int u = (int)(blockIdx.x & 7) * 32 + (int)(blockIdx.x >> 3); u < n_ttiles * n_groups; u += kUnitsPerRound, ++r) {
+            // 32 token tiles by all groups > 8 groups > 4 token tiles > group > token tile
+            const int sp = u / (32 * n_groups), in_sp = u - sp * 32 * n_groups, tt_sp = min(32, n_ttiles - sp * 32);
+            const int block = in_sp / (tt_sp * 8), in_block = in_sp - block * tt_sp * 8, gw = min(8, n_groups - block * 8);
+            const int panel = in_block / (4 * gw), in_panel = in_block - panel * 4 * gw;
+            const int width = min(4, tt_sp - panel * 4), group = block * 8 + in_panel / width;
+            const int first = leaves.begin_tile((int)((int64_t)group * leaves.n / n_groups));
+            if (threadIdx.x == 0) units[r] = {seq.n_tiles, first, sp * 32 + panel * 4 + in_panel % width};
+            seq.n_tiles += leaves.begin_tile((int)((int64_t)(group + 1) * leaves.n / n_groups)) - first;
+        }
+        if (threadIdx.x == 0) units[r] = {seq.n_tiles, 0, 0};
+    }
+    const int tiles_per_leaf = leaves.tiles_per_leaf, n_vtiles = leaves.n_tiles;
+    __syncthreads();
 
     // a lane holds one token of each of its wavefront's 8 token blocks
     Stats st[kBlocks];
 #pragma unroll
     for (int tb = 0; tb < kBlocks; ++tb) st[tb] = {kMaxInit, 0.f, 0.f};
 
+    // A leaf is finished: combine the four lane quarters (same token, other vocabulary rows), then the two
+    // vocabulary wavefronts; thread t writes token t.
+    auto finish_leaf = [&](int leaf, int tn) {
+#pragma unroll
+        for (int tb = 0; tb < kBlocks; ++tb) {
+#pragma unroll
+            for (int off = 16; off <= 32; off <<= 1) {
+                Stats o;
+                o.m = __shfl_xor(st[tb].m, off, 64);
+                o.s = __shfl_xor(st[tb].s, off, 64);
+                o.u = __shfl_xor(st[tb].u, off, 64);
+                st[tb] = merge<true>(st[tb], o, k_scale);
+            }
+            if (lane < 16) comb[wv][wt * 128 + tb * 16 + lane] = st[tb];
+            st[tb] = {kMaxInit, 0.f, 0.f};
+        }
+        // LDS accesses only: a full fence would wait for the requests of the next stages as well.  The
+        // next leaf's writes to comb lie behind the barriers of at least one more tile.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        const int t = tn * BN + (int)threadIdx.x;
+        if (t < n_tokens) {
+            const Stats r = merge<true>(comb[0][threadIdx.x], comb[1][threadIdx.x], k_scale);
+            float* p = partial + (int64_t)leaf * 3 * n_tokens + t;
+            p[0] = r.m;
+            p[n_tokens] = r.s;
+            p[2 * (int64_t)n_tokens] = r.u;
+        }
+    };
+
     // online softmax statistics of a tile: per token block a lane holds 8 x 4 vocabulary rows
-    auto tile_stats = [&](Accumulators& acc, int tm, int /*tn*/) {
+    auto tile_stats = [&](Accumulators& acc, int tm, int tn) {
         const int v0 = tm * BM + wv * 128 + 4 * (lane >> 4);       // + 16 vb + r
         const bool ragged = (tm * BM + BM > vocab);
 #pragma unroll
         for (int tb = 0; tb < kBlocks; ++tb) {
+            // one block of tokens at a time: without this the compiler copies many blocks out of the
+            // accumulator half of the register file at once and parks them in scratch memory
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int vb = 0; vb < kBlocks; ++vb) asm volatile("" : "+a"(acc[vb][tb]));
             if (ragged) {
 #pragma unroll
                 for (int vb = 0; vb < kBlocks; ++vb)
@@ -92,7 +173,7 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) vmax = fmaxf(vmax, acc[vb][tb][r]);
             grow_max<true>(st[tb], vmax, k_scale);
-            // A lane that has seen no valid vocabulary row yet (the first tile of its group is ragged and
+            // A lane that has seen no valid vocabulary row yet (the first tile of its leaf is ragged and
             // ends above its rows) still holds the start value as its maximum: z * k - m * k of the masked
             // entries would then be the rounding residual of two numbers of magnitude 1e30 instead of
             // zero.  With an infinite m * k their exponentials are exactly 0.
@@ -102,102 +183,116 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) add_one<true>(st[tb], acc[vb][tb][r], k_scale, mk);
         }
+        const int leaf = tm / tiles_per_leaf;                      // uniform over the workgroup
+        if (tm + 1 == n_vtiles || tm + 1 == (leaf + 1) * tiles_per_leaf) finish_leaf(leaf, tn);
     };
-    mfma_tile_loop<false, false, 4>(smem, weight, hdim, vocab, hidden, hdim, (int)n_tokens, hdim, seq, tile_stats);
+    mfma_tile_loop<false, false, 4>(smem, weight, hdim, vocab, hidden, hdim, n_tokens, hdim, seq, tile_stats);
+}
 
-    // combine the four lane quarters (same token, other vocabulary rows), then the two vocabulary wavefronts
-#pragma unroll
-    for (int tb = 0; tb < kBlocks; ++tb) {
-#pragma unroll
-        for (int off = 16; off <= 32; off <<= 1) {
-            Stats o;
-            o.m = __shfl_xor(st[tb].m, off, 64);
-            o.s = __shfl_xor(st[tb].s, off, 64);
-            o.u = __shfl_xor(st[tb].u, off, 64);
-            st[tb] = merge<true>(st[tb], o, k_scale);
+// A workgroup finishes 16 tokens.  16 threads per token merge the leaves (thread q takes leaves q, q + 16,
+// ...; the loads of 16 neighbouring tokens are 64 contiguous bytes), then the 16 partial results are merged
+// in order; and one wavefront per token computes the label logit as an fp32 dot product of the token's
+// hidden row with the label's weight row.
+constexpr int kFinishTokens = 16;
+template <typename LabelT>
+__global__ __launch_bounds__(256) void lmhead_finish_kernel(
+    const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, const LabelT* __restrict__ labels,
+    const float* __restrict__ partial, int n_tokens, int vocab, int hdim, int n_leaves, float inv_t,
+    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
+    __shared__ Stats part[16][kFinishTokens];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t0 = (int)blockIdx.x * kFinishTokens;
+    const float k = inv_t * kLog2e;
+    {
+        const int mine = threadIdx.x & 15, q = threadIdx.x >> 4;
+        const int t = min(t0 + mine, n_tokens - 1);
+        Stats r = {kMaxInit, 0.f, 0.f};
+#pragma unroll 4
+        for (int leaf = q; leaf < n_leaves; leaf += 16) {
+            const float* p = partial + (int64_t)leaf * 3 * n_tokens + t;
+            const Stats o = {p[0], p[n_tokens], p[2 * (int64_t)n_tokens]};
+            r = merge<true>(r, o, k);
         }
+        part[q][mine] = r;
     }
     __syncthreads();
-    if (wv == 1 && lane < 16) {
+    for (int i = wave; i < kFinishTokens; i += 4) {
+        const int t = t0 + i;
+        if (t >= n_tokens) return;
+        const int64_t y = (int64_t)labels[t];
+        const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
+        float dot = 0.f;
+        if (y_ok) {
+            const uint16_t* hrow = hidden + (int64_t)t * hdim;
+            const uint16_t* wrow = weight + y * hdim;
+            for (int j = lane * 8; j < hdim; j += 64 * 8) {
+                const u32x4 hv = *reinterpret_cast<const u32x4*>(hrow + j);
+                const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + j);
+                float a[8], b[8];
+                Elem<MRL_BF16>::unpack(hv, a);
+                Elem<MRL_BF16>::unpack(wv, b);
 #pragma unroll
-        for (int tb = 0; tb < kBlocks; ++tb) comb[wt][tb][lane] = st[tb];
-    }
-    __syncthreads();
-    if (wv == 0 && lane < 16) {
-#pragma unroll
-        for (int tb = 0; tb < kBlocks; ++tb) {
-            const Stats r = merge<true>(st[tb], comb[wt][tb][lane], k_scale);
-            const int64_t t = t0 + wt * 128 + tb * 16 + lane;
-            if (t < n_tokens) {
-                float* p = partial + ((int64_t)group * n_tokens + t) * 4;
-                p[0] = r.m;
-                p[1] = r.s;
-                p[2] = r.u;
-                p[3] = 0.f;
+                for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(a[e], b[e], dot);
             }
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        Stats r = part[lane & 15][i];
+#pragma unroll
+        for (int off = 1; off <= 8; off <<= 1) {
+            const Stats o = {__shfl_xor(r.m, off, 64), __shfl_xor(r.s, off, 64), __shfl_xor(r.u, off, 64)};
+            r = merge<true>(r, o, k);
+        }
+        if (lane == 0) {
+            const float lse = (r.m * k + fast_log2(r.s)) * kLn2;
+            logp[t] = (y_ok ? dot * inv_t : r.m * inv_t) - lse;
+            if (entropy) entropy[t] = lse - (r.u / r.s) * inv_t;
+            if (lse_out) lse_out[t] = lse;
         }
     }
 }
 
-// One wavefront per token: merges the per-group partial statistics and computes the label logit
-// as an fp32 dot product of the token's hidden row with the label's weight row.
-template <typename LabelT>
-__global__ __launch_bounds__(256) void lmhead_finish_kernel(
-    const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, const LabelT* __restrict__ labels,
-    const float* __restrict__ partial, int64_t n_tokens, int vocab, int hdim, int n_groups, float inv_t,
-    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
-    const int lane = threadIdx.x & 63;
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= n_tokens) return;
-    const float k = inv_t * kLog2e;
-    const int64_t y = (int64_t)labels[t];
-    const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
-    float dot = 0.f;
-    if (y_ok) {
-        const uint16_t* hrow = hidden + t * hdim;
-        const uint16_t* wrow = weight + y * hdim;
-        for (int j = lane * 8; j < hdim; j += 64 * 8) {
-            const u32x4 hv = *reinterpret_cast<const u32x4*>(hrow + j);
-            const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + j);
-            float a[8], b[8];
-            Elem<MRL_BF16>::unpack(hv, a);
-            Elem<MRL_BF16>::unpack(wv, b);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dot = __builtin_fmaf(a[i], b[i], dot);
+// The number of groups that the leaves are dealt into.  A launch takes ceil(token tiles x groups / 256)
+// rounds of the chip, each as long as its largest group plus a little (a unit's first tiles come from
+// beyond the L2); the cheapest count wins, the smallest among equals.  One and two groups stream more
+// different hidden blocks through an L2 than it holds (65 536 tokens: 71.1 ms with 1, 49.7 with 2, 48.9
+// with 3, 49.2 with 8).  What this replaces, 8 groups for every size and a launch of as many workgroups
+// as that makes, gave 17 122 tokens (67 token tiles) 3 rounds for 2.1 rounds of work, and 1 380 tokens 48
+// of the 256 CUs.  Measured with it / now:
+//     tokens  vocabulary  hidden     before       now        tokens  vocabulary  hidden    before       now
+//        162      95 920    2944   3 184 us    187 us        17 122    152 064    3584  19.77 ms  13.24 ms
+//        704      67 512    1344     937 us    153 us        19 202    148 784    1088   6.91 ms   5.14 ms
+//      1 380      27 600    2880     803 us    223 us        32 768    152 064    3584  25.69 ms  24.66 ms
+int pick_groups(int64_t n_tokens, const VocabLeaves& leaves) {
+    const int64_t n_ttiles = (n_tokens + mrl_tile::BN - 1) / mrl_tile::BN;
+    int best = 1;
+    int64_t best_cost = INT64_MAX;
+    for (int g = 1; g <= leaves.n; ++g) {
+        const int64_t rounds = (n_ttiles * g + kUnitsPerRound - 1) / kUnitsPerRound;
+        if (rounds > kMaxRounds) break;
+        int64_t tiles = (int64_t)((leaves.n + g - 1) / g) * leaves.tiles_per_leaf;
+        if (tiles > leaves.n_tiles) tiles = leaves.n_tiles;
+        const int64_t cost = rounds * (10 * tiles + 3) * (g == 1 ? 140 : (g == 2 ? 102 : 100));
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = g;
         }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
-    if (lane == 0) {
-        Stats r = {kMaxInit, 0.f, 0.f};
-        for (int g = 0; g < n_groups; ++g) {
-            const float* p = partial + ((int64_t)g * n_tokens + t) * 4;
-            const Stats o = {p[0], p[1], p[2]};
-            r = merge<true>(r, o, k);
-        }
-        const float lse = (r.m * k + fast_log2(r.s)) * kLn2;
-        logp[t] = (y_ok ? dot * inv_t : r.m * inv_t) - lse;
-        if (entropy) entropy[t] = lse - (r.u / r.s) * inv_t;
-        if (lse_out) lse_out[t] = lse;
-    }
+    return best;
 }
 
 }  // namespace
 
 extern "C" int64_t mrl_lmhead_workspace_bytes(int64_t n_tokens, int64_t vocab) {
     if (n_tokens < 0 || vocab <= 0) return 0;
-    return (int64_t)MRL_LMHEAD_GROUPS * n_tokens * 4 * (int64_t)sizeof(float);
+    return (int64_t)VocabLeaves(vocab).n * (n_tokens < kMaxSlice ? n_tokens : kMaxSlice) * 3 * (int64_t)sizeof(float);
 }
 
-// Checks and launches shared by the two forward entry points; `partial` holds
-// mrl_lmhead_workspace_bytes(n_tokens, vocab) bytes.
+// Checks and launches shared by the two forward entry points.  `partial` holds the statistics of `slice`
+// tokens; more are taken in slices, one after the other on the stream.
 static int lmhead_forward(const char* fn, const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
                           int64_t hidden_dim, const void* labels, int labels_dtype, float inv_temperature, float* logp,
-                          float* entropy, float* lse, float* partial, hipStream_t s) {
-    const int n_groups = MRL_LMHEAD_GROUPS;
-    const int n_vtiles = (int)((vocab + mrl_tile::BM - 1) / mrl_tile::BM);
-    // a group without tiles (tiny vocabularies) still writes its neutral partials
-    const int tiles_per_group = (n_vtiles + n_groups - 1) / n_groups;
+                          float* entropy, float* lse, float* partial, int64_t slice, hipStream_t s) {
     // 256-token tiles, operands straight into two LDS stages (128 KiB of dynamic LDS).  Function
     // attributes belong to a device, so the reservation is made with every launch, on whichever
     // device is current.
@@ -208,26 +303,31 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
                 hipGetErrorString(attr));
     MRL_REQUIRE(256 * hidden_dim * 2 < (1LL << 31) && n_tokens <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED,
                 "%s: size out of range", fn);
-    const int64_t n_ttiles = (n_tokens + mrl_tile::BN - 1) / mrl_tile::BN;
-    const int64_t n_rounds = (n_ttiles + 31) / 32;       // 32 token tiles x 8 groups per round of 256 workgroups
-    MRL_REQUIRE(n_rounds * 256 <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED, "%s: grid too large", fn);
-    static_assert(MRL_LMHEAD_GROUPS == 8, "the workgroup mapping assumes 8 vocabulary groups");
-    hipLaunchKernelGGL(lmhead_fwd_kernel, dim3((unsigned)(n_rounds * 256)), dim3(mrl_tile::kThreads), kLdsBytes, s,
-                       (const uint16_t*)hidden, (const uint16_t*)weight, n_tokens, (int)vocab, (int)hidden_dim,
-                       n_groups, tiles_per_group, inv_temperature * kLog2e, partial);
-    int rc = mrl::check_launch(fn);
-    if (rc != MRL_OK) return rc;
-    const dim3 fgrid((unsigned)((n_tokens + 3) / 4)), fblock(256);
-    if (labels_dtype == MRL_I32) {
-        hipLaunchKernelGGL(lmhead_finish_kernel<int32_t>, fgrid, fblock, 0, s, (const uint16_t*)hidden,
-                           (const uint16_t*)weight, (const int32_t*)labels, (const float*)partial, n_tokens, (int)vocab,
-                           (int)hidden_dim, n_groups, inv_temperature, logp, entropy, lse);
-    } else {
-        hipLaunchKernelGGL(lmhead_finish_kernel<int64_t>, fgrid, fblock, 0, s, (const uint16_t*)hidden,
-                           (const uint16_t*)weight, (const int64_t*)labels, (const float*)partial, n_tokens, (int)vocab,
-                           (int)hidden_dim, n_groups, inv_temperature, logp, entropy, lse);
+    const VocabLeaves leaves(vocab);
+    for (int64_t lo = 0; lo < n_tokens; lo += slice) {
+        const int n = (int)(n_tokens - lo < slice ? n_tokens - lo : slice);
+        const uint16_t* h = (const uint16_t*)hidden + lo * hidden_dim;
+        hipLaunchKernelGGL(lmhead_fwd_kernel, dim3(kUnitsPerRound), dim3(mrl_tile::kThreads), kLdsBytes, s, h,
+                           (const uint16_t*)weight, n, (int)vocab, (int)hidden_dim, pick_groups(n, leaves),
+                           inv_temperature * kLog2e, partial);
+        int rc = mrl::check_launch(fn);
+        if (rc != MRL_OK) return rc;
+        const dim3 fgrid((unsigned)((n + kFinishTokens - 1) / kFinishTokens)), fblock(256);
+        float* ent = entropy ? entropy + lo : nullptr;
+        float* lse_out = lse ? lse + lo : nullptr;
+        if (labels_dtype == MRL_I32) {
+            hipLaunchKernelGGL(lmhead_finish_kernel<int32_t>, fgrid, fblock, 0, s, h, (const uint16_t*)weight,
+                               (const int32_t*)labels + lo, (const float*)partial, n, (int)vocab, (int)hidden_dim,
+                               leaves.n, inv_temperature, logp + lo, ent, lse_out);
+        } else {
+            hipLaunchKernelGGL(lmhead_finish_kernel<int64_t>, fgrid, fblock, 0, s, h, (const uint16_t*)weight,
+                               (const int64_t*)labels + lo, (const float*)partial, n, (int)vocab, (int)hidden_dim,
+                               leaves.n, inv_temperature, logp + lo, ent, lse_out);
+        }
+        rc = mrl::check_launch(fn);
+        if (rc != MRL_OK) return rc;
     }
-    return mrl::check_launch(fn);
+    return MRL_OK;
 }
 
 #define MRL_LMHEAD_CHECK_ARGS(fn)                                                                                      \
@@ -256,7 +356,7 @@ extern "C" int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, in
                 "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
                 (long long)mrl_lmhead_workspace_bytes(n_tokens, vocab));
     return lmhead_forward(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, logp,
-                          entropy, lse, (float*)workspace, mrl::as_stream(stream));
+                          entropy, lse, (float*)workspace, kMaxSlice, mrl::as_stream(stream));
 }
 
 // Address of `scratch` on the current device, looked up once per device (each GPU holds its own
@@ -299,6 +399,8 @@ extern "C" int mrl_lmhead_logprob_fwd_static(const void* hidden, const void* wei
                 "%s: hidden and weight must be 16-byte aligned", fn);
     float* partial = static_scratch(fn);
     if (!partial) return MRL_ERR_LAUNCH;
+    // whole token tiles that the scratch memory holds the statistics of (27 904 tokens at 152 064 entries)
+    const int64_t slice = MRL_LMHEAD_STATIC_BYTES / (VocabLeaves(vocab).n * 12LL) / 256 * 256;
     return lmhead_forward(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, logp,
-                          entropy, lse, partial, mrl::as_stream(stream));
+                          entropy, lse, partial, slice, mrl::as_stream(stream));
 }

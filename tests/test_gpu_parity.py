@@ -1410,6 +1410,28 @@ def test_lmhead_logprob_forward(dev, tokens, vocab, hdim):
     assert torch.allclose(lp2.view(-1).cpu(), o_vocab.lmhead_logprob_entropy(h, w, y)[0], atol=2e-4)
 
 
+@pytest.mark.parametrize("tokens,vocab,hdim", [(1, 8, 64), (1, 20000, 64), (256, 33000, 64), (257, 5000, 64),
+                                               (1025, 16392, 64), (8448, 2064, 128)])
+def test_lmhead_logprob_forward_work_distribution(dev, tokens, vocab, hdim):
+    """How the work is dealt follows from both sizes: one tile in all, one token tile by many leaves of 1 and of 2
+    tiles, uneven groups, a last panel of fewer than 4 token tiles, more than 32 token tiles.  A token's result
+    must not depend on it: a call with fewer tokens gives the same bits."""
+    gen = torch.Generator().manual_seed(tokens + vocab)
+    h = torch.randn(tokens, hdim, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(vocab, hdim, generator=gen) * (2.0 / hdim ** 0.5)).to(torch.bfloat16)
+    y = torch.randint(0, vocab, (tokens,), generator=gen)
+    lp_o, h_o, lse_o = o_vocab.lmhead_logprob_entropy(h, w, y)
+    h, w, y = h.to(dev), w.to(dev), y.to(dev)
+    lp, ent, lse = mrl.lmhead_logprob(h, w, y)
+    # fp32 sums of hdim products of about 2 / hdim^0.5, then lse <= 2 + log(vocab) in fp32: under 1e-5 each way
+    assert (lse.cpu() - lse_o).abs().max().item() < 2e-5
+    assert (lp.cpu() - lp_o).abs().max().item() < 4e-5
+    assert (ent.cpu() - h_o).abs().max().item() < 4e-5
+    lo = tokens // 3
+    for part, whole in zip(mrl.lmhead_logprob(h[lo:], w, y[lo:]), (lp, ent, lse)):
+        assert torch.equal(part, whole[lo:])
+
+
 @pytest.mark.parametrize("chunk_rows", [64, 8192])
 def test_fused_lmhead_policy_loss(dev, chunk_rows):
     """Loss and gradients straight from the hidden states (per chunk: logits product -> fused sweep ->
