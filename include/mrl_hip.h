@@ -485,6 +485,14 @@ int mrl_kl_token_rewards(const float* old_log_prob, const float* ref_log_prob,
 int mrl_gae_scan(const float* rewards, const float* values, int64_t batch, int64_t width, float gamma,
                  float gamma_lam, float* advantages, float* returns, void* stream);
 
+/* mrl_gae_whiten: the whole of compute_gae_advantage_return: mrl_gae_scan, then the advantages whitened
+ * in place with `mask` (as mrl_masked_whiten with shift_mean).  info as there.  workspace: 8-byte
+ * aligned, mrl_gae_whiten_workspace_bytes(batch) bytes, no clearing needed. */
+int64_t mrl_gae_whiten_workspace_bytes(int64_t batch);
+int mrl_gae_whiten(const float* rewards, const float* values, const void* mask, int mask_dtype,
+                   int64_t batch, int64_t width, float gamma, float gamma_lam, float* advantages,
+                   float* returns, double* info, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* mrl_masked_whiten: masked_whiten / masked_var / masked_mean (mindspeed_rl/utils/
  * torch_functional.py:46-106) over n entries: mean = sum(x*mask)/(sum(mask)+1e-8), var the same of
  * (x-mean)^2 times sum(mask)/(sum(mask)-1) unless sum(mask) == 1, out = (x-mean)*rsqrt(var+1e-8)
@@ -504,6 +512,14 @@ int mrl_masked_whiten(const float* x, const void* mask, int mask_dtype, int64_t 
 int mrl_value_loss_fwd(const float* vpreds, const float* returns, const float* values, const void* mask,
                        int mask_dtype, const void* response_length, int length_dtype, int64_t batch,
                        int64_t width, float cliprange_value, float loss_scale, float* out, void* stream);
+/* The forward with scratch memory, spread over the whole GPU: workspace (8-byte aligned,
+ * mrl_value_loss_workspace_bytes(batch) bytes, no clearing needed).  loss_out (nullable): out[0] again. */
+int64_t mrl_value_loss_workspace_bytes(int64_t batch);
+int mrl_value_loss_fwd_split(const float* vpreds, const float* returns, const float* values,
+                             const void* mask, int mask_dtype, const void* response_length,
+                             int length_dtype, int64_t batch, int64_t width, float cliprange_value,
+                             float loss_scale, float* out, float* loss_out, void* workspace,
+                             int64_t workspace_bytes, void* stream);
 int mrl_value_loss_bwd(const float* vpreds, const float* returns, const float* values, const void* mask,
                        int mask_dtype, const void* response_length, int length_dtype, int64_t batch,
                        int64_t width, float cliprange_value, float loss_scale, const float* out,

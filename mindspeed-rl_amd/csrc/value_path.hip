@@ -10,8 +10,8 @@ namespace {
 
 using namespace mrl_loss;
 
-constexpr int kScanBlock = 256;
-constexpr int kScanChunk = 2048;     // entries of a row staged in LDS per step of the scan
+constexpr int kScanBlock = 512;
+constexpr int kScanChunk = 4096;     // entries of a row staged in LDS per step of the scan
 constexpr int kReduceBlock = 1024;
 
 // Sum of one double per thread over a workgroup of kReduceBlock threads, fixed order; every thread
@@ -75,42 +75,129 @@ __global__ __launch_bounds__(256) void kl_rewards_kernel(const float* __restrict
 // ---------------------------------------------------------------------------- GAE reverse scan
 // One workgroup per sample.  The recurrence lastgaelam = delta_t + (gamma*lam) * lastgaelam is
 // evaluated by ONE thread in the reference's order and with its roundings (separate multiply and
-// add, no contraction), so advantages and returns are bit-identical to the torch loop; the other
-// threads stage the row through LDS in coalesced chunks and write the results.  gl is gamma*lam as
-// the host formed it: python multiplies the two in double and torch rounds the product to fp32 once.
+// add, no contraction), so advantages and returns are bit-identical to the torch loop.  gl is gamma*lam
+// as the host formed it: python multiplies the two in double and torch rounds the product to fp32 once.
+//
+// Bound by that chain: two dependent operations per token.  So nothing else is left on it: all threads
+// form the deltas, and the chain takes them from LDS four at a time, 16 steps ahead of their use
+// (batch 128 x width 2048: 28 us; with the deltas formed inside the chain from single entries 69 us).
+//
+// kMoments: leaves the masked moments (sum m, sum m x, sum m x^2) of the sample's advantages, in fp64, for
+// the whitening that follows.
+struct Moments {
+    double w, x, xx;
+};
+
+template <bool kMoments>
 __global__ __launch_bounds__(kScanBlock) void gae_scan_kernel(const float* __restrict__ rewards,
                                                               const float* __restrict__ values, int64_t width,
                                                               float gamma, float gl, float* __restrict__ adv,
-                                                              float* __restrict__ ret) {
-    __shared__ float r_s[kScanChunk];
-    __shared__ float v_s[kScanChunk + 1];
-    __shared__ float a_s[kScanChunk];
-    __shared__ float carry;
+                                                              float* __restrict__ ret, const void* __restrict__ mask,
+                                                              int mdtype, Moments* __restrict__ moments) {
+    // A chunk of n tokens lies at the END of n rounded up to a multiple of 4 slots, so that the chain
+    // starts on a whole group of 4; only the last chunk (the row's beginning) can have empty slots in front.
+    __shared__ float4 chunk[kScanChunk / 4];
+    float* slot = reinterpret_cast<float*>(chunk);
     const int64_t base = (int64_t)blockIdx.x * width;
-    if (threadIdx.x == 0) carry = 0.f;
+    Moments mom = {0.0, 0.0, 0.0};
+    constexpr int kPer = kScanChunk / kScanBlock;
+    float last = 0.f;                                      // thread 0's
     for (int64_t hi = width; hi > 0; hi -= kScanChunk) {
         const int64_t lo = hi > kScanChunk ? hi - kScanChunk : 0;
-        const int n = (int)(hi - lo);
-        __syncthreads();
-        for (int t = threadIdx.x; t < n; t += kScanBlock) {
-            r_s[t] = rewards[base + lo + t];
-            v_s[t] = values[base + lo + t];
+        const int n = (int)(hi - lo), groups = (n + 3) >> 2, pad = groups * 4 - n;
+        const float* r = rewards + base + lo;
+        const float* v = values + base + lo;
+        // everything the chunk needs of memory is requested here, in one go; values and mask stay in registers
+        float v_mine[kPer], m_mine[kPer], r_mine[kPer], v_next[kPer];
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            const int t = min(q * kScanBlock + (int)threadIdx.x, n - 1);
+            r_mine[q] = r[t];
+            v_mine[q] = v[t];
+            v_next[q] = v[lo + t + 1 < width ? t + 1 : t];
+            if (kMoments) m_mine[q] = mask_at(mask, mdtype, nullptr, 0, 0, base + lo + t, 0);
         }
-        if (threadIdx.x == 0) v_s[n] = hi < width ? values[base + hi] : 0.f;
+        __syncthreads();                                   // the previous chunk has been written out
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            const int t = q * kScanBlock + (int)threadIdx.x;
+            const float next = lo + t + 1 < width ? v_next[q] : 0.f;
+            if (t < n) slot[pad + t] = mrl::sub_rn(mrl::add_rn(r_mine[q], mrl::mul_rn(gamma, next)), v_mine[q]);
+        }
+        if ((int)threadIdx.x < pad) slot[threadIdx.x] = 0.f;
         __syncthreads();
         if (threadIdx.x == 0) {
-            float last = carry;
-            for (int t = n - 1; t >= 0; --t) {
-                const float delta = mrl::sub_rn(mrl::add_rn(r_s[t], mrl::mul_rn(gamma, v_s[t + 1])), v_s[t]);
-                last = mrl::add_rn(delta, mrl::mul_rn(gl, last));
-                a_s[t] = last;
+            auto four = [&](float4& d) {
+                d.w = last = mrl::add_rn(d.w, mrl::mul_rn(gl, last));
+                d.z = last = mrl::add_rn(d.z, mrl::mul_rn(gl, last));
+                d.y = last = mrl::add_rn(d.y, mrl::mul_rn(gl, last));
+                d.x = last = mrl::add_rn(d.x, mrl::mul_rn(gl, last));
+            };
+            int g = groups - 1;
+            for (; (g + 1) & 7; --g) {                     // down to a multiple of 8 groups
+                float4 d = chunk[g];
+                four(d);
+                chunk[g] = d;
             }
-            carry = last;
+            // 16 steps from one set of registers while the next 16 deltas arrive in the other
+            auto load = [&](float4(&d)[4], int at) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) d[q] = chunk[at - q];
+            };
+            auto sixteen = [&](float4(&d)[4], int at) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    four(d[q]);
+                    chunk[at - q] = d[q];
+                }
+            };
+            if (g >= 0) {
+                float4 even[4], odd[4];
+                load(even, g);
+                __builtin_amdgcn_s_waitcnt(0xC07F);        // nothing outstanding into the loop on either path
+                for (; g >= 0; g -= 8) {
+                    load(odd, g - 4);
+                    sixteen(even, g);
+                    load(even, g >= 8 ? g - 8 : g);        // these once more at the end, unused
+                    sixteen(odd, g - 4);
+                }
+            }
         }
         __syncthreads();
-        for (int t = threadIdx.x; t < n; t += kScanBlock) {
-            adv[base + lo + t] = a_s[t];
-            ret[base + lo + t] = mrl::add_rn(a_s[t], v_s[t]);
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            const int t = q * kScanBlock + (int)threadIdx.x;
+            if (t >= n) break;
+            const float a = slot[pad + t];
+            adv[base + lo + t] = a;
+            ret[base + lo + t] = mrl::add_rn(a, v_mine[q]);
+            if (kMoments && m_mine[q] != 0.f) {
+                const double m = (double)m_mine[q];
+                mom.w += m;
+                mom.x += m * (double)a;
+                mom.xx += m * ((double)a * (double)a);
+            }
+        }
+    }
+    if (kMoments) {
+        __shared__ double lds[3][kScanBlock / 64];
+        const double part[3] = {mom.w, mom.x, mom.xx};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            double s = part[q];
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+            if ((threadIdx.x & 63) == 0) lds[q][threadIdx.x >> 6] = s;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                s[q] = lds[q][0];
+                for (int w = 1; w < kScanBlock / 64; ++w) s[q] += lds[q][w];
+            }
+            moments[blockIdx.x] = {s[0], s[1], s[2]};
         }
     }
 }
@@ -160,6 +247,40 @@ __global__ __launch_bounds__(kReduceBlock) void masked_whiten_kernel(const float
     }
 }
 
+// The same from the moments that gae_scan_kernel left, in place: every workgroup adds the rows' moments
+// up in the same fixed order and whitens its share.  sum m (x - mean)^2 is expanded about the fp32 mean, in
+// fp64: its cancellation error, (mean / std)^2 * 2^-52, stays below what the rounding of the mean to fp32
+// already costs the two-pass form, (mean / std)^2 * 2^-50.  One launch over the chip in place of three
+// passes by one workgroup (128 x 2048: 5.5 us, was 314 us).
+__global__ __launch_bounds__(kReduceBlock) void whiten_moments_kernel(float* __restrict__ x,
+                                                                     const Moments* __restrict__ moments,
+                                                                     int64_t n_moments, int64_t n,
+                                                                     double* __restrict__ info) {
+    __shared__ double lds[kReduceBlock / 64 + 1];
+    Moments mom = {0.0, 0.0, 0.0};
+    for (int64_t i = threadIdx.x; i < n_moments; i += kReduceBlock) {
+        const Moments o = moments[i];
+        mom.w += o.w;
+        mom.x += o.x;
+        mom.xx += o.xx;
+    }
+    const double count = block_sum(mom.w, lds), total = block_sum(mom.x, lds), squares = block_sum(mom.xx, lds);
+    const float fc = (float)count, denom = fc + 1e-8f;
+    const float mean = (float)total / denom;
+    const double md = (double)mean;
+    const double about = squares - md * (2.0 * total - md * count);
+    float var = (float)(about < 0.0 ? 0.0 : about) / denom;           // a NaN stays one
+    if (fc != 1.f) var = var * (fc / (fc - 1.f));
+    const float scale = 1.f / sqrtf(var + 1e-8f);
+    for (int64_t e = (int64_t)blockIdx.x * kReduceBlock + threadIdx.x; e < n; e += (int64_t)gridDim.x * kReduceBlock)
+        x[e] = (x[e] - mean) * scale;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        info[0] = count;
+        info[1] = md;
+        info[2] = (double)var;
+    }
+}
+
 // ---------------------------------------------------------------------------- clipped value loss
 struct ValueTerm {
     float loss;      // max((vp - ret)^2, (clamp(vp, v - c, v + c) - ret)^2)
@@ -186,6 +307,18 @@ __device__ __forceinline__ ValueTerm value_term(float vp, float ret, float v, fl
 
 // out[0] = loss_scale * vf_loss, out[1] = vf_loss = 0.5 * masked_mean(max(l1, l2)), out[2] =
 // masked_mean(l2 > l1), out[3] = sum(mask)
+// (loss_out, if given: out[0] once more, a 0-dim tensor of its own for autograd)
+__device__ __forceinline__ void write_value_loss(double ssum, double csum, double count, float loss_scale,
+                                                 float* __restrict__ out, float* __restrict__ loss_out) {
+    const float denom = (float)count + 1e-8f;
+    const float vf = 0.5f * ((float)ssum / denom);
+    out[0] = loss_scale * vf;
+    out[1] = vf;
+    out[2] = (float)csum / denom;
+    out[3] = (float)count;
+    if (loss_out) *loss_out = loss_scale * vf;
+}
+
 __global__ __launch_bounds__(kReduceBlock) void value_loss_fwd_kernel(
     const float* __restrict__ vpreds, const float* __restrict__ returns, const float* __restrict__ values,
     const void* __restrict__ mask, int mdtype, const void* __restrict__ lens, int ldtype, int64_t batch,
@@ -206,15 +339,60 @@ __global__ __launch_bounds__(kReduceBlock) void value_loss_fwd_kernel(
     const double ssum = block_sum(s, lds);
     const double csum = block_sum(cf, lds);
     const double count = block_sum(cnt, lds);
+    if (threadIdx.x == 0) write_value_loss(ssum, csum, count, loss_scale, out, nullptr);
+}
+
+// The same spread over the chip: one workgroup per row (rows strided beyond kLossRows of them) leaves its
+// three sums in fp64, a second launch adds them up in a fixed order.  128 x 2048: 11 us for both, was
+// 167 us by one workgroup, which pays off only where no scratch memory is at hand.
+constexpr int64_t kLossRows = 1024;
+struct LossSums {
+    double loss, clipped, count;
+};
+
+__global__ __launch_bounds__(256) void value_loss_rows_kernel(
+    const float* __restrict__ vpreds, const float* __restrict__ returns, const float* __restrict__ values,
+    const void* __restrict__ mask, int mdtype, const void* __restrict__ lens, int ldtype, int64_t batch,
+    int64_t width, float clip, LossSums* __restrict__ sums) {
+    __shared__ double part[3][256 / 64];
+    double acc[3] = {0.0, 0.0, 0.0};
+    for (int64_t i = blockIdx.x; i < batch; i += gridDim.x) {
+        for (int64_t j = threadIdx.x; j < width; j += 256) {
+            const float m = mask_at(mask, mdtype, lens, ldtype, i, j, width);
+            acc[2] += (double)m;
+            if (m != 0.f) {
+                const int64_t e = i * width + j;
+                const ValueTerm t = value_term(vpreds[e], returns[e], values[e], clip);
+                acc[0] += (double)(t.loss * m);
+                acc[1] += (double)(t.clipped * m);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) acc[q] += __shfl_xor(acc[q], off, 64);
+        if ((threadIdx.x & 63) == 0) part[q][threadIdx.x >> 6] = acc[q];
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        const float denom = (float)count + 1e-8f;
-        const float vf = 0.5f * ((float)ssum / denom);
-        out[0] = loss_scale * vf;
-        out[1] = vf;
-        out[2] = (float)csum / denom;
-        out[3] = (float)count;
+        double s[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) s[q] = (part[q][0] + part[q][1]) + (part[q][2] + part[q][3]);
+        sums[blockIdx.x] = {s[0], s[1], s[2]};
     }
 }
+
+__global__ __launch_bounds__(kReduceBlock) void value_loss_finish_kernel(const LossSums* __restrict__ sums, int n,
+                                                                        float loss_scale, float* __restrict__ out,
+                                                                        float* __restrict__ loss_out) {
+    __shared__ double lds[kReduceBlock / 64 + 1];
+    LossSums s = {0.0, 0.0, 0.0};
+    if ((int)threadIdx.x < n) s = sums[threadIdx.x];       // n <= kLossRows = kReduceBlock
+    const double ssum = block_sum(s.loss, lds), csum = block_sum(s.clipped, lds), count = block_sum(s.count, lds);
+    if (threadIdx.x == 0) write_value_loss(ssum, csum, count, loss_scale, out, loss_out);
+}
+static_assert(kLossRows == kReduceBlock, "the finishing workgroup takes one partial sum per thread");
 
 __global__ __launch_bounds__(256) void value_loss_bwd_kernel(
     const float* __restrict__ vpreds, const float* __restrict__ returns, const float* __restrict__ values,
@@ -273,8 +451,46 @@ extern "C" int mrl_gae_scan(const float* rewards, const float* values, int64_t b
     MRL_REQUIRE(advantages != rewards && advantages != values && returns != rewards && returns != values &&
                     advantages != returns,
                 MRL_ERR_INVALID_ARG, "%s: outputs must not alias the inputs or each other", fn);
-    hipLaunchKernelGGL(gae_scan_kernel, dim3((unsigned)batch), dim3(kScanBlock), 0, mrl::as_stream(stream), rewards,
-                       values, width, gamma, gamma_lam, advantages, returns);
+    hipLaunchKernelGGL(gae_scan_kernel<false>, dim3((unsigned)batch), dim3(kScanBlock), 0, mrl::as_stream(stream),
+                       rewards, values, width, gamma, gamma_lam, advantages, returns, (const void*)nullptr, 0,
+                       (Moments*)nullptr);
+    return mrl::check_launch(fn);
+}
+
+extern "C" int64_t mrl_gae_whiten_workspace_bytes(int64_t batch) {
+    return batch < 0 ? 0 : batch * (int64_t)sizeof(Moments);
+}
+
+extern "C" int mrl_gae_whiten(const float* rewards, const float* values, const void* mask, int mask_dtype, int64_t batch,
+                              int64_t width, float gamma, float gamma_lam, float* advantages, float* returns,
+                              double* info, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "mrl_gae_whiten";
+    MRL_REQUIRE(batch >= 0 && width > 0 && batch <= 0x7fffffffLL, MRL_ERR_INVALID_ARG, "%s: batch=%lld width=%lld", fn,
+                (long long)batch, (long long)width);
+    MRL_REQUIRE(mrl::mask_dtype_bytes(mask_dtype) != 0, MRL_ERR_UNSUPPORTED, "%s: mask dtype %d", fn, mask_dtype);
+    MRL_REQUIRE(info != nullptr, MRL_ERR_INVALID_ARG, "%s: info is NULL", fn);
+    MRL_REQUIRE(batch == 0 || (rewards && values && mask && advantages && returns && workspace), MRL_ERR_INVALID_ARG,
+                "%s: NULL pointer", fn);
+    MRL_REQUIRE(mrl::aligned(workspace, 8) && mrl::aligned(info, 8), MRL_ERR_MISALIGNED,
+                "%s: workspace and info must be 8-byte aligned", fn);
+    MRL_REQUIRE(workspace_bytes >= mrl_gae_whiten_workspace_bytes(batch), MRL_ERR_INVALID_ARG,
+                "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
+                (long long)mrl_gae_whiten_workspace_bytes(batch));
+    MRL_REQUIRE(batch == 0 || (advantages != rewards && advantages != values && returns != rewards && returns != values &&
+                               advantages != returns),
+                MRL_ERR_INVALID_ARG, "%s: outputs must not alias the inputs or each other", fn);
+    hipStream_t s = mrl::as_stream(stream);
+    Moments* moments = reinterpret_cast<Moments*>(workspace);
+    if (batch > 0) {
+        hipLaunchKernelGGL(gae_scan_kernel<true>, dim3((unsigned)batch), dim3(kScanBlock), 0, s, rewards, values, width,
+                           gamma, gamma_lam, advantages, returns, mask, mask_dtype, moments);
+        const int rc = mrl::check_launch(fn);
+        if (rc != MRL_OK) return rc;
+    }
+    // one entry per thread up to a workgroup per CU; every workgroup reads all moments
+    const int64_t n = batch * width, want = (n + kReduceBlock - 1) / kReduceBlock;
+    hipLaunchKernelGGL(whiten_moments_kernel, dim3((unsigned)(want < 1 ? 1 : (want < 256 ? want : 256))),
+                       dim3(kReduceBlock), 0, s, advantages, (const Moments*)moments, batch, n, info);
     return mrl::check_launch(fn);
 }
 
@@ -303,6 +519,39 @@ extern "C" int mrl_value_loss_fwd(const float* vpreds, const float* returns, con
     hipLaunchKernelGGL(value_loss_fwd_kernel, dim3(1), dim3(kReduceBlock), 0, mrl::as_stream(stream), vpreds, returns,
                        values, mask, mask_dtype, response_length, length_dtype, batch, width, cliprange_value, loss_scale,
                        out);
+    return mrl::check_launch(fn);
+}
+
+extern "C" int64_t mrl_value_loss_workspace_bytes(int64_t batch) {
+    return batch < 0 ? 0 : (batch < kLossRows ? batch : kLossRows) * (int64_t)sizeof(LossSums);
+}
+
+extern "C" int mrl_value_loss_fwd_split(const float* vpreds, const float* returns, const float* values, const void* mask,
+                                        int mask_dtype, const void* response_length, int length_dtype, int64_t batch,
+                                        int64_t width, float cliprange_value, float loss_scale, float* out,
+                                        float* loss_out, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "mrl_value_loss_fwd_split";
+    MRL_REQUIRE(batch >= 0 && width > 0, MRL_ERR_INVALID_ARG, "%s: batch=%lld width=%lld", fn, (long long)batch,
+                (long long)width);
+    int rc = check_mask(fn, mask, mask_dtype, response_length, length_dtype);
+    if (rc != MRL_OK) return rc;
+    MRL_REQUIRE(out != nullptr && (batch == 0 || (vpreds && returns && values && workspace)), MRL_ERR_INVALID_ARG,
+                "%s: NULL pointer", fn);
+    MRL_REQUIRE(mrl::aligned(workspace, 8), MRL_ERR_MISALIGNED, "%s: workspace must be 8-byte aligned", fn);
+    MRL_REQUIRE(workspace_bytes >= mrl_value_loss_workspace_bytes(batch), MRL_ERR_INVALID_ARG,
+                "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
+                (long long)mrl_value_loss_workspace_bytes(batch));
+    hipStream_t s = mrl::as_stream(stream);
+    LossSums* sums = reinterpret_cast<LossSums*>(workspace);
+    const int rows = (int)(batch < kLossRows ? batch : kLossRows);
+    if (rows > 0) {
+        hipLaunchKernelGGL(value_loss_rows_kernel, dim3((unsigned)rows), dim3(256), 0, s, vpreds, returns, values, mask,
+                           mask_dtype, response_length, length_dtype, batch, width, cliprange_value, sums);
+        rc = mrl::check_launch(fn);
+        if (rc != MRL_OK) return rc;
+    }
+    hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums, rows,
+                       loss_scale, out, loss_out);
     return mrl::check_launch(fn);
 }
 

@@ -70,15 +70,20 @@ SIGNATURES = {
     "mrl_first_match": [_vp, _int, _i64, _i64, _i64, _int, _vp, _vp],
     "mrl_kl_token_rewards": [_vp, _vp, _vp, _int, _vp, _i64, _i64, _int, _f32, _vp, _vp, _vp],
     "mrl_gae_scan": [_vp, _vp, _i64, _i64, _f32, _f32, _vp, _vp, _vp],
+    "mrl_gae_whiten_workspace_bytes": [_i64],
+    "mrl_gae_whiten": [_vp, _vp, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
     "mrl_masked_whiten": [_vp, _vp, _int, _i64, _int, _vp, _vp, _vp],
     "mrl_value_loss_fwd": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp],
+    "mrl_value_loss_workspace_bytes": [_i64],
+    "mrl_value_loss_fwd_split": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _i64, _vp],
     "mrl_value_loss_bwd": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _vp],
     "mrl_copy_bytes": [_vp, _vp, _i64, _vp],
     "mrl_bandwidth_probe": [_int, _vp, _vp, _i64, _i64, _vp],
 }
 _RESTYPES = {"mrl_last_error": ctypes.c_char_p, "mrl_fused_workspace_bytes": ctypes.c_int64, "mrl_fused_max_vocab": ctypes.c_int64,
              "mrl_lmhead_workspace_bytes": ctypes.c_int64, "mrl_lmhead_static_max_tokens": ctypes.c_int64,
-             "mrl_set_wide_spin_limit": ctypes.c_int64}
+             "mrl_set_wide_spin_limit": ctypes.c_int64, "mrl_gae_whiten_workspace_bytes": ctypes.c_int64,
+             "mrl_value_loss_workspace_bytes": ctypes.c_int64}
 
 _lib = None
 

@@ -103,13 +103,18 @@ def compute_gae_advantage_return(token_level_rewards, values, eos_mask, gamma, l
     if rewards.dim() != 2 or rewards.shape != vals.shape:
         raise ValueError("token_level_rewards and values must both be [batch, response_length]")
     batch, width = rewards.shape
+    mask, _ = _mask_args(eos_mask.expand_as(rewards) if eos_mask.shape != rewards.shape else eos_mask, None, dev)
     adv = torch.empty_like(rewards)
     ret = torch.empty_like(rewards)
+    small = torch.empty(3 + 3 * batch, dtype=torch.float64, device=dev)     # info, then the rows' moments
     # `gamma * lam` as python evaluates it inside the reference's `gamma * lam * lastgaelam`: in double
     # for python floats (the config's values), in the tensors' own precision for 0-dim tensors
-    _lib.call("mrl_gae_scan", _lib.ptr(rewards), _lib.ptr(vals), batch, width, float(gamma), float(gamma * lam),
-              _lib.ptr(adv), _lib.ptr(ret), _lib.stream(dev))
-    return masked_whiten(adv, eos_mask), ret
+    _lib.call("mrl_gae_whiten", _lib.ptr(rewards), _lib.ptr(vals), _lib.ptr(mask), _lib.dtype_code(mask), batch, width,
+              float(gamma), float(gamma * lam), _lib.ptr(adv), _lib.ptr(ret), small.data_ptr(), small.data_ptr() + 24,
+              24 * batch, _lib.stream(dev))
+    if small[0].item() == 0:
+        raise ValueError("At least one element in the mask has to be 1.")
+    return adv, ret
 
 
 class _ValueLoss(torch.autograd.Function):
@@ -122,15 +127,18 @@ class _ValueLoss(torch.autograd.Function):
         ret, val = _f32(returns, dev), _f32(values, dev)
         batch, width = vp.shape
         out = torch.empty(4, dtype=torch.float32, device=dev)
-        args = (_lib.ptr(vp), _lib.ptr(ret), _lib.ptr(val), _lib.ptr(mask),
-                _lib.dtype_code(mask) if mask is not None else _lib.F32, _lib.ptr(lens),
-                _lib.dtype_code(lens) if lens is not None else _lib.I32, batch, width, float(clip), float(loss_scale))
-        _lib.call("mrl_value_loss_fwd", *args, _lib.ptr(out), _lib.stream(dev))
+        loss = torch.empty((), dtype=torch.float32, device=dev)     # autograd outputs must not alias
+        ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(batch)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        _lib.call("mrl_value_loss_fwd_split", _lib.ptr(vp), _lib.ptr(ret), _lib.ptr(val), _lib.ptr(mask),
+                  _lib.dtype_code(mask) if mask is not None else _lib.F32, _lib.ptr(lens),
+                  _lib.dtype_code(lens) if lens is not None else _lib.I32, batch, width, float(clip), float(loss_scale),
+                  _lib.ptr(out), _lib.ptr(loss), _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
         ctx.save_for_backward(vp, ret, val, mask, lens, out)
         ctx.scalars = (float(clip), float(loss_scale))
         ctx.in_dtype = vpreds.dtype
         ctx.mark_non_differentiable(out)
-        return out[0].clone(), out
+        return loss, out
 
     @staticmethod
     def backward(ctx, g_loss, _g_out):

@@ -569,6 +569,39 @@ def test_gae_and_whitening_parity(dev, batch, width):
         1.0, r.abs().max().item() * 2)
 
 
+@pytest.mark.parametrize("batch,width", [(1, 1), (2, 2), (1025, 3), (5, 17), (3, 4095), (2, 4096), (2, 4097), (1, 8195)])
+def test_gae_whitening_and_value_loss_at_the_edges_of_their_split(dev, batch, width):
+    """Rows of one and of several staging chunks with every remainder of the groups of 4, more rows than
+    the value loss has workgroups, and advantages far from zero (a constant reward without discount: the
+    expanded second moment).  The variance is checked against fp64: the fp32 mean's rounding, 2^-24 of it,
+    enters squared; the quotient and the root cost a few fp32 roundings."""
+    gen = torch.Generator().manual_seed(batch + width)
+    v = torch.randn(batch, width, generator=gen)
+    mask = (torch.rand(batch, width, generator=gen) < 0.7).long()
+    mask.view(-1)[:2] = 1
+    for r in (torch.randn(batch, width, generator=gen), torch.full((batch, width), 3.0)):
+        _, want_ret = o_adv.compute_gae_advantage_return(r, v, mask, 1.0, 0.95)
+        adv, ret = mrl.compute_gae_advantage_return(r.to(dev), v.to(dev), mask.to(dev), 1.0, 0.95)
+        assert torch.equal(ret.cpu(), want_ret)
+        if batch * width == 1:
+            continue                                                    # one entry has no spread to whiten by
+        raw = (want_ret - v).double()                                   # to 2^-24 of the returns
+        m = mask.double()
+        mean = (raw * m).sum() / m.sum()
+        var = (((raw - mean) ** 2) * m).sum() / (m.sum() - 1)
+        want = (raw - mean) / (var + 1e-8).sqrt()
+        slack = 2.0 ** -22 * (want_ret.abs().max().item() + mean.abs().item()) / (var + 1e-8).sqrt().item()
+        assert (adv.cpu().double() - want).abs().max().item() < slack + 1e-6 * want.abs().max().item()
+    with pytest.raises(ValueError, match="At least one element"):
+        mrl.compute_gae_advantage_return(v.to(dev), v.to(dev), torch.zeros_like(mask).to(dev), 1.0, 0.95)
+    returns = v + torch.randn(batch, width, generator=gen)
+    vp = v + torch.randn(batch, width, generator=gen)
+    want, want_frac = o_loss.value_loss(vp.double(), returns.double(), v.double(), mask.double(), 0.5)
+    got, out = mrl.value_loss(vp.to(dev), returns.to(dev), v.to(dev), mask.to(dev), cliprange_value=0.5)
+    assert got.item() == pytest.approx(want.item(), rel=TOL_LOSS_REL) and out[0].item() == got.item()
+    assert out[2].item() == pytest.approx(want_frac.item(), rel=1e-5, abs=1e-8) and out[3].item() == mask.sum().item()
+
+
 @pytest.mark.parametrize("penalty", ["kl", "abs", "mse", "low_var_kl"])
 def test_kl_token_rewards_parity(dev, penalty):
     gen = torch.Generator().manual_seed(17)
