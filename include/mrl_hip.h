@@ -334,9 +334,10 @@ int mrl_fused_loss_prepare(int layout, int64_t batch, int64_t width, int64_t n_r
  * workspace must not be shared by sweeps that can be in flight at the same time, and a captured
  * graph keeps using the address it was captured with.  NULL is allowed for rows that one workgroup
  * holds: every row then gets a workgroup of its own, which costs large batches about a quarter more
- * time.  Needs 16-byte aligned rows, vocab % (16/elem) == 0 and
- * vocab <= mrl_fused_max_vocab(dtype); else MRL_ERR_UNSUPPORTED (use the split fwd/bwd entry points
- * then).  The wait of a workgroup for the other half of its row is bounded
+ * time.  Needs 16-byte aligned rows, vocab % (16/elem) == 0 and vocab <= mrl_fused_max_vocab(dtype),
+ * or rows of at least 8 KiB and at most half that vocab at any element alignment, if every row of
+ * dlogits lies at the same address modulo 16 as its row of logits (the same strides and equally
+ * aligned tensors); else MRL_ERR_UNSUPPORTED (use the split fwd/bwd entry points then).  The wait of a workgroup for the other half of its row is bounded
  * (mrl_set_wide_spin_limit): past the bound it computes that half's statistics itself from memory,
  * with the same result to the last bit; in place that is safe because a workgroup overwrites its
  * half only after its record has reached memory, and a reader that finds the record after all
@@ -375,7 +376,8 @@ int mrl_fused_loss_reduce(const float* row_terms, const int64_t* row_start,
  * exits without touching memory).  upstream and applied are DEVICE scalars: the gradient autograd
  * delivers and the scale x already carries.  Lets the eager gradient honour whatever scalar arrives
  * (Megatron's 1/num_microbatches and loss scale) without a host synchronisation.  Neither scalar is
- * written; follow the last mrl_scale_rows of a backward with mrl_grad_scale_note. */
+ * written; follow the last mrl_scale_rows of a backward with mrl_grad_scale_note.  x is 16-byte
+ * aligned; its rows are, too (row_stride and vocab whole vectors), or they are dense. */
 int mrl_scale_rows(void* x, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,
                    const float* upstream, const float* applied, void* stream);
 

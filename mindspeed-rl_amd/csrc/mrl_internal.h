@@ -39,6 +39,12 @@ __device__ __forceinline__ void buf_store_nt(u32x4 v, rsrc_t r, uint32_t byte_of
     __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)byte_off, 0, 2);
 }
 // single entries, same cache policy as the vectors
+__device__ __forceinline__ uint32_t buf_load_b16(rsrc_t r, uint32_t byte_off) {
+    return (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, (int)byte_off, 0, 2);
+}
+__device__ __forceinline__ uint32_t buf_load_b32(rsrc_t r, uint32_t byte_off) {
+    return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)byte_off, 0, 2);
+}
 __device__ __forceinline__ void buf_store_b16(uint16_t v, rsrc_t r, uint32_t byte_off) {
     __builtin_amdgcn_raw_buffer_store_b16((short)v, r, (int)byte_off, 0, 2);
 }
@@ -55,6 +61,8 @@ struct rsrc_t {};
 __device__ inline rsrc_t make_rsrc(const void*, uint32_t) { return rsrc_t(); }
 __device__ inline u32x4 buf_load_nt(rsrc_t, uint32_t) { return make_u32x4(0, 0, 0, 0); }
 __device__ inline u32x4 buf_load(rsrc_t, uint32_t, uint32_t) { return make_u32x4(0, 0, 0, 0); }
+__device__ inline uint32_t buf_load_b16(rsrc_t, uint32_t) { return 0; }
+__device__ inline uint32_t buf_load_b32(rsrc_t, uint32_t) { return 0; }
 __device__ inline void buf_store_nt(u32x4, rsrc_t, uint32_t) {}
 __device__ inline void buf_store_b16(uint16_t, rsrc_t, uint32_t) {}
 __device__ inline void buf_store_b32(uint32_t, rsrc_t, uint32_t) {}

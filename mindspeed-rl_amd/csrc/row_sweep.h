@@ -24,6 +24,7 @@ struct FusedArgs {
     void* workspace;                // nullable for narrow rows: row counter (+ half-row records)
     bool workspace_cleared;         // the caller has zeroed it on this stream
     bool wide;                      // rows cut in two halves held by two workgroups
+    bool edge;                      // rows do not all start on a 128-byte line
     int64_t half_elems;             // entries of the first half
     void* dlogits; int64_t d_stride;
     float* logp; float* entropy; float* row_terms;
@@ -45,8 +46,10 @@ int launch_bwd_chunks(const BwdArgs& a);
 bool bwd_chunks_supported(int dtype, int64_t vocab, const void* in, int64_t in_stride, const void* out,
                           int64_t out_stride, int64_t n_rows);
 
-// True if rows of this dtype / vocab / alignment fit the row-in-registers kernels.
-bool row_sweep_supported(int dtype, int64_t vocab, const void* in, int64_t in_stride, const void* out,
-                         int64_t out_stride, int64_t n_rows);
+enum class RowLayout { none, vectors, edges };
+
+// How the row-in-registers kernel takes rows of this dtype / vocab / alignment; none: it does not.
+RowLayout row_sweep_layout(int dtype, int64_t vocab, const void* in, int64_t in_stride, const void* out,
+                           int64_t out_stride, int64_t n_rows);
 
 }  // namespace mrl

@@ -1,18 +1,17 @@
 // Row-in-registers vocabulary sweeps for gfx950.
 //
-// One workgroup of 1024 threads (16 wavefronts, one workgroup per CU) owns one logits row and
-// keeps ALL of it in registers: up to 19 16-byte vectors per thread = 311 296 bytes, enough for a
-// 152 064-entry bf16 row.  The softmax statistics are taken vector by vector as the data arrives,
-// the token's loss gradient follows from them, and dlogits are written from the same registers -
+// A workgroup owns one logits row and keeps ALL of it in registers: 256 threads for the shortest rows,
+// several workgroups per CU, up to 1024 threads with 19 16-byte vectors each = 311 296 bytes, one per CU,
+// enough for a 152 064-entry bf16 row.  The softmax statistics are taken vector by vector as the data
+// arrives, the token's loss gradient follows from them, and dlogits are written from the same registers -
 // one HBM read and one HBM write per element for the whole forward + backward of the log-prob /
 // policy-loss path.  The requests of a row are issued together (the HBM system serves a row best
 // that way) and all accesses are range-checked buffer accesses, so the unrolled bodies contain no
 // branch (see mrl_internal.h for why that matters).
 //
-// fused_sweep_kernel launches one workgroup per row (small batches, or no workspace);
-// fused_sweep_persistent_kernel launches one workgroup per CU that takes rows in ticket order and
-// requests its next row while it writes the current one.  bwd_chunk_kernel is the split path's backward
-// (upstream gradients and the log-sum-exp are inputs, so there is no statistics pass and nothing
+// fused_sweep_persistent_kernel launches as many workgroups as the chip holds; they take rows in ticket
+// order and request the next row while they write the current one.  bwd_chunk_kernel is the split path's
+// backward (upstream gradients and the log-sum-exp are inputs, so there is no statistics pass and nothing
 // has to stay on chip): a plain stream of one vector per thread.
 #include <atomic>
 
@@ -38,14 +37,12 @@ using namespace mrl_loss;
 #define MRL_BWD_CHUNK_THREADS 256
 #endif
 
-constexpr int kBlock = 1024;
-constexpr int kWaves = kBlock / 64;
-
-// Two-level reduction for 16 wavefronts: shuffles inside each wavefront, then the first
-// wavefront combines the 16 partials with shuffles again (a serial combine by every thread
-// would cost more ALU time than a sixth of the row).
-template <bool kEntropy>
-__device__ __forceinline__ Stats block_reduce_1024(Stats st, float k, Stats* lds) {
+// Two-level reduction for the BLK / 64 wavefronts of a workgroup: shuffles inside each wavefront, then the
+// first wavefront combines the partials with shuffles again (a serial combine of 16 of them by every thread
+// would cost more ALU time than a sixth of the row).  lds: BLK / 64 + 1 entries.
+template <int BLK, bool kEntropy>
+__device__ __forceinline__ Stats reduce_workgroup(Stats st, float k, Stats* lds) {
+    constexpr int kWaves = BLK / 64;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         Stats o;
@@ -92,15 +89,16 @@ __device__ __forceinline__ float grad_elem(const RowGrad& g, float z) {
     return e * w;
 }
 
-// The kernels are instantiated for NV in {4, 8, 12, 16, 19} vectors per thread and the host picks
-// the smallest NV that holds the row, so the vectors below kFull are complete for every thread;
-// only the last few can reach past the end of the row.
-template <int NV>
+// Vectors that are complete for every thread of a row that the host gives to a workgroup of BLK threads
+// with NV vectors each (see pick_shape for the shortest such rows); the later ones may be partly or wholly
+// past the end of the row.  A row with edges has up to 8 vectors less than its length suggests.
+template <int BLK, int NV, bool kEdge>
 struct Tail {
-    static constexpr int kFull = NV == 19 ? 16 : NV - 4;
+    static constexpr int kRow = NV <= 4 ? 0 : (NV <= 8 || BLK * NV == 512 * 12 ? 4 : (NV == 19 ? 16 : NV - 4));
+    static constexpr int kFull = kRow - (kEdge && kRow > 0 ? 1 : 0);
 };
 
-// Vector q of a row is addressed through a descriptor of its own (the row from byte q * 16 KiB on,
+// Vector q of a row is addressed through a descriptor of its own (the row from byte q * 16 * BLK on,
 // clamped to empty) with the same per-thread byte offset for every q: the descriptors live in
 // scalar registers and cost scalar instructions, where one vector offset per q would cost 19
 // vector registers that the row itself needs.
@@ -114,10 +112,11 @@ __device__ __forceinline__ RowRef row_ref(const void* base, uint32_t bytes) {
     return r;
 }
 
+template <int BLK>
 __device__ __forceinline__ mrl::rsrc_t vec_rsrc(const RowRef& row, int q) {
     // signed arithmetic on purpose: an unsigned saturating subtraction is selected as a VECTOR
     // instruction, which would make the descriptor non-uniform
-    const int skip = q * (kBlock * 16);
+    const int skip = q * (BLK * 16);
     const int rest = (int)row.bytes - skip;
     return mrl::make_rsrc(row.base + skip, (uint32_t)(rest > 0 ? rest : 0));
 }
@@ -129,40 +128,23 @@ __device__ __forceinline__ void vector_fence() { __builtin_amdgcn_sched_barrier(
 
 __device__ __forceinline__ uint32_t lane_offset() { return (uint32_t)threadIdx.x * 16u; }
 
-// All loads of a row, back to back and without a branch: vectors past the end of the row come back
-// as zeros from the range check of the buffer access.
-template <int NV>
-__device__ __forceinline__ void load_row(u32x4 (&v)[NV], const RowRef& src) {
+// Vectors [A, B) of a row: loads (back to back and without a branch: vectors past the end of the row come
+// back as zeros from the range check of the buffer access), zero stores.
+template <int BLK, int A, int B, int NV>
+__device__ __forceinline__ void load_part(u32x4 (&v)[NV], const RowRef& src) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        v[q] = mrl::buf_load_nt(vec_rsrc(src, q), lane_offset());
+    for (int q = A; q < B; ++q) {
+        v[q] = mrl::buf_load_nt(vec_rsrc<BLK>(src, q), lane_offset());
         vector_fence();     // keeps the requests in this order wherever a row is loaded
     }
 }
 
-template <int NV>
-__device__ __forceinline__ void zero_row(const RowRef& dst) {
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int q = 0; q < NV; ++q) mrl::buf_store_nt(zero, vec_rsrc(dst, q), lane_offset());
-}
-
-// Vectors [A, B) of a row: loads, zero stores.
-template <int A, int B, int NV>
-__device__ __forceinline__ void load_part(u32x4 (&v)[NV], const RowRef& src) {
-#pragma unroll
-    for (int q = A; q < B; ++q) {
-        v[q] = mrl::buf_load_nt(vec_rsrc(src, q), lane_offset());
-        vector_fence();
-    }
-}
-
-template <int A, int B>
+template <int BLK, int A, int B>
 __device__ __forceinline__ void zero_part(const RowRef& dst) {
     const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int q = A; q < B; ++q) {
-        mrl::buf_store_nt(zero, vec_rsrc(dst, q), lane_offset());
+        mrl::buf_store_nt(zero, vec_rsrc<BLK>(dst, q), lane_offset());
         vector_fence();
     }
 }
@@ -172,7 +154,7 @@ __device__ __forceinline__ void zero_part(const RowRef& dst) {
 // (infinities and NaN included).  A vector past the end of the row (zeros from the range-checked load)
 // is processed like any other and its result discarded, which costs three selects on the few vectors
 // that can be affected and keeps the pass free of branches.
-template <int DT, int NV, bool kEntropy>
+template <int DT, int BLK, int NV, bool kEntropy, bool kEdge>
 __device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int n_vec, float k) {
     using E = Elem<DT>;
     constexpr int kVec = E::kVec;
@@ -193,8 +175,8 @@ __device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int 
         const float mk = nx.m * k;
 #pragma unroll
         for (int i = 0; i < kVec; ++i) add_one<kEntropy>(nx, z[i], k, mk);
-        if (q >= Tail<NV>::kFull) {
-            const bool valid = q * kBlock + (int)threadIdx.x < n_vec;
+        if (q >= Tail<BLK, NV, kEdge>::kFull) {
+            const bool valid = q * BLK + (int)threadIdx.x < n_vec;
             st.m = valid ? nx.m : st.m;
             st.s = valid ? nx.s : st.s;
             st.u = valid ? nx.u : st.u;
@@ -247,34 +229,46 @@ __device__ __forceinline__ float vector_max(const u32x4& vec) {
 
 // want_max (uniform over the workgroup): the caller needs the true maximum of the row in m (a label
 // outside the vocabulary scores the row maximum), which only the careful pass delivers.
-template <int DT, int NV, bool kEntropy>
-__device__ __forceinline__ Stats thread_stats(const u32x4 (&v)[NV], int n_vec, float k, bool want_max) {
+// kEdge: the thread also holds one entry of the row outside its vectors, z_edge, if has_edge.
+template <int DT, int BLK, int NV, bool kEntropy, bool kEdge>
+__device__ __forceinline__ Stats thread_stats(const u32x4 (&v)[NV], int n_vec, float k, bool want_max, bool has_edge,
+                                              float z_edge) {
     Stats st = {kMaxInit, 0.f, 0.f};
-    // rows so short that a thread may hold no complete vector at all have nothing to gain
-    bool careful = Tail<NV>::kFull == 0 || want_max;
+    // in a row so short that a thread may hold no complete vector there is no reference to take
+    bool careful = (Tail<BLK, NV, kEdge>::kFull == 0 && n_vec < BLK) || want_max;
     if (!careful) {
         st.m = vector_max<DT>(v[0]);
         const float rk = st.m * k;
 #pragma unroll
         for (int q = 0; q < NV; ++q) {
-            float s = st.s, u = st.u;
-            add_vector<DT, kEntropy>(v[q], k, rk, s, u);
-            if (q >= Tail<NV>::kFull) {
-                const bool valid = q * kBlock + (int)threadIdx.x < n_vec;
+            if (q < Tail<BLK, NV, kEdge>::kFull) {
+                add_vector<DT, kEntropy>(v[q], k, rk, st.s, st.u);
+            } else if (q * BLK < n_vec) {               // uniform: nothing to compute past the end of the row
+                float s = st.s, u = st.u;
+                add_vector<DT, kEntropy>(v[q], k, rk, s, u);
+                const bool valid = q * BLK + (int)threadIdx.x < n_vec;
                 st.s = valid ? s : st.s;
                 st.u = valid ? u : st.u;
-            } else {
-                st.s = s;
-                st.u = u;
             }
             asm volatile("" : "+v"(st.s), "+v"(st.u));       // as in the careful pass
             // nothing but the two sums links one vector to the next here, so the scheduler would
             // unpack many vectors ahead of their use; keep each vector's work together
             vector_fence();
         }
+        if (kEdge) {
+            const float e = fast_exp2(__builtin_fmaf(z_edge, k, -rk));
+            st.s = has_edge ? st.s + e : st.s;
+            if (kEntropy) st.u = has_edge ? __builtin_fmaf(e, z_edge, st.u) : st.u;
+        }
         careful = !(st.s < kSumLimit);
     }
-    if (careful) st = thread_stats_careful<DT, NV, kEntropy>(v, n_vec, k);
+    if (careful) {
+        st = thread_stats_careful<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k);
+        if (kEdge && has_edge) {
+            grow_max<kEntropy>(st, z_edge, k);
+            add_one<kEntropy>(st, z_edge, k, st.m * k);
+        }
+    }
     return st;
 }
 
@@ -295,25 +289,64 @@ __device__ __forceinline__ u32x4 grad_vec(const u32x4& v, const RowGrad& g) {
 }
 
 // dlogits of vectors [A, B) of the row in registers, stored as they are computed.
-template <int DT, bool kEntropy, int A, int B, int NV>
+template <int DT, int BLK, bool kEntropy, int A, int B, int NV>
 __device__ __forceinline__ void grad_part(const u32x4 (&v)[NV], const RowGrad& g, const RowRef& dst) {
 #pragma unroll
     for (int q = A; q < B; ++q) {
-        mrl::buf_store_nt(grad_vec<DT, kEntropy>(v[q], g), vec_rsrc(dst, q), lane_offset());
+        mrl::buf_store_nt(grad_vec<DT, kEntropy>(v[q], g), vec_rsrc<BLK>(dst, q), lane_offset());
         vector_fence();
     }
 }
 
+// Rows that do not all start on a 128-byte line: `head` entries before the first line, n_vec 16-byte vectors
+// from there, the rest behind them.  The entries outside the vectors ("edge": at most 63 + 7) go to the first
+// threads, one each, through accesses of a single entry; the vectors are accessed like those of an aligned
+// row.  16-byte alignment would do for the accesses, but then every wavefront's 1 KiB cuts two lines in
+// half: 32 003 bf16 logits 4 958 GB/s, on lines 5 433; 129 288 5 334 -> 5 901; 50 260 fp32 5 580 -> 6 095
+// (what rows of 32 000, 129 280 and 50 304 reach).
+struct RowSpan {
+    int head, n_vec;
+};
+constexpr int kEdgeAlign = 128;
+
+template <int DT>
+__device__ __forceinline__ RowSpan row_span(const typename Elem<DT>::T* row, int vocab) {
+    constexpr int kVec = Elem<DT>::kVec;
+    const int mis = (int)((reinterpret_cast<uintptr_t>(row) % kEdgeAlign) / sizeof(typename Elem<DT>::T));
+    RowSpan s;
+    s.head = mis ? kEdgeAlign / (int)sizeof(typename Elem<DT>::T) - mis : 0;
+    s.n_vec = (vocab - s.head) / kVec;
+    return s;
+}
+
+// Byte offset inside the row of this thread's edge entry, out of range for a thread without one.
+template <int DT>
+__device__ __forceinline__ uint32_t edge_offset(const RowSpan& s, int vocab) {
+    constexpr int kVec = Elem<DT>::kVec;
+    const int tid = (int)threadIdx.x;
+    const int j = tid < s.head ? tid : tid + s.n_vec * kVec;
+    return j < vocab ? (uint32_t)j * (uint32_t)sizeof(typename Elem<DT>::T) : 0x80000000u;
+}
+
 // The label's entry gets the one-hot term on top of the softmax term.  The thread that has just
-// stored the vector holding it re-stores that single entry; for every other thread the byte offset
-// is out of range and the hardware drops the store, so there is no branch here either.  Two stores
-// of one thread to the same address stay in program order.
-template <int DT, bool kEntropy>
-__device__ __forceinline__ void store_label_grad(const RowRef& dst, const RowGrad& g, bool y_ok, int64_t y, float z_y) {
+// stored the entry re-stores it; for every other thread the byte offset is out of range and the hardware
+// drops the store, so there is no branch here either.  Two stores of one thread to the same address stay
+// in program order.  y and dst (of `bytes` bytes) are relative to the unit; span: its vectors.
+template <int DT, int BLK, bool kEntropy, bool kEdge>
+__device__ __forceinline__ void store_label_grad(const typename Elem<DT>::T* dst, uint32_t bytes, const RowSpan& span,
+                                                 const RowGrad& g, bool y_ok, int64_t y, float z_y) {
     using E = Elem<DT>;
-    const bool owner = y_ok && (int)((y / E::kVec) % kBlock) == (int)threadIdx.x;
+    int writer;
+    if (kEdge) {
+        const int body = (int)y - span.head, n_body = span.n_vec * E::kVec;
+        const bool inside = body >= 0 && body < n_body;
+        writer = inside ? (body / E::kVec) % BLK : (body < 0 ? (int)y : (int)y - n_body);
+    } else {
+        writer = (int)((y / E::kVec) % BLK);
+    }
+    const bool owner = y_ok && writer == (int)threadIdx.x;
     const uint32_t off = owner ? (uint32_t)y * (uint32_t)sizeof(typename E::T) : 0x80000000u;
-    E::buf_store(mrl::make_rsrc(dst.base, dst.bytes), off, grad_elem<kEntropy>(g, z_y) + g.onehot);
+    E::buf_store(mrl::make_rsrc(dst, bytes), off, grad_elem<kEntropy>(g, z_y) + g.onehot);
 }
 
 struct RowScalars {
@@ -369,63 +402,6 @@ __device__ __forceinline__ void write_masked_row_outputs(int64_t r, float* __res
     if (entropy) entropy[r] = 0.f;
 #pragma unroll
     for (int q = 0; q < S_N; ++q) row_terms[r * S_N + q] = 0.f;
-}
-
-template <int DT, int NV, bool kEntropy>
-__global__ __launch_bounds__(kBlock) void fused_sweep_kernel(
-    const typename Elem<DT>::T* logits, int64_t row_stride, int vocab, const void* __restrict__ labels,
-    int labels_dtype, float inv_t, const float* __restrict__ row_ops, int has_old, Params p, float grad_scale,
-    const float* __restrict__ grad_scale_dev, typename Elem<DT>::T* dlogits, int64_t d_stride,
-    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ row_terms) {
-    using E = Elem<DT>;
-    using T = typename E::T;
-    constexpr int kVec = E::kVec;
-    __shared__ Stats lds[kWaves + 1];
-
-    if (grad_scale_dev) grad_scale *= *grad_scale_dev;
-    const int64_t r = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int n_vec = vocab / kVec;
-    const uint32_t row_bytes = (uint32_t)vocab * (uint32_t)sizeof(T);
-    const T* row = logits + r * row_stride;
-    const RowRef src = row_ref(row, row_bytes);
-    const RowRef dst = row_ref(dlogits + r * d_stride, row_bytes);
-
-    const float* ops = row_ops + r * MRL_ROW_OPS;
-    const float m = ops[MRL_OP_MASK];
-    if (m == 0.f) {                       // not a response token: no gradient, nothing to read
-        zero_row<NV>(dst);
-        if (tid == 0) write_masked_row_outputs(r, logp, entropy, row_terms);
-        return;
-    }
-
-    // the whole row: every load is in flight before the first use
-    u32x4 v[NV];
-    load_row<NV>(v, src);
-    const int64_t y = load_label(labels, labels_dtype, r);
-    const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
-    const float z_y = E::load(row + (y_ok ? y : 0));
-
-    const float k = inv_t * kLog2e;
-    const Stats st = thread_stats<DT, NV, kEntropy>(v, n_vec, k, !y_ok);
-    const Stats tot = block_reduce_1024<kEntropy>(st, k, lds);
-
-    // row scalars, computed redundantly by every thread (uniform values)
-    float lse;
-    const RowScalars s = row_scalars<kEntropy>(tot, k, inv_t, y_ok, z_y, ops, has_old, p, grad_scale, m, lse);
-    if (tid == 0) write_row_outputs(r, s, m, logp, entropy, row_terms);
-
-    if (s.g_lp == 0.f && s.g_h == 0.f) {
-        zero_row<NV>(dst);
-    } else {
-        const RowGrad g = row_grad<kEntropy>(s, k, inv_t, lse);
-#pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            mrl::buf_store_nt(grad_vec<DT, kEntropy>(v[q], g), vec_rsrc(dst, q), lane_offset());
-            vector_fence();
-        }
-        store_label_grad<DT, kEntropy>(dst, g, y_ok, y, z_y);
-    }
 }
 
 // ------------------------------------------------------------------------------ row tickets
@@ -487,6 +463,8 @@ __device__ __forceinline__ unsigned long long pack2f(float lo, float hi) {
 // thread holds - the same reference, the same sums, the same second attempt - and the reduction is
 // the same.  `whole`: every thread has at least one vector and the row maximum is not asked for (what
 // makes thread_stats take the short way).
+constexpr int kWideBlock = 1024;        // threads of a workgroup that holds half a row
+
 template <int DT, bool kEntropy>
 __device__ __forceinline__ Stats stream_stats(const typename Elem<DT>::T* base, int n_vec, float k, bool whole,
                                               Stats* lds) {
@@ -498,13 +476,13 @@ __device__ __forceinline__ Stats stream_stats(const typename Elem<DT>::T* base, 
     if (whole) {
         st.m = vector_max<DT>(__builtin_nontemporal_load(vec + threadIdx.x));
         const float rk = st.m * k;
-        for (int idx = threadIdx.x; idx < n_vec; idx += kBlock)
+        for (int idx = threadIdx.x; idx < n_vec; idx += kWideBlock)
             add_vector<DT, kEntropy>(__builtin_nontemporal_load(vec + idx), k, rk, st.s, st.u);
         careful = !(st.s < kSumLimit);
     }
     if (careful) {
         st = {kMaxInit, 0.f, 0.f};
-        for (int idx = threadIdx.x; idx < n_vec; idx += kBlock) {
+        for (int idx = threadIdx.x; idx < n_vec; idx += kWideBlock) {
             float z[kVec];
             E::unpack(__builtin_nontemporal_load(vec + idx), z);
             float vmax = st.m;
@@ -517,7 +495,7 @@ __device__ __forceinline__ Stats stream_stats(const typename Elem<DT>::T* base, 
         }
     }
     __syncthreads();            // lds may still be read by a slow wavefront of the previous reduction
-    return block_reduce_1024<kEntropy>(st, k, lds);
+    return reduce_workgroup<kWideBlock, kEntropy>(st, k, lds);
 }
 
 // What thread 0 found in the other half's record.
@@ -590,24 +568,31 @@ __device__ __forceinline__ Stats exchange_halves(const Stats& mine, int half, Ha
     return half == 0 ? merge<kEntropy>(mine, other, k) : merge<kEntropy>(other, mine, k);
 }
 
-// Persistent variant of the fused sweep: one workgroup per CU walks rows and, as it turns the
+// The fused sweep: persistent workgroups walk rows and, as one turns the
 // registers of a row into dlogits, refills them with its NEXT row, so the statistics pass of the next
 // row starts on its first vectors while the last are still arriving - the register file never has to
 // hold two rows.  The next row is the next unclaimed one (see "row tickets" above), taken while the
 // row is being written.
+// row_ticket NULL: a workgroup per row, each ends with its first.
+// Wavefronts per SIMD that the register allocator leaves room for: 4 hold the widest rows (76 registers of
+// row), short rows leave more of the register file to further workgroups.
+constexpr int waves_per_simd(int nv) { return nv <= 4 ? 8 : (nv <= 8 ? 6 : 4); }
+
+// kEdge: rows of any element alignment (see RowSpan); dlogits rows are misaligned alike.
 // kWide: the units of work are half rows (see "wide rows" above): unit 2 r is the first
 // half_elems entries of row r, unit 2 r + 1 the rest; n_rows then counts units.
-template <int DT, int NV, bool kEntropy, bool kWide>
-__global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
+template <int DT, int BLK, int NV, bool kEntropy, bool kWide, bool kEdge>
+__global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persistent_kernel(
     const typename Elem<DT>::T* logits, int64_t row_stride, int vocab, int64_t n_rows,
     const void* __restrict__ labels, int labels_dtype, float inv_t, const float* __restrict__ row_ops, int has_old,
     Params p, float grad_scale, const float* __restrict__ grad_scale_dev, typename Elem<DT>::T* dlogits,
     int64_t d_stride, float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ row_terms,
-    unsigned int* row_ticket, int half_elems, HalfRecord* half_records, uint32_t spin_limit) {
+    unsigned int* row_ticket, int group, int half_elems, HalfRecord* half_records, uint32_t spin_limit) {
     using E = Elem<DT>;
     using T = typename E::T;
-    constexpr int kVec = E::kVec;
-    __shared__ Stats lds[kWaves + 1];
+    static_assert(!kWide || BLK == kWideBlock, "halves of a row are held by workgroups of kWideBlock threads");
+    static_assert(!(kWide && kEdge), "a row that two workgroups hold is aligned");
+    __shared__ Stats lds[BLK / 64 + 1];
     // two slots used in turn: thread 0 may write the ticket of the following row while a slow
     // wavefront has yet to read this one's (one barrier per row separates a slot's reuse)
     __shared__ uint32_t next_row[2];
@@ -618,10 +603,10 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
     const uint32_t unit_bytes[2] = {(uint32_t)(kWide ? half_elems : vocab) * (uint32_t)sizeof(T),
                                     (uint32_t)(kWide ? vocab - half_elems : 0) * (uint32_t)sizeof(T)};
     const float k = inv_t * kLog2e;
-    const int64_t step = gridDim.x;
     if (grad_scale_dev) grad_scale *= *grad_scale_dev;
     // the counter as a 4-byte buffer: only the lane with offset 0 (thread 0) is inside it
-    const mrl::rsrc_t ticket = mrl::make_rsrc(row_ticket, 4u);
+    const mrl::rsrc_t ticket = mrl::make_rsrc(row_ticket, row_ticket ? 4u : 0u);
+    const mrl::rsrc_t no_ticket = mrl::make_rsrc(row_ticket, 0u);
 
     // What a workgroup needs to know of the row it fetches next.  A row that is not a response token
     // is never read: its descriptor gets zero bytes, so the (unconditional) loads return zeros
@@ -631,8 +616,22 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
         int64_t y;
         const T* zy_ptr;
         RowRef row;
+        uint32_t edge_off;      // where this thread's edge entry lies in the row (kEdge)
+        const T* edge_base;
+        uint32_t edge_bytes;    // 0: not read
     };
-    int64_t r = blockIdx.x;
+    int64_t r = (int64_t)blockIdx.x * group;
+    int left = group - 1;                   // rows of the current ticket behind r
+    // the unit behind r: the next of the ticket, or the first of a new ticket (asked for in `mine`)
+    auto following = [&](uint32_t mine, int parity) {
+        if (left > 0) {
+            --left;
+            return r + 1;
+        }
+        left = group - 1;
+        const int64_t t = (int64_t)broadcast_ticket(mine, &next_row[parity]);
+        return row_ticket ? t + (int64_t)gridDim.x * group : n_rows;
+    };
     auto plan = [&](int64_t r2) {
         Next n;
         n.r = r2;
@@ -642,7 +641,15 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
         const int hn = kWide ? (int)(un & 1) : 0;
         const bool live = has && (row_ops[rn * MRL_ROW_OPS + MRL_OP_MASK] != 0.f);
         const T* nrow = logits + rn * row_stride;
-        n.row = row_ref(nrow + (hn ? half_elems : 0), live ? unit_bytes[hn] : 0u);
+        if (kEdge) {
+            const RowSpan span = row_span<DT>(nrow, vocab);
+            n.row = row_ref(nrow + span.head, live ? (uint32_t)span.n_vec * 16u : 0u);
+            n.edge_base = nrow;
+            n.edge_bytes = live ? unit_bytes[0] : 0u;
+            n.edge_off = edge_offset<DT>(span, vocab);
+        } else {
+            n.row = row_ref(nrow + (hn ? half_elems : 0), live ? unit_bytes[hn] : 0u);
+        }
         n.y = load_label(labels, labels_dtype, rn);
         n.zy_ptr = nrow + ((n.y >= 0 && n.y < (int64_t)vocab) ? n.y : 0);
         return n;
@@ -657,6 +664,10 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
     u32x4 v[NV];
     int64_t y = 0;
     uint32_t zy_bits = 0;                   // the logit at the label as loaded; converted where it is used
+    uint32_t edge_bits = 0;                 // the thread's edge entry, likewise
+    auto load_edge = [&](const Next& n) {
+        return kEdge ? E::buf_load_bits(mrl::make_rsrc(n.edge_base, n.edge_bytes), n.edge_off) : 0u;
+    };
     if (r < n_rows) {
         const Next first = plan(r);
         y = first.y;
@@ -666,11 +677,13 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
         // on every path into it
         const RowRef none = row_ref(dlogits, 0u);
         mrl::buf_atomic_add_u32(mrl::make_rsrc(dlogits, 0u), lane_offset(), 0u);
-        zero_part<0, H>(none);
-        load_part<0, H>(v, first.row);
-        zero_part<H, NV>(none);
+        zero_part<BLK, 0, H>(none);
+        load_part<BLK, 0, H>(v, first.row);
+        zero_part<BLK, H, NV>(none);
+        if (kEdge) E::buf_store(mrl::make_rsrc(dlogits, 0u), 0u, 0.f);
         mrl::buf_store_b32(0u, mrl::make_rsrc(dlogits, 0u), 0u);
-        load_part<H, NV>(v, first.row);
+        load_part<BLK, H, NV>(v, first.row);
+        edge_bits = load_edge(first);
         zy_bits = E::load_bits(first.zy_ptr);
     }
     int parity = 0;
@@ -678,8 +691,12 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
         const int64_t row = kWide ? (r >> 1) : r;
         const int half = kWide ? (int)(r & 1) : 0;
         const int my_first = half ? half_elems : 0;         // first entry of this unit within the row
-        const int n_vec = (int)(unit_bytes[half] / 16u);
-        const RowRef dst = row_ref(dlogits + row * d_stride + my_first, unit_bytes[half]);
+        RowSpan span = {0, (int)(unit_bytes[half] / 16u)};
+        if (kEdge) span = row_span<DT>(logits + row * row_stride, vocab);
+        const int n_vec = span.n_vec;
+        T* const drow = dlogits + row * d_stride + my_first;
+        const RowRef dst = row_ref(drow + span.head, kEdge ? (uint32_t)n_vec * 16u : unit_bytes[half]);
+        const uint32_t edge_off = kEdge ? edge_offset<DT>(span, vocab) : 0u;
         const float* ops = row_ops + row * MRL_ROW_OPS;
         const float m = ops[MRL_OP_MASK];
         const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
@@ -687,20 +704,21 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
         const int64_t y_here = y - my_first;
         const bool y_mine = y_ok && (!kWide || (y_here >= 0 && y_here < (int64_t)(unit_bytes[half] / sizeof(T))));
         Next nx;
-        uint32_t zy_next = 0;
+        uint32_t zy_next = 0, edge_next = 0;
 
         bool wrote = false;                 // dlogits of row r written and the next row requested
         if (m != 0.f) {
             float z_y = E::from_bits(zy_bits);
-            const Stats st = thread_stats<DT, NV, kEntropy>(v, n_vec, k, !y_ok);
-            Stats tot = block_reduce_1024<kEntropy>(st, k, lds);
+            const float z_edge = kEdge ? E::from_bits(edge_bits) : 0.f;
+            const Stats st = thread_stats<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k, !y_ok, edge_off != 0x80000000u, z_edge);
+            Stats tot = reduce_workgroup<BLK, kEntropy>(st, k, lds);
             if (kWide) {
                 // the logit at the label as this unit loaded it counts only if the label lies in this
                 // half: the other half may already hold gradients when dlogits overwrite the logits
                 const int other_first = half ? 0 : half_elems;
                 const T* whole = logits + row * row_stride;
                 tot = exchange_halves<DT, kEntropy>(tot, half, half_records + row * 2, spin_limit, whole + other_first,
-                                                    (int)(unit_bytes[half ^ 1] / 16u), k, Tail<NV>::kFull != 0 && y_ok, lds, &inbox, y_mine,
+                                                    (int)(unit_bytes[half ^ 1] / 16u), k, Tail<BLK, NV, kEdge>::kFull != 0 && y_ok, lds, &inbox, y_mine,
                                                     y_ok && !y_mine, whole + (y_ok ? y : 0), z_y);
             }
             float lse;
@@ -710,13 +728,15 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
                 const RowGrad g = row_grad<kEntropy>(s, k, inv_t, lse);
                 // the ticket is asked for ahead of the stores and picked up behind the first H of
                 // them: it is older than every store, so waiting for it does not wait for them
-                const uint32_t mine = mrl::buf_atomic_add_u32(ticket, lane_offset(), 1u);
-                grad_part<DT, kEntropy, 0, H>(v, g, dst);
-                nx = plan((int64_t)broadcast_ticket(mine, &next_row[parity]) + step);
-                load_part<0, H>(v, nx.row);
-                grad_part<DT, kEntropy, H, NV>(v, g, dst);
-                store_label_grad<DT, kEntropy>(dst, g, y_mine, y_here, z_y);
-                load_part<H, NV>(v, nx.row);
+                const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset(), (uint32_t)group);
+                grad_part<DT, BLK, kEntropy, 0, H>(v, g, dst);
+                nx = plan(following(mine, parity));
+                load_part<BLK, 0, H>(v, nx.row);
+                grad_part<DT, BLK, kEntropy, H, NV>(v, g, dst);
+                if (kEdge) E::buf_store(mrl::make_rsrc(drow, unit_bytes[0]), edge_off, grad_elem<kEntropy>(g, z_edge));
+                store_label_grad<DT, BLK, kEntropy, kEdge>(drow, unit_bytes[half], span, g, y_mine, y_here, z_y);
+                load_part<BLK, H, NV>(v, nx.row);
+                edge_next = load_edge(nx);
                 zy_next = E::load_bits(nx.zy_ptr);
                 wrote = true;
             }
@@ -724,17 +744,20 @@ __global__ __launch_bounds__(kBlock) void fused_sweep_persistent_kernel(
             write_masked_row_outputs(row, logp, entropy, row_terms);
         }
         if (!wrote) {                       // no gradient for this row: zeros, same order of operations
-            const uint32_t mine = mrl::buf_atomic_add_u32(ticket, lane_offset(), 1u);
-            zero_part<0, H>(dst);
-            nx = plan((int64_t)broadcast_ticket(mine, &next_row[parity]) + step);
-            load_part<0, H>(v, nx.row);
-            zero_part<H, NV>(dst);
+            const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset(), (uint32_t)group);
+            zero_part<BLK, 0, H>(dst);
+            nx = plan(following(mine, parity));
+            load_part<BLK, 0, H>(v, nx.row);
+            zero_part<BLK, H, NV>(dst);
+            if (kEdge) E::buf_store(mrl::make_rsrc(drow, unit_bytes[0]), edge_off, 0.f);
             mrl::buf_store_b32(0u, mrl::make_rsrc(dlogits, 0u), 0u);
-            load_part<H, NV>(v, nx.row);
+            load_part<BLK, H, NV>(v, nx.row);
+            edge_next = load_edge(nx);
             zy_next = E::load_bits(nx.zy_ptr);
         }
         y = nx.y;
         zy_bits = zy_next;
+        edge_bits = edge_next;
         r = nx.r;
         parity ^= 1;
     }
@@ -801,13 +824,10 @@ __global__ __launch_bounds__(kThreads) void bwd_chunk_kernel(
 // Conditional in-place rescale: multiplies every row by upstream/applied unless that ratio is 1
 // (then every workgroup exits at once; the grid is kept small so that this costs microseconds).
 template <int DT>
-__global__ __launch_bounds__(256) void scale_rows_kernel(typename Elem<DT>::T* x, int64_t row_stride, int vocab,
-                                                         int64_t n_rows, const float* __restrict__ upstream,
-                                                         const float* __restrict__ applied) {
+__device__ __forceinline__ void scale_rows(typename Elem<DT>::T* x, int64_t row_stride, int vocab, int64_t n_rows, int tail,
+                                           float ratio) {
     using E = Elem<DT>;
     constexpr int kVec = E::kVec;
-    const float ratio = *upstream / *applied;
-    if (ratio == 1.f) return;
     const int n_vec = vocab / kVec;
     for (int64_t r = blockIdx.x; r < n_rows; r += gridDim.x) {
         u32x4* vec = reinterpret_cast<u32x4*>(x + r * row_stride);
@@ -819,6 +839,21 @@ __global__ __launch_bounds__(256) void scale_rows_kernel(typename Elem<DT>::T* x
             vec[idx] = E::pack(z);
         }
     }
+    // entries behind the last row (see flat_rows)
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < tail) {
+        typename E::T* p = x + n_rows * row_stride + i;
+        E::store(p, E::load(p) * ratio);
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void scale_rows_kernel(typename Elem<DT>::T* x, int64_t row_stride, int vocab,
+                                                         int64_t n_rows, int tail, const float* __restrict__ upstream,
+                                                         const float* __restrict__ applied) {
+    const float ratio = *upstream / *applied;
+    if (ratio == 1.f) return;
+    scale_rows<DT>(x, row_stride, vocab, n_rows, tail, ratio);
 }
 
 // One backward of one buffer in a single launch: the conditional rescale above, then the book-keeping
@@ -829,10 +864,9 @@ __global__ __launch_bounds__(256) void scale_rows_kernel(typename Elem<DT>::T* x
 // it counts itself, so the last one may overwrite it).
 template <int DT>
 __global__ __launch_bounds__(256) void scale_rows_note_kernel(typename Elem<DT>::T* x, int64_t row_stride, int vocab,
-                                                              int64_t n_rows, const float* __restrict__ upstream,
-                                                              float* applied, float* learned, uint32_t* rescales) {
-    using E = Elem<DT>;
-    constexpr int kVec = E::kVec;
+                                                              int64_t n_rows, int tail,
+                                                              const float* __restrict__ upstream, float* applied,
+                                                              float* learned, uint32_t* rescales) {
     const float u = *upstream;
     const float was = applied[0];
     const float ratio = u / was;
@@ -843,17 +877,7 @@ __global__ __launch_bounds__(256) void scale_rows_note_kernel(typename Elem<DT>:
         }
         return;
     }
-    const int n_vec = vocab / kVec;
-    for (int64_t r = blockIdx.x; r < n_rows; r += gridDim.x) {
-        u32x4* vec = reinterpret_cast<u32x4*>(x + r * row_stride);
-        for (int idx = threadIdx.x; idx < n_vec; idx += 256) {
-            float z[kVec];
-            E::unpack(vec[idx], z);
-#pragma unroll
-            for (int i = 0; i < kVec; ++i) z[i] *= ratio;
-            vec[idx] = E::pack(z);
-        }
-    }
+    scale_rows<DT>(x, row_stride, vocab, n_rows, tail, ratio);
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t* done = reinterpret_cast<uint32_t*>(applied) + 1;
@@ -880,14 +904,32 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
 }
 
 // ----------------------------------------------------------------------------- host dispatch
-constexpr int kMaxVecPerThread = 19;
+// Workgroup size and vectors per thread.  A row shorter than the 1024 x 12 that the register files were
+// laid out for leaves lanes and registers of a lone workgroup idle, and nothing computes while it waits for
+// its loads; several smaller workgroups per CU overlap each other.  Upper ends by measurement (forward +
+// backward of a row, 2.5 GB of logits, GB/s; 1024 threads with the fewest vectors before):
+//   bf16:  16 KB 1 517 -> 5 467, 32 KB 2 980 -> 5 595, 48 KB 4 197 -> 5 731, 64 KB 5 144 -> 6 139,
+//          80 KB 4 417 -> 5 906, 100 KB 5 199 -> 5 879 (512 x 16; 512 x 12 where both fit within 2 %)
+//   fp32 (half the entries per byte to compute): 32 KB 3 802 -> 5 599, 48 KB 4 859 -> 6 205, 64 KB 5 832 -> 6 083;
+//          96 and 128 KB stay with 1024 x 8 (6 190 and 6 250 against 5 800 and 5 700 with 512 x 16)
+// The choice depends on the row's length alone, so a row's result does not depend on the other rows.
+enum Shape { k256x4, k256x8, k256x12, k512x12, k512x16, k1024x8, k1024x12, k1024x16, k1024x19, kTooLong };
+constexpr int64_t kMaxVec = 19 * 1024;              // vectors of the widest row that one workgroup holds
 
-inline int pick_nv(int64_t n_vec) {
-    const int64_t need = (n_vec + kBlock - 1) / kBlock;
-    const int sizes[] = {4, 8, 12, 16, 19};
-    for (int s : sizes)
-        if (need <= s) return s;
-    return 0;
+inline Shape pick_shape(int dtype, int64_t n_vec) {
+    if (n_vec <= 1024) return k256x4;
+    if (n_vec <= 2048) return k256x8;
+    if (dtype == MRL_F32) {
+        if (n_vec <= 4096) return k512x12;
+        if (n_vec <= 8192) return k1024x8;
+    } else {
+        if (n_vec <= 3072) return k256x12;
+        if (n_vec <= 6144) return k512x12;
+        if (n_vec <= 8192) return k512x16;
+    }
+    if (n_vec <= 12288) return k1024x12;
+    if (n_vec <= 16384) return k1024x16;
+    return n_vec <= kMaxVec ? k1024x19 : kTooLong;
 }
 
 // Number of CUs of the current device (one persistent workgroup each); 0 if the query fails.
@@ -904,65 +946,72 @@ constexpr uint32_t kDefaultSpinLimit = 1u << 18;
 std::atomic<uint32_t> g_wide_spin_limit{kDefaultSpinLimit};
 
 constexpr int64_t kWorkspaceHeader = 16;    // the row counter, padded to the alignment of the records
+// Unaligned rows below this go to the split kernels: a thread then holds less than half of its 4 vectors.
+constexpr int64_t kMinEdgeRowBytes = 8192;
 
-// Rows that go to the persistent workgroups; fewer get one workgroup each.
-inline bool wants_persistent(int64_t n_rows, int cus) { return cus > 0 && n_rows > 2 * (int64_t)cus; }
-
-template <int DT, int NV>
-int launch_fused(const mrl::FusedArgs& a) {
+template <int DT, int BLK, int NV, bool kEntropy, bool kWide, bool kEdge>
+int launch_sweep(const mrl::FusedArgs& a) {
     using T = typename Elem<DT>::T;
-    const dim3 block(kBlock);
     const Params p = {a.clip_lo, a.clip_hi, a.kl_coef, a.entropy_coeff, 1.f, a.kl_penalty, 0};
     unsigned int* counter = reinterpret_cast<unsigned int*>(a.workspace);
-    const int cus = cu_count();
-    const bool persistent = a.wide || (counter != nullptr && wants_persistent(a.n_rows, cus));
-    if (persistent) {
+    const int64_t units = kWide ? 2 * a.n_rows : a.n_rows;
+    int64_t grid = units;
+    int group = 1;
+    if (counter != nullptr) {
+        const int cus = cu_count();
         if (cus < 2) return mrl::fail(MRL_ERR_LAUNCH, "mrl_fused_logprob_loss: cannot query the device");
         // half rows: an even number of workgroups, so that the halves of a row start side by side
-        const int64_t units = a.wide ? 2 * a.n_rows : a.n_rows;
-        const int64_t want = a.wide ? (cus & ~1) : cus;
-        const dim3 pgrid((unsigned)(want < units ? want : units));
-        HalfRecord* rec = reinterpret_cast<HalfRecord*>(reinterpret_cast<char*>(a.workspace) + kWorkspaceHeader);
+        const int64_t cap = kWide ? (cus & ~1) : (int64_t)cus * (waves_per_simd(NV) * 4 / (BLK / 64));
+        // Rows per ticket: the counter serves about 85 tickets per microsecond, rows below 32 KiB go faster
+        // than that (8 000 bf16 logits, rows per ticket 1 / 2 / 4: 2 728 / 5 085 / 5 276 GB/s for 155 648 rows,
+        // 1 819 / 2 537 / 2 479 for 2 048; 16 384: 5 241 / 5 481 / 5 294; 24 576: 5 681 / 5 466 / 5 253).
+        if (BLK == 256 && NV <= 8 && a.n_rows > 512) group = NV <= 4 && a.n_rows >= 4096 ? 4 : 2;
+        grid = (units + group - 1) / group;
+        if (cap < grid) grid = cap;
         if (!a.workspace_cleared) {
-            const int64_t words = (kWorkspaceHeader + (a.wide ? a.n_rows * 2 * (int64_t)sizeof(HalfRecord) : 0)) / 8;
+            const int64_t words = (kWorkspaceHeader + (kWide ? a.n_rows * 2 * (int64_t)sizeof(HalfRecord) : 0)) / 8;
             hipLaunchKernelGGL(clear_words_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, a.stream,
                                reinterpret_cast<unsigned long long*>(a.workspace), words);
         }
-        const uint32_t spin = g_wide_spin_limit.load(std::memory_order_relaxed);
-#define MRL_FUSEDP_LAUNCH(ENT, WIDE)                                                                               \
-    hipLaunchKernelGGL((fused_sweep_persistent_kernel<DT, NV, ENT, WIDE>), pgrid, block, 0, a.stream,               \
-                       (const T*)a.logits, a.row_stride, (int)a.vocab, units, a.labels, a.labels_dtype, a.inv_t,    \
-                       a.row_ops, a.has_old, p, a.grad_scale, a.grad_scale_dev, (T*)a.dlogits, a.d_stride, a.logp,  \
-                       a.entropy, a.row_terms, counter, (int)a.half_elems, rec, spin)
-        if (a.wide && a.with_entropy) MRL_FUSEDP_LAUNCH(true, true);
-        else if (a.wide) MRL_FUSEDP_LAUNCH(false, true);
-        else if (a.with_entropy) MRL_FUSEDP_LAUNCH(true, false);
-        else MRL_FUSEDP_LAUNCH(false, false);
-#undef MRL_FUSEDP_LAUNCH
-        return mrl::check_launch("mrl_fused_logprob_loss");
     }
-    const dim3 grid((unsigned)a.n_rows);
-#define MRL_FUSED_LAUNCH(ENT)                                                                                  \
-    hipLaunchKernelGGL((fused_sweep_kernel<DT, NV, ENT>), grid, block, 0, a.stream, (const T*)a.logits,        \
-                       a.row_stride, (int)a.vocab, a.labels, a.labels_dtype, a.inv_t, a.row_ops, a.has_old, p, \
-                       a.grad_scale, a.grad_scale_dev, (T*)a.dlogits, a.d_stride, a.logp, a.entropy, a.row_terms)
-    if (a.with_entropy) MRL_FUSED_LAUNCH(true);
-    else MRL_FUSED_LAUNCH(false);
-#undef MRL_FUSED_LAUNCH
+    HalfRecord* rec = kWide ? reinterpret_cast<HalfRecord*>(reinterpret_cast<char*>(a.workspace) + kWorkspaceHeader) : nullptr;
+    hipLaunchKernelGGL((fused_sweep_persistent_kernel<DT, BLK, NV, kEntropy, kWide, kEdge>), dim3((unsigned)grid), dim3(BLK),
+                       0, a.stream, (const T*)a.logits, a.row_stride, (int)a.vocab, units, a.labels, a.labels_dtype,
+                       a.inv_t, a.row_ops, a.has_old, p, a.grad_scale, a.grad_scale_dev, (T*)a.dlogits, a.d_stride, a.logp,
+                       a.entropy, a.row_terms, counter, group, (int)a.half_elems, rec,
+                       g_wide_spin_limit.load(std::memory_order_relaxed));
     return mrl::check_launch("mrl_fused_logprob_loss");
 }
 
-#define MRL_NV_SWITCH(FUNC, DT, nv, a)      \
-    switch (nv) {                           \
-        case 4: return FUNC<DT, 4>(a);      \
-        case 8: return FUNC<DT, 8>(a);      \
-        case 12: return FUNC<DT, 12>(a);    \
-        case 16: return FUNC<DT, 16>(a);    \
-        default: return FUNC<DT, 19>(a);    \
-    }
+template <int DT, int BLK, int NV>
+int launch_narrow(const mrl::FusedArgs& a) {
+    if (a.edge)
+        return a.with_entropy ? launch_sweep<DT, BLK, NV, true, false, true>(a) : launch_sweep<DT, BLK, NV, false, false, true>(a);
+    return a.with_entropy ? launch_sweep<DT, BLK, NV, true, false, false>(a) : launch_sweep<DT, BLK, NV, false, false, false>(a);
+}
+
+template <int DT, int NV>
+int launch_1024(const mrl::FusedArgs& a) {
+    if (!a.wide) return launch_narrow<DT, kWideBlock, NV>(a);
+    return a.with_entropy ? launch_sweep<DT, kWideBlock, NV, true, true, false>(a)
+                          : launch_sweep<DT, kWideBlock, NV, false, true, false>(a);
+}
 
 template <int DT>
-int fused_by_nv(int nv, const mrl::FusedArgs& a) { MRL_NV_SWITCH(launch_fused, DT, nv, a) }
+int fused_by_shape(Shape shape, const mrl::FusedArgs& a) {
+    if (shape == k256x4) return launch_narrow<DT, 256, 4>(a);
+    if (shape == k256x8) return launch_narrow<DT, 256, 8>(a);
+    if (shape == k512x12) return launch_narrow<DT, 512, 12>(a);
+    if constexpr (DT == MRL_F32) {
+        if (shape == k1024x8) return launch_narrow<DT, 1024, 8>(a);
+    } else {
+        if (shape == k256x12) return launch_narrow<DT, 256, 12>(a);
+        if (shape == k512x16) return launch_narrow<DT, 512, 16>(a);
+    }
+    if (shape == k1024x12) return launch_1024<DT, 12>(a);
+    if (shape == k1024x16) return launch_1024<DT, 16>(a);
+    return launch_1024<DT, 19>(a);
+}
 
 }  // namespace
 
@@ -1019,18 +1068,23 @@ bool bwd_chunks_supported(int dtype, int64_t vocab, const void* in, int64_t in_s
     return true;
 }
 
-bool row_sweep_supported(int dtype, int64_t vocab, const void* in, int64_t in_stride, const void* out,
-                         int64_t out_stride, int64_t n_rows) {
-    const int eb = float_dtype_bytes(dtype);
-    if (eb == 0) return false;
-    const int64_t per_vec = 16 / eb;
-    if (vocab % per_vec != 0) return false;
-    const int64_t n_vec = vocab / per_vec;
-    // wider rows: two halves held by two workgroups (see "wide rows")
-    if (pick_nv(n_vec) == 0 && pick_nv((n_vec + 1) / 2) == 0) return false;
-    if (!aligned(in, 16) || !aligned(out, 16)) return false;
-    if (n_rows > 1 && ((in_stride * eb) % 16 != 0 || (out_stride * eb) % 16 != 0)) return false;
-    return true;
+// How rows of this shape and place are swept: as whole 16-byte vectors (also the only way for rows that two
+// workgroups hold), or line by line with edges, for which every row of dlogits must be misaligned as its row
+// of logits is.
+RowLayout row_sweep_layout(int dtype, int64_t vocab, const void* in, int64_t in_stride, const void* out,
+                           int64_t out_stride, int64_t n_rows) {
+    const int64_t eb = float_dtype_bytes(dtype);
+    if (eb == 0) return RowLayout::none;
+    const uintptr_t pi = reinterpret_cast<uintptr_t>(in), po = reinterpret_cast<uintptr_t>(out);
+    const int64_t n_vec = vocab / (16 / eb);
+    const int64_t si = n_rows > 1 ? in_stride * eb : 0, so = n_rows > 1 ? out_stride * eb : 0;
+    const bool vectors = vocab % (16 / eb) == 0 && (n_vec + 1) / 2 <= kMaxVec && pi % 16 == 0 && po % 16 == 0 &&
+                         si % 16 == 0 && so % 16 == 0;
+    if (vectors && (n_vec > kMaxVec || (pi % kEdgeAlign == 0 && si % kEdgeAlign == 0))) return RowLayout::vectors;
+    const int64_t alike = vectors ? kEdgeAlign : 16;        // taken from the vectors only if both sides gain
+    const bool edges = vocab * eb >= kMinEdgeRowBytes && n_vec <= kMaxVec && pi % eb == 0 && pi % alike == po % alike &&
+                       (si - so) % alike == 0;
+    return edges ? RowLayout::edges : (vectors ? RowLayout::vectors : RowLayout::none);
 }
 
 }  // namespace mrl
@@ -1038,15 +1092,16 @@ bool row_sweep_supported(int dtype, int64_t vocab, const void* in, int64_t in_st
 extern "C" int64_t mrl_fused_max_vocab(int logits_dtype) {
     const int eb = mrl::float_dtype_bytes(logits_dtype);
     if (eb == 0) return 0;
-    return 2 * (int64_t)kMaxVecPerThread * kBlock * (16 / eb);      // two workgroups hold a wide row
+    return 2 * kMaxVec * (16 / eb);                 // two workgroups hold a wide row
 }
 
 extern "C" int64_t mrl_fused_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t vocab) {
     const int eb = mrl::float_dtype_bytes(logits_dtype);
-    if (eb == 0 || n_rows < 0 || vocab <= 0 || vocab % (16 / eb) != 0) return 0;
+    if (eb == 0 || n_rows < 0 || vocab <= 0) return 0;
     const int64_t n_vec = vocab / (16 / eb);
-    if (pick_nv(n_vec) != 0) return kWorkspaceHeader;
-    if (pick_nv((n_vec + 1) / 2) == 0) return 0;
+    if (vocab % (16 / eb) != 0) return vocab * eb >= kMinEdgeRowBytes && n_vec <= kMaxVec ? kWorkspaceHeader : 0;
+    if (n_vec <= kMaxVec) return kWorkspaceHeader;
+    if ((n_vec + 1) / 2 > kMaxVec) return 0;
     return kWorkspaceHeader + n_rows * (int64_t)sizeof(HalfRecord) * 2;
 }
 
@@ -1080,10 +1135,12 @@ extern "C" int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int6
     MRL_REQUIRE(logits && labels && row_ops && dlogits && row_terms, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
     MRL_REQUIRE(mrl::aligned(workspace, 16) && mrl::aligned(grad_scale_dev, 4), MRL_ERR_MISALIGNED,
                 "%s: workspace must be 16-byte and grad_scale_dev 4-byte aligned", fn);
-    MRL_REQUIRE(mrl::row_sweep_supported(logits_dtype, vocab, logits, row_stride, dlogits, dlogits_row_stride, n_rows),
-                MRL_ERR_UNSUPPORTED,
-                "%s: needs 16-byte aligned rows, vocab %% %d == 0 and vocab <= %lld for this dtype (got vocab=%lld)", fn,
-                16 / eb, (long long)mrl_fused_max_vocab(logits_dtype), (long long)vocab);
+    const mrl::RowLayout layout =
+        mrl::row_sweep_layout(logits_dtype, vocab, logits, row_stride, dlogits, dlogits_row_stride, n_rows);
+    MRL_REQUIRE(layout != mrl::RowLayout::none, MRL_ERR_UNSUPPORTED,
+                "%s: needs 16-byte aligned rows, vocab %% %d == 0 and vocab <= %lld for this dtype, or rows of 8 KiB to "
+                "half that vocab whose dlogits are misaligned alike (got vocab=%lld)", fn, 16 / eb,
+                (long long)mrl_fused_max_vocab(logits_dtype), (long long)vocab);
     if (dlogits != logits) {
         const char* x = (const char*)logits;
         const char* y = (const char*)dlogits;
@@ -1101,12 +1158,13 @@ extern "C" int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int6
     a.logp = logp; a.entropy = entropy; a.row_terms = row_terms; a.with_entropy = (entropy != nullptr);
     a.stream = mrl::as_stream(stream);
     const int64_t n_vec = vocab / (16 / eb);
-    int nv = pick_nv(n_vec);
-    a.wide = (nv == 0);
+    a.edge = layout == mrl::RowLayout::edges;
+    Shape shape = pick_shape(logits_dtype, n_vec);
+    a.wide = shape == kTooLong;
     a.half_elems = 0;
     if (a.wide) {
         a.half_elems = (n_vec + 1) / 2 * (16 / eb);
-        nv = pick_nv((n_vec + 1) / 2);
+        shape = pick_shape(logits_dtype, (n_vec + 1) / 2);
     }
     if (workspace != nullptr || a.wide) {
         const int64_t need = a.wide ? mrl_fused_workspace_bytes(logits_dtype, n_rows, vocab) : kWorkspaceHeader;
@@ -1115,10 +1173,20 @@ extern "C" int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int6
                     "their statistics through it)", fn, (long long)(workspace ? workspace_bytes : 0), (long long)need);
     }
     switch (logits_dtype) {
-        case MRL_F32: return fused_by_nv<MRL_F32>(nv, a);
-        case MRL_BF16: return fused_by_nv<MRL_BF16>(nv, a);
-        default: return fused_by_nv<MRL_F16>(nv, a);
+        case MRL_F32: return fused_by_shape<MRL_F32>(shape, a);
+        case MRL_BF16: return fused_by_shape<MRL_BF16>(shape, a);
+        default: return fused_by_shape<MRL_F16>(shape, a);
     }
+}
+
+// Dense rows of an odd vocabulary are one stretch of entries: cut into rows of 2048 (fewer when there are
+// fewer) and a tail of less than that, which is returned.  Other rows stay as they are.
+static int flat_rows(int eb, int64_t& n_rows, int64_t& vocab, int64_t& row_stride) {
+    if (vocab % (16 / eb) == 0 || row_stride != vocab) return 0;
+    const int64_t total = n_rows * vocab;
+    vocab = row_stride = 2048;
+    n_rows = total / vocab;
+    return (int)(total % vocab);
 }
 
 extern "C" int mrl_scale_rows(void* x, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,
@@ -1133,22 +1201,23 @@ extern "C" int mrl_scale_rows(void* x, int dtype, int64_t n_rows, int64_t vocab,
     MRL_REQUIRE(x && upstream && applied, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
     MRL_REQUIRE(mrl::aligned(upstream, 4) && mrl::aligned(applied, 4), MRL_ERR_MISALIGNED,
                 "%s: upstream and applied must be 4-byte aligned", fn);
+    const int tail = flat_rows(eb, n_rows, vocab, row_stride);
     MRL_REQUIRE(vocab % (16 / eb) == 0 && mrl::aligned(x, 16) && (n_rows == 1 || (row_stride * eb) % 16 == 0),
-                MRL_ERR_UNSUPPORTED, "%s: needs 16-byte aligned rows", fn);
+                MRL_ERR_UNSUPPORTED, "%s: needs 16-byte aligned or dense rows", fn);
     hipStream_t s = mrl::as_stream(stream);
-    const dim3 grid((unsigned)(n_rows < 4096 ? n_rows : 4096)), block(256);
+    const dim3 grid((unsigned)(n_rows < 8 ? 8 : (n_rows < 4096 ? n_rows : 4096))), block(256);
     switch (dtype) {
         case MRL_F32:
             hipLaunchKernelGGL(scale_rows_kernel<MRL_F32>, grid, block, 0, s, (float*)x, row_stride, (int)vocab,
-                               n_rows, upstream, applied);
+                               n_rows, tail, upstream, applied);
             break;
         case MRL_BF16:
             hipLaunchKernelGGL(scale_rows_kernel<MRL_BF16>, grid, block, 0, s, (uint16_t*)x, row_stride, (int)vocab,
-                               n_rows, upstream, applied);
+                               n_rows, tail, upstream, applied);
             break;
         default:
             hipLaunchKernelGGL(scale_rows_kernel<MRL_F16>, grid, block, 0, s, (uint16_t*)x, row_stride, (int)vocab,
-                               n_rows, upstream, applied);
+                               n_rows, tail, upstream, applied);
             break;
     }
     return mrl::check_launch(fn);
@@ -1179,22 +1248,23 @@ extern "C" int mrl_scale_rows_note(void* x, int dtype, int64_t n_rows, int64_t v
     MRL_REQUIRE(mrl::aligned(upstream, 4) && mrl::aligned(applied, 8) && mrl::aligned(learned, 4) &&
                     mrl::aligned(rescales, 4),
                 MRL_ERR_MISALIGNED, "%s: applied must be 8-byte, the other scalars 4-byte aligned", fn);
+    const int tail = flat_rows(eb, n_rows, vocab, row_stride);
     MRL_REQUIRE(vocab % (16 / eb) == 0 && mrl::aligned(x, 16) && (n_rows == 1 || (row_stride * eb) % 16 == 0),
-                MRL_ERR_UNSUPPORTED, "%s: needs 16-byte aligned rows", fn);
+                MRL_ERR_UNSUPPORTED, "%s: needs 16-byte aligned or dense rows", fn);
     hipStream_t s = mrl::as_stream(stream);
-    const dim3 grid((unsigned)(n_rows < 2048 ? n_rows : 2048)), block(256);
+    const dim3 grid((unsigned)(n_rows < 8 ? 8 : (n_rows < 2048 ? n_rows : 2048))), block(256);
     switch (dtype) {
         case MRL_F32:
             hipLaunchKernelGGL(scale_rows_note_kernel<MRL_F32>, grid, block, 0, s, (float*)x, row_stride, (int)vocab,
-                               n_rows, upstream, applied, learned, rescales);
+                               n_rows, tail, upstream, applied, learned, rescales);
             break;
         case MRL_BF16:
             hipLaunchKernelGGL(scale_rows_note_kernel<MRL_BF16>, grid, block, 0, s, (uint16_t*)x, row_stride,
-                               (int)vocab, n_rows, upstream, applied, learned, rescales);
+                               (int)vocab, n_rows, tail, upstream, applied, learned, rescales);
             break;
         default:
             hipLaunchKernelGGL(scale_rows_note_kernel<MRL_F16>, grid, block, 0, s, (uint16_t*)x, row_stride,
-                               (int)vocab, n_rows, upstream, applied, learned, rescales);
+                               (int)vocab, n_rows, tail, upstream, applied, learned, rescales);
             break;
     }
     return mrl::check_launch(fn);

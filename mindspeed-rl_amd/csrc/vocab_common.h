@@ -41,6 +41,9 @@ struct Elem<MRL_F32> {
     static __device__ __forceinline__ void buf_store(mrl::rsrc_t r, uint32_t byte_off, float v) {
         mrl::buf_store_b32(__float_as_uint(v), r, byte_off);
     }
+    static __device__ __forceinline__ uint32_t buf_load_bits(mrl::rsrc_t r, uint32_t byte_off) {
+        return mrl::buf_load_b32(r, byte_off);
+    }
 };
 
 template <>
@@ -73,6 +76,9 @@ struct Elem<MRL_BF16> {
     static __device__ __forceinline__ void buf_store(mrl::rsrc_t r, uint32_t byte_off, float v) {
         __bf16 h = (__bf16)v;
         mrl::buf_store_b16(__builtin_bit_cast(uint16_t, h), r, byte_off);
+    }
+    static __device__ __forceinline__ uint32_t buf_load_bits(mrl::rsrc_t r, uint32_t byte_off) {
+        return mrl::buf_load_b16(r, byte_off);
     }
 };
 
@@ -111,6 +117,9 @@ struct Elem<MRL_F16> {
     static __device__ __forceinline__ void buf_store(mrl::rsrc_t r, uint32_t byte_off, float v) {
         _Float16 h = (_Float16)v;
         mrl::buf_store_b16(__builtin_bit_cast(uint16_t, h), r, byte_off);
+    }
+    static __device__ __forceinline__ uint32_t buf_load_bits(mrl::rsrc_t r, uint32_t byte_off) {
+        return mrl::buf_load_b16(r, byte_off);
     }
 };
 

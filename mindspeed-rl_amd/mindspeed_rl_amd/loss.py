@@ -143,16 +143,13 @@ def policy_loss(log_prob, entropy, old_log_prob, ref_log_prob, advantages, mask=
 
 # ------------------------------------------------------------------------------------ fused sweep
 def fused_supported(output, grad_inplace=False):
-    """True if the row-in-registers kernel can take these logits: a floating dtype it knows,
-    16-byte aligned dense rows and a vocabulary that fits the register files of one workgroup
-    or of two.  (``grad_inplace`` is accepted for call compatibility: every supported shape can
+    """True if the row-in-registers kernel can take these logits: a floating dtype it knows, a
+    16-byte aligned dense tensor and a vocabulary that fits the register files of one workgroup or - if
+    it is a whole number of 16-byte vectors - of two (other vocabularies from 8 KiB a row on).  (``grad_inplace`` is accepted for call compatibility: every supported shape can
     also be swept in place.)"""
     if output.dtype not in (torch.float32, torch.bfloat16, torch.float16) or not output.is_cuda:
         return False
-    vocab = output.shape[-1]
-    per_vec = 16 // output.element_size()
-    limit = _lib.load().mrl_fused_max_vocab(_lib.dtype_code(output))
-    if vocab % per_vec != 0 or vocab > limit:
+    if _lib.load().mrl_fused_workspace_bytes(_lib.dtype_code(output), 1, output.shape[-1]) == 0:
         return False
     return output.is_contiguous() and output.data_ptr() % 16 == 0
 

@@ -1166,6 +1166,61 @@ def test_fused_sweep_vocab_sizes(dev, dtype, vocab):
         assert got2.item() == got.item() and torch.equal(dz2, dz), limit
 
 
+@pytest.mark.parametrize("dtype,vocab", [
+    (torch.bfloat16, 4097), (torch.float16, 1024 * 8 + 7), (torch.bfloat16, 1025 * 8 + 1), (torch.bfloat16, 2056 * 8),
+    (torch.bfloat16, 2049 * 8 + 3), (torch.float16, 3073 * 8 + 5), (torch.bfloat16, 6144 * 8 + 7), (torch.bfloat16, 6145 * 8),
+    (torch.bfloat16, 8193 * 8 + 1), (torch.bfloat16, 12289 * 8 + 1), (torch.bfloat16, 16385 * 8 + 1),
+    (torch.bfloat16, 19456 * 8 + 7), (torch.float32, 2049), (torch.float32, 2049 * 4 + 1), (torch.float32, 4097 * 4 + 1),
+    (torch.float32, 8193 * 4 + 2), (torch.float32, 19456 * 4 + 3)])
+def test_fused_sweep_rows_off_a_line(dev, dtype, vocab):
+    """Rows that start anywhere: the shortest and the longest row of every shape of the sweep's workgroups (a
+    row's vectors begin at its first 128-byte line, so it has up to 8 fewer than its length suggests), labels
+    in the entries in front of and behind the vectors, a row whose last entry is far above all others,
+    gradients in place, and a backward whose scale the sweep did not know (the rows are rescaled as one
+    stretch)."""
+    gen = torch.Generator().manual_seed(vocab)
+    logits, b, kw, _, _ = _make_batch(gen, 1, 4, 5, 9, vocab, dtype, 3.0, 1, prompt_hi=2)
+    b["labels"][0, :12] = torch.tensor([0, vocab - 1, vocab - 2, 1, 7, vocab // 2, vocab - 3, 31, 63, 64, vocab - 8, 2])
+    logits[0, 3, vocab - 1] = 200.0         # overflows sums taken against the thread's first vector
+    logits[0, 4, 0] = 200.0
+    meta = dict(clip_ratio=0.2, kl_coef=0.02, kl_penalty="low_var_kl", entropy_coeff=0.002)
+    zo = logits.float().requires_grad_()
+    want, want_stats = o_loss.grpo_compute_loss(zo, b, meta, **kw)
+    (dz_o,) = torch.autograd.grad(want, zo)
+    f = mrl.LossFuncFactory.get_instance("ray_grpo", "actor")
+    f.add_loss_meta_info({"clip_ratio": 0.2, "kl_ctrl": mrl.FixedKLController(0.02), "kl_penalty": "low_var_kl",
+                          "entropy_coeff": 0.002})
+    zd = logits.to(dev).requires_grad_()
+    assert mrl.fused_supported(zd)
+    got, got_stats = f.compute_loss(zd, _to_dev(b, dev), **_to_dev(kw, dev))
+    (dz,) = torch.autograd.grad(got, zd)
+    assert abs(got.item() - want.item()) <= TOL_LOSS_REL * abs(want.item()) + 1e-7
+    for k in want_stats:
+        assert abs(got_stats[k] - want_stats[k]) <= TOL_LOSS_REL * abs(want_stats[k]) + 1e-6, k
+    assert (dz.float().cpu() - dz_o).abs().max().item() <= 2 ** -8 * dz_o.abs().max().item() + 1e-9
+    (dz_4,) = torch.autograd.grad(f.compute_loss(zd, _to_dev(b, dev), expected_grad_scale=1.0, **_to_dev(kw, dev))[0] / 4.0, zd)
+    if dtype == torch.float16:              # a quarter of a subnormal is rounded again
+        assert (dz_4.float() * 4.0 - dz.float()).abs().max().item() <= 2 ** -22
+    else:
+        assert torch.equal(dz_4.float() * 4.0, dz.float())
+    z2 = logits.to(dev).requires_grad_()
+    got2, _ = f.compute_loss(z2 * 1.0, _to_dev(b, dev), grad_inplace=True, expected_grad_scale=1.0, **_to_dev(kw, dev))
+    (dz2,) = torch.autograd.grad(got2, z2)
+    assert got2.item() == got.item() and torch.equal(dz2, dz)
+
+
+@pytest.mark.parametrize("rows,vocab", [(513, 4096), (4098, 4097), (2050, 8200), (1021, 16392), (1300, 32003), (600, 49153)])
+def test_fused_sweep_rows_per_ticket(dev, rows, vocab):
+    """Workgroups that take one, two or four rows with a ticket, more rows than fit on the chip at once: every
+    row comes out as a workgroup of its own delivers it, bit for bit."""
+    z, y, ops = _raw_fused_case(dev, rows, rows, vocab)
+    outs = [(torch.full_like(z, 7.0), torch.empty(rows, device=dev), torch.empty(rows, 8, device=dev)) for _ in range(2)]
+    _raw_fused_sweep(z, y, ops, *outs[0], _lib.stream(dev), torch.empty(4, dtype=torch.int32, device=dev))
+    _raw_fused_sweep(z, y, ops, *outs[1], _lib.stream(dev), None)
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,vocab", [(torch.float32, 152064), (torch.bfloat16, 262144)])
 def test_fused_sweep_wide_rows(dev, dtype, vocab):
     """Rows that two workgroups hold: more half rows than workgroups (tickets are recycled, partners
