@@ -416,7 +416,7 @@ def run_lmhead_train(args, steps=None, warmup=None):
     gemm_events, lmhead.kernel_events = lmhead.kernel_events, None
     sweep_ms = sum(s.elapsed_time(e) for (_, s, e, _) in events) / steps
     logits_ms = sum(s.elapsed_time(e) for (n, s, e, _) in gemm_events if n == "mrl_lmhead_logits") / steps
-    bwd_ms = sum(s.elapsed_time(e) for (n, s, e, _) in gemm_events if n == "mrl_lmhead_logprob_bwd") / steps
+    bwd_ms = sum(s.elapsed_time(e) for (n, s, e, _) in gemm_events if n.startswith("mrl_lmhead_logprob_bwd")) / steps
     ms = elapsed * 1e3 / steps
     flops = 6.0 * total * vocab * hdim                       # forward GEMM + dHidden GEMM + dW GEMM
     tflops = flops / (ms * 1e-3) / 1e12

@@ -446,6 +446,21 @@ int mrl_lmhead_logprob_bwd(const void* hidden, const void* weight, const void* d
                            int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab,
                            int64_t hidden_dim, void* d_hidden, float* d_weight, void* stream);
 
+/* The same two products for one chunk of a step whose dWeight ends as bf16 [vocab, hidden_dim]: the first
+ * chunk overwrites d_weight_sums (fp32, need not be cleared), the chunks between add to it, the last adds
+ * to it and writes the sum to d_weight; a chunk that is both first and last writes d_weight at once
+ * (d_weight_sums may be NULL).  Every entry is rounded once, as by mrl_lmhead_logprob_bwd and a conversion.
+ * workspace (nullable): mrl_lmhead_bwd_workspace_bytes(n_tokens, vocab, hidden_dim) bytes, 16-byte aligned,
+ * for dHidden tiles that are cut along the vocabulary when they do not fill the chip (0 bytes where they
+ * do); with NULL or fewer bytes none is cut.  dHidden is the same to rounding either way (the fp32 sums
+ * group differently), and bit for bit independent of the chunking when none is.  n_tokens > 0. */
+int64_t mrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t hidden_dim);
+int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weight, const void* dlogits,
+                                 int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab,
+                                 int64_t hidden_dim, void* d_hidden, void* d_weight,
+                                 float* d_weight_sums, int first, int last, void* workspace,
+                                 int64_t workspace_bytes, void* stream);
+
 /* mrl_lmhead_logprob_fwd for callers that cannot allocate device memory or pass a workspace (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in
  * the reference.  Same arguments, kernels and results as mrl_lmhead_logprob_fwd, but the partial

@@ -71,7 +71,7 @@ struct UnitInfo {
     int start;                                  // flattened number of the unit's first tile
     int tm, tn;                                 // its first vocabulary tile, its token tile
 };
-struct UnitTiles {
+struct UnitTiles : mrl_tile::WholeK {
     const UnitInfo* units;                      // LDS, n_units + 1 entries (the last: start = n_tiles)
     int n_tiles;
     __device__ __forceinline__ void coords(int j, int& tm, int& tn) const {
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wv = wave >> 1, wt = wave & 1;
     const VocabLeaves leaves(vocab);
-    UnitTiles seq = {units, 0};
+    UnitTiles seq = {{}, units, 0};
     {
         const int n_ttiles = (n_tokens + BN - 1) / BN;
         int r = 0;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     };
 
     // online softmax statistics of a tile: per token block a lane holds 8 x 4 vocabulary rows
-    auto tile_stats = [&](Accumulators& acc, int tm, int tn) {
+    auto tile_stats = [&](Accumulators& acc, int, int tm, int tn) {
         const int v0 = tm * BM + wv * 128 + 4 * (lane >> 4);       // + 16 vb + r
         const bool ragged = (tm * BM + BM > vocab);
 #pragma unroll

@@ -18,9 +18,15 @@
 // that share an XCD (and its L2) take 32 consecutive numbers at a time: the 4 that stream the same A
 // tile and the 8 that stream the same B tile run side by side (see tile_coords for the order of the
 // groups of 32).
-#include <stdlib.h>
+//
+// dHidden has few tiles and a long K (the vocabulary): 162 tokens x 2 944 is 12 tiles on 256 CUs, 4 000 x 5 120
+// is 1.25 rounds of the chip.  Tiles behind the last whole round may therefore be cut along K into slices
+// (plan_split); a slice leaves its fp32 sums in the caller's workspace and merge_slices_kernel adds them in
+// the order of the slices.  Units are numbered slice by slice, so the workgroups of an XCD still share operand
+// tiles.  Both backward products, uncut and cut: 162 x 95 920 x 2 944 2 193 -> 416 us, 300 x 32 000 x 1 024
+// 588 -> 115, 1 380 x 152 064 x 3 584 4 695 -> 2 969, 4 000 x 129 280 x 5 120 10 936 -> 8 629.
+#include <type_traits>
 
-#include "lmhead_gemm.h"
 #include "lmhead_tile.h"
 #include "mrl_internal.h"
 #include "vocab_common.h"
@@ -58,39 +64,101 @@ __device__ __forceinline__ void tile_coords(const TileGrid& g, int64_t t, int& t
     tn = ng * kTilesAlongN + rem % width;
 }
 
+__host__ __device__ inline TileGrid make_grid(int64_t M, int64_t N) {
+    TileGrid g;
+    g.tiles_m = (int)((M + BM - 1) / BM);
+    g.tiles_n = (int)((N + BN - 1) / BN);
+    g.total = (int64_t)g.tiles_m * g.tiles_n;
+    // panels of up to 8 rows of tiles (8 x 4 blocks per XCD), tall products up to 32; all panels the same
+    // height (14 rows of tiles as 7 + 7 measured 1.7 % faster than as 8 + 6)
+    const int panel_cap = g.tiles_m >= 64 ? 32 : 8;
+    const int n_panels = (g.tiles_m + panel_cap - 1) / panel_cap;
+    g.panel_m = (g.tiles_m + n_panels - 1) / n_panels;
+    return g;
+}
+
+// Tiles from number `whole` on are cut into n_slices along K (n_slices 1: none is).
+struct SplitPlan {
+    int64_t whole;
+    int rest, n_slices;
+};
+
+constexpr int64_t kTileElems = (int64_t)BM * BN;
+constexpr int64_t kMaxSlices = 1024;                // of all tiles together: 256 MiB of fp32 sums
+
+// The number of slices with the least expected time, in k-steps (about 1.5 microseconds each): the rounds that
+// the units take, and per unit of a round about 10 for turning out the sums and 0.1 for each slice's trip
+// through memory to the merge.  A partly filled round of whole tiles is cheaper than a full one, since the
+// board's power goes to fewer CUs: 174 of 256 CUs (12 356 x 152 064 x 3 584) measured 21 486 us uncut against
+// 21 846 in four slices, 120 of 256 (20 000 x 60 000 x 2 048) 8 251 against 7 855 in two.
+inline SplitPlan plan_split(int64_t total, int grid, int64_t n_ksteps) {
+    SplitPlan p = {total / grid * grid, (int)(total % grid), 1};
+    if (p.rest == 0) return p;
+    double best = (double)n_ksteps * (0.35 + 0.65 * (double)p.rest / grid);
+    for (int64_t s = 2; s * p.rest <= kMaxSlices && s * 4 <= n_ksteps; ++s) {
+        const int64_t rounds = (s * p.rest + grid - 1) / grid;
+        const double cost = (double)rounds * ((double)((n_ksteps + s - 1) / s) + 10.0) + 0.1 * (double)(s * p.rest) + 10.0;
+        if (cost < best) {
+            best = cost;
+            p.n_slices = (int)s;
+        }
+    }
+    if (p.n_slices == 1) p.whole = total, p.rest = 0;
+    return p;
+}
+
 // The tiles of one workgroup: number first + j * stride.
-struct StridedTiles {
+struct StridedTiles : WholeK {
     TileGrid grid;
     int64_t first, stride;
     int n_tiles;
     __device__ __forceinline__ void coords(int j, int& tm, int& tn) const { tile_coords(grid, first + j * stride, tm, tn); }
 };
 
-// kAccumulate: out is fp32 and the product is added to it; else out is bf16 and overwritten.
-// kATrans / kBTrans: the operand is k-major, [K, M] or [K, N]; else [M, K] or [N, K].
-template <bool kAccumulate, bool kATrans, bool kBTrans>
+// The slices of one workgroup: unit u = first + j * stride is slice u / rest of tile whole + u % rest.
+struct SlicedTiles {
+    TileGrid grid;
+    int64_t first, stride;
+    int n_tiles;
+    SplitPlan plan;
+    __device__ __forceinline__ void coords(int j, int& tm, int& tn) const {
+        tile_coords(grid, plan.whole + (first + j * stride) % plan.rest, tm, tn);
+    }
+    __device__ __forceinline__ void k_range(int j, int n_ksteps, int& begin, int& end) const {
+        const int64_t s = (first + j * stride) / plan.rest;
+        begin = (int)(s * n_ksteps / plan.n_slices);
+        end = (int)((s + 1) * n_ksteps / plan.n_slices);
+    }
+};
+
+// What becomes of a finished tile: stored as bf16, stored as fp32, added to the fp32 there, or added to the
+// fp32 at `acc` and the sum stored as bf16.
+enum Out { kBf16, kF32, kF32Add, kSumToBf16 };
+
+// kATrans / kBTrans: the operand is k-major, [K, M] or [K, N]; else [M, K] or [N, K].  sums: fp32 [N, M] with
+// the leading dimension of out (kSumToBf16), or with kSliced (kOut kF32) what the slices' tiles go to; the
+// plan says which tiles are whole and how the rest are cut, and a launch does the one or the other (both in
+// one kernel need two epilogues and spill).
+template <int kOut, bool kATrans, bool kBTrans, bool kSliced>
 __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __restrict__ A, int64_t lda, int M,
                                                            const uint16_t* __restrict__ B, int64_t ldb, int N, int K,
-                                                           void* __restrict__ out, int64_t ldo) {
+                                                           void* __restrict__ out, int64_t ldo, float* __restrict__ sums,
+                                                           SplitPlan plan) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wv = wave / kWavesN, wt = wave % kWavesN;
 
-    StridedTiles seq;
-    seq.grid.tiles_m = (M + BM - 1) / BM;
-    seq.grid.tiles_n = (N + BN - 1) / BN;
-    seq.grid.total = (int64_t)seq.grid.tiles_m * seq.grid.tiles_n;
-    // panels of up to 8 rows of tiles (8 x 4 blocks per XCD), tall products up to 32; all panels the same
-    // height (14 rows of tiles as 7 + 7 measured 1.7 % faster than as 8 + 6)
-    const int panel_cap = seq.grid.tiles_m >= 64 ? 32 : 8;
-    const int n_panels = (seq.grid.tiles_m + panel_cap - 1) / panel_cap;
-    seq.grid.panel_m = (seq.grid.tiles_m + n_panels - 1) / n_panels;
+    static_assert(!kSliced || kOut == kF32, "a slice leaves fp32 sums");
+    std::conditional_t<kSliced, SlicedTiles, StridedTiles> seq;
+    seq.grid = make_grid(M, N);
+    const int64_t n_units = kSliced ? (int64_t)plan.rest * plan.n_slices : plan.whole;
+    if constexpr (kSliced) seq.plan = plan;
     // workgroups are dealt round-robin to the 8 XCDs: the gridDim / 8 workgroups of an XCD take
     // consecutive tile numbers
     const int per_xcd = gridDim.x >> 3;
     seq.first = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     seq.stride = gridDim.x;
-    seq.n_tiles = seq.first < seq.grid.total ? (int)((seq.grid.total - 1 - seq.first) / seq.stride) + 1 : 0;
+    seq.n_tiles = seq.first < n_units ? (int)((n_units - 1 - seq.first) / seq.stride) + 1 : 0;
 
     // The finished tile.  A lane holds column n = lane & 15 of each 16 x 16 block and rows
     // 4 (lane >> 4) .. + 3 of it: stored like that, a store instruction would touch 16 output rows with
@@ -99,16 +167,22 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
     // chunks XOR-swizzled by the row pair, written in the MFMA layout and read back as 8 lanes x 16 bytes
     // per output row, so that every store covers whole 128-byte lines.
     unsigned char* turn = smem + kLdsStages + wave * (kLdsTurn / kWaves);
-    auto store_tile = [&](mrl_tile::Accumulators& acc, int tm, int tn) {
+    auto store_tile = [&](mrl_tile::Accumulators& acc, int j, int tm, int tn) {
+        constexpr bool kWideEntries = kOut != kBf16;              // turned as fp32
+        // a slice's tile is a matrix of its own
+        const int m_tile = kSliced ? 0 : tm * BM, n_tile = kSliced ? 0 : tn * BN;
+        const int m_end = kSliced ? M - tm * BM : M, n_end = kSliced ? N - tn * BN : N;
+        const int64_t ld = kSliced ? BM : ldo;
+        float* const slice = sums + (kSliced ? (seq.first + j * seq.stride) * kTileElems : 0);
         const int row_w = lane & 15, quarter = lane >> 4;        // writer: its n, its run of 4 m inside the block
         const int row_r = lane >> 3, chunk_r = lane & 7;          // reader: n within a group of 8, 16-byte chunk
-        constexpr int kMPerPass = kAccumulate ? 2 : 4;            // 32 fp32 or 64 bf16 entries of m are 128 bytes
+        constexpr int kMPerPass = kWideEntries ? 2 : 4;            // 32 fp32 or 64 bf16 entries of m are 128 bytes
 #pragma unroll
         for (int tb0 = 0; tb0 < kBlocks; tb0 += 4) {
-            const int n0 = tn * BN + wt * 128 + tb0 * 16;
+            const int n0 = n_tile + wt * 128 + tb0 * 16;
 #pragma unroll
             for (int vb0 = 0; vb0 < kBlocks; vb0 += kMPerPass) {
-                const int m0 = tm * BM + wv * 128 + vb0 * 16;
+                const int m0 = m_tile + wv * 128 + vb0 * 16;
 #pragma unroll
                 for (int tbi = 0; tbi < 4; ++tbi) {
                     const int row = tbi * 16 + row_w;
@@ -117,7 +191,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
 #pragma unroll
                     for (int vbi = 0; vbi < kMPerPass; ++vbi) {
                         const floatx4& c = acc[vb0 + vbi][tb0 + tbi];
-                        if (kAccumulate) {
+                        if (kWideEntries) {
                             *reinterpret_cast<float4*>(line + (((vbi * 4 + quarter) ^ key) * 16)) =
                                 make_float4(c[0], c[1], c[2], c[3]);
                         } else {
@@ -136,18 +210,24 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
                     const u32x4 v =
                         *reinterpret_cast<const u32x4*>(turn + row * 128 + ((chunk_r ^ ((row >> 1) & 7)) * 16));
                     const int n = n0 + row;
-                    const int m = m0 + chunk_r * (kAccumulate ? 4 : 8);
-                    if (n < N && m < M) {                      // M % 8 == 0: a chunk is inside or outside
-                        if (kAccumulate) {
-                            float4* p = reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + (int64_t)n * ldo + m);
-                            float4 c = *p;
-                            c.x += __uint_as_float(v.x);
-                            c.y += __uint_as_float(v.y);
-                            c.z += __uint_as_float(v.z);
-                            c.w += __uint_as_float(v.w);
-                            *p = c;
+                    const int m = m0 + chunk_r * (kWideEntries ? 4 : 8);
+                    if (n < n_end && m < m_end) {              // M % 8 == 0: a chunk is inside or outside
+                        const int64_t at = (int64_t)n * ld + m;
+                        if constexpr (kOut == kBf16) {
+                            *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(out) + at) = v;
                         } else {
-                            *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(out) + (int64_t)n * ldo + m) = v;
+                            float* const dst = kSliced ? slice : reinterpret_cast<float*>(out);
+                            float4 c = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
+                                                   __uint_as_float(v.w));
+                            if constexpr (kOut != kF32) {
+                                const float4 o = *reinterpret_cast<const float4*>((kOut == kF32Add ? dst : sums) + at);
+                                c = make_float4(o.x + c.x, o.y + c.y, o.z + c.z, o.w + c.w);
+                            }
+                            if constexpr (kOut == kSumToBf16)
+                                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + at) =
+                                    make_uint2(Elem<MRL_BF16>::pack2(c.x, c.y), Elem<MRL_BF16>::pack2(c.z, c.w));
+                            else
+                                *reinterpret_cast<float4*>(dst + at) = c;
                         }
                     }
                 }
@@ -161,6 +241,30 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
     mfma_tile_loop<kATrans, kBTrans, 0>(smem, A, lda, M, B, ldb, N, K, seq, store_tile);
 }
 
+// out[n][m] = sum over the slices, in their order, of the tiles that SlicedTiles cut.  Grid: (tile, 16 rows of
+// it); a wavefront per row of 256 entries, 16 bytes per lane and slice: a read of memory, 4 to 5 TB/s.
+__global__ __launch_bounds__(256) void merge_slices_kernel(const float* __restrict__ sums, SplitPlan plan, int M, int N,
+                                                           uint16_t* __restrict__ out, int64_t ldo) {
+    const TileGrid grid = make_grid(M, N);
+    int tm, tn;
+    tile_coords(grid, plan.whole + blockIdx.x, tm, tn);
+    const int m = (threadIdx.x & 63) * 4;
+    if (tm * BM + m >= M) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = (int)blockIdx.y * 16 + i * 4 + (int)(threadIdx.x >> 6);
+        if (tn * BN + n >= N) return;
+        const float* p = sums + (int64_t)blockIdx.x * kTileElems + n * BM + m;
+        float4 c = *reinterpret_cast<const float4*>(p);
+        for (int s = 1; s < plan.n_slices; ++s) {
+            const float4 o = *reinterpret_cast<const float4*>(p + (int64_t)s * plan.rest * kTileElems);
+            c = make_float4(c.x + o.x, c.y + o.y, c.z + o.z, c.w + o.w);
+        }
+        *reinterpret_cast<uint2*>(out + (int64_t)(tn * BN + n) * ldo + tm * BM + m) =
+            make_uint2(Elem<MRL_BF16>::pack2(c.x, c.y), Elem<MRL_BF16>::pack2(c.z, c.w));
+    }
+}
+
 int persistent_grid() {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
@@ -172,48 +276,97 @@ int persistent_grid() {
 
 namespace mrl {
 
-template <bool kAccumulate, bool kATrans, bool kBTrans>
-static int launch_gemm(const char* fn, int grid, const void* a, int64_t lda, int64_t m, const void* b, int64_t ldb, int64_t n,
-                       int64_t k, void* out, int64_t ldo, hipStream_t stream) {
-    // function attributes belong to a device: reserved with every launch, on whichever device is current
-    const hipError_t attr = hipFuncSetAttribute((const void*)gemm_kernel<kAccumulate, kATrans, kBTrans>,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    MRL_REQUIRE(attr == hipSuccess, MRL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", fn, kLdsBytes);
-    hipLaunchKernelGGL((gemm_kernel<kAccumulate, kATrans, kBTrans>), dim3((unsigned)grid), dim3(kThreads), kLdsBytes, stream,
-                       (const uint16_t*)a, lda, (int)m, (const uint16_t*)b, ldb, (int)n, (int)k, out, ldo);
-    return check_launch(fn);
-}
+struct Product {
+    const void* a; int64_t lda, m;
+    const void* b; int64_t ldb, n;
+    int64_t k;
+    void* out; int64_t ldo;
+    float* sums;
+    hipStream_t stream;
+};
 
-int gemm_bf16(const char* fn, const void* a, int64_t lda, int64_t m, bool a_kmajor, const void* b, int64_t ldb, int64_t n,
-              bool b_kmajor, int64_t k, void* out, int64_t ldo, bool accumulate_f32, hipStream_t stream) {
-    MRL_REQUIRE(m > 0 && n > 0 && k > 0 && m % 8 == 0, MRL_ERR_UNSUPPORTED, "%s: product of m=%lld n=%lld k=%lld (m must be a multiple of 8)",
-                fn, (long long)m, (long long)n, (long long)k);
-    MRL_REQUIRE(m <= 0x7fffffffLL && n <= 0x7fffffffLL && k <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED, "%s: size out of range",
-                fn);
-    const int64_t k_steps = (k + BK - 1) / BK * BK;        // what a k-contiguous operand is read up to
-    MRL_REQUIRE((a_kmajor || b_kmajor) || k % BK == 0, MRL_ERR_UNSUPPORTED,
-                "%s: k=%lld must be a multiple of %d when no operand is k-major", fn, (long long)k, BK);
-    MRL_REQUIRE(!b_kmajor || n % 8 == 0, MRL_ERR_UNSUPPORTED, "%s: n=%lld must be a multiple of 8 for a k-major b", fn,
-                (long long)n);
-    MRL_REQUIRE(lda >= (a_kmajor ? m : k_steps) && ldb >= (b_kmajor ? n : k_steps) && ldo >= m && lda % 8 == 0 &&
-                    ldb % 8 == 0 && ldo % 8 == 0,
-                MRL_ERR_INVALID_ARG, "%s: leading dimensions lda=%lld ldb=%lld ldo=%lld", fn, (long long)lda, (long long)ldb,
-                (long long)ldo);
+template <int kOut, bool kATrans, bool kBTrans, bool kSliced>
+static int launch_gemm(const char* fn, const Product& p, const SplitPlan& plan) {
+    // k-contiguous operands are read up to the next multiple of 64 in k
+    const int64_t k_steps = (p.k + BK - 1) / BK * BK;
+    MRL_REQUIRE(p.m > 0 && p.n > 0 && p.k > 0 && p.m % 8 == 0, MRL_ERR_UNSUPPORTED,
+                "%s: product of m=%lld n=%lld k=%lld (m must be a multiple of 8)", fn, (long long)p.m, (long long)p.n,
+                (long long)p.k);
+    MRL_REQUIRE(p.m <= 0x7fffffffLL && p.n <= 0x7fffffffLL && p.k <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED,
+                "%s: size out of range", fn);
+    MRL_REQUIRE((kATrans || kBTrans) || p.k % BK == 0, MRL_ERR_UNSUPPORTED,
+                "%s: k=%lld must be a multiple of %d when no operand is k-major", fn, (long long)p.k, BK);
+    MRL_REQUIRE(!kBTrans || p.n % 8 == 0, MRL_ERR_UNSUPPORTED, "%s: n=%lld must be a multiple of 8 for a k-major b", fn,
+                (long long)p.n);
+    MRL_REQUIRE(p.lda >= (kATrans ? p.m : k_steps) && p.ldb >= (kBTrans ? p.n : k_steps) && p.ldo >= p.m && p.lda % 8 == 0 &&
+                    p.ldb % 8 == 0 && p.ldo % 8 == 0,
+                MRL_ERR_INVALID_ARG, "%s: leading dimensions lda=%lld ldb=%lld ldo=%lld", fn, (long long)p.lda,
+                (long long)p.ldb, (long long)p.ldo);
     // what one buffer descriptor has to span: a tile of 256 rows, or a stage of 64 k-rows
-    MRL_REQUIRE(256 * lda * 2 < (1LL << 31) && 256 * ldb * 2 < (1LL << 31), MRL_ERR_UNSUPPORTED,
+    MRL_REQUIRE(256 * p.lda * 2 < (1LL << 31) && 256 * p.ldb * 2 < (1LL << 31), MRL_ERR_UNSUPPORTED,
                 "%s: 256 rows of an operand must stay below 2 GiB", fn);
-    MRL_REQUIRE(aligned(a, 16) && aligned(b, 16) && aligned(out, 16), MRL_ERR_MISALIGNED,
+    MRL_REQUIRE(aligned(p.a, 16) && aligned(p.b, 16) && aligned(p.out, 16) && aligned(p.sums, 16), MRL_ERR_MISALIGNED,
                 "%s: operands must be 16-byte aligned", fn);
     const int grid = persistent_grid();
     MRL_REQUIRE(grid >= 8, MRL_ERR_LAUNCH, "%s: cannot query the device", fn);
-    if (!a_kmajor && !b_kmajor && !accumulate_f32)
-        return launch_gemm<false, false, false>(fn, grid, a, lda, m, b, ldb, n, k, out, ldo, stream);
-    if (a_kmajor && !b_kmajor && !accumulate_f32)
-        return launch_gemm<false, true, false>(fn, grid, a, lda, m, b, ldb, n, k, out, ldo, stream);
-    if (a_kmajor && b_kmajor && accumulate_f32)
-        return launch_gemm<true, true, true>(fn, grid, a, lda, m, b, ldb, n, k, out, ldo, stream);
-    MRL_REQUIRE(false, MRL_ERR_UNSUPPORTED, "%s: this combination of operand layouts is not built", fn);
-    return MRL_ERR_UNSUPPORTED;
+    // function attributes belong to a device: reserved with every launch, on whichever device is current
+    const hipError_t attr = hipFuncSetAttribute((const void*)gemm_kernel<kOut, kATrans, kBTrans, kSliced>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    MRL_REQUIRE(attr == hipSuccess, MRL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", fn, kLdsBytes);
+    hipLaunchKernelGGL((gemm_kernel<kOut, kATrans, kBTrans, kSliced>), dim3((unsigned)grid), dim3(kThreads), kLdsBytes,
+                       p.stream, (const uint16_t*)p.a, p.lda, (int)p.m, (const uint16_t*)p.b, p.ldb, (int)p.n, (int)p.k,
+                       p.out, p.ldo, p.sums, plan);
+    return check_launch(fn);
+}
+
+static int64_t slice_bytes(const SplitPlan& plan) {
+    return plan.n_slices > 1 ? plan.rest * plan.n_slices * kTileElems * (int64_t)sizeof(float) : 0;
+}
+
+static SplitPlan whole_tiles(const Product& p) { return SplitPlan{make_grid(p.m, p.n).total, 0, 1}; }
+
+static SplitPlan plan_dhidden(int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
+    const int grid = persistent_grid();
+    return plan_split(make_grid(hidden_dim, n_tokens).total, grid < 8 ? 1 : grid, (vocab + BK - 1) / BK);
+}
+
+// dHidden[t][h] = sum_v W[v][h] * dlogits[t][v]: the weight as it lies is the k-major operand; its rows
+// beyond vocab read as zero, dlogits is read up to the next multiple of 64 columns.  Cut along the vocabulary
+// as far as the workspace reaches.
+static int dhidden(const char* fn, const void* weight, const void* dlogits, int64_t dlogits_row_stride, int64_t n_tokens,
+                   int64_t vocab, int64_t hidden_dim, void* d_hidden, void* workspace, int64_t workspace_bytes,
+                   hipStream_t s) {
+    const Product p = {weight, hidden_dim, hidden_dim, dlogits, dlogits_row_stride, n_tokens, vocab, d_hidden, hidden_dim,
+                       reinterpret_cast<float*>(workspace), s};
+    const SplitPlan plan = plan_dhidden(n_tokens, vocab, hidden_dim);
+    if (plan.n_slices == 1 || workspace == nullptr || workspace_bytes < slice_bytes(plan))
+        return launch_gemm<kBf16, true, false, false>(fn, p, whole_tiles(p));
+    int rc = plan.whole > 0 ? launch_gemm<kBf16, true, false, false>(fn, p, plan) : MRL_OK;
+    if (rc == MRL_OK) rc = launch_gemm<kF32, true, false, true>(fn, p, plan);
+    if (rc != MRL_OK) return rc;
+    hipLaunchKernelGGL(merge_slices_kernel, dim3((unsigned)plan.rest, BN / 16), dim3(256), 0, s, p.sums, plan, (int)p.m,
+                       (int)p.n, (uint16_t*)p.out, p.ldo);
+    return check_launch(fn);
+}
+
+// dW[v][h] (+)= sum_t hidden[t][h] * dlogits[t][v]: both operands k-major as they lie, any n_tokens
+template <int kOut>
+static int dweight(const char* fn, const void* hidden, const void* dlogits, int64_t dlogits_row_stride, int64_t n_tokens,
+                   int64_t vocab, int64_t hidden_dim, void* out, float* sums, hipStream_t s) {
+    const Product p = {hidden, hidden_dim, hidden_dim, dlogits, dlogits_row_stride, vocab, n_tokens, out, hidden_dim, sums, s};
+    return launch_gemm<kOut, true, true, false>(fn, p, whole_tiles(p));
+}
+
+static int check_bwd(const char* fn, int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
+    MRL_REQUIRE(n_tokens >= 0 && vocab > 0 && hidden_dim > 0, MRL_ERR_INVALID_ARG,
+                "%s: n_tokens=%lld vocab=%lld hidden_dim=%lld", fn, (long long)n_tokens, (long long)vocab,
+                (long long)hidden_dim);
+    MRL_REQUIRE(hidden_dim % 8 == 0 && vocab % 8 == 0, MRL_ERR_UNSUPPORTED,
+                "%s: hidden_dim=%lld and vocab=%lld must be multiples of 8", fn, (long long)hidden_dim, (long long)vocab);
+    MRL_REQUIRE(dlogits_row_stride % BK == 0 && dlogits_row_stride >= vocab, MRL_ERR_INVALID_ARG,
+                "%s: dlogits_row_stride=%lld must be a multiple of %d and at least vocab (the padding columns must hold "
+                "zeros)", fn, (long long)dlogits_row_stride, BK);
+    return MRL_OK;
 }
 
 }  // namespace mrl
@@ -231,31 +384,46 @@ extern "C" int mrl_lmhead_logits(const void* hidden, const void* weight, int64_t
     MRL_REQUIRE(logits_row_stride >= vocab, MRL_ERR_INVALID_ARG, "%s: logits_row_stride below vocab", fn);
     if (n_tokens == 0) return MRL_OK;
     MRL_REQUIRE(hidden && weight && logits, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
-    return mrl::gemm_bf16(fn, weight, hidden_dim, vocab, false, hidden, hidden_dim, n_tokens, false, hidden_dim, logits,
-                          logits_row_stride, false, mrl::as_stream(stream));
+    const mrl::Product p = {weight, hidden_dim, vocab, hidden, hidden_dim, n_tokens, hidden_dim, logits, logits_row_stride,
+                            nullptr, mrl::as_stream(stream)};
+    return mrl::launch_gemm<kBf16, false, false, false>(fn, p, mrl::whole_tiles(p));
 }
 
 extern "C" int mrl_lmhead_logprob_bwd(const void* hidden, const void* weight, const void* dlogits,
                                       int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab, int64_t hidden_dim,
                                       void* d_hidden, float* d_weight, void* stream) {
     const char* fn = "mrl_lmhead_logprob_bwd";
-    MRL_REQUIRE(n_tokens >= 0 && vocab > 0 && hidden_dim > 0, MRL_ERR_INVALID_ARG,
-                "%s: n_tokens=%lld vocab=%lld hidden_dim=%lld", fn, (long long)n_tokens, (long long)vocab,
-                (long long)hidden_dim);
-    MRL_REQUIRE(hidden_dim % 8 == 0 && vocab % 8 == 0, MRL_ERR_UNSUPPORTED,
-                "%s: hidden_dim=%lld and vocab=%lld must be multiples of 8", fn, (long long)hidden_dim, (long long)vocab);
-    MRL_REQUIRE(dlogits_row_stride % BK == 0 && dlogits_row_stride >= vocab, MRL_ERR_INVALID_ARG,
-                "%s: dlogits_row_stride=%lld must be a multiple of %d and at least vocab (the padding columns must hold "
-                "zeros)", fn, (long long)dlogits_row_stride, BK);
-    if (n_tokens == 0) return MRL_OK;
+    int rc = mrl::check_bwd(fn, dlogits_row_stride, n_tokens, vocab, hidden_dim);
+    if (rc != MRL_OK || n_tokens == 0) return rc;
     MRL_REQUIRE(hidden && weight && dlogits && d_hidden && d_weight, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
     hipStream_t s = mrl::as_stream(stream);
-    // dHidden[t][h] = sum_v W[v][h] * dlogits[t][v]: the weight as it lies is the k-major operand; its rows
-    // beyond vocab read as zero, dlogits is read up to the next multiple of 64 columns
-    int rc = mrl::gemm_bf16(fn, weight, hidden_dim, hidden_dim, true, dlogits, dlogits_row_stride, n_tokens, false, vocab,
-                            d_hidden, hidden_dim, false, s);
+    rc = mrl::dhidden(fn, weight, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_hidden, nullptr, 0, s);
     if (rc != MRL_OK) return rc;
-    // dW[v][h] += sum_t hidden[t][h] * dlogits[t][v]: both operands k-major as they lie, any n_tokens
-    return mrl::gemm_bf16(fn, hidden, hidden_dim, hidden_dim, true, dlogits, dlogits_row_stride, vocab, true, n_tokens,
-                          d_weight, hidden_dim, true, s);
+    return mrl::dweight<kF32Add>(fn, hidden, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_weight, d_weight, s);
+}
+
+extern "C" int64_t mrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
+    if (n_tokens <= 0 || vocab <= 0 || hidden_dim <= 0) return 0;
+    return mrl::slice_bytes(mrl::plan_dhidden(n_tokens, vocab, hidden_dim));
+}
+
+extern "C" int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weight, const void* dlogits,
+                                            int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab, int64_t hidden_dim,
+                                            void* d_hidden, void* d_weight, float* d_weight_sums, int first, int last,
+                                            void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "mrl_lmhead_logprob_bwd_chunk";
+    int rc = mrl::check_bwd(fn, dlogits_row_stride, n_tokens, vocab, hidden_dim);
+    if (rc != MRL_OK) return rc;
+    MRL_REQUIRE(n_tokens > 0, MRL_ERR_INVALID_ARG, "%s: an empty chunk", fn);
+    MRL_REQUIRE(hidden && weight && dlogits && d_hidden && (d_weight || !last) && (d_weight_sums || (first && last)),
+                MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    hipStream_t s = mrl::as_stream(stream);
+    rc = mrl::dhidden(fn, weight, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_hidden, workspace,
+                      workspace_bytes, s);
+    if (rc != MRL_OK) return rc;
+#define MRL_DWEIGHT(OUT, dst) \
+    mrl::dweight<OUT>(fn, hidden, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, dst, d_weight_sums, s)
+    if (first) return last ? MRL_DWEIGHT(kBf16, d_weight) : MRL_DWEIGHT(kF32, d_weight_sums);
+    return last ? MRL_DWEIGHT(kSumToBf16, d_weight) : MRL_DWEIGHT(kF32Add, d_weight_sums);
+#undef MRL_DWEIGHT
 }

@@ -73,9 +73,18 @@ __device__ __forceinline__ int64_t stage_src_offset_kmajor(int wave, int lane, i
 
 typedef floatx4 Accumulators[kBlocks][kBlocks];
 
+// The k_range of a sequence whose tiles all run over the whole of K.
+struct WholeK {
+    __device__ __forceinline__ void k_range(int, int n_ksteps, int& begin, int& end) const {
+        begin = 0;
+        end = n_ksteps;
+    }
+};
+
 // Runs the workgroup's tiles.  `smem`: kLdsStages bytes of LDS, 16-byte aligned (more is the caller's).
-// `seq`: n_tiles and coords(j, tm, tn), the tile coordinates (in units of 256 rows of A and of B) of the
-// j-th tile of this workgroup, uniform over the workgroup.  `epilogue(acc, tm, tn)` is called with the
+// `seq`: n_tiles; coords(j, tm, tn), the tile coordinates (in units of 256 rows of A and of B) of the j-th
+// tile of this workgroup, and k_range(j, n_ksteps, begin, end), the k-steps of 64 that go into it (at least
+// one), all uniform over the workgroup.  `epilogue(acc, j, tm, tn)` is called with the
 // finished tile: wavefront (wv, wt) = (wave / 2, wave % 2) holds rows wv * 128 .. + 127 of A (m) and
 // wt * 128 .. + 127 of B (n); acc[vb][tb] is the 16 x 16 block at m = 16 vb, n = 16 tb of it, of which a
 // lane holds column n = lane & 15 and rows m = 4 (lane >> 4) .. + 3.  Rows of a ragged last tile beyond
@@ -95,7 +104,7 @@ __device__ __forceinline__ void mfma_tile_loop(unsigned char* smem, const uint16
 
     // ---- loader state: the tile whose stages are being requested
     int load_j = 0;                                   // index into the workgroup's tile sequence
-    int load_k = 0;
+    int load_k = 0, load_begin = 0, load_end = 0;     // k-step being requested, the tile's range
     int a_off[kLoadsPerWave], b_off[kLoadsPerWave];
     mrl::rsrc_t a_rsrc, b_rsrc;
     int load_tm = 0, load_tn = 0;
@@ -125,6 +134,8 @@ __device__ __forceinline__ void mfma_tile_loop(unsigned char* smem, const uint16
         // one descriptor per tile: byte offsets inside a tile stay below 2^32 for any operand size
         if (!kATrans) a_rsrc = mrl::make_rsrc(A + (int64_t)load_tm * BM * lda, 0xffffffffu);
         if (!kBTrans) b_rsrc = mrl::make_rsrc(B + (int64_t)load_tn * BN * ldb, 0xffffffffu);
+        seq.k_range(j, n_ksteps, load_begin, load_end);
+        load_k = load_begin;
         set_load_stage();
     };
     // request i (0..15) of the stage being requested: the wavefront's 8 groups of A, then of B
@@ -142,8 +153,8 @@ __device__ __forceinline__ void mfma_tile_loop(unsigned char* smem, const uint16
     // After the last stage of the last tile the requests go on (the schedule below has no branches):
     // they fetch valid bytes of the last tile into a buffer that nobody reads any more.
     auto stage_issued = [&]() {
-        if (++load_k == n_ksteps) {
-            load_k = 0;
+        if (++load_k == load_end) {
+            load_k = load_begin;
             if (++load_j < n_tiles) set_load_tile(load_j);
             else set_load_stage();
         } else {
@@ -290,7 +301,9 @@ __device__ __forceinline__ void mfma_tile_loop(unsigned char* smem, const uint16
     for (int mine = 0; mine < n_tiles; ++mine) {
         zero_acc();
         pin_acc();
-        for (int kstep = 0; kstep < n_ksteps; ++kstep, ++stage_idx) {
+        int k_begin, k_end;
+        seq.k_range(mine, n_ksteps, k_begin, k_end);
+        for (int kstep = k_begin; kstep < k_end; ++kstep, ++stage_idx) {
             const int buf = stage_idx & 1;
             const unsigned char* stage = smem + buf * kStageBytes;
             const unsigned char* other = smem + (buf ^ 1) * kStageBytes;
@@ -334,7 +347,7 @@ __device__ __forceinline__ void mfma_tile_loop(unsigned char* smem, const uint16
         pin_acc();
         int tm, tn;
         seq.coords(mine, tm, tn);
-        epilogue(acc, tm, tn);
+        epilogue(acc, mine, tm, tn);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);                // nothing is in flight into LDS when the workgroup ends
 #undef MRL_SB

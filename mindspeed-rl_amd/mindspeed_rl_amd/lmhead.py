@@ -97,7 +97,7 @@ class _FusedLmHeadLoss(torch.autograd.Function):
     The rows are processed in chunks: ``logits_c = hidden_c @ weight^T`` (``mrl_lmhead_logits``),
     the fused sweep turns the chunk into dlogits in place (one read, one write), then
     ``dHidden_c = dlogits_c @ weight`` and ``dWeight += dlogits_c^T @ hidden_c``
-    (``mrl_lmhead_logprob_bwd``, fp32 accumulation across chunks in stream order).  All three
+    (``mrl_lmhead_logprob_bwd_chunk``, fp32 accumulation across chunks in stream order).  All three
     products run on the hand-written bf16 MFMA kernels; only ``chunk_rows x V`` logits exist at any
     time."""
 
@@ -149,7 +149,14 @@ class _FusedLmHeadLoss(torch.autograd.Function):
         else:
             logits = torch.empty((chunk, v_pad), dtype=h2d.dtype, device=dev)
         d_hidden = torch.empty_like(h2d)
-        d_weight32 = torch.zeros((vocab, hdim), dtype=torch.float32, device=dev)
+        # dWeight leaves the last chunk's product as bf16; fp32 sums exist only between chunks.  dHidden of a
+        # step in one chunk may be cut along the vocabulary; in several it never is, so that it does not
+        # depend on the chunking.
+        one_chunk = n_rows <= chunk
+        d_weight = torch.empty((vocab, hdim), dtype=w.dtype, device=dev) if n_rows > 0 else torch.zeros_like(w)
+        d_weight32 = None if one_chunk else torch.empty((vocab, hdim), dtype=torch.float32, device=dev)
+        cut_bytes = _lib.load().mrl_lmhead_bwd_workspace_bytes(n_rows, vocab, hdim) if one_chunk else 0
+        cut = torch.empty(cut_bytes, dtype=torch.uint8, device=dev) if cut_bytes else None
         esz = h2d.element_size()
         for c0 in range(0, n_rows, chunk):
             rows = min(n_rows, c0 + chunk) - c0
@@ -163,8 +170,9 @@ class _FusedLmHeadLoss(torch.autograd.Function):
                 cfg["kl_coef"], cfg["entropy_coeff"], cfg["loss_scale"], _lib.ptr(ops.applied), _lib.ptr(logits), v_pad,
                 None, (ent.data_ptr() + c0 * 4) if want_ent else None, p_terms + c0 * 32, ops.workspace,
                 ops.ws_bytes, 1 if c0 == 0 else 0, stream)
-            _timed("mrl_lmhead_logprob_bwd", rows, dev, h_c, _lib.ptr(w), _lib.ptr(logits), v_pad, rows, vocab, hdim,
-                   d_hidden.data_ptr() + c0 * hdim * esz, _lib.ptr(d_weight32), stream)
+            _timed("mrl_lmhead_logprob_bwd_chunk", rows, dev, h_c, _lib.ptr(w), _lib.ptr(logits), v_pad, rows, vocab, hdim,
+                   d_hidden.data_ptr() + c0 * hdim * esz, _lib.ptr(d_weight), _lib.ptr(d_weight32), 1 if c0 == 0 else 0,
+                   1 if c0 + rows == n_rows else 0, _lib.ptr(cut), cut_bytes, stream)
         if live is not None:
             compact_dh = d_hidden
             d_hidden = torch.zeros_like(h_all)
@@ -173,7 +181,6 @@ class _FusedLmHeadLoss(torch.autograd.Function):
             terms_all.view(all_rows, 8).index_copy_(0, live, row_terms[:n_rows * 8].view(n_rows, 8))
         ops.reduce(stream)
         applied = ops.applied
-        d_weight = d_weight32.to(w.dtype)
         ctx.save_for_backward(d_hidden, d_weight, applied)
         ctx.meta = (tuple(hidden.shape), cfg.get("scale_state"))
         ctx.handed_out = False

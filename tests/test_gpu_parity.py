@@ -2725,6 +2725,60 @@ def test_standard_computer_sweeps_only_window_rows(dev, layout):
     assert torch.equal(lp3, lp.detach()) and torch.equal(ent3, ent.detach())
 
 
+@pytest.mark.parametrize("tokens,vocab,hdim", [(1, 8200, 64), (162, 8200, 512), (257, 16392, 264), (4352, 16392, 4096),
+                                               (700, 40000, 1544)])
+def test_lmhead_backward_chunk(dev, tokens, vocab, hdim):
+    """The backward products of one chunk: dHidden tiles cut along the vocabulary (a single tile, ragged tiles,
+    a last k-step of 8, whole rounds of the chip and a rest) against the fp32 product and the uncut call;
+    dWeight written as bf16 at once, and through fp32 sums over three chunks, equals the fp32 accumulation
+    rounded once, bit for bit."""
+    g = torch.Generator(device=dev).manual_seed(tokens + vocab)
+    v_pad = (vocab + 63) // 64 * 64
+    h = torch.randn(tokens, hdim, generator=g, device=dev).to(torch.bfloat16)
+    w = torch.randn(vocab, hdim, generator=g, device=dev).to(torch.bfloat16)
+    dz = torch.zeros(tokens, v_pad, dtype=torch.bfloat16, device=dev)
+    dz[:, :vocab] = torch.randn(tokens, vocab, generator=g, device=dev)
+    lib, stream = _lib.load(), _lib.stream(dev)
+    need = lib.mrl_lmhead_bwd_workspace_bytes(tokens, vocab, hdim)
+    assert need > 0 and need % (256 * 256 * 4) == 0
+    ws = torch.full((need + 64,), 0xFF, dtype=torch.uint8, device=dev)      # NaNs, should a slice not be written
+
+    def chunk(lo, hi, dh, dw, sums, first, last, ws_bytes):
+        _lib.call("mrl_lmhead_logprob_bwd_chunk", h[lo:hi].data_ptr(), w.data_ptr(), dz[lo:hi].data_ptr(), v_pad, hi - lo,
+                  vocab, hdim, dh[lo:hi].data_ptr(), _lib.ptr(dw), _lib.ptr(sums), first, last,
+                  ws.data_ptr() if ws_bytes else None, ws_bytes, stream)
+
+    dw32 = torch.zeros(vocab, hdim, device=dev)
+    dh0 = torch.empty_like(h)
+    _lib.call("mrl_lmhead_logprob_bwd", h.data_ptr(), w.data_ptr(), dz.data_ptr(), v_pad, tokens, vocab, hdim,
+              dh0.data_ptr(), dw32.data_ptr(), stream)
+    dh, dw = torch.full_like(h, 7.0), torch.full_like(w, 7.0)
+    chunk(0, tokens, dh, dw, None, 1, 1, need)
+    torch.cuda.synchronize()
+    assert (ws[need:] == 0xFF).all().item()
+    assert torch.equal(dw, dw32.to(torch.bfloat16))
+    # one rounding to bf16 (2^-8 of the value at most) and fp32 sums of `vocab` products of spread sqrt(vocab)
+    want = dz[:, :vocab].float() @ w.float()
+    bound = 2 ** -8 * want.abs() + 1e-5 * vocab ** 0.5
+    assert ((dh.float() - want).abs() <= bound).all().item()
+    assert ((dh.float() - dh0.float()).abs() <= 2 * bound).all().item()       # two roundings
+    again = torch.empty_like(h)
+    chunk(0, tokens, again, dw, None, 1, 1, need)
+    assert torch.equal(again, dh)
+    # less workspace than it takes: not cut
+    chunk(0, tokens, again, dw, None, 1, 1, need - 16)
+    assert torch.equal(again, dh0)
+    if tokens >= 3:
+        cuts = [0, tokens // 3, tokens // 2, tokens]
+        dw32.zero_()
+        sums = torch.full_like(dw32, float("nan"))
+        for i in range(3):
+            _lib.call("mrl_lmhead_logprob_bwd", h[cuts[i]:].data_ptr(), w.data_ptr(), dz[cuts[i]:].data_ptr(), v_pad,
+                      cuts[i + 1] - cuts[i], vocab, hdim, again[cuts[i]:].data_ptr(), dw32.data_ptr(), stream)
+            chunk(cuts[i], cuts[i + 1], dh, dw if i == 2 else None, sums, int(i == 0), int(i == 2), 0)
+        assert torch.equal(again, dh) and torch.equal(dw, dw32.to(torch.bfloat16))
+
+
 def test_fused_lmhead_policy_loss_skips_rows_without_response(dev):
     """With long prompts most rows carry no live response token: the chunked lm_head step gathers the
     live rows and runs its GEMMs on them alone.  Same loss, statistics, dHidden and dWeight as with
