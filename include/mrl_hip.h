@@ -159,6 +159,24 @@ int mrl_window_scatter(const float* g_out, int64_t batch, int64_t width, const v
 /* mrl_generate_mask: generate_mask (mindspeed_rl/utils/utils.py:57-67): out[i, j] =
  * (j < lengths[i]) as int64, [batch, width]; lengths is I32 or I64.  Negative lengths give an
  * all-zero row, lengths above width an all-one row. */
+/* The response windows in rows of the logits, for the scoring passes (reference: logprob_computer.py:73-145).
+ *   layout 0, packed: the rows that mrl_unpad_gather copies with prompt_length (seqlens, cu_seqlens_padded);
+ *   layout 1, padded [batch, padded_s]: rows [P - 1, P + R - 1) of each sequence, clamped to it.
+ * mrl_window_rows: active[t] = 1 for the rows that lie in a window (its first `width` rows), 0 for all others
+ * of the n_rows; active: 16-byte aligned, n_rows rounded up to 16 bytes.
+ * mrl_window_cut: log-probs and entropies of the rows as [batch, width], zero behind a window; with
+ * entropy_rows NULL the entropies are zeros.  Length columns are I32 or I64; response_length is read in
+ * layout 1 only. */
+int mrl_window_rows(int layout, int64_t batch, int64_t width, int64_t n_rows, const int32_t* seqlens,
+                    const int32_t* cu_seqlens_padded, int64_t padded_s, const void* prompt_length,
+                    int prompt_dtype, const void* response_length, int response_dtype, uint8_t* active,
+                    void* stream);
+int mrl_window_cut(int layout, int64_t batch, int64_t width, int64_t n_rows, const int32_t* seqlens,
+                   const int32_t* cu_seqlens_padded, int64_t padded_s, const void* prompt_length,
+                   int prompt_dtype, const void* response_length, int response_dtype,
+                   const float* logp_rows, const float* entropy_rows, float* logp, float* entropy,
+                   void* stream);
+
 int mrl_generate_mask(const void* lengths, int lengths_dtype, int64_t batch, int64_t width,
                       int64_t* out, void* stream);
 

@@ -38,6 +38,8 @@ SIGNATURES = {
     "mrl_pad_scatter": [_vp, _i64, _i64, _vp, _vp, _vp, _int, _i64, _vp, _vp],
     "mrl_window_gather": [_vp, _int, _i64, _i64, _i64, _vp, _int, _i64, ctypes.c_uint64, _vp, _vp],
     "mrl_window_scatter": [_vp, _i64, _i64, _vp, _int, _i64, _vp, _vp],
+    "mrl_window_rows": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp],
+    "mrl_window_cut": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _vp],
     "mrl_generate_mask": [_vp, _int, _i64, _i64, _vp, _vp],
     "mrl_ragged_layout": [_vp, _int, _i64, _i64, _vp, _int, _i64, _int, _vp, _vp, _vp, _vp],
     "mrl_ragged_to_padded": [_vp, _int, _i64, _i64, _vp, _i64, _i64, ctypes.c_uint64, _vp, _vp],

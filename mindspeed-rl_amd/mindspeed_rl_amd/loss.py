@@ -16,8 +16,8 @@ import torch
 
 from . import _lib, vocab_ops
 from .functional import is_multimodal
-from .packing import (generate_mask, postprocess_packed_seqs, response_window, truncate_middle_and_pad,
-                      truncate_prompt_and_pad)
+from .packing import (ResponseWindows, generate_mask, postprocess_packed_seqs, response_window,
+                      truncate_middle_and_pad, truncate_prompt_and_pad)
 from .vocab_ops import compute_log_probs, vocab_logprob_entropy, vocab_parallel_entropy
 
 STAT_KEYS = ("actor/pg_loss", "actor/pg_clipfrac", "actor/ppo_kl", "actor/kl_loss", "actor/entropy")
@@ -407,47 +407,29 @@ class StandardLogProbComputer(LogProbComputer):
         return truncate_prompt_and_pad(batch["responses"], logprob, window)
 
     @staticmethod
-    def _rows_in_windows(output, batch, kwargs):
-        """uint8 flag per logits row: 1 where the row lies in a response window, i.e. where the cut
-        below reads it.  Rows outside every window (prompts, padding) are not swept at all: their
-        log-prob, entropy and gradient are never looked at by the reference either."""
-        dev = output.device
-        width = batch["responses"].shape[-1]
-        prompt = batch["prompt_length"].reshape(-1).to(device=dev, dtype=torch.int64)
-        if kwargs.get("use_remove_padding", False):
-            n_rows = output.shape[-2]
-            n = kwargs["seqlens_in_batch"].reshape(-1).to(device=dev, dtype=torch.int64)
-            start = kwargs["cu_seqlens_padded"].reshape(-1).to(device=dev, dtype=torch.int64)[:-1]
-            cut = (prompt - 1) < n                     # postprocess_packed_seqs: start += P-1, len -= P
-            start = torch.where(cut, start + prompt - 1, start)
-            n = torch.where(cut, n - prompt, n)
-        else:
-            n_seq, padded = output.shape[0], output.shape[1]
-            n_rows = n_seq * padded
-            resp = batch["response_length"].reshape(-1).to(device=dev, dtype=torch.int64)
-            lo = (prompt - 1).clamp(0, padded)
-            hi = (prompt + resp - 1).clamp(0, padded)
-            start = lo + torch.arange(n_seq, device=dev, dtype=torch.int64) * padded
-            n = hi - lo
-        n = n.clamp(0, width)
-        start = start.clamp(0, n_rows)
-        end = (start + n).clamp(max=n_rows)
-        edge = torch.zeros(n_rows + 1, dtype=torch.int32, device=dev)
-        one = torch.ones_like(start, dtype=torch.int32)
-        edge.index_add_(0, start, one)
-        edge.index_add_(0, end, -one)
-        return (torch.cumsum(edge[:-1], 0) > 0).to(torch.uint8)
+    def _windows(output, batch, kwargs):
+        """Rows outside every response window (prompts, padding) are not swept at all: their log-prob,
+        entropy and gradient are never looked at by the reference either."""
+        packed = kwargs.get("use_remove_padding", False)
+        return ResponseWindows(output.shape[:-1], batch, packed, kwargs.get("seqlens_in_batch"),
+                               kwargs.get("cu_seqlens_padded"))
+
+    @classmethod
+    def _rows_in_windows(cls, output, batch, kwargs):
+        return cls._windows(output, batch, kwargs).rows()
 
     def compute(self, output, batch, skip_entropy, **kwargs):
         labels = batch["labels"]
         inv_t = float(kwargs.get("inv_temperature", 1.0))
         injected = vocab_ops.get_vocab_parallel()
         weight = kwargs.get("lm_head_weight")
+        windows = None
         if weight is not None:
             # `output` holds the hidden states: the rows of the response windows are projected and scored
             # tile by tile on the matrix cores, no logits are written (forward only, no autograd)
             from .lmhead import lmhead_logprob
-            active = self._rows_in_windows(output, batch, kwargs).view(labels.shape)
+            windows = self._windows(output, batch, kwargs)
+            active = windows.rows().view(labels.shape)
             log_probs, entropy, _ = lmhead_logprob(output, weight, labels, inv_temperature=inv_t,
                                                    want_entropy=not skip_entropy, row_active=active)
         elif injected is not None and injected is not vocab_ops.vocab_parallel_cross_entropy:
@@ -456,10 +438,14 @@ class StandardLogProbComputer(LogProbComputer):
             log_probs = compute_log_probs(scaled, labels)
             entropy = None if skip_entropy else vocab_parallel_entropy(scaled)
         else:
-            active = self._rows_in_windows(output, batch, kwargs).view(labels.shape)
+            windows = self._windows(output, batch, kwargs)
+            active = windows.rows().view(labels.shape)
             log_probs, entropy, _ = vocab_logprob_entropy(output, labels, inv_temperature=inv_t,
-                                                          want_entropy=not skip_entropy, row_active=active,
+                                                          want_entropy=None if skip_entropy else True,
+                                                          row_active=active,
                                                           grad_inplace=bool(kwargs.get("grad_inplace", False)))
+        if windows is not None and not log_probs.requires_grad:
+            return windows.cut(log_probs, None if skip_entropy else entropy)
         if kwargs.get("use_remove_padding", False):
             seqlens = kwargs.get("seqlens_in_batch", None)
             cu = kwargs.get("cu_seqlens_padded", None)

@@ -222,3 +222,48 @@ def truncate_middle_and_pad(responses, input_tensor, truncate_lengths, pad_value
 def response_window(prompt_length, response_length):
     """``cat([P, P+R], dim=1) - 1`` (reference: ``models/loss/base_loss_func.py:47-53``)."""
     return torch.cat([prompt_length, prompt_length + response_length], dim=1) - 1
+
+
+class ResponseWindows:
+    """The response windows of a batch in rows of the logits: which rows they cover, and the cut of per-row
+    results to ``[B, L]`` (what ``postprocess_packed_seqs`` with ``prompt_length``, or ``truncate_prompt_and_pad``
+    over :func:`response_window`, does to one tensor)."""
+
+    def __init__(self, lead, batch, packed, seqlens=None, cu_seqlens=None):
+        self.width = batch["responses"].shape[-1]
+        self.prompt, self.resp = batch["prompt_length"], batch.get("response_length")
+        if packed:
+            self.layout, self.padded, self.n_rows = 0, 0, lead[-1]
+            self.seqlens = seqlens.to(torch.int32).contiguous()
+            self.cu = cu_seqlens.to(torch.int32).contiguous()
+            self.n_seq, self.resp = self.seqlens.numel(), None
+            if self.cu.numel() != self.n_seq + 1:
+                raise ValueError("cu_seqlens_padded needs one entry more than seqlens_in_batch")
+        else:
+            self.layout, self.n_seq, self.padded = 1, lead[0], lead[1]
+            self.n_rows, self.seqlens, self.cu = lead[0] * lead[1], None, None
+            if self.prompt.dim() != 2 or self.resp.dim() != 2:
+                raise ValueError("prompt_length and response_length must have shape (mbs, 1)")
+            self.resp = _as_index(self.resp)
+        self.prompt = _as_index(self.prompt)
+        if self.prompt.numel() != self.n_seq or (self.resp is not None and self.resp.numel() != self.n_seq):
+            raise ValueError("prompt_length and response_length need one entry per sequence")
+        self.dev = _lib.require_device(self.prompt, self.resp, self.seqlens, self.cu)
+        self._args = (self.layout, self.n_seq, self.width, self.n_rows, _lib.ptr(self.seqlens), _lib.ptr(self.cu),
+                      self.padded, _lib.ptr(self.prompt), _lib.dtype_code(self.prompt), _lib.ptr(self.resp),
+                      _lib.dtype_code(self.resp) if self.resp is not None else _lib.I32)
+
+    def rows(self):
+        """uint8 flag per row: 1 where the row lies in a window, i.e. where the cut reads it."""
+        flags = torch.empty((self.n_rows + 15) // 16 * 16, dtype=torch.uint8, device=self.dev)
+        _lib.call("mrl_window_rows", *self._args, flags.data_ptr() if self.n_rows else None, _lib.stream(self.dev))
+        return flags[:self.n_rows]
+
+    def cut(self, logp_rows, entropy_rows):
+        """``(log_probs, entropy)`` ``[B, L]`` fp32 in one launch; entropies are zeros for ``None``.  No autograd."""
+        _lib.require_device(self.prompt, logp_rows, entropy_rows)
+        logp = torch.empty((self.n_seq, self.width), dtype=torch.float32, device=self.dev)
+        ent = torch.empty_like(logp)
+        _lib.call("mrl_window_cut", *self._args, _lib.ptr(logp_rows), _lib.ptr(entropy_rows), _lib.ptr(logp), _lib.ptr(ent),
+                  _lib.stream(self.dev))
+        return logp, ent

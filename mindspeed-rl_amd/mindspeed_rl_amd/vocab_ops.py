@@ -88,6 +88,9 @@ class _VocabLogprobEntropy(torch.autograd.Function):
         ctx.save_for_backward(flat, lab, lse, ent if want_entropy else None)
         ctx.meta = (tuple(logits.shape), float(inv_temperature), row_stride, bool(grad_inplace))
         lse_out = lse.view(lead)
+        if want_entropy is None:            # nobody looks at the entropies: no zeros in their place
+            ctx.mark_non_differentiable(lse_out)
+            return logp.view(lead), None, lse_out
         ent_out = ent.view(lead) if want_entropy else torch.zeros(lead, dtype=torch.float32, device=dev)
         if want_entropy:
             ctx.mark_non_differentiable(lse_out)
@@ -124,7 +127,7 @@ def vocab_logprob_entropy(logits, labels, inv_temperature=1.0, want_entropy=True
     caller's ``logits / temperature`` into the sweep.  ``row_active`` (bool/uint8, optional)
     skips rows whose result is not needed.  ``grad_inplace=True`` lets the backward overwrite the
     logits storage with dlogits (saves one ``[T, V]`` buffer; the caller must not read the logits
-    afterwards).  With ``want_entropy=False`` the entropy output is zeros.
+    afterwards).  With ``want_entropy=False`` the entropy output is zeros, with ``None`` it is None.
     """
     return _VocabLogprobEntropy.apply(logits, labels, inv_temperature, want_entropy, row_active, grad_inplace)
 

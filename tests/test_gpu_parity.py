@@ -2663,6 +2663,50 @@ def test_injected_cross_entropy_reaches_the_loss_objects(dev):
 
 
 @pytest.mark.parametrize("layout", ["padded", "packed"])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_response_windows(dev, layout, index):
+    """Row flags and the cut of both results in one launch, against the reference's index arithmetic: windows
+    that start in front of the rows, end behind them or behind `width`, empty ones, a response width of 1."""
+    from mindspeed_rl_amd.packing import ResponseWindows
+    plen = torch.tensor([[1], [7], [3], [40], [4], [9], [2]], dtype=index)
+    rlen = torch.tensor([[5], [0], [50], [3], [60], [31], [38]], dtype=index)
+    n_seq, padded = plen.shape[0], 37
+    for width in (1, 12, 70):
+        b = {"responses": torch.zeros(n_seq, width, dtype=torch.int64, device=dev), "prompt_length": plen.to(dev),
+             "response_length": rlen.to(dev)}
+        if layout == "padded":
+            n_rows = n_seq * padded
+            windows = ResponseWindows((n_seq, padded), b, False)
+            spans = [(i * padded + min(int(p) - 1, padded), i * padded + min(int(p + r) - 1, padded))
+                     for i, (p, r) in enumerate(zip(plen, rlen))]
+        else:
+            seqlens = torch.tensor([6, 7, 40, 43, 4, 40, 30], dtype=torch.int32)
+            cu = torch.zeros(n_seq + 1, dtype=torch.int32)
+            cu[1:] = torch.cumsum(seqlens, 0)
+            n_rows = int(cu[-1]) - 5                                    # the last window ends behind the rows
+            windows = ResponseWindows((1, n_rows), b, True, seqlens.to(dev), cu.to(dev))
+            spans = [(int(c) + int(p) - 1, int(c) + int(n) - 1) if int(p) - 1 < int(n) else (int(c), int(c) + int(n))
+                     for c, n, p in zip(cu, seqlens, plen)]
+        lp_rows = torch.randn(n_rows, generator=torch.Generator().manual_seed(width))
+        ent_rows = torch.rand(n_rows)
+        flags, lp, ent = torch.zeros(n_rows, dtype=torch.uint8), torch.zeros(n_seq, width), torch.zeros(n_seq, width)
+        for i, (lo, hi) in enumerate(spans):
+            hi = min(hi, lo + width, n_rows)
+            if hi > lo:
+                flags[lo:hi] = 1
+                lp[i, :hi - lo], ent[i, :hi - lo] = lp_rows[lo:hi], ent_rows[lo:hi]
+        assert torch.equal(windows.rows().cpu(), flags)
+        got = windows.cut(lp_rows.to(dev), ent_rows.to(dev))
+        assert torch.equal(got[0].cpu(), lp) and torch.equal(got[1].cpu(), ent)
+        got = windows.cut(lp_rows.to(dev), None)
+        assert torch.equal(got[0].cpu(), lp) and not got[1].any().item()
+    with pytest.raises(ValueError):
+        ResponseWindows((n_seq + 1, padded), b, False)
+    with pytest.raises(RuntimeError):
+        ResponseWindows((n_seq, padded), dict(b, prompt_length=plen), False)
+
+
+@pytest.mark.parametrize("layout", ["padded", "packed"])
 def test_standard_computer_sweeps_only_window_rows(dev, layout):
     """The split path's log-prob strategy skips the logits rows that the response-window cut never
     reads (prompt rows, the last row, padding): same [B, L] values bit for bit as a sweep over every
