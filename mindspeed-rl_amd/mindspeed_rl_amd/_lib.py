@@ -90,6 +90,7 @@ _RESTYPES = {"mrl_last_error": ctypes.c_char_p, "mrl_fused_workspace_bytes": cty
              "mrl_value_loss_workspace_bytes": ctypes.c_int64, "mrl_lmhead_bwd_workspace_bytes": ctypes.c_int64}
 
 _lib = None
+_entry = {}             # name -> bound function, looked up once
 
 
 class MrlError(RuntimeError):
@@ -120,16 +121,18 @@ def load():
         fn = getattr(lib, name)       # AttributeError if the library lacks a declared symbol
         fn.argtypes = argtypes
         fn.restype = _RESTYPES.get(name, ctypes.c_int)
+        _entry[name] = fn
     _lib = lib
     return lib
 
 
 def call(name, *args):
     """Calls an entry point; a negative status becomes MrlError (ValueError-like codes included)."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    if _lib is None:
+        load()
+    rc = _entry[name](*args)
     if rc != 0:
-        raise MrlError(name, rc, lib.mrl_last_error().decode("utf-8", "replace"))
+        raise MrlError(name, rc, _lib.mrl_last_error().decode("utf-8", "replace"))
 
 
 def dtype_code(t):
@@ -164,6 +167,31 @@ def require_device(*tensors):
     return dev
 
 
+# the handle alone, without a Stream object around it (3 us of a call that takes 10); part of every torch that
+# compiles for this device, and where it is not, the public way serves
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream(device):
     """Raw hipStream_t of torch's current stream on `device` (kernels are enqueued there)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def dense(t, dtype, dev):
+    """`t` as a contiguous tensor of `dtype` on `dev`; None stays None.  The usual case is that it is one already."""
+    if t is None or (t.dtype is dtype and t.device == dev and t.is_contiguous()):
+        return t
+    return t.to(dev).to(dtype).contiguous()
+
+
+def index_column(t, dev):
+    """A length column as a flat, dense int32 / int64 tensor on `dev`; None stays None."""
+    if t is None:
+        return None
+    if t.dtype is not torch.int32 and t.dtype is not torch.int64:
+        t = t.to(torch.int64)
+    if t.device != dev:
+        t = t.to(dev)
+    return (t if t.dim() == 1 else t.reshape(-1)).contiguous()

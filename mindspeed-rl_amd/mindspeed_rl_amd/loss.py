@@ -224,24 +224,15 @@ class _FusedOperands:
     def __init__(self, dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, sweep_dtype_code, vocab, sweep_rows):
         lib = _lib.load()
 
-        def f32(t):
-            return None if t is None else t.to(dev).to(torch.float32).contiguous()
-
-        def idx(t):
-            if t is None:
-                return None
-            if t.dtype not in (torch.int32, torch.int64):
-                t = t.to(torch.int64)
-            return t.to(dev).reshape(-1).contiguous()
-
+        f32, i32 = torch.float32, torch.int32
         self.dev, self.cfg = dev, cfg
         self.n_rows, self.n_seq, self.width, self.layout, self.padded_s = n_rows, n_seq, width, layout, padded_s
-        self.old, self.ref, self.adv = f32(batch.get("old_log_prob")), f32(cfg["ref_log_prob"]), f32(batch.get("advantages"))
+        self.old, self.ref, self.adv = (_lib.dense(batch.get("old_log_prob"), f32, dev), _lib.dense(cfg["ref_log_prob"], f32, dev),
+                                        _lib.dense(batch.get("advantages"), f32, dev))
         self.mask_t, _ = _mask_args(cfg["mask"], batch["response_length"], dev)
-        self.prompt, self.resp = idx(batch["prompt_length"]), idx(batch["response_length"])
+        self.prompt, self.resp = _lib.index_column(batch["prompt_length"], dev), _lib.index_column(batch["response_length"], dev)
         if layout == 0:
-            self.seqlens = cfg["seqlens"].to(dev).to(torch.int32).contiguous()
-            self.cu = cfg["cu"].to(dev).to(torch.int32).contiguous()
+            self.seqlens, self.cu = _lib.dense(cfg["seqlens"], i32, dev), _lib.dense(cfg["cu"], i32, dev)
         else:
             self.seqlens = self.cu = None
         self.mdt = _lib.dtype_code(self.mask_t) if self.mask_t is not None else _lib.F32

@@ -7,6 +7,8 @@ map kernels.  Where the reference runs a Python loop with two or three ``.item()
 sequence, these launch one kernel; ``preprocess_packed_seqs`` keeps a single host read (the
 packed length, needed to size its outputs).
 """
+import math
+
 import torch
 
 from . import _lib
@@ -155,6 +157,8 @@ class _WindowGather(torch.autograd.Function):
 
 
 def _pad_bits(dtype, pad_value):
+    if type(pad_value) in (int, float) and pad_value == 0 and math.copysign(1.0, pad_value) > 0:
+        return 0                # the usual pad: all bits clear in every dtype
     t = torch.tensor([pad_value], dtype=dtype)
     if t.element_size() == 2:
         return int(t.view(torch.int16).item()) & 0xFFFF
