@@ -342,6 +342,30 @@ __global__ __launch_bounds__(kReduceBlock) void value_loss_fwd_kernel(
     if (threadIdx.x == 0) write_value_loss(ssum, csum, count, loss_scale, out, nullptr);
 }
 
+// The critic's loss reads the value head's output where it lies: with the windows cut out first and scattered
+// back by the backward, five more launches and an autograd node went into 2 MB (128 x (256 + 2048) tokens: PPO
+// value side 278 us a pass, now 217).
+//
+// Where the predicted value of token j of sample i lies: element i * width + j of [batch, width], or (kHead)
+// in the value head's output [batch, padded_s] at the response window [P - 1, P + R - 1) of the sample,
+// clamped to its row; tokens behind the window have the value 0 and no gradient.
+struct ValuePlace {
+    int64_t width, padded_s;
+    const void* prompt;
+    int prompt_dtype;
+    const void* resp;
+    int resp_dtype;
+    __device__ __forceinline__ int64_t at(const void* p, int dtype, int64_t i) const {
+        return dtype == MRL_I32 ? (int64_t) reinterpret_cast<const int32_t*>(p)[i]
+                                : reinterpret_cast<const int64_t*>(p)[i];
+    }
+    __device__ __forceinline__ void window(int64_t i, int64_t& lo, int64_t& hi) const {
+        const int64_t p = at(prompt, prompt_dtype, i), e = p + at(resp, resp_dtype, i) - 1;
+        lo = p - 1 < 0 ? 0 : (p - 1 > padded_s ? padded_s : p - 1);
+        hi = e < 0 ? 0 : (e > padded_s ? padded_s : e);
+    }
+};
+
 // The same spread over the chip: one workgroup per row (rows strided beyond kLossRows of them) leaves its
 // three sums in fp64, a second launch adds them up in a fixed order.  128 x 2048: 11 us for both, was
 // 167 us by one workgroup, which pays off only where no scratch memory is at hand.
@@ -350,19 +374,24 @@ struct LossSums {
     double loss, clipped, count;
 };
 
+template <bool kHead>
 __global__ __launch_bounds__(256) void value_loss_rows_kernel(
-    const float* __restrict__ vpreds, const float* __restrict__ returns, const float* __restrict__ values,
-    const void* __restrict__ mask, int mdtype, const void* __restrict__ lens, int ldtype, int64_t batch,
-    int64_t width, float clip, LossSums* __restrict__ sums) {
+    const float* __restrict__ vpreds, ValuePlace place, const float* __restrict__ returns,
+    const float* __restrict__ values, const void* __restrict__ mask, int mdtype, const void* __restrict__ lens, int ldtype,
+    int64_t batch, float clip, LossSums* __restrict__ sums) {
+    const int64_t width = place.width;
     __shared__ double part[3][256 / 64];
     double acc[3] = {0.0, 0.0, 0.0};
     for (int64_t i = blockIdx.x; i < batch; i += gridDim.x) {
+        int64_t lo = 0, hi = width;
+        if (kHead) place.window(i, lo, hi);
+        const float* row = vpreds + (kHead ? i * place.padded_s + lo : i * width);
         for (int64_t j = threadIdx.x; j < width; j += 256) {
             const float m = mask_at(mask, mdtype, lens, ldtype, i, j, width);
             acc[2] += (double)m;
             if (m != 0.f) {
                 const int64_t e = i * width + j;
-                const ValueTerm t = value_term(vpreds[e], returns[e], values[e], clip);
+                const ValueTerm t = value_term(j < hi - lo ? row[j] : 0.f, returns[e], values[e], clip);
                 acc[0] += (double)(t.loss * m);
                 acc[1] += (double)(t.clipped * m);
             }
@@ -407,6 +436,28 @@ __global__ __launch_bounds__(256) void value_loss_bwd_kernel(
         float g = 0.f;
         if (m != 0.f) g = coef * m * value_term(vpreds[e], returns[e], values[e], clip).d;
         g_vpreds[e] = g;
+    }
+}
+
+// The gradient of the whole value head output: every entry finds its token, entries outside the windows get 0.
+__global__ __launch_bounds__(256) void critic_loss_bwd_kernel(
+    const float* __restrict__ head, ValuePlace place, const float* __restrict__ returns, const float* __restrict__ values,
+    int64_t batch, float clip, float loss_scale, const float* __restrict__ out, const float* __restrict__ upstream,
+    float* __restrict__ g_head) {
+    const float coef = (*upstream) * loss_scale * 0.5f / (out[3] + 1e-8f);
+    const int64_t n = batch * place.padded_s;
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+        const int64_t i = e / place.padded_s, s = e - i * place.padded_s;
+        int64_t lo, hi;
+        place.window(i, lo, hi);
+        const int64_t j = s - lo;
+        float g = 0.f;
+        if (j >= 0 && s < hi && j < place.width) {
+            const float m = mask_at(nullptr, 0, place.resp, place.resp_dtype, i, j, place.width);
+            const int64_t t = i * place.width + j;
+            if (m != 0.f) g = coef * m * value_term(head[e], returns[t], values[t], clip).d;
+        }
+        g_head[e] = g;
     }
 }
 
@@ -545,13 +596,68 @@ extern "C" int mrl_value_loss_fwd_split(const float* vpreds, const float* return
     LossSums* sums = reinterpret_cast<LossSums*>(workspace);
     const int rows = (int)(batch < kLossRows ? batch : kLossRows);
     if (rows > 0) {
-        hipLaunchKernelGGL(value_loss_rows_kernel, dim3((unsigned)rows), dim3(256), 0, s, vpreds, returns, values, mask,
-                           mask_dtype, response_length, length_dtype, batch, width, cliprange_value, sums);
+        const ValuePlace place = {width, 0, nullptr, 0, nullptr, 0};
+        hipLaunchKernelGGL(value_loss_rows_kernel<false>, dim3((unsigned)rows), dim3(256), 0, s, vpreds, place, returns,
+                           values, mask, mask_dtype, response_length, length_dtype, batch, cliprange_value, sums);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
     hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums, rows,
                        loss_scale, out, loss_out);
+    return mrl::check_launch(fn);
+}
+
+static int check_critic(const char* fn, int64_t batch, int64_t padded_s, int64_t width, int prompt_dtype, int response_dtype) {
+    MRL_REQUIRE(batch >= 0 && padded_s >= 0 && width > 0, MRL_ERR_INVALID_ARG, "%s: batch=%lld padded_s=%lld width=%lld", fn,
+                (long long)batch, (long long)padded_s, (long long)width);
+    MRL_REQUIRE(mrl::int_dtype_bytes(prompt_dtype) != 0 && mrl::int_dtype_bytes(response_dtype) != 0, MRL_ERR_UNSUPPORTED,
+                "%s: length dtypes %d and %d (want I32 or I64)", fn, prompt_dtype, response_dtype);
+    return MRL_OK;
+}
+
+extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
+                                   int prompt_dtype, const void* response_length, int response_dtype, const float* returns,
+                                   const float* values, int64_t width, float cliprange_value, float loss_scale, float* out,
+                                   float* loss_out, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "mrl_critic_loss_fwd";
+    int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
+    if (rc != MRL_OK) return rc;
+    MRL_REQUIRE(out != nullptr && (batch == 0 || ((head || padded_s == 0) && prompt_length && response_length && returns &&
+                                                  values && workspace)),
+                MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    MRL_REQUIRE(mrl::aligned(workspace, 8), MRL_ERR_MISALIGNED, "%s: workspace must be 8-byte aligned", fn);
+    MRL_REQUIRE(workspace_bytes >= mrl_value_loss_workspace_bytes(batch), MRL_ERR_INVALID_ARG,
+                "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
+                (long long)mrl_value_loss_workspace_bytes(batch));
+    hipStream_t s = mrl::as_stream(stream);
+    LossSums* sums = reinterpret_cast<LossSums*>(workspace);
+    const int rows = (int)(batch < kLossRows ? batch : kLossRows);
+    if (rows > 0) {
+        const ValuePlace place = {width, padded_s, prompt_length, prompt_dtype, response_length, response_dtype};
+        hipLaunchKernelGGL(value_loss_rows_kernel<true>, dim3((unsigned)rows), dim3(256), 0, s, head, place, returns, values,
+                           (const void*)nullptr, 0, response_length, response_dtype, batch, cliprange_value, sums);
+        rc = mrl::check_launch(fn);
+        if (rc != MRL_OK) return rc;
+    }
+    hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums, rows,
+                       loss_scale, out, loss_out);
+    return mrl::check_launch(fn);
+}
+
+extern "C" int mrl_critic_loss_bwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
+                                   int prompt_dtype, const void* response_length, int response_dtype, const float* returns,
+                                   const float* values, int64_t width, float cliprange_value, float loss_scale,
+                                   const float* out, const float* upstream, float* g_head, void* stream) {
+    const char* fn = "mrl_critic_loss_bwd";
+    int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
+    if (rc != MRL_OK || batch * padded_s == 0) return rc;
+    MRL_REQUIRE(head && prompt_length && response_length && returns && values && out && upstream && g_head,
+                MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    const ValuePlace place = {width, padded_s, prompt_length, prompt_dtype, response_length, response_dtype};
+    const int64_t n = batch * padded_s;
+    const unsigned grid = (unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
+    hipLaunchKernelGGL(critic_loss_bwd_kernel, dim3(grid), dim3(256), 0, mrl::as_stream(stream), head, place, returns, values,
+                       batch, cliprange_value, loss_scale, out, upstream, g_head);
     return mrl::check_launch(fn);
 }
 

@@ -31,7 +31,7 @@ class AdaptiveKLController:
 
 
 def _f32(t, dev):
-    return t.detach().to(device=dev, dtype=torch.float32).contiguous()
+    return _lib.dense(t.detach(), torch.float32, dev)
 
 
 def _lengths(response_length, dev):
@@ -60,7 +60,8 @@ def kl_token_level_rewards(old_log_prob, ref_log_prob, response_length, rm_score
     _lib.call("mrl_kl_token_rewards", _lib.ptr(old), _lib.ptr(ref), _lib.ptr(lens), _lib.dtype_code(lens),
               _lib.ptr(scores), batch, width, _lib.KL_BY_NAME[penalty], float(beta), _lib.ptr(rewards),
               _lib.ptr(row_kl), _lib.stream(dev))
-    return rewards, torch.mean(row_kl, dim=0).item()
+    # the copy waits for the kernel either way: the mean of `batch` numbers is taken where they land
+    return rewards, torch.mean(row_kl.cpu().double(), dim=0).float().item()
 
 
 def _whiten(values, mask, shift_mean):
@@ -154,6 +155,44 @@ class _ValueLoss(torch.autograd.Function):
         return g.to(ctx.in_dtype), None, None, None, None, None, None
 
 
+class _CriticLoss(torch.autograd.Function):
+    """The value head's output [B, S, 1] -> (scaled loss, out[4]) through mrl_critic_loss_fwd / _bwd: the response
+    windows are read and their gradients written where they lie."""
+
+    @staticmethod
+    def forward(ctx, head, prompt, lens, returns, values, clip, loss_scale):
+        dev = _lib.require_device(head, prompt, lens, returns, values)
+        head = head.contiguous()
+        ret, val = _f32(returns, dev), _f32(values, dev)
+        (batch, padded, _), width = head.shape, ret.shape[1]
+        out = torch.empty(4, dtype=torch.float32, device=dev)
+        loss = torch.empty((), dtype=torch.float32, device=dev)     # autograd outputs must not alias
+        ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(batch)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        scalars = (float(clip), float(loss_scale))
+        _lib.call("mrl_critic_loss_fwd", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
+                  _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, *scalars, _lib.ptr(out),
+                  _lib.ptr(loss), _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
+        ctx.save_for_backward(head, prompt, lens, ret, val, out)
+        ctx.scalars = scalars
+        ctx.mark_non_differentiable(out)
+        ctx.set_materialize_grads(False)
+        return loss, out
+
+    @staticmethod
+    def backward(ctx, g_loss, _g_out):
+        if g_loss is None:
+            return (None,) * 7
+        head, prompt, lens, ret, val, out = ctx.saved_tensors
+        dev = head.device
+        upstream = _lib.dense(g_loss, torch.float32, dev)
+        g = torch.empty_like(head)
+        _lib.call("mrl_critic_loss_bwd", _lib.ptr(head), head.shape[0], head.shape[1], _lib.ptr(prompt),
+                  _lib.dtype_code(prompt), _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), ret.shape[1],
+                  *ctx.scalars, _lib.ptr(out), _lib.ptr(upstream), _lib.ptr(g), _lib.stream(dev))
+        return g, None, None, None, None, None, None
+
+
 def value_loss(vpreds, returns, values, response_mask=None, response_length=None, *, cliprange_value,
                loss_scale=1.0):
     """Clipped value loss: ``(loss_scale * vf_loss, out)`` with ``out = [scaled loss, vf_loss,
@@ -199,12 +238,31 @@ class CriticLossFunc(BaseLossFunc):
                                      dim=1) - 1
         return truncate_middle_and_pad(responses, output, truncate_lengths)
 
+    def _reads_windows_in_place(self, output, batch):
+        """The value head's own layout, fp32 [B, S, 1] with [B, 1] lengths and [B, L] operands that belong to
+        it: what the loss kernels read without a copy of the windows."""
+        if type(self)._get_compute_vpreds is not CriticLossFunc._get_compute_vpreds:
+            return False                    # a subclass cuts them itself
+        if not (output.is_cuda and output.dim() == 3 and output.shape[2] == 1 and output.dtype is torch.float32):
+            return False
+        shape = tuple(batch["responses"].shape)
+        columns = (batch["prompt_length"], batch["response_length"])
+        rows = (batch.get("returns"), batch.get("values"))
+        return (len(shape) == 2 and shape[0] == output.shape[0] and shape[1] > 0
+                and all(tuple(c.shape) == (shape[0], 1) and c.dtype in (torch.int32, torch.int64) for c in columns)
+                and all(t is not None and tuple(t.shape) == shape for t in rows))
+
     def compute_loss(self, output: torch.Tensor, batch: Dict[str, torch.Tensor], forward_only=False,
                      non_loss_data=True, **kwargs) -> Tuple[torch.Tensor, Dict]:
         if kwargs.get("use_remove_padding", False):
             output = postprocess_packed_seqs(output=output, seqlens_in_batch=kwargs.get("seqlens_in_batch", None),
                                              cu_seqlens_padded=kwargs.get("cu_seqlens_padded", None),
                                              seq_len=kwargs.get("seq_len", None))
+        if not forward_only and "responses" in batch and self._reads_windows_in_place(output, batch):
+            loss, out = _CriticLoss.apply(output, batch["prompt_length"].contiguous(), batch["response_length"].contiguous(),
+                                          batch["returns"], batch["values"], self.cliprange_value,
+                                          _dynamic_scale(batch, forward_only, kwargs))
+            return loss, self._statistics(out)
         vpreds = self._get_compute_vpreds(output, batch)
         if forward_only:
             return vpreds
@@ -215,9 +273,12 @@ class CriticLossFunc(BaseLossFunc):
         loss, out = value_loss(vpreds.reshape(vpreds.shape[0], vpreds.shape[1]), batch.get("returns"),
                                batch.get("values"), None, batch["response_length"],
                                cliprange_value=self.cliprange_value, loss_scale=scale)
+        return loss, self._statistics(out)
+
+    @staticmethod
+    def _statistics(out):
         host = out.detach().cpu().tolist()      # one device-to-host copy for both statistics
-        stats = {"critic/vf_loss": abs(host[1]), "critic/vf_clipfrac": host[2]}
-        return loss, stats
+        return {"critic/vf_loss": abs(host[1]), "critic/vf_clipfrac": host[2]}
 
     @staticmethod
     def _compute_value_loss(vpreds, returns, values, response_mask, cliprange_value):

@@ -2662,6 +2662,36 @@ def test_injected_cross_entropy_reaches_the_loss_objects(dev):
     assert abs(loss_plain.item() - loss.item()) > 1e-6             # the doubled scoring did change the loss
 
 
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+@pytest.mark.parametrize("padded,width", [(37, 1), (37, 12), (300, 70), (20, 257)])
+def test_critic_loss_reads_the_windows_in_place(dev, index, padded, width):
+    """The critic's loss from the value head's output, windows read where they lie, against the same loss of the
+    windows cut out first: windows that end behind the row, empty ones, responses longer than the window,
+    a strided head.  Same loss, statistics and gradient, bit for bit."""
+    g = torch.Generator().manual_seed(padded + width)
+    plen = torch.tensor([[1], [7], [3], [40], [4], [9], [2]], dtype=index)
+    rlen = torch.tensor([[5], [0], [50], [3], [60], [31], [38]], dtype=index).clamp(max=width)
+    n = plen.shape[0]
+    head = torch.randn(n, padded, 2, generator=g).to(dev)[:, :, :1]
+    b = {"responses": torch.zeros(n, width, dtype=torch.int64), "prompt_length": plen, "response_length": rlen,
+         "returns": torch.randn(n, width, generator=g), "values": torch.randn(n, width, generator=g)}
+    b = _to_dev(b, dev)
+    f = mrl.LossFuncFactory.get_instance("ray_ppo", "critic")
+    f.add_loss_meta_info({"cliprange_value": 0.4})
+    x = head.detach().requires_grad_()
+    assert not x.is_contiguous() and f._reads_windows_in_place(x, b)
+    loss, stats = f.compute_loss(x, b, use_dynamic_bsz=True, actual_micro_batch_size=4)
+    (got,) = torch.autograd.grad(loss / 3.0, x)
+    y = head.detach().contiguous().requires_grad_()
+    vpreds = f._get_compute_vpreds(y, b)
+    want_loss, out = mrl.value_loss(vpreds.reshape(n, width), b["returns"], b["values"], None, b["response_length"],
+                                    cliprange_value=0.4, loss_scale=n / 4)
+    (want,) = torch.autograd.grad(want_loss / 3.0, y)
+    assert loss.item() == want_loss.item()
+    assert stats == {"critic/vf_loss": abs(out[1].item()), "critic/vf_clipfrac": out[2].item()}
+    assert torch.equal(got, want) and (want.abs().sum().item() > 0)
+
+
 @pytest.mark.parametrize("layout", ["padded", "packed"])
 @pytest.mark.parametrize("index", [torch.int32, torch.int64])
 def test_response_windows(dev, layout, index):
