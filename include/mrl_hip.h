@@ -192,6 +192,30 @@ int mrl_generate_mask(const void* lengths, int lengths_dtype, int64_t batch, int
  * ([batch, width] integers, elem_bytes 4 or 8) is given, 0 where lengths[i] == 0 and
  * rows[i, 0] == -1.  eff_len (nullable int32 [batch]) receives the len_i.  One workgroup;
  * batch <= 2^20. */
+/* Several columns at once (at most MRL_RAGGED_COLUMNS), each as by the calls for one below: mrl_ragged_layouts
+ * as mrl_ragged_layout without `rows`, mrl_ragged_columns as mrl_ragged_to_padded (to_padded != 0) or
+ * mrl_padded_to_ragged.  The columns are read on the host during the call.  Fields that a call does not name
+ * are not looked at beyond their range. */
+#define MRL_RAGGED_COLUMNS 16
+typedef struct mrl_ragged_column {
+    const void* lengths;    /* layouts: [batch] I32 or I64 */
+    int32_t* eff_len;       /* layouts, nullable */
+    int32_t* cu;            /* [batch + 1]: written by layouts, read by columns */
+    int64_t* info;          /* layouts: {total, longest row rounded up to `multiple`} */
+    const void* src;        /* columns */
+    void* dst;              /* columns */
+    uint64_t pad_bits;      /* to padded */
+    int64_t batch;
+    int64_t width;          /* layouts: 0, or the width that lengths are clamped to; columns: of the padded rows */
+    int64_t multiple;
+    int64_t first_dim;      /* to padded: [batch, first_dim, width] from [first_dim, src_stride] */
+    int64_t src_stride;
+    int64_t total;          /* to ragged: entries of dst */
+    int lengths_dtype, elem_bytes, left_pad, reserved;
+} mrl_ragged_column;
+int mrl_ragged_layouts(const mrl_ragged_column* columns, int n_columns, void* stream);
+int mrl_ragged_columns(int to_padded, const mrl_ragged_column* columns, int n_columns, void* stream);
+
 int mrl_ragged_layout(const void* lengths, int lengths_dtype, int64_t batch, int64_t multiple,
                       const void* rows, int elem_bytes, int64_t width, int left_pad, int32_t* eff_len,
                       int32_t* cu, int64_t* info, void* stream);

@@ -54,14 +54,17 @@ __device__ __forceinline__ GroupMoments group_moments(const void* rewards, int r
     return m;
 }
 
-// One workgroup per GROUP: its first wavefront reduces the group's rewards (above), then the four
-// wavefronts share the group's rows and write score * mask across each of them.
+// One workgroup per ROW: its first wavefront reduces the rewards of the row's group (above), then all four write
+// score * mask across the row.  A group's rewards are read once per row of the group, which is nothing next to
+// the rows themselves, and the chip is filled (256 rows of 2048 in groups of 8: 28.7 us with a workgroup per
+// group, 8.4 us now).
 __global__ __launch_bounds__(kBlock) void group_advantage_kernel(const void* __restrict__ rewards, int rdtype,
                                                                  int64_t group, const void* __restrict__ mask,
                                                                  int mdtype, int64_t width,
                                                                  float* __restrict__ adv, float* __restrict__ ret) {
     __shared__ double moments_s[2];
-    const int64_t g0 = (int64_t)blockIdx.x * group;
+    const int64_t i = blockIdx.x;
+    const int64_t g0 = i / group * group;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (wave == 0) {
         const GroupMoments m = group_moments(rewards, rdtype, g0, group);
@@ -72,14 +75,12 @@ __global__ __launch_bounds__(kBlock) void group_advantage_kernel(const void* __r
     }
     __syncthreads();
     const double mean = moments_s[0], sd = moments_s[1];
-    for (int64_t q = wave; q < group; q += kBlock / 64) {
-        const int64_t i = g0 + q;
-        const float score = (float)((reward_at(rewards, rdtype, i) - mean) / (sd + 1e-6));
-        for (int64_t j = lane; j < width; j += 64) {
-            const float v = score * mask_as_float(mask, mdtype, i * width + j);
-            adv[i * width + j] = v;
-            if (ret) ret[i * width + j] = v;
-        }
+    const float score = (float)((reward_at(rewards, rdtype, i) - mean) / (sd + 1e-6));
+#pragma unroll 4
+    for (int64_t j = threadIdx.x; j < width; j += kBlock) {
+        const float v = score * mask_as_float(mask, mdtype, i * width + j);
+        adv[i * width + j] = v;
+        if (ret) ret[i * width + j] = v;
     }
 }
 
@@ -181,7 +182,7 @@ extern "C" int mrl_group_advantage(const void* rewards, int rewards_dtype, int64
                     mrl::aligned(returns, 4),
                 MRL_ERR_MISALIGNED, "%s: misaligned buffer", fn);
     if (width == 0) return MRL_OK;
-    hipLaunchKernelGGL(group_advantage_kernel, dim3((unsigned)(batch / group)), dim3(kBlock), 0, mrl::as_stream(stream),
+    hipLaunchKernelGGL(group_advantage_kernel, dim3((unsigned)batch), dim3(kBlock), 0, mrl::as_stream(stream),
                        rewards, rewards_dtype, group, mask, mask_dtype, width, advantages, returns);
     return mrl::check_launch(fn);
 }

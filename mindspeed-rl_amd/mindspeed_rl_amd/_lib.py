@@ -26,6 +26,17 @@ _i64 = ctypes.c_int64
 _int = ctypes.c_int
 _f32 = ctypes.c_float
 
+class RaggedColumn(ctypes.Structure):
+    """struct mrl_ragged_column"""
+    _fields_ = [(name, _vp) for name in ("lengths", "eff_len", "cu", "info", "src", "dst")] + [
+        ("pad_bits", ctypes.c_uint64)] + [
+        (name, _i64) for name in ("batch", "width", "multiple", "first_dim", "src_stride", "total")] + [
+        (name, _int) for name in ("lengths_dtype", "elem_bytes", "left_pad", "reserved")]
+
+
+RAGGED_COLUMNS = 16         # MRL_RAGGED_COLUMNS
+
+
 # name -> argtypes; the order is that of include/mrl_hip.h
 SIGNATURES = {
     "mrl_version": [],
@@ -41,6 +52,8 @@ SIGNATURES = {
     "mrl_window_rows": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp],
     "mrl_window_cut": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _vp],
     "mrl_generate_mask": [_vp, _int, _i64, _i64, _vp, _vp],
+    "mrl_ragged_layouts": [_vp, _int, _vp],
+    "mrl_ragged_columns": [_int, _vp, _int, _vp],
     "mrl_ragged_layout": [_vp, _int, _i64, _i64, _vp, _int, _i64, _int, _vp, _vp, _vp, _vp],
     "mrl_ragged_to_padded": [_vp, _int, _i64, _i64, _vp, _i64, _i64, ctypes.c_uint64, _vp, _vp],
     "mrl_padded_to_ragged": [_vp, _int, _i64, _i64, _vp, _int, _i64, _vp, _vp],

@@ -3,8 +3,8 @@
 Host-side mirror of ``pack_experience_columns`` / ``unpack_pad_experience``
 (``mindspeed_rl/trainer/utils/transfer_dock.py:1014-1198``) and ``truncate_rows`` (``mindspeed_rl/utils/pad_process.py:144-166``) with the
 reference's signatures.  The reference walks the rows in Python with one or two ``.item()`` calls
-per row; here each column costs one scan launch, one host read of two integers (to size the
-output) and one gather launch.
+per row; here all columns of a batch cost one scan launch, one host read (two integers a column, to size
+the outputs) and one copy launch.
 """
 import torch
 
@@ -25,36 +25,83 @@ def pack_padded_columns(padded, lengths, left_pad=False):
     elements), ``lengths`` column -> ``[B]`` or ``[B, 1]`` integer lengths.  Returns
     ``(batch_data, batch_data_length)`` in the layout of :func:`pack_experience_columns`: one flat
     tensor per column holding ``padded[i, :len_i]`` back to back (``padded[i, W - len_i:]`` with
-    ``left_pad``) and the int32 lengths.  One scan launch, one host read (the total, to size the
-    output) and one gather launch per column."""
+    ``left_pad``) and the int32 lengths.  One scan launch, one host read (the totals, to size the
+    outputs) and one copy launch for all columns."""
     if not padded:
         raise ValueError("ERROR: when pack, get an empty experience_dict")
     if set(padded.keys()) != set(lengths.keys()):
         raise ValueError("ERROR: when pack, keys of the columns and of their lengths do not match")
-    batch_data, batch_data_length = {}, {}
+    columns = []
     for key, src in padded.items():
         dev = _lib.require_device(src)
         src = src.contiguous()
         if src.dim() != 2 or src.element_size() not in (4, 8):
             raise TypeError("pack_padded_columns takes [B, W] columns with 4- or 8-byte elements")
-        batch, width = src.shape
-        idx = _index(lengths[key].to(dev))
-        if idx.numel() != batch:
+        idx = _lib.index_column(lengths[key], dev)
+        if idx.numel() != src.shape[0]:
             raise ValueError("ERROR: when pack, experience '%s' number=%d does not match experience_count=%d"
-                             % (key, idx.numel(), batch))
-        eff = torch.empty(batch, dtype=torch.int32, device=dev)
-        cu = torch.empty(batch + 1, dtype=torch.int32, device=dev)
-        info = torch.empty(2, dtype=torch.int64, device=dev)
-        stream = _lib.stream(dev)
-        _lib.call("mrl_ragged_layout", _lib.ptr(idx), _lib.dtype_code(idx), batch, 1, None, src.element_size(), width,
-                  0, _lib.ptr(eff), _lib.ptr(cu), _lib.ptr(info), stream)
-        total = int(info[0].item())
-        flat = torch.empty(total, dtype=src.dtype, device=dev)
-        _lib.call("mrl_padded_to_ragged", _lib.ptr(src), src.element_size(), batch, width, _lib.ptr(cu),
-                  1 if left_pad else 0, total, _lib.ptr(flat), stream)
-        batch_data[key] = flat
-        batch_data_length[key] = eff
+                             % (key, idx.numel(), src.shape[0]))
+        eff = torch.empty(src.shape[0], dtype=torch.int32, device=dev)
+        columns.append(_Column(key, src, idx, eff, dev, width=src.shape[1], left_pad=1 if left_pad else 0))
+    _lay_out(columns)
+    batch_data, batch_data_length = {}, {}
+    for c in columns:
+        batch_data[c.key] = c.out = torch.empty(c.total, dtype=c.src.dtype, device=c.dev)
+        batch_data_length[c.key] = c.eff
+    _copy(columns, False)
     return batch_data, batch_data_length
+
+
+class _Column:
+    """One column of a batch between its layout and its copy."""
+
+    def __init__(self, key, src, lengths, eff, dev, width=0, multiple=1, first_dim=1, stride=0, left_pad=0, pad=0):
+        self.key, self.src, self.lengths, self.eff, self.dev = key, src, lengths, eff, dev
+        self.width, self.multiple, self.first_dim, self.stride, self.left_pad, self.pad = (width, multiple, first_dim, stride,
+                                                                                           left_pad, pad)
+        self.total = self.longest = 0
+        self.cu = self.out = None
+
+    def fill(self, c, info):
+        c.lengths, c.lengths_dtype, c.batch = self.lengths.data_ptr(), _lib.dtype_code(self.lengths), self.lengths.numel()
+        c.eff_len, c.cu, c.info = _lib.ptr(self.eff), self.cu.data_ptr(), info
+        c.src, c.dst = self.src.data_ptr(), _lib.ptr(self.out)
+        c.elem_bytes, c.width, c.multiple, c.first_dim = self.src.element_size(), self.width, self.multiple, self.first_dim
+        c.src_stride, c.total, c.left_pad, c.pad_bits = self.stride, self.total, self.left_pad, self.pad
+
+
+def _by_device(columns):
+    """Batches of columns that one launch takes."""
+    devices = []
+    for c in columns:
+        if c.dev not in devices:
+            devices.append(c.dev)
+    for dev in devices:
+        mine = [c for c in columns if c.dev == dev]
+        for lo in range(0, len(mine), _lib.RAGGED_COLUMNS):
+            yield dev, mine[lo:lo + _lib.RAGGED_COLUMNS]
+
+
+def _lay_out(columns):
+    """Offsets of every column, and its size on the host: one scan launch and one host read for all of them."""
+    for dev, part in _by_device(columns):
+        info = torch.empty((len(part), 2), dtype=torch.int64, device=dev)
+        args = (_lib.RaggedColumn * len(part))()
+        for i, c in enumerate(part):
+            c.cu = torch.empty(c.lengths.numel() + 1, dtype=torch.int32, device=dev)
+            c.fill(args[i], info.data_ptr() + 16 * i)
+        _lib.call("mrl_ragged_layouts", args, len(part), _lib.stream(dev))
+        for c, (total, longest) in zip(part, info.tolist()):
+            c.total, c.longest = total, longest
+
+
+def _copy(columns, to_padded):
+    """The copies of every column, in one launch."""
+    for dev, part in _by_device(columns):
+        args = (_lib.RaggedColumn * len(part))()
+        for i, c in enumerate(part):
+            c.fill(args[i], None)
+        _lib.call("mrl_ragged_columns", 1 if to_padded else 0, args, len(part), _lib.stream(dev))
 
 
 def pack_experience_columns(experience_consumer_stage, experience_dict, experience_count, enable_partial_rollout=False):
@@ -98,34 +145,27 @@ def unpack_pad_experience(batch_data, batch_data_length, pad_id, multiple):
         raise ValueError("ERROR: empty batch_data")
     if set(batch_data.keys()) != set(batch_data_length.keys()):
         raise ValueError("ERROR: when unpack, keys from batch_data and batch_data_length dictionaries do not match")
-    out = {}
+    out, columns = {}, []
     for key, length_list in batch_data_length.items():
         data = batch_data[key]
         if key in _SCALAR_COLUMNS:
             out[key] = data.view(-1, 1)
             continue
         dev = _lib.require_device(data)
-        lengths = _index(length_list.to(dev))
-        batch = lengths.numel()
-        cu = torch.empty(batch + 1, dtype=torch.int32, device=dev)
-        info = torch.empty(2, dtype=torch.int64, device=dev)
-        stream = _lib.stream(dev)
-        _lib.call("mrl_ragged_layout", _lib.ptr(lengths), _lib.dtype_code(lengths), batch, int(multiple), None, 0, 0, 0,
-                  None, _lib.ptr(cu), _lib.ptr(info), stream)
-        width = int(info[1].item())              # the one host read per column: sizes the output
         src = data.contiguous()
         if src.element_size() not in (2, 4, 8):
             raise TypeError("unsupported element size %d" % src.element_size())
-        pad = 0.0 if src.is_floating_point() else pad_id
-        if src.dim() > 1:
-            first_dim, stride = src.shape[0], src.shape[1]
-            result = torch.empty((batch, first_dim, width), dtype=src.dtype, device=dev)
-        else:
-            first_dim, stride = 1, src.shape[0]
-            result = torch.empty((batch, width), dtype=src.dtype, device=dev)
-        _lib.call("mrl_ragged_to_padded", _lib.ptr(src), src.element_size(), first_dim, stride, _lib.ptr(cu), batch,
-                  width, _pad_bits(src.dtype, pad), _lib.ptr(result), stream)
-        out[key] = result
+        first_dim, stride = (src.shape[0], src.shape[1]) if src.dim() > 1 else (1, src.shape[0])
+        pad = _pad_bits(src.dtype, 0.0 if src.is_floating_point() else pad_id)
+        out[key] = None                          # the order of the lengths' keys
+        columns.append(_Column(key, src, _lib.index_column(length_list, dev), None, dev, multiple=int(multiple),
+                               first_dim=first_dim, stride=stride, pad=pad))
+    _lay_out(columns)
+    for c in columns:
+        batch, c.width = c.lengths.numel(), c.longest
+        shape = (batch, c.first_dim, c.width) if c.src.dim() > 1 else (batch, c.width)
+        out[c.key] = c.out = torch.empty(shape, dtype=c.src.dtype, device=c.dev)
+    _copy(columns, True)
     return out
 
 

@@ -2662,6 +2662,42 @@ def test_injected_cross_entropy_reaches_the_loss_objects(dev):
     assert abs(loss_plain.item() - loss.item()) > 1e-6             # the doubled scoring did change the loss
 
 
+@pytest.mark.parametrize("n_columns", [1, 16, 19])
+def test_ragged_columns_together(dev, n_columns):
+    """Columns of every element size, one- and two-dimensional, with lengths of their own (zeros, a single
+    sample, lengths beyond the padded width), more of them than one launch takes: each comes out as alone."""
+    g = torch.Generator().manual_seed(n_columns)
+    kinds = [torch.int64, torch.float32, torch.bfloat16, torch.int32]
+    flat, lens, padded, plens, want, packed = {}, {}, {}, {}, {}, {}
+    for c in range(n_columns):
+        dtype, batch = kinds[c % 4], [1, 7, 1500][c % 3]
+        n = torch.randint(0, 9, (batch,), generator=g, dtype=torch.int32 if c % 2 else torch.int64)
+        n[0] = 5
+        total, dims = int(n.sum()), (3,) if c % 5 == 4 else ()
+        flat["c%d" % c] = torch.randint(1, 99, dims + (total,), generator=g).to(dtype)
+        lens["c%d" % c] = n
+        width = (int(n.max()) + 3) // 4 * 4
+        ref = torch.full((batch,) + dims + (width,), 0 if dtype.is_floating_point else 77, dtype=dtype)
+        lo = 0
+        for i, k in enumerate(n.tolist()):
+            ref[i, ..., :k] = flat["c%d" % c][..., lo:lo + k]
+            lo += k
+        want["c%d" % c] = ref
+        if dtype != torch.bfloat16:
+            src = torch.randint(1, 99, (batch, 6), generator=g).to(dtype)
+            padded["c%d" % c], plens["c%d" % c] = src, n.view(-1, 1)
+            packed["c%d" % c] = n.clamp(max=6)
+    got = mrl.unpack_pad_experience(_to_dev(flat, dev), _to_dev(lens, dev), 77, 4)
+    assert list(got) == list(lens)
+    for key, ref in want.items():
+        assert torch.equal(got[key].cpu(), ref), key
+    for left in (False, True):
+        data, length = mrl.pack_padded_columns(_to_dev(padded, dev), _to_dev(plens, dev), left_pad=left)
+        for key, n in packed.items():
+            rows = [r[6 - k:] if left else r[:k] for r, k in zip(padded[key], n.tolist())]
+            assert torch.equal(data[key].cpu(), torch.cat(rows)) and torch.equal(length[key].cpu(), n.to(torch.int32)), key
+
+
 @pytest.mark.parametrize("index", [torch.int32, torch.int64])
 @pytest.mark.parametrize("padded,width", [(37, 1), (37, 12), (300, 70), (20, 257)])
 def test_critic_loss_reads_the_windows_in_place(dev, index, padded, width):
