@@ -2662,6 +2662,44 @@ def test_injected_cross_entropy_reaches_the_loss_objects(dev):
     assert abs(loss_plain.item() - loss.item()) > 1e-6             # the doubled scoring did change the loss
 
 
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                             (torch.float16, torch.float16), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("vocab", [1, 31, 70, 2055, 8001, 8192 + 63, 16385])
+def test_split_sweeps_at_odd_vocabularies(dev, dtype, out_dtype, vocab):
+    """The split forward and backward on rows that start anywhere: dense rows of an odd vocabulary, a tensor that
+    starts off a line, rows shorter than a line, rows of less than a group of vectors and one vector more than a
+    group, a row without gradient, labels at both ends - against an fp64 chain."""
+    rows = 37
+    g = torch.Generator(device=dev).manual_seed(vocab)
+    esz = torch.empty(0, dtype=dtype).element_size()
+    for shift in (0, 1, 16 // esz):
+        z = torch.empty(rows * vocab + shift, dtype=dtype, device=dev)[shift:].view(rows, vocab)
+        z.copy_(torch.randn(rows, vocab, generator=g, device=dev) * 3)
+        # the output starts at the same element of a vector as the input, or (the last) elsewhere
+        for out_shift in (shift % (16 // torch.empty(0, dtype=out_dtype).element_size()), shift + 1):
+            dz = torch.full((rows * vocab + out_shift,), 7.0, dtype=out_dtype, device=dev)[out_shift:].view(rows, vocab)
+            y = torch.randint(0, vocab, (rows,), generator=g, device=dev)
+            y[0], y[1] = 0, vocab - 1
+            g_lp, g_h = torch.randn(rows, generator=g, device=dev), torch.randn(rows, generator=g, device=dev) * 0.1
+            g_lp[3], g_h[3] = 0.0, 0.0
+            lp, ent, lse = (torch.empty(rows, device=dev) for _ in range(3))
+            _lib.call("mrl_vocab_logprob_fwd", z.data_ptr(), _lib.dtype_code(z), rows, vocab, vocab, y.data_ptr(), _lib.I64,
+                      None, 1.0, lp.data_ptr(), ent.data_ptr(), lse.data_ptr(), _lib.stream(dev))
+            _lib.call("mrl_vocab_logprob_bwd", z.data_ptr(), _lib.dtype_code(z), rows, vocab, vocab, y.data_ptr(), _lib.I64,
+                      1.0, lse.data_ptr(), ent.data_ptr(), g_lp.data_ptr(), g_h.data_ptr(), dz.data_ptr(),
+                      _lib.dtype_code(dz), vocab, _lib.stream(dev))
+            x = z.double().requires_grad_()
+            logp = torch.log_softmax(x, -1)
+            want_lp, want_ent = logp.gather(1, y[:, None])[:, 0], -(logp.exp() * logp).sum(-1)
+            (want,) = torch.autograd.grad((want_lp * g_lp.double()).sum() + (want_ent * g_h.double()).sum(), x)
+            # fp32 sums of up to 16 385 terms; log-probs of magnitude up to 30
+            assert (lp - want_lp).abs().max().item() < 1e-4 and (ent - want_ent).abs().max().item() < 1e-4
+            # one rounding to the output type and fp32 arithmetic on factors of magnitude up to 4
+            ulp = {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11, torch.float32: 0.0}[out_dtype]
+            assert ((dz.double() - want).abs() <= ulp * want.abs() + 2e-5).all().item(), (shift, out_shift)
+            assert not dz[3].any().item()
+
+
 @pytest.mark.parametrize("n_columns", [1, 16, 19])
 def test_ragged_columns_together(dev, n_columns):
     """Columns of every element size, one- and two-dimensional, with lengths of their own (zeros, a single
