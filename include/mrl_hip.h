@@ -192,6 +192,23 @@ int mrl_generate_mask(const void* lengths, int lengths_dtype, int64_t batch, int
  * ([batch, width] integers, elem_bytes 4 or 8) is given, 0 where lengths[i] == 0 and
  * rows[i, 0] == -1.  eff_len (nullable int32 [batch]) receives the len_i.  One workgroup;
  * batch <= 2^20. */
+/* Rows that count, for the lm_head passes (no counterpart in the reference, which projects every row).
+ * mrl_live_rows: row r is live if flags[r * stride] (U8 or F32) is not zero; live [n] receives the live rows in
+ *   order, place [n] the position of each row among them or -1, *total their number; counts: scratch of
+ *   ceil(n / 1024) int32.
+ * mrl_move_rows: row i of a_out / b_out is row index[i] of a / b (whole 16-byte vectors a row, b at most 4 KiB),
+ *   zeros where index[i] is -1; c: one entry of 4 or 8 bytes a row, left alone there.  index = live gathers,
+ *   index = place spreads.  A table of 0 bytes is left out.
+ * mrl_spread_scalars: n_columns fp32 columns of n_src entries to n_columns of n: dst[c][r] = src[c][place[r]],
+ *   0 where place[r] is -1. */
+int mrl_live_rows(const void* flags, int flags_dtype, int64_t stride, int64_t n, int32_t* live,
+                  int32_t* place, int32_t* counts, int64_t* total, void* stream);
+int mrl_move_rows(const int32_t* index, int64_t n_rows, const void* a, void* a_out, int64_t a_bytes,
+                  const void* b, void* b_out, int64_t b_bytes, const void* c, void* c_out, int c_bytes,
+                  void* stream);
+int mrl_spread_scalars(const float* src, int64_t n_src, int n_columns, const int32_t* place, int64_t n,
+                       float* dst, void* stream);
+
 /* Several columns at once (at most MRL_RAGGED_COLUMNS), each as by the calls for one below: mrl_ragged_layouts
  * as mrl_ragged_layout without `rows`, mrl_ragged_columns as mrl_ragged_to_padded (to_padded != 0) or
  * mrl_padded_to_ragged.  The columns are read on the host during the call.  Fields that a call does not name

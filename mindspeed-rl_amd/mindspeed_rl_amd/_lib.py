@@ -52,6 +52,9 @@ SIGNATURES = {
     "mrl_window_rows": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp],
     "mrl_window_cut": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _vp],
     "mrl_generate_mask": [_vp, _int, _i64, _i64, _vp, _vp],
+    "mrl_live_rows": [_vp, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
+    "mrl_move_rows": [_vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _int, _vp],
+    "mrl_spread_scalars": [_vp, _i64, _int, _vp, _i64, _vp, _vp],
     "mrl_ragged_layouts": [_vp, _int, _vp],
     "mrl_ragged_columns": [_int, _vp, _int, _vp],
     "mrl_ragged_layout": [_vp, _int, _i64, _i64, _vp, _int, _i64, _int, _vp, _vp, _vp, _vp],

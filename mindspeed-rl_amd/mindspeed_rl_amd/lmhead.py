@@ -38,18 +38,28 @@ def lmhead_logprob(hidden, weight, labels, inv_temperature=1.0, want_entropy=Tru
         if tuple(row_active.shape) != tuple(labels.shape):
             raise ValueError("row_active must have the shape of labels")
         dev = _lib.require_device(hidden, weight, labels, row_active)
-        live = torch.nonzero(row_active.reshape(-1) != 0).flatten()
-        n_all = labels.numel()
-        if live.numel() == 0:
-            return tuple(torch.zeros(labels.shape, dtype=torch.float32, device=dev) for _ in range(3))
-        res = lmhead_logprob(hidden.reshape(-1, hidden.shape[-1]).index_select(0, live), weight,
-                             labels.reshape(-1).index_select(0, live), inv_temperature, want_entropy)
-        outs = []
-        for part in res:
-            full = torch.zeros(n_all, dtype=torch.float32, device=dev)
-            full.index_copy_(0, live, part)
-            outs.append(full.view(labels.shape))
-        return tuple(outs)
+        hdim, n_all = hidden.shape[-1], labels.numel()
+        if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+            raise TypeError("hidden and weight must be bfloat16")
+        flat = hidden.detach().reshape(-1, hdim)
+        if flat.shape[0] != n_all:
+            raise ValueError("labels shape %s does not match hidden leading shape %s"
+                             % (tuple(labels.shape), tuple(hidden.shape[:-1])))
+        flags = row_active.reshape(-1)
+        if flags.dtype is not torch.uint8:
+            flags = (flags != 0).view(torch.uint8)
+        rows = _LiveRows(flags.contiguous(), _lib.U8, 1, n_all, dev)
+        out = torch.zeros if rows.n == 0 else torch.empty
+        full = out((3, n_all), dtype=torch.float32, device=dev)
+        if rows.n > 0:
+            lab = _lib.index_column(labels, dev)
+            h, y, _ = rows.gather(flat, lab, None)
+            part = torch.empty((3, rows.n), dtype=torch.float32, device=dev)
+            _forward(h, weight, y, inv_temperature, part[0], part[1] if want_entropy else None, part[2])
+            if not want_entropy:
+                part[1].zero_()
+            rows.spread_scalars(part, full)
+        return tuple(full[k].view(labels.shape) for k in range(3))
     dev = _lib.require_device(hidden, weight, labels)
     if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         raise TypeError("hidden and weight must be bfloat16")
@@ -60,15 +70,22 @@ def lmhead_logprob(hidden, weight, labels, inv_temperature=1.0, want_entropy=Tru
     if tuple(labels.shape) != tuple(lead):
         raise ValueError("labels shape %s does not match hidden leading shape %s" % (tuple(labels.shape), tuple(lead)))
     h = hidden.detach().reshape(-1, hdim).contiguous()
-    w = weight.detach().contiguous()
-    lab = labels.reshape(-1)
-    if lab.dtype not in (torch.int32, torch.int64):
-        lab = lab.to(torch.int64)
-    lab = lab.contiguous()
-    n_tokens, vocab = h.shape[0], w.shape[0]
+    lab = _lib.index_column(labels, dev)
+    n_tokens = h.shape[0]
     logp = torch.empty(n_tokens, dtype=torch.float32, device=dev)
     lse = torch.empty(n_tokens, dtype=torch.float32, device=dev)
     ent = torch.empty(n_tokens, dtype=torch.float32, device=dev) if want_entropy else None
+    _forward(h, weight, lab, inv_temperature, logp, ent, lse)
+    ent_out = ent.view(lead) if want_entropy else torch.zeros(lead, dtype=torch.float32, device=dev)
+    return logp.view(lead), ent_out, lse.view(lead)
+
+
+def _forward(h, weight, lab, inv_temperature, logp, ent, lse):
+    """The forward of dense rows into the given outputs (ent None: not wanted)."""
+    dev, w = h.device, weight.detach().contiguous()
+    if w.dim() != 2 or w.shape[1] != h.shape[1]:
+        raise ValueError("weight must have shape (vocab, hidden_dim)")
+    (n_tokens, hdim), vocab = h.shape, w.shape[0]
     ws_bytes = _lib.load().mrl_lmhead_workspace_bytes(n_tokens, vocab)
     workspace = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     args = (_lib.ptr(h), _lib.ptr(w), n_tokens, vocab, hdim, _lib.ptr(lab), _lib.dtype_code(lab),
@@ -83,8 +100,44 @@ def lmhead_logprob(hidden, weight, labels, inv_temperature=1.0, want_entropy=Tru
         _lib.call("mrl_lmhead_logprob_fwd", *args)
         end.record(stream)
         kernel_events.append(("mrl_lmhead_logprob_fwd", start, end, n_tokens))
-    ent_out = ent.view(lead) if want_entropy else torch.zeros(lead, dtype=torch.float32, device=dev)
-    return logp.view(lead), ent_out, lse.view(lead)
+
+
+class _LiveRows:
+    """The rows with a non-zero flag: how many (one host read), which, and moves there and back."""
+
+    def __init__(self, flags, dtype, stride, n, dev):
+        self.dev, self.n_all = dev, n
+        blocks = (n + 1023) // 1024
+        index = torch.empty(2 * n + blocks, dtype=torch.int32, device=dev)
+        total = torch.empty(1, dtype=torch.int64, device=dev)
+        self.live, self.place = index[:n], index[n:2 * n]
+        _lib.call("mrl_live_rows", flags if isinstance(flags, int) else _lib.ptr(flags), dtype, stride, n,
+                  index.data_ptr(), index.data_ptr() + 4 * n, index.data_ptr() + 8 * n, _lib.ptr(total), _lib.stream(dev))
+        self.n = int(total.item()) if n > 0 else 0
+
+    def gather(self, table, labels, ops):
+        """The live rows of `table` [n, W] (W whole 16-byte vectors), of `labels` [n] and - unless None - of `ops`
+        [n, 8] fp32."""
+        table = table.contiguous()
+        if table.data_ptr() % 16:
+            table = table.clone()
+        out = torch.empty((self.n, table.shape[1]), dtype=table.dtype, device=self.dev)
+        lab = torch.empty(self.n, dtype=labels.dtype, device=self.dev)
+        few = None if ops is None else torch.empty((self.n, 8), dtype=torch.float32, device=self.dev)
+        _lib.call("mrl_move_rows", _lib.ptr(self.live), self.n, _lib.ptr(table), _lib.ptr(out),
+                  table.shape[1] * table.element_size(), _lib.ptr(ops), _lib.ptr(few), 0 if ops is None else 32,
+                  _lib.ptr(labels), _lib.ptr(lab), labels.element_size(), _lib.stream(self.dev))
+        return out, lab, few
+
+    def spread(self, table, out, terms, p_terms_out):
+        """Back to all rows, zeros in the others: `table` [n_live, W] to `out`, `terms` [n_live, 8] to an address."""
+        _lib.call("mrl_move_rows", _lib.ptr(self.place), self.n_all, _lib.ptr(table), _lib.ptr(out),
+                  table.shape[1] * table.element_size(), _lib.ptr(terms), p_terms_out, 32, None, None, 0,
+                  _lib.stream(self.dev))
+
+    def spread_scalars(self, part, full):
+        _lib.call("mrl_spread_scalars", _lib.ptr(part), self.n, part.shape[0], _lib.ptr(self.place), self.n_all,
+                  _lib.ptr(full), _lib.stream(self.dev))
 
 
 def _round_up(x, to):
@@ -128,17 +181,15 @@ class _FusedLmHeadLoss(torch.autograd.Function):
         # host synchronisation per call; compact_rows=False avoids it).
         live = None
         if cfg["compact_rows"] and n_rows > 0:
-            live = torch.nonzero(row_ops.view(n_rows, 8)[:, 3] != 0).flatten()
-            if live.numel() * 20 > n_rows * 19:
+            live = _LiveRows(ops.p_ops + 12, _lib.F32, 8, n_rows, dev)
+            if live.n * 20 > n_rows * 19:
                 live = None
         all_rows, h_all = n_rows, h2d
         p_ops, p_terms = ops.p_ops, ops.p_terms
         if live is not None:
-            n_rows = live.numel()
-            h2d = h_all.index_select(0, live)
-            lab = lab.index_select(0, live)
-            row_ops = row_ops.view(all_rows, 8).index_select(0, live).reshape(-1)
-            row_terms = torch.empty(max(n_rows, 1) * 8, dtype=torch.float32, device=dev)
+            n_rows = live.n
+            h2d, lab, row_ops = live.gather(h_all, lab, row_ops.view(-1, 8))
+            row_terms = torch.empty((max(n_rows, 1), 8), dtype=torch.float32, device=dev)
             p_ops, p_terms = row_ops.data_ptr(), row_terms.data_ptr()
         chunk = max(1, min(chunk_cap, n_rows))
         # the chunk of logits: rows padded to whole k-steps of the dHidden product; the padding columns
@@ -175,10 +226,8 @@ class _FusedLmHeadLoss(torch.autograd.Function):
                    1 if c0 + rows == n_rows else 0, _lib.ptr(cut), cut_bytes, stream)
         if live is not None:
             compact_dh = d_hidden
-            d_hidden = torch.zeros_like(h_all)
-            d_hidden.index_copy_(0, live, compact_dh)
-            terms_all = ops.rows[all_rows * 8:all_rows * 16].zero_()
-            terms_all.view(all_rows, 8).index_copy_(0, live, row_terms[:n_rows * 8].view(n_rows, 8))
+            d_hidden = torch.empty_like(h_all)
+            live.spread(compact_dh, d_hidden, row_terms, ops.p_terms)
         ops.reduce(stream)
         applied = ops.applied
         ctx.save_for_backward(d_hidden, d_weight, applied)

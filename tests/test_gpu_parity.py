@@ -2700,6 +2700,38 @@ def test_split_sweeps_at_odd_vocabularies(dev, dtype, out_dtype, vocab):
             assert not dz[3].any().item()
 
 
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 70001])
+@pytest.mark.parametrize("share", [0.0, 0.6, 1.0])
+def test_live_rows(dev, n, share):
+    """The rows that count: their list and places against nonzero, gathered operands and spread results against
+    torch's indexing, from byte flags and from a strided fp32 mask; none, some and all rows live."""
+    from mindspeed_rl_amd.lmhead import _LiveRows
+    g = torch.Generator(device=dev).manual_seed(n)
+    flags = (torch.rand(n, generator=g, device=dev) < share).to(torch.uint8)
+    ops = torch.randn(n, 8, generator=g, device=dev)
+    ops[:, 3] = flags.float() * 0.5
+    want = torch.nonzero(flags).flatten()
+    table = torch.randn(n, 24, generator=g, device=dev).to(torch.bfloat16)
+    for rows in (_LiveRows(flags, _lib.U8, 1, n, dev), _LiveRows(ops.data_ptr() + 12, _lib.F32, 8, n, dev)):
+        assert rows.n == want.numel() and torch.equal(rows.live[:rows.n].long(), want)
+        place = torch.full((n,), -1, dtype=torch.int32, device=dev)
+        place[want] = torch.arange(rows.n, dtype=torch.int32, device=dev)
+        assert torch.equal(rows.place, place)
+        for labels in (torch.arange(n, device=dev), torch.arange(n, dtype=torch.int32, device=dev)):
+            t, y, o = rows.gather(table, labels, ops)
+            assert torch.equal(t, table[want]) and torch.equal(y, labels[want]) and torch.equal(o, ops[want])
+        back, terms = torch.full_like(table, 7.0), torch.full_like(ops, 7.0)
+        rows.spread(t, back, o, terms.data_ptr())
+        keep = flags.bool()[:, None]
+        assert torch.equal(back, table * keep) and torch.equal(terms, torch.where(keep, ops, torch.zeros_like(ops)))
+        full = torch.full((3, n), 7.0, device=dev)
+        part = torch.randn(3, max(rows.n, 1), generator=g, device=dev)[:, :rows.n].contiguous()
+        rows.spread_scalars(part, full)
+        ref = torch.zeros(3, n, device=dev)
+        ref[:, want] = part
+        assert torch.equal(full, ref)
+
+
 @pytest.mark.parametrize("n_columns", [1, 16, 19])
 def test_ragged_columns_together(dev, n_columns):
     """Columns of every element size, one- and two-dimensional, with lengths of their own (zeros, a single
