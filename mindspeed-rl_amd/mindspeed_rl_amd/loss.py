@@ -435,7 +435,8 @@ class StandardLogProbComputer(LogProbComputer):
                                                           want_entropy=None if skip_entropy else True,
                                                           row_active=active,
                                                           grad_inplace=bool(kwargs.get("grad_inplace", False)))
-        if windows is not None and not log_probs.requires_grad:
+        own_cut = self._get_log_probs_remove_prompt_pad is StandardLogProbComputer._get_log_probs_remove_prompt_pad
+        if windows is not None and own_cut and not log_probs.requires_grad:
             return windows.cut(log_probs, None if skip_entropy else entropy)
         if kwargs.get("use_remove_padding", False):
             seqlens = kwargs.get("seqlens_in_batch", None)

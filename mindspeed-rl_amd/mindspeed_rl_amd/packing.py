@@ -246,7 +246,7 @@ class ResponseWindows:
         else:
             self.layout, self.n_seq, self.padded = 1, lead[0], lead[1]
             self.n_rows, self.seqlens, self.cu = lead[0] * lead[1], None, None
-            if self.prompt.dim() != 2 or self.resp.dim() != 2:
+            if tuple(self.prompt.shape) != (self.n_seq, 1) or tuple(self.resp.shape) != (self.n_seq, 1):
                 raise ValueError("prompt_length and response_length must have shape (mbs, 1)")
             self.resp = _as_index(self.resp)
         self.prompt = _as_index(self.prompt)

@@ -2840,6 +2840,27 @@ def test_response_windows(dev, layout, index):
         ResponseWindows((n_seq + 1, padded), b, False)
     with pytest.raises(RuntimeError):
         ResponseWindows((n_seq, padded), dict(b, prompt_length=plen), False)
+    with pytest.raises(ValueError):                     # padded: columns [B, 1], as the cut itself wants them
+        ResponseWindows((n_seq, padded), {k: v.t() if k != "responses" else v for k, v in b.items()}, False)
+
+
+def test_log_prob_computer_uses_a_subclass_cut(dev):
+    """A subclass that cuts the padded rows itself is asked to, in a pass without gradient as in one with."""
+    from mindspeed_rl_amd.loss import StandardLogProbComputer
+
+    class Negated(StandardLogProbComputer):
+        @staticmethod
+        def _get_log_probs_remove_prompt_pad(logprob, batch):
+            return -StandardLogProbComputer._get_log_probs_remove_prompt_pad(logprob, batch)
+
+    gen = torch.Generator().manual_seed(5)
+    out = torch.randn(3, 20, 640, generator=gen).to(dev)
+    b = _to_dev({"responses": torch.zeros(3, 8, dtype=torch.int64), "prompt_length": torch.tensor([[1], [4], [9]]),
+                 "response_length": torch.tensor([[8], [3], [5]]), "labels": torch.randint(0, 640, (3, 20), generator=gen)},
+                dev)
+    with torch.no_grad():
+        want, got = StandardLogProbComputer().compute(out, b, False), Negated().compute(out, b, False)
+    assert all(torch.equal(g, -w) for g, w in zip(got, want)) and want[0].any().item()
 
 
 @pytest.mark.parametrize("layout", ["padded", "packed"])
