@@ -409,9 +409,9 @@ __device__ __forceinline__ void write_masked_row_outputs(int64_t r, float* __res
 // the next unclaimed one.  With a fixed stride (row r, r + grid, ...) the workgroups drift apart and
 // the rows in flight spread over a wide stretch of memory; with tickets the rows in flight are always
 // the most recent `grid` consecutive ones, which the HBM system serves about a tenth faster.
-// The counter is the first four bytes of the caller's workspace and starts at ZERO: workgroup b
-// begins with unit b, and ticket t (the value the fetch-and-add returns) stands for unit
-// t + gridDim.x.  So "reset" means "clear": the workspace is zeroed by whoever prepares the sweep
+// The counter is the first four bytes of the caller's workspace and starts at ZERO: a ticket stands for
+// `group` consecutive units, workgroup b begins with units b * group .. + group - 1, and the value t that
+// the fetch-and-add (of group) returns stands for units t + gridDim.x * group .. + group - 1.  So "reset" means "clear": the workspace is zeroed by whoever prepares the sweep
 // (the prepare kernel of the loss, or clear_words_kernel below).
 __global__ void clear_words_kernel(unsigned long long* p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -593,9 +593,11 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     static_assert(!kWide || BLK == kWideBlock, "halves of a row are held by workgroups of kWideBlock threads");
     static_assert(!(kWide && kEdge), "a row that two workgroups hold is aligned");
     __shared__ Stats lds[BLK / 64 + 1];
-    // two slots used in turn: thread 0 may write the ticket of the following row while a slow
-    // wavefront has yet to read this one's (one barrier per row separates a slot's reuse)
+    // Two slots used in turn, one per BROADCAST: thread 0 may write the next ticket while a slow wavefront
+    // has yet to read this one's, and the barrier of the broadcast in between separates a slot's reuse.
+    // (Between two broadcasts there may be no other: rows without a mask are not reduced.)
     __shared__ uint32_t next_row[2];
+    int slot = 0;
     __shared__ Inbox inbox;                 // the other half's record (wide rows)
 
     const int tid = threadIdx.x;
@@ -623,13 +625,14 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     int64_t r = (int64_t)blockIdx.x * group;
     int left = group - 1;                   // rows of the current ticket behind r
     // the unit behind r: the next of the ticket, or the first of a new ticket (asked for in `mine`)
-    auto following = [&](uint32_t mine, int parity) {
+    auto following = [&](uint32_t mine) {
         if (left > 0) {
             --left;
             return r + 1;
         }
         left = group - 1;
-        const int64_t t = (int64_t)broadcast_ticket(mine, &next_row[parity]);
+        const int64_t t = (int64_t)broadcast_ticket(mine, &next_row[slot]);
+        slot ^= 1;
         return row_ticket ? t + (int64_t)gridDim.x * group : n_rows;
     };
     auto plan = [&](int64_t r2) {
@@ -686,7 +689,6 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         edge_bits = load_edge(first);
         zy_bits = E::load_bits(first.zy_ptr);
     }
-    int parity = 0;
     while (r < n_rows) {
         const int64_t row = kWide ? (r >> 1) : r;
         const int half = kWide ? (int)(r & 1) : 0;
@@ -730,7 +732,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
                 // them: it is older than every store, so waiting for it does not wait for them
                 const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset(), (uint32_t)group);
                 grad_part<DT, BLK, kEntropy, 0, H>(v, g, dst);
-                nx = plan(following(mine, parity));
+                nx = plan(following(mine));
                 load_part<BLK, 0, H>(v, nx.row);
                 grad_part<DT, BLK, kEntropy, H, NV>(v, g, dst);
                 if (kEdge) E::buf_store(mrl::make_rsrc(drow, unit_bytes[0]), edge_off, grad_elem<kEntropy>(g, z_edge));
@@ -746,7 +748,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         if (!wrote) {                       // no gradient for this row: zeros, same order of operations
             const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset(), (uint32_t)group);
             zero_part<BLK, 0, H>(dst);
-            nx = plan(following(mine, parity));
+            nx = plan(following(mine));
             load_part<BLK, 0, H>(v, nx.row);
             zero_part<BLK, H, NV>(dst);
             if (kEdge) E::buf_store(mrl::make_rsrc(drow, unit_bytes[0]), edge_off, 0.f);
@@ -759,7 +761,6 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         zy_bits = zy_next;
         edge_bits = edge_next;
         r = nx.r;
-        parity ^= 1;
     }
 }
 

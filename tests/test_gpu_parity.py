@@ -1221,6 +1221,29 @@ def test_fused_sweep_rows_per_ticket(dev, rows, vocab):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("rows,vocab", [(16390, 4096), (9001, 12291), (2500, 24576)])     # 4, 2 and 1 rows per ticket
+@pytest.mark.parametrize("runs", ["whole_tickets", "from_inside_a_ticket", "prompts", "all"])
+def test_fused_sweep_tickets_of_masked_rows(dev, rows, vocab, runs):
+    """Rows without a mask are not reduced, so through a run of them (a prompt, padding) a workgroup takes
+    ticket after ticket with no barrier but those of the tickets themselves: every row still comes out as a
+    workgroup of its own delivers it, bit for bit, and a masked row as zeros."""
+    z, y, ops = _raw_fused_case(dev, rows, rows, vocab)
+    r = torch.arange(rows, device=dev)
+    live = {"whole_tickets": (r // 4) % 5 == 0,                         # 16 masked rows, 4 live ones
+            "from_inside_a_ticket": (r % 37) < 3,                       # 34 masked rows from anywhere on
+            "prompts": (r % 1500) >= 1400,
+            "all": r < 0}[runs]
+    ops[:, 3] = live.float()
+    outs = [(torch.full_like(z, 7.0), torch.empty(rows, device=dev), torch.full((rows, 8), 7.0, device=dev)) for _ in range(2)]
+    _raw_fused_sweep(z, y, ops, *outs[0], _lib.stream(dev), torch.empty(4, dtype=torch.int32, device=dev))
+    _raw_fused_sweep(z, y, ops, *outs[1], _lib.stream(dev), None)
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    dz, _, terms = outs[0]
+    assert not dz[~live].any().item() and not terms[~live].any().item()
+    assert bool(terms[live, 5].all().item())                            # the mask, of every live row
+
+
 @pytest.mark.parametrize("dtype,vocab", [(torch.float32, 152064), (torch.bfloat16, 262144)])
 def test_fused_sweep_wide_rows(dev, dtype, vocab):
     """Rows that two workgroups hold: more half rows than workgroups (tickets are recycled, partners
