@@ -410,6 +410,21 @@ int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int64_t n_rows,
                            float* row_terms, void* workspace, int64_t workspace_bytes,
                            int workspace_cleared, void* stream);
 
+/* The gradients of step 2 once more, at another scale, and the book-keeping of mrl_grad_scale_note:
+ * dlogits = grad_scale * (*upstream) * d(loss)/d(logits), taken from the logits again and rounded once.
+ * Nothing is touched if *upstream / carried[0] is exactly 1 (dlogits hold that already), unless `always`.
+ * carried, learned, rescales: as for mrl_scale_rows_note.  All other arguments as they went into
+ * mrl_fused_logprob_loss, with logits, labels and row_ops unchanged since and dlogits elsewhere.  For rows that
+ * the sweep takes at element alignment (others: MRL_ERR_UNSUPPORTED; mrl_scale_rows_note rescales them). */
+int mrl_fused_logprob_regrad(const void* logits, int logits_dtype, int64_t n_rows, int64_t vocab,
+                             int64_t row_stride, const void* labels, int labels_dtype,
+                             float inv_temperature, const float* row_ops, int has_old,
+                             float clip_lo, float clip_hi, int kl_penalty, float kl_coef,
+                             float entropy_coeff, float grad_scale, const float* upstream,
+                             float* carried, float* learned, uint32_t* rescales, int always,
+                             void* dlogits, int64_t dlogits_row_stride, void* workspace,
+                             int64_t workspace_bytes, int workspace_cleared, void* stream);
+
 /* Polls a workgroup spends waiting for the record of the other half of a wide row before it reads
  * that half itself (default 2^18; 0 = never wait, which exercises the fallback; negative restores
  * the default).  Process-wide, read at every launch; returns the previous value.  No counterpart

@@ -15,19 +15,29 @@
 
 namespace mrl {
 
+// Gradients at a new scale, *grad_scale_dev: what dlogits carry and a counter that is zero between calls, and
+// where the new scale is noted (both nullable).  Nothing is done where the two scales are equal, unless `always`.
+struct Again {
+    float* carried;
+    float* learned;
+    uint32_t* rescales;
+    int always;
+};
+
 struct FusedArgs {
     const void* logits; int dtype; int64_t n_rows, vocab, row_stride;
     const void* labels; int labels_dtype; float inv_t;
     const float* row_ops; int has_old;
     float clip_lo, clip_hi; int kl_penalty; float kl_coef, entropy_coeff, grad_scale;
     const float* grad_scale_dev;    // nullable device scalar that multiplies grad_scale
+    Again again;                    // carried not NULL: gradients only, of edge rows swept before
     void* workspace;                // nullable for narrow rows: row counter (+ half-row records)
     bool workspace_cleared;         // the caller has zeroed it on this stream
     bool wide;                      // rows cut in two halves held by two workgroups
     bool edge;                      // rows do not all start on a 128-byte line
     int64_t half_elems;             // entries of the first half
     void* dlogits; int64_t d_stride;
-    float* logp; float* entropy; float* row_terms;
+    float* logp; float* entropy; float* row_terms;     // row_terms: NULL for gradients only
     bool with_entropy;
     hipStream_t stream;
 };

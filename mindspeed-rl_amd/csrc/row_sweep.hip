@@ -404,6 +404,25 @@ __device__ __forceinline__ void write_masked_row_outputs(int64_t r, float* __res
     for (int q = 0; q < S_N; ++q) row_terms[r * S_N + q] = 0.f;
 }
 
+// Book-keeping of a backward: applied[0], the scale that the gradients carry, becomes u, and u the scale that
+// the next sweep starts from (learned, nullable) if it can be one: finite and not zero.
+__device__ __forceinline__ void note_scale(float u, float* applied, float* learned) {
+    applied[0] = u;
+    if (learned && u != 0.f && __builtin_isfinite(u)) *learned = u;
+}
+
+// The same by the workgroup that comes here last (one thread of each does): applied[1] counts them and is zero
+// again afterwards.  Every workgroup has read applied[0] before it counts itself.
+__device__ __forceinline__ void note_scale_last(float u, float* applied, float* learned, uint32_t* rescales) {
+    uint32_t* done = reinterpret_cast<uint32_t*>(applied) + 1;
+    const uint32_t before = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (before == gridDim.x - 1) {
+        if (rescales) *rescales += 1u;
+        note_scale(u, applied, learned);
+        __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // ------------------------------------------------------------------------------ row tickets
 // The persistent kernel hands out rows through a counter: a workgroup that has finished a row takes
 // the next unclaimed one.  With a fixed stride (row r, r + grid, ...) the workgroups drift apart and
@@ -578,15 +597,16 @@ __device__ __forceinline__ Stats exchange_halves(const Stats& mine, int half, Ha
 // row), short rows leave more of the register file to further workgroups.
 constexpr int waves_per_simd(int nv) { return nv <= 4 ? 8 : (nv <= 8 ? 6 : 4); }
 
-// kEdge: rows of any element alignment (see RowSpan); dlogits rows are misaligned alike.
+// kEdge: rows of any element alignment (see RowSpan); dlogits rows are misaligned alike.  Only these rows are
+// ever swept a second time (mrl_fused_logprob_regrad): again.carried is then given and row_terms NULL.
 // kWide: the units of work are half rows (see "wide rows" above): unit 2 r is the first
 // half_elems entries of row r, unit 2 r + 1 the rest; n_rows then counts units.
 template <int DT, int BLK, int NV, bool kEntropy, bool kWide, bool kEdge>
 __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persistent_kernel(
     const typename Elem<DT>::T* logits, int64_t row_stride, int vocab, int64_t n_rows,
     const void* __restrict__ labels, int labels_dtype, float inv_t, const float* __restrict__ row_ops, int has_old,
-    Params p, float grad_scale, const float* __restrict__ grad_scale_dev, typename Elem<DT>::T* dlogits,
-    int64_t d_stride, float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ row_terms,
+    Params p, float grad_scale, const float* __restrict__ grad_scale_dev, mrl::Again again,
+    typename Elem<DT>::T* dlogits, int64_t d_stride, float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ row_terms,
     unsigned int* row_ticket, int group, int half_elems, HalfRecord* half_records, uint32_t spin_limit) {
     using E = Elem<DT>;
     using T = typename E::T;
@@ -601,6 +621,17 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     __shared__ Inbox inbox;                 // the other half's record (wide rows)
 
     const int tid = threadIdx.x;
+    const bool outputs = tid == 0 && (!kEdge || row_terms != nullptr);
+    // as in scale_rows_note_kernel: equal scales are noted by workgroup 0 at once, others by whoever ends last
+    bool moved = false;
+    if (kEdge && again.carried) {
+        const float u = *grad_scale_dev;
+        moved = u / again.carried[0] != 1.f;
+        if (!moved && !again.always) {
+            if (blockIdx.x == 0 && tid == 0) note_scale(u, again.carried, again.learned);
+            return;
+        }
+    }
     // bytes and vectors of a unit: the whole row, or its first / second half
     const uint32_t unit_bytes[2] = {(uint32_t)(kWide ? half_elems : vocab) * (uint32_t)sizeof(T),
                                     (uint32_t)(kWide ? vocab - half_elems : 0) * (uint32_t)sizeof(T)};
@@ -725,7 +756,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
             }
             float lse;
             const RowScalars s = row_scalars<kEntropy>(tot, k, inv_t, y_ok, z_y, ops, has_old, p, grad_scale, m, lse);
-            if (tid == 0 && half == 0) write_row_outputs(row, s, m, logp, entropy, row_terms);
+            if (outputs && half == 0) write_row_outputs(row, s, m, logp, entropy, row_terms);
             if (s.g_lp != 0.f || s.g_h != 0.f) {
                 const RowGrad g = row_grad<kEntropy>(s, k, inv_t, lse);
                 // the ticket is asked for ahead of the stores and picked up behind the first H of
@@ -742,7 +773,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
                 zy_next = E::load_bits(nx.zy_ptr);
                 wrote = true;
             }
-        } else if (tid == 0 && half == 0) {
+        } else if (outputs && half == 0) {
             write_masked_row_outputs(row, logp, entropy, row_terms);
         }
         if (!wrote) {                       // no gradient for this row: zeros, same order of operations
@@ -762,6 +793,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         edge_bits = edge_next;
         r = nx.r;
     }
+    if (kEdge && again.carried && tid == 0) note_scale_last(*grad_scale_dev, again.carried, again.learned, moved ? again.rescales : nullptr);
 }
 
 // Backward of the split path as a plain stream: one 16-byte vector per thread, small workgroups that
@@ -872,24 +904,12 @@ __global__ __launch_bounds__(256) void scale_rows_note_kernel(typename Elem<DT>:
     const float was = applied[0];
     const float ratio = u / was;
     if (ratio == 1.f) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            applied[0] = u;
-            if (learned && u != 0.f && __builtin_isfinite(u)) *learned = u;
-        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) note_scale(u, applied, learned);
         return;
     }
     scale_rows<DT>(x, row_stride, vocab, n_rows, tail, ratio);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t* done = reinterpret_cast<uint32_t*>(applied) + 1;
-        const uint32_t before = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before == gridDim.x - 1) {
-            if (rescales) *rescales += 1u;
-            applied[0] = u;
-            __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (learned && u != 0.f && __builtin_isfinite(u)) *learned = u;
-        }
-    }
+    if (threadIdx.x == 0) note_scale_last(u, applied, learned, rescales);
 }
 
 // Book-keeping behind one or more scale_rows_kernel launches: the buffers now carry `upstream`.
@@ -899,9 +919,7 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
     const float u = *upstream;
     const float was = *applied;
     if (rescales && u / was != 1.f) *rescales += 1u;
-    *applied = u;
-    // a scale that the next sweep can start from: finite and non-zero
-    if (learned && u != 0.f && __builtin_isfinite(u)) *learned = u;
+    note_scale(u, applied, learned);
 }
 
 // ----------------------------------------------------------------------------- host dispatch
@@ -978,7 +996,7 @@ int launch_sweep(const mrl::FusedArgs& a) {
     HalfRecord* rec = kWide ? reinterpret_cast<HalfRecord*>(reinterpret_cast<char*>(a.workspace) + kWorkspaceHeader) : nullptr;
     hipLaunchKernelGGL((fused_sweep_persistent_kernel<DT, BLK, NV, kEntropy, kWide, kEdge>), dim3((unsigned)grid), dim3(BLK),
                        0, a.stream, (const T*)a.logits, a.row_stride, (int)a.vocab, units, a.labels, a.labels_dtype,
-                       a.inv_t, a.row_ops, a.has_old, p, a.grad_scale, a.grad_scale_dev, (T*)a.dlogits, a.d_stride, a.logp,
+                       a.inv_t, a.row_ops, a.has_old, p, a.grad_scale, a.grad_scale_dev, a.again, (T*)a.dlogits, a.d_stride, a.logp,
                        a.entropy, a.row_terms, counter, group, (int)a.half_elems, rec,
                        g_wide_spin_limit.load(std::memory_order_relaxed));
     return mrl::check_launch("mrl_fused_logprob_loss");
@@ -1111,6 +1129,65 @@ extern "C" int64_t mrl_set_wide_spin_limit(int64_t polls) {
     return (int64_t)g_wide_spin_limit.exchange(next, std::memory_order_relaxed);
 }
 
+// Checks and launch shared by the two entry points of the sweep.
+static int run_sweep(const char* fn, mrl::FusedArgs& a, int64_t workspace_bytes) {
+    MRL_REQUIRE(a.n_rows >= 0 && a.vocab > 0 && a.n_rows <= 0x3fffffffLL, MRL_ERR_INVALID_ARG, "%s: n_rows=%lld vocab=%lld",
+                fn, (long long)a.n_rows, (long long)a.vocab);
+    const int eb = mrl::float_dtype_bytes(a.dtype);
+    MRL_REQUIRE(eb != 0, MRL_ERR_UNSUPPORTED, "%s: logits dtype %d (want F32, BF16 or F16)", fn, a.dtype);
+    MRL_REQUIRE(mrl::int_dtype_bytes(a.labels_dtype) != 0, MRL_ERR_UNSUPPORTED, "%s: labels dtype %d (want I32 or I64)",
+                fn, a.labels_dtype);
+    MRL_REQUIRE(a.row_stride >= a.vocab && a.d_stride >= a.vocab, MRL_ERR_INVALID_ARG, "%s: row stride below vocab", fn);
+    MRL_REQUIRE(a.kl_penalty >= MRL_KL_NONE && a.kl_penalty <= MRL_KL_LOW_VAR, MRL_ERR_INVALID_ARG, "%s: kl_penalty=%d", fn,
+                a.kl_penalty);
+    MRL_REQUIRE(a.inv_t > 0.f && a.inv_t < 1.0e6f, MRL_ERR_INVALID_ARG, "%s: inv_temperature=%g must be in (0, 1e6)", fn,
+                (double)a.inv_t);
+    if (a.n_rows == 0) return MRL_OK;
+    const bool again = a.again.carried != nullptr;
+    MRL_REQUIRE(a.logits && a.labels && a.row_ops && a.dlogits && (a.row_terms || again), MRL_ERR_INVALID_ARG,
+                "%s: NULL pointer", fn);
+    MRL_REQUIRE(mrl::aligned(a.workspace, 16) && mrl::aligned(a.grad_scale_dev, 4) &&
+                    mrl::aligned(a.again.carried, 8) && mrl::aligned(a.again.learned, 4) && mrl::aligned(a.again.rescales, 4),
+                MRL_ERR_MISALIGNED, "%s: workspace must be 16-byte, a scale with its counter 8-byte and the other scalars "
+                "4-byte aligned", fn);
+    const mrl::RowLayout layout =
+        mrl::row_sweep_layout(a.dtype, a.vocab, a.logits, a.row_stride, a.dlogits, a.d_stride, a.n_rows);
+    MRL_REQUIRE(layout != mrl::RowLayout::none, MRL_ERR_UNSUPPORTED,
+                "%s: needs 16-byte aligned rows, vocab %% %d == 0 and vocab <= %lld for this dtype, or rows of 8 KiB to "
+                "half that vocab whose dlogits are misaligned alike (got vocab=%lld)", fn, 16 / eb,
+                (long long)mrl_fused_max_vocab(a.dtype), (long long)a.vocab);
+    a.edge = layout == mrl::RowLayout::edges;
+    MRL_REQUIRE(!again || a.edge, MRL_ERR_UNSUPPORTED, "%s: rows of whole aligned vectors are not swept again", fn);
+    if (a.dlogits != a.logits) {
+        const char* x = (const char*)a.logits;
+        const char* y = (const char*)a.dlogits;
+        const int64_t xb = ((a.n_rows - 1) * a.row_stride + a.vocab) * eb, yb = ((a.n_rows - 1) * a.d_stride + a.vocab) * eb;
+        MRL_REQUIRE(x + xb <= y || y + yb <= x, MRL_ERR_INVALID_ARG, "%s: dlogits partially overlaps logits", fn);
+    } else {
+        MRL_REQUIRE(!again, MRL_ERR_INVALID_ARG, "%s: the logits have been overwritten", fn);
+        MRL_REQUIRE(a.d_stride == a.row_stride, MRL_ERR_INVALID_ARG, "%s: in-place needs identical strides", fn);
+    }
+    const int64_t n_vec = a.vocab / (16 / eb);
+    Shape shape = pick_shape(a.dtype, n_vec);
+    a.wide = shape == kTooLong;
+    a.half_elems = 0;
+    if (a.wide) {
+        a.half_elems = (n_vec + 1) / 2 * (16 / eb);
+        shape = pick_shape(a.dtype, (n_vec + 1) / 2);
+    }
+    if (a.workspace != nullptr || a.wide) {
+        const int64_t need = a.wide ? mrl_fused_workspace_bytes(a.dtype, a.n_rows, a.vocab) : kWorkspaceHeader;
+        MRL_REQUIRE(a.workspace != nullptr && workspace_bytes >= need, MRL_ERR_INVALID_ARG,
+                    "%s: workspace of %lld bytes, need %lld (rows of this width are cut in two halves that exchange "
+                    "their statistics through it)", fn, (long long)(a.workspace ? workspace_bytes : 0), (long long)need);
+    }
+    switch (a.dtype) {
+        case MRL_F32: return fused_by_shape<MRL_F32>(shape, a);
+        case MRL_BF16: return fused_by_shape<MRL_BF16>(shape, a);
+        default: return fused_by_shape<MRL_F16>(shape, a);
+    }
+}
+
 extern "C" int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int64_t n_rows, int64_t vocab,
                                       int64_t row_stride, const void* labels, int labels_dtype,
                                       float inv_temperature, const float* row_ops, int has_old, float clip_lo,
@@ -1119,38 +1196,7 @@ extern "C" int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int6
                                       int64_t dlogits_row_stride, float* logp, float* entropy, float* row_terms,
                                       void* workspace, int64_t workspace_bytes, int workspace_cleared,
                                       void* stream) {
-    const char* fn = "mrl_fused_logprob_loss";
-    MRL_REQUIRE(n_rows >= 0 && vocab > 0 && n_rows <= 0x3fffffffLL, MRL_ERR_INVALID_ARG, "%s: n_rows=%lld vocab=%lld",
-                fn, (long long)n_rows, (long long)vocab);
-    const int eb = mrl::float_dtype_bytes(logits_dtype);
-    MRL_REQUIRE(eb != 0, MRL_ERR_UNSUPPORTED, "%s: logits dtype %d (want F32, BF16 or F16)", fn, logits_dtype);
-    MRL_REQUIRE(mrl::int_dtype_bytes(labels_dtype) != 0, MRL_ERR_UNSUPPORTED, "%s: labels dtype %d (want I32 or I64)",
-                fn, labels_dtype);
-    MRL_REQUIRE(row_stride >= vocab && dlogits_row_stride >= vocab, MRL_ERR_INVALID_ARG, "%s: row stride below vocab",
-                fn);
-    MRL_REQUIRE(kl_penalty >= MRL_KL_NONE && kl_penalty <= MRL_KL_LOW_VAR, MRL_ERR_INVALID_ARG, "%s: kl_penalty=%d", fn,
-                kl_penalty);
-    MRL_REQUIRE(inv_temperature > 0.f && inv_temperature < 1.0e6f, MRL_ERR_INVALID_ARG,
-                "%s: inv_temperature=%g must be in (0, 1e6)", fn, (double)inv_temperature);
-    if (n_rows == 0) return MRL_OK;
-    MRL_REQUIRE(logits && labels && row_ops && dlogits && row_terms, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
-    MRL_REQUIRE(mrl::aligned(workspace, 16) && mrl::aligned(grad_scale_dev, 4), MRL_ERR_MISALIGNED,
-                "%s: workspace must be 16-byte and grad_scale_dev 4-byte aligned", fn);
-    const mrl::RowLayout layout =
-        mrl::row_sweep_layout(logits_dtype, vocab, logits, row_stride, dlogits, dlogits_row_stride, n_rows);
-    MRL_REQUIRE(layout != mrl::RowLayout::none, MRL_ERR_UNSUPPORTED,
-                "%s: needs 16-byte aligned rows, vocab %% %d == 0 and vocab <= %lld for this dtype, or rows of 8 KiB to "
-                "half that vocab whose dlogits are misaligned alike (got vocab=%lld)", fn, 16 / eb,
-                (long long)mrl_fused_max_vocab(logits_dtype), (long long)vocab);
-    if (dlogits != logits) {
-        const char* x = (const char*)logits;
-        const char* y = (const char*)dlogits;
-        const int64_t xb = ((n_rows - 1) * row_stride + vocab) * eb, yb = ((n_rows - 1) * dlogits_row_stride + vocab) * eb;
-        MRL_REQUIRE(x + xb <= y || y + yb <= x, MRL_ERR_INVALID_ARG, "%s: dlogits partially overlaps logits", fn);
-    } else {
-        MRL_REQUIRE(dlogits_row_stride == row_stride, MRL_ERR_INVALID_ARG, "%s: in-place needs identical strides", fn);
-    }
-    mrl::FusedArgs a;
+    mrl::FusedArgs a = {};
     a.logits = logits; a.dtype = logits_dtype; a.n_rows = n_rows; a.vocab = vocab; a.row_stride = row_stride;
     a.labels = labels; a.labels_dtype = labels_dtype; a.inv_t = inv_temperature; a.row_ops = row_ops;
     a.has_old = has_old; a.clip_lo = clip_lo; a.clip_hi = clip_hi; a.kl_penalty = kl_penalty; a.kl_coef = kl_coef;
@@ -1158,26 +1204,28 @@ extern "C" int mrl_fused_logprob_loss(const void* logits, int logits_dtype, int6
     a.workspace = workspace; a.workspace_cleared = workspace_cleared != 0; a.dlogits = dlogits; a.d_stride = dlogits_row_stride;
     a.logp = logp; a.entropy = entropy; a.row_terms = row_terms; a.with_entropy = (entropy != nullptr);
     a.stream = mrl::as_stream(stream);
-    const int64_t n_vec = vocab / (16 / eb);
-    a.edge = layout == mrl::RowLayout::edges;
-    Shape shape = pick_shape(logits_dtype, n_vec);
-    a.wide = shape == kTooLong;
-    a.half_elems = 0;
-    if (a.wide) {
-        a.half_elems = (n_vec + 1) / 2 * (16 / eb);
-        shape = pick_shape(logits_dtype, (n_vec + 1) / 2);
-    }
-    if (workspace != nullptr || a.wide) {
-        const int64_t need = a.wide ? mrl_fused_workspace_bytes(logits_dtype, n_rows, vocab) : kWorkspaceHeader;
-        MRL_REQUIRE(workspace != nullptr && workspace_bytes >= need, MRL_ERR_INVALID_ARG,
-                    "%s: workspace of %lld bytes, need %lld (rows of this width are cut in two halves that exchange "
-                    "their statistics through it)", fn, (long long)(workspace ? workspace_bytes : 0), (long long)need);
-    }
-    switch (logits_dtype) {
-        case MRL_F32: return fused_by_shape<MRL_F32>(shape, a);
-        case MRL_BF16: return fused_by_shape<MRL_BF16>(shape, a);
-        default: return fused_by_shape<MRL_F16>(shape, a);
-    }
+    return run_sweep("mrl_fused_logprob_loss", a, workspace_bytes);
+}
+
+extern "C" int mrl_fused_logprob_regrad(const void* logits, int logits_dtype, int64_t n_rows, int64_t vocab,
+                                        int64_t row_stride, const void* labels, int labels_dtype,
+                                        float inv_temperature, const float* row_ops, int has_old, float clip_lo,
+                                        float clip_hi, int kl_penalty, float kl_coef, float entropy_coeff,
+                                        float grad_scale, const float* upstream, float* carried, float* learned,
+                                        uint32_t* rescales, int always, void* dlogits, int64_t dlogits_row_stride, void* workspace, int64_t workspace_bytes,
+                                        int workspace_cleared, void* stream) {
+    const char* fn = "mrl_fused_logprob_regrad";
+    MRL_REQUIRE(n_rows == 0 || (upstream && carried), MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    mrl::FusedArgs a = {};
+    a.logits = logits; a.dtype = logits_dtype; a.n_rows = n_rows; a.vocab = vocab; a.row_stride = row_stride;
+    a.labels = labels; a.labels_dtype = labels_dtype; a.inv_t = inv_temperature; a.row_ops = row_ops;
+    a.has_old = has_old; a.clip_lo = clip_lo; a.clip_hi = clip_hi; a.kl_penalty = kl_penalty; a.kl_coef = kl_coef;
+    a.entropy_coeff = entropy_coeff; a.grad_scale = grad_scale; a.grad_scale_dev = upstream;
+    a.again = {carried, learned, rescales, always};
+    a.workspace = workspace; a.workspace_cleared = workspace_cleared != 0; a.dlogits = dlogits; a.d_stride = dlogits_row_stride;
+    a.with_entropy = entropy_coeff != 0.f;
+    a.stream = mrl::as_stream(stream);
+    return run_sweep(fn, a, workspace_bytes);
 }
 
 // Dense rows of an odd vocabulary are one stretch of entries: cut into rows of 2048 (fewer when there are

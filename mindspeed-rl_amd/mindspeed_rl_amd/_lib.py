@@ -72,6 +72,8 @@ SIGNATURES = {
     "mrl_fused_workspace_bytes": [_int, _i64, _i64],
     "mrl_fused_logprob_loss": [_vp, _int, _i64, _i64, _i64, _vp, _int, _f32, _vp, _int, _f32, _f32, _int, _f32, _f32,
                                _f32, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _int, _vp],
+    "mrl_fused_logprob_regrad": [_vp, _int, _i64, _i64, _i64, _vp, _int, _f32, _vp, _int, _f32, _f32, _int, _f32, _f32,
+                                 _f32, _vp, _vp, _vp, _vp, _int, _vp, _i64, _vp, _i64, _int, _vp],
     "mrl_set_wide_spin_limit": [_i64],
     "mrl_fused_loss_reduce": [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _int, _vp, _int, _f32, _f32, _int, _f32,
                               _f32, _int, _f32, _vp, _vp, _vp, _vp, _vp],

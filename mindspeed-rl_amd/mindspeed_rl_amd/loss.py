@@ -145,13 +145,23 @@ def policy_loss(log_prob, entropy, old_log_prob, ref_log_prob, advantages, mask=
 def fused_supported(output, grad_inplace=False):
     """True if the row-in-registers kernel can take these logits: a floating dtype it knows, a
     16-byte aligned dense tensor and a vocabulary that fits the register files of one workgroup or - if
-    it is a whole number of 16-byte vectors - of two (other vocabularies from 8 KiB a row on).  (``grad_inplace`` is accepted for call compatibility: every supported shape can
-    also be swept in place.)"""
+    it is a whole number of 16-byte vectors - of two (other vocabularies from 8 KiB a row on).  With
+    ``grad_inplace`` only whole vectors: see :func:`_swept_again`."""
     if output.dtype not in (torch.float32, torch.bfloat16, torch.float16) or not output.is_cuda:
         return False
     if _lib.load().mrl_fused_workspace_bytes(_lib.dtype_code(output), 1, output.shape[-1]) == 0:
         return False
+    if grad_inplace and _swept_again(output):
+        return False
     return output.is_contiguous() and output.data_ptr() % 16 == 0
+
+
+def _swept_again(output):
+    """True for rows that are not whole 16-byte vectors.  Their gradients are never rescaled in the logits'
+    dtype: a backward whose scale the sweep did not know takes them from the logits once more (any scale is
+    applied in fp32 and rounded once, as on the split path, which these rows take where the sweep cannot).  So
+    the logits have to be there until the backward, and in place the caller has to state the scale."""
+    return output.shape[-1] % (16 // output.element_size()) != 0
 
 
 class GradScaleState:
@@ -210,6 +220,31 @@ def _deliver_eager_grads(ctx, buffers, applied, state, g_loss):
     return buffers
 
 
+def _deliver_swept_grads(ctx, dlogits, flat, lab, rows, small, state, g_loss):
+    """The same for rows that are swept again: at another scale than ``dlogits`` carry the gradients come from
+    the logits, so nothing that an earlier backward was given can spoil them."""
+    dev = flat.device
+    upstream = g_loss.to(torch.float32).reshape(1).contiguous()
+    shape, scalars, o_applied, o_workspace, ws_bytes = ctx.sweep
+    first = not ctx.handed_out
+    ctx.handed_out = True
+    p_applied = small.data_ptr() + o_applied
+    if not first:                       # what was handed out stays; its workspace has been used
+        dlogits = torch.empty_like(flat)
+        applied = small[o_applied:o_applied + 8].clone()
+        p_applied = applied.data_ptr()
+    learned = _lib.ptr(state.learned) if state is not None else None
+    rescales = _lib.ptr(state.rescales) if state is not None else None
+    if flat.shape[0] == 0:
+        _lib.call("mrl_grad_scale_note", _lib.ptr(upstream), p_applied, learned, rescales, _lib.stream(dev))
+        return dlogits
+    vocab_ops._timed_call("mrl_fused_logprob_regrad", shape[1], dev, flat.data_ptr(), *shape, lab.data_ptr(),
+                          _lib.dtype_code(lab), scalars[0], rows.data_ptr(), *scalars[1:], upstream.data_ptr(), p_applied,
+                          learned, rescales, 0 if first else 1, dlogits.data_ptr(), shape[2], small.data_ptr() + o_workspace,
+                          ws_bytes, 1 if first else 0, _lib.stream(dev))
+    return dlogits
+
+
 def _align(n, to):
     return (n + to - 1) // to * to
 
@@ -221,7 +256,8 @@ class _FusedOperands:
     scalars, the gradient scale with its counter, the sweep's workspace) and the per-row operands and
     terms in a second one; the kernels get addresses inside them."""
 
-    def __init__(self, dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, sweep_dtype_code, vocab, sweep_rows):
+    def __init__(self, dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, sweep_dtype_code, vocab, sweep_rows,
+                 sweeps=1):
         lib = _lib.load()
 
         f32, i32 = torch.float32, torch.int32
@@ -240,11 +276,12 @@ class _FusedOperands:
         # the sweep's workspace is sized for the largest launch (a chunk, for the lm_head step)
         # (at least its 16-byte header, whose second word the reduce step borrows as its counter)
         self.ws_bytes = max(16, lib.mrl_fused_workspace_bytes(sweep_dtype_code, sweep_rows, vocab))
+        self.cleared_bytes = self.ws_bytes * sweeps     # one for each sweep over the rows
         seqs = max(n_seq, 1)
         o_out = 0                                   # float[8]
         o_applied = 32                              # float[2]
         o_ws = 48                                   # the sweep workspace, 16-byte aligned
-        o_start = _align(o_ws + self.ws_bytes, 16)  # int64[n_seq]
+        o_start = _align(o_ws + self.cleared_bytes, 16)  # int64[n_seq]
         o_sums = o_start + 8 * seqs                 # float[n_seq * 8]
         o_count = o_sums + 32 * seqs                # int32[n_seq]
         o_msum = o_count + 4 * seqs                 # float[n_seq]
@@ -252,7 +289,7 @@ class _FusedOperands:
         base = self.small.data_ptr()
         self.out = self.small[o_out:o_out + 32].view(torch.float32)
         self.applied = self.small[o_applied:o_applied + 8].view(torch.float32)
-        self.workspace = base + o_ws
+        self.workspace, self.o_applied, self.o_second = base + o_ws, o_applied, o_ws + self.ws_bytes
         self.p_start, self.p_sums, self.p_count, self.p_msum = base + o_start, base + o_sums, base + o_count, base + o_msum
         self.rows = torch.empty(max(n_rows, 1) * 16, dtype=torch.float32, device=dev)
         self.p_ops = self.rows.data_ptr()
@@ -266,7 +303,7 @@ class _FusedOperands:
                   _lib.ptr(self.cu), self.padded_s, _lib.ptr(self.prompt), self.pdt, _lib.ptr(self.resp), self.rdt,
                   _lib.ptr(self.old), _lib.ptr(self.ref), _lib.ptr(self.adv), _lib.ptr(self.mask_t), self.mdt,
                   cfg["seq_mean"], self.p_start, self.p_count, self.p_msum, self.p_ops,
-                  self.workspace if self.n_rows > 0 else None, self.ws_bytes if self.n_rows > 0 else 0,
+                  self.workspace if self.n_rows > 0 else None, self.cleared_bytes if self.n_rows > 0 else 0,
                   _lib.ptr(scale_dev), scale_host, _lib.ptr(self.applied) if self.n_rows > 0 else None, stream)
         if self.n_rows == 0:
             self.applied[0] = scale_host if scale_dev is None else scale_dev[0] * scale_host
@@ -288,7 +325,8 @@ class _FusedLogprobLoss(torch.autograd.Function):
     the [T, V] tensor for forward + backward).  The backward only rescales the stored dlogits if
     the upstream gradient differs from the scale they already carry (kept in a device scalar, so
     a second backward over a retained graph rescales by the ratio of the two upstream values).
-    Three launches in the forward (prepare, sweep, reduce) and one in the backward."""
+    Three launches in the forward (prepare, sweep, reduce) and one in the backward.  Rows that are
+    not whole vectors are swept again instead of rescaled (:func:`_swept_again`)."""
 
     @staticmethod
     def forward(ctx, output, labels, batch, cfg):
@@ -302,20 +340,26 @@ class _FusedLogprobLoss(torch.autograd.Function):
         lab = lab.contiguous()
         n_seq, width = batch["responses"].shape[0], batch["responses"].shape[-1]
         layout, padded_s = (0, 0) if cfg["packed"] else (1, output.shape[1])
+        again = _swept_again(flat) and not cfg["grad_inplace"]
         ops = _FusedOperands(dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, _lib.dtype_code(flat), vocab,
-                             n_rows)
+                             n_rows, sweeps=2 if again else 1)
         ent = torch.empty(n_rows, dtype=torch.float32, device=dev) if cfg["entropy_coeff"] != 0 else None
         dlogits = flat if cfg["grad_inplace"] else torch.empty_like(flat)
         stream = _lib.stream(dev)
         ops.prepare(stream)
-        vocab_ops._timed_call("mrl_fused_logprob_loss", n_rows, dev, _lib.ptr(flat), _lib.dtype_code(flat), n_rows,
-                              vocab, vocab, _lib.ptr(lab), _lib.dtype_code(lab), cfg["inv_temperature"],
-                              ops.p_ops, 0 if ops.old is None else 1, cfg["clip_lo"], cfg["clip_hi"],
-                              cfg["kl_penalty"], cfg["kl_coef"], cfg["entropy_coeff"], cfg["loss_scale"],
-                              _lib.ptr(ops.applied), _lib.ptr(dlogits), vocab, None, _lib.ptr(ent), ops.p_terms,
-                              ops.workspace, ops.ws_bytes, 1, stream)
+        shape = (_lib.dtype_code(flat), n_rows, vocab, vocab)
+        scalars = (cfg["inv_temperature"], 0 if ops.old is None else 1, cfg["clip_lo"], cfg["clip_hi"], cfg["kl_penalty"],
+                   cfg["kl_coef"], cfg["entropy_coeff"], cfg["loss_scale"])
+        vocab_ops._timed_call("mrl_fused_logprob_loss", n_rows, dev, _lib.ptr(flat), *shape, _lib.ptr(lab),
+                              _lib.dtype_code(lab), scalars[0], ops.p_ops, *scalars[1:], _lib.ptr(ops.applied),
+                              _lib.ptr(dlogits), vocab, None, _lib.ptr(ent), ops.p_terms, ops.workspace, ops.ws_bytes, 1,
+                              stream)
         ops.reduce(stream)
-        ctx.save_for_backward(dlogits, ops.applied)
+        if again:
+            ctx.save_for_backward(dlogits, flat, lab, ops.rows, ops.small)
+            ctx.sweep = (shape, scalars, ops.o_applied, ops.o_second, ops.ws_bytes)
+        else:
+            ctx.save_for_backward(dlogits, ops.applied)
         ctx.meta = (tuple(output.shape), cfg.get("scale_state"))
         ctx.handed_out = False
         ctx.mark_non_differentiable(ops.out)
@@ -326,9 +370,11 @@ class _FusedLogprobLoss(torch.autograd.Function):
     def backward(ctx, g_loss, _g_out):
         if g_loss is None:
             return None, None, None, None
-        dlogits, applied = ctx.saved_tensors
-        shape, state = ctx.meta
-        (grad,) = _deliver_eager_grads(ctx, (dlogits,), applied, state, g_loss)
+        saved, (shape, state) = ctx.saved_tensors, ctx.meta
+        if len(saved) > 2:
+            grad = _deliver_swept_grads(ctx, *saved, state, g_loss)
+        else:
+            (grad,) = _deliver_eager_grads(ctx, saved[:1], saved[1], state, g_loss)
         return grad.view(shape), None, None, None
 
 
@@ -351,6 +397,9 @@ def fused_logprob_policy_loss(output, batch, *, packed, seqlens=None, cu_seqlens
         kl_code = _lib.KL_BY_NAME[kl_penalty]
     else:
         raise NotImplementedError
+    if grad_inplace and expected_upstream is None and _swept_again(output):
+        raise ValueError("grad_inplace=True needs expected_upstream= for a vocabulary of %d: rows that are not whole "
+                         "16-byte vectors take their gradients at another scale from the logits" % output.shape[-1])
     cfg = dict(packed=bool(packed), seqlens=seqlens, cu=cu_seqlens, mask=mask, ref_log_prob=ref_log_prob,
                clip_lo=float(1.0 - clip_low), clip_hi=float(1.0 + clip_high), kl_penalty=kl_code,
                kl_coef=float(kl_coef), entropy_coeff=float(entropy_coeff), seq_mean=0 if token_level_loss else 1,
@@ -368,8 +417,8 @@ def _use_fused(output, kwargs):
     injected = vocab_ops.get_vocab_parallel()
     if injected is not None and injected is not vocab_ops.vocab_parallel_cross_entropy:
         return False            # a caller's own cross entropy must be the one that scores the rows
-    return (torch.is_grad_enabled() and output.requires_grad
-            and fused_supported(output, bool(kwargs.get("grad_inplace", False))))
+    inplace = bool(kwargs.get("grad_inplace", False)) and kwargs.get("expected_grad_scale") is None
+    return torch.is_grad_enabled() and output.requires_grad and fused_supported(output, inplace)
 
 
 def _fused_kwargs(kwargs, scale_state=None):

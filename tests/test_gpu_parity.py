@@ -1209,6 +1209,60 @@ def test_fused_sweep_rows_off_a_line(dev, dtype, vocab):
     assert got2.item() == got.item() and torch.equal(dz2, dz)
 
 
+@pytest.mark.parametrize("dtype,vocab,upstream", [(torch.bfloat16, 4097, 1.0 / 3.0), (torch.float16, 32003, 65536.0),
+                                                  (torch.float16, 8193 * 8 + 1, 1024.0 / 3.0), (torch.float32, 2051, 1.0 / 3.0),
+                                                  (torch.bfloat16, 12289 * 8 + 1, 5.0)])
+@pytest.mark.parametrize("entropy_coeff", [0.0, 0.001])
+def test_odd_rows_round_their_gradient_once(dev, dtype, vocab, upstream, entropy_coeff):
+    """Rows that are not whole 16-byte vectors, back-propagated at a scale that the sweep did not know (the
+    first backward of a loss object, a changed loss scale): the scale is applied in fp32 and the gradient
+    rounded once, so it is as far from the exact one as the split kernels' - which it replaces - and not
+    further, and an fp16 gradient that needs its loss scale to be representable has it.  The same holds for
+    every further backward over the graph, after an infinite one too."""
+    gen = torch.Generator().manual_seed(vocab)
+    logits, b, kw, _, _ = _make_batch(gen, 1, 4, 5, 9, vocab, dtype, 1.0, 1, prompt_hi=2)
+    b["advantages"] = torch.randn(b["advantages"].shape, generator=gen) / 60.0      # as a mean over 2 000 tokens has it
+    meta = dict(clip_ratio=0.2, kl_coef=0.0, kl_penalty="low_var_kl", entropy_coeff=entropy_coeff / 60.0)
+    zo = logits.double().requires_grad_()
+    (exact,) = torch.autograd.grad(o_loss.grpo_compute_loss(zo, {k: v.double() if v.is_floating_point() else v for k, v in b.items()},
+                                                            meta, **kw)[0] * upstream, zo)
+    f = mrl.GRPOActorLossFunc()
+    f.add_loss_meta_info({"clip_ratio": 0.2, "kl_ctrl": mrl.FixedKLController(0.0), "kl_penalty": "low_var_kl",
+                          "entropy_coeff": entropy_coeff / 60.0})
+    bd, kwd = _to_dev(b, dev), _to_dev(kw, dev)
+    state = f.grad_scale_state(dev)
+
+    def error(dz):
+        assert torch.isfinite(dz).all().item()
+        return ((dz.double().cpu() - exact).norm() / exact.norm()).item(), (dz == 0).sum().item()
+
+    z = logits.to(dev).requires_grad_()
+    split_err, split_zeros = error(torch.autograd.grad(f.compute_loss(z, bd, fused=False, **kwd)[0] * upstream, z)[0])
+    assert mrl.fused_supported(z)
+    loss, _ = f.compute_loss(z, bd, **kwd)
+    (unknown,) = torch.autograd.grad(loss * upstream, z, retain_graph=True)
+    kept = unknown.clone()
+    (known,) = torch.autograd.grad(f.compute_loss(z, bd, **kwd)[0] * upstream, z)
+    assert state.rescales.item() == 1 and state.learned.item() == torch.tensor(upstream).item()
+    # both paths round the same fp32 values once; the fp32 values themselves differ by a few 2^-24 of the row's sums
+    err, zeros = error(unknown)
+    assert err <= split_err * 1.01 + 2.0 ** -20, (err, split_err)
+    assert abs(zeros - split_zeros) <= unknown.numel() // 1000
+    assert torch.equal(unknown, known)                          # whether the sweep knew the scale makes no difference
+    (inf,) = torch.autograd.grad(loss * float("inf"), z, retain_graph=True)
+    assert not torch.isfinite(inf[unknown != 0]).any().item()
+    (again,) = torch.autograd.grad(loss * upstream, z)
+    assert torch.equal(again, kept) and torch.equal(unknown, kept) and again.data_ptr() != unknown.data_ptr()
+    # in place the logits are gone by then: the split kernels, unless the caller states the scale
+    assert not mrl.fused_supported(z, True)
+    z2 = logits.to(dev).requires_grad_()
+    (dz2,) = torch.autograd.grad(f.compute_loss(z2 * 1.0, bd, grad_inplace=True, **kwd)[0] * upstream, z2)
+    assert error(dz2)[0] <= split_err * 1.01 + 2.0 ** -20
+    with pytest.raises(ValueError, match="expected_upstream"):
+        mrl.fused_logprob_policy_loss(z2 * 1.0, bd, packed=True, seqlens=kwd["seqlens_in_batch"], clip_low=0.2, clip_high=0.2,
+                                      cu_seqlens=kwd["cu_seqlens_padded"], grad_inplace=True)
+
+
 @pytest.mark.parametrize("rows,vocab", [(513, 4096), (4098, 4097), (2050, 8200), (1021, 16392), (1300, 32003), (600, 49153)])
 def test_fused_sweep_rows_per_ticket(dev, rows, vocab):
     """Workgroups that take one, two or four rows with a ticket, more rows than fit on the chip at once: every

@@ -123,6 +123,10 @@ def test_argument_validation_launches_nothing():
                                       None, p, 64, None, None, p, None, 0, 0, None) == -1  # no row operands
     assert lib.mrl_fused_logprob_loss(p, _lib.BF16, 2, 64, 64, p, _lib.I64, 1.0, p, 1, 0.8, 1.2, 4, 0.0, 0.0, 1.0,
                                       None, p, 64, None, None, p, p + 2, 16, 0, None) == -3  # misaligned workspace
+    # the gradients once more: rows off whole vectors only, not over the logits, an upstream gradient
+    for vocab, upstream, out, want in ((64, p, p + (1 << 20), -2), (4097, p, p, -1), (4097, None, p + (1 << 20), -1)):
+        assert lib.mrl_fused_logprob_regrad(p, _lib.BF16, 2, vocab, vocab, p, _lib.I64, 1.0, p, 1, 0.8, 1.2, 4, 0.0, 0.0, 1.0,
+                                            upstream, p, None, None, 0, out, vocab, None, 0, 0, None) == want
     assert lib.mrl_scale_rows(p, _lib.I32, 2, 64, 64, p, p, None) == -2
     assert lib.mrl_scale_rows(p, _lib.BF16, 2, 64, 64, p, None, None) == -1                # no applied scale
     assert lib.mrl_grad_scale_note(p, None, None, None, None) == -1
