@@ -619,18 +619,18 @@ int mrl_value_loss_bwd(const float* vpreds, const float* returns, const float* v
 /* The same loss from the value head's output itself, [batch, padded_s] fp32, without a copy of the response
  * windows (critic_loss_func.py:47-80): token j of sample i is element P_i - 1 + j, as far as that lies in
  * the window [P - 1, P + R - 1) clamped to the row; a token of the mask (j < response_length) outside it has
- * the value 0 and no gradient.  Forward: as mrl_value_loss_fwd_split, with its workspace.  Backward: g_head
- * [batch, padded_s], zero outside the windows. */
+ * the value 0 and no gradient.  Forward: as mrl_value_loss_fwd_split, with its workspace; slope [batch, width]
+ * receives d(loss)/d(value) of the tokens of the mask, which is all the backward needs of the operands (they
+ * may change in between).  Backward: g_head [batch, padded_s], zero outside the windows. */
 int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
                         int prompt_dtype, const void* response_length, int response_dtype,
                         const float* returns, const float* values, int64_t width,
-                        float cliprange_value, float loss_scale, float* out, float* loss_out,
-                        void* workspace, int64_t workspace_bytes, void* stream);
-int mrl_critic_loss_bwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
+                        float cliprange_value, float loss_scale, float* slope, float* out,
+                        float* loss_out, void* workspace, int64_t workspace_bytes, void* stream);
+int mrl_critic_loss_bwd(const float* slope, int64_t batch, int64_t padded_s, const void* prompt_length,
                         int prompt_dtype, const void* response_length, int response_dtype,
-                        const float* returns, const float* values, int64_t width,
-                        float cliprange_value, float loss_scale, const float* out,
-                        const float* upstream, float* g_head, void* stream);
+                        int64_t width, float loss_scale, const float* out, const float* upstream,
+                        float* g_head, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Plain device-to-device copy kernel of n_bytes (multiple of 16, 16-byte aligned pointers);

@@ -344,7 +344,8 @@ __global__ __launch_bounds__(kReduceBlock) void value_loss_fwd_kernel(
 
 // The critic's loss reads the value head's output where it lies: with the windows cut out first and scattered
 // back by the backward, five more launches and an autograd node went into 2 MB (128 x (256 + 2048) tokens: PPO
-// value side 278 us a pass, now 217).
+// value side 278 us a pass, now 217).  The forward leaves each token's slope, d loss / d vp, for the backward,
+// which so depends neither on the head's output nor on the operands (the caller may overwrite them).
 //
 // Where the predicted value of token j of sample i lies: element i * width + j of [batch, width], or (kHead)
 // in the value head's output [batch, padded_s] at the response window [P - 1, P + R - 1) of the sample,
@@ -378,7 +379,7 @@ template <bool kHead>
 __global__ __launch_bounds__(256) void value_loss_rows_kernel(
     const float* __restrict__ vpreds, ValuePlace place, const float* __restrict__ returns,
     const float* __restrict__ values, const void* __restrict__ mask, int mdtype, const void* __restrict__ lens, int ldtype,
-    int64_t batch, float clip, LossSums* __restrict__ sums) {
+    int64_t batch, float clip, LossSums* __restrict__ sums, float* __restrict__ slope) {
     const int64_t width = place.width;
     __shared__ double part[3][256 / 64];
     double acc[3] = {0.0, 0.0, 0.0};
@@ -394,6 +395,7 @@ __global__ __launch_bounds__(256) void value_loss_rows_kernel(
                 const ValueTerm t = value_term(j < hi - lo ? row[j] : 0.f, returns[e], values[e], clip);
                 acc[0] += (double)(t.loss * m);
                 acc[1] += (double)(t.clipped * m);
+                if (kHead) slope[e] = t.d;
             }
         }
     }
@@ -441,9 +443,8 @@ __global__ __launch_bounds__(256) void value_loss_bwd_kernel(
 
 // The gradient of the whole value head output: every entry finds its token, entries outside the windows get 0.
 __global__ __launch_bounds__(256) void critic_loss_bwd_kernel(
-    const float* __restrict__ head, ValuePlace place, const float* __restrict__ returns, const float* __restrict__ values,
-    int64_t batch, float clip, float loss_scale, const float* __restrict__ out, const float* __restrict__ upstream,
-    float* __restrict__ g_head) {
+    const float* __restrict__ slope, ValuePlace place, int64_t batch, float loss_scale, const float* __restrict__ out,
+    const float* __restrict__ upstream, float* __restrict__ g_head) {
     const float coef = (*upstream) * loss_scale * 0.5f / (out[3] + 1e-8f);
     const int64_t n = batch * place.padded_s;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
@@ -454,8 +455,7 @@ __global__ __launch_bounds__(256) void critic_loss_bwd_kernel(
         float g = 0.f;
         if (j >= 0 && s < hi && j < place.width) {
             const float m = mask_at(nullptr, 0, place.resp, place.resp_dtype, i, j, place.width);
-            const int64_t t = i * place.width + j;
-            if (m != 0.f) g = coef * m * value_term(head[e], returns[t], values[t], clip).d;
+            if (m != 0.f) g = coef * m * slope[i * place.width + j];
         }
         g_head[e] = g;
     }
@@ -598,7 +598,8 @@ extern "C" int mrl_value_loss_fwd_split(const float* vpreds, const float* return
     if (rows > 0) {
         const ValuePlace place = {width, 0, nullptr, 0, nullptr, 0};
         hipLaunchKernelGGL(value_loss_rows_kernel<false>, dim3((unsigned)rows), dim3(256), 0, s, vpreds, place, returns,
-                           values, mask, mask_dtype, response_length, length_dtype, batch, cliprange_value, sums);
+                           values, mask, mask_dtype, response_length, length_dtype, batch, cliprange_value, sums,
+                           (float*)nullptr);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
@@ -617,13 +618,14 @@ static int check_critic(const char* fn, int64_t batch, int64_t padded_s, int64_t
 
 extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
                                    int prompt_dtype, const void* response_length, int response_dtype, const float* returns,
-                                   const float* values, int64_t width, float cliprange_value, float loss_scale, float* out,
-                                   float* loss_out, void* workspace, int64_t workspace_bytes, void* stream) {
+                                   const float* values, int64_t width, float cliprange_value, float loss_scale,
+                                   float* slope, float* out, float* loss_out, void* workspace, int64_t workspace_bytes,
+                                   void* stream) {
     const char* fn = "mrl_critic_loss_fwd";
     int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
     if (rc != MRL_OK) return rc;
     MRL_REQUIRE(out != nullptr && (batch == 0 || ((head || padded_s == 0) && prompt_length && response_length && returns &&
-                                                  values && workspace)),
+                                                  values && slope && workspace)),
                 MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
     MRL_REQUIRE(mrl::aligned(workspace, 8), MRL_ERR_MISALIGNED, "%s: workspace must be 8-byte aligned", fn);
     MRL_REQUIRE(workspace_bytes >= mrl_value_loss_workspace_bytes(batch), MRL_ERR_INVALID_ARG,
@@ -635,7 +637,7 @@ extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t pad
     if (rows > 0) {
         const ValuePlace place = {width, padded_s, prompt_length, prompt_dtype, response_length, response_dtype};
         hipLaunchKernelGGL(value_loss_rows_kernel<true>, dim3((unsigned)rows), dim3(256), 0, s, head, place, returns, values,
-                           (const void*)nullptr, 0, response_length, response_dtype, batch, cliprange_value, sums);
+                           (const void*)nullptr, 0, response_length, response_dtype, batch, cliprange_value, sums, slope);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
@@ -644,20 +646,19 @@ extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t pad
     return mrl::check_launch(fn);
 }
 
-extern "C" int mrl_critic_loss_bwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
-                                   int prompt_dtype, const void* response_length, int response_dtype, const float* returns,
-                                   const float* values, int64_t width, float cliprange_value, float loss_scale,
-                                   const float* out, const float* upstream, float* g_head, void* stream) {
+extern "C" int mrl_critic_loss_bwd(const float* slope, int64_t batch, int64_t padded_s, const void* prompt_length,
+                                   int prompt_dtype, const void* response_length, int response_dtype, int64_t width,
+                                   float loss_scale, const float* out, const float* upstream, float* g_head, void* stream) {
     const char* fn = "mrl_critic_loss_bwd";
     int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
     if (rc != MRL_OK || batch * padded_s == 0) return rc;
-    MRL_REQUIRE(head && prompt_length && response_length && returns && values && out && upstream && g_head,
-                MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    MRL_REQUIRE(slope && prompt_length && response_length && out && upstream && g_head, MRL_ERR_INVALID_ARG,
+                "%s: NULL pointer", fn);
     const ValuePlace place = {width, padded_s, prompt_length, prompt_dtype, response_length, response_dtype};
     const int64_t n = batch * padded_s;
     const unsigned grid = (unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
-    hipLaunchKernelGGL(critic_loss_bwd_kernel, dim3(grid), dim3(256), 0, mrl::as_stream(stream), head, place, returns, values,
-                       batch, cliprange_value, loss_scale, out, upstream, g_head);
+    hipLaunchKernelGGL(critic_loss_bwd_kernel, dim3(grid), dim3(256), 0, mrl::as_stream(stream), slope, place, batch, loss_scale,
+                       out, upstream, g_head);
     return mrl::check_launch(fn);
 }
 

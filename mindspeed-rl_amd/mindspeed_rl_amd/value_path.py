@@ -157,7 +157,8 @@ class _ValueLoss(torch.autograd.Function):
 
 class _CriticLoss(torch.autograd.Function):
     """The value head's output [B, S, 1] -> (scaled loss, out[4]) through mrl_critic_loss_fwd / _bwd: the response
-    windows are read and their gradients written where they lie."""
+    windows are read and their gradients written where they lie.  The head's output is not kept: the caller may
+    overwrite it before the backward."""
 
     @staticmethod
     def forward(ctx, head, prompt, lens, returns, values, clip, loss_scale):
@@ -167,14 +168,14 @@ class _CriticLoss(torch.autograd.Function):
         (batch, padded, _), width = head.shape, ret.shape[1]
         out = torch.empty(4, dtype=torch.float32, device=dev)
         loss = torch.empty((), dtype=torch.float32, device=dev)     # autograd outputs must not alias
+        slope = torch.empty_like(ret)
         ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(batch)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        scalars = (float(clip), float(loss_scale))
         _lib.call("mrl_critic_loss_fwd", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
-                  _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, *scalars, _lib.ptr(out),
-                  _lib.ptr(loss), _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
-        ctx.save_for_backward(head, prompt, lens, ret, val, out)
-        ctx.scalars = scalars
+                  _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, float(clip), float(loss_scale),
+                  _lib.ptr(slope), _lib.ptr(out), _lib.ptr(loss), _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
+        ctx.save_for_backward(slope, prompt, lens, out)
+        ctx.meta = (tuple(head.shape), float(loss_scale))
         ctx.mark_non_differentiable(out)
         ctx.set_materialize_grads(False)
         return loss, out
@@ -183,13 +184,14 @@ class _CriticLoss(torch.autograd.Function):
     def backward(ctx, g_loss, _g_out):
         if g_loss is None:
             return (None,) * 7
-        head, prompt, lens, ret, val, out = ctx.saved_tensors
-        dev = head.device
+        slope, prompt, lens, out = ctx.saved_tensors
+        shape, loss_scale = ctx.meta
+        dev = slope.device
         upstream = _lib.dense(g_loss, torch.float32, dev)
-        g = torch.empty_like(head)
-        _lib.call("mrl_critic_loss_bwd", _lib.ptr(head), head.shape[0], head.shape[1], _lib.ptr(prompt),
-                  _lib.dtype_code(prompt), _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), ret.shape[1],
-                  *ctx.scalars, _lib.ptr(out), _lib.ptr(upstream), _lib.ptr(g), _lib.stream(dev))
+        g = torch.empty(shape, dtype=torch.float32, device=dev)
+        _lib.call("mrl_critic_loss_bwd", _lib.ptr(slope), shape[0], shape[1], _lib.ptr(prompt), _lib.dtype_code(prompt),
+                  _lib.ptr(lens), _lib.dtype_code(lens), slope.shape[1], loss_scale, _lib.ptr(out), _lib.ptr(upstream),
+                  _lib.ptr(g), _lib.stream(dev))
         return g, None, None, None, None, None, None
 
 

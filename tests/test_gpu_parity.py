@@ -2875,6 +2875,34 @@ def test_critic_loss_reads_the_windows_in_place(dev, index, padded, width):
     assert torch.equal(got, want) and (want.abs().sum().item() > 0)
 
 
+@pytest.mark.parametrize("packed", [False, True])
+def test_critic_loss_operands_may_change_before_the_backward(dev, packed):
+    """The value head's output may be overwritten between compute_loss and backward (the reference saves a cut
+    copy of it), and the gradient is that of the values the loss was taken from."""
+    gen = torch.Generator().manual_seed(31)
+    n_seq, seq, resp_w = 3, 40, 16
+    plen, rlen = torch.tensor([[1], [7], [20]], dtype=torch.int32), torch.tensor([[16], [3], [11]], dtype=torch.int32)
+    b = _to_dev({"responses": torch.zeros(n_seq, resp_w, dtype=torch.int64), "prompt_length": plen, "response_length": rlen,
+                 "values": torch.randn(n_seq, resp_w, generator=gen), "returns": torch.randn(n_seq, resp_w, generator=gen)}, dev)
+    kw = {}
+    head = torch.randn(n_seq, seq, 1, generator=gen)
+    if packed:
+        lens = (plen + rlen).view(-1)
+        cu = torch.cat([torch.zeros(1, dtype=torch.int32), torch.cumsum(lens, 0, dtype=torch.int32)])
+        head = torch.randn(1, int(cu[-1]), 1, generator=gen)
+        kw = dict(use_remove_padding=True, seqlens_in_batch=lens.to(dev), cu_seqlens_padded=cu.to(dev), seq_len=seq)
+    crit = mrl.CriticLossFunc()
+    crit.add_loss_meta_info({"cliprange_value": 0.3})
+    leaf = head.to(dev).requires_grad_()
+    (want,) = torch.autograd.grad(crit.compute_loss(leaf, b, **kw)[0], leaf)
+    out = leaf * 1.0
+    loss, _ = crit.compute_loss(out, b, **kw)
+    with torch.no_grad():
+        out.fill_(7.0)
+    (got,) = torch.autograd.grad(loss, leaf)
+    assert want.any().item() and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("layout", ["padded", "packed"])
 @pytest.mark.parametrize("index", [torch.int32, torch.int64])
 def test_response_windows(dev, layout, index):
