@@ -448,15 +448,22 @@ class StandardLogProbComputer(LogProbComputer):
 
     @staticmethod
     def _windows(output, batch, kwargs):
-        """Rows outside every response window (prompts, padding) are not swept at all: their log-prob,
-        entropy and gradient are never looked at by the reference either."""
         packed = kwargs.get("use_remove_padding", False)
         return ResponseWindows(output.shape[:-1], batch, packed, kwargs.get("seqlens_in_batch"),
                                kwargs.get("cu_seqlens_padded"))
 
-    @classmethod
-    def _rows_in_windows(cls, output, batch, kwargs):
-        return cls._windows(output, batch, kwargs).rows()
+    @staticmethod
+    def _rows_in_windows(output, batch, kwargs):
+        """uint8 flag per logits row.  Rows outside every response window (prompts, padding) are not swept at
+        all: their log-prob, entropy and gradient are never looked at by the reference either."""
+        return StandardLogProbComputer._windows(output, batch, kwargs).rows()
+
+    def _active_rows(self, output, batch, kwargs):
+        """The windows and their rows' flags; no windows where a subclass chooses the rows."""
+        if self._rows_in_windows is not StandardLogProbComputer._rows_in_windows:
+            return None, self._rows_in_windows(output, batch, kwargs).view(batch["labels"].shape)
+        windows = self._windows(output, batch, kwargs)
+        return windows, windows.rows().view(batch["labels"].shape)
 
     def compute(self, output, batch, skip_entropy, **kwargs):
         labels = batch["labels"]
@@ -468,8 +475,7 @@ class StandardLogProbComputer(LogProbComputer):
             # `output` holds the hidden states: the rows of the response windows are projected and scored
             # tile by tile on the matrix cores, no logits are written (forward only, no autograd)
             from .lmhead import lmhead_logprob
-            windows = self._windows(output, batch, kwargs)
-            active = windows.rows().view(labels.shape)
+            windows, active = self._active_rows(output, batch, kwargs)
             log_probs, entropy, _ = lmhead_logprob(output, weight, labels, inv_temperature=inv_t,
                                                    want_entropy=not skip_entropy, row_active=active)
         elif injected is not None and injected is not vocab_ops.vocab_parallel_cross_entropy:
@@ -478,8 +484,7 @@ class StandardLogProbComputer(LogProbComputer):
             log_probs = compute_log_probs(scaled, labels)
             entropy = None if skip_entropy else vocab_parallel_entropy(scaled)
         else:
-            windows = self._windows(output, batch, kwargs)
-            active = windows.rows().view(labels.shape)
+            windows, active = self._active_rows(output, batch, kwargs)
             log_probs, entropy, _ = vocab_logprob_entropy(output, labels, inv_temperature=inv_t,
                                                           want_entropy=None if skip_entropy else True,
                                                           row_active=active,

@@ -2969,6 +2969,36 @@ def test_log_prob_computer_uses_a_subclass_cut(dev):
 
 
 @pytest.mark.parametrize("layout", ["padded", "packed"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_log_prob_computer_uses_a_subclass_choice_of_rows(dev, layout, grad):
+    """A subclass that says which rows are swept is asked, in every kind of pass: rows it leaves out score 0."""
+    from mindspeed_rl_amd.loss import StandardLogProbComputer
+
+    class EveryOther(StandardLogProbComputer):
+        @staticmethod
+        def _rows_in_windows(output, batch, kwargs):
+            rows = StandardLogProbComputer._rows_in_windows(output, batch, kwargs)
+            return rows * (torch.arange(rows.numel(), device=rows.device) % 2).to(torch.uint8)
+
+    gen = torch.Generator().manual_seed(5)
+    b = {"responses": torch.zeros(3, 8, dtype=torch.int64), "prompt_length": torch.tensor([[1], [4], [9]]),
+         "response_length": torch.tensor([[8], [3], [5]])}
+    lead, kw, first_row = (3, 20), {}, torch.tensor([[0], [20 + 3], [40 + 8]])
+    if layout == "packed":
+        lens = (b["prompt_length"] + b["response_length"]).view(-1)
+        cu = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(lens, 0)]).to(torch.int32)
+        kw = dict(use_remove_padding=True, seqlens_in_batch=lens.to(torch.int32).to(dev), cu_seqlens_padded=cu.to(dev), seq_len=20)
+        lead, first_row = (1, int(cu[-1])), cu[:-1].view(-1, 1) + b["prompt_length"] - 1
+    out = torch.randn(*lead, 640, generator=gen).to(dev).requires_grad_(grad)
+    b["labels"] = torch.randint(0, 640, lead, generator=gen)
+    bd = _to_dev(b, dev)
+    (want, _), (got, ent) = (c.compute(out, bd, False, **kw) for c in (StandardLogProbComputer(), EveryOther()))
+    odd = ((first_row + torch.arange(8)[None, :]) % 2 == 1).to(dev)
+    assert torch.equal(got, want * odd) and want.any().item() and not torch.equal(got, want)
+    assert bool((ent[odd & (want != 0)] > 0).all().item())
+
+
+@pytest.mark.parametrize("layout", ["padded", "packed"])
 def test_standard_computer_sweeps_only_window_rows(dev, layout):
     """The split path's log-prob strategy skips the logits rows that the response-window cut never
     reads (prompt rows, the last row, padding): same [B, L] values bit for bit as a sweep over every
