@@ -237,6 +237,8 @@ class ResponseWindows:
         self.width = batch["responses"].shape[-1]
         self.prompt, self.resp = batch["prompt_length"], batch.get("response_length")
         if packed:
+            if lead[0] != 1:
+                raise ValueError("Expected output tensor to have shape[0] == 1 (packed batch dimension)")
             self.layout, self.padded, self.n_rows = 0, 0, lead[-1]
             self.seqlens = seqlens.to(torch.int32).contiguous()
             self.cu = cu_seqlens.to(torch.int32).contiguous()
@@ -244,6 +246,8 @@ class ResponseWindows:
             if self.cu.numel() != self.n_seq + 1:
                 raise ValueError("cu_seqlens_padded needs one entry more than seqlens_in_batch")
         else:
+            if len(lead) != 2:
+                raise ValueError("output must have shape (mbs, seq_len, vocab_size)")
             self.layout, self.n_seq, self.padded = 1, lead[0], lead[1]
             self.n_rows, self.seqlens, self.cu = lead[0] * lead[1], None, None
             if tuple(self.prompt.shape) != (self.n_seq, 1) or tuple(self.resp.shape) != (self.n_seq, 1):

@@ -2968,6 +2968,30 @@ def test_log_prob_computer_uses_a_subclass_cut(dev):
     assert all(torch.equal(g, -w) for g, w in zip(got, want)) and want[0].any().item()
 
 
+@pytest.mark.parametrize("grad", [False, True])
+def test_log_prob_computer_refuses_other_shapes(dev, grad):
+    """Packed logits come with their batch dimension of 1, padded ones as [B, S, V], in every kind of pass."""
+    b = _to_dev({"responses": torch.zeros(2, 4, dtype=torch.int64), "prompt_length": torch.tensor([[1], [2]]),
+                 "response_length": torch.tensor([[4], [3]])}, dev)
+    lens = torch.tensor([5, 5], dtype=torch.int32, device=dev)
+    packed = dict(use_remove_padding=True, seqlens_in_batch=lens, seq_len=5,
+                  cu_seqlens_padded=torch.tensor([0, 5, 10], dtype=torch.int32, device=dev))
+    comp = mrl.StandardLogProbComputer()
+
+    def score(*shape, **kw):
+        out = torch.randn(*shape, device=dev).requires_grad_(grad)
+        return comp.compute(out, dict(b, labels=torch.zeros(shape[:-1], dtype=torch.int64, device=dev)), True, **kw)
+
+    assert score(1, 10, 64, **packed)[0].shape == score(2, 5, 64)[0].shape == (2, 4)
+    with pytest.raises(ValueError, match="shape\\[0\\] == 1"):
+        score(10, 64, **packed)
+    with pytest.raises((ValueError, RuntimeError)):
+        score(2, 10, 64, **packed)
+    for shape in ((2, 5, 1, 64), (2, 1, 5, 64)):
+        with pytest.raises((ValueError, RuntimeError)):
+            score(*shape)
+
+
 @pytest.mark.parametrize("layout", ["padded", "packed"])
 @pytest.mark.parametrize("grad", [False, True])
 def test_log_prob_computer_uses_a_subclass_choice_of_rows(dev, layout, grad):
