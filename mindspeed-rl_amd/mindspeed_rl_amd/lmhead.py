@@ -39,12 +39,6 @@ def lmhead_logprob(hidden, weight, labels, inv_temperature=1.0, want_entropy=Tru
             raise ValueError("row_active must have the shape of labels")
         dev = _lib.require_device(hidden, weight, labels, row_active)
         hdim, n_all = hidden.shape[-1], labels.numel()
-        if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
-            raise TypeError("hidden and weight must be bfloat16")
-        flat = hidden.detach().reshape(-1, hdim)
-        if flat.shape[0] != n_all:
-            raise ValueError("labels shape %s does not match hidden leading shape %s"
-                             % (tuple(labels.shape), tuple(hidden.shape[:-1])))
         flags = row_active.reshape(-1)
         if flags.dtype is not torch.uint8:
             flags = (flags != 0).view(torch.uint8)
@@ -52,6 +46,12 @@ def lmhead_logprob(hidden, weight, labels, inv_temperature=1.0, want_entropy=Tru
         out = torch.zeros if rows.n == 0 else torch.empty
         full = out((3, n_all), dtype=torch.float32, device=dev)
         if rows.n > 0:
+            if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+                raise TypeError("hidden and weight must be bfloat16")
+            flat = hidden.detach().reshape(-1, hdim)
+            if flat.shape[0] < n_all:           # rows behind the last label count as little as inactive ones
+                raise ValueError("labels shape %s does not match hidden leading shape %s"
+                                 % (tuple(labels.shape), tuple(hidden.shape[:-1])))
             lab = _lib.index_column(labels, dev)
             h, y, _ = rows.gather(flat, lab, None)
             part = torch.empty((3, rows.n), dtype=torch.float32, device=dev)

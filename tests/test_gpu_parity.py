@@ -3200,6 +3200,24 @@ def test_lmhead_logprob_row_active(dev):
         mrl.lmhead_logprob(h, w, y, row_active=act[:-1])
 
 
+def test_lmhead_logprob_row_active_looks_at_live_rows_only(dev):
+    """What lies outside the flagged rows is not looked at: hidden rows behind the last label, and with no row
+    flagged nothing at all."""
+    gen = torch.Generator().manual_seed(9)
+    h = torch.randn(40, 128, generator=gen).to(torch.bfloat16).to(dev)
+    w = (torch.randn(200, 128, generator=gen) * 0.1).to(torch.bfloat16).to(dev)
+    y = torch.randint(0, 200, (33,), generator=gen).to(dev)
+    act = (torch.arange(33, device=dev) % 3 == 0)
+    for got, want in zip(mrl.lmhead_logprob(h, w, y, row_active=act), mrl.lmhead_logprob(h[:33], w, y, row_active=act)):
+        assert torch.equal(got, want) and want.any().item()
+    none = mrl.lmhead_logprob(h.float(), w, y, row_active=torch.zeros_like(act))
+    assert all(t.shape == (33,) and not t.any().item() for t in none)
+    with pytest.raises(ValueError):
+        mrl.lmhead_logprob(h[:32], w, y, row_active=act)
+    with pytest.raises(TypeError):
+        mrl.lmhead_logprob(h.float(), w, y, row_active=act)
+
+
 @pytest.mark.parametrize("fused", [True, False])
 def test_loss_on_logits_that_are_views_or_products(dev, fused):
     """The logits a model hands over are the result of a projection, possibly a transposed or sliced
