@@ -367,10 +367,13 @@ struct ValuePlace {
     }
 };
 
-// The same spread over the chip: one workgroup per row (rows strided beyond kLossRows of them) leaves its
-// three sums in fp64, a second launch adds them up in a fixed order.  128 x 2048: 11 us for both, was
-// 167 us by one workgroup, which pays off only where no scratch memory is at hand.
-constexpr int64_t kLossRows = 1024;
+// The same spread over the chip: one workgroup per row (rows strided beyond kLossRows of them), or per part of a
+// row where few wide rows would leave the chip idle, leaves its three sums in fp64, a second launch adds them
+// up in a fixed order.  128 x 2048: 11 us for both, was 167 us by one workgroup, which pays off only where no
+// scratch memory is at hand.  Rows are cut into parts of up to kLossPart entries as far as there are workgroups
+// (1 x 32 768, a call: 44.5 us whole, 22.9 us in 16 parts; one workgroup of 1024 threads 25.1 us).
+constexpr int64_t kLossRows = 1024;             // workgroups, and partial sums
+constexpr int64_t kLossPart = 2048;
 struct LossSums {
     double loss, clipped, count;
 };
@@ -383,11 +386,12 @@ __global__ __launch_bounds__(256) void value_loss_rows_kernel(
     const int64_t width = place.width;
     __shared__ double part[3][256 / 64];
     double acc[3] = {0.0, 0.0, 0.0};
+    const int64_t begin = width * blockIdx.y / gridDim.y, end = width * (blockIdx.y + 1) / gridDim.y;
     for (int64_t i = blockIdx.x; i < batch; i += gridDim.x) {
         int64_t lo = 0, hi = width;
         if (kHead) place.window(i, lo, hi);
         const float* row = vpreds + (kHead ? i * place.padded_s + lo : i * width);
-        for (int64_t j = threadIdx.x; j < width; j += 256) {
+        for (int64_t j = begin + threadIdx.x; j < end; j += 256) {
             const float m = mask_at(mask, mdtype, lens, ldtype, i, j, width);
             acc[2] += (double)m;
             if (m != 0.f) {
@@ -410,7 +414,7 @@ __global__ __launch_bounds__(256) void value_loss_rows_kernel(
         double s[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) s[q] = (part[q][0] + part[q][1]) + (part[q][2] + part[q][3]);
-        sums[blockIdx.x] = {s[0], s[1], s[2]};
+        sums[blockIdx.y * gridDim.x + blockIdx.x] = {s[0], s[1], s[2]};
     }
 }
 
@@ -459,6 +463,13 @@ __global__ __launch_bounds__(256) void critic_loss_bwd_kernel(
         }
         g_head[e] = g;
     }
+}
+
+// Workgroups of value_loss_rows_kernel: rows by parts, at most kLossRows.
+dim3 loss_grid(int64_t batch, int64_t width) {
+    const int64_t rows = batch < kLossRows ? batch : kLossRows, most = rows > 0 ? kLossRows / rows : 1;
+    const int64_t parts = (width + kLossPart - 1) / kLossPart;
+    return dim3((unsigned)rows, (unsigned)(parts < most ? parts : most));
 }
 
 int check_mask(const char* fn, const void* mask, int mask_dtype, const void* lens, int lens_dtype) {
@@ -574,7 +585,7 @@ extern "C" int mrl_value_loss_fwd(const float* vpreds, const float* returns, con
 }
 
 extern "C" int64_t mrl_value_loss_workspace_bytes(int64_t batch) {
-    return batch < 0 ? 0 : (batch < kLossRows ? batch : kLossRows) * (int64_t)sizeof(LossSums);
+    return batch <= 0 ? 0 : kLossRows * (int64_t)sizeof(LossSums);
 }
 
 extern "C" int mrl_value_loss_fwd_split(const float* vpreds, const float* returns, const float* values, const void* mask,
@@ -594,17 +605,17 @@ extern "C" int mrl_value_loss_fwd_split(const float* vpreds, const float* return
                 (long long)mrl_value_loss_workspace_bytes(batch));
     hipStream_t s = mrl::as_stream(stream);
     LossSums* sums = reinterpret_cast<LossSums*>(workspace);
-    const int rows = (int)(batch < kLossRows ? batch : kLossRows);
-    if (rows > 0) {
+    const dim3 grid = loss_grid(batch, width);
+    if (grid.x > 0) {
         const ValuePlace place = {width, 0, nullptr, 0, nullptr, 0};
-        hipLaunchKernelGGL(value_loss_rows_kernel<false>, dim3((unsigned)rows), dim3(256), 0, s, vpreds, place, returns,
+        hipLaunchKernelGGL(value_loss_rows_kernel<false>, grid, dim3(256), 0, s, vpreds, place, returns,
                            values, mask, mask_dtype, response_length, length_dtype, batch, cliprange_value, sums,
                            (float*)nullptr);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
-    hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums, rows,
-                       loss_scale, out, loss_out);
+    hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums,
+                       (int)(grid.x * grid.y), loss_scale, out, loss_out);
     return mrl::check_launch(fn);
 }
 
@@ -633,16 +644,16 @@ extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t pad
                 (long long)mrl_value_loss_workspace_bytes(batch));
     hipStream_t s = mrl::as_stream(stream);
     LossSums* sums = reinterpret_cast<LossSums*>(workspace);
-    const int rows = (int)(batch < kLossRows ? batch : kLossRows);
-    if (rows > 0) {
+    const dim3 grid = loss_grid(batch, width);
+    if (grid.x > 0) {
         const ValuePlace place = {width, padded_s, prompt_length, prompt_dtype, response_length, response_dtype};
-        hipLaunchKernelGGL(value_loss_rows_kernel<true>, dim3((unsigned)rows), dim3(256), 0, s, head, place, returns, values,
+        hipLaunchKernelGGL(value_loss_rows_kernel<true>, grid, dim3(256), 0, s, head, place, returns, values,
                            (const void*)nullptr, 0, response_length, response_dtype, batch, cliprange_value, sums, slope);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
-    hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums, rows,
-                       loss_scale, out, loss_out);
+    hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums,
+                       (int)(grid.x * grid.y), loss_scale, out, loss_out);
     return mrl::check_launch(fn);
 }
 

@@ -602,6 +602,33 @@ def test_gae_whitening_and_value_loss_at_the_edges_of_their_split(dev, batch, wi
     assert out[2].item() == pytest.approx(want_frac.item(), rel=1e-5, abs=1e-8) and out[3].item() == mask.sum().item()
 
 
+@pytest.mark.parametrize("batch,width", [(1, 2049), (1, 40001), (3, 6145), (512, 4100), (513, 4100), (1024, 2050), (2000, 2049)])
+def test_value_losses_of_rows_in_parts(dev, batch, width):
+    """Few wide rows are dealt to several workgroups each: the loss, its statistics and the critic's gradient
+    against fp64, for every count of parts from one to a workgroup's share, and more rows than workgroups."""
+    gen = torch.Generator().manual_seed(batch + width)
+    v, vp, ret = (torch.randn(batch, width, generator=gen) for _ in range(3))
+    lens = torch.randint(0, width + 1, (batch, 1), generator=gen)
+    lens[0] = width
+    mask = (torch.arange(width)[None, :] < lens).double()
+    want, want_frac = o_loss.value_loss(vp.double(), ret.double(), v.double(), mask, 0.5)
+    got, out = mrl.value_loss(vp.to(dev), ret.to(dev), v.to(dev), None, lens.to(dev), cliprange_value=0.5)
+    assert got.item() == pytest.approx(want.item(), rel=1e-5) and out[3].item() == mask.sum().item()
+    assert out[2].item() == pytest.approx(want_frac.item(), rel=1e-5)
+    head = torch.cat([torch.zeros(batch, 3), vp, torch.zeros(batch, 2)], 1).unsqueeze(-1).to(dev).requires_grad_()
+    b = _to_dev({"responses": torch.zeros(batch, width, dtype=torch.int64), "prompt_length": torch.full((batch, 1), 4),
+                 "response_length": lens, "values": v, "returns": ret}, dev)
+    crit = mrl.CriticLossFunc()
+    loss, stats = crit.compute_loss(head, b)
+    assert loss.item() == got.item() and stats["critic/vf_clipfrac"] == out[2].item()
+    (g,) = torch.autograd.grad(loss, head)
+    vo = vp.double().requires_grad_()
+    (g_o,) = torch.autograd.grad(o_loss.value_loss(vo, ret.double(), v.double(), mask, 0.5)[0], vo)
+    assert not g[:, :3].any().item() and not g[:, 3 + width:].any().item()
+    # a few fp32 roundings of the slope and of the count
+    assert (g[:, 3:3 + width, 0].cpu().double() - g_o).abs().max().item() <= 2.0 ** -21 * g_o.abs().max().item()
+
+
 @pytest.mark.parametrize("penalty", ["kl", "abs", "mse", "low_var_kl"])
 def test_kl_token_rewards_parity(dev, penalty):
     gen = torch.Generator().manual_seed(17)
