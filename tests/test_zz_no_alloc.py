@@ -61,3 +61,21 @@ def test_static_scratch_entry_point_matches_the_workspace_one():
     torch.cuda.synchronize()
     assert torch.isnan(out[0]).all().item()
     assert lib.mrl_lmhead_logprob_fwd_static(None, None, 0, 256, 64, None, _lib.I64, 1.0, None, None, None, None) == 0
+
+
+def test_static_scratch_in_equal_slices():
+    """More tokens than the static array holds the statistics of (21 760 at 256 leaves of the vocabulary), in
+    slices that do not end on a whole tile: bit-identical to one pass with a workspace."""
+    dev = torch.device("cuda:0")
+    lib, stream = _lib.load(), _lib.stream(dev)
+    tokens, vocab, hdim = 21760 + 129, 256 * 3 * 256, 64
+    hidden, weight, labels = _case(dev, 4, tokens, vocab, hdim)
+    ws_bytes = lib.mrl_lmhead_workspace_bytes(tokens, vocab)
+    assert ws_bytes == tokens * 256 * 12
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    want, got = _outputs(dev, tokens), _outputs(dev, tokens)
+    args = (hidden.data_ptr(), weight.data_ptr(), tokens, vocab, hdim, labels.data_ptr(), _lib.I64, 1.0)
+    _lib.call("mrl_lmhead_logprob_fwd", *args, *(t.data_ptr() for t in want), workspace.data_ptr(), ws_bytes, stream)
+    _lib.call("mrl_lmhead_logprob_fwd_static", *args, *(t.data_ptr() for t in got), stream)
+    for a, b in zip(got, want):
+        assert torch.isfinite(b).all().item() and torch.equal(a, b)
