@@ -487,8 +487,10 @@ int mrl_scale_rows_note(void* x, int dtype, int64_t n_rows, int64_t vocab, int64
  * mrl_lmhead_workspace_bytes(n_tokens, vocab) bytes of device memory, 16-byte aligned, holding
  * partial statistics of the vocabulary, 12 bytes per token and leaf of up to 3 x 256 entries (2.4 KB
  * per token at 152 064 entries; more than 65 536 tokens are taken in equal slices of up to as many, so
- * 192 MiB at most).  A token's result does not depend on the other tokens of the call.
+ * 192 MiB at most).  MRL_LMHEAD_GROUPS x n_tokens x 16 bytes are enough whatever the vocabulary.  A token's
+ * result does not depend on the other tokens of the call.
  */
+#define MRL_LMHEAD_GROUPS 192
 int64_t mrl_lmhead_workspace_bytes(int64_t n_tokens, int64_t vocab);
 int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
                            int64_t hidden_dim, const void* labels, int labels_dtype,

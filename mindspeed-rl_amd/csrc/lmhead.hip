@@ -39,6 +39,7 @@ using namespace mrl_vocab;
 // 95 920 entries: 187 us with leaves of 2 tiles, 240 us with 3), but a leaf costs its statistics' last
 // reduction (19 202 x 148 784 at 1088 hidden: 5.30 ms with 2, 5.20 ms with 3) and 12 bytes per token.
 constexpr int kMaxLeaves = 256;
+static_assert(kMaxLeaves * 3 * sizeof(float) <= MRL_LMHEAD_GROUPS * 16, "what the header promises to suffice");
 struct VocabLeaves {
     int n_tiles, tiles_per_leaf, n;
     __host__ __device__ explicit VocabLeaves(int64_t vocab) {

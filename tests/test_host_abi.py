@@ -54,6 +54,16 @@ def test_header_is_plain_c_and_arities_match(tmp_path):
         assert len(_lib.SIGNATURES[name]) == n, name
 
 
+def test_lmhead_workspace_sized_by_the_macro_is_enough():
+    """A caller may size the forward's workspace with the header's MRL_LMHEAD_GROUPS and no call."""
+    text = open(os.path.join(ROOT, "include", "mrl_hip.h")).read()
+    groups = int(re.search(r"#define\s+MRL_LMHEAD_GROUPS\s+(\d+)", text).group(1))
+    lib = _lib.load()
+    for vocab in (1, 256, 257, 32000, 128 * 256 + 1, 152064, 256 * 3 * 256, 256 * 3 * 256 + 1, 1 << 20, 1 << 30):
+        for n_tokens in (0, 1, 255, 65536, 65537, 1 << 20):
+            assert lib.mrl_lmhead_workspace_bytes(n_tokens, vocab) <= groups * n_tokens * 16
+
+
 def test_argument_validation_launches_nothing():
     lib = _lib.load()
     # NULL logits
