@@ -156,9 +156,6 @@ int mrl_window_gather(const void* src, int elem_bytes, int64_t batch, int64_t wi
 int mrl_window_scatter(const float* g_out, int64_t batch, int64_t width, const void* window,
                        int window_dtype, int64_t out_len, float* g_src, void* stream);
 
-/* mrl_generate_mask: generate_mask (mindspeed_rl/utils/utils.py:57-67): out[i, j] =
- * (j < lengths[i]) as int64, [batch, width]; lengths is I32 or I64.  Negative lengths give an
- * all-zero row, lengths above width an all-one row. */
 /* The response windows in rows of the logits, for the scoring passes (reference: logprob_computer.py:73-145).
  *   layout 0, packed: the rows that mrl_unpad_gather copies with prompt_length (seqlens, cu_seqlens_padded);
  *   layout 1, padded [batch, padded_s]: rows [P - 1, P + R - 1) of each sequence, clamped to it.
@@ -177,21 +174,12 @@ int mrl_window_cut(int layout, int64_t batch, int64_t width, int64_t n_rows, con
                    const float* logp_rows, const float* entropy_rows, float* logp, float* entropy,
                    void* stream);
 
+/* mrl_generate_mask: generate_mask (mindspeed_rl/utils/utils.py:57-67): out[i, j] =
+ * (j < lengths[i]) as int64, [batch, width]; lengths is I32 or I64.  Negative lengths give an
+ * all-zero row, lengths above width an all-one row. */
 int mrl_generate_mask(const void* lengths, int lengths_dtype, int64_t batch, int64_t width,
                       int64_t* out, void* stream);
 
-/* ------------------------------------------------------------------------------------------
- * Ragged <-> padded experience columns: the wire format either side of the path.  Replace the
- * per-row Python loops of unpack_pad_experience (mindspeed_rl/trainer/utils/transfer_dock.py:
- * 1092-1198) and truncate_rows (mindspeed_rl/utils/pad_process.py:144-166).  Bit-exact copies.
- *
- * mrl_ragged_layout: cu[0] = 0, cu[i+1] = cu[i] + len_i (int32 [batch+1]); info[0] = cu[batch],
- * info[1] = max_i len_i rounded up to `multiple` (int64 [2]).  len_i = lengths[i] (I32 / I64), < 0
- * counts as 0.  With width > 0, len_i follows truncate_rows for rows of that width: clamped to
- * width; with left_pad a zero length keeps the whole row (python's x[-0:]); and if `rows`
- * ([batch, width] integers, elem_bytes 4 or 8) is given, 0 where lengths[i] == 0 and
- * rows[i, 0] == -1.  eff_len (nullable int32 [batch]) receives the len_i.  One workgroup;
- * batch <= 2^20. */
 /* Rows that count, for the lm_head passes (no counterpart in the reference, which projects every row).
  * mrl_live_rows: row r is live if flags[r * stride] (U8 or F32) is not zero; live [n] receives the live rows in
  *   order, place [n] the position of each row among them or -1, *total their number; counts: scratch of
@@ -209,7 +197,40 @@ int mrl_move_rows(const int32_t* index, int64_t n_rows, const void* a, void* a_o
 int mrl_spread_scalars(const float* src, int64_t n_src, int n_columns, const int32_t* place, int64_t n,
                        float* dst, void* stream);
 
-/* Several columns at once (at most MRL_RAGGED_COLUMNS), each as by the calls for one below: mrl_ragged_layouts
+/* ------------------------------------------------------------------------------------------
+ * Ragged <-> padded experience columns: the wire format either side of the path.  Replace the
+ * per-row Python loops of unpack_pad_experience (mindspeed_rl/trainer/utils/transfer_dock.py:
+ * 1092-1198) and truncate_rows (mindspeed_rl/utils/pad_process.py:144-166).  Bit-exact copies.
+ *
+ * mrl_ragged_layout: cu[0] = 0, cu[i+1] = cu[i] + len_i (int32 [batch+1]); info[0] = cu[batch],
+ * info[1] = max_i len_i rounded up to `multiple` (int64 [2]).  len_i = lengths[i] (I32 / I64), < 0
+ * counts as 0.  With width > 0, len_i follows truncate_rows for rows of that width: clamped to
+ * width; with left_pad a zero length keeps the whole row (python's x[-0:]); and if `rows`
+ * ([batch, width] integers, elem_bytes 4 or 8) is given, 0 where lengths[i] == 0 and
+ * rows[i, 0] == -1.  eff_len (nullable int32 [batch]) receives the len_i.  One workgroup;
+ * batch <= 2^20. */
+int mrl_ragged_layout(const void* lengths, int lengths_dtype, int64_t batch, int64_t multiple,
+                      const void* rows, int elem_bytes, int64_t width, int left_pad, int32_t* eff_len,
+                      int32_t* cu, int64_t* info, void* stream);
+
+/* mrl_first_match: the search inside remove_padding_and_split_to_list
+ * (mindspeed_rl/utils/pad_process.py:44-62): first[i] = index of the first entry of integer row i
+ * (elem_bytes 4 or 8) that equals `value`, plus `extra` (0 or 1), clamped to width; width if the
+ * row has no such entry.  int32 [batch]. */
+int mrl_first_match(const void* rows, int elem_bytes, int64_t batch, int64_t width, int64_t value, int extra,
+                    int32_t* first, void* stream);
+
+/* out[i, d, j] = flat[d * flat_stride + cu[i] + j] for j < cu[i+1] - cu[i], else pad_bits; out is
+ * [batch, first_dim, width] (first_dim = 1 for ordinary columns, 3 for mrope position ids). */
+int mrl_ragged_to_padded(const void* flat, int elem_bytes, int64_t first_dim, int64_t flat_stride,
+                         const int32_t* cu, int64_t batch, int64_t width, uint64_t pad_bits, void* out,
+                         void* stream);
+
+/* flat[cu[i] + j] = padded[i, j] (left_pad = 0) or padded[i, width - len_i + j] (left_pad = 1). */
+int mrl_padded_to_ragged(const void* padded, int elem_bytes, int64_t batch, int64_t width,
+                         const int32_t* cu, int left_pad, int64_t total, void* flat, void* stream);
+
+/* Several columns at once (at most MRL_RAGGED_COLUMNS), each as by the calls for one above: mrl_ragged_layouts
  * as mrl_ragged_layout without `rows`, mrl_ragged_columns as mrl_ragged_to_padded (to_padded != 0) or
  * mrl_padded_to_ragged.  The columns are read on the host during the call.  Fields that a call does not name
  * are not looked at beyond their range. */
@@ -232,27 +253,6 @@ typedef struct mrl_ragged_column {
 } mrl_ragged_column;
 int mrl_ragged_layouts(const mrl_ragged_column* columns, int n_columns, void* stream);
 int mrl_ragged_columns(int to_padded, const mrl_ragged_column* columns, int n_columns, void* stream);
-
-int mrl_ragged_layout(const void* lengths, int lengths_dtype, int64_t batch, int64_t multiple,
-                      const void* rows, int elem_bytes, int64_t width, int left_pad, int32_t* eff_len,
-                      int32_t* cu, int64_t* info, void* stream);
-
-/* mrl_first_match: the search inside remove_padding_and_split_to_list
- * (mindspeed_rl/utils/pad_process.py:44-62): first[i] = index of the first entry of integer row i
- * (elem_bytes 4 or 8) that equals `value`, plus `extra` (0 or 1), clamped to width; width if the
- * row has no such entry.  int32 [batch]. */
-int mrl_first_match(const void* rows, int elem_bytes, int64_t batch, int64_t width, int64_t value, int extra,
-                    int32_t* first, void* stream);
-
-/* out[i, d, j] = flat[d * flat_stride + cu[i] + j] for j < cu[i+1] - cu[i], else pad_bits; out is
- * [batch, first_dim, width] (first_dim = 1 for ordinary columns, 3 for mrope position ids). */
-int mrl_ragged_to_padded(const void* flat, int elem_bytes, int64_t first_dim, int64_t flat_stride,
-                         const int32_t* cu, int64_t batch, int64_t width, uint64_t pad_bits, void* out,
-                         void* stream);
-
-/* flat[cu[i] + j] = padded[i, j] (left_pad = 0) or padded[i, width - len_i + j] (left_pad = 1). */
-int mrl_padded_to_ragged(const void* padded, int elem_bytes, int64_t batch, int64_t width,
-                         const int32_t* cu, int left_pad, int64_t total, void* flat, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Group-relative advantages.  Replaces compute_group_norm_advantage_return
@@ -624,15 +624,16 @@ int mrl_value_loss_bwd(const float* vpreds, const float* returns, const float* v
  * the value 0 and no gradient.  Forward: as mrl_value_loss_fwd_split, with its workspace; slope [batch, width]
  * receives d(loss)/d(value) of the tokens of the mask, which is all the backward needs of the operands (they
  * may change in between).  Backward: g_head [batch, padded_s], zero outside the windows. */
-int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
-                        int prompt_dtype, const void* response_length, int response_dtype,
-                        const float* returns, const float* values, int64_t width,
-                        float cliprange_value, float loss_scale, float* slope, float* out,
-                        float* loss_out, void* workspace, int64_t workspace_bytes, void* stream);
-int mrl_critic_loss_bwd(const float* slope, int64_t batch, int64_t padded_s, const void* prompt_length,
-                        int prompt_dtype, const void* response_length, int response_dtype,
-                        int64_t width, float loss_scale, const float* out, const float* upstream,
-                        float* g_head, void* stream);
+int mrl_critic_loss_fwd_slope(const float* head, int64_t batch, int64_t padded_s,
+                              const void* prompt_length, int prompt_dtype, const void* response_length,
+                              int response_dtype, const float* returns, const float* values,
+                              int64_t width, float cliprange_value, float loss_scale, float* slope,
+                              float* out, float* loss_out, void* workspace, int64_t workspace_bytes,
+                              void* stream);
+int mrl_critic_loss_bwd_slope(const float* slope, int64_t batch, int64_t padded_s,
+                              const void* prompt_length, int prompt_dtype, const void* response_length,
+                              int response_dtype, int64_t width, float loss_scale, const float* out,
+                              const float* upstream, float* g_head, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Plain device-to-device copy kernel of n_bytes (multiple of 16, 16-byte aligned pointers);

@@ -627,12 +627,12 @@ static int check_critic(const char* fn, int64_t batch, int64_t padded_s, int64_t
     return MRL_OK;
 }
 
-extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
-                                   int prompt_dtype, const void* response_length, int response_dtype, const float* returns,
-                                   const float* values, int64_t width, float cliprange_value, float loss_scale,
-                                   float* slope, float* out, float* loss_out, void* workspace, int64_t workspace_bytes,
-                                   void* stream) {
-    const char* fn = "mrl_critic_loss_fwd";
+extern "C" int mrl_critic_loss_fwd_slope(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
+                                         int prompt_dtype, const void* response_length, int response_dtype,
+                                         const float* returns, const float* values, int64_t width,
+                                         float cliprange_value, float loss_scale, float* slope, float* out,
+                                         float* loss_out, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "mrl_critic_loss_fwd_slope";
     int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
     if (rc != MRL_OK) return rc;
     MRL_REQUIRE(out != nullptr && (batch == 0 || ((head || padded_s == 0) && prompt_length && response_length && returns &&
@@ -657,10 +657,11 @@ extern "C" int mrl_critic_loss_fwd(const float* head, int64_t batch, int64_t pad
     return mrl::check_launch(fn);
 }
 
-extern "C" int mrl_critic_loss_bwd(const float* slope, int64_t batch, int64_t padded_s, const void* prompt_length,
-                                   int prompt_dtype, const void* response_length, int response_dtype, int64_t width,
-                                   float loss_scale, const float* out, const float* upstream, float* g_head, void* stream) {
-    const char* fn = "mrl_critic_loss_bwd";
+extern "C" int mrl_critic_loss_bwd_slope(const float* slope, int64_t batch, int64_t padded_s,
+                                         const void* prompt_length, int prompt_dtype, const void* response_length,
+                                         int response_dtype, int64_t width, float loss_scale, const float* out,
+                                         const float* upstream, float* g_head, void* stream) {
+    const char* fn = "mrl_critic_loss_bwd_slope";
     int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
     if (rc != MRL_OK || batch * padded_s == 0) return rc;
     MRL_REQUIRE(slope && prompt_length && response_length && out && upstream && g_head, MRL_ERR_INVALID_ARG,

@@ -98,8 +98,8 @@ SIGNATURES = {
     "mrl_value_loss_fwd": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp],
     "mrl_value_loss_workspace_bytes": [_i64],
     "mrl_value_loss_fwd_split": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _i64, _vp],
-    "mrl_critic_loss_fwd": [_vp, _i64, _i64, _vp, _int, _vp, _int, _vp, _vp, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
-    "mrl_critic_loss_bwd": [_vp, _i64, _i64, _vp, _int, _vp, _int, _i64, _f32, _vp, _vp, _vp, _vp],
+    "mrl_critic_loss_fwd_slope": [_vp, _i64, _i64, _vp, _int, _vp, _int, _vp, _vp, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
+    "mrl_critic_loss_bwd_slope": [_vp, _i64, _i64, _vp, _int, _vp, _int, _i64, _f32, _vp, _vp, _vp, _vp],
     "mrl_value_loss_bwd": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _vp],
     "mrl_copy_bytes": [_vp, _vp, _i64, _vp],
     "mrl_bandwidth_probe": [_int, _vp, _vp, _i64, _i64, _vp],

@@ -156,7 +156,7 @@ class _ValueLoss(torch.autograd.Function):
 
 
 class _CriticLoss(torch.autograd.Function):
-    """The value head's output [B, S, 1] -> (scaled loss, out[4]) through mrl_critic_loss_fwd / _bwd: the response
+    """The value head's output [B, S, 1] -> (scaled loss, out[4]) through mrl_critic_loss_fwd_slope / _bwd: the response
     windows are read and their gradients written where they lie.  The head's output is not kept: the caller may
     overwrite it before the backward."""
 
@@ -171,7 +171,7 @@ class _CriticLoss(torch.autograd.Function):
         slope = torch.empty_like(ret)
         ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(batch)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        _lib.call("mrl_critic_loss_fwd", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
+        _lib.call("mrl_critic_loss_fwd_slope", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
                   _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, float(clip), float(loss_scale),
                   _lib.ptr(slope), _lib.ptr(out), _lib.ptr(loss), _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
         ctx.save_for_backward(slope, prompt, lens, out)
@@ -189,7 +189,7 @@ class _CriticLoss(torch.autograd.Function):
         dev = slope.device
         upstream = _lib.dense(g_loss, torch.float32, dev)
         g = torch.empty(shape, dtype=torch.float32, device=dev)
-        _lib.call("mrl_critic_loss_bwd", _lib.ptr(slope), shape[0], shape[1], _lib.ptr(prompt), _lib.dtype_code(prompt),
+        _lib.call("mrl_critic_loss_bwd_slope", _lib.ptr(slope), shape[0], shape[1], _lib.ptr(prompt), _lib.dtype_code(prompt),
                   _lib.ptr(lens), _lib.dtype_code(lens), slope.shape[1], loss_scale, _lib.ptr(out), _lib.ptr(upstream),
                   _lib.ptr(g), _lib.stream(dev))
         return g, None, None, None, None, None, None
