@@ -629,6 +629,29 @@ def test_value_losses_of_rows_in_parts(dev, batch, width):
     assert (g[:, 3:3 + width, 0].cpu().double() - g_o).abs().max().item() <= 2.0 ** -21 * g_o.abs().max().item()
 
 
+@pytest.mark.parametrize("batch,width", [(1, 1), (5, 17), (3, 4095), (130, 2048), (2, 8195)])
+def test_value_side_entries_without_scratch_memory(dev, batch, width):
+    """mrl_gae_scan and mrl_value_loss_fwd, the forms for callers that bring no workspace, against the forms that
+    the Python side uses: the scan is the same operations (returns bit for bit, and returns are advantages plus
+    values), the loss the same fp64 sums in another order, rounded to fp32 (2^-24 each)."""
+    gen = torch.Generator().manual_seed(batch * 7 + width)
+    r, v, vp = (torch.randn(batch, width, generator=gen).to(dev) for _ in range(3))
+    mask = (torch.rand(batch, width, generator=gen) < 0.7).long().to(dev)
+    mask.view(-1)[0] = 1
+    stream = _lib.stream(dev)
+    adv, ret = torch.empty_like(r), torch.empty_like(r)
+    _lib.call("mrl_gae_scan", r.data_ptr(), v.data_ptr(), batch, width, 0.99, 0.99 * 0.95, adv.data_ptr(), ret.data_ptr(), stream)
+    _, want = mrl.compute_gae_advantage_return(r, v, mask, 0.99, 0.95)
+    assert torch.equal(ret, want) and torch.equal(adv + v, ret)
+    out = torch.empty(4, device=dev)
+    _lib.call("mrl_value_loss_fwd", vp.data_ptr(), ret.data_ptr(), v.data_ptr(), mask.data_ptr(), _lib.I64, None, 0, batch, width,
+              0.5, 3.0, out.data_ptr(), stream)
+    _, want = mrl.value_loss(vp, ret, v, mask, cliprange_value=0.5, loss_scale=3.0)
+    assert out[3].item() == want[3].item()
+    for got, ref in zip(out.tolist()[:3], want.tolist()[:3]):
+        assert abs(got - ref) <= 2.0 ** -21 * abs(ref)
+
+
 @pytest.mark.parametrize("penalty", ["kl", "abs", "mse", "low_var_kl"])
 def test_kl_token_rewards_parity(dev, penalty):
     gen = torch.Generator().manual_seed(17)
