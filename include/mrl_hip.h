@@ -73,7 +73,9 @@ const char* mrl_last_error(void);
  * logits: [n_rows, vocab] of logits_dtype (F32, BF16, F16), row t at logits + t*row_stride
  * elements; it is only read.  labels: [n_rows] I32 or I64.  row_active (nullable): [n_rows]
  * bytes, rows with 0 are skipped and get logp = entropy = lse = 0.  entropy and lse are
- * nullable; logp is required.  Accumulation is fp32.
+ * nullable; logp is required.  Accumulation is fp32.  The same entries at the same address modulo
+ * 128 give the same bits, whatever the other rows hold: rows of whole 128-byte lines do anywhere
+ * in a tensor that starts on a line, others differ in the rounding of the sums from place to place.
  */
 int mrl_vocab_logprob_fwd(const void* logits, int logits_dtype, int64_t n_rows, int64_t vocab,
                           int64_t row_stride, const void* labels, int labels_dtype,
@@ -384,7 +386,8 @@ int mrl_fused_loss_prepare(int layout, int64_t batch, int64_t width, int64_t n_r
  * autograd (models/base/base_training_engine.py:238-270), so the host never knows them in time.  Rows with mask 0 get zero dlogits and are not read.  dlogits may
  * alias logits exactly (in-place).  row_terms float [n_rows * 8] receives {pg, clipped, old-lp,
  * kl, entropy, 1} * mask per row for step 3.  logp / entropy: nullable [n_rows] outputs.
- * has_old = 0 means old_log_prob = log_prob.detach() (ratio 1).  workspace:
+ * has_old = 0 means old_log_prob = log_prob.detach() (ratio 1).  A row's bits follow from its place
+ * as for mrl_vocab_logprob_fwd.  workspace:
  * mrl_fused_workspace_bytes(dtype, n_rows, vocab) bytes of device memory owned by the caller: the
  * counter from which the persistent workgroups take their next row and, for rows wider than one
  * workgroup holds, the records through which the two halves of a row exchange their statistics.
@@ -528,8 +531,10 @@ int mrl_lmhead_logprob_bwd(const void* hidden, const void* weight, const void* d
  * (d_weight_sums may be NULL).  Every entry is rounded once, as by mrl_lmhead_logprob_bwd and a conversion.
  * workspace (nullable): mrl_lmhead_bwd_workspace_bytes(n_tokens, vocab, hidden_dim) bytes, 16-byte aligned,
  * for dHidden tiles that are cut along the vocabulary when they do not fill the chip (0 bytes where they
- * do); with NULL or fewer bytes none is cut.  dHidden is the same to rounding either way (the fp32 sums
- * group differently), and bit for bit independent of the chunking when none is.  n_tokens > 0. */
+ * do); with NULL or fewer bytes none is cut.  dHidden is the same to rounding either way: cut tiles group
+ * their fp32 sums by slices, whose number follows from n_tokens, so a token's dHidden then differs in its
+ * rounding with the number of tokens beside it; uncut it depends on neither that nor the chunking.
+ * n_tokens > 0. */
 int64_t mrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t hidden_dim);
 int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weight, const void* dlogits,
                                  int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab,

@@ -931,7 +931,9 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
 //          80 KB 4 417 -> 5 906, 100 KB 5 199 -> 5 879 (512 x 16; 512 x 12 where both fit within 2 %)
 //   fp32 (half the entries per byte to compute): 32 KB 3 802 -> 5 599, 48 KB 4 859 -> 6 205, 64 KB 5 832 -> 6 083;
 //          96 and 128 KB stay with 1024 x 8 (6 190 and 6 250 against 5 800 and 5 700 with 512 x 16)
-// The choice depends on the row's length alone, so a row's result does not depend on the other rows.
+// The choice depends on the row's length alone, so a row's result does not depend on the other rows' contents.
+// Its place does enter for rows that are not whole 128-byte lines (see RowSpan): which thread adds which entry
+// follows from the row's address modulo 128, so the fp32 sums round differently at another place in the batch.
 enum Shape { k256x4, k256x8, k256x12, k512x12, k512x16, k1024x8, k1024x12, k1024x16, k1024x19, kTooLong };
 constexpr int64_t kMaxVec = 19 * 1024;              // vectors of the widest row that one workgroup holds
 

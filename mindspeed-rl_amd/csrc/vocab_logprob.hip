@@ -29,7 +29,8 @@ constexpr int kWaves = kBlock / 64;
 constexpr int kUnroll = MRL_VOCAB_UNROLL;
 // Splits a row of `vocab` elements starting at `row` into head scalars up to a 128-byte line (with vectors
 // that are 16-byte aligned only, every wavefront's 1 KiB cuts two lines in half: 129 281 bf16 logits forward
-// 6 437 GB/s, on lines 6 870), 16-byte vectors and tail scalars.
+// 6 437 GB/s, on lines 6 870), 16-byte vectors and tail scalars.  So the order of the fp32 sums, and their
+// last bits, follow from the row's address modulo 128.
 template <typename T, int kVec>
 struct RowSplit {
     int head;       // scalar elements before the first vector

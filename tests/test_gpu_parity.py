@@ -1325,6 +1325,42 @@ def test_fused_sweep_rows_per_ticket(dev, rows, vocab):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 8192), (torch.float32, 16416), (torch.bfloat16, 8200),
+                                         (torch.bfloat16, 50264), (torch.float32, 50260), (torch.float16, 8201)])
+def test_what_a_row_s_place_does_to_its_bits(dev, dtype, vocab):
+    """The same row many times over in one batch, through the one-pass sweep and the split sweeps: the same bits
+    wherever its address modulo 128 is the same - everywhere, for rows of whole lines - and elsewhere only the
+    rounding of the fp32 sums.  A thread adds up at most vocab / 256 + 80 entries in sequence and 16 partial
+    sums are merged, 2^-24 each of a sum of positive terms; the logarithm, the subtraction and the entropy's
+    quotient round a few times more."""
+    rows = 40
+    gen = torch.Generator().manual_seed(vocab)
+    row = _logits(gen, 1, vocab, dtype)
+    z = row.expand(rows, vocab).contiguous().to(dev)
+    y = torch.full((rows,), vocab // 3, device=dev)
+    ops = torch.tensor([[-8.0, -8.5, 0.7, 1.0, 1.0 / rows, 1.0 / rows, 0.0, 0.0]]).repeat(rows, 1).to(dev)
+    esz = z.element_size()
+    assert z.data_ptr() % 128 == 0
+    place = (torch.arange(rows, device=dev) * vocab * esz) % 128
+    assert (place.unique().numel() == 1) == (vocab * esz % 128 == 0)
+    dz, ent, terms = torch.empty_like(z), torch.empty(rows, device=dev), torch.empty(rows, 8, device=dev)
+    _raw_fused_sweep(z, y, ops, dz, ent, terms, _lib.stream(dev), torch.empty(4, dtype=torch.int32, device=dev))
+    zl = z.requires_grad_()
+    lp, ent_s, lse = mrl.vocab_logprob_entropy(zl, y)
+    (dz_s,) = torch.autograd.grad(lp.sum() + 0.1 * ent_s.sum(), zl)
+    bound = (vocab / 256 + 80 + 16 + 16) * 2.0 ** -24 * max(1.0, lse[0].item())
+    for t, grad in ((dz, True), (ent, False), (terms, False), (lp.detach(), False), (ent_s.detach(), False), (lse, False),
+                    (dz_s, True)):
+        for p in place.unique().tolist():
+            same = t[place == p]
+            assert torch.equal(same, same[:1].expand_as(same))
+        far = (t.float() - t[:1].float()).abs().max().item()
+        if grad:                            # and the rounding to the dtype of the logits
+            assert far <= (bound + 2 * torch.finfo(dtype).eps) * t.float().abs().max().item()
+        else:
+            assert far <= bound * max(1.0, t.abs().max().item())
+
+
 @pytest.mark.parametrize("rows,vocab", [(16390, 4096), (9001, 12291), (2500, 24576)])     # 4, 2 and 1 rows per ticket
 @pytest.mark.parametrize("runs", ["whole_tickets", "from_inside_a_ticket", "prompts", "all"])
 def test_fused_sweep_tickets_of_masked_rows(dev, rows, vocab, runs):
