@@ -511,6 +511,7 @@ int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, int64_t n_tok
  *   mrl_fused_logprob_loss       turns the chunk into dlogits in place (see above)
  *   mrl_lmhead_logprob_bwd       dHidden[t, h] = sum_v dlogits[t, v] * weight[v, h]     (bf16 out)
  *                                dWeight[v, h] += sum_t dlogits[t, v] * hidden[t, h]    (fp32, added)
+ *                                (or mrl_lmhead_logprob_bwd_chunk, whose dWeight ends as bf16)
  *
  * hidden [n_tokens, hidden_dim] and weight [vocab, hidden_dim] are dense bf16, hidden_dim % 64 == 0,
  * vocab % 8 == 0; logits / dlogits rows are logits_row_stride / dlogits_row_stride apart.  The

@@ -14,8 +14,6 @@
 // logit (one fp32 dot product per token).  So a token's result does not depend on which other tokens
 // share the call, whatever the work distribution is: units of 256 tokens by a group of leaves, as many
 // groups as fill the chip (pick_groups), walked by one persistent workgroup per CU.
-#include <stdlib.h>
-
 #include <atomic>
 
 #include "lmhead_tile.h"
