@@ -3817,6 +3817,49 @@ def test_whole_step_captured_in_a_graph_and_replayed(dev, source):
     assert len(seen) == 4                               # the replays did see different inputs
 
 
+@pytest.mark.parametrize("expected", [None, 1.0])
+def test_odd_rows_captured_in_a_graph_and_under_saved_tensor_hooks(dev, expected):
+    """Rows that are swept again in the backward: the step captured once and replayed on new inputs, with the
+    gradients at their scale already (learned) and taken again in every replay (stated otherwise), next to
+    eager steps whose saved tensors go through host memory.  Bit-identical each time."""
+    gen = torch.Generator().manual_seed(78)
+    f = mrl.GRPOActorLossFunc()
+    f.add_loss_meta_info({"clip_ratio": 0.2, "kl_ctrl": mrl.FixedKLController(0.01), "kl_penalty": "low_var_kl",
+                          "entropy_coeff": 0.001})
+    logits, b, kw, _, _ = _make_batch(gen, 2, 4, 5, 30, 4099, torch.bfloat16, 2.0, 1)
+    bd, kwd = _to_dev(b, dev), _to_dev(kw, dev)
+    fresh = lambda: (torch.randn(logits.shape, generator=gen) * 2).to(torch.bfloat16).to(dev)
+
+    def step(z):
+        assert mrl.fused_supported(z)
+        loss, stats = f.compute_loss(z, bd, expected_grad_scale=expected, **kwd)
+        return loss, stats, torch.autograd.grad(loss / 3.0, z)[0]
+
+    static = fresh().requires_grad_()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step(static)
+    torch.cuda.current_stream(dev).wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        loss_g, stats_g, grad_g = step(static)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        new = fresh()
+        with torch.no_grad():
+            static.copy_(new)
+        with torch.autograd.graph.save_on_cpu():
+            loss_e, stats_e, grad_e = step(new.requires_grad_())
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert loss_g.item() == loss_e.item() and dict(stats_g) == stats_e
+        assert torch.equal(grad_g, grad_e) and grad_e.any().item()
+
+
 @pytest.mark.parametrize("upstream", [0.0, float("inf")])
 def test_backward_with_a_zero_or_infinite_upstream_gradient(dev, upstream):
     """A skipped or overflowed loss-scale step reaches the loss as an upstream gradient of 0 or Inf.  It
