@@ -793,7 +793,10 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         edge_bits = edge_next;
         r = nx.r;
     }
-    if (kEdge && again.carried && tid == 0) note_scale_last(*grad_scale_dev, again.carried, again.learned, moved ? again.rescales : nullptr);
+    // Every wavefront of a workgroup with rows has read the old scale by now: it has passed the barrier of at
+    // least one ticket.  One without rows has nothing to do whatever it reads.
+    if (kEdge && again.carried && tid == 0)
+        note_scale_last(*grad_scale_dev, again.carried, again.learned, moved ? again.rescales : nullptr);
 }
 
 // Backward of the split path as a plain stream: one 16-byte vector per thread, small workgroups that
