@@ -6,7 +6,7 @@
 //
 // Mapping.  The product runs on the shared tile loop of lmhead_tile.h (256 x 256 tiles, one
 // wavefront per SIMD with a 128 x 128 sub-tile of v_mfma_f32_16x16x32_bf16 blocks, operands straight
-// from global memory into two LDS stages) with the vocabulary as the MFMA's M and the tokens as its
+// from global memory into LDS) with the vocabulary as the MFMA's M and the tokens as its
 // N: in the 16x16 result layout a lane then owns ONE token column of each block and 4 vocabulary
 // rows, so the softmax statistics of a token accumulate inside a lane.  The vocabulary is cut into leaves
 // of a few tiles (VocabLeaves) that follow from the vocabulary alone; every leaf leaves its own partial
@@ -67,18 +67,18 @@ constexpr int kMaxRounds = 64;                  // units a workgroup may take
 // block and those that stream the same weight tiles run side by side and share them in the XCD's L2; and
 // so that the 8 XCDs hold 32 token tiles x the SAME 8 groups, so that a weight tile comes from HBM once
 // for all of them (numbering all groups of 4 token tiles first: 2 % slower at 8 and more groups).
-struct UnitInfo {
-    int start;                                  // flattened number of the unit's first tile
-    int tm, tn;                                 // its first vocabulary tile, its token tile
-};
 struct UnitTiles : mrl_tile::WholeK {
-    const UnitInfo* units;                      // LDS, n_units + 1 entries (the last: start = n_tiles)
+    // The epilogue below needs more registers than there are and puts some aside: their return is waited for
+    // before the loop, where the wait would be for the requests in flight (they have landed by then).
+    static constexpr bool kSettle = true;
     int n_tiles;
+    // lane r of a wavefront holds the workgroup's unit r: the flattened number of its first tile (beyond every
+    // tile where there is no such unit), its first vocabulary tile less that number, its token tile
+    int start, tm0, tn0;
     __device__ __forceinline__ void coords(int j, int& tm, int& tn) const {
-        int r = 0;
-        while (j >= units[r + 1].start) ++r;
-        tm = __builtin_amdgcn_readfirstlane(units[r].tm - units[r].start) + j;
-        tn = __builtin_amdgcn_readfirstlane(units[r].tn);
+        const int r = __popcll(__ballot(start <= j)) - 1;
+        tm = __builtin_amdgcn_readlane(tm0, r) + j;
+        tn = __builtin_amdgcn_readlane(tn0, r);
     }
 };
 
@@ -88,13 +88,12 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     int n_groups, float k_scale, float* __restrict__ partial) {
     using namespace mrl_tile;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ Stats comb[2][kThreads];          // [vocabulary wavefront][token]: a finished leaf
-    __shared__ UnitInfo units[kMaxRounds + 1];
+    static_assert(kMaxRounds <= 64, "a lane for each unit");
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wv = wave >> 1, wt = wave & 1;
     const VocabLeaves leaves(vocab);
-    UnitTiles seq = {{}, units, 0};
+    UnitTiles seq = {{}, 0, 0x7fffffff, 0, 0};
     {
         const int n_ttiles = (n_tokens + BN - 1) / BN;
         int r = 0;
@@ -105,13 +104,15 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
             const int panel = in_block / (4 * gw), in_panel = in_block - panel * 4 * gw;
             const int width = min(4, tt_sp - panel * 4), group = block * 8 + in_panel / width;
             const int first = leaves.begin_tile((int)((int64_t)group * leaves.n / n_groups));
-            if (threadIdx.x == 0) units[r] = {seq.n_tiles, first, sp * 32 + panel * 4 + in_panel % width};
+            if (lane == r) {
+                seq.start = seq.n_tiles;
+                seq.tm0 = first - seq.n_tiles;
+                seq.tn0 = sp * 32 + panel * 4 + in_panel % width;
+            }
             seq.n_tiles += leaves.begin_tile((int)((int64_t)(group + 1) * leaves.n / n_groups)) - first;
         }
-        if (threadIdx.x == 0) units[r] = {seq.n_tiles, 0, 0};
     }
     const int tiles_per_leaf = leaves.tiles_per_leaf, n_vtiles = leaves.n_tiles;
-    __syncthreads();
 
     // a lane holds one token of each of its wavefront's 8 token blocks
     Stats st[kBlocks];
@@ -120,9 +121,12 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
 
     // A leaf is finished: combine the four lane quarters (same token, other vocabulary rows), then the two
     // vocabulary wavefronts; thread t writes token t.
-    auto finish_leaf = [&](int leaf, int tn) {
+    auto finish_leaf = [&](int leaf, int tn, unsigned char* spare) {
+        Stats* const comb = reinterpret_cast<Stats*>(spare);       // [vocabulary wavefront][token]
+        static_assert(2 * kThreads * sizeof(Stats) <= kSpareBytes, "the statistics of a leaf");
 #pragma unroll
         for (int tb = 0; tb < kBlocks; ++tb) {
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int off = 16; off <= 32; off <<= 1) {
                 Stats o;
@@ -131,17 +135,20 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
                 o.u = __shfl_xor(st[tb].u, off, 64);
                 st[tb] = merge<true>(st[tb], o, k_scale);
             }
-            if (lane < 16) comb[wv][wt * 128 + tb * 16 + lane] = st[tb];
+            if (lane < 16) comb[wv * kThreads + wt * 128 + tb * 16 + lane] = st[tb];
             st[tb] = {kMaxInit, 0.f, 0.f};
         }
-        // LDS accesses only: a full fence would wait for the requests of the next stages as well.  The
-        // next leaf's writes to comb lie behind the barriers of at least one more tile.
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        // LDS accesses only: a full fence would wait for the requests of the next stages as well
+        auto lds_barrier = [&]() {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        };
+        lds_barrier();
+        const Stats r = merge<true>(comb[threadIdx.x], comb[kThreads + threadIdx.x], k_scale);
+        lds_barrier();                          // what lies here next is requested by any of the wavefronts
         const int t = tn * BN + (int)threadIdx.x;
         if (t < n_tokens) {
-            const Stats r = merge<true>(comb[0][threadIdx.x], comb[1][threadIdx.x], k_scale);
             float* p = partial + (int64_t)leaf * 3 * n_tokens + t;
             p[0] = r.m;
             p[n_tokens] = r.s;
@@ -150,8 +157,8 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     };
 
     // online softmax statistics of a tile: per token block a lane holds 8 x 4 vocabulary rows
-    auto tile_stats = [&](Accumulators& acc, int, int tm, int tn) {
-        const int v0 = tm * BM + wv * 128 + 4 * (lane >> 4);       // + 16 vb + r
+    auto tile_stats = [&](Accumulators& acc, int, int tm, int tn, unsigned char* spare) {
+        int valid = vocab - (tm * BM + wv * 128 + 4 * (lane >> 4));       // 16 vb + r below it
         const bool ragged = (tm * BM + BM > vocab);
 #pragma unroll
         for (int tb = 0; tb < kBlocks; ++tb) {
@@ -160,18 +167,17 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int vb = 0; vb < kBlocks; ++vb) asm volatile("" : "+a"(acc[vb][tb]));
+            float z[4 * kBlocks];
+#pragma unroll
+            for (int i = 0; i < 4 * kBlocks; ++i) z[i] = acc[i / 4][tb][i % 4];
             if (ragged) {
 #pragma unroll
-                for (int vb = 0; vb < kBlocks; ++vb)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (v0 + 16 * vb + r >= vocab) acc[vb][tb][r] = kMaxInit;
+                for (int i = 0; i < 4 * kBlocks; ++i)
+                    if (16 * (i / 4) + i % 4 >= valid) z[i] = kMaxInit;
             }
             float vmax = st[tb].m;
 #pragma unroll
-            for (int vb = 0; vb < kBlocks; ++vb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) vmax = fmaxf(vmax, acc[vb][tb][r]);
+            for (int i = 0; i < 4 * kBlocks; ++i) vmax = fmaxf(vmax, z[i]);
             grow_max<true>(st[tb], vmax, k_scale);
             // A lane that has seen no valid vocabulary row yet (the first tile of its leaf is ragged and
             // ends above its rows) still holds the start value as its maximum: z * k - m * k of the masked
@@ -179,14 +185,12 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
             // zero.  With an infinite m * k their exponentials are exactly 0.
             const float mk = st[tb].m > kMaxInit ? st[tb].m * k_scale : __builtin_inff();
 #pragma unroll
-            for (int vb = 0; vb < kBlocks; ++vb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) add_one<true>(st[tb], acc[vb][tb][r], k_scale, mk);
+            for (int i = 0; i < 4 * kBlocks; ++i) add_one<true>(st[tb], z[i], k_scale, mk);
         }
         const int leaf = tm / tiles_per_leaf;                      // uniform over the workgroup
-        if (tm + 1 == n_vtiles || tm + 1 == (leaf + 1) * tiles_per_leaf) finish_leaf(leaf, tn);
+        if (tm + 1 == n_vtiles || tm + 1 == (leaf + 1) * tiles_per_leaf) finish_leaf(leaf, tn, spare);
     };
-    mfma_tile_loop<false, false, 4>(smem, weight, hdim, vocab, hidden, hdim, n_tokens, hdim, seq, tile_stats);
+    mfma_tile_loop<false, false>(smem, weight, hdim, vocab, hidden, hdim, n_tokens, hdim, seq, tile_stats);
 }
 
 // A workgroup finishes 16 tokens.  16 threads per token merge the leaves (thread q takes leaves q, q + 16,
@@ -294,10 +298,10 @@ extern "C" int64_t mrl_lmhead_workspace_bytes(int64_t n_tokens, int64_t vocab) {
 static int lmhead_forward(const char* fn, const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
                           int64_t hidden_dim, const void* labels, int labels_dtype, float inv_temperature, float* logp,
                           float* entropy, float* lse, float* partial, int64_t slice, hipStream_t s) {
-    // 256-token tiles, operands straight into two LDS stages (128 KiB of dynamic LDS).  Function
+    // 256-token tiles, all of a CU's LDS for the tile loop.  Function
     // attributes belong to a device, so the reservation is made with every launch, on whichever
     // device is current.
-    constexpr int kLdsBytes = mrl_tile::kLdsStages;
+    constexpr int kLdsBytes = mrl_tile::kLdsBytes;
     const hipError_t attr = hipFuncSetAttribute((const void*)lmhead_fwd_kernel,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     MRL_REQUIRE(attr == hipSuccess, MRL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", fn, kLdsBytes,

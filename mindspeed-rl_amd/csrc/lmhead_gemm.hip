@@ -23,8 +23,8 @@
 // is 1.25 rounds of the chip.  Tiles behind the last whole round may therefore be cut along K into slices
 // (plan_split); a slice leaves its fp32 sums in the caller's workspace and merge_slices_kernel adds them in
 // the order of the slices.  Units are numbered slice by slice, so the workgroups of an XCD still share operand
-// tiles.  Both backward products, uncut and cut: 162 x 95 920 x 2 944 2 193 -> 416 us, 300 x 32 000 x 1 024
-// 588 -> 115, 1 380 x 152 064 x 3 584 4 695 -> 2 969, 4 000 x 129 280 x 5 120 10 936 -> 8 629.
+// tiles.  Both backward products, uncut and cut: 300 x 32 000 x 1 024 557 -> 99 us, 1 380 x 152 064 x 3 584
+// 4 466 -> 2 404, 4 000 x 129 280 x 5 120 10 030 -> 7 650.
 #include <type_traits>
 
 #include "lmhead_tile.h"
@@ -36,8 +36,6 @@ namespace {
 using namespace mrl_vocab;
 using namespace mrl_tile;
 
-constexpr int kLdsTurn = 32 * 1024;              // where the wavefronts turn their result blocks (store_tile)
-constexpr int kLdsBytes = kLdsStages + kLdsTurn;
 constexpr int kTilesAlongN = 4;                  // tiles along n in a group of consecutive tile numbers
 
 struct TileGrid {
@@ -52,10 +50,10 @@ struct TileGrid {
 // 8 x 32; with 32 an XCD still holds 8 x 4 and the chip 32 x 8, which fetches less from beyond the L2
 // (B is passed over a quarter as often).
 // A workgroup keeps its tile of A from one of its tiles to the next.
-__device__ __forceinline__ void tile_coords(const TileGrid& g, int64_t t, int& tm, int& tn) {
-    const int64_t per_panel = (int64_t)g.panel_m * g.tiles_n;
-    const int p = (int)(t / per_panel);
-    const int idx = (int)(t - (int64_t)p * per_panel);
+__device__ __forceinline__ void tile_coords(const TileGrid& g, int t, int& tm, int& tn) {
+    const int per_panel = g.panel_m * g.tiles_n;
+    const int p = t / per_panel;
+    const int idx = t - p * per_panel;
     const int pm = min(g.panel_m, g.tiles_m - p * g.panel_m);   // rows of tiles in this panel
     const int ng = idx / (pm * kTilesAlongN);
     const int rem = idx - ng * (pm * kTilesAlongN);
@@ -88,13 +86,13 @@ constexpr int64_t kMaxSlices = 1024;                // of all tiles together: 25
 
 // The number of slices with the least expected time, in k-steps (about 1.5 microseconds each): the rounds that
 // the units take, and per unit of a round about 10 for turning out the sums and 0.1 for each slice's trip
-// through memory to the merge.  A partly filled round of whole tiles is cheaper than a full one, since the
-// board's power goes to fewer CUs: 174 of 256 CUs (12 356 x 152 064 x 3 584) measured 21 486 us uncut against
-// 21 846 in four slices, 120 of 256 (20 000 x 60 000 x 2 048) 8 251 against 7 855 in two.
+// through memory to the merge.  dHidden and dWeight together, uncut and in the slices it chooses, ms: 174 of 256
+// tiles (12 356 x 152 064 x 3 584) 20.55 and in 4 19.73 (in 3 20.76, in 5 19.98); 104 (9 000 x 152 064 x 2 560)
+// 12.33 and in 7 10.27; 144 (2 300 x 32 000 x 4 096) 1.118 and in 3 0.978.
 inline SplitPlan plan_split(int64_t total, int grid, int64_t n_ksteps) {
     SplitPlan p = {total / grid * grid, (int)(total % grid), 1};
     if (p.rest == 0) return p;
-    double best = (double)n_ksteps * (0.35 + 0.65 * (double)p.rest / grid);
+    double best = (double)n_ksteps;
     for (int64_t s = 2; s * p.rest <= kMaxSlices && s * 4 <= n_ksteps; ++s) {
         const int64_t rounds = (s * p.rest + grid - 1) / grid;
         const double cost = (double)rounds * ((double)((n_ksteps + s - 1) / s) + 10.0) + 0.1 * (double)(s * p.rest) + 10.0;
@@ -110,19 +108,20 @@ inline SplitPlan plan_split(int64_t total, int grid, int64_t n_ksteps) {
 // The tiles of one workgroup: number first + j * stride.
 struct StridedTiles : WholeK {
     TileGrid grid;
-    int64_t first, stride;
+    int first, stride;
     int n_tiles;
     __device__ __forceinline__ void coords(int j, int& tm, int& tn) const { tile_coords(grid, first + j * stride, tm, tn); }
 };
 
 // The slices of one workgroup: unit u = first + j * stride is slice u / rest of tile whole + u % rest.
 struct SlicedTiles {
+    static constexpr bool kSettle = false;
     TileGrid grid;
-    int64_t first, stride;
+    int first, stride;
     int n_tiles;
     SplitPlan plan;
     __device__ __forceinline__ void coords(int j, int& tm, int& tn) const {
-        tile_coords(grid, plan.whole + (first + j * stride) % plan.rest, tm, tn);
+        tile_coords(grid, (int)plan.whole + (first + j * stride) % plan.rest, tm, tn);
     }
     __device__ __forceinline__ void k_range(int j, int n_ksteps, int& begin, int& end) const {
         const int64_t s = (first + j * stride) / plan.rest;
@@ -156,9 +155,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
     // workgroups are dealt round-robin to the 8 XCDs: the gridDim / 8 workgroups of an XCD take
     // consecutive tile numbers
     const int per_xcd = gridDim.x >> 3;
-    seq.first = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    seq.stride = gridDim.x;
-    seq.n_tiles = seq.first < n_units ? (int)((n_units - 1 - seq.first) / seq.stride) + 1 : 0;
+    seq.first = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    seq.stride = (int)gridDim.x;
+    seq.n_tiles = seq.first < n_units ? ((int)n_units - 1 - seq.first) / seq.stride + 1 : 0;
 
     // The finished tile.  A lane holds column n = lane & 15 of each 16 x 16 block and rows
     // 4 (lane >> 4) .. + 3 of it: stored like that, a store instruction would touch 16 output rows with
@@ -166,14 +165,14 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
     // [64 n][128 bytes of m] at a time (4 blocks along n by 4 along m for bf16, by 2 for fp32), 16-byte
     // chunks XOR-swizzled by the row pair, written in the MFMA layout and read back as 8 lanes x 16 bytes
     // per output row, so that every store covers whole 128-byte lines.
-    unsigned char* turn = smem + kLdsStages + wave * (kLdsTurn / kWaves);
-    auto store_tile = [&](mrl_tile::Accumulators& acc, int j, int tm, int tn) {
+    auto store_tile = [&](mrl_tile::Accumulators& acc, int j, int tm, int tn, unsigned char* spare) {
+        unsigned char* const turn = spare + wave * (kSpareBytes / kWaves);
         constexpr bool kWideEntries = kOut != kBf16;              // turned as fp32
         // a slice's tile is a matrix of its own
         const int m_tile = kSliced ? 0 : tm * BM, n_tile = kSliced ? 0 : tn * BN;
         const int m_end = kSliced ? M - tm * BM : M, n_end = kSliced ? N - tn * BN : N;
         const int64_t ld = kSliced ? BM : ldo;
-        float* const slice = sums + (kSliced ? (seq.first + j * seq.stride) * kTileElems : 0);
+        float* const slice = sums + (kSliced ? (int64_t)(seq.first + j * seq.stride) * kTileElems : 0);
         const int row_w = lane & 15, quarter = lane >> 4;        // writer: its n, its run of 4 m inside the block
         const int row_r = lane >> 3, chunk_r = lane & 7;          // reader: n within a group of 8, 16-byte chunk
         constexpr int kMPerPass = kWideEntries ? 2 : 4;            // 32 fp32 or 64 bf16 entries of m are 128 bytes
@@ -238,7 +237,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(const uint16_t* __res
         }
     };
 
-    mfma_tile_loop<kATrans, kBTrans, 0>(smem, A, lda, M, B, ldb, N, K, seq, store_tile);
+    mfma_tile_loop<kATrans, kBTrans>(smem, A, lda, M, B, ldb, N, K, seq, store_tile);
 }
 
 // out[n][m] = sum over the slices, in their order, of the tiles that SlicedTiles cut.  Grid: (tile, 16 rows of
@@ -302,7 +301,7 @@ static int launch_gemm(const char* fn, const Product& p, const SplitPlan& plan) 
                     p.ldb % 8 == 0 && p.ldo % 8 == 0,
                 MRL_ERR_INVALID_ARG, "%s: leading dimensions lda=%lld ldb=%lld ldo=%lld", fn, (long long)p.lda,
                 (long long)p.ldb, (long long)p.ldo);
-    // what one buffer descriptor has to span: a tile of 256 rows, or a stage of 64 k-rows
+    // what one buffer descriptor has to span: a tile of 256 rows, or a slot of 32 k-rows
     MRL_REQUIRE(256 * p.lda * 2 < (1LL << 31) && 256 * p.ldb * 2 < (1LL << 31), MRL_ERR_UNSUPPORTED,
                 "%s: 256 rows of an operand must stay below 2 GiB", fn);
     MRL_REQUIRE(aligned(p.a, 16) && aligned(p.b, 16) && aligned(p.out, 16) && aligned(p.sums, 16), MRL_ERR_MISALIGNED,

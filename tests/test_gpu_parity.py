@@ -3225,6 +3225,33 @@ def test_lmhead_backward_chunk(dev, tokens, vocab, hdim):
         assert torch.equal(again, dh) and torch.equal(dw, dw32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("hdim", [8, 264])
+@pytest.mark.parametrize("tokens", [1, 31, 32, 33, 63, 65, 96, 97, 127, 129, 193])
+def test_lmhead_products_at_the_edges_of_a_slot(dev, tokens, hdim):
+    """Operands that are requested 32 k-rows at a time: token counts (k of dWeight) and a vocabulary (k of dHidden)
+    that end inside the first or second half of a k-step, on its border, or leave its second half empty, in tiles
+    that are all ragged; NaN lies behind every operand.  One rounding to bf16
+    for dHidden, fp32 sums of k products of spread 1 for dWeight."""
+    vocab = 8 * (tokens + 32)
+    g = torch.Generator(device=dev).manual_seed(tokens + hdim)
+    v_pad = (vocab + 63) // 64 * 64
+
+    def guarded(rows, cols):
+        buf = torch.full((rows + 64, cols), float("nan"), dtype=torch.bfloat16, device=dev)
+        buf[:rows] = torch.randn(rows, cols, generator=g, device=dev)
+        return buf[:rows]
+
+    h, w, dz = guarded(tokens, hdim), guarded(vocab, hdim), guarded(tokens, v_pad)
+    dz[:, vocab:] = 0
+    dh, dw = torch.full_like(h, 7.0), torch.zeros(vocab, hdim, device=dev)
+    _lib.call("mrl_lmhead_logprob_bwd", h.data_ptr(), w.data_ptr(), dz.data_ptr(), v_pad, tokens, vocab, hdim,
+              dh.data_ptr(), dw.data_ptr(), _lib.stream(dev))
+    want_dh = dz[:, :vocab].double() @ w.double()
+    want_dw = dz[:, :vocab].double().t().contiguous() @ h.double()
+    assert ((dh.double() - want_dh).abs() <= 2 ** -8 * want_dh.abs() + 1e-5 * vocab ** 0.5).all().item()
+    assert ((dw.double() - want_dw).abs() <= 1e-5 * tokens ** 0.5).all().item()
+
+
 def test_fused_lmhead_policy_loss_skips_rows_without_response(dev):
     """With long prompts most rows carry no live response token: the chunked lm_head step gathers the
     live rows and runs its GEMMs on them alone.  Same loss, statistics, dHidden and dWeight as with
