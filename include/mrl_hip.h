@@ -176,6 +176,16 @@ int mrl_window_cut(int layout, int64_t batch, int64_t width, int64_t n_rows, con
                    const float* logp_rows, const float* entropy_rows, float* logp, float* entropy,
                    void* stream);
 
+/* mrl_window_logprob: a whole scoring pass in one launch: what mrl_vocab_logprob_fwd over the rows that
+ * mrl_window_rows flags, followed by mrl_window_cut, leaves in logp and entropy ([batch, width], both written;
+ * entropies are zeros unless want_entropy), bit for bit.  labels: one per row of the logits. */
+int mrl_window_logprob(const void* logits, int logits_dtype, int64_t n_rows, int64_t vocab,
+                       int64_t row_stride, const void* labels, int labels_dtype, float inv_temperature,
+                       int layout, int64_t batch, int64_t width, const int32_t* seqlens,
+                       const int32_t* cu_seqlens_padded, int64_t padded_s, const void* prompt_length,
+                       int prompt_dtype, const void* response_length, int response_dtype, int want_entropy,
+                       float* logp, float* entropy, void* stream);
+
 /* mrl_generate_mask: generate_mask (mindspeed_rl/utils/utils.py:57-67): out[i, j] =
  * (j < lengths[i]) as int64, [batch, width]; lengths is I32 or I64.  Negative lengths give an
  * all-zero row, lengths above width an all-one row. */

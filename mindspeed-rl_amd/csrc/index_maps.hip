@@ -6,16 +6,16 @@
 // by a binary search in cu_seqlens_padded), so no atomics are needed, every output element is
 // written exactly once, and results are deterministic.
 #include "mrl_internal.h"
+#include "seq_windows.h"
 
 namespace {
 
 constexpr int kBlock = 256;
 constexpr int kScanBlock = 1024;
 
-__device__ __forceinline__ int64_t load_index(const void* p, int dtype, int64_t i) {
-    return dtype == MRL_I32 ? (int64_t) reinterpret_cast<const int32_t*>(p)[i]
-                            : reinterpret_cast<const int64_t*>(p)[i];
-}
+using mrl::load_index;
+using mrl::SeqWindows;
+using mrl::unpad_window;
 
 // mask element != 0 counted as its integer value (torch's sum(dtype=int32) adds the values)
 __device__ __forceinline__ int32_t mask_value(const void* p, int dtype, int64_t i) {
@@ -126,21 +126,6 @@ __global__ __launch_bounds__(kBlock) void pack_rows_kernel(const T* __restrict__
     if (pos) pos[t] = p;
 }
 
-// (start, n) of the window that postprocess_packed_seqs copies for sequence i
-__device__ __forceinline__ void unpad_window(const int32_t* __restrict__ seqlens, const int32_t* __restrict__ cu,
-                                             const void* __restrict__ prompt, int prompt_dtype, int i,
-                                             int64_t& start, int64_t& n) {
-    start = (int64_t)cu[i];
-    n = (int64_t)seqlens[i];
-    if (prompt != nullptr) {
-        const int64_t skip = load_index(prompt, prompt_dtype, i) - 1;
-        if (skip < n) {
-            n -= skip + 1;
-            start += skip;
-        }
-    }
-}
-
 // out[i, j, :] for one (i, j) per thread-group of `inner` elements; T is the element's storage type.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void unpad_gather_kernel(const T* __restrict__ packed, int64_t total,
@@ -212,30 +197,7 @@ __global__ __launch_bounds__(kBlock) void window_gather_kernel(const T* __restri
 // element-wise ops they were 24 launches around a sweep of 11 us (1 208 padded rows x 32 000 bf16: 233 us a
 // pass, now 55), so the flags take a clear and a scatter, and both results are cut by one gather.
 //
-// What a sequence's response window is in rows of the logits, for both layouts: `n` rows from row `start` on.
-struct SeqWindows {
-    int packed;
-    const int32_t* seqlens;         // packed
-    const int32_t* cu;
-    int64_t padded_s;               // padded: rows per sequence
-    const void* prompt;
-    int prompt_dtype;
-    const void* resp;               // padded
-    int resp_dtype;
-    __device__ __forceinline__ void window(int64_t i, int64_t& start, int64_t& n) const {
-        if (packed) {
-            unpad_window(seqlens, cu, prompt, prompt_dtype, (int)i, start, n);
-        } else {
-            const int64_t p = load_index(prompt, prompt_dtype, i);
-            int64_t lo = p - 1, hi = p + load_index(resp, resp_dtype, i) - 1;
-            lo = lo < 0 ? 0 : (lo > padded_s ? padded_s : lo);
-            hi = hi < 0 ? 0 : (hi > padded_s ? padded_s : hi);
-            start = i * padded_s + lo;
-            n = hi - lo;
-        }
-    }
-};
-
+//
 // active[t] = 1 for the rows of the windows, at most `width` of each (active is zero before).  A workgroup per
 // sequence; windows may overlap, everyone writes the same.
 __global__ __launch_bounds__(kBlock) void window_rows_kernel(SeqWindows seqs, int64_t width, int64_t n_rows,
@@ -726,13 +688,8 @@ extern "C" int mrl_window_scatter(const float* g_out, int64_t batch, int64_t wid
 }
 
 static int check_windows(const char* fn, const SeqWindows& q, int64_t batch, int64_t width, int64_t n_rows) {
-    MRL_REQUIRE(batch >= 0 && batch <= (1LL << 20) && width >= 0 && n_rows >= 0, MRL_ERR_INVALID_ARG,
-                "%s: batch=%lld width=%lld n_rows=%lld", fn, (long long)batch, (long long)width, (long long)n_rows);
-    MRL_REQUIRE(mrl::int_dtype_bytes(q.prompt_dtype) != 0 && (q.packed || mrl::int_dtype_bytes(q.resp_dtype) != 0),
-                MRL_ERR_UNSUPPORTED, "%s: length dtypes %d and %d (want I32 or I64)", fn, q.prompt_dtype, q.resp_dtype);
-    MRL_REQUIRE(batch == 0 || (q.prompt && (q.packed ? q.seqlens && q.cu : q.resp && q.padded_s >= 0)), MRL_ERR_INVALID_ARG,
-                "%s: NULL pointer", fn);
-    return check_elems(fn, batch * width);
+    const int rc = mrl::check_seq_windows(fn, q, batch, width, n_rows);
+    return rc != MRL_OK ? rc : check_elems(fn, batch * width);
 }
 
 extern "C" int mrl_window_rows(int layout, int64_t batch, int64_t width, int64_t n_rows, const int32_t* seqlens,

@@ -51,6 +51,8 @@ SIGNATURES = {
     "mrl_window_scatter": [_vp, _i64, _i64, _vp, _int, _i64, _vp, _vp],
     "mrl_window_rows": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp],
     "mrl_window_cut": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _vp],
+    "mrl_window_logprob": [_vp, _int, _i64, _i64, _i64, _vp, _int, _f32, _int, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp,
+                           _int, _int, _vp, _vp, _vp],
     "mrl_generate_mask": [_vp, _int, _i64, _i64, _vp, _vp],
     "mrl_live_rows": [_vp, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
     "mrl_move_rows": [_vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _int, _vp],

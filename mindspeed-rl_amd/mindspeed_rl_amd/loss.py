@@ -458,11 +458,11 @@ class StandardLogProbComputer(LogProbComputer):
         all: their log-prob, entropy and gradient are never looked at by the reference either."""
         return StandardLogProbComputer._windows(output, batch, kwargs).rows()
 
-    def _active_rows(self, output, batch, kwargs):
+    def _active_rows(self, output, batch, kwargs, windows=None):
         """The windows and their rows' flags; no windows where a subclass chooses the rows."""
         if self._rows_in_windows is not StandardLogProbComputer._rows_in_windows:
             return None, self._rows_in_windows(output, batch, kwargs).view(batch["labels"].shape)
-        windows = self._windows(output, batch, kwargs)
+        windows = windows or self._windows(output, batch, kwargs)
         return windows, windows.rows().view(batch["labels"].shape)
 
     def compute(self, output, batch, skip_entropy, **kwargs):
@@ -471,6 +471,7 @@ class StandardLogProbComputer(LogProbComputer):
         injected = vocab_ops.get_vocab_parallel()
         weight = kwargs.get("lm_head_weight")
         windows = None
+        own_cut = self._get_log_probs_remove_prompt_pad is StandardLogProbComputer._get_log_probs_remove_prompt_pad
         if weight is not None:
             # `output` holds the hidden states: the rows of the response windows are projected and scored
             # tile by tile on the matrix cores, no logits are written (forward only, no autograd)
@@ -484,12 +485,16 @@ class StandardLogProbComputer(LogProbComputer):
             log_probs = compute_log_probs(scaled, labels)
             entropy = None if skip_entropy else vocab_parallel_entropy(scaled)
         else:
-            windows, active = self._active_rows(output, batch, kwargs)
+            if own_cut and self._rows_in_windows is StandardLogProbComputer._rows_in_windows:
+                windows = self._windows(output, batch, kwargs)
+                scores = vocab_ops.score_windows(output, labels, windows, inv_t, not skip_entropy)
+                if scores is not None:
+                    return scores
+            windows, active = self._active_rows(output, batch, kwargs, windows)
             log_probs, entropy, _ = vocab_logprob_entropy(output, labels, inv_temperature=inv_t,
                                                           want_entropy=None if skip_entropy else True,
                                                           row_active=active,
                                                           grad_inplace=bool(kwargs.get("grad_inplace", False)))
-        own_cut = self._get_log_probs_remove_prompt_pad is StandardLogProbComputer._get_log_probs_remove_prompt_pad
         if windows is not None and own_cut and not log_probs.requires_grad:
             return windows.cut(log_probs, None if skip_entropy else entropy)
         if kwargs.get("use_remove_padding", False):

@@ -11,7 +11,7 @@ import math
 
 import torch
 
-from . import _lib
+from . import _lib, vocab_ops
 
 
 def _as_index(t):
@@ -266,6 +266,17 @@ class ResponseWindows:
         flags = torch.empty((self.n_rows + 15) // 16 * 16, dtype=torch.uint8, device=self.dev)
         _lib.call("mrl_window_rows", *self._args, flags.data_ptr() if self.n_rows else None, _lib.stream(self.dev))
         return flags[:self.n_rows]
+
+    def score(self, flat, row_stride, labels, inv_temperature, want_entropy):
+        """``(log_probs, entropy)`` as :meth:`cut` returns them, straight from rows of logits and their labels."""
+        logp = torch.empty((self.n_seq, self.width), dtype=torch.float32, device=self.dev)
+        ent = torch.empty_like(logp)
+        layout, n_seq, width, n_rows, *lengths = self._args
+        vocab_ops._timed_call("mrl_window_logprob", n_rows, self.dev, _lib.ptr(flat), _lib.dtype_code(flat), n_rows,
+                              flat.shape[1], row_stride, _lib.ptr(labels), _lib.dtype_code(labels), float(inv_temperature),
+                              layout, n_seq, width, *lengths, 1 if want_entropy else 0, _lib.ptr(logp), _lib.ptr(ent),
+                              _lib.stream(self.dev))
+        return logp, ent
 
     def cut(self, logp_rows, entropy_rows):
         """``(log_probs, entropy)`` ``[B, L]`` fp32 in one launch; entropies are zeros for ``None``.  No autograd."""

@@ -3035,6 +3035,49 @@ def test_response_windows(dev, layout, index):
         ResponseWindows((n_seq, padded), {k: v.t() if k != "responses" else v for k, v in b.items()}, False)
 
 
+@pytest.mark.parametrize("layout", ["padded", "packed"])
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1000), (torch.bfloat16, 1003), (torch.float32, 4096),
+                                         (torch.float32, 77), (torch.float16, 8200)])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_scoring_pass_in_one_launch(dev, monkeypatch, layout, dtype, vocab, index):
+    """Windows scored cell by cell equal flagged rows, swept and cut, to the last bit: windows that start in front of
+    the rows, end behind them or behind the result, empty ones, rows with a stride, labels outside the vocabulary."""
+    from mindspeed_rl_amd import vocab_ops
+    gen = torch.Generator().manual_seed(vocab)
+    plen = torch.tensor([[1], [7], [3], [40], [4], [9], [0]], dtype=index)
+    rlen = torch.tensor([[5], [0], [50], [3], [60], [31], [38]], dtype=index)
+    n_seq, padded, kw = plen.shape[0], 37, {}
+    lead = (n_seq, padded)
+    if layout == "packed":
+        seqlens = torch.tensor([6, 7, 40, 43, 4, 40, 30], dtype=torch.int32)
+        cu = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(seqlens, 0)]).to(torch.int32)
+        lead = (1, int(cu[-1]) - 5)                                         # the last window ends behind the rows
+        kw = dict(use_remove_padding=True, seqlens_in_batch=seqlens.to(dev), cu_seqlens_padded=cu.to(dev), seq_len=43)
+    wide = (torch.randn(*lead, vocab + 5, generator=gen) * 3).to(dtype).to(dev)
+    labels = torch.randint(-1, vocab + 1, lead, generator=gen).to(index)
+    comp = mrl.StandardLogProbComputer()
+    calls = []
+    real = vocab_ops._timed_call
+    monkeypatch.setattr(vocab_ops, "_timed_call", lambda name, *a: (calls.append(name), real(name, *a)))
+    for width in (1, 12, 70):
+        b = _to_dev({"responses": torch.zeros(n_seq, width, dtype=torch.int64), "prompt_length": plen,
+                     "response_length": rlen, "labels": labels}, dev)
+        for out in (wide[..., :vocab].contiguous(), wide[..., :vocab]):
+            for skip in (False, True):
+                with torch.no_grad():
+                    got = comp.compute(out, b, skip, inv_temperature=1.25, **kw)
+                    monkeypatch.setattr(vocab_ops, "_EXTRA_CELLS", -(1 << 40))
+                    want = comp.compute(out, b, skip, inv_temperature=1.25, **kw)
+                    monkeypatch.undo()
+                    monkeypatch.setattr(vocab_ops, "_timed_call", lambda name, *a: (calls.append(name), real(name, *a)))
+                assert calls == ["mrl_window_logprob", "mrl_vocab_logprob_fwd"]
+                calls.clear()
+                assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and want[0].any().item()
+    with pytest.raises(RuntimeError), torch.autograd.forward_ad.dual_level():   # no forward-mode rule, as before
+        x = wide[..., :vocab].float().contiguous()
+        comp.compute(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), b, True, **kw)
+
+
 def test_log_prob_computer_uses_a_subclass_cut(dev):
     """A subclass that cuts the padded rows itself is asked to, in a pass without gradient as in one with."""
     from mindspeed_rl_amd.loss import StandardLogProbComputer
