@@ -12,6 +12,7 @@ using namespace mrl_loss;
 
 constexpr int kScanBlock = 512;
 constexpr int kScanChunk = 4096;     // entries of a row staged in LDS per step of the scan
+constexpr int kReplay = 16;          // steps of the scan between two results that the chain keeps
 constexpr int kReduceBlock = 1024;
 
 // Sum of one double per thread over a workgroup of kReduceBlock threads, fixed order; every thread
@@ -74,13 +75,18 @@ __global__ __launch_bounds__(256) void kl_rewards_kernel(const float* __restrict
 
 // ---------------------------------------------------------------------------- GAE reverse scan
 // One workgroup per sample.  The recurrence lastgaelam = delta_t + (gamma*lam) * lastgaelam is
-// evaluated by ONE thread in the reference's order and with its roundings (separate multiply and
+// evaluated in the reference's order and with its roundings (separate multiply and
 // add, no contraction), so advantages and returns are bit-identical to the torch loop.  gl is gamma*lam
 // as the host formed it: python multiplies the two in double and torch rounds the product to fp32 once.
 //
-// Bound by that chain: two dependent operations per token.  So nothing else is left on it: all threads
-// form the deltas, and the chain takes them from LDS four at a time, 16 steps ahead of their use
-// (batch 128 x width 2048: 28 us; with the deltas formed inside the chain from single entries 69 us).
+// Bound by that chain: two dependent operations per token, 13.3 cycles measured without anything else.  So
+// nothing else is left on it.  All threads form the deltas; one wavefront runs through them, 64 at a time in
+// the lanes of one register and read from there (v_readlane fits into the chain's own gaps, where a lane's own
+// LDS reads and writes of four entries took another 12 cycles a token), and keeps every 16th result only.  From
+// those all threads then take the 16 steps in between once more, side by side: the same operations on the same
+// operands, so the same bits.
+// Batch 128 x width 2048: 14.9 us, 14.4 cycles a token (24.4 with the chain in one lane, its entries by LDS);
+// x 4096 46.3 -> 27.1; 16 x 512 7.8 -> 5.5.  16 steps apart: each kept result costs the chain an LDS write.
 //
 // kMoments: leaves the masked moments (sum m, sum m x, sum m x^2) of the sample's advantages, in fp64, for
 // the whitening that follows.
@@ -94,81 +100,79 @@ __global__ __launch_bounds__(kScanBlock) void gae_scan_kernel(const float* __res
                                                               float gamma, float gl, float* __restrict__ adv,
                                                               float* __restrict__ ret, const void* __restrict__ mask,
                                                               int mdtype, Moments* __restrict__ moments) {
-    // A chunk of n tokens lies at the END of n rounded up to a multiple of 4 slots, so that the chain
-    // starts on a whole group of 4; only the last chunk (the row's beginning) can have empty slots in front.
-    __shared__ float4 chunk[kScanChunk / 4];
-    float* slot = reinterpret_cast<float*>(chunk);
+    // in the order of the chain: slot e is the chunk's e-th token from its end
+    __shared__ __attribute__((aligned(16))) float slot[kScanChunk + 64];
+    __shared__ float kept[kScanChunk / kReplay];           // results of steps kReplay - 1, 2 kReplay - 1, ...
     const int64_t base = (int64_t)blockIdx.x * width;
+    const int tid = (int)threadIdx.x;
     Moments mom = {0.0, 0.0, 0.0};
     constexpr int kPer = kScanChunk / kScanBlock;
-    float last = 0.f;                                      // thread 0's
+    float last = 0.f;                                      // result behind the chunk
     for (int64_t hi = width; hi > 0; hi -= kScanChunk) {
         const int64_t lo = hi > kScanChunk ? hi - kScanChunk : 0;
-        const int n = (int)(hi - lo), groups = (n + 3) >> 2, pad = groups * 4 - n;
+        const int n = (int)(hi - lo);
         const float* r = rewards + base + lo;
         const float* v = values + base + lo;
         // everything the chunk needs of memory is requested here, in one go; values and mask stay in registers
         float v_mine[kPer], m_mine[kPer], r_mine[kPer], v_next[kPer];
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int t = min(q * kScanBlock + (int)threadIdx.x, n - 1);
+            const int t = min(q * kScanBlock + tid, n - 1);
             r_mine[q] = r[t];
             v_mine[q] = v[t];
             v_next[q] = v[lo + t + 1 < width ? t + 1 : t];
-            if (kMoments) m_mine[q] = mask_at(mask, mdtype, nullptr, 0, 0, base + lo + t, 0);
+        }
+        if (kMoments) {
+#pragma unroll
+            for (int q = 0; q < kPer; ++q)
+                m_mine[q] = q * kScanBlock < n ? mask_at(mask, mdtype, nullptr, 0, 0, base + lo + min(q * kScanBlock + tid, n - 1), 0)
+                                               : 0.f;
         }
         __syncthreads();                                   // the previous chunk has been written out
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int t = q * kScanBlock + (int)threadIdx.x;
+            const int t = q * kScanBlock + tid;
             const float next = lo + t + 1 < width ? v_next[q] : 0.f;
-            if (t < n) slot[pad + t] = mrl::sub_rn(mrl::add_rn(r_mine[q], mrl::mul_rn(gamma, next)), v_mine[q]);
+            if (t < n) slot[n - 1 - t] = mrl::sub_rn(mrl::add_rn(r_mine[q], mrl::mul_rn(gamma, next)), v_mine[q]);
         }
-        if ((int)threadIdx.x < pad) slot[threadIdx.x] = 0.f;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            auto four = [&](float4& d) {
-                d.w = last = mrl::add_rn(d.w, mrl::mul_rn(gl, last));
-                d.z = last = mrl::add_rn(d.z, mrl::mul_rn(gl, last));
-                d.y = last = mrl::add_rn(d.y, mrl::mul_rn(gl, last));
-                d.x = last = mrl::add_rn(d.x, mrl::mul_rn(gl, last));
-            };
-            int g = groups - 1;
-            for (; (g + 1) & 7; --g) {                     // down to a multiple of 8 groups
-                float4 d = chunk[g];
-                four(d);
-                chunk[g] = d;
-            }
-            // 16 steps from one set of registers while the next 16 deltas arrive in the other
-            auto load = [&](float4(&d)[4], int at) {
+        const float behind = last;
+        if (tid < 64) {
+            // steps past the n-th take what lies in their slots; nobody looks at them
+            const int blocks = (n + 63) >> 6;
+            float d = slot[tid], x = behind;
+            for (int g = 0; g < blocks; ++g) {
+                const float d_next = slot[(g + 1) * 64 + tid];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) d[q] = chunk[at - q];
-            };
-            auto sixteen = [&](float4(&d)[4], int at) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    four(d[q]);
-                    chunk[at - q] = d[q];
+                for (int e = 0; e < 64; ++e) {
+                    const float delta = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(d), e));
+                    x = mrl::add_rn(delta, mrl::mul_rn(gl, x));
+                    if (e % kReplay == kReplay - 1) kept[(g * 64 + e) / kReplay] = x;      // the same from every lane
                 }
-            };
-            if (g >= 0) {
-                float4 even[4], odd[4];
-                load(even, g);
-                __builtin_amdgcn_s_waitcnt(0xC07F);        // nothing outstanding into the loop on either path
-                for (; g >= 0; g -= 8) {
-                    load(odd, g - 4);
-                    sixteen(even, g);
-                    load(even, g >= 8 ? g - 8 : g);        // these once more at the end, unused
-                    sixteen(odd, g - 4);
-                }
+                d = d_next;
             }
         }
+        __syncthreads();
+        if (tid * kReplay < n) {
+            float x = tid == 0 ? behind : kept[tid - 1];
+            float4* mine = reinterpret_cast<float4*>(slot + tid * kReplay);
+#pragma unroll
+            for (int g = 0; g < kReplay / 4; ++g) {
+                float4 d = mine[g];
+                d.x = x = mrl::add_rn(d.x, mrl::mul_rn(gl, x));
+                d.y = x = mrl::add_rn(d.y, mrl::mul_rn(gl, x));
+                d.z = x = mrl::add_rn(d.z, mrl::mul_rn(gl, x));
+                d.w = x = mrl::add_rn(d.w, mrl::mul_rn(gl, x));
+                mine[g] = d;
+            }
+        }
+        last = kept[kScanChunk / kReplay - 1];             // of a whole chunk; behind another there is none
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int t = q * kScanBlock + (int)threadIdx.x;
+            const int t = q * kScanBlock + tid;
             if (t >= n) break;
-            const float a = slot[pad + t];
+            const float a = slot[n - 1 - t];
             adv[base + lo + t] = a;
             ret[base + lo + t] = mrl::add_rn(a, v_mine[q]);
             if (kMoments && m_mine[q] != 0.f) {

@@ -569,6 +569,27 @@ def test_gae_and_whitening_parity(dev, batch, width):
         1.0, r.abs().max().item() * 2)
 
 
+@pytest.mark.parametrize("width", [1, 15, 16, 17, 63, 64, 65, 128, 129, 4096 + 15, 4096 + 65, 3 * 4096])
+def test_gae_scan_between_kept_results(dev, width):
+    """Every remainder of the chain's groups of 64, of the 16 steps taken once more and of a staged chunk, no decay, and
+    rewards that are infinite or NaN: the bits of the serial loop."""
+    gen = torch.Generator().manual_seed(width)
+    r, v = torch.randn(3, width, generator=gen), torch.randn(3, width, generator=gen)
+    r[1, width // 2], r[2, width - 1] = float("inf"), float("nan")
+    for gl in (1.0, 0.95, 0.5):
+        last, want = torch.zeros(3), torch.empty(3, width)
+        for t in reversed(range(width)):
+            following = v[:, t + 1] if t < width - 1 else torch.zeros(3)
+            last = (r[:, t] + 0.99 * following - v[:, t]) + gl * last
+            want[:, t] = last
+        rd, vd = r.to(dev), v.to(dev)
+        adv, ret = torch.empty_like(rd), torch.empty_like(rd)
+        _lib.call("mrl_gae_scan", rd.data_ptr(), vd.data_ptr(), 3, width, 0.99, gl, adv.data_ptr(), ret.data_ptr(),
+                  _lib.stream(dev))
+        assert torch.equal(adv.cpu().nan_to_num(7.0), want.nan_to_num(7.0)) and torch.equal(adv.cpu().isnan(), want.isnan())
+        assert torch.equal(ret.cpu().nan_to_num(7.0), (want + v).nan_to_num(7.0))
+
+
 @pytest.mark.parametrize("batch,width", [(1, 1), (2, 2), (1025, 3), (5, 17), (3, 4095), (2, 4096), (2, 4097), (1, 8195)])
 def test_gae_whitening_and_value_loss_at_the_edges_of_their_split(dev, batch, width):
     """Rows of one and of several staging chunks with every remainder of the groups of 4, more rows than
