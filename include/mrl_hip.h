@@ -58,6 +58,14 @@ int mrl_version(void);
 /* Message of the calling thread's last failed call ("" if none). */
 const char* mrl_last_error(void);
 
+/* Results for the host without a copy: an output may lie in pinned, coherent host memory (hipHostMalloc).  The
+ * caller fills it with MRL_HOST_EMPTY words, launches, and mrl_host_wait returns when none of the n_words 4-byte
+ * words is empty any more: it watches them for a millisecond, then synchronises the stream instead, so that a
+ * result that is MRL_HOST_EMPTY itself is waited for as well.  The one entry point that waits; not for a stream
+ * that is being captured. */
+#define MRL_HOST_EMPTY 0xffffffffu
+int mrl_host_wait(const void* words, int64_t n_words, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Vocabulary sweep, forward.  Replaces compute_log_probs (mindspeed_rl/utils/compute.py:29-51,
  * i.e. Megatron's vocab_parallel_cross_entropy at tp=1), _VocabParallelEntropy.forward
@@ -458,6 +466,15 @@ int mrl_fused_loss_reduce(const float* row_terms, const int64_t* row_start,
                           float clip_hi, int kl_penalty, float kl_coef, float entropy_coeff,
                           int seq_mean, float loss_scale, float* row_sums, float* out,
                           uint32_t* done_counter, float* loss_out, void* stream);
+/* The same; host_out (nullable): out[8] once more, in host memory (see mrl_host_wait). */
+int mrl_fused_loss_reduce_host(const float* row_terms, const int64_t* row_start,
+                               const int32_t* row_count, int64_t batch, int64_t width,
+                               const float* old_log_prob, const float* ref_log_prob,
+                               const float* advantages, const void* mask, int mask_dtype,
+                               const void* response_length, int response_dtype, float clip_lo,
+                               float clip_hi, int kl_penalty, float kl_coef, float entropy_coeff,
+                               int seq_mean, float loss_scale, float* row_sums, float* out,
+                               uint32_t* done_counter, float* loss_out, float* host_out, void* stream);
 
 /* x[r, :] *= (*upstream / *applied) in place, unless that ratio is exactly 1 (then the kernel
  * exits without touching memory).  upstream and applied are DEVICE scalars: the gradient autograd
@@ -601,6 +618,12 @@ int64_t mrl_gae_whiten_workspace_bytes(int64_t batch);
 int mrl_gae_whiten(const float* rewards, const float* values, const void* mask, int mask_dtype,
                    int64_t batch, int64_t width, float gamma, float gamma_lam, float* advantages,
                    float* returns, double* info, void* workspace, int64_t workspace_bytes, void* stream);
+/* The same; host_sums (nullable, [batch] in host memory, see mrl_host_wait): the sum of each row's mask, which the
+ * scan has before its serial part starts. */
+int mrl_gae_whiten_host(const float* rewards, const float* values, const void* mask, int mask_dtype,
+                        int64_t batch, int64_t width, float gamma, float gamma_lam, float* advantages,
+                        float* returns, double* info, double* host_sums, void* workspace,
+                        int64_t workspace_bytes, void* stream);
 
 /* mrl_masked_whiten: masked_whiten / masked_var / masked_mean (mindspeed_rl/utils/
  * torch_functional.py:46-106) over n entries: mean = sum(x*mask)/(sum(mask)+1e-8), var the same of
@@ -646,6 +669,13 @@ int mrl_critic_loss_fwd_slope(const float* head, int64_t batch, int64_t padded_s
                               int64_t width, float cliprange_value, float loss_scale, float* slope,
                               float* out, float* loss_out, void* workspace, int64_t workspace_bytes,
                               void* stream);
+/* The forward with host_out (nullable): out[4] once more, in host memory (see mrl_host_wait). */
+int mrl_critic_loss_fwd_slope_host(const float* head, int64_t batch, int64_t padded_s,
+                                   const void* prompt_length, int prompt_dtype,
+                                   const void* response_length, int response_dtype, const float* returns,
+                                   const float* values, int64_t width, float cliprange_value,
+                                   float loss_scale, float* slope, float* out, float* loss_out,
+                                   float* host_out, void* workspace, int64_t workspace_bytes, void* stream);
 int mrl_critic_loss_bwd_slope(const float* slope, int64_t batch, int64_t padded_s,
                               const void* prompt_length, int prompt_dtype, const void* response_length,
                               int response_dtype, int64_t width, float loss_scale, const float* out,

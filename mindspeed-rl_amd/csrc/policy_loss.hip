@@ -29,6 +29,30 @@ __device__ __forceinline__ double block_sum(double v, double* lds) {
     return r;
 }
 
+// N sums at once, each as block_sum takes it: one pair of barriers for all of them.
+template <int N>
+__device__ __forceinline__ void block_sums(double (&v)[N], double (*lds)[kWaves]) {
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) lds[q][threadIdx.x >> 6] = v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        double r = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) r += lds[q][w];
+        v[q] = r;
+    }
+}
+constexpr int kSums = 7;                // the most that are taken at once
+
 __device__ __forceinline__ int64_t load_i64(const void* p, int dtype, int64_t i) {
     return dtype == MRL_I32 ? (int64_t) reinterpret_cast<const int32_t*>(p)[i] : reinterpret_cast<const int64_t*>(p)[i];
 }
@@ -69,26 +93,24 @@ __global__ __launch_bounds__(kBlock) void policy_loss_rows_kernel(
 // written by other workgroups of the SAME launch with device-scope stores and are read likewise.
 template <bool kCoherent>
 __device__ __forceinline__ void finalize_sums(const float* row_sums, int64_t batch, const Params& p,
-                                              float* __restrict__ out, float* __restrict__ loss_out, double* lds) {
+                                              float* __restrict__ out, float* __restrict__ loss_out,
+                                              float* __restrict__ host_out, double (*lds)[kWaves]) {
     auto at = [&](int64_t e) {
         return kCoherent ? __hip_atomic_load(row_sums + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : row_sums[e];
     };
-    double acc[6] = {0, 0, 0, 0, 0, 0};
-    double seq_acc = 0.0;
+    double tot[kSums] = {0, 0, 0, 0, 0, 0, 0};             // the six sums, and the sequences' means
     for (int64_t i = threadIdx.x; i < batch; i += kBlock) {
         float v[6];
 #pragma unroll
         for (int q = 0; q < 6; ++q) {
             v[q] = at(i * S_N + q);
-            acc[q] += (double)v[q];
+            tot[q] += (double)v[q];
         }
         // per-sequence token mean, no epsilon: 0/0 = NaN for an all-masked row (as the reference)
-        seq_acc += (double)(v[S_PG] / v[S_MASK]);
+        tot[6] += (double)(v[S_PG] / v[S_MASK]);
     }
-    double tot[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) tot[q] = block_sum(acc[q], lds);
-    const double seq_tot = block_sum(seq_acc, lds);
+    block_sums(tot, lds);
+    const double seq_tot = tot[6];
     if (threadIdx.x == 0) {
         const double denom = tot[S_MASK] + 1e-8;
         const float clipfrac = p.seq_mean ? 0.f : (float)(tot[S_CLIP] / denom);
@@ -97,14 +119,12 @@ __device__ __forceinline__ void finalize_sums(const float* row_sums, int64_t bat
         const float kl_mean = p.kl_penalty == MRL_KL_NONE ? 0.f : (float)(tot[S_KL] / denom);
         const float ent_mean = (float)(tot[S_ENT] / denom);
         const float pg_loss = pg_mean + kl_mean * p.kl_coef - p.entropy_coeff * ent_mean;
-        out[0] = pg_loss * p.loss_scale;
-        out[1] = pg_loss;
-        out[2] = clipfrac;
-        out[3] = ppo_kl;
-        out[4] = kl_mean;
-        out[5] = ent_mean;
-        out[6] = (float)tot[S_MASK];
-        out[7] = (float)batch;
+        const float all[8] = {pg_loss * p.loss_scale, pg_loss, clipfrac, ppo_kl, kl_mean, ent_mean, (float)tot[S_MASK], (float)batch};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            out[q] = all[q];
+            if (host_out) host_out[q] = all[q];
+        }
         if (loss_out) *loss_out = pg_loss * p.loss_scale;
     }
 }
@@ -112,9 +132,10 @@ __device__ __forceinline__ void finalize_sums(const float* row_sums, int64_t bat
 __global__ __launch_bounds__(kBlock) void policy_loss_finalize_kernel(const float* __restrict__ row_sums,
                                                                       int64_t batch, Params p,
                                                                       float* __restrict__ out,
-                                                                      float* __restrict__ loss_out) {
-    __shared__ double lds[kWaves];
-    finalize_sums<false>(row_sums, batch, p, out, loss_out, lds);
+                                                                      float* __restrict__ loss_out,
+                                                                      float* __restrict__ host_out) {
+    __shared__ double lds[kSums][kWaves];
+    finalize_sums<false>(row_sums, batch, p, out, loss_out, host_out, lds);
 }
 
 __global__ __launch_bounds__(kBlock) void policy_loss_bwd_kernel(
@@ -307,8 +328,9 @@ __global__ __launch_bounds__(kBlock) void fused_seq_reduce_kernel(
     const float* __restrict__ row_terms, const int64_t* __restrict__ row_start, const int32_t* __restrict__ row_count,
     int64_t width, const float* __restrict__ old, const float* __restrict__ ref, const float* __restrict__ adv,
     const void* __restrict__ mask, int mdtype, const void* __restrict__ resp, int rdtype, Params p,
-    float* row_sums, uint32_t* done, float* __restrict__ out, float* __restrict__ loss_out) {
-    __shared__ double lds[kWaves];
+    float* row_sums, uint32_t* done, float* __restrict__ out, float* __restrict__ loss_out,
+    float* __restrict__ host_out) {
+    __shared__ double lds[kSums][kWaves];
     __shared__ uint32_t last;
     const int64_t i = blockIdx.x;
     const int64_t start = row_start[i];
@@ -332,8 +354,12 @@ __global__ __launch_bounds__(kBlock) void fused_seq_reduce_kernel(
         }
     }
     float sums[S_N] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    double wide[6];
 #pragma unroll
-    for (int q = 0; q < 6; ++q) sums[q] = (float)block_sum((double)acc[q], lds);
+    for (int q = 0; q < 6; ++q) wide[q] = (double)acc[q];
+    block_sums(wide, lds);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) sums[q] = (float)wide[q];
     if (threadIdx.x == 0) {
         if (done == nullptr) {
 #pragma unroll
@@ -349,7 +375,7 @@ __global__ __launch_bounds__(kBlock) void fused_seq_reduce_kernel(
     if (done == nullptr) return;
     __syncthreads();
     if (last == 0u) return;                                    // uniform
-    finalize_sums<true>(row_sums, (int64_t)gridDim.x, p, out, loss_out, lds);
+    finalize_sums<true>(row_sums, (int64_t)gridDim.x, p, out, loss_out, host_out, lds);
     if (threadIdx.x == 0) __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -398,7 +424,7 @@ extern "C" int mrl_policy_loss_fwd(const float* log_prob, const float* old_log_p
         if (rc != MRL_OK) return rc;
     }
     hipLaunchKernelGGL(policy_loss_finalize_kernel, dim3(1), dim3(kBlock), 0, s, (const float*)row_sums, batch, p,
-                       out, (float*)nullptr);
+                       out, (float*)nullptr, (float*)nullptr);
     return mrl::check_launch(fn);
 }
 
@@ -497,24 +523,38 @@ extern "C" int mrl_fused_loss_reduce(const float* row_terms, const int64_t* row_
                                      float clip_hi, int kl_penalty, float kl_coef, float entropy_coeff, int seq_mean,
                                      float loss_scale, float* row_sums, float* out, uint32_t* done_counter,
                                      float* loss_out, void* stream) {
+    return mrl_fused_loss_reduce_host(row_terms, row_start, row_count, batch, width, old_log_prob, ref_log_prob, advantages,
+                                      mask, mask_dtype, response_length, response_dtype, clip_lo, clip_hi, kl_penalty,
+                                      kl_coef, entropy_coeff, seq_mean, loss_scale, row_sums, out, done_counter, loss_out,
+                                      nullptr, stream);
+}
+
+extern "C" int mrl_fused_loss_reduce_host(const float* row_terms, const int64_t* row_start, const int32_t* row_count,
+                                          int64_t batch, int64_t width, const float* old_log_prob,
+                                          const float* ref_log_prob, const float* advantages, const void* mask,
+                                          int mask_dtype, const void* response_length, int response_dtype,
+                                          float clip_lo, float clip_hi, int kl_penalty, float kl_coef,
+                                          float entropy_coeff, int seq_mean, float loss_scale, float* row_sums,
+                                          float* out, uint32_t* done_counter, float* loss_out, float* host_out,
+                                          void* stream) {
     const char* fn = "mrl_fused_loss_reduce";
     int rc = check_args(fn, (const float*)row_terms, ref_log_prob, advantages, mask, mask_dtype, response_length,
                         response_dtype, batch, width, kl_penalty, seq_mean);
     if (rc != MRL_OK) return rc;
     MRL_REQUIRE(out != nullptr && (batch == 0 || (row_sums && row_start && row_count)), MRL_ERR_INVALID_ARG,
                 "%s: NULL pointer", fn);
-    MRL_REQUIRE(mrl::aligned(done_counter, 4) && mrl::aligned(loss_out, 4), MRL_ERR_MISALIGNED,
-                "%s: done_counter and loss_out must be 4-byte aligned", fn);
+    MRL_REQUIRE(mrl::aligned(done_counter, 4) && mrl::aligned(loss_out, 4) && mrl::aligned(host_out, 4), MRL_ERR_MISALIGNED,
+                "%s: done_counter, loss_out and host_out must be 4-byte aligned", fn);
     const Params p = {clip_lo, clip_hi, kl_coef, entropy_coeff, loss_scale, kl_penalty, seq_mean};
     hipStream_t s = mrl::as_stream(stream);
     if (batch > 0) {
         hipLaunchKernelGGL(fused_seq_reduce_kernel, dim3((unsigned)batch), dim3(kBlock), 0, s, row_terms, row_start,
                            row_count, width, old_log_prob, ref_log_prob, advantages, mask, mask_dtype, response_length,
-                           response_dtype, p, row_sums, done_counter, out, loss_out);
+                           response_dtype, p, row_sums, done_counter, out, loss_out, host_out);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK || done_counter != nullptr) return rc;
     }
     hipLaunchKernelGGL(policy_loss_finalize_kernel, dim3(1), dim3(kBlock), 0, s, (const float*)row_sums, batch, p, out,
-                       loss_out);
+                       loss_out, host_out);
     return mrl::check_launch(fn);
 }

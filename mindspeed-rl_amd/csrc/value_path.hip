@@ -99,12 +99,15 @@ __global__ __launch_bounds__(kScanBlock) void gae_scan_kernel(const float* __res
                                                               const float* __restrict__ values, int64_t width,
                                                               float gamma, float gl, float* __restrict__ adv,
                                                               float* __restrict__ ret, const void* __restrict__ mask,
-                                                              int mdtype, Moments* __restrict__ moments) {
+                                                              int mdtype, Moments* __restrict__ moments,
+                                                              double* __restrict__ host_sums) {
     // in the order of the chain: slot e is the chunk's e-th token from its end
     __shared__ __attribute__((aligned(16))) float slot[kScanChunk + 64];
     __shared__ float kept[kScanChunk / kReplay];           // results of steps kReplay - 1, 2 kReplay - 1, ...
     const int64_t base = (int64_t)blockIdx.x * width;
     const int tid = (int)threadIdx.x;
+    __shared__ double wave_masked[kScanBlock / 64];
+    double masked = 0.0;
     Moments mom = {0.0, 0.0, 0.0};
     constexpr int kPer = kScanChunk / kScanBlock;
     float last = 0.f;                                      // result behind the chunk
@@ -135,7 +138,22 @@ __global__ __launch_bounds__(kScanBlock) void gae_scan_kernel(const float* __res
             const float next = lo + t + 1 < width ? v_next[q] : 0.f;
             if (t < n) slot[n - 1 - t] = mrl::sub_rn(mrl::add_rn(r_mine[q], mrl::mul_rn(gamma, next)), v_mine[q]);
         }
+        if (kMoments && host_sums) {
+            // the row's mask sum, for a caller that waits for nothing else; on its way before the chain starts
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) masked += q * kScanBlock + tid < n ? (double)m_mine[q] : 0.0;
+            double s = masked;
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+            if ((tid & 63) == 0) wave_masked[tid >> 6] = s;
+        }
         __syncthreads();
+        if (kMoments && host_sums && lo == 0 && tid == kScanBlock - 1) {
+            double s = wave_masked[0];
+            for (int w = 1; w < kScanBlock / 64; ++w) s += wave_masked[w];
+            // past the caches, which would keep it until the kernel ends
+            __hip_atomic_store(host_sums + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         const float behind = last;
         if (tid < 64) {
             // steps past the n-th take what lies in their slots; nobody looks at them
@@ -313,7 +331,8 @@ __device__ __forceinline__ ValueTerm value_term(float vp, float ret, float v, fl
 // masked_mean(l2 > l1), out[3] = sum(mask)
 // (loss_out, if given: out[0] once more, a 0-dim tensor of its own for autograd)
 __device__ __forceinline__ void write_value_loss(double ssum, double csum, double count, float loss_scale,
-                                                 float* __restrict__ out, float* __restrict__ loss_out) {
+                                                 float* __restrict__ out, float* __restrict__ loss_out,
+                                                 float* __restrict__ host_out = nullptr) {
     const float denom = (float)count + 1e-8f;
     const float vf = 0.5f * ((float)ssum / denom);
     out[0] = loss_scale * vf;
@@ -321,6 +340,10 @@ __device__ __forceinline__ void write_value_loss(double ssum, double csum, doubl
     out[2] = (float)csum / denom;
     out[3] = (float)count;
     if (loss_out) *loss_out = loss_scale * vf;
+    if (host_out) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) host_out[q] = out[q];
+    }
 }
 
 __global__ __launch_bounds__(kReduceBlock) void value_loss_fwd_kernel(
@@ -424,12 +447,13 @@ __global__ __launch_bounds__(256) void value_loss_rows_kernel(
 
 __global__ __launch_bounds__(kReduceBlock) void value_loss_finish_kernel(const LossSums* __restrict__ sums, int n,
                                                                         float loss_scale, float* __restrict__ out,
-                                                                        float* __restrict__ loss_out) {
+                                                                        float* __restrict__ loss_out,
+                                                                        float* __restrict__ host_out) {
     __shared__ double lds[kReduceBlock / 64 + 1];
     LossSums s = {0.0, 0.0, 0.0};
     if ((int)threadIdx.x < n) s = sums[threadIdx.x];       // n <= kLossRows = kReduceBlock
     const double ssum = block_sum(s.loss, lds), csum = block_sum(s.clipped, lds), count = block_sum(s.count, lds);
-    if (threadIdx.x == 0) write_value_loss(ssum, csum, count, loss_scale, out, loss_out);
+    if (threadIdx.x == 0) write_value_loss(ssum, csum, count, loss_scale, out, loss_out, host_out);
 }
 static_assert(kLossRows == kReduceBlock, "the finishing workgroup takes one partial sum per thread");
 
@@ -519,7 +543,7 @@ extern "C" int mrl_gae_scan(const float* rewards, const float* values, int64_t b
                 MRL_ERR_INVALID_ARG, "%s: outputs must not alias the inputs or each other", fn);
     hipLaunchKernelGGL(gae_scan_kernel<false>, dim3((unsigned)batch), dim3(kScanBlock), 0, mrl::as_stream(stream),
                        rewards, values, width, gamma, gamma_lam, advantages, returns, (const void*)nullptr, 0,
-                       (Moments*)nullptr);
+                       (Moments*)nullptr, (double*)nullptr);
     return mrl::check_launch(fn);
 }
 
@@ -530,6 +554,14 @@ extern "C" int64_t mrl_gae_whiten_workspace_bytes(int64_t batch) {
 extern "C" int mrl_gae_whiten(const float* rewards, const float* values, const void* mask, int mask_dtype, int64_t batch,
                               int64_t width, float gamma, float gamma_lam, float* advantages, float* returns,
                               double* info, void* workspace, int64_t workspace_bytes, void* stream) {
+    return mrl_gae_whiten_host(rewards, values, mask, mask_dtype, batch, width, gamma, gamma_lam, advantages, returns, info,
+                               nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mrl_gae_whiten_host(const float* rewards, const float* values, const void* mask, int mask_dtype,
+                                   int64_t batch, int64_t width, float gamma, float gamma_lam, float* advantages,
+                                   float* returns, double* info, double* host_sums, void* workspace,
+                                   int64_t workspace_bytes, void* stream) {
     const char* fn = "mrl_gae_whiten";
     MRL_REQUIRE(batch >= 0 && width > 0 && batch <= 0x7fffffffLL, MRL_ERR_INVALID_ARG, "%s: batch=%lld width=%lld", fn,
                 (long long)batch, (long long)width);
@@ -537,8 +569,8 @@ extern "C" int mrl_gae_whiten(const float* rewards, const float* values, const v
     MRL_REQUIRE(info != nullptr, MRL_ERR_INVALID_ARG, "%s: info is NULL", fn);
     MRL_REQUIRE(batch == 0 || (rewards && values && mask && advantages && returns && workspace), MRL_ERR_INVALID_ARG,
                 "%s: NULL pointer", fn);
-    MRL_REQUIRE(mrl::aligned(workspace, 8) && mrl::aligned(info, 8), MRL_ERR_MISALIGNED,
-                "%s: workspace and info must be 8-byte aligned", fn);
+    MRL_REQUIRE(mrl::aligned(workspace, 8) && mrl::aligned(info, 8) && mrl::aligned(host_sums, 8), MRL_ERR_MISALIGNED,
+                "%s: workspace, info and host_sums must be 8-byte aligned", fn);
     MRL_REQUIRE(workspace_bytes >= mrl_gae_whiten_workspace_bytes(batch), MRL_ERR_INVALID_ARG,
                 "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
                 (long long)mrl_gae_whiten_workspace_bytes(batch));
@@ -549,7 +581,7 @@ extern "C" int mrl_gae_whiten(const float* rewards, const float* values, const v
     Moments* moments = reinterpret_cast<Moments*>(workspace);
     if (batch > 0) {
         hipLaunchKernelGGL(gae_scan_kernel<true>, dim3((unsigned)batch), dim3(kScanBlock), 0, s, rewards, values, width,
-                           gamma, gamma_lam, advantages, returns, mask, mask_dtype, moments);
+                           gamma, gamma_lam, advantages, returns, mask, mask_dtype, moments, host_sums);
         const int rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
@@ -619,7 +651,7 @@ extern "C" int mrl_value_loss_fwd_split(const float* vpreds, const float* return
         if (rc != MRL_OK) return rc;
     }
     hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums,
-                       (int)(grid.x * grid.y), loss_scale, out, loss_out);
+                       (int)(grid.x * grid.y), loss_scale, out, loss_out, (float*)nullptr);
     return mrl::check_launch(fn);
 }
 
@@ -636,13 +668,25 @@ extern "C" int mrl_critic_loss_fwd_slope(const float* head, int64_t batch, int64
                                          const float* returns, const float* values, int64_t width,
                                          float cliprange_value, float loss_scale, float* slope, float* out,
                                          float* loss_out, void* workspace, int64_t workspace_bytes, void* stream) {
+    return mrl_critic_loss_fwd_slope_host(head, batch, padded_s, prompt_length, prompt_dtype, response_length, response_dtype,
+                                          returns, values, width, cliprange_value, loss_scale, slope, out, loss_out,
+                                          nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mrl_critic_loss_fwd_slope_host(const float* head, int64_t batch, int64_t padded_s, const void* prompt_length,
+                                              int prompt_dtype, const void* response_length, int response_dtype,
+                                              const float* returns, const float* values, int64_t width,
+                                              float cliprange_value, float loss_scale, float* slope, float* out,
+                                              float* loss_out, float* host_out, void* workspace,
+                                              int64_t workspace_bytes, void* stream) {
     const char* fn = "mrl_critic_loss_fwd_slope";
     int rc = check_critic(fn, batch, padded_s, width, prompt_dtype, response_dtype);
     if (rc != MRL_OK) return rc;
     MRL_REQUIRE(out != nullptr && (batch == 0 || ((head || padded_s == 0) && prompt_length && response_length && returns &&
                                                   values && slope && workspace)),
                 MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
-    MRL_REQUIRE(mrl::aligned(workspace, 8), MRL_ERR_MISALIGNED, "%s: workspace must be 8-byte aligned", fn);
+    MRL_REQUIRE(mrl::aligned(workspace, 8) && mrl::aligned(host_out, 4), MRL_ERR_MISALIGNED,
+                "%s: workspace must be 8-byte and host_out 4-byte aligned", fn);
     MRL_REQUIRE(workspace_bytes >= mrl_value_loss_workspace_bytes(batch), MRL_ERR_INVALID_ARG,
                 "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
                 (long long)mrl_value_loss_workspace_bytes(batch));
@@ -657,7 +701,7 @@ extern "C" int mrl_critic_loss_fwd_slope(const float* head, int64_t batch, int64
         if (rc != MRL_OK) return rc;
     }
     hipLaunchKernelGGL(value_loss_finish_kernel, dim3(1), dim3(kReduceBlock), 0, s, (const LossSums*)sums,
-                       (int)(grid.x * grid.y), loss_scale, out, loss_out);
+                       (int)(grid.x * grid.y), loss_scale, out, loss_out, host_out);
     return mrl::check_launch(fn);
 }
 

@@ -41,6 +41,7 @@ RAGGED_COLUMNS = 16         # MRL_RAGGED_COLUMNS
 SIGNATURES = {
     "mrl_version": [],
     "mrl_last_error": [],
+    "mrl_host_wait": [_vp, _i64, _vp],
     "mrl_vocab_logprob_fwd": [_vp, _int, _i64, _i64, _i64, _vp, _int, _vp, _f32, _vp, _vp, _vp, _vp],
     "mrl_vocab_logprob_bwd": [_vp, _int, _i64, _i64, _i64, _vp, _int, _f32, _vp, _vp, _vp, _vp, _vp, _int, _i64, _vp],
     "mrl_pack_index_build": [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp, _vp],
@@ -79,6 +80,8 @@ SIGNATURES = {
     "mrl_set_wide_spin_limit": [_i64],
     "mrl_fused_loss_reduce": [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _int, _vp, _int, _f32, _f32, _int, _f32,
                               _f32, _int, _f32, _vp, _vp, _vp, _vp, _vp],
+    "mrl_fused_loss_reduce_host": [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _int, _vp, _int, _f32, _f32, _int, _f32,
+                              _f32, _int, _f32, _vp, _vp, _vp, _vp, _vp, _vp],
     "mrl_scale_rows": [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp],
     "mrl_grad_scale_note": [_vp, _vp, _vp, _vp, _vp],
     "mrl_scale_rows_note": [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
@@ -96,11 +99,13 @@ SIGNATURES = {
     "mrl_gae_scan": [_vp, _vp, _i64, _i64, _f32, _f32, _vp, _vp, _vp],
     "mrl_gae_whiten_workspace_bytes": [_i64],
     "mrl_gae_whiten": [_vp, _vp, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
+    "mrl_gae_whiten_host": [_vp, _vp, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "mrl_masked_whiten": [_vp, _vp, _int, _i64, _int, _vp, _vp, _vp],
     "mrl_value_loss_fwd": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp],
     "mrl_value_loss_workspace_bytes": [_i64],
     "mrl_value_loss_fwd_split": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _i64, _vp],
     "mrl_critic_loss_fwd_slope": [_vp, _i64, _i64, _vp, _int, _vp, _int, _vp, _vp, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
+    "mrl_critic_loss_fwd_slope_host": [_vp, _i64, _i64, _vp, _int, _vp, _int, _vp, _vp, _i64, _f32, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "mrl_critic_loss_bwd_slope": [_vp, _i64, _i64, _vp, _int, _vp, _int, _i64, _f32, _vp, _vp, _vp, _vp],
     "mrl_value_loss_bwd": [_vp, _vp, _vp, _vp, _int, _vp, _int, _i64, _i64, _f32, _f32, _vp, _vp, _vp, _vp],
     "mrl_copy_bytes": [_vp, _vp, _i64, _vp],
@@ -217,3 +222,52 @@ def index_column(t, dev):
     if t.device != dev:
         t = t.to(dev)
     return (t if t.dim() == 1 else t.reshape(-1)).contiguous()
+
+
+# ------------------------------------------------------------------------------------ results for the host
+class HostWords:
+    """A slot of pinned host memory that a kernel leaves a few numbers in: the host watches it instead of copying
+    from the device and waiting for the copy.  ``addr`` goes to the kernel as the address of its output; one of the
+    readers waits for the numbers, takes them and gives the slot back.  Where that fails the slot is not used again:
+    a kernel may still write to it."""
+
+    BYTES = 4096
+    _free = {}                  # device index -> slots that nothing writes to (list operations are atomic)
+    _BLOCK = 16                 # slots that are allocated together; there are as many as were ever taken at once
+
+    def __init__(self, f32, key):
+        self.f32, self.addr, self._key = f32, f32.data_ptr(), key
+
+    @classmethod
+    def take(cls, dev, n_bytes):
+        """An empty slot of ``n_bytes``, or None: more than a slot holds, or the stream is being captured (the
+        numbers will be there after a replay, not now)."""
+        if n_bytes > cls.BYTES or torch.cuda.is_current_stream_capturing():
+            return None
+        free = cls._free.setdefault(dev.index, [])
+        try:
+            slot = free.pop()
+        except IndexError:
+            block = torch.empty((cls._BLOCK, cls.BYTES // 4), dtype=torch.float32, pin_memory=True)
+            slot, *more = [cls(row, dev.index) for row in block.unbind(0)]
+            free.extend(more)
+        ctypes.memset(slot.addr, 0xff, n_bytes)
+        return slot
+
+    def _arrived(self, n_bytes, stream):
+        call("mrl_host_wait", self.addr, n_bytes // 4, stream)
+
+    def read(self, ctype, n, stream):
+        """``n`` numbers of a ctypes type, as a list."""
+        kind = ctype * n
+        self._arrived(ctypes.sizeof(kind), stream)
+        values = kind.from_address(self.addr)[:]
+        self._free[self._key].append(self)
+        return values
+
+    def read_doubles_of(self, n, stream):
+        """``n`` fp32 numbers as a host tensor of doubles."""
+        self._arrived(4 * n, stream)
+        values = self.f32[:n].double()
+        self._free[self._key].append(self)
+        return values

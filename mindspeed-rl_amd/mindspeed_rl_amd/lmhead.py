@@ -6,6 +6,8 @@ The reference has no such function: ``GPTModel.output_layer`` materialises the l
 forward-only form, which serves ``compute_log_prob`` / ``compute_ref_log_prob`` (two of the three
 vocabulary sweeps of a GRPO iteration).
 """
+import ctypes
+
 import torch
 
 from . import _lib, vocab_ops
@@ -109,11 +111,15 @@ class _LiveRows:
         self.dev, self.n_all = dev, n
         blocks = (n + 1023) // 1024
         index = torch.empty(2 * n + blocks, dtype=torch.int32, device=dev)
-        total = torch.empty(1, dtype=torch.int64, device=dev)
+        slot = _lib.HostWords.take(dev, 8) if n > 0 else None
+        total = torch.empty(1, dtype=torch.int64, device=dev) if slot is None else None
         self.live, self.place = index[:n], index[n:2 * n]
         _lib.call("mrl_live_rows", flags if isinstance(flags, int) else _lib.ptr(flags), dtype, stride, n,
-                  index.data_ptr(), index.data_ptr() + 4 * n, index.data_ptr() + 8 * n, _lib.ptr(total), _lib.stream(dev))
-        self.n = int(total.item()) if n > 0 else 0
+                  index.data_ptr(), index.data_ptr() + 4 * n, index.data_ptr() + 8 * n, slot.addr if slot is not None else _lib.ptr(total), _lib.stream(dev))
+        if slot is not None:
+            (self.n,) = slot.read(ctypes.c_int64, 1, _lib.stream(dev))
+        else:
+            self.n = int(total.item()) if n > 0 else 0
 
     def gather(self, table, labels, ops):
         """The live rows of `table` [n, W] (W whole 16-byte vectors), of `labels` [n] and - unless None - of `ops`
@@ -251,7 +257,7 @@ class _FusedLmHeadLoss(torch.autograd.Function):
 def fused_lmhead_policy_loss(hidden, weight, batch, *, packed, seqlens=None, cu_seqlens=None, mask=None,
                              ref_log_prob=None, clip_low, clip_high, kl_penalty=None, kl_coef=0.0, entropy_coeff=0.0,
                              token_level_loss=True, loss_scale=1.0, inv_temperature=1.0, expected_upstream=None,
-                             scale_state=None, chunk_rows=32768, compact_rows=True):
+                             scale_state=None, chunk_rows=32768, compact_rows=True, sent=None):
     """Policy loss straight from the hidden states: ``hidden`` is packed ``[1, T, H]`` (or padded
     ``[B, S, H]``) bf16, ``weight`` the ``[V, H]`` bf16 lm_head weight; ``batch`` as for
     :func:`mindspeed_rl_amd.fused_logprob_policy_loss` (``labels, responses, response_length,
@@ -276,5 +282,5 @@ def fused_lmhead_policy_loss(hidden, weight, batch, *, packed, seqlens=None, cu_
                kl_coef=float(kl_coef), entropy_coeff=float(entropy_coeff), seq_mean=0 if token_level_loss else 1,
                loss_scale=float(loss_scale), inv_temperature=float(inv_temperature),
                expected_upstream=None if expected_upstream is None else float(expected_upstream),
-               scale_state=scale_state, chunk_rows=int(chunk_rows), compact_rows=bool(compact_rows))
+               scale_state=scale_state, chunk_rows=int(chunk_rows), compact_rows=bool(compact_rows), sent=sent)
     return _FusedLmHeadLoss.apply(hidden, weight, batch["labels"], batch, cfg)

@@ -8,6 +8,7 @@ text-only log-prob strategy (``logprob_computer.py:73-145``), ``GRPOActorLossFun
 signatures, keyword arguments, return values and error behaviour are the reference's; the work
 is done by the HIP kernels of libmrl_hip.so.
 """
+import ctypes
 import os
 from abc import ABC, abstractmethod
 from typing import Dict, Tuple
@@ -313,11 +314,15 @@ class _FusedOperands:
         cfg = self.cfg
         # word 1 of the cleared sweep workspace counts the workgroups of the reduce step
         done = self.workspace + 4 if self.n_rows > 0 else None
-        _lib.call("mrl_fused_loss_reduce", self.p_terms if p_terms is None else p_terms, self.p_start, self.p_count,
+        sent = cfg.get("sent")
+        slot = _lib.HostWords.take(self.dev, 32) if sent is not None else None
+        _lib.call("mrl_fused_loss_reduce_host", self.p_terms if p_terms is None else p_terms, self.p_start, self.p_count,
                   self.n_seq, self.width, _lib.ptr(self.old), _lib.ptr(self.ref), _lib.ptr(self.adv),
                   _lib.ptr(self.mask_t), self.mdt, _lib.ptr(self.resp), self.rdt, cfg["clip_lo"], cfg["clip_hi"],
                   cfg["kl_penalty"], cfg["kl_coef"], cfg["entropy_coeff"], cfg["seq_mean"], cfg["loss_scale"],
-                  self.p_sums, _lib.ptr(self.out), done, _lib.ptr(self.loss), stream)
+                  self.p_sums, _lib.ptr(self.out), done, _lib.ptr(self.loss), slot.addr if slot is not None else None, stream)
+        if slot is not None:
+            sent.append(slot)
 
 
 class _FusedLogprobLoss(torch.autograd.Function):
@@ -381,7 +386,7 @@ class _FusedLogprobLoss(torch.autograd.Function):
 def fused_logprob_policy_loss(output, batch, *, packed, seqlens=None, cu_seqlens=None, mask=None, ref_log_prob=None,
                               clip_low, clip_high, kl_penalty=None, kl_coef=0.0, entropy_coeff=0.0,
                               token_level_loss=True, loss_scale=1.0, inv_temperature=1.0, grad_inplace=False,
-                              expected_upstream=None, scale_state=None):
+                              expected_upstream=None, scale_state=None, sent=None):
     """Log-prob, entropy, policy loss AND dlogits in one sweep over the logits.
 
     ``output`` is the packed ``[1, T, V]`` (``packed=True``, with ``seqlens`` / ``cu_seqlens``) or
@@ -390,7 +395,8 @@ def fused_logprob_policy_loss(output, batch, *, packed, seqlens=None, cu_seqlens
     :func:`policy_loss`.  The gradients are written with the scale the caller is expected to
     multiply the loss by before ``backward()``: ``expected_upstream`` if given, else what
     ``scale_state`` (a :class:`GradScaleState`) learned from the previous backward, else 1; any
-    other upstream value is honoured by one rescale pass in the backward."""
+    other upstream value is honoured by one rescale pass in the backward.  ``sent``: a list that receives the
+    :class:`_lib.HostWords` which ``out`` arrives in as well, for a caller that reads it at once."""
     if kl_penalty is None:
         kl_code = _lib.KL_NONE
     elif kl_penalty in _lib.KL_BY_NAME:
@@ -405,7 +411,7 @@ def fused_logprob_policy_loss(output, batch, *, packed, seqlens=None, cu_seqlens
                kl_coef=float(kl_coef), entropy_coeff=float(entropy_coeff), seq_mean=0 if token_level_loss else 1,
                loss_scale=float(loss_scale), inv_temperature=float(inv_temperature), grad_inplace=bool(grad_inplace),
                expected_upstream=None if expected_upstream is None else float(expected_upstream),
-               scale_state=scale_state)
+               scale_state=scale_state, sent=sent)
     return _FusedLogprobLoss.apply(output, batch["labels"], batch, cfg)
 
 
@@ -421,8 +427,8 @@ def _use_fused(output, kwargs):
     return torch.is_grad_enabled() and output.requires_grad and fused_supported(output, inplace)
 
 
-def _fused_kwargs(kwargs, scale_state=None):
-    return dict(packed=kwargs.get("use_remove_padding", False), seqlens=kwargs.get("seqlens_in_batch"),
+def _fused_kwargs(kwargs, scale_state=None, sent=None):
+    return dict(sent=sent, packed=kwargs.get("use_remove_padding", False), seqlens=kwargs.get("seqlens_in_batch"),
                 cu_seqlens=kwargs.get("cu_seqlens_padded"), inv_temperature=float(kwargs.get("inv_temperature", 1.0)),
                 grad_inplace=bool(kwargs.get("grad_inplace", False)),
                 expected_upstream=kwargs.get("expected_grad_scale"), scale_state=scale_state)
@@ -721,18 +727,22 @@ class _PinnedRing:
 _pinned_rings = {}
 
 
-def _finish(loss, out, kwargs=None, skip=()):
-    """The five statistics as python floats from ONE device-to-host copy (the reference issues five
-    ``.item()`` calls); ``abs`` on the policy loss as in ``grpo_actor_loss_func.py:91-97``.  With
-    deferred statistics the copy is asynchronous and the floats are made on first access."""
+def _deferred(kwargs):
+    return (kwargs or {}).get("deferred_stats", os.environ.get("MRL_DEFERRED_STATS", "0") == "1")
+
+
+def _finish(loss, out, kwargs=None, skip=(), sent=()):
+    """The five statistics as python floats from ONE host read (the reference issues five ``.item()`` calls): of the
+    slot that the last kernel left them in (``sent``), else of a device-to-host copy; ``abs`` on the policy loss as
+    in ``grpo_actor_loss_func.py:91-97``.  With deferred statistics the copy is asynchronous and the floats are made
+    on first access."""
     spec = [(STAT_KEYS[i], i + 1, i == 0) for i in range(5) if STAT_KEYS[i] not in skip]
-    deferred = (kwargs or {}).get("deferred_stats", os.environ.get("MRL_DEFERRED_STATS", "0") == "1")
     if out.is_cuda and torch.cuda.is_current_stream_capturing():
         # under graph capture nothing may wait for the device: the dict reads the device scalars when it
         # is looked at (after a replay), whatever was asked for
         return loss, DeferredStats(spec, out, None)
-    if not deferred:
-        host = out.detach().cpu().tolist()
+    if not _deferred(kwargs):
+        host = sent[0].read(ctypes.c_float, 8, _lib.stream(out.device)) if sent else out.detach().cpu().tolist()
         return loss, {key: (abs(host[index]) if use_abs else host[index]) for key, index, use_abs in spec}
     dev = out.device
     ring = _pinned_rings.get(dev)
@@ -787,21 +797,22 @@ class GRPOActorLossFunc(BaseLossFunc):
         if forward_only:
             log_probs, _ = super().compute_log_probs(output=output, batch=batch, **kwargs)
             return log_probs
+        sent = None if _deferred(kwargs) else []
         if kwargs.get("lm_head_weight") is not None:
             loss, out = self._from_hidden(
                 output, batch, kwargs, ref_log_prob=batch.get("ref_log_prob"), clip_low=self.clip_ratio,
                 clip_high=self.clip_ratio, kl_penalty=self.kl_penalty, kl_coef=self.kl_ctrl.value,
                 entropy_coeff=self.entropy_coeff, token_level_loss=True,
-                loss_scale=_dynamic_scale(batch, forward_only, kwargs))
-            return _finish(loss, out, kwargs)
+                loss_scale=_dynamic_scale(batch, forward_only, kwargs), sent=sent)
+            return _finish(loss, out, kwargs, sent=sent or ())
         if self._fused(output, kwargs):
             loss, out = fused_logprob_policy_loss(
                 output, batch, ref_log_prob=batch.get("ref_log_prob"), clip_low=self.clip_ratio,
                 clip_high=self.clip_ratio, kl_penalty=self.kl_penalty, kl_coef=self.kl_ctrl.value,
                 entropy_coeff=self.entropy_coeff, token_level_loss=True,
                 loss_scale=_dynamic_scale(batch, forward_only, kwargs),
-                **_fused_kwargs(kwargs, self.grad_scale_state(output.device)))
-            return _finish(loss, out, kwargs)
+                **_fused_kwargs(kwargs, self.grad_scale_state(output.device), sent))
+            return _finish(loss, out, kwargs, sent=sent or ())
         log_probs, entropy = super().compute_log_probs(output=output, batch=batch,
                                                        skip_entropy=(self.entropy_coeff == 0), **kwargs)
         # batch['response_mask'] is ignored here, as in the reference: the mask is j < response_length
@@ -860,20 +871,21 @@ class DAPOActorLossFunc(BaseLossFunc):
         if not self.clip_higher_enable:
             self.clip_ratio_low = self.clip_ratio
             self.clip_ratio_high = self.clip_ratio
+        sent = None if _deferred(kwargs) else []
         mask = batch["response_mask"] if "response_mask" in batch else None
         if kwargs.get("lm_head_weight") is not None:
             loss, out = self._from_hidden(
                 output, batch, kwargs, mask=mask, clip_low=self.clip_ratio_low, clip_high=self.clip_ratio_high,
                 kl_penalty=None, entropy_coeff=self.entropy_coeff, token_level_loss=self.token_level_loss,
-                loss_scale=_dynamic_scale(batch, forward_only, kwargs))
-            return _finish(loss, out, kwargs)
+                loss_scale=_dynamic_scale(batch, forward_only, kwargs), sent=sent)
+            return _finish(loss, out, kwargs, sent=sent or ())
         if self._fused(output, kwargs):
             loss, out = fused_logprob_policy_loss(
                 output, batch, mask=mask, clip_low=self.clip_ratio_low, clip_high=self.clip_ratio_high,
                 kl_penalty=None, entropy_coeff=self.entropy_coeff, token_level_loss=self.token_level_loss,
                 loss_scale=_dynamic_scale(batch, forward_only, kwargs),
-                **_fused_kwargs(kwargs, self.grad_scale_state(output.device)))
-            return _finish(loss, out, kwargs)
+                **_fused_kwargs(kwargs, self.grad_scale_state(output.device), sent))
+            return _finish(loss, out, kwargs, sent=sent or ())
         log_probs, entropy = super().compute_log_probs(output=output, batch=batch,
                                                        skip_entropy=(self.entropy_coeff == 0), **kwargs)
         loss, out = policy_loss(log_probs, entropy if self.entropy_coeff != 0 else None, batch.get("old_log_prob"),
@@ -928,21 +940,22 @@ class PPOActorLossFunc(BaseLossFunc):
         if forward_only:
             log_probs, _ = super().compute_log_probs(output=output, batch=batch, **kwargs)
             return log_probs
+        sent = None if _deferred(kwargs) else []
         common = dict(clip_low=self.clip_ratio, clip_high=self.clip_ratio, kl_penalty=None,
                       entropy_coeff=self.entropy_coeff, token_level_loss=True,
                       loss_scale=_dynamic_scale(batch, forward_only, kwargs))
         if kwargs.get("lm_head_weight") is not None:
-            loss, out = self._from_hidden(output, batch, kwargs, **common)
+            loss, out = self._from_hidden(output, batch, kwargs, sent=sent, **common)
         elif self._fused(output, kwargs):
             loss, out = fused_logprob_policy_loss(output, batch, **common,
-                                                  **_fused_kwargs(kwargs, self.grad_scale_state(output.device)))
+                                                  **_fused_kwargs(kwargs, self.grad_scale_state(output.device), sent))
         else:
             log_probs, entropy = super().compute_log_probs(output=output, batch=batch,
                                                            skip_entropy=(self.entropy_coeff == 0), **kwargs)
             loss, out = policy_loss(log_probs, entropy if self.entropy_coeff != 0 else None,
                                     batch.get("old_log_prob"), None, batch.get("advantages"),
                                     response_length=batch["response_length"], **common)
-        return _finish(loss, out, kwargs, skip=(STAT_KEYS[3],))          # PPO reports no actor/kl_loss
+        return _finish(loss, out, kwargs, skip=(STAT_KEYS[3],), sent=sent or ())          # PPO reports no actor/kl_loss
 
     @staticmethod
     def _compute_ppo_policy_loss(old_log_prob, log_prob, advantages, eos_mask, cliprange, entropy, entropy_coeff):

@@ -7,6 +7,7 @@ map kernels.  Where the reference runs a Python loop with two or three ``.item()
 sequence, these launch one kernel; ``preprocess_packed_seqs`` keeps a single host read (the
 packed length, needed to size its outputs).
 """
+import ctypes
 import math
 
 import torch
@@ -38,6 +39,12 @@ def generate_mask(data_pad, seq_lengths):
 def pack_index(attention_mask_1d, tp_size):
     """``(seqlens_in_batch int32 [B], cu_seqlens_padded int32 [B+1], total int64 [1])`` on the
     device, without any host synchronisation."""
+    dev = attention_mask_1d.device
+    total = torch.empty(1, dtype=torch.int64, device=dev)
+    return (*_pack_index(attention_mask_1d, tp_size, total.data_ptr()), total)
+
+
+def _pack_index(attention_mask_1d, tp_size, p_total):
     mask = attention_mask_1d
     if mask.dtype not in (torch.int64, torch.int32, torch.uint8, torch.bool, torch.float32):
         mask = mask.to(torch.int64)
@@ -46,10 +53,9 @@ def pack_index(attention_mask_1d, tp_size):
     batch, width = mask.shape
     seqlens = torch.empty(batch, dtype=torch.int32, device=dev)
     cu = torch.empty(batch + 1, dtype=torch.int32, device=dev)
-    total = torch.empty(1, dtype=torch.int64, device=dev)
     _lib.call("mrl_pack_index_build", _lib.ptr(mask), _lib.dtype_code(mask), batch, width, int(tp_size),
-              _lib.ptr(seqlens), _lib.ptr(cu), _lib.ptr(total), _lib.stream(dev))
-    return seqlens, cu, total
+              _lib.ptr(seqlens), _lib.ptr(cu), p_total, _lib.stream(dev))
+    return seqlens, cu
 
 
 def preprocess_packed_seqs(input_ids, labels, attention_mask_1d, tp_size):
@@ -60,8 +66,14 @@ def preprocess_packed_seqs(input_ids, labels, attention_mask_1d, tp_size):
     if attention_mask_1d.shape != (batch, width):
         raise ValueError("attention_mask_1d must have shape (batch_size, seq_len) matching input_ids")
     dev = _lib.require_device(input_ids, labels, attention_mask_1d)
-    seqlens, cu, total = pack_index(attention_mask_1d, tp_size)
-    pack_length = int(total.item())          # the one host read: sizes the packed outputs
+    # the one host read: sizes the packed outputs
+    slot = _lib.HostWords.take(dev, 8)
+    if slot is not None:
+        seqlens, cu = _pack_index(attention_mask_1d, tp_size, slot.addr)
+        (pack_length,) = slot.read(ctypes.c_int64, 1, _lib.stream(dev))
+    else:
+        seqlens, cu, total = pack_index(attention_mask_1d, tp_size)
+        pack_length = int(total.item())
     ids = input_ids.contiguous()
     lab = labels.to(ids.dtype).contiguous()
     if ids.dtype not in (torch.int32, torch.int64):

@@ -6,6 +6,7 @@ Host-side mirror of ``AdaptiveKLController``, the arithmetic inside ``apply_kl_p
 ``CriticLossFunc`` (``mindspeed_rl/models/loss/critic_loss_func.py``), with the reference's names,
 signatures and error behaviour; the arithmetic runs in the kernels of ``csrc/value_path.hip``.
 """
+import ctypes
 from typing import Dict, Tuple
 
 import numpy as np
@@ -56,12 +57,14 @@ def kl_token_level_rewards(old_log_prob, ref_log_prob, response_length, rm_score
     if lens.numel() != batch or scores.numel() != batch:
         raise ValueError("response_length and rm_scores need one entry per sample")
     rewards = torch.empty_like(old)
-    row_kl = torch.empty(batch, dtype=torch.float32, device=dev)
+    slot = _lib.HostWords.take(dev, 4 * batch) if batch > 0 else None
+    row_kl = torch.empty(batch, dtype=torch.float32, device=dev) if slot is None else None
     _lib.call("mrl_kl_token_rewards", _lib.ptr(old), _lib.ptr(ref), _lib.ptr(lens), _lib.dtype_code(lens),
               _lib.ptr(scores), batch, width, _lib.KL_BY_NAME[penalty], float(beta), _lib.ptr(rewards),
-              _lib.ptr(row_kl), _lib.stream(dev))
-    # the copy waits for the kernel either way: the mean of `batch` numbers is taken where they land
-    return rewards, torch.mean(row_kl.cpu().double(), dim=0).float().item()
+              slot.addr if slot is not None else _lib.ptr(row_kl), _lib.stream(dev))
+    # the host waits for the kernel either way: the mean of `batch` numbers is taken where they land
+    row_kl = slot.read_doubles_of(batch, _lib.stream(dev)) if slot is not None else row_kl.cpu().double()
+    return rewards, torch.mean(row_kl, dim=0).float().item()
 
 
 def _whiten(values, mask, shift_mean):
@@ -108,12 +111,16 @@ def compute_gae_advantage_return(token_level_rewards, values, eos_mask, gamma, l
     adv = torch.empty_like(rewards)
     ret = torch.empty_like(rewards)
     small = torch.empty(3 + 3 * batch, dtype=torch.float64, device=dev)     # info, then the rows' moments
+    # whether the mask is empty is all that the host waits for: its rows' sums leave before the scan has ended (whole
+    # numbers, so their sum has no order)
+    slot = _lib.HostWords.take(dev, 8 * batch) if batch > 0 and mask.dtype is not torch.float32 else None
     # `gamma * lam` as python evaluates it inside the reference's `gamma * lam * lastgaelam`: in double
     # for python floats (the config's values), in the tensors' own precision for 0-dim tensors
-    _lib.call("mrl_gae_whiten", _lib.ptr(rewards), _lib.ptr(vals), _lib.ptr(mask), _lib.dtype_code(mask), batch, width,
-              float(gamma), float(gamma * lam), _lib.ptr(adv), _lib.ptr(ret), small.data_ptr(), small.data_ptr() + 24,
-              24 * batch, _lib.stream(dev))
-    if small[0].item() == 0:
+    _lib.call("mrl_gae_whiten_host", _lib.ptr(rewards), _lib.ptr(vals), _lib.ptr(mask), _lib.dtype_code(mask), batch, width,
+              float(gamma), float(gamma * lam), _lib.ptr(adv), _lib.ptr(ret), small.data_ptr(),
+              slot.addr if slot is not None else None, small.data_ptr() + 24, 24 * batch, _lib.stream(dev))
+    count = sum(slot.read(ctypes.c_double, batch, _lib.stream(dev))) if slot is not None else small[0].item()
+    if count == 0:
         raise ValueError("At least one element in the mask has to be 1.")
     return adv, ret
 
@@ -161,7 +168,7 @@ class _CriticLoss(torch.autograd.Function):
     overwrite it before the backward."""
 
     @staticmethod
-    def forward(ctx, head, prompt, lens, returns, values, clip, loss_scale):
+    def forward(ctx, head, prompt, lens, returns, values, clip, loss_scale, sent):
         dev = _lib.require_device(head, prompt, lens, returns, values)
         head = head.contiguous()
         ret, val = _f32(returns, dev), _f32(values, dev)
@@ -171,9 +178,13 @@ class _CriticLoss(torch.autograd.Function):
         slope = torch.empty_like(ret)
         ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(batch)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        _lib.call("mrl_critic_loss_fwd_slope", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
+        slot = _lib.HostWords.take(dev, 16) if sent is not None else None
+        _lib.call("mrl_critic_loss_fwd_slope_host", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
                   _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, float(clip), float(loss_scale),
-                  _lib.ptr(slope), _lib.ptr(out), _lib.ptr(loss), _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
+                  _lib.ptr(slope), _lib.ptr(out), _lib.ptr(loss), slot.addr if slot is not None else None,
+                  _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
+        if slot is not None:
+            sent.append(slot)
         ctx.save_for_backward(slope, prompt, lens, out)
         ctx.meta = (tuple(head.shape), float(loss_scale))
         ctx.mark_non_differentiable(out)
@@ -183,7 +194,7 @@ class _CriticLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_loss, _g_out):
         if g_loss is None:
-            return (None,) * 7
+            return (None,) * 8
         slope, prompt, lens, out = ctx.saved_tensors
         shape, loss_scale = ctx.meta
         dev = slope.device
@@ -192,7 +203,7 @@ class _CriticLoss(torch.autograd.Function):
         _lib.call("mrl_critic_loss_bwd_slope", _lib.ptr(slope), shape[0], shape[1], _lib.ptr(prompt), _lib.dtype_code(prompt),
                   _lib.ptr(lens), _lib.dtype_code(lens), slope.shape[1], loss_scale, _lib.ptr(out), _lib.ptr(upstream),
                   _lib.ptr(g), _lib.stream(dev))
-        return g, None, None, None, None, None, None
+        return g, None, None, None, None, None, None, None
 
 
 def value_loss(vpreds, returns, values, response_mask=None, response_length=None, *, cliprange_value,
@@ -261,10 +272,11 @@ class CriticLossFunc(BaseLossFunc):
                                              cu_seqlens_padded=kwargs.get("cu_seqlens_padded", None),
                                              seq_len=kwargs.get("seq_len", None))
         if not forward_only and "responses" in batch and self._reads_windows_in_place(output, batch):
+            sent = []
             loss, out = _CriticLoss.apply(output, batch["prompt_length"].contiguous(), batch["response_length"].contiguous(),
                                           batch["returns"], batch["values"], self.cliprange_value,
-                                          _dynamic_scale(batch, forward_only, kwargs))
-            return loss, self._statistics(out)
+                                          _dynamic_scale(batch, forward_only, kwargs), sent)
+            return loss, self._statistics(out, sent)
         vpreds = self._get_compute_vpreds(output, batch)
         if forward_only:
             return vpreds
@@ -278,8 +290,9 @@ class CriticLossFunc(BaseLossFunc):
         return loss, self._statistics(out)
 
     @staticmethod
-    def _statistics(out):
-        host = out.detach().cpu().tolist()      # one device-to-host copy for both statistics
+    def _statistics(out, sent=()):
+        # the slot that the kernel left them in, else one device-to-host copy for both statistics
+        host = sent[0].read(ctypes.c_float, 4, _lib.stream(out.device)) if sent else out.detach().cpu().tolist()
         return {"critic/vf_loss": abs(host[1]), "critic/vf_clipfrac": host[2]}
 
     @staticmethod

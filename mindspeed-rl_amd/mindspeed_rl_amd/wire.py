@@ -6,6 +6,8 @@ reference's signatures.  The reference walks the rows in Python with one or two 
 per row; here all columns of a batch cost one scan launch, one host read (two integers a column, to size
 the outputs) and one copy launch.
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -85,14 +87,17 @@ def _by_device(columns):
 def _lay_out(columns):
     """Offsets of every column, and its size on the host: one scan launch and one host read for all of them."""
     for dev, part in _by_device(columns):
-        info = torch.empty((len(part), 2), dtype=torch.int64, device=dev)
+        slot = _lib.HostWords.take(dev, 16 * len(part))
+        info = None if slot is not None else torch.empty((len(part), 2), dtype=torch.int64, device=dev)
+        p_info = slot.addr if slot is not None else info.data_ptr()
         args = (_lib.RaggedColumn * len(part))()
         for i, c in enumerate(part):
             c.cu = torch.empty(c.lengths.numel() + 1, dtype=torch.int32, device=dev)
-            c.fill(args[i], info.data_ptr() + 16 * i)
+            c.fill(args[i], p_info + 16 * i)
         _lib.call("mrl_ragged_layouts", args, len(part), _lib.stream(dev))
-        for c, (total, longest) in zip(part, info.tolist()):
-            c.total, c.longest = total, longest
+        sizes = slot.read(ctypes.c_int64, 2 * len(part), _lib.stream(dev)) if slot is not None else info.view(-1).tolist()
+        for i, c in enumerate(part):
+            c.total, c.longest = sizes[2 * i:2 * i + 2]
 
 
 def _copy(columns, to_padded):

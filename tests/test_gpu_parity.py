@@ -569,6 +569,72 @@ def test_gae_and_whitening_parity(dev, batch, width):
         1.0, r.abs().max().item() * 2)
 
 
+def test_numbers_left_in_host_memory(dev, monkeypatch):
+    """What kernels leave in pinned memory equals what a copy brings: sizes, sums and statistics, from several threads
+    with streams of their own at once, a batch wider than a slot, a number that looks like an empty slot's, a mask that
+    is empty; no slot is lost, and under capture none is taken."""
+    import ctypes
+    import threading
+
+    def values(seed, batch):
+        gen = torch.Generator(device=dev).manual_seed(seed)
+        width = 70
+        old, ref = torch.randn(2, batch, width, generator=gen, device=dev).unbind(0)
+        lens = torch.randint(1, width + 1, (batch, 1), generator=gen, device=dev, dtype=torch.int32)
+        mask = mrl.generate_mask(old, lens)
+        out = [mrl.kl_token_level_rewards(old, ref, lens, old[:, 0], 0.1)[1]]
+        out += [t.cpu() for t in mrl.compute_gae_advantage_return(old, ref, mask, 1.0, 0.95)]
+        with pytest.raises(ValueError, match="At least one element"):
+            mrl.compute_gae_advantage_return(old, ref, torch.zeros_like(mask), 1.0, 0.95)
+        out += [t.cpu() for t in mrl.preprocess_packed_seqs(mask, mask, mask, 4)]
+        critic = mrl.LossFuncFactory.get_instance("ray_ppo", "critic")
+        head = torch.randn(batch, width + 9, 1, generator=gen, device=dev).requires_grad_()
+        out.append(critic.compute_loss(head, {"responses": mask, "response_length": lens, "values": ref, "returns": old,
+                                              "prompt_length": torch.full_like(lens, 3)})[1])
+        logits = torch.randn(1, batch * width, 256, generator=gen, device=dev).requires_grad_()
+        cu = torch.arange(batch + 1, dtype=torch.int32, device=dev) * width
+        actor = mrl.LossFuncFactory.get_instance("ray_ppo", "actor")
+        out.append(actor.compute_loss(logits, {
+            "labels": mask.view(1, -1), "responses": mask[:, 1:], "prompt_length": torch.ones_like(lens),
+            "response_length": (lens - 1).clamp(min=1), "advantages": old[:, 1:] * mask[:, 1:],
+            "old_log_prob": ref[:, 1:] - 5.5}, use_remove_padding=True, seqlens_in_batch=torch.full_like(lens, width).view(-1),
+            cu_seqlens_padded=cu, seq_len=width)[1])
+        return out
+
+    def same(a, b):
+        return all(torch.equal(x, y) if torch.is_tensor(x) else x == y for x, y in zip(a, b)) and len(a) == len(b)
+
+    jobs = [(1, 8), (2, 40), (3, 600), (4, 1100)]           # 600 rows of doubles, 1 100 of floats: more than a slot
+    take = _lib.HostWords.take
+    monkeypatch.setattr(_lib.HostWords, "take", lambda *a: None)
+    want = [values(*j) for j in jobs]
+    monkeypatch.setattr(_lib.HostWords, "take", take)
+    assert all(same(values(*j), w) for j, w in zip(jobs, want))
+    wrong = []
+
+    def work(j, w):
+        torch.cuda.set_device(dev)
+        with torch.cuda.stream(torch.cuda.Stream(dev)):
+            wrong.extend(j for _ in range(10) if not same(values(*j), w))
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=a) for a in zip(jobs, want)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not wrong
+    free = _lib.HostWords._free[dev.index]
+    slots = len(free)
+    assert slots % _lib.HostWords._BLOCK == 0 and len({s.addr for s in free}) == slots
+    slot = take(dev, 8)
+    torch.full((1,), -1, device=dev).sum()
+    assert slot.read(ctypes.c_int64, 1, _lib.stream(dev)) == [-1]       # never seen to arrive: waited for by the stream
+    assert take(dev, _lib.HostWords.BYTES + 4) is None and len(free) == slots
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert take(dev, 8) is None
+        torch.zeros(1, device=dev).add_(1)
+
+
 @pytest.mark.parametrize("width", [1, 15, 16, 17, 63, 64, 65, 128, 129, 4096 + 15, 4096 + 65, 3 * 4096])
 def test_gae_scan_between_kept_results(dev, width):
     """Every remainder of the chain's groups of 64, of the 16 steps taken once more and of a staged chunk, no decay, and
