@@ -15,6 +15,7 @@
 // share the call, whatever the work distribution is: units of 256 tokens by a group of leaves, as many
 // groups as fill the chip (pick_groups), walked by one persistent workgroup per CU.
 #include <atomic>
+#include <type_traits>
 
 #include "lmhead_tile.h"
 #include "mrl_internal.h"
@@ -67,10 +68,12 @@ constexpr int kMaxRounds = 64;                  // units a workgroup may take
 // block and those that stream the same weight tiles run side by side and share them in the XCD's L2; and
 // so that the 8 XCDs hold 32 token tiles x the SAME 8 groups, so that a weight tile comes from HBM once
 // for all of them (numbering all groups of 4 token tiles first: 2 % slower at 8 and more groups).
+template <bool kEntropy>
 struct UnitTiles : mrl_tile::WholeK {
-    // The epilogue below needs more registers than there are and puts some aside: their return is waited for
-    // before the loop, where the wait would be for the requests in flight (they have landed by then).
-    static constexpr bool kSettle = true;
+    // With the entropy's sums the epilogue below needs more registers than there are and puts some aside: their
+    // return is waited for before the loop, where the wait would be for the requests in flight (they have landed
+    // by then).
+    static constexpr bool kSettle = kEntropy;
     int n_tiles;
     // lane r of a wavefront holds the workgroup's unit r: the flattened number of its first tile (beyond every
     // tile where there is no such unit), its first vocabulary tile less that number, its token tile
@@ -82,7 +85,15 @@ struct UnitTiles : mrl_tile::WholeK {
     }
 };
 
-// partial: [leaf][m, s, u][token of the slice]
+// What bounds it: the matrix cores (1.33 us per k-step of a tile), and between tiles the statistics, 4 us in
+// which they idle: per entry a read out of the accumulators, half a max3, an FMA, an exponential and an addition;
+// the entropy's sum is one more FMA and taken only where it is asked for.  The lanes' parts of a leaf meet in LDS
+// (eight of them merged by a thread per token) and not in two rounds of shuffles, and the statistics' stores are
+// not waited for.  us, before -> now: 23 255 x 8 600 x 640 283 -> 249 (256 with entropy), 9 477 x 18 840 x 640
+// 246 -> 218 (227), 16 384 x 65 536 x 1 024 1 667 -> 1 594 (1 617), 12 356 x 152 064 x 3 584 9 307 -> 9 284.
+//
+// partial: [leaf][m, s, u][token of the slice]; without kEntropy u is left out
+template <bool kEntropy>
 __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, int n_tokens, int vocab, int hdim,
     int n_groups, float k_scale, float* __restrict__ partial) {
@@ -93,7 +104,7 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wv = wave >> 1, wt = wave & 1;
     const VocabLeaves leaves(vocab);
-    UnitTiles seq = {{}, 0, 0x7fffffff, 0, 0};
+    UnitTiles<kEntropy> seq = {{}, 0, 0x7fffffff, 0, 0};
     {
         const int n_ttiles = (n_tokens + BN - 1) / BN;
         int r = 0;
@@ -119,23 +130,29 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
 #pragma unroll
     for (int tb = 0; tb < kBlocks; ++tb) st[tb] = {kMaxInit, 0.f, 0.f};
 
-    // A leaf is finished: combine the four lane quarters (same token, other vocabulary rows), then the two
-    // vocabulary wavefronts; thread t writes token t.
+    // threadIdx.x, computed where it is needed: kept from one tile to the next, it and what follows from it take
+    // registers that the tile loop needs
+    auto my_thread = [&]() {
+        int t = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        asm volatile("" : "+v"(t));
+        return t + wave * 64;
+    };
+
+    // A leaf is finished: every lane leaves its 8 tokens' statistics in LDS, [part][m, s, u][token] with a part
+    // for each quarter of each of the two vocabulary wavefronts, and thread t merges the parts of token t in
+    // their order and writes them.
     auto finish_leaf = [&](int leaf, int tn, unsigned char* spare) {
-        Stats* const comb = reinterpret_cast<Stats*>(spare);       // [vocabulary wavefront][token]
-        static_assert(2 * kThreads * sizeof(Stats) <= kSpareBytes, "the statistics of a leaf");
+        constexpr int kParts = 8, kValues = kEntropy ? 3 : 2;
+        constexpr int kPitch = kValues * kThreads + 16;            // the quarters of a wavefront on different banks
+        static_assert(kParts * kPitch * sizeof(float) <= kSpareBytes, "the statistics of a leaf");
+        float* const comb = reinterpret_cast<float*>(spare);
+        const int tid = my_thread();
+        float* const mine = comb + (wv * 4 + ((tid & 63) >> 4)) * kPitch + wt * 128 + (tid & 15);
 #pragma unroll
         for (int tb = 0; tb < kBlocks; ++tb) {
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int off = 16; off <= 32; off <<= 1) {
-                Stats o;
-                o.m = __shfl_xor(st[tb].m, off, 64);
-                o.s = __shfl_xor(st[tb].s, off, 64);
-                o.u = __shfl_xor(st[tb].u, off, 64);
-                st[tb] = merge<true>(st[tb], o, k_scale);
-            }
-            if (lane < 16) comb[wv * kThreads + wt * 128 + tb * 16 + lane] = st[tb];
+            mine[tb * 16] = st[tb].m;
+            mine[tb * 16 + kThreads] = st[tb].s;
+            if (kEntropy) mine[tb * 16 + 2 * kThreads] = st[tb].u;
             st[tb] = {kMaxInit, 0.f, 0.f};
         }
         // LDS accesses only: a full fence would wait for the requests of the next stages as well
@@ -145,21 +162,29 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         };
         lds_barrier();
-        const Stats r = merge<true>(comb[threadIdx.x], comb[kThreads + threadIdx.x], k_scale);
+        const float* const part = comb + tid;
+        Stats r = {part[0], 0.f, 0.f};
+#pragma unroll
+        for (int p = 1; p < kParts; ++p) r.m = fmaxf(r.m, part[p * kPitch]);
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) {
+            const float f = fast_exp2((part[p * kPitch] - r.m) * k_scale);
+            r.s = __builtin_fmaf(part[p * kPitch + kThreads], f, r.s);
+            if (kEntropy) r.u = __builtin_fmaf(part[p * kPitch + 2 * kThreads], f, r.u);
+        }
         lds_barrier();                          // what lies here next is requested by any of the wavefronts
-        const int t = tn * BN + (int)threadIdx.x;
+        const int t = tn * BN + tid;
         if (t < n_tokens) {
             float* p = partial + (int64_t)leaf * 3 * n_tokens + t;
             p[0] = r.m;
             p[n_tokens] = r.s;
-            p[2 * (int64_t)n_tokens] = r.u;
+            if (kEntropy) p[2 * (int64_t)n_tokens] = r.u;
         }
     };
 
-    // online softmax statistics of a tile: per token block a lane holds 8 x 4 vocabulary rows
-    auto tile_stats = [&](Accumulators& acc, int, int tm, int tn, unsigned char* spare) {
-        int valid = vocab - (tm * BM + wv * 128 + 4 * (lane >> 4));       // 16 vb + r below it
-        const bool ragged = (tm * BM + BM > vocab);
+    // online softmax statistics of a tile: per token block a lane holds 8 x 4 vocabulary rows, of which a ragged
+    // tile has those 16 vb + r below `valid`
+    auto tokens_stats = [&](Accumulators& acc, int valid, bool ragged) {
 #pragma unroll
         for (int tb = 0; tb < kBlocks; ++tb) {
             // one block of tokens at a time: without this the compiler copies many blocks out of the
@@ -178,15 +203,19 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
             float vmax = st[tb].m;
 #pragma unroll
             for (int i = 0; i < 4 * kBlocks; ++i) vmax = fmaxf(vmax, z[i]);
-            grow_max<true>(st[tb], vmax, k_scale);
+            grow_max<kEntropy>(st[tb], vmax, k_scale);
             // A lane that has seen no valid vocabulary row yet (the first tile of its leaf is ragged and
             // ends above its rows) still holds the start value as its maximum: z * k - m * k of the masked
             // entries would then be the rounding residual of two numbers of magnitude 1e30 instead of
             // zero.  With an infinite m * k their exponentials are exactly 0.
             const float mk = st[tb].m > kMaxInit ? st[tb].m * k_scale : __builtin_inff();
 #pragma unroll
-            for (int i = 0; i < 4 * kBlocks; ++i) add_one<true>(st[tb], z[i], k_scale, mk);
+            for (int i = 0; i < 4 * kBlocks; ++i) add_one<kEntropy>(st[tb], z[i], k_scale, mk);
         }
+    };
+    auto tile_stats = [&](Accumulators& acc, int, int tm, int tn, unsigned char* spare) {
+        const int tid = my_thread();
+        tokens_stats(acc, vocab - (tm * BM + wv * 128 + 4 * ((tid & 63) >> 4)), tm * BM + BM > vocab);
         const int leaf = tm / tiles_per_leaf;                      // uniform over the workgroup
         if (tm + 1 == n_vtiles || tm + 1 == (leaf + 1) * tiles_per_leaf) finish_leaf(leaf, tn, spare);
     };
@@ -198,7 +227,7 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
 // in order; and one wavefront per token computes the label logit as an fp32 dot product of the token's
 // hidden row with the label's weight row.
 constexpr int kFinishTokens = 16;
-template <typename LabelT>
+template <typename LabelT, bool kEntropy>
 __global__ __launch_bounds__(256) void lmhead_finish_kernel(
     const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, const LabelT* __restrict__ labels,
     const float* __restrict__ partial, int n_tokens, int vocab, int hdim, int n_leaves, float inv_t,
@@ -214,8 +243,8 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(
 #pragma unroll 4
         for (int leaf = q; leaf < n_leaves; leaf += 16) {
             const float* p = partial + (int64_t)leaf * 3 * n_tokens + t;
-            const Stats o = {p[0], p[n_tokens], p[2 * (int64_t)n_tokens]};
-            r = merge<true>(r, o, k);
+            const Stats o = {p[0], p[n_tokens], kEntropy ? p[2 * (int64_t)n_tokens] : 0.f};
+            r = merge<kEntropy>(r, o, k);
         }
         part[q][mine] = r;
     }
@@ -244,13 +273,13 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(
         Stats r = part[lane & 15][i];
 #pragma unroll
         for (int off = 1; off <= 8; off <<= 1) {
-            const Stats o = {__shfl_xor(r.m, off, 64), __shfl_xor(r.s, off, 64), __shfl_xor(r.u, off, 64)};
-            r = merge<true>(r, o, k);
+            const Stats o = {__shfl_xor(r.m, off, 64), __shfl_xor(r.s, off, 64), kEntropy ? __shfl_xor(r.u, off, 64) : 0.f};
+            r = merge<kEntropy>(r, o, k);
         }
         if (lane == 0) {
             const float lse = (r.m * k + fast_log2(r.s)) * kLn2;
             logp[t] = (y_ok ? dot * inv_t : r.m * inv_t) - lse;
-            if (entropy) entropy[t] = lse - (r.u / r.s) * inv_t;
+            if (kEntropy) entropy[t] = lse - (r.u / r.s) * inv_t;
             if (lse_out) lse_out[t] = lse;
         }
     }
@@ -302,8 +331,10 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
     // attributes belong to a device, so the reservation is made with every launch, on whichever
     // device is current.
     constexpr int kLdsBytes = mrl_tile::kLdsBytes;
-    const hipError_t attr = hipFuncSetAttribute((const void*)lmhead_fwd_kernel,
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    const auto fwd = entropy ? lmhead_fwd_kernel<true> : lmhead_fwd_kernel<false>;
+    const bool wide_labels = labels_dtype != MRL_I32;
+    const hipError_t attr =
+        hipFuncSetAttribute((const void*)fwd, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     MRL_REQUIRE(attr == hipSuccess, MRL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", fn, kLdsBytes,
                 hipGetErrorString(attr));
     MRL_REQUIRE(256 * hidden_dim * 2 < (1LL << 31) && n_tokens <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED,
@@ -314,7 +345,7 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
     for (int64_t lo = 0; lo < n_tokens; lo += slice) {
         const int n = (int)(n_tokens - lo < slice ? n_tokens - lo : slice);
         const uint16_t* h = (const uint16_t*)hidden + lo * hidden_dim;
-        hipLaunchKernelGGL(lmhead_fwd_kernel, dim3(kUnitsPerRound), dim3(mrl_tile::kThreads), kLdsBytes, s, h,
+        hipLaunchKernelGGL(fwd, dim3(kUnitsPerRound), dim3(mrl_tile::kThreads), kLdsBytes, s, h,
                            (const uint16_t*)weight, n, (int)vocab, (int)hidden_dim, pick_groups(n, leaves),
                            inv_temperature * kLog2e, partial);
         int rc = mrl::check_launch(fn);
@@ -322,15 +353,14 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
         const dim3 fgrid((unsigned)((n + kFinishTokens - 1) / kFinishTokens)), fblock(256);
         float* ent = entropy ? entropy + lo : nullptr;
         float* lse_out = lse ? lse + lo : nullptr;
-        if (labels_dtype == MRL_I32) {
-            hipLaunchKernelGGL(lmhead_finish_kernel<int32_t>, fgrid, fblock, 0, s, h, (const uint16_t*)weight,
-                               (const int32_t*)labels + lo, (const float*)partial, n, (int)vocab, (int)hidden_dim,
-                               leaves.n, inv_temperature, logp + lo, ent, lse_out);
-        } else {
-            hipLaunchKernelGGL(lmhead_finish_kernel<int64_t>, fgrid, fblock, 0, s, h, (const uint16_t*)weight,
-                               (const int64_t*)labels + lo, (const float*)partial, n, (int)vocab, (int)hidden_dim,
-                               leaves.n, inv_temperature, logp + lo, ent, lse_out);
-        }
+        auto finish = [&](auto kernel, auto* lab) {
+            hipLaunchKernelGGL(kernel, fgrid, fblock, 0, s, h, (const uint16_t*)weight, lab + lo, (const float*)partial, n,
+                               (int)vocab, (int)hidden_dim, leaves.n, inv_temperature, logp + lo, ent, lse_out);
+        };
+        if (wide_labels)
+            finish(entropy ? lmhead_finish_kernel<int64_t, true> : lmhead_finish_kernel<int64_t, false>, (const int64_t*)labels);
+        else
+            finish(entropy ? lmhead_finish_kernel<int32_t, true> : lmhead_finish_kernel<int32_t, false>, (const int32_t*)labels);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }

@@ -1748,6 +1748,24 @@ def test_lmhead_logprob_forward(dev, tokens, vocab, hdim):
     assert torch.allclose(lp2.view(-1).cpu(), o_vocab.lmhead_logprob_entropy(h, w, y)[0], atol=2e-4)
 
 
+@pytest.mark.parametrize("tokens,vocab", [(1, 8), (17, 120), (255, 136), (257, 264), (300, 32776), (129, 33288), (40, 98568)])
+def test_lmhead_logprob_without_entropy(dev, tokens, vocab):
+    """The statistics without the entropy's sums are a kernel of their own: the same bits in what both give, and
+    both right, where the last tile ends inside either half of a wavefront pair's rows and leaves are 1, 2 and 3
+    tiles."""
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    h = torch.randn(tokens, 64, generator=gen, device=dev).to(torch.bfloat16)
+    w = (torch.randn(vocab, 64, generator=gen, device=dev) * 0.3).to(torch.bfloat16)
+    y = torch.randint(0, vocab, (tokens,), generator=gen, device=dev)
+    lp, ent, lse = mrl.lmhead_logprob(h, w, y)
+    lp2, none, lse2 = mrl.lmhead_logprob(h, w, y, want_entropy=False)
+    assert torch.equal(lp, lp2) and torch.equal(lse, lse2) and not none.any().item()
+    logsm = torch.log_softmax(h.double() @ w.double().t(), -1)
+    # |z| below 20 in fp32 (2e-6 each), as are lse and the entropy's sum of z: under 1e-5 each way
+    assert (lp - logsm.gather(1, y[:, None])[:, 0]).abs().max().item() < 2e-5
+    assert (ent + (logsm.exp() * logsm).sum(1)).abs().max().item() < 4e-5
+
+
 @pytest.mark.parametrize("tokens,vocab,hdim", [(1, 8, 64), (1, 20000, 64), (256, 33000, 64), (257, 5000, 64),
                                                (1025, 16392, 64), (8448, 2064, 128)])
 def test_lmhead_logprob_forward_work_distribution(dev, tokens, vocab, hdim):
