@@ -4,6 +4,7 @@ The library is the only compute path of this package: if it is missing, loading 
 is no CPU or eager-torch fallback.  torch is used for device memory and streams only.
 """
 import ctypes
+import functools
 import os
 
 import torch
@@ -169,9 +170,20 @@ def dtype_code(t):
         raise TypeError("unsupported tensor dtype %s" % t.dtype) from None
 
 
+@functools.lru_cache(maxsize=256)
+def fused_workspace_bytes(dtype, n_rows, vocab):
+    """mrl_fused_workspace_bytes: a function of its arguments alone."""
+    return load().mrl_fused_workspace_bytes(dtype, n_rows, vocab)
+
+
 def ptr(t):
     """Device pointer of a tensor (None -> NULL)."""
     return None if t is None else t.data_ptr()
+
+
+# without the checks that the device has been initialised (a tensor on it is there) and other detours
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", None) or torch.cuda.is_current_stream_capturing
 
 
 def require_device(*tensors):
@@ -187,7 +199,7 @@ def require_device(*tensors):
             dev = t.device
         elif t.device != dev:
             raise RuntimeError("tensors on different devices: %s and %s" % (dev, t.device))
-    if dev is not None and dev.index is not None and dev.index != torch.cuda.current_device():
+    if dev is not None and dev.index is not None and dev.index != _current_device():
         # kernels are launched on the current device's context: one process drives one GPU here
         raise RuntimeError("tensors live on %s but the current device is cuda:%d (call torch.cuda.set_device first)"
                            % (dev, torch.cuda.current_device()))
@@ -214,9 +226,12 @@ def dense(t, dtype, dev):
 
 
 def index_column(t, dev):
-    """A length column as a flat, dense int32 / int64 tensor on `dev`; None stays None."""
+    """A length column as a dense int32 / int64 tensor on `dev`, flat unless it was dense already: what the kernels
+    get is its address.  None stays None."""
     if t is None:
         return None
+    if (t.dtype is torch.int64 or t.dtype is torch.int32) and t.is_contiguous() and t.device == dev:
+        return t
     if t.dtype is not torch.int32 and t.dtype is not torch.int64:
         t = t.to(torch.int64)
     if t.device != dev:
@@ -242,7 +257,7 @@ class HostWords:
     def take(cls, dev, n_bytes):
         """An empty slot of ``n_bytes``, or None: more than a slot holds, or the stream is being captured (the
         numbers will be there after a replay, not now)."""
-        if n_bytes > cls.BYTES or torch.cuda.is_current_stream_capturing():
+        if n_bytes > cls.BYTES or _capturing():
             return None
         free = cls._free.setdefault(dev.index, [])
         try:

@@ -34,7 +34,8 @@ def compute_group_norm_advantage_return(token_level_rewards, eos_mask, response_
     rewards = torch.as_tensor(token_level_rewards).detach()
     if rewards.dtype not in (torch.float32, torch.float64):
         rewards = rewards.to(torch.float64)
-    rewards = rewards.to(dev).reshape(-1).contiguous()
+    if rewards.device != dev or not rewards.is_contiguous():
+        rewards = rewards.to(dev).reshape(-1).contiguous()
     batch = rewards.numel()
     if batch != response_length.numel():
         raise RuntimeError("shape '%s' is invalid for input of size %d" % (list(response_length.shape), batch))
@@ -42,7 +43,8 @@ def compute_group_norm_advantage_return(token_level_rewards, eos_mask, response_
         raise RuntimeError("shape '[-1, %d]' is invalid for input of size %d" % (n_sample_per_prompt, batch))
     if mask.dim() != 2 or mask.shape[0] not in (1, batch):
         raise RuntimeError("eos_mask must have shape (%d, L) or (1, L)" % batch)
-    mask = mask.expand(batch, mask.shape[1]).contiguous()      # the reference broadcasts the mask
+    if mask.shape[0] != batch or not mask.is_contiguous():
+        mask = mask.expand(batch, mask.shape[1]).contiguous()  # the reference broadcasts the mask
     width = mask.shape[1]
     adv = torch.empty((batch, width), dtype=torch.float32, device=dev)
     ret = torch.empty((batch, width), dtype=torch.float32, device=dev)
@@ -76,7 +78,7 @@ def dynamic_sampling_keep_mask(metric_values, n_samples_per_prompt):
     metric = torch.as_tensor(metric_values)
     if metric.dtype not in (torch.float32, torch.float64):
         metric = metric.to(torch.float64)
-    metric = metric.reshape(-1).contiguous()
+    metric = metric.contiguous()
     dev = _lib.require_device(metric)
     keep = torch.empty(metric.numel(), dtype=torch.uint8, device=dev)
     _lib.call("mrl_group_keep_mask", _lib.ptr(metric), _lib.dtype_code(metric), metric.numel(),

@@ -176,8 +176,6 @@ class _FusedLmHeadLoss(torch.autograd.Function):
         layout, padded_s = (0, 0) if cfg["packed"] else (1, hidden.shape[1])
         chunk_cap = max(1, min(int(cfg["chunk_rows"]), max(n_rows, 1)))
         ops = _FusedOperands(dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, _lib.BF16, vocab, chunk_cap)
-        want_ent = cfg["entropy_coeff"] != 0
-        ent = torch.empty(max(n_rows, 1), dtype=torch.float32, device=dev) if want_ent else None
         stream = _lib.stream(dev)
         ops.prepare(stream)
         row_ops = ops.rows[:max(n_rows, 1) * 8]
@@ -224,8 +222,8 @@ class _FusedLmHeadLoss(torch.autograd.Function):
                 "mrl_fused_logprob_loss", rows, dev, _lib.ptr(logits), _lib.dtype_code(logits), rows, vocab, v_pad,
                 lab.data_ptr() + c0 * lab.element_size(), _lib.dtype_code(lab), cfg["inv_temperature"],
                 p_ops + c0 * 32, 0 if ops.old is None else 1, cfg["clip_lo"], cfg["clip_hi"], cfg["kl_penalty"],
-                cfg["kl_coef"], cfg["entropy_coeff"], cfg["loss_scale"], _lib.ptr(ops.applied), _lib.ptr(logits), v_pad,
-                None, (ent.data_ptr() + c0 * 4) if want_ent else None, p_terms + c0 * 32, ops.workspace,
+                cfg["kl_coef"], cfg["entropy_coeff"], cfg["loss_scale"], ops.p_applied, _lib.ptr(logits), v_pad,
+                None, ops.p_ent + c0 * 4 if ops.p_ent is not None else None, p_terms + c0 * 32, ops.workspace,
                 ops.ws_bytes, 1 if c0 == 0 else 0, stream)
             _timed("mrl_lmhead_logprob_bwd_chunk", rows, dev, h_c, _lib.ptr(w), _lib.ptr(logits), v_pad, rows, vocab, hdim,
                    d_hidden.data_ptr() + c0 * hdim * esz, _lib.ptr(d_weight), _lib.ptr(d_weight32), 1 if c0 == 0 else 0,

@@ -9,6 +9,7 @@ signatures, keyword arguments, return values and error behaviour are the referen
 is done by the HIP kernels of libmrl_hip.so.
 """
 import ctypes
+import functools
 import os
 from abc import ABC, abstractmethod
 from typing import Dict, Tuple
@@ -150,7 +151,7 @@ def fused_supported(output, grad_inplace=False):
     ``grad_inplace`` only whole vectors: see :func:`_swept_again`."""
     if output.dtype not in (torch.float32, torch.bfloat16, torch.float16) or not output.is_cuda:
         return False
-    if _lib.load().mrl_fused_workspace_bytes(_lib.dtype_code(output), 1, output.shape[-1]) == 0:
+    if _lib.fused_workspace_bytes(_lib.dtype_code(output), 1, output.shape[-1]) == 0:
         return False
     if grad_inplace and _swept_again(output):
         return False
@@ -199,7 +200,7 @@ def _deliver_eager_grads(ctx, buffers, applied, state, g_loss):
     same graph then yields NaN."""
     dev = buffers[0].device
     stream = _lib.stream(dev)
-    upstream = g_loss.to(torch.float32).reshape(1).contiguous()
+    upstream = _lib.dense(g_loss, torch.float32, dev)
     first = not ctx.handed_out
     ctx.handed_out = True
     if not first:
@@ -207,15 +208,13 @@ def _deliver_eager_grads(ctx, buffers, applied, state, g_loss):
         applied = applied.clone()
     learned = _lib.ptr(state.learned) if state is not None else None
     rescales = _lib.ptr(state.rescales) if state is not None else None
-    flats = [t.view(-1, t.shape[-1]) for t in buffers]
-    if len(flats) == 1 and flats[0].shape[0] > 0:
-        flat = flats[0]
-        _lib.call("mrl_scale_rows_note", _lib.ptr(flat), _lib.dtype_code(flat), flat.shape[0], flat.shape[1],
-                  flat.shape[1], _lib.ptr(upstream), _lib.ptr(applied), learned, rescales, stream)
+    rows = [(t.numel() // t.shape[-1], t.shape[-1], t.shape[-1]) for t in buffers]
+    if len(buffers) == 1 and rows[0][0] > 0:
+        _lib.call("mrl_scale_rows_note", _lib.ptr(buffers[0]), _lib.dtype_code(buffers[0]), *rows[0], _lib.ptr(upstream),
+                  _lib.ptr(applied), learned, rescales, stream)
         return buffers
-    for flat in flats:
-        _lib.call("mrl_scale_rows", _lib.ptr(flat), _lib.dtype_code(flat), flat.shape[0], flat.shape[1],
-                  flat.shape[1], _lib.ptr(upstream), _lib.ptr(applied), stream)
+    for t, shape in zip(buffers, rows):
+        _lib.call("mrl_scale_rows", _lib.ptr(t), _lib.dtype_code(t), *shape, _lib.ptr(upstream), _lib.ptr(applied), stream)
     # the stored buffers now carry `upstream` (first backward) or still what they carried (copies)
     _lib.call("mrl_grad_scale_note", _lib.ptr(upstream), _lib.ptr(applied), learned, rescales, stream)
     return buffers
@@ -225,13 +224,13 @@ def _deliver_swept_grads(ctx, dlogits, flat, lab, rows, small, state, g_loss):
     """The same for rows that are swept again: at another scale than ``dlogits`` carry the gradients come from
     the logits, so nothing that an earlier backward was given can spoil them."""
     dev = flat.device
-    upstream = g_loss.to(torch.float32).reshape(1).contiguous()
+    upstream = _lib.dense(g_loss, torch.float32, dev)
     shape, scalars, o_applied, o_workspace, ws_bytes = ctx.sweep
     first = not ctx.handed_out
     ctx.handed_out = True
     p_applied = small.data_ptr() + o_applied
     if not first:                       # what was handed out stays; its workspace has been used
-        dlogits = torch.empty_like(flat)
+        dlogits = torch.empty_like(dlogits)
         applied = small[o_applied:o_applied + 8].clone()
         p_applied = applied.data_ptr()
     learned = _lib.ptr(state.learned) if state is not None else None
@@ -259,14 +258,12 @@ class _FusedOperands:
 
     def __init__(self, dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, sweep_dtype_code, vocab, sweep_rows,
                  sweeps=1):
-        lib = _lib.load()
-
         f32, i32 = torch.float32, torch.int32
         self.dev, self.cfg = dev, cfg
         self.n_rows, self.n_seq, self.width, self.layout, self.padded_s = n_rows, n_seq, width, layout, padded_s
         self.old, self.ref, self.adv = (_lib.dense(batch.get("old_log_prob"), f32, dev), _lib.dense(cfg["ref_log_prob"], f32, dev),
                                         _lib.dense(batch.get("advantages"), f32, dev))
-        self.mask_t, _ = _mask_args(cfg["mask"], batch["response_length"], dev)
+        self.mask_t = None if cfg["mask"] is None else _mask_args(cfg["mask"], None, dev)[0]
         self.prompt, self.resp = _lib.index_column(batch["prompt_length"], dev), _lib.index_column(batch["response_length"], dev)
         if layout == 0:
             self.seqlens, self.cu = _lib.dense(cfg["seqlens"], i32, dev), _lib.dense(cfg["cu"], i32, dev)
@@ -276,7 +273,7 @@ class _FusedOperands:
         self.pdt, self.rdt = _lib.dtype_code(self.prompt), _lib.dtype_code(self.resp)
         # the sweep's workspace is sized for the largest launch (a chunk, for the lm_head step)
         # (at least its 16-byte header, whose second word the reduce step borrows as its counter)
-        self.ws_bytes = max(16, lib.mrl_fused_workspace_bytes(sweep_dtype_code, sweep_rows, vocab))
+        self.ws_bytes = max(16, _lib.fused_workspace_bytes(sweep_dtype_code, sweep_rows, vocab))
         self.cleared_bytes = self.ws_bytes * sweeps     # one for each sweep over the rows
         seqs = max(n_seq, 1)
         o_out = 0                                   # float[8]
@@ -288,14 +285,28 @@ class _FusedOperands:
         o_msum = o_count + 4 * seqs                 # float[n_seq]
         self.small = torch.empty(o_msum + 4 * seqs, dtype=torch.uint8, device=dev)
         base = self.small.data_ptr()
-        self.out = self.small[o_out:o_out + 32].view(torch.float32)
-        self.applied = self.small[o_applied:o_applied + 8].view(torch.float32)
+        self.p_out, self.p_applied = base + o_out, base + o_applied
         self.workspace, self.o_applied, self.o_second = base + o_ws, o_applied, o_ws + self.ws_bytes
         self.p_start, self.p_sums, self.p_count, self.p_msum = base + o_start, base + o_sums, base + o_count, base + o_msum
-        self.rows = torch.empty(max(n_rows, 1) * 16, dtype=torch.float32, device=dev)
+        # operands and terms of a row, 8 numbers each, and one more for whoever wants the rows' entropies
+        self.rows = torch.empty(max(n_rows, 1) * (17 if cfg["entropy_coeff"] != 0 else 16), dtype=torch.float32, device=dev)
         self.p_ops = self.rows.data_ptr()
         self.p_terms = self.p_ops + max(n_rows, 1) * 32
-        self.loss = torch.empty((), dtype=torch.float32, device=dev)
+        self.p_ent = self.p_terms + max(n_rows, 1) * 32 if cfg["entropy_coeff"] != 0 else None
+
+    # Tensors of these places, and the loss's own, are made when the sweep has been launched: the launches ahead of
+    # it need addresses only, and the device has nothing to do until they are there.
+    @functools.cached_property
+    def out(self):
+        return self.small[:32].view(torch.float32)
+
+    @functools.cached_property
+    def applied(self):
+        return self.small[self.o_applied:self.o_applied + 8].view(torch.float32)
+
+    @functools.cached_property
+    def loss(self):
+        return torch.empty((), dtype=torch.float32, device=self.dev)
 
     def prepare(self, stream):
         cfg = self.cfg
@@ -305,7 +316,7 @@ class _FusedOperands:
                   _lib.ptr(self.old), _lib.ptr(self.ref), _lib.ptr(self.adv), _lib.ptr(self.mask_t), self.mdt,
                   cfg["seq_mean"], self.p_start, self.p_count, self.p_msum, self.p_ops,
                   self.workspace if self.n_rows > 0 else None, self.cleared_bytes if self.n_rows > 0 else 0,
-                  _lib.ptr(scale_dev), scale_host, _lib.ptr(self.applied) if self.n_rows > 0 else None, stream)
+                  _lib.ptr(scale_dev), scale_host, self.p_applied if self.n_rows > 0 else None, stream)
         if self.n_rows == 0:
             self.applied[0] = scale_host if scale_dev is None else scale_dev[0] * scale_host
             self.applied[1] = 0.0
@@ -320,7 +331,7 @@ class _FusedOperands:
                   self.n_seq, self.width, _lib.ptr(self.old), _lib.ptr(self.ref), _lib.ptr(self.adv),
                   _lib.ptr(self.mask_t), self.mdt, _lib.ptr(self.resp), self.rdt, cfg["clip_lo"], cfg["clip_hi"],
                   cfg["kl_penalty"], cfg["kl_coef"], cfg["entropy_coeff"], cfg["seq_mean"], cfg["loss_scale"],
-                  self.p_sums, _lib.ptr(self.out), done, _lib.ptr(self.loss), slot.addr if slot is not None else None, stream)
+                  self.p_sums, self.p_out, done, _lib.ptr(self.loss), slot.addr if slot is not None else None, stream)
         if slot is not None:
             sent.append(slot)
 
@@ -337,31 +348,27 @@ class _FusedLogprobLoss(torch.autograd.Function):
     def forward(ctx, output, labels, batch, cfg):
         dev = _lib.require_device(output, labels)
         vocab = output.shape[-1]
-        flat = output.reshape(-1, vocab)
-        n_rows = flat.shape[0]
-        lab = labels.reshape(-1)
-        if lab.dtype not in (torch.int32, torch.int64):
-            lab = lab.to(torch.int64)
-        lab = lab.contiguous()
+        flat = output if output.is_contiguous() and vocab > 0 else output.reshape(-1, vocab)
+        n_rows = flat.numel() // vocab
+        lab = _lib.index_column(labels, dev)
         n_seq, width = batch["responses"].shape[0], batch["responses"].shape[-1]
         layout, padded_s = (0, 0) if cfg["packed"] else (1, output.shape[1])
         again = _swept_again(flat) and not cfg["grad_inplace"]
         ops = _FusedOperands(dev, batch, cfg, n_rows, n_seq, width, layout, padded_s, _lib.dtype_code(flat), vocab,
                              n_rows, sweeps=2 if again else 1)
-        ent = torch.empty(n_rows, dtype=torch.float32, device=dev) if cfg["entropy_coeff"] != 0 else None
-        dlogits = flat if cfg["grad_inplace"] else torch.empty_like(flat)
+        dlogits = flat.detach() if cfg["grad_inplace"] else torch.empty_like(flat, memory_format=torch.contiguous_format)
         stream = _lib.stream(dev)
         ops.prepare(stream)
         shape = (_lib.dtype_code(flat), n_rows, vocab, vocab)
         scalars = (cfg["inv_temperature"], 0 if ops.old is None else 1, cfg["clip_lo"], cfg["clip_hi"], cfg["kl_penalty"],
                    cfg["kl_coef"], cfg["entropy_coeff"], cfg["loss_scale"])
         vocab_ops._timed_call("mrl_fused_logprob_loss", n_rows, dev, _lib.ptr(flat), *shape, _lib.ptr(lab),
-                              _lib.dtype_code(lab), scalars[0], ops.p_ops, *scalars[1:], _lib.ptr(ops.applied),
-                              _lib.ptr(dlogits), vocab, None, _lib.ptr(ent), ops.p_terms, ops.workspace, ops.ws_bytes, 1,
+                              _lib.dtype_code(lab), scalars[0], ops.p_ops, *scalars[1:], ops.p_applied,
+                              _lib.ptr(dlogits), vocab, None, ops.p_ent, ops.p_terms, ops.workspace, ops.ws_bytes, 1,
                               stream)
         ops.reduce(stream)
         if again:
-            ctx.save_for_backward(dlogits, flat, lab, ops.rows, ops.small)
+            ctx.save_for_backward(dlogits, flat.reshape(-1, vocab), lab, ops.rows, ops.small)
             ctx.sweep = (shape, scalars, ops.o_applied, ops.o_second, ops.ws_bytes)
         else:
             ctx.save_for_backward(dlogits, ops.applied)
@@ -380,7 +387,7 @@ class _FusedLogprobLoss(torch.autograd.Function):
             grad = _deliver_swept_grads(ctx, *saved, state, g_loss)
         else:
             (grad,) = _deliver_eager_grads(ctx, saved[:1], saved[1], state, g_loss)
-        return grad.view(shape), None, None, None
+        return grad if tuple(grad.shape) == shape else grad.view(shape), None, None, None
 
 
 def fused_logprob_policy_loss(output, batch, *, packed, seqlens=None, cu_seqlens=None, mask=None, ref_log_prob=None,

@@ -16,6 +16,8 @@ from . import _lib, vocab_ops
 
 
 def _as_index(t):
+    if (t.dtype is torch.int64 or t.dtype is torch.int32) and t.is_contiguous():
+        return t
     """int32 / int64 tensor, flattened and dense, for a [B] or [B,1] length column."""
     if t.dtype not in (torch.int32, torch.int64):
         t = t.to(torch.int64)
@@ -78,13 +80,13 @@ def preprocess_packed_seqs(input_ids, labels, attention_mask_1d, tp_size):
     lab = labels.to(ids.dtype).contiguous()
     if ids.dtype not in (torch.int32, torch.int64):
         raise TypeError("input_ids must be int32 or int64")
-    ids_packed = torch.empty(pack_length, dtype=ids.dtype, device=dev)
-    labels_packed = torch.empty(pack_length, dtype=ids.dtype, device=dev)
-    pos_packed = torch.empty(pack_length, dtype=torch.int32, device=dev)
+    ids_packed = torch.empty((1, pack_length), dtype=ids.dtype, device=dev)
+    labels_packed = torch.empty((1, pack_length), dtype=ids.dtype, device=dev)
+    pos_packed = torch.empty((1, pack_length), dtype=torch.int32, device=dev)
     _lib.call("mrl_pack_rows", _lib.ptr(ids), _lib.ptr(ids_packed), _lib.ptr(lab), _lib.ptr(labels_packed),
               ids.element_size(), batch, width, _lib.ptr(seqlens), _lib.ptr(cu), pack_length, _lib.ptr(pos_packed),
               _lib.stream(dev))
-    return (ids_packed.unsqueeze(0), pos_packed.unsqueeze(0), labels_packed.unsqueeze(0), seqlens, cu)
+    return ids_packed, pos_packed, labels_packed, seqlens, cu
 
 
 class _UnpadGather(torch.autograd.Function):

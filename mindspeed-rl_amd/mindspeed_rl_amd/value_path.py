@@ -32,14 +32,10 @@ class AdaptiveKLController:
 
 
 def _f32(t, dev):
+    """Outside of autograd (what the kernels get is the address)."""
+    if t.dtype is torch.float32 and t.is_contiguous() and t.device == dev:
+        return t
     return _lib.dense(t.detach(), torch.float32, dev)
-
-
-def _lengths(response_length, dev):
-    lens = response_length
-    if lens.dtype not in (torch.int32, torch.int64):
-        lens = lens.to(torch.int64)
-    return lens.to(dev).reshape(-1).contiguous()
 
 
 def kl_token_level_rewards(old_log_prob, ref_log_prob, response_length, rm_scores, beta, penalty="kl"):
@@ -52,8 +48,8 @@ def kl_token_level_rewards(old_log_prob, ref_log_prob, response_length, rm_score
     dev = _lib.require_device(old_log_prob, ref_log_prob)
     old, ref = _f32(old_log_prob, dev), _f32(ref_log_prob, dev)
     batch, width = old.shape
-    lens = _lengths(response_length, dev)
-    scores = _f32(torch.as_tensor(rm_scores), dev).reshape(-1)
+    lens = _lib.index_column(response_length, dev)
+    scores = _f32(torch.as_tensor(rm_scores), dev)
     if lens.numel() != batch or scores.numel() != batch:
         raise ValueError("response_length and rm_scores need one entry per sample")
     rewards = torch.empty_like(old)

@@ -45,12 +45,12 @@ def pack_padded_columns(padded, lengths, left_pad=False):
                              % (key, idx.numel(), src.shape[0]))
         eff = torch.empty(src.shape[0], dtype=torch.int32, device=dev)
         columns.append(_Column(key, src, idx, eff, dev, width=src.shape[1], left_pad=1 if left_pad else 0))
-    _lay_out(columns)
+    batches = _lay_out(columns)
     batch_data, batch_data_length = {}, {}
     for c in columns:
         batch_data[c.key] = c.out = torch.empty(c.total, dtype=c.src.dtype, device=c.dev)
         batch_data_length[c.key] = c.eff
-    _copy(columns, False)
+    _copy(batches, False)
     return batch_data, batch_data_length
 
 
@@ -65,11 +65,15 @@ class _Column:
         self.cu = self.out = None
 
     def fill(self, c, info):
+        """For the scan; the copy differs in what ``fill_copy`` sets."""
         c.lengths, c.lengths_dtype, c.batch = self.lengths.data_ptr(), _lib.dtype_code(self.lengths), self.lengths.numel()
         c.eff_len, c.cu, c.info = _lib.ptr(self.eff), self.cu.data_ptr(), info
-        c.src, c.dst = self.src.data_ptr(), _lib.ptr(self.out)
+        c.src, c.dst = self.src.data_ptr(), None
         c.elem_bytes, c.width, c.multiple, c.first_dim = self.src.element_size(), self.width, self.multiple, self.first_dim
-        c.src_stride, c.total, c.left_pad, c.pad_bits = self.stride, self.total, self.left_pad, self.pad
+        c.src_stride, c.total, c.left_pad, c.pad_bits = self.stride, 0, self.left_pad, self.pad
+
+    def fill_copy(self, c):
+        c.info, c.dst, c.width, c.total = None, self.out.data_ptr(), self.width, self.total
 
 
 def _by_device(columns):
@@ -85,7 +89,9 @@ def _by_device(columns):
 
 
 def _lay_out(columns):
-    """Offsets of every column, and its size on the host: one scan launch and one host read for all of them."""
+    """Offsets of every column, and its size on the host: one scan launch and one host read for all of them.  Returns
+    what the copy takes."""
+    batches = []
     for dev, part in _by_device(columns):
         slot = _lib.HostWords.take(dev, 16 * len(part))
         info = None if slot is not None else torch.empty((len(part), 2), dtype=torch.int64, device=dev)
@@ -98,14 +104,15 @@ def _lay_out(columns):
         sizes = slot.read(ctypes.c_int64, 2 * len(part), _lib.stream(dev)) if slot is not None else info.view(-1).tolist()
         for i, c in enumerate(part):
             c.total, c.longest = sizes[2 * i:2 * i + 2]
+        batches.append((dev, part, args))
+    return batches
 
 
-def _copy(columns, to_padded):
+def _copy(batches, to_padded):
     """The copies of every column, in one launch."""
-    for dev, part in _by_device(columns):
-        args = (_lib.RaggedColumn * len(part))()
+    for dev, part, args in batches:
         for i, c in enumerate(part):
-            c.fill(args[i], None)
+            c.fill_copy(args[i])
         _lib.call("mrl_ragged_columns", 1 if to_padded else 0, args, len(part), _lib.stream(dev))
 
 
@@ -165,12 +172,12 @@ def unpack_pad_experience(batch_data, batch_data_length, pad_id, multiple):
         out[key] = None                          # the order of the lengths' keys
         columns.append(_Column(key, src, _lib.index_column(length_list, dev), None, dev, multiple=int(multiple),
                                first_dim=first_dim, stride=stride, pad=pad))
-    _lay_out(columns)
+    batches = _lay_out(columns)
     for c in columns:
         batch, c.width = c.lengths.numel(), c.longest
         shape = (batch, c.first_dim, c.width) if c.src.dim() > 1 else (batch, c.width)
         out[c.key] = c.out = torch.empty(shape, dtype=c.src.dtype, device=c.dev)
-    _copy(columns, True)
+    _copy(batches, True)
     return out
 
 

@@ -4111,3 +4111,32 @@ def test_vocabulary_shards_merge_to_the_full_sweep(dev, dtype, bounds):
     assert not dz[5].any().item()
     # a label outside every shard: the oracle (Megatron's target mask) scores the row maximum there,
     # a sharded run scores 0 - documented difference, no rank owns such a label
+
+
+@pytest.mark.parametrize("packed", [True, False])
+def test_fused_gradients_have_a_tensor_of_their_own(dev, packed):
+    """The sweep takes logits in the shape they come in.  What the backward hands out is outside of autograd and has
+    the logits' shape and dense strides, in place as well (where it shares their memory), and with lengths as columns
+    or flat, int32 or int64."""
+    gen = torch.Generator().manual_seed(3)
+    n, seq, vocab = 3, 6, 512
+    z = torch.randn(n * seq, vocab, generator=gen).to(dev)
+    lead = (1, n * seq) if packed else (n, seq)
+    y = torch.randint(0, vocab, lead, generator=gen).to(dev)
+    plen, rlen = torch.tensor([[1], [2], [2]], dtype=torch.int32), torch.tensor([[5], [3], [4]], dtype=torch.int32)
+    batch = {"labels": y, "responses": torch.zeros(n, 5, dtype=torch.int64, device=dev),
+             "advantages": torch.randn(n, 5, generator=gen).to(dev), "old_log_prob": -torch.rand(n, 5, generator=gen).to(dev)}
+    cu = torch.arange(0, n * seq + 1, seq, dtype=torch.int32, device=dev)
+    seqlens = (plen + rlen).flatten().to(dev)
+    got = []
+    for inplace in (False, True):
+        for shape, dtype in (((n, 1), torch.int32), ((n,), torch.int64)):
+            leaf = z.clone().view(*lead, vocab).requires_grad_()
+            b = dict(batch, prompt_length=plen.view(shape).to(dtype).to(dev), response_length=rlen.view(shape).to(dtype).to(dev))
+            loss, _ = mrl.fused_logprob_policy_loss(leaf, b, packed=packed, seqlens=seqlens, cu_seqlens=cu, clip_low=0.2,
+                                                    clip_high=0.2, grad_inplace=inplace)
+            (g,) = torch.autograd.grad(loss, leaf)
+            assert g.shape == leaf.shape and g.is_contiguous() and not g.requires_grad and g.grad_fn is None
+            assert (g.data_ptr() == leaf.data_ptr()) is inplace
+            got.append(g)
+    assert all(torch.equal(g, got[0]) for g in got)
