@@ -196,13 +196,13 @@ class _FusedLmHeadLoss(torch.autograd.Function):
             row_terms = torch.empty((max(n_rows, 1), 8), dtype=torch.float32, device=dev)
             p_ops, p_terms = row_ops.data_ptr(), row_terms.data_ptr()
         chunk = max(1, min(chunk_cap, n_rows))
-        # the chunk of logits: rows padded to whole k-steps of the dHidden product; the padding columns
-        # are zeroed once and never written (they meet rows of the weight that read as zero)
+        # the chunk of logits: rows padded to whole k-steps of the dHidden product; the padding columns, up to 56, are
+        # zeroed once and never written (they meet rows of the weight that read as zero).  Zeroing the whole chunk
+        # took 146 us of 9.7 ms at 5 519 x 99 760 x 3 712.
         v_pad = _round_up(vocab, 64)
+        logits = torch.empty((chunk, v_pad), dtype=h2d.dtype, device=dev)
         if v_pad != vocab:
-            logits = torch.zeros((chunk, v_pad), dtype=h2d.dtype, device=dev)
-        else:
-            logits = torch.empty((chunk, v_pad), dtype=h2d.dtype, device=dev)
+            logits[:, vocab:].zero_()
         d_hidden = torch.empty_like(h2d)
         # dWeight leaves the last chunk's product as bf16; fp32 sums exist only between chunks.  dHidden of a
         # step in one chunk may be cut along the vocabulary; in several it never is, so that it does not

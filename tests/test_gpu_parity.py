@@ -4140,3 +4140,29 @@ def test_fused_gradients_have_a_tensor_of_their_own(dev, packed):
             assert (g.data_ptr() == leaf.data_ptr()) is inplace
             got.append(g)
     assert all(torch.equal(g, got[0]) for g in got)
+
+
+@pytest.mark.parametrize("vocab,chunk_rows", [(1000, 32768), (1000, 64), (8, 32768), (1016, 1)])
+def test_lmhead_step_in_memory_full_of_nan(dev, vocab, chunk_rows):
+    """The chunk of logits has padding columns where the vocabulary is no multiple of 64: whatever its memory held
+    before must not reach dHidden.  The same call on zeroed memory and on memory full of NaN."""
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    n, seq, hdim = 4, 40, 128
+    h = torch.randn(1, n * seq, hdim, generator=gen, device=dev).to(torch.bfloat16)
+    w = (torch.randn(vocab, hdim, generator=gen, device=dev) * 0.1).to(torch.bfloat16)
+    length = torch.full((n, 1), seq - 1, dtype=torch.int32, device=dev)
+    batch = {"labels": torch.randint(0, vocab, (1, n * seq), generator=gen, device=dev),
+             "responses": torch.zeros(n, seq - 1, dtype=torch.int64, device=dev), "response_length": length,
+             "prompt_length": torch.ones_like(length), "advantages": torch.randn(n, seq - 1, generator=gen, device=dev),
+             "old_log_prob": torch.full((n, seq - 1), -6.0, device=dev)}
+    cu = torch.arange(0, n * seq + 1, seq, dtype=torch.int32, device=dev)
+    grads = []
+    for value in (0.0, float("nan")):
+        dirt = [torch.full((rows * 1024,), value, dtype=torch.bfloat16, device=dev) for rows in (1, 64, 160, 320)]
+        del dirt                                # the next allocations of these sizes get this memory
+        hv, wv = h.clone().requires_grad_(), w.clone().requires_grad_()
+        loss, _ = mrl.fused_lmhead_policy_loss(hv, wv, batch, packed=True, seqlens=torch.full((n,), seq, dtype=torch.int32, device=dev),
+                                               cu_seqlens=cu, clip_low=0.2, clip_high=0.2, chunk_rows=chunk_rows)
+        grads.append(torch.autograd.grad(loss, (hv, wv)))
+    for a, b in zip(*grads):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
