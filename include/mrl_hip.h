@@ -194,6 +194,16 @@ int mrl_window_logprob(const void* logits, int logits_dtype, int64_t n_rows, int
                        int prompt_dtype, const void* response_length, int response_dtype, int want_entropy,
                        float* logp, float* entropy, void* stream);
 
+/* mrl_window_cells: the rows that mrl_window_cut reads, in the order of the cells they are for: live[k] is a row,
+ * cell[k] its cell i * width + j of the result, *total their number (at most batch * width, the length of both).
+ * Cells without a row are zeroed in logp and entropy, all of entropy's unless want_entropy.  At most
+ * MRL_WINDOW_CELLS_SEQS sequences, at least one cell and row. */
+#define MRL_WINDOW_CELLS_SEQS 2048
+int mrl_window_cells(int layout, int64_t batch, int64_t width, int64_t n_rows, const int32_t* seqlens,
+                     const int32_t* cu_seqlens_padded, int64_t padded_s, const void* prompt_length,
+                     int prompt_dtype, const void* response_length, int response_dtype, int want_entropy,
+                     int32_t* live, int32_t* cell, int64_t* total, float* logp, float* entropy, void* stream);
+
 /* mrl_generate_mask: generate_mask (mindspeed_rl/utils/utils.py:57-67): out[i, j] =
  * (j < lengths[i]) as int64, [batch, width]; lengths is I32 or I64.  Negative lengths give an
  * all-zero row, lengths above width an all-one row. */
@@ -526,6 +536,11 @@ int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, int64_t n_tok
                            int64_t hidden_dim, const void* labels, int labels_dtype,
                            float inv_temperature, float* logp, float* entropy, float* lse,
                            void* workspace, int64_t workspace_bytes, void* stream);
+/* The same with token t's results in entry cells[t] of logp and entropy, which may be longer. */
+int mrl_lmhead_logprob_fwd_cells(const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
+                                 int64_t hidden_dim, const void* labels, int labels_dtype,
+                                 float inv_temperature, const int32_t* cells, float* logp, float* entropy,
+                                 void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * Training step from the hidden states (configs "fused lm_head"): the three matrix products around

@@ -231,7 +231,8 @@ template <typename LabelT, bool kEntropy>
 __global__ __launch_bounds__(256) void lmhead_finish_kernel(
     const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, const LabelT* __restrict__ labels,
     const float* __restrict__ partial, int n_tokens, int vocab, int hdim, int n_leaves, float inv_t,
-    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
+    const int32_t* __restrict__ cells, float* __restrict__ logp, float* __restrict__ entropy,
+    float* __restrict__ lse_out) {
     __shared__ Stats part[16][kFinishTokens];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t0 = (int)blockIdx.x * kFinishTokens;
@@ -278,9 +279,10 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(
         }
         if (lane == 0) {
             const float lse = (r.m * k + fast_log2(r.s)) * kLn2;
-            logp[t] = (y_ok ? dot * inv_t : r.m * inv_t) - lse;
-            if (kEntropy) entropy[t] = lse - (r.u / r.s) * inv_t;
-            if (lse_out) lse_out[t] = lse;
+            const int64_t at = cells ? (int64_t)cells[t] : (int64_t)t;
+            logp[at] = (y_ok ? dot * inv_t : r.m * inv_t) - lse;
+            if (kEntropy) entropy[at] = lse - (r.u / r.s) * inv_t;
+            if (lse_out) lse_out[at] = lse;
         }
     }
 }
@@ -321,12 +323,14 @@ extern "C" int64_t mrl_lmhead_workspace_bytes(int64_t n_tokens, int64_t vocab) {
     return (int64_t)VocabLeaves(vocab).n * (n_tokens < kMaxSlice ? n_tokens : kMaxSlice) * 3 * (int64_t)sizeof(float);
 }
 
-// Checks and launches shared by the two forward entry points.  `partial` holds the statistics of `slice`
+// Checks and launches shared by the forward entry points; token t's results go to entry t of the outputs, or with
+// `cells` to entry cells[t].  `partial` holds the statistics of `slice`
 // tokens (whole tiles); more are taken in equal slices, one after the other on the stream (32 768 tokens x
 // 152 064 x 3 584 where 28 160 fit: 26.2 ms as 28 160 + 4 608, 25.2 ms as 2 x 16 384).
 static int lmhead_forward(const char* fn, const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
-                          int64_t hidden_dim, const void* labels, int labels_dtype, float inv_temperature, float* logp,
-                          float* entropy, float* lse, float* partial, int64_t slice, hipStream_t s) {
+                          int64_t hidden_dim, const void* labels, int labels_dtype, float inv_temperature,
+                          const int32_t* cells, float* logp, float* entropy, float* lse, float* partial, int64_t slice,
+                          hipStream_t s) {
     // 256-token tiles, all of a CU's LDS for the tile loop.  Function
     // attributes belong to a device, so the reservation is made with every launch, on whichever
     // device is current.
@@ -351,11 +355,13 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
         int rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
         const dim3 fgrid((unsigned)((n + kFinishTokens - 1) / kFinishTokens)), fblock(256);
-        float* ent = entropy ? entropy + lo : nullptr;
-        float* lse_out = lse ? lse + lo : nullptr;
+        const int64_t out_lo = cells ? 0 : lo;
+        float* ent = entropy ? entropy + out_lo : nullptr;
+        float* lse_out = lse ? lse + out_lo : nullptr;
+        const int32_t* to = cells ? cells + lo : nullptr;
         auto finish = [&](auto kernel, auto* lab) {
             hipLaunchKernelGGL(kernel, fgrid, fblock, 0, s, h, (const uint16_t*)weight, lab + lo, (const float*)partial, n,
-                               (int)vocab, (int)hidden_dim, leaves.n, inv_temperature, logp + lo, ent, lse_out);
+                               (int)vocab, (int)hidden_dim, leaves.n, inv_temperature, to, logp + out_lo, ent, lse_out);
         };
         if (wide_labels)
             finish(entropy ? lmhead_finish_kernel<int64_t, true> : lmhead_finish_kernel<int64_t, false>, (const int64_t*)labels);
@@ -379,11 +385,10 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
     MRL_REQUIRE(inv_temperature > 0.f && inv_temperature < 1.0e6f, MRL_ERR_INVALID_ARG,                                \
                 "%s: inv_temperature=%g must be in (0, 1e6)", fn, (double)inv_temperature)
 
-extern "C" int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
-                                      int64_t hidden_dim, const void* labels, int labels_dtype,
-                                      float inv_temperature, float* logp, float* entropy, float* lse,
-                                      void* workspace, int64_t workspace_bytes, void* stream) {
-    const char* fn = "mrl_lmhead_logprob_fwd";
+static int forward_in_workspace(const char* fn, const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
+                                int64_t hidden_dim, const void* labels, int labels_dtype, float inv_temperature,
+                                const int32_t* cells, float* logp, float* entropy, float* lse, void* workspace,
+                                int64_t workspace_bytes, void* stream) {
     MRL_LMHEAD_CHECK_ARGS(fn);
     if (n_tokens == 0) return MRL_OK;
     MRL_REQUIRE(hidden && weight && labels && logp && workspace, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
@@ -392,8 +397,26 @@ extern "C" int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, in
     MRL_REQUIRE(workspace_bytes >= mrl_lmhead_workspace_bytes(n_tokens, vocab), MRL_ERR_INVALID_ARG,
                 "%s: workspace of %lld bytes, need %lld", fn, (long long)workspace_bytes,
                 (long long)mrl_lmhead_workspace_bytes(n_tokens, vocab));
-    return lmhead_forward(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, logp,
-                          entropy, lse, (float*)workspace, kMaxSlice, mrl::as_stream(stream));
+    return lmhead_forward(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, cells,
+                          logp, entropy, lse, (float*)workspace, kMaxSlice, mrl::as_stream(stream));
+}
+
+extern "C" int mrl_lmhead_logprob_fwd(const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
+                                      int64_t hidden_dim, const void* labels, int labels_dtype,
+                                      float inv_temperature, float* logp, float* entropy, float* lse,
+                                      void* workspace, int64_t workspace_bytes, void* stream) {
+    return forward_in_workspace("mrl_lmhead_logprob_fwd", hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype,
+                                inv_temperature, nullptr, logp, entropy, lse, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mrl_lmhead_logprob_fwd_cells(const void* hidden, const void* weight, int64_t n_tokens, int64_t vocab,
+                                            int64_t hidden_dim, const void* labels, int labels_dtype,
+                                            float inv_temperature, const int32_t* cells, float* logp, float* entropy,
+                                            void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "mrl_lmhead_logprob_fwd_cells";
+    MRL_REQUIRE(cells != nullptr || n_tokens == 0, MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    return forward_in_workspace(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, cells,
+                                logp, entropy, nullptr, workspace, workspace_bytes, stream);
 }
 
 // Address of `scratch` on the current device, looked up once per device (each GPU holds its own
@@ -438,6 +461,6 @@ extern "C" int mrl_lmhead_logprob_fwd_static(const void* hidden, const void* wei
     if (!partial) return MRL_ERR_LAUNCH;
     // whole token tiles that the scratch memory holds the statistics of (28 160 tokens at 152 064 entries)
     const int64_t slice = MRL_LMHEAD_STATIC_BYTES / (VocabLeaves(vocab).n * 12LL) / 256 * 256;
-    return lmhead_forward(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, logp,
-                          entropy, lse, partial, slice, mrl::as_stream(stream));
+    return lmhead_forward(fn, hidden, weight, n_tokens, vocab, hidden_dim, labels, labels_dtype, inv_temperature, nullptr,
+                          logp, entropy, lse, partial, slice, mrl::as_stream(stream));
 }

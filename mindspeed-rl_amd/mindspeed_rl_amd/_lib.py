@@ -55,6 +55,7 @@ SIGNATURES = {
     "mrl_window_cut": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _vp],
     "mrl_window_logprob": [_vp, _int, _i64, _i64, _i64, _vp, _int, _f32, _int, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp,
                            _int, _int, _vp, _vp, _vp],
+    "mrl_window_cells": [_int, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _int, _vp, _int, _int, _vp, _vp, _vp, _vp, _vp, _vp],
     "mrl_generate_mask": [_vp, _int, _i64, _i64, _vp, _vp],
     "mrl_live_rows": [_vp, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
     "mrl_move_rows": [_vp, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _int, _vp],
@@ -88,6 +89,7 @@ SIGNATURES = {
     "mrl_scale_rows_note": [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
     "mrl_lmhead_workspace_bytes": [_i64, _i64],
     "mrl_lmhead_logprob_fwd": [_vp, _vp, _i64, _i64, _i64, _vp, _int, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
+    "mrl_lmhead_logprob_fwd_cells": [_vp, _vp, _i64, _i64, _i64, _vp, _int, _f32, _vp, _vp, _vp, _vp, _i64, _vp],
     "mrl_lmhead_logits": [_vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp],
     "mrl_lmhead_logprob_bwd": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp],
     "mrl_lmhead_bwd_workspace_bytes": [_i64, _i64, _i64],

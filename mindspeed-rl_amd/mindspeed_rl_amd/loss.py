@@ -488,9 +488,14 @@ class StandardLogProbComputer(LogProbComputer):
         if weight is not None:
             # `output` holds the hidden states: the rows of the response windows are projected and scored
             # tile by tile on the matrix cores, no logits are written (forward only, no autograd)
-            from .lmhead import lmhead_logprob
-            windows, active = self._active_rows(output, batch, kwargs)
-            log_probs, entropy, _ = lmhead_logprob(output, weight, labels, inv_temperature=inv_t,
+            from . import lmhead
+            if own_cut and self._rows_in_windows is StandardLogProbComputer._rows_in_windows:
+                windows = self._windows(output, batch, kwargs)
+                scores = lmhead.score_windows(output, weight, labels, windows, inv_t, not skip_entropy)
+                if scores is not None:
+                    return scores
+            windows, active = self._active_rows(output, batch, kwargs, windows)
+            log_probs, entropy, _ = lmhead.lmhead_logprob(output, weight, labels, inv_temperature=inv_t,
                                                    want_entropy=not skip_entropy, row_active=active)
         elif injected is not None and injected is not vocab_ops.vocab_parallel_cross_entropy:
             # a caller's own cross entropy (the reference's hook) scores the rows, as in the reference

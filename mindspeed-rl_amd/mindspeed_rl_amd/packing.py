@@ -292,6 +292,19 @@ class ResponseWindows:
                               _lib.stream(self.dev))
         return logp, ent
 
+    MAX_CELL_SEQS = 2048        # MRL_WINDOW_CELLS_SEQS
+
+    def cells(self, want_entropy, slot):
+        """``(live, cell, logp, entropy)``: the rows that :meth:`cut` reads, the cells of the ``[B, L]`` results that
+        they are for, and these results with zeros in every other cell; how many rows there are arrives in ``slot``."""
+        index = torch.empty((2, self.n_seq * self.width), dtype=torch.int32, device=self.dev)
+        logp = torch.empty((self.n_seq, self.width), dtype=torch.float32, device=self.dev)
+        ent = torch.empty_like(logp)
+        p_live, p_cell = index.data_ptr(), index.data_ptr() + 4 * self.n_seq * self.width
+        _lib.call("mrl_window_cells", *self._args, 1 if want_entropy else 0, p_live, p_cell, slot.addr, _lib.ptr(logp),
+                  _lib.ptr(ent), _lib.stream(self.dev))
+        return index, p_live, p_cell, logp, ent
+
     def cut(self, logp_rows, entropy_rows):
         """``(log_probs, entropy)`` ``[B, L]`` fp32 in one launch; entropies are zeros for ``None``.  No autograd."""
         _lib.require_device(self.prompt, logp_rows, entropy_rows)

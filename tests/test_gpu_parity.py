@@ -4166,3 +4166,40 @@ def test_lmhead_step_in_memory_full_of_nan(dev, vocab, chunk_rows):
         grads.append(torch.autograd.grad(loss, (hv, wv)))
     for a, b in zip(*grads):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("layout", ["padded", "packed"])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_scoring_pass_from_hidden_states_cell_by_cell(dev, monkeypatch, layout, index):
+    """Rows found with their cells equal flagged rows, spread and cut, to the last bit: overlapping windows, windows
+    that start in front of the rows, end behind them or behind the result, empty ones, none at all, more sequences
+    than a workgroup has threads, hidden states that are not dense, labels outside the vocabulary."""
+    from mindspeed_rl_amd import lmhead
+    gen = torch.Generator().manual_seed(17)
+    vocab, hdim, kw = 520, 64, {}
+    p0, r0 = [0, 1, 7, 3, 40, 4, 9], [38, 5, 0, 50, 3, 60, 31]
+    comp = mrl.StandardLogProbComputer()
+    for repeat, empty in ((1, False), (43, False), (1, True)):
+        plen = torch.tensor(p0 * repeat, dtype=index).view(-1, 1)
+        rlen = torch.tensor(r0 * repeat, dtype=index).view(-1, 1) * (0 if empty else 1)
+        n_seq, padded = plen.shape[0], 37
+        lead = (n_seq, padded)
+        if layout == "packed":
+            seqlens = (plen.flatten() if empty else torch.tensor([30, 6, 7, 40, 43, 4, 40] * repeat)).to(torch.int32)
+            cu = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(seqlens, 0)]).to(torch.int32)
+            lead = (1, int(cu[-1]) - 5)                                     # the last window ends behind the rows
+            kw = dict(use_remove_padding=True, seqlens_in_batch=seqlens.to(dev), cu_seqlens_padded=cu.to(dev), seq_len=43)
+        wide = torch.randn(*lead, hdim + 8, generator=gen).to(torch.bfloat16).to(dev)
+        weight = (torch.randn(vocab, hdim, generator=gen) * 0.3).to(torch.bfloat16).to(dev)
+        labels = torch.randint(-1, vocab + 1, lead, generator=gen).to(index)
+        for width in (1, 12, 300):
+            b = _to_dev({"responses": torch.zeros(n_seq, width, dtype=torch.int64), "prompt_length": plen,
+                         "response_length": rlen, "labels": labels}, dev)
+            for out in (wide[..., :hdim].contiguous(), wide[..., :hdim]):
+                for skip in (False, True):
+                    got = comp.compute(out, b, skip, inv_temperature=1.25, lm_head_weight=weight, **kw)
+                    with monkeypatch.context() as m:
+                        m.setattr(lmhead, "score_windows", lambda *a: None)
+                        want = comp.compute(out, b, skip, inv_temperature=1.25, lm_head_weight=weight, **kw)
+                    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+                    assert want[0].any().item() is not empty and (empty or want[1].any().item() is not skip)
