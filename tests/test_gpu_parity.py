@@ -4203,3 +4203,52 @@ def test_scoring_pass_from_hidden_states_cell_by_cell(dev, monkeypatch, layout, 
                         want = comp.compute(out, b, skip, inv_temperature=1.25, lm_head_weight=weight, **kw)
                     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
                     assert want[0].any().item() is not empty and (empty or want[1].any().item() is not skip)
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 8192), (torch.float16, 14208), (torch.float32, 32000),
+                                         (torch.bfloat16, 40003), (torch.bfloat16, 72608), (torch.bfloat16, 152064),
+                                         (torch.float32, 152064)])
+@pytest.mark.parametrize("entropy_coeff", [0.0, 0.01])
+def test_fused_sweep_statistics_across_threads(dev, dtype, vocab, entropy_coeff):
+    """The row's statistics come from threads whose references differ: rows that rise or fall over the whole row, whose
+    weight lies in one entry of any wavefront, or - without the entropy, which is undefined there - whose entries are
+    all -inf but a few.  Workgroups of 4, 8 and 16 wavefronts and two per row, against 64 bits."""
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    ramp = torch.linspace(-80.0, 80.0, vocab, device=dev)
+    rows = [torch.randn(vocab, generator=gen, device=dev) * 3, ramp, -ramp]
+    vec = 16 // torch.finfo(dtype).bits * 8
+    for at in [0, vocab - 1, 63 * vec, 64 * vec, 1023 * vec + 1, vocab // 2 - 1, vocab // 2] + list(range(5, vocab, vocab // 9)):
+        spike = torch.randn(vocab, generator=gen, device=dev)
+        spike[at] = 30.0
+        rows.append(spike)
+        if entropy_coeff == 0:
+            few = torch.full((vocab,), float("-inf"), device=dev)
+            few[at], few[(at * 7 + 3) % vocab] = 1.0, 0.5
+            rows.append(few)
+    z = torch.stack(rows).to(dtype)
+    n = z.shape[0]
+    y = torch.argmax(z, -1)
+    # one sequence: a prompt token, n response tokens (scored by rows 0 .. n - 1), the last row not looked at
+    leaf = torch.cat([z, z[:1]]).view(1, n + 1, vocab).requires_grad_()
+    batch = {"labels": torch.cat([y, y[:1]]).view(1, n + 1), "responses": torch.zeros(1, n, dtype=torch.int64, device=dev),
+             "response_length": torch.tensor([[n]], device=dev), "prompt_length": torch.tensor([[1]], device=dev),
+             "advantages": torch.ones(1, n, device=dev)}
+    loss, out = mrl.fused_logprob_policy_loss(leaf, batch, packed=True, clip_low=0.2, clip_high=0.2, entropy_coeff=entropy_coeff,
+                                              seqlens=torch.tensor([n + 1], dtype=torch.int32, device=dev),
+                                              cu_seqlens=torch.tensor([0, n + 1], dtype=torch.int32, device=dev))
+    (g,) = torch.autograd.grad(loss, leaf)
+    logp = torch.log_softmax(z.double(), -1)
+    p = logp.exp()
+    want = p.clone()
+    want[torch.arange(n, device=dev), y] -= 1.0
+    if entropy_coeff != 0:
+        ent = -(p * logp).sum(-1, keepdim=True)
+        want += entropy_coeff * p * (logp + ent)
+        # entropies below 12, sums of 152 064 terms in fp32 chains of at most 152: 2e-5 of 12
+        assert abs(out[5].item() - ent.mean().item()) < 3e-4
+    want /= n
+    # one rounding of the result; in fp32 exp2 of arguments up to 230 (1.5e-5 of p) and 1 - p near the label
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 4e-5}[dtype]
+    tiny = 2.0 ** -24 if dtype is torch.float16 else 0.0       # fp16 below its normal range
+    bound = want.abs() * (unit + 4e-5) + 4e-5 * p / n + tiny + 1e-12
+    assert ((g[0, :n].double() - want).abs() <= bound).all() and not g[0, n].any().item()
