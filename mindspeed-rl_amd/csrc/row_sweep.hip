@@ -236,10 +236,16 @@ __device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int 
 // (the largest entry then contributes at least 1), and for ordinary logits it is within a few units
 // of the maximum, so nothing comes near the 2^127 an fp32 holds.  Taking the largest entry of the
 // thread's first vector saves the maximum over every vector and the rescale that follows it - a
-// quarter of the arithmetic of the pass.  If a sum does end up beyond 2^120, infinite or NaN (logits
-// that climb by more than 80 above that entry, infinities, NaN), the thread takes its statistics
+// quarter of the arithmetic of the pass.  If a sum does end up beyond 2^90, infinite or NaN (logits
+// that climb by more than 62 above that entry, infinities, NaN), the thread takes its statistics
 // once more, carefully.  Which way a thread went depends only on its own entries.
-constexpr float kSumLimit = 1.329228e36f;      // 2^120
+//
+// The limit is what the reduction below can bring to another reference.  A reference that lies 126 or
+// more powers of two under the largest one is scaled by a flushed zero, and with it goes up to 2^90 x
+// 2^-126 of the row's weight (which is 1 at least) a thread: 2^-26 from all 1024 threads, below half
+// an ulp.  (With 2^120 it was up to 2^-6 a thread: a logsumexp of 0.003 for 1.336.)  Sums of 1024
+// threads against one reference stay below 2^100.
+constexpr float kSumLimit = 1.2379400392853803e27f;     // 2^90
 
 template <int DT, bool kEntropy>
 __device__ __forceinline__ void add_vector(const u32x4& vec, float k, float rk, float& s, float& u) {

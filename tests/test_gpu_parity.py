@@ -4252,3 +4252,51 @@ def test_fused_sweep_statistics_across_threads(dev, dtype, vocab, entropy_coeff)
     tiny = 2.0 ** -24 if dtype is torch.float16 else 0.0       # fp16 below its normal range
     bound = want.abs() * (unit + 4e-5) + 4e-5 * p / n + tiny + 1e-12
     assert ((g[0, :n].double() - want).abs() <= bound).all() and not g[0, n].any().item()
+
+
+@pytest.mark.parametrize("dtype,vocab,threads,vectors", [
+    (torch.bfloat16, 8192, 256, 4), (torch.float16, 14208, 256, 7), (torch.bfloat16, 40003, 512, 9),
+    (torch.float32, 32000, 1024, 7), (torch.bfloat16, 72608, 1024, 8), (torch.bfloat16, 152064, 1024, 18),
+    (torch.float32, 152064, 1024, 18)])
+@pytest.mark.parametrize("inv_t", [1.0, 5.0])
+def test_fused_sweep_threads_far_below_the_maximum(dev, dtype, vocab, threads, vectors, inv_t):
+    """Threads whose first vector - their reference - lies 88 to 90 nats below the row's largest, where 2 to that is no
+    fp32 any more, while a later vector of theirs competes with it: 4.5 to 8 nats below the maximum, together up to ten
+    times its weight.  Every thread of the workgroup (which takes vectors t, t + threads, ... of a row, or of half of
+    one), those of one wavefront, one thread; entries of any depth in between as well.  Against 64 bits."""
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    per = 16 // (torch.finfo(dtype).bits // 8)
+    wide = vocab * torch.finfo(dtype).bits // 8 > 19 * 1024 * 16
+    first = vocab // 2 if wide else 0                       # the second half of a row that two workgroups hold
+    rows = []
+    for below, near in ((88.0, 4.75), (88.5, 5.25), (89.0, 5.75), (89.5, 6.25), (90.0, 6.75), (90.0, 8.0), (88.5, 20.0), (80.0, 1.0)):
+        for who in (range(threads), range(64, 128), (100,)):
+            row = torch.full((vocab,), -below, device=dev)
+            at = first + (torch.tensor(list(who), device=dev) + threads * (1 + len(rows) % (vectors - 1))) * per
+            row[at[at < vocab]] = -near
+            row[first + 37 * per] = 0.0
+            rows.append(row)
+    for spread in (0.0, 45.0, 90.0):
+        row = -spread * torch.rand(vocab, generator=gen, device=dev)
+        row[first:first + threads * per] = -88.5
+        row[first + 5 * per] = 0.0
+        rows.append(row)
+    z = (torch.stack(rows) / inv_t).to(dtype)
+    n = z.shape[0]
+    y = torch.argmax(z, -1)
+    leaf = torch.cat([z, z[:1]]).view(1, n + 1, vocab).requires_grad_()
+    batch = {"labels": torch.cat([y, y[:1]]).view(1, n + 1), "responses": torch.zeros(1, n, dtype=torch.int64, device=dev),
+             "response_length": torch.tensor([[n]], device=dev), "prompt_length": torch.tensor([[1]], device=dev),
+             "advantages": torch.ones(1, n, device=dev)}
+    loss, _ = mrl.fused_logprob_policy_loss(leaf, batch, packed=True, clip_low=0.2, clip_high=0.2, inv_temperature=inv_t,
+                                            seqlens=torch.tensor([n + 1], dtype=torch.int32, device=dev),
+                                            cu_seqlens=torch.tensor([0, n + 1], dtype=torch.int32, device=dev))
+    (g,) = torch.autograd.grad(loss, leaf)
+    want = torch.softmax(z.double() * inv_t, -1)
+    p = want.clone()
+    want[torch.arange(n, device=dev), y] -= 1.0
+    # one rounding of the result, exp2 of arguments up to 130 in fp32 (2^-17 of p); p - 1 near the label
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
+    tiny = 2.0 ** -24 if dtype is torch.float16 else 0.0
+    bound = (want.abs() * (unit + 2e-5) + 2e-5 * p) * inv_t / n + tiny + 1e-12
+    assert ((g[0, :n].double() - want * inv_t / n).abs() <= bound).all()
