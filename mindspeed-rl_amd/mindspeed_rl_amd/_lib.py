@@ -36,6 +36,7 @@ class RaggedColumn(ctypes.Structure):
 
 
 RAGGED_COLUMNS = 16         # MRL_RAGGED_COLUMNS
+ERR_LAUNCH = -4             # MRL_ERR_LAUNCH
 
 
 # name -> argtypes; the order is that of include/mrl_hip.h
@@ -244,32 +245,47 @@ def index_column(t, dev):
 # ------------------------------------------------------------------------------------ results for the host
 class HostWords:
     """A slot of pinned host memory that a kernel leaves a few numbers in: the host watches it instead of copying
-    from the device and waiting for the copy.  ``addr`` goes to the kernel as the address of its output; one of the
-    readers waits for the numbers, takes them and gives the slot back.  Where that fails the slot is not used again:
-    a kernel may still write to it."""
+    from the device and waiting for the copy.  ``addr`` goes to the kernel as the address of its output, by ``launch``;
+    one of the readers waits for the numbers, takes them and gives the slot back.  A slot that is never read, or not
+    to its end, is not used again: a kernel may still write to it.  So its memory is not freed either."""
 
     BYTES = 4096
     _free = {}                  # device index -> slots that nothing writes to (list operations are atomic)
+    _blocks = []                # all memory that slots lie in, as long as the process lives
     _BLOCK = 16                 # slots that are allocated together; there are as many as were ever taken at once
+    _MOST_BLOCKS = 64           # 4 MiB; where they are all taken or lost, results are copied
 
     def __init__(self, f32, key):
         self.f32, self.addr, self._key = f32, f32.data_ptr(), key
 
     @classmethod
     def take(cls, dev, n_bytes):
-        """An empty slot of ``n_bytes``, or None: more than a slot holds, or the stream is being captured (the
-        numbers will be there after a replay, not now)."""
+        """An empty slot of ``n_bytes``, or None: more than a slot holds, no more slots, or the stream is being
+        captured (the numbers will be there after a replay, not now)."""
         if n_bytes > cls.BYTES or _capturing():
             return None
         free = cls._free.setdefault(dev.index, [])
         try:
             slot = free.pop()
         except IndexError:
+            if len(cls._blocks) >= cls._MOST_BLOCKS:
+                return None
             block = torch.empty((cls._BLOCK, cls.BYTES // 4), dtype=torch.float32, pin_memory=True)
+            cls._blocks.append(block)
             slot, *more = [cls(row, dev.index) for row in block.unbind(0)]
             free.extend(more)
         ctypes.memset(slot.addr, 0xff, n_bytes)
         return slot
+
+    def launch(self, name, *args):
+        """:func:`call` of an entry point that gets ``addr``.  One that refuses its arguments has launched nothing, and
+        the slot goes back; what a failed launch leaves behind is not known."""
+        try:
+            call(name, *args)
+        except Exception as e:
+            if getattr(e, "code", None) != ERR_LAUNCH:
+                self._free[self._key].append(self)
+            raise
 
     def _arrived(self, n_bytes, stream):
         call("mrl_host_wait", self.addr, n_bytes // 4, stream)

@@ -96,10 +96,10 @@ def score_windows(hidden, weight, labels, windows, inv_temperature, want_entropy
     if windows.n_seq * windows.width > 0x7fffffff or vocab_ops._transformed():
         return None
     dev = _lib.require_device(hidden, weight, labels, windows.prompt)
-    slot = _lib.HostWords.take(dev, 8)
-    if slot is None:
+    found = windows.cells(want_entropy)
+    if found is None:
         return None
-    index, p_live, p_cell, logp, ent = windows.cells(want_entropy, slot)
+    slot, index, p_live, p_cell, logp, ent = found
     (n,) = slot.read(ctypes.c_int64, 1, _lib.stream(dev))
     if n > 0:
         flat = hidden.detach().reshape(-1, hidden.shape[-1])
@@ -153,14 +153,16 @@ class _LiveRows:
         self.dev, self.n_all = dev, n
         blocks = (n + 1023) // 1024
         index = torch.empty(2 * n + blocks, dtype=torch.int32, device=dev)
-        slot = _lib.HostWords.take(dev, 8) if n > 0 else None
-        total = torch.empty(1, dtype=torch.int64, device=dev) if slot is None else None
         self.live, self.place = index[:n], index[n:2 * n]
-        _lib.call("mrl_live_rows", flags if isinstance(flags, int) else _lib.ptr(flags), dtype, stride, n,
-                  index.data_ptr(), index.data_ptr() + 4 * n, index.data_ptr() + 8 * n, slot.addr if slot is not None else _lib.ptr(total), _lib.stream(dev))
+        args = (flags if isinstance(flags, int) else _lib.ptr(flags), dtype, stride, n,
+                index.data_ptr(), index.data_ptr() + 4 * n, index.data_ptr() + 8 * n)
+        slot = _lib.HostWords.take(dev, 8) if n > 0 else None
         if slot is not None:
+            slot.launch("mrl_live_rows", *args, slot.addr, _lib.stream(dev))
             (self.n,) = slot.read(ctypes.c_int64, 1, _lib.stream(dev))
         else:
+            total = torch.empty(1, dtype=torch.int64, device=dev)
+            _lib.call("mrl_live_rows", *args, _lib.ptr(total), _lib.stream(dev))
             self.n = int(total.item()) if n > 0 else 0
 
     def gather(self, table, labels, ops):

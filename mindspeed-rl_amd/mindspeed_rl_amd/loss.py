@@ -325,13 +325,14 @@ class _FusedOperands:
         cfg = self.cfg
         # word 1 of the cleared sweep workspace counts the workgroups of the reduce step
         done = self.workspace + 4 if self.n_rows > 0 else None
-        sent = cfg.get("sent")
+        sent, p_loss = cfg.get("sent"), _lib.ptr(self.loss)
         slot = _lib.HostWords.take(self.dev, 32) if sent is not None else None
-        _lib.call("mrl_fused_loss_reduce_host", self.p_terms if p_terms is None else p_terms, self.p_start, self.p_count,
-                  self.n_seq, self.width, _lib.ptr(self.old), _lib.ptr(self.ref), _lib.ptr(self.adv),
-                  _lib.ptr(self.mask_t), self.mdt, _lib.ptr(self.resp), self.rdt, cfg["clip_lo"], cfg["clip_hi"],
-                  cfg["kl_penalty"], cfg["kl_coef"], cfg["entropy_coeff"], cfg["seq_mean"], cfg["loss_scale"],
-                  self.p_sums, self.p_out, done, _lib.ptr(self.loss), slot.addr if slot is not None else None, stream)
+        launch = _lib.call if slot is None else slot.launch
+        launch("mrl_fused_loss_reduce_host", self.p_terms if p_terms is None else p_terms, self.p_start, self.p_count,
+               self.n_seq, self.width, _lib.ptr(self.old), _lib.ptr(self.ref), _lib.ptr(self.adv),
+               _lib.ptr(self.mask_t), self.mdt, _lib.ptr(self.resp), self.rdt, cfg["clip_lo"], cfg["clip_hi"],
+               cfg["kl_penalty"], cfg["kl_coef"], cfg["entropy_coeff"], cfg["seq_mean"], cfg["loss_scale"],
+               self.p_sums, self.p_out, done, p_loss, slot.addr if slot is not None else None, stream)
         if slot is not None:
             sent.append(slot)
 

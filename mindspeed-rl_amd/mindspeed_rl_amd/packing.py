@@ -46,7 +46,7 @@ def pack_index(attention_mask_1d, tp_size):
     return (*_pack_index(attention_mask_1d, tp_size, total.data_ptr()), total)
 
 
-def _pack_index(attention_mask_1d, tp_size, p_total):
+def _pack_index(attention_mask_1d, tp_size, p_total, launch=_lib.call):
     mask = attention_mask_1d
     if mask.dtype not in (torch.int64, torch.int32, torch.uint8, torch.bool, torch.float32):
         mask = mask.to(torch.int64)
@@ -55,8 +55,8 @@ def _pack_index(attention_mask_1d, tp_size, p_total):
     batch, width = mask.shape
     seqlens = torch.empty(batch, dtype=torch.int32, device=dev)
     cu = torch.empty(batch + 1, dtype=torch.int32, device=dev)
-    _lib.call("mrl_pack_index_build", _lib.ptr(mask), _lib.dtype_code(mask), batch, width, int(tp_size),
-              _lib.ptr(seqlens), _lib.ptr(cu), p_total, _lib.stream(dev))
+    launch("mrl_pack_index_build", _lib.ptr(mask), _lib.dtype_code(mask), batch, width, int(tp_size),
+           _lib.ptr(seqlens), _lib.ptr(cu), p_total, _lib.stream(dev))
     return seqlens, cu
 
 
@@ -68,10 +68,11 @@ def preprocess_packed_seqs(input_ids, labels, attention_mask_1d, tp_size):
     if attention_mask_1d.shape != (batch, width):
         raise ValueError("attention_mask_1d must have shape (batch_size, seq_len) matching input_ids")
     dev = _lib.require_device(input_ids, labels, attention_mask_1d)
+    tp_size = int(tp_size)
     # the one host read: sizes the packed outputs
     slot = _lib.HostWords.take(dev, 8)
     if slot is not None:
-        seqlens, cu = _pack_index(attention_mask_1d, tp_size, slot.addr)
+        seqlens, cu = _pack_index(attention_mask_1d, tp_size, slot.addr, slot.launch)
         (pack_length,) = slot.read(ctypes.c_int64, 1, _lib.stream(dev))
     else:
         seqlens, cu, total = pack_index(attention_mask_1d, tp_size)
@@ -294,16 +295,20 @@ class ResponseWindows:
 
     MAX_CELL_SEQS = 2048        # MRL_WINDOW_CELLS_SEQS
 
-    def cells(self, want_entropy, slot):
-        """``(live, cell, logp, entropy)``: the rows that :meth:`cut` reads, the cells of the ``[B, L]`` results that
-        they are for, and these results with zeros in every other cell; how many rows there are arrives in ``slot``."""
+    def cells(self, want_entropy):
+        """``(slot, memory, live, cell, logp, entropy)``: the addresses of the rows that :meth:`cut` reads and of the
+        cells of the ``[B, L]`` results that they are for, and these results with zeros in every other cell; how many
+        rows there are arrives in ``slot``.  None where there is no slot."""
         index = torch.empty((2, self.n_seq * self.width), dtype=torch.int32, device=self.dev)
         logp = torch.empty((self.n_seq, self.width), dtype=torch.float32, device=self.dev)
         ent = torch.empty_like(logp)
         p_live, p_cell = index.data_ptr(), index.data_ptr() + 4 * self.n_seq * self.width
-        _lib.call("mrl_window_cells", *self._args, 1 if want_entropy else 0, p_live, p_cell, slot.addr, _lib.ptr(logp),
-                  _lib.ptr(ent), _lib.stream(self.dev))
-        return index, p_live, p_cell, logp, ent
+        slot = _lib.HostWords.take(self.dev, 8)
+        if slot is None:
+            return None
+        slot.launch("mrl_window_cells", *self._args, 1 if want_entropy else 0, p_live, p_cell, slot.addr, _lib.ptr(logp),
+                    _lib.ptr(ent), _lib.stream(self.dev))
+        return slot, index, p_live, p_cell, logp, ent
 
     def cut(self, logp_rows, entropy_rows):
         """``(log_probs, entropy)`` ``[B, L]`` fp32 in one launch; entropies are zeros for ``None``.  No autograd."""

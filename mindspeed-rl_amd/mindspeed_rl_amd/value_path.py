@@ -53,13 +53,17 @@ def kl_token_level_rewards(old_log_prob, ref_log_prob, response_length, rm_score
     if lens.numel() != batch or scores.numel() != batch:
         raise ValueError("response_length and rm_scores need one entry per sample")
     rewards = torch.empty_like(old)
+    args = (_lib.ptr(old), _lib.ptr(ref), _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(scores), batch, width,
+            _lib.KL_BY_NAME[penalty], float(beta), _lib.ptr(rewards))
     slot = _lib.HostWords.take(dev, 4 * batch) if batch > 0 else None
-    row_kl = torch.empty(batch, dtype=torch.float32, device=dev) if slot is None else None
-    _lib.call("mrl_kl_token_rewards", _lib.ptr(old), _lib.ptr(ref), _lib.ptr(lens), _lib.dtype_code(lens),
-              _lib.ptr(scores), batch, width, _lib.KL_BY_NAME[penalty], float(beta), _lib.ptr(rewards),
-              slot.addr if slot is not None else _lib.ptr(row_kl), _lib.stream(dev))
     # the host waits for the kernel either way: the mean of `batch` numbers is taken where they land
-    row_kl = slot.read_doubles_of(batch, _lib.stream(dev)) if slot is not None else row_kl.cpu().double()
+    if slot is not None:
+        slot.launch("mrl_kl_token_rewards", *args, slot.addr, _lib.stream(dev))
+        row_kl = slot.read_doubles_of(batch, _lib.stream(dev))
+    else:
+        row_kl = torch.empty(batch, dtype=torch.float32, device=dev)
+        _lib.call("mrl_kl_token_rewards", *args, _lib.ptr(row_kl), _lib.stream(dev))
+        row_kl = row_kl.cpu().double()
     return rewards, torch.mean(row_kl, dim=0).float().item()
 
 
@@ -107,14 +111,16 @@ def compute_gae_advantage_return(token_level_rewards, values, eos_mask, gamma, l
     adv = torch.empty_like(rewards)
     ret = torch.empty_like(rewards)
     small = torch.empty(3 + 3 * batch, dtype=torch.float64, device=dev)     # info, then the rows' moments
+    # `gamma * lam` as python evaluates it inside the reference's `gamma * lam * lastgaelam`: in double
+    # for python floats (the config's values), in the tensors' own precision for 0-dim tensors
+    decays = float(gamma), float(gamma * lam)
     # whether the mask is empty is all that the host waits for: its rows' sums leave before the scan has ended (whole
     # numbers, so their sum has no order)
     slot = _lib.HostWords.take(dev, 8 * batch) if batch > 0 and mask.dtype is not torch.float32 else None
-    # `gamma * lam` as python evaluates it inside the reference's `gamma * lam * lastgaelam`: in double
-    # for python floats (the config's values), in the tensors' own precision for 0-dim tensors
-    _lib.call("mrl_gae_whiten_host", _lib.ptr(rewards), _lib.ptr(vals), _lib.ptr(mask), _lib.dtype_code(mask), batch, width,
-              float(gamma), float(gamma * lam), _lib.ptr(adv), _lib.ptr(ret), small.data_ptr(),
-              slot.addr if slot is not None else None, small.data_ptr() + 24, 24 * batch, _lib.stream(dev))
+    launch = _lib.call if slot is None else slot.launch
+    launch("mrl_gae_whiten_host", _lib.ptr(rewards), _lib.ptr(vals), _lib.ptr(mask), _lib.dtype_code(mask), batch, width,
+           *decays, _lib.ptr(adv), _lib.ptr(ret), small.data_ptr(), slot.addr if slot is not None else None,
+           small.data_ptr() + 24, 24 * batch, _lib.stream(dev))
     count = sum(slot.read(ctypes.c_double, batch, _lib.stream(dev))) if slot is not None else small[0].item()
     if count == 0:
         raise ValueError("At least one element in the mask has to be 1.")
@@ -174,15 +180,17 @@ class _CriticLoss(torch.autograd.Function):
         slope = torch.empty_like(ret)
         ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(batch)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        clip, loss_scale = float(clip), float(loss_scale)
         slot = _lib.HostWords.take(dev, 16) if sent is not None else None
-        _lib.call("mrl_critic_loss_fwd_slope_host", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
-                  _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, float(clip), float(loss_scale),
-                  _lib.ptr(slope), _lib.ptr(out), _lib.ptr(loss), slot.addr if slot is not None else None,
-                  _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
+        launch = _lib.call if slot is None else slot.launch
+        launch("mrl_critic_loss_fwd_slope_host", _lib.ptr(head), batch, padded, _lib.ptr(prompt), _lib.dtype_code(prompt),
+               _lib.ptr(lens), _lib.dtype_code(lens), _lib.ptr(ret), _lib.ptr(val), width, clip, loss_scale,
+               _lib.ptr(slope), _lib.ptr(out), _lib.ptr(loss), slot.addr if slot is not None else None,
+               _lib.ptr(workspace), ws_bytes, _lib.stream(dev))
         if slot is not None:
             sent.append(slot)
         ctx.save_for_backward(slope, prompt, lens, out)
-        ctx.meta = (tuple(head.shape), float(loss_scale))
+        ctx.meta = (tuple(head.shape), loss_scale)
         ctx.mark_non_differentiable(out)
         ctx.set_materialize_grads(False)
         return loss, out

@@ -93,14 +93,15 @@ def _lay_out(columns):
     what the copy takes."""
     batches = []
     for dev, part in _by_device(columns):
+        args = (_lib.RaggedColumn * len(part))()
+        for c in part:
+            c.cu = torch.empty(c.lengths.numel() + 1, dtype=torch.int32, device=dev)
         slot = _lib.HostWords.take(dev, 16 * len(part))
         info = None if slot is not None else torch.empty((len(part), 2), dtype=torch.int64, device=dev)
-        p_info = slot.addr if slot is not None else info.data_ptr()
-        args = (_lib.RaggedColumn * len(part))()
+        launch, p_info = (_lib.call, info.data_ptr()) if slot is None else (slot.launch, slot.addr)
         for i, c in enumerate(part):
-            c.cu = torch.empty(c.lengths.numel() + 1, dtype=torch.int32, device=dev)
             c.fill(args[i], p_info + 16 * i)
-        _lib.call("mrl_ragged_layouts", args, len(part), _lib.stream(dev))
+        launch("mrl_ragged_layouts", args, len(part), _lib.stream(dev))
         sizes = slot.read(ctypes.c_int64, 2 * len(part), _lib.stream(dev)) if slot is not None else info.view(-1).tolist()
         for i, c in enumerate(part):
             c.total, c.longest = sizes[2 * i:2 * i + 2]

@@ -4300,3 +4300,38 @@ def test_fused_sweep_threads_far_below_the_maximum(dev, dtype, vocab, threads, v
     tiny = 2.0 ** -24 if dtype is torch.float16 else 0.0
     bound = (want.abs() * (unit + 2e-5) + 2e-5 * p) * inv_t / n + tiny + 1e-12
     assert ((g[0, :n].double() - want * inv_t / n).abs() <= bound).all()
+
+
+def test_slots_of_host_memory_are_kept(dev, monkeypatch):
+    """A call that is refused gives its slot back; one that nobody reads is lost, but its memory stays allocated and is
+    not handed out again; and where there are no more, results are copied."""
+    words = _lib.HostWords
+    monkeypatch.setattr(words, "_free", {})
+    monkeypatch.setattr(words, "_blocks", [])
+    none, lens, ids = torch.zeros(2, 0, device=dev), torch.ones(2, 1, dtype=torch.int32, device=dev), torch.ones(2, 5, dtype=torch.int64, device=dev)
+    critic = mrl.LossFuncFactory.get_instance("ray_ppo", "critic")
+    empty = {"responses": none, "response_length": lens, "prompt_length": lens, "values": none, "returns": none}
+    for _ in range(2 * words._BLOCK):
+        for call in (lambda: mrl.kl_token_level_rewards(none, none, lens, torch.zeros(2, device=dev), 0.1),
+                     lambda: mrl.compute_gae_advantage_return(none, none, ids[:, :0], 1.0, 0.95),
+                     lambda: mrl.preprocess_packed_seqs(ids, ids, ids, 0),
+                     lambda: mrl.unpack_pad_experience({"a": ids.view(-1)}, {"a": lens}, 0, 0),
+                     lambda: critic.compute_loss(torch.zeros(2, 4, 1, device=dev).requires_grad_(), empty)):
+            with pytest.raises(_lib.MrlError):
+                call()
+    assert [len(words._free[dev.index]), len(words._blocks)] == [words._BLOCK, 1]
+    lost, cu = words.take(dev, 8), torch.empty(3, dtype=torch.int32, device=dev)
+    lost.launch("mrl_pack_index_build", ids.data_ptr(), _lib.I64, 2, 5, 1, lens.data_ptr(), cu.data_ptr(), lost.addr,
+                _lib.stream(dev))
+    addr = lost.addr
+    del lost
+    taken = [words.take(dev, 8) for _ in range(words._BLOCK)]           # one more than are left
+    assert len(words._blocks) == 2 and addr not in [s.addr for s in taken]
+    first = words._blocks[0]
+    assert first.data_ptr() <= addr < first.data_ptr() + first.numel() * 4
+    torch.cuda.synchronize()
+    assert first.view(-1)[(addr - first.data_ptr()) // 4:][:2].view(torch.int64).item() == 10
+    monkeypatch.setattr(words, "_free", {})
+    monkeypatch.setattr(words, "_MOST_BLOCKS", 2)
+    assert words.take(dev, 8) is None and len(words._blocks) == 2
+    assert mrl.preprocess_packed_seqs(ids, ids, ids, 4)[0].shape == (1, 16)
