@@ -76,9 +76,13 @@ def _flat_labels(labels):
     return lab.contiguous()
 
 
+# torch says so under private names only; without them every pass goes by way of the autograd function
+_functorch_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: True)
+
+
 def _transformed():
     """True under a function transform or a forward-mode level, which an autograd function has to see (and refuses)."""
-    return torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0
+    return _functorch_active() or getattr(forward_ad, "_current_level", 0) >= 0
 
 
 def score_windows(logits, labels, windows, inv_temperature, want_entropy):

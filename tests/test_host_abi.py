@@ -336,3 +336,24 @@ def test_deferred_stats_behaves_like_the_dict_of_floats_it_stands_for():
     assert dict(live) == want
     live._pending[1].mul_(2.0)
     assert live[STAT_KEYS[1]] == 4.0 and dict(live) == {k: 2.0 * v for k, v in want.items()}
+
+
+def test_transforms_are_seen_or_assumed(monkeypatch):
+    """Scoring passes leave the autograd function out unless a transform has to see it.  torch tells under private
+    names: one that lacks them must not break the passes, it only costs them the shorter way."""
+    import importlib.util
+    from torch.autograd import forward_ad
+    from mindspeed_rl_amd import vocab_ops
+    assert not vocab_ops._transformed()
+    with forward_ad.dual_level():
+        assert vocab_ops._transformed()
+    assert torch.func.vmap(lambda x: x * float(vocab_ops._transformed()))(torch.ones(2)).tolist() == [1.0, 1.0]
+    with monkeypatch.context() as m:
+        m.delattr(forward_ad, "_current_level")
+        assert vocab_ops._transformed()
+    with monkeypatch.context() as m:
+        m.delattr(torch._C, "_are_functorch_transforms_active")
+        spec = importlib.util.spec_from_file_location("mindspeed_rl_amd._vocab_ops_again", vocab_ops.__file__)
+        again = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(again)
+        assert again._transformed()
