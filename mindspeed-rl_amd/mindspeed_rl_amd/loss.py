@@ -388,6 +388,10 @@ class _FusedLogprobLoss(torch.autograd.Function):
             grad = _deliver_swept_grads(ctx, *saved, state, g_loss)
         else:
             (grad,) = _deliver_eager_grads(ctx, saved[:1], saved[1], state, g_loss)
+        # The saved tensor itself, not a view of it: over a retained graph autograd then copies it into a leaf's .grad,
+        # which may be added to, clipped or cleared without spoiling (and, by the version they would share,
+        # forbidding) the next backward.  That costs such a leaf one copy; a graph that ends here, or logits
+        # that a model made, take the tensor as it is.
         return grad if tuple(grad.shape) == shape else grad.view(shape), None, None, None
 
 

@@ -4335,3 +4335,38 @@ def test_slots_of_host_memory_are_kept(dev, monkeypatch):
     monkeypatch.setattr(words, "_MOST_BLOCKS", 2)
     assert words.take(dev, 8) is None and len(words._blocks) == 2
     assert mrl.preprocess_packed_seqs(ids, ids, ids, 4)[0].shape == (1, 16)
+
+
+@pytest.mark.parametrize("vocab", [1024, 2051])
+def test_leaf_gradients_over_a_retained_graph_may_be_changed(dev, vocab):
+    """The .grad of leaf logits shares nothing with what a retained graph keeps: it accumulates over any number of
+    backwards, and is scaled in place between them.  Where the graph ends, .grad is what the sweep wrote: no copy."""
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    rows = 400
+    z = torch.randn(1, rows, vocab, generator=gen, device=dev)
+    batch = {"labels": torch.randint(0, vocab, (1, rows), generator=gen, device=dev),
+             "responses": torch.zeros(1, rows - 1, dtype=torch.int64, device=dev), "response_length": torch.tensor([[rows - 1]], device=dev),
+             "prompt_length": torch.tensor([[1]], device=dev), "advantages": torch.randn(1, rows - 1, generator=gen, device=dev)}
+    ends = torch.tensor([0, rows], dtype=torch.int32, device=dev)
+
+    def graph():
+        leaf = z.clone().requires_grad_()
+        return leaf, mrl.fused_logprob_policy_loss(leaf, batch, packed=True, clip_low=0.2, clip_high=0.2, seqlens=ends[1:],
+                                                   cu_seqlens=ends)[0]
+
+    leaf, loss = graph()
+    (once,) = torch.autograd.grad(loss, leaf)
+    leaf, loss = graph()
+    for factor in (1.0, 2.0, 3.0):
+        loss.backward(retain_graph=True)
+        assert torch.equal(leaf.grad, once * factor)
+    leaf.grad.mul_(0.5)
+    loss.backward(retain_graph=True)
+    assert torch.equal(leaf.grad, once * 3.0 * 0.5 + once)          # as it was rounded
+    leaf, loss = graph()
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats(dev)
+    before = torch.cuda.memory_allocated(dev)
+    loss.backward()
+    assert torch.cuda.max_memory_allocated(dev) - before < z.numel()
+    assert torch.equal(leaf.grad, once)
