@@ -230,7 +230,10 @@ __global__ __launch_bounds__(kBlock) void window_cut_kernel(SeqWindows seqs, int
 // to; the cells without a row are zeroed here.  A workgroup per sequence: it adds up the counts of those in front of
 // it itself (kCellSeqs of them at most, out of L2), so that one launch does what flags, their count, their
 // positions, the spread of per-row results and the cut of both took six more for.  Bound by its launch; the gain is
-// theirs: a lm_head scoring pass of 1 944 rows x 42 384 x 1 344 239 -> 220 us.  More sequences keep the flags.
+// theirs: a lm_head scoring pass of 1 944 rows x 42 384 x 1 344 239 -> 220 us.  Every workgroup looks at every
+// sequence, so more of them cost their square: a pass over 8-token responses takes 45 us from 8 to 512 sequences, 46
+// at 1 024 and 50.5 at 2 048 (86 to 89 with the flags at all of these); from 4 096 on it would grow fourfold each
+// time, and more than 2 048 keep the flags.
 constexpr int64_t kCellSeqs = MRL_WINDOW_CELLS_SEQS;
 __global__ __launch_bounds__(kBlock) void window_cells_kernel(SeqWindows seqs, int batch, int64_t width, int64_t n_rows,
                                                               int32_t* __restrict__ live, int32_t* __restrict__ cell,

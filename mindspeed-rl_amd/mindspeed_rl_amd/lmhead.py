@@ -12,6 +12,13 @@ import torch
 
 from . import _lib, vocab_ops
 
+# Cells that a scoring pass's result may have beyond the rows for these to be found with their cells (score_windows):
+# the two tables of them take 8 bytes a cell, 32 MiB here, which a result of one long response among many short ones
+# would make twice the memory of a pass without gaining more than before.  us and MiB a pass, flagged rows / this
+# way, 64-wide hidden states: 64 x 4 096 cells 88, 2 / 46, 5; 2 048 x 2 048 87, 33 / 60, 69; 512 x 16 384 88, 64 / 52, 131;
+# 1 024 x 32 768 150, 257 / 90, 519.
+_EXTRA_CELLS = 1 << 22
+
 # (name, start, end, rows) appended per call when set to a list, like vocab_ops.kernel_events
 kernel_events = None
 
@@ -93,7 +100,8 @@ def score_windows(hidden, weight, labels, windows, inv_temperature, want_entropy
         return None
     if not (0 < windows.n_seq <= windows.MAX_CELL_SEQS and windows.width > 0 and windows.n_rows > 0):
         return None
-    if windows.n_seq * windows.width > 0x7fffffff or vocab_ops._transformed():
+    cells = windows.n_seq * windows.width
+    if cells > windows.n_rows + _EXTRA_CELLS or cells > 0x7fffffff or vocab_ops._transformed():
         return None
     dev = _lib.require_device(hidden, weight, labels, windows.prompt)
     found = windows.cells(want_entropy)

@@ -4370,3 +4370,36 @@ def test_leaf_gradients_over_a_retained_graph_may_be_changed(dev, vocab):
     loss.backward()
     assert torch.cuda.max_memory_allocated(dev) - before < z.numel()
     assert torch.equal(leaf.grad, once)
+
+
+def test_scoring_results_much_larger_than_the_rows(dev, monkeypatch):
+    """One long response among many short ones: rows are not looked for cell by cell where the tables of them would be
+    as large as the result; the result is the same either way, and so is the line between the two."""
+    from mindspeed_rl_amd import lmhead
+    gen = torch.Generator(device=dev).manual_seed(4)
+    n_seq, width = 2048, 4096
+    rlen = torch.full((n_seq, 1), 2, dtype=torch.int32, device=dev)
+    rlen[7] = width
+    plen = torch.ones_like(rlen)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int32, device=dev), torch.cumsum((rlen + plen).view(-1), 0).to(torch.int32)])
+    rows = int(cu[-1])
+    hidden = torch.randn(1, rows, 64, generator=gen, device=dev).to(torch.bfloat16)
+    weight = torch.randn(256, 64, generator=gen, device=dev).to(torch.bfloat16)
+    batch = {"responses": torch.zeros(1, 1, dtype=torch.int64, device=dev).expand(n_seq, width), "prompt_length": plen,
+             "response_length": rlen, "labels": torch.randint(0, 256, (1, rows), generator=gen, device=dev)}
+    kw = dict(use_remove_padding=True, seqlens_in_batch=(rlen + plen).view(-1), cu_seqlens_padded=cu, seq_len=width + 1)
+    comp, found = mrl.StandardLogProbComputer(), []
+    real = mrl.packing.ResponseWindows.cells
+    monkeypatch.setattr(mrl.packing.ResponseWindows, "cells", lambda *a: found.append(1) or real(*a))
+    results, outputs, more = [], 8 * n_seq * width, n_seq * width - rows
+    for extra, by_cells in ((lmhead._EXTRA_CELLS, False), (more, True), (more - 1, False)):
+        monkeypatch.setattr(lmhead, "_EXTRA_CELLS", extra)
+        found.clear()
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats(dev)
+        before = torch.cuda.memory_allocated(dev)
+        results.append(comp.compute(hidden, batch, False, lm_head_weight=weight, **kw))
+        peak = torch.cuda.max_memory_allocated(dev) - before
+        assert found == [1] * by_cells and (peak < outputs + (8 << 20)) is not by_cells
+    for a in results[1:]:
+        assert torch.equal(a[0], results[0][0]) and torch.equal(a[1], results[0][1]) and a[0].any().item()
