@@ -193,10 +193,11 @@ __global__ __launch_bounds__(kBlock) void window_gather_kernel(const T* __restri
     out[e] = v;
 }
 
-// The two index maps of a scoring pass.  Both are bound by their launches (2 to 4 us each): written with torch's
-// element-wise ops they were 24 launches around a sweep of 11 us (1 208 padded rows x 32 000 bf16: 233 us a
-// pass, now 55), so the flags take a clear and a scatter, and both results are cut by one gather.
-//
+// The two index maps of a pass over flagged rows: one with gradients, or one that the two shorter ways of a scoring
+// pass (mrl_window_logprob; window_cells_kernel below) do not take.  Both are bound by their launches (2 to 4 us
+// each): written with torch's element-wise ops they were 24 launches around a sweep of 11 us (1 208 padded rows x
+// 32 000 bf16: 233 us a pass, 55 with these, 18 in one launch), so the flags take a clear and a scatter, and both
+// results are cut by one gather.
 //
 // active[t] = 1 for the rows of the windows, at most `width` of each (active is zero before).  A workgroup per
 // sequence; windows may overlap, everyone writes the same.

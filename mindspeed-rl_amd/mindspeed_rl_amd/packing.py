@@ -16,12 +16,8 @@ from . import _lib, vocab_ops
 
 
 def _as_index(t):
-    if (t.dtype is torch.int64 or t.dtype is torch.int32) and t.is_contiguous():
-        return t
-    """int32 / int64 tensor, flattened and dense, for a [B] or [B,1] length column."""
-    if t.dtype not in (torch.int32, torch.int64):
-        t = t.to(torch.int64)
-    return t.reshape(-1).contiguous()
+    """A ``[B]`` or ``[B, 1]`` length column as a dense int32 / int64 tensor, in its shape if it was dense already."""
+    return _lib.index_column(t, t.device)
 
 
 def generate_mask(data_pad, seq_lengths):
