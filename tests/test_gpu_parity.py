@@ -5,6 +5,7 @@ Tolerances (fp32 accumulate against the oracle's fp32 up-cast): index maps, mask
 assignment bit-exact; logp / entropy / advantages 1e-3 abs; loss 1e-4 rel; dlogits 2e-3 abs.
 The observed errors are far smaller; tighter bounds are asserted where the arithmetic allows.
 """
+import ctypes
 import math
 import os
 import random
@@ -4179,6 +4180,8 @@ def test_scoring_pass_from_hidden_states_cell_by_cell(dev, monkeypatch, layout, 
     vocab, hdim, kw = 520, 64, {}
     p0, r0 = [0, 1, 7, 3, 40, 4, 9], [38, 5, 0, 50, 3, 60, 31]
     comp = mrl.StandardLogProbComputer()
+    by_cells, real = [], lmhead.score_windows
+    monkeypatch.setattr(lmhead, "score_windows", lambda *x: (by_cells.append(real(*x)), by_cells[-1])[1])
     for repeat, empty in ((1, False), (43, False), (1, True)):
         plen = torch.tensor(p0 * repeat, dtype=index).view(-1, 1)
         rlen = torch.tensor(r0 * repeat, dtype=index).view(-1, 1) * (0 if empty else 1)
@@ -4198,6 +4201,7 @@ def test_scoring_pass_from_hidden_states_cell_by_cell(dev, monkeypatch, layout, 
             for out in (wide[..., :hdim].contiguous(), wide[..., :hdim]):
                 for skip in (False, True):
                     got = comp.compute(out, b, skip, inv_temperature=1.25, lm_head_weight=weight, **kw)
+                    assert len(by_cells) == 1 and by_cells.pop() is not None
                     with monkeypatch.context() as m:
                         m.setattr(lmhead, "score_windows", lambda *a: None)
                         want = comp.compute(out, b, skip, inv_temperature=1.25, lm_head_weight=weight, **kw)
@@ -4403,3 +4407,52 @@ def test_scoring_results_much_larger_than_the_rows(dev, monkeypatch):
         assert found == [1] * by_cells and (peak < outputs + (8 << 20)) is not by_cells
     for a in results[1:]:
         assert torch.equal(a[0], results[0][0]) and torch.equal(a[1], results[0][1]) and a[0].any().item()
+
+
+@pytest.mark.parametrize("counter", [True, False])
+def test_entry_points_without_host_memory(dev, counter):
+    """The loss's reduce step, GAE with whitening and the critic's forward as callers have them who read no host
+    memory: the same bits as the forms that the package uses, whose host memory holds what the device has."""
+    gen = torch.Generator(device=dev).manual_seed(8)
+    n, width, padded = 5, 300, 340
+    f32 = dict(dtype=torch.float32, device=dev)
+    old, ref, adv, val = torch.randn(4, n, width, generator=gen, device=dev).unbind(0)
+    lens = torch.tensor([[300], [1], [0], [250], [77]], dtype=torch.int32, device=dev)
+    prompt = torch.full_like(lens, 20)
+    mask, stream = mrl.generate_mask(old, lens), _lib.stream(dev)
+    terms = torch.randn(n * padded, 8, generator=gen, device=dev)
+    start = torch.arange(n, dtype=torch.int64, device=dev) * padded + 19
+    count = torch.tensor([300, 0, 0, 200, 77], dtype=torch.int32, device=dev)
+    head = torch.randn(n, padded, generator=gen, device=dev)
+    outputs, sent = [], []
+    for host in (False, True):
+        slots = [_lib.HostWords.take(dev, b) for b in (32, 8 * n, 16)] if host else [None] * 3
+        calls = [s.launch if host else _lib.call for s in slots]
+        to = [[s.addr] if host else [] for s in slots]
+        tail = "_host" if host else ""
+        sums, out, loss = torch.zeros(n, 8, **f32), torch.empty(8, **f32), torch.empty(1, **f32)
+        done = torch.zeros(1, dtype=torch.int32, device=dev)
+        calls[0]("mrl_fused_loss_reduce" + tail, terms.data_ptr(), start.data_ptr(), count.data_ptr(), n, width, old.data_ptr(),
+                 ref.data_ptr(), adv.data_ptr(), None, _lib.F32, lens.data_ptr(), _lib.I32, 0.8, 1.2,
+                 _lib.KL_BY_NAME["low_var_kl"], 0.1, 0.01, 0, 0.5, sums.data_ptr(), out.data_ptr(),
+                 done.data_ptr() if counter else None, loss.data_ptr(), *to[0], stream)
+        info, work = torch.empty(3, dtype=torch.float64, device=dev), torch.empty(24 * n, dtype=torch.uint8, device=dev)
+        white, ret = torch.empty_like(old), torch.empty_like(old)
+        calls[1]("mrl_gae_whiten" + tail, old.data_ptr(), val.data_ptr(), mask.data_ptr(), _lib.I64, n, width, 1.0, 0.95,
+                 white.data_ptr(), ret.data_ptr(), info.data_ptr(), *to[1], work.data_ptr(), 24 * n, stream)
+        slope, stats, critic = torch.empty_like(old), torch.empty(4, **f32), torch.empty(1, **f32)
+        ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(n)
+        scratch = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        calls[2]("mrl_critic_loss_fwd_slope" + tail, head.data_ptr(), n, padded, prompt.data_ptr(), _lib.I32, lens.data_ptr(),
+                 _lib.I32, ref.data_ptr(), val.data_ptr(), width, 0.5, 0.25, slope.data_ptr(), stats.data_ptr(),
+                 critic.data_ptr(), *to[2], scratch.data_ptr(), ws_bytes, stream)
+        outputs.append([sums, out, loss, done, white, ret, info, slope, stats, critic])
+        if host:
+            sent = [slots[0].read_doubles_of(8, stream), torch.tensor(slots[1].read(ctypes.c_double, n, stream), dtype=torch.float64),
+                    slots[2].read_doubles_of(4, stream)]
+    for a, b in zip(*outputs):
+        assert torch.equal(a, b) and torch.isfinite(a.double()).all()
+    sums, out, loss, done, white, ret, info, slope, stats, critic = outputs[0]
+    assert torch.equal(sent[0], out.cpu().double()) and out[0] == loss and not done.any()
+    assert torch.equal(sent[1], mask.sum(1).cpu().double()) and info[0].item() == mask.sum().item()
+    assert torch.equal(sent[2], stats.cpu().double()) and stats[0] == critic and stats[3].item() == mask.sum().item()
