@@ -4440,7 +4440,7 @@ def test_entry_points_without_host_memory(dev, counter):
         white, ret = torch.empty_like(old), torch.empty_like(old)
         calls[1]("mrl_gae_whiten" + tail, old.data_ptr(), val.data_ptr(), mask.data_ptr(), _lib.I64, n, width, 1.0, 0.95,
                  white.data_ptr(), ret.data_ptr(), info.data_ptr(), *to[1], work.data_ptr(), 24 * n, stream)
-        slope, stats, critic = torch.empty_like(old), torch.empty(4, **f32), torch.empty(1, **f32)
+        slope, stats, critic = torch.zeros_like(old), torch.empty(4, **f32), torch.empty(1, **f32)
         ws_bytes = _lib.load().mrl_value_loss_workspace_bytes(n)
         scratch = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         calls[2]("mrl_critic_loss_fwd_slope" + tail, head.data_ptr(), n, padded, prompt.data_ptr(), _lib.I32, lens.data_ptr(),
