@@ -52,6 +52,9 @@ struct SeqWindows {
 inline int check_seq_windows(const char* fn, const SeqWindows& q, int64_t batch, int64_t width, int64_t n_rows) {
     MRL_REQUIRE(batch >= 0 && batch <= (1LL << 20) && width >= 0 && n_rows >= 0, MRL_ERR_INVALID_ARG,
                 "%s: batch=%lld width=%lld n_rows=%lld", fn, (long long)batch, (long long)width, (long long)n_rows);
+    // callers multiply the two
+    MRL_REQUIRE(batch == 0 || width <= 0x7fffffffffffffffLL / batch, MRL_ERR_UNSUPPORTED, "%s: batch=%lld x width=%lld out of range",
+                fn, (long long)batch, (long long)width);
     MRL_REQUIRE(int_dtype_bytes(q.prompt_dtype) != 0 && (q.packed || int_dtype_bytes(q.resp_dtype) != 0),
                 MRL_ERR_UNSUPPORTED, "%s: length dtypes %d and %d (want I32 or I64)", fn, q.prompt_dtype, q.resp_dtype);
     MRL_REQUIRE(batch == 0 || (q.prompt && (q.packed ? q.seqlens && q.cu : q.resp && q.padded_s >= 0)), MRL_ERR_INVALID_ARG,

@@ -175,6 +175,25 @@ def test_argument_validation_launches_nothing():
     assert lib.mrl_masked_whiten(p, p, _lib.F32, 8, 1, p, None, None) == -1
     assert lib.mrl_value_loss_fwd(p, p, p, None, 0, None, 0, 2, 4, 0.5, 1.0, p, None) == -1  # no mask, no lengths
     assert lib.mrl_value_loss_bwd(p, p, p, p, _lib.F32, None, 0, 2, 4, 0.5, 1.0, p, None, p, None) == -1
+    # response windows: sizes whose product leaves the 64 bits, more sequences than one launch looks through, outputs
+    windows = (p, p, 0, p, _lib.I32, p, _lib.I32)
+    score = (p, _lib.BF16, 4, 128, 128, p, _lib.I64, 1.0, 0)
+    for width in (1 << 60, 1 << 31):
+        assert lib.mrl_window_cells(0, 16, width, 4, *windows, 1, p, p, p, p, p, None) == -2
+        assert lib.mrl_window_logprob(*score, 16, width, *windows, 1, p, p, None) == -2
+    assert lib.mrl_window_cut(0, 16, 1 << 60, 4, *windows, p, p, p, p, None) == -2
+    assert lib.mrl_window_rows(0, 16, 1 << 60, 4, *windows, p, None) == -2
+    assert lib.mrl_window_cells(0, 2049, 8, 4, *windows, 1, p, p, p, p, p, None) == -2
+    assert lib.mrl_window_cells(0, 2, 8, 0, *windows, 1, p, p, p, p, p, None) == -1          # nothing to find
+    assert lib.mrl_window_cells(0, 2, 8, 4, *windows, 1, p, p, p + 4, p, p, None) == -3      # total
+    assert lib.mrl_window_cells(0, 2, 8, 4, *windows, 1, p, p, p, p, None, None) == -1
+    assert lib.mrl_window_logprob(*score, 2, 8, *windows, 1, p, None, None) == -1
+    assert lib.mrl_window_logprob(*score, 0, 8, *windows, 1, None, None, None) == 0
+    assert lib.mrl_lmhead_logprob_fwd_cells(p, p, 4, 1000, 128, p, _lib.I64, 1.0, None, p, None, p, 1 << 20, None) == -1
+    # results in host memory: alignment, and the wait for words that are there already
+    assert lib.mrl_gae_whiten_host(p, p, p, _lib.I64, 2, 8, 1.0, 0.95, p, p, p, p + 4, p, 48, None) == -3
+    assert lib.mrl_host_wait(p, 4, None) == 0 and lib.mrl_host_wait(None, 0, None) == 0
+    assert lib.mrl_host_wait(p, -1, None) == -1 and lib.mrl_host_wait(None, 1, None) == -1
     # bandwidth probe
     assert lib.mrl_bandwidth_probe(6, p, p, 1, 1024, None) == -1
     assert lib.mrl_bandwidth_probe(2, p, p, 1, 1000, None) == -1
