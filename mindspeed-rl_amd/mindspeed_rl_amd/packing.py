@@ -17,6 +17,8 @@ from . import _lib, vocab_ops
 
 def _as_index(t):
     """A ``[B]`` or ``[B, 1]`` length column as a dense int32 / int64 tensor, in its shape if it was dense already."""
+    if (t.dtype is torch.int64 or t.dtype is torch.int32) and t.is_contiguous():
+        return t
     return _lib.index_column(t, t.device)
 
 
