@@ -543,7 +543,7 @@ int mrl_lmhead_logprob_fwd_cells(const void* hidden, const void* weight, int64_t
                                  void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------------
- * Training step from the hidden states (configs "fused lm_head"): the three matrix products around
+ * Training step from the hidden states (fused lm_head): the three matrix products around
  * the fused sweep, hand-written for the bf16 matrix cores (same tile loop as the forward above).
  * The reference has no counterpart: its model materialises all [T, V] logits
  * (models/base/base_training_engine.py:221-258) and autograd runs the two backward products of the

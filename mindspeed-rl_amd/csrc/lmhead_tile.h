@@ -22,8 +22,9 @@
 // a k-contiguous A has a third one (its bytes lie a whole k-step ahead), and a k-major operand is requested by
 // halves of a k-step (32 k-rows, still whole 128-byte lines; halves of a k-contiguous operand would be half
 // lines, which measured 10 % slower).  With two buffers and all 16 requests in every other sub-step, before ->
-// now, ms (12 356 x 152 064 x 3 584; 4 000 x 129 280 x 5 120): logits 9.57 -> 9.27, 3.81 -> 3.66; dHidden of whole
-// tiles 10.88 -> 10.45, 3.37 -> 2.93; dWeight 10.56 -> 10.02, 4.11 -> 3.92; fused forward 9.37 -> 9.40, 3.87 -> 3.72.
+// now, ms (12 356 x 152 064 x 3 584; 4 000 x 129 280 x 5 120; medians of 12 steps in turn on one board): logits 9.58 ->
+// 9.33, 3.86 -> 3.72; dWeight 10.41 -> 9.92, 4.05 -> 3.97; dHidden 10.76 -> 9.70, 4.41 -> 3.73, of which its whole tiles at
+// the second size 3.32 -> 2.93 (the rest are cut, see plan_split); fused forward 9.37 -> 9.31, 3.87 -> 3.75.
 #pragma once
 
 #include "mrl_internal.h"

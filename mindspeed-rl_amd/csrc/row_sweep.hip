@@ -244,7 +244,9 @@ __device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int 
 // more powers of two under the largest one is scaled by a flushed zero, and with it goes up to 2^90 x
 // 2^-126 of the row's weight (which is 1 at least) a thread: 2^-26 from all 1024 threads, below half
 // an ulp.  (With 2^120 it was up to 2^-6 a thread: a logsumexp of 0.003 for 1.336.)  Sums of 1024
-// threads against one reference stay below 2^100.
+// threads against one reference stay below 2^100.  What it costs: rows that climb by 62 to 83, us a
+// sweep, 430 -> 447 (4 096 x 152 064 bf16), 175 -> 179 (4 096 x 32 000 fp32), 185 -> 216 (8 192 x 32 000
+// bf16), as rows that climb further always did; the others are as before.
 constexpr float kSumLimit = 1.2379400392853803e27f;     // 2^90
 
 template <int DT, bool kEntropy>
