@@ -176,8 +176,21 @@ __device__ __forceinline__ Stats block_reduce(Stats st, float k, Stats* lds) {
     if ((threadIdx.x & 63) == 0) lds[wave] = st;
     __syncthreads();
     Stats r = lds[0];
+    if (kWaves <= 4) {
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) r = merge<kEntropy>(r, lds[w], k);
+        for (int w = 1; w < kWaves; ++w) r = merge<kEntropy>(r, lds[w], k);
+        return r;
+    }
+    // more partials: the largest reference first, so that no exponential waits for the one before
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) r.m = fmaxf(r.m, lds[w].m);
+    r.s = r.u = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const float f = fast_exp2((lds[w].m - r.m) * k);
+        r.s = __builtin_fmaf(lds[w].s, f, r.s);
+        if (kEntropy) r.u = __builtin_fmaf(lds[w].u, f, r.u);
+    }
     return r;
 }
 

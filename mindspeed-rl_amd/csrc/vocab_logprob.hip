@@ -1,13 +1,14 @@
 // Streaming vocabulary sweeps for gfx950: per-row log-softmax gather + entropy + logsumexp
 // (forward, one read of the logits) and the fused dlogits (backward, one read + one write).
 //
-// Mapping: one workgroup of 256 threads (4 wavefronts) per token row.  A row is addressed as
+// Mapping: one workgroup per token row, 256 threads (4 wavefronts) in the backward, 256 to 1024 by the row's
+// length in the forward.  A row is addressed as
 // a run of 16-byte vectors from its first 128-byte line on; elements in front of it and after the last
 // vector (only present for odd vocab sizes or strides) are handled with scalar loads by the first lanes.
 // Each thread keeps an online (max, sum exp, sum exp*z) triple in fp32; a rescale happens at
-// most once per group of kUnroll vectors and only when the running maximum grows, so the steady
+// most once per round of vectors and only when the running maximum grows, so the steady
 // state costs one convert, one FMA and one v_exp_f32 per element.  Wavefront reduction uses
-// cross-lane shuffles, the four wavefronts combine through LDS.
+// cross-lane shuffles, the wavefronts combine through LDS.
 #include <stdlib.h>
 
 #include "mrl_internal.h"
@@ -26,7 +27,6 @@ using namespace mrl_vocab;
 #define MRL_VOCAB_UNROLL 4
 #endif
 constexpr int kBlock = MRL_VOCAB_BLOCK;
-constexpr int kWaves = kBlock / 64;
 constexpr int kUnroll = MRL_VOCAB_UNROLL;
 // Splits a row of `vocab` elements starting at `row` into head scalars up to a 128-byte line (with vectors
 // that are 16-byte aligned only, every wavefront's 1 KiB cuts two lines in half: 129 281 bf16 logits forward
@@ -72,15 +72,15 @@ struct WindowCells {
     }
 };
 
-template <int DT, typename LabelT, bool kEntropy, typename Rows>
-__global__ __launch_bounds__(kBlock) void vocab_fwd_kernel(
+template <int DT, typename LabelT, bool kEntropy, int kBlk, int kDeep, typename Rows>
+__global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
     const typename Elem<DT>::T* __restrict__ logits, int64_t row_stride, int vocab,
     const LabelT* __restrict__ labels, Rows rows, float inv_t,
     float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int kVec = E::kVec;
-    __shared__ Stats lds[kWaves];
+    __shared__ Stats lds[kBlk / 64];
 
     const int64_t out = blockIdx.x, r = rows.row(out);
     if (r < 0) {
@@ -106,17 +106,16 @@ __global__ __launch_bounds__(kBlock) void vocab_fwd_kernel(
     Stats st = {kMaxInit, 0.f, 0.f};
     const int tid = threadIdx.x;
 
-    // full groups of kUnroll vectors per thread: all loads issued before any use
-    const int group = kBlock * kUnroll;
-    const int n_full = (sp.n_vec / group) * group;
-    for (int base = 0; base < n_full; base += group) {
-        u32x4 v[kUnroll];
+    // rounds of kDeep vectors a thread, all requested before any is used
+    const int n_full = sp.n_vec / (kBlk * kDeep) * (kBlk * kDeep);
+    for (int base = 0; base < n_full; base += kBlk * kDeep) {
+        u32x4 v[kDeep];
 #pragma unroll
-        for (int q = 0; q < kUnroll; ++q) v[q] = __builtin_nontemporal_load(vec + base + q * kBlock + tid);
-        float z[kUnroll][kVec];
+        for (int q = 0; q < kDeep; ++q) v[q] = __builtin_nontemporal_load(vec + base + q * kBlk + tid);
+        float z[kDeep][kVec];
         float vmax = st.m;
 #pragma unroll
-        for (int q = 0; q < kUnroll; ++q) {
+        for (int q = 0; q < kDeep; ++q) {
             E::unpack(v[q], z[q]);
 #pragma unroll
             for (int i = 0; i < kVec; ++i) vmax = fmaxf(vmax, z[q][i]);
@@ -124,23 +123,31 @@ __global__ __launch_bounds__(kBlock) void vocab_fwd_kernel(
         grow_max<kEntropy>(st, vmax, k);
         const float mk = st.m * k;
 #pragma unroll
-        for (int q = 0; q < kUnroll; ++q) {
+        for (int q = 0; q < kDeep; ++q) {
 #pragma unroll
             for (int i = 0; i < kVec; ++i) add_one<kEntropy>(st, z[q][i], k, mk);
         }
     }
-    // remaining whole vectors
-    for (int idx = n_full + tid; idx < sp.n_vec; idx += kBlock) {
-        const u32x4 v = __builtin_nontemporal_load(vec + idx);
-        float z[kVec];
-        E::unpack(v, z);
-        float vmax = st.m;
+    // the last round, in which a thread may have fewer: requested together as well, range-checked
+    if (n_full < sp.n_vec) {
+        const mrl::rsrc_t rest = mrl::make_rsrc(vec + n_full, (uint32_t)(sp.n_vec - n_full) * 16u);
+        u32x4 v[kDeep];
 #pragma unroll
-        for (int i = 0; i < kVec; ++i) vmax = fmaxf(vmax, z[i]);
-        grow_max<kEntropy>(st, vmax, k);
-        const float mk = st.m * k;
+        for (int q = 0; q < kDeep; ++q) v[q] = mrl::buf_load_nt(rest, (uint32_t)(q * kBlk + tid) * 16u);
 #pragma unroll
-        for (int i = 0; i < kVec; ++i) add_one<kEntropy>(st, z[i], k, mk);
+        for (int q = 0; q < kDeep; ++q) {
+            if (n_full + q * kBlk + tid < sp.n_vec) {
+                float z[kVec];
+                E::unpack(v[q], z);
+                float vmax = st.m;
+#pragma unroll
+                for (int i = 0; i < kVec; ++i) vmax = fmaxf(vmax, z[i]);
+                grow_max<kEntropy>(st, vmax, k);
+                const float mk = st.m * k;
+#pragma unroll
+                for (int i = 0; i < kVec; ++i) add_one<kEntropy>(st, z[i], k, mk);
+            }
+        }
     }
     // head and tail scalars (absent when the row starts on a line and vocab % kVec == 0)
     {
@@ -153,7 +160,7 @@ __global__ __launch_bounds__(kBlock) void vocab_fwd_kernel(
         }
     }
 
-    const Stats tot = block_reduce<kEntropy, kWaves>(st, k, lds);
+    const Stats tot = block_reduce<kEntropy, kBlk / 64>(st, k, lds);
     if (tid == 0) {
         // natural-log units of z' = z * inv_t
         const float lse = (tot.m * k + fast_log2(tot.s)) * kLn2;
@@ -324,17 +331,36 @@ struct FwdArgs {
     hipStream_t stream;
 };
 
-template <int DT, typename LabelT, typename Rows>
-int launch_fwd(const char* fn, const FwdArgs& a, const Rows& rows) {
+template <int DT, typename LabelT, int kBlk, int kDeep, typename Rows>
+int launch_fwd_shape(const char* fn, const FwdArgs& a, const Rows& rows) {
     using T = typename Elem<DT>::T;
-    const dim3 grid((unsigned)a.n_out), block(kBlock);
+    const dim3 grid((unsigned)a.n_out), block(kBlk);
 #define MRL_FWD_LAUNCH(ENT)                                                                                           \
-    hipLaunchKernelGGL((vocab_fwd_kernel<DT, LabelT, ENT, Rows>), grid, block, 0, a.stream, (const T*)a.logits,       \
-                       a.row_stride, (int)a.vocab, (const LabelT*)a.labels, rows, a.inv_t, a.logp, a.entropy, a.lse)
+    hipLaunchKernelGGL((vocab_fwd_kernel<DT, LabelT, ENT, kBlk, kDeep, Rows>), grid, block, 0, a.stream,              \
+                       (const T*)a.logits, a.row_stride, (int)a.vocab, (const LabelT*)a.labels, rows, a.inv_t, a.logp, \
+                       a.entropy, a.lse)
     if (a.with_entropy) MRL_FWD_LAUNCH(true);
     else MRL_FWD_LAUNCH(false);
 #undef MRL_FWD_LAUNCH
     return mrl::check_launch(fn);
+}
+
+// Threads of a row's workgroup and vectors a thread and round, by the row's length alone, so that a row's result
+// does not depend on how many rows there are.  Many rows are bound by memory whatever the shape (within 3 %); few
+// of them, a workgroup to a CU or less, by the rounds that a thread waits for one after the other, which more threads
+// make fewer of, up to where most of a workgroup has nothing to load.  us a pass, 256 x 4 for all rows -> now:
+// 98 x 152 064 bf16 20.2 -> 12.4, 116 x 129 280 18.0 -> 11.9, 49 x 152 064 fp32 29.5 -> 15.6; 2 GB of rows of
+// 152 064 bf16 293 -> 286, 63 712 299 -> 286, 32 000 294 -> 288.
+// The lines: 2 GB of rows of 3 750 vectors (30 000 bf16) 291 with 256 threads and 281 with 512, of 3 250 287 and
+// 298; of 4 096 fp32 vectors 286 and 290; of 6 500 284 with 512 and 285 with 1024, of 7 964 290 and 286.  Rows of 512
+// vectors and less would gain from a wavefront each (4 000 bf16 458 -> 324), but entropies of merged vocabulary
+// shards then differ by up to 2.3e-5 from the whole row's, more than they may.
+template <int DT, typename LabelT, typename Rows>
+int launch_fwd(const char* fn, const FwdArgs& a, const Rows& rows) {
+    const int64_t n_vec = a.vocab / Elem<DT>::kVec;
+    if (n_vec <= (DT == MRL_F32 ? 4096 : 3584)) return launch_fwd_shape<DT, LabelT, 256, 4>(fn, a, rows);
+    if (n_vec <= 7168) return launch_fwd_shape<DT, LabelT, 512, 4>(fn, a, rows);
+    return launch_fwd_shape<DT, LabelT, 1024, 3>(fn, a, rows);
 }
 
 template <typename Rows>

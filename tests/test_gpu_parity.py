@@ -3141,6 +3141,31 @@ def test_response_windows(dev, layout, index):
         ResponseWindows((n_seq, padded), {k: v.t() if k != "responses" else v for k, v in b.items()}, False)
 
 
+@pytest.mark.parametrize("dtype,vectors", [(torch.bfloat16, n) for n in (1, 63, 511, 512, 513, 1025, 3583, 3584, 3585, 4097, 7167,
+                                                                         7168, 7169, 9215, 9216, 9217, 19008)] +
+                         [(torch.float32, n) for n in (512, 513, 4095, 4096, 4097, 7168, 7169, 12288, 38016)] +
+                         [(torch.float16, n) for n in (512, 3585, 7169)])
+def test_forward_sweep_by_row_length(dev, dtype, vectors):
+    """Rows around the lengths at which another workgroup size takes over, and around whole rounds of it; dense
+    rows of whole vectors, and rows with edges at a stride.  A thread adds up vocab / threads entries and two
+    edges (fewer than 256 in all), 6 steps of a wavefront's and 16 partials follow: 2^-24 each of a sum of
+    positive terms, and 2^-21 for the exponents' rounding (|z| below 2^4, in units of log 2)."""
+    per = 16 // torch.empty(0, dtype=dtype).element_size()
+    gen = torch.Generator().manual_seed(vectors)
+    for vocab, stride in ((vectors * per, vectors * per), (vectors * per + 3, vectors * per + 9)):
+        z = _logits(gen, 5, stride, dtype).to(dev)[:, :vocab]
+        y = torch.randint(0, vocab, (5,), generator=gen).to(dev)
+        lp, ent, lse = mrl.vocab_logprob_entropy(z, y)
+        only, _, _ = mrl.vocab_logprob_entropy(z, y, want_entropy=False)
+        ref = torch.log_softmax(z.double(), -1)
+        want_lse = torch.logsumexp(z.double(), -1)
+        bound = (256 + 6 + 16) * 2.0 ** -24 + 2.0 ** -21
+        for got, want in ((lp, ref.gather(-1, y[:, None]).squeeze(-1)), (lse, want_lse), (only, ref.gather(-1, y[:, None]).squeeze(-1)),
+                          (ent, -(ref.exp() * ref).sum(-1))):
+            scale = max(1.0, want_lse.abs().max().item(), want.abs().max().item())
+            assert (got.double() - want).abs().max().item() <= bound * scale, (vocab, stride)
+
+
 @pytest.mark.parametrize("layout", ["padded", "packed"])
 @pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1000), (torch.bfloat16, 1003), (torch.float32, 4096),
                                          (torch.float32, 77), (torch.float16, 8200)])
