@@ -1,7 +1,7 @@
 // Row-in-registers vocabulary sweeps for gfx950.
 //
-// A workgroup owns one logits row and keeps ALL of it in registers: 256 threads for the shortest rows,
-// several workgroups per CU, up to 1024 threads with 19 16-byte vectors each = 311 296 bytes, one per CU,
+// A workgroup owns one logits row (of the shortest rows, up to four side by side) and keeps ALL of it in registers:
+// 256 threads for the shortest rows, several workgroups per CU, up to 1024 threads with 19 16-byte vectors each = 311 296 bytes, one per CU,
 // enough for a 152 064-entry bf16 row.  The softmax statistics are taken vector by vector as the data
 // arrives, the token's loss gradient follows from them, and dlogits are written from the same registers -
 // one HBM read and one HBM write per element for the whole forward + backward of the log-prob /
@@ -68,7 +68,7 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), lane));
 }
 
-// Two-level reduction for the BLK / 64 wavefronts of a workgroup: the largest reference first, so that a part is
+// Two-level reduction for the BLK / 64 wavefronts that hold a row: the largest reference first, so that a part is
 // rescaled once and the rest is sums; inside a wavefront over its 4 rows of 16 lanes and these through scalar
 // registers, then every wavefront combines the BLK / 64 partials for itself.  It is a serial chain in which the
 // workgroup neither computes on its row nor writes it; before, it went through shuffles with a rescale in every step
@@ -76,9 +76,10 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // 291, 2 367 x 32 000 fp32 109.5 -> 107.7 (108.3 -> 104.9 without entropy), 16 384 x 72 608 bf16 847 -> 835, x
 // 100 352 1 114 -> 1 099; the other shapes are at what memory gives (129 280 and 152 064 bf16, short rows) and
 // within 0.6 %.
-// lds: BLK / 64 entries that nothing else touches until the workgroup has passed another barrier.
+// lds: BLK / 64 entries of this row that nothing else touches until the workgroup has passed another barrier.  Every
+// wavefront of the workgroup comes here.
 template <int BLK, bool kEntropy>
-__device__ __forceinline__ Stats reduce_workgroup(Stats st, float k, Stats* lds) {
+__device__ __forceinline__ Stats reduce_row(Stats st, float k, Stats* lds, int tid) {
     constexpr int kWaves = BLK / 64;
     constexpr int kSteps = kWaves == 16 ? 4 : (kWaves == 8 ? 3 : 2);
     static_assert(kWaves == 4 || kWaves == 8 || kWaves == 16, "partials of 4, 8 or 16 wavefronts");
@@ -93,7 +94,7 @@ __device__ __forceinline__ Stats reduce_workgroup(Stats st, float k, Stats* lds)
         const float u16 = row_sum<4>(st.u * f);
         t.u = (lane_value(u16, 0) + lane_value(u16, 16)) + (lane_value(u16, 32) + lane_value(u16, 48));
     }
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = tid >> 6, lane = tid & 63;
     if (lane == 0) lds[wave] = t;
     // LDS accesses only, as in broadcast_ticket
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -166,25 +167,25 @@ __device__ __forceinline__ mrl::rsrc_t vec_rsrc(const RowRef& row, int q) {
 // spill the row.
 __device__ __forceinline__ void vector_fence() { __builtin_amdgcn_sched_barrier(0); }
 
-__device__ __forceinline__ uint32_t lane_offset() { return (uint32_t)threadIdx.x * 16u; }
+__device__ __forceinline__ uint32_t lane_offset(int tid) { return (uint32_t)tid * 16u; }
 
 // Vectors [A, B) of a row: loads (back to back and without a branch: vectors past the end of the row come
 // back as zeros from the range check of the buffer access), zero stores.
 template <int BLK, int A, int B, int NV>
-__device__ __forceinline__ void load_part(u32x4 (&v)[NV], const RowRef& src) {
+__device__ __forceinline__ void load_part(u32x4 (&v)[NV], const RowRef& src, int tid) {
 #pragma unroll
     for (int q = A; q < B; ++q) {
-        v[q] = mrl::buf_load_nt(vec_rsrc<BLK>(src, q), lane_offset());
+        v[q] = mrl::buf_load_nt(vec_rsrc<BLK>(src, q), lane_offset(tid));
         vector_fence();     // keeps the requests in this order wherever a row is loaded
     }
 }
 
 template <int BLK, int A, int B>
-__device__ __forceinline__ void zero_part(const RowRef& dst) {
+__device__ __forceinline__ void zero_part(const RowRef& dst, int tid) {
     const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int q = A; q < B; ++q) {
-        mrl::buf_store_nt(zero, vec_rsrc<BLK>(dst, q), lane_offset());
+        mrl::buf_store_nt(zero, vec_rsrc<BLK>(dst, q), lane_offset(tid));
         vector_fence();
     }
 }
@@ -195,7 +196,7 @@ __device__ __forceinline__ void zero_part(const RowRef& dst) {
 // is processed like any other and its result discarded, which costs three selects on the few vectors
 // that can be affected and keeps the pass free of branches.
 template <int DT, int BLK, int NV, bool kEntropy, bool kEdge>
-__device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int n_vec, float k) {
+__device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int n_vec, float k, int tid) {
     using E = Elem<DT>;
     constexpr int kVec = E::kVec;
     Stats st = {kMaxInit, 0.f, 0.f};
@@ -216,7 +217,7 @@ __device__ __forceinline__ Stats thread_stats_careful(const u32x4 (&v)[NV], int 
 #pragma unroll
         for (int i = 0; i < kVec; ++i) add_one<kEntropy>(nx, z[i], k, mk);
         if (q >= Tail<BLK, NV, kEdge>::kFull) {
-            const bool valid = q * BLK + (int)threadIdx.x < n_vec;
+            const bool valid = q * BLK + tid < n_vec;
             st.m = valid ? nx.m : st.m;
             st.s = valid ? nx.s : st.s;
             st.u = valid ? nx.u : st.u;
@@ -280,7 +281,7 @@ __device__ __forceinline__ float vector_max(const u32x4& vec) {
 // kEdge: the thread also holds one entry of the row outside its vectors, z_edge, if has_edge.
 template <int DT, int BLK, int NV, bool kEntropy, bool kEdge>
 __device__ __forceinline__ Stats thread_stats(const u32x4 (&v)[NV], int n_vec, float k, bool want_max, bool has_edge,
-                                              float z_edge) {
+                                              float z_edge, int tid) {
     Stats st = {kMaxInit, 0.f, 0.f};
     // in a row so short that a thread may hold no complete vector there is no reference to take
     bool careful = (Tail<BLK, NV, kEdge>::kFull == 0 && n_vec < BLK) || want_max;
@@ -294,7 +295,7 @@ __device__ __forceinline__ Stats thread_stats(const u32x4 (&v)[NV], int n_vec, f
             } else if (q * BLK < n_vec) {               // uniform: nothing to compute past the end of the row
                 float s = st.s, u = st.u;
                 add_vector<DT, kEntropy>(v[q], k, rk, s, u);
-                const bool valid = q * BLK + (int)threadIdx.x < n_vec;
+                const bool valid = q * BLK + tid < n_vec;
                 st.s = valid ? s : st.s;
                 st.u = valid ? u : st.u;
             }
@@ -311,7 +312,7 @@ __device__ __forceinline__ Stats thread_stats(const u32x4 (&v)[NV], int n_vec, f
         careful = !(st.s < kSumLimit);
     }
     if (careful) {
-        st = thread_stats_careful<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k);
+        st = thread_stats_careful<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k, tid);
         if (kEdge && has_edge) {
             grow_max<kEntropy>(st, z_edge, k);
             add_one<kEntropy>(st, z_edge, k, st.m * k);
@@ -338,10 +339,10 @@ __device__ __forceinline__ u32x4 grad_vec(const u32x4& v, const RowGrad& g) {
 
 // dlogits of vectors [A, B) of the row in registers, stored as they are computed.
 template <int DT, int BLK, bool kEntropy, int A, int B, int NV>
-__device__ __forceinline__ void grad_part(const u32x4 (&v)[NV], const RowGrad& g, const RowRef& dst) {
+__device__ __forceinline__ void grad_part(const u32x4 (&v)[NV], const RowGrad& g, const RowRef& dst, int tid) {
 #pragma unroll
     for (int q = A; q < B; ++q) {
-        mrl::buf_store_nt(grad_vec<DT, kEntropy>(v[q], g), vec_rsrc<BLK>(dst, q), lane_offset());
+        mrl::buf_store_nt(grad_vec<DT, kEntropy>(v[q], g), vec_rsrc<BLK>(dst, q), lane_offset(tid));
         vector_fence();
     }
 }
@@ -369,9 +370,8 @@ __device__ __forceinline__ RowSpan row_span(const typename Elem<DT>::T* row, int
 
 // Byte offset inside the row of this thread's edge entry, out of range for a thread without one.
 template <int DT>
-__device__ __forceinline__ uint32_t edge_offset(const RowSpan& s, int vocab) {
+__device__ __forceinline__ uint32_t edge_offset(const RowSpan& s, int vocab, int tid) {
     constexpr int kVec = Elem<DT>::kVec;
-    const int tid = (int)threadIdx.x;
     const int j = tid < s.head ? tid : tid + s.n_vec * kVec;
     return j < vocab ? (uint32_t)j * (uint32_t)sizeof(typename Elem<DT>::T) : 0x80000000u;
 }
@@ -382,7 +382,7 @@ __device__ __forceinline__ uint32_t edge_offset(const RowSpan& s, int vocab) {
 // in program order.  y and dst (of `bytes` bytes) are relative to the unit; span: its vectors.
 template <int DT, int BLK, bool kEntropy, bool kEdge>
 __device__ __forceinline__ void store_label_grad(const typename Elem<DT>::T* dst, uint32_t bytes, const RowSpan& span,
-                                                 const RowGrad& g, bool y_ok, int64_t y, float z_y) {
+                                                 const RowGrad& g, bool y_ok, int64_t y, float z_y, int tid) {
     using E = Elem<DT>;
     int writer;
     if (kEdge) {
@@ -392,9 +392,12 @@ __device__ __forceinline__ void store_label_grad(const typename Elem<DT>::T* dst
     } else {
         writer = (int)((y / E::kVec) % BLK);
     }
-    const bool owner = y_ok && writer == (int)threadIdx.x;
+    const bool owner = y_ok && writer == tid;
     const uint32_t off = owner ? (uint32_t)y * (uint32_t)sizeof(typename E::T) : 0x80000000u;
-    E::buf_store(mrl::make_rsrc(dst, bytes), off, grad_elem<kEntropy>(g, z_y) + g.onehot);
+    // product and sum in one operation by name, so that every instance of the kernel rounds alike
+    const float e = fast_exp2(__builtin_fmaf(z_y, g.k, -g.lse2));
+    const float w = kEntropy ? __builtin_fmaf(g.c1, z_y, g.c0) : g.c0;
+    E::buf_store(mrl::make_rsrc(dst, bytes), off, __builtin_fmaf(e, w, g.onehot));
 }
 
 struct RowScalars {
@@ -562,7 +565,7 @@ __device__ __forceinline__ Stats stream_stats(const typename Elem<DT>::T* base, 
         }
     }
     __syncthreads();            // lds may still be read by a slow wavefront of the previous reduction
-    return reduce_workgroup<kWideBlock, kEntropy>(st, k, lds);
+    return reduce_row<kWideBlock, kEntropy>(st, k, lds, (int)threadIdx.x);
 }
 
 // What thread 0 found in the other half's record.
@@ -643,15 +646,16 @@ __device__ __forceinline__ Stats exchange_halves(const Stats& mine, int half, Ha
 // row_ticket NULL: a workgroup per row, each ends with its first.
 // Wavefronts per SIMD that the register allocator leaves room for: 4 hold the widest rows (76 registers of
 // row), short rows leave more of the register file to further workgroups.
-constexpr int waves_per_simd(int nv) { return nv <= 4 ? 8 : (nv <= 8 ? 6 : 4); }
+constexpr int waves_per_simd(int nv, int rows) { return nv <= 4 ? 8 : (nv <= 8 && rows == 1 ? 6 : 4); }
 
 // kEdge: rows of any element alignment (see RowSpan); dlogits rows are misaligned alike.  Only these rows are
 // ever swept a second time (mrl_fused_logprob_regrad): again.carried is then given and row_terms NULL.
 // kWide: the units of work are half rows (see "wide rows" above): unit 2 r is the first
 // half_elems entries of row r, unit 2 r + 1 the rest; n_rows then counts units.
-template <int DT, int BLK, int NV, bool kEntropy, bool kWide, bool kEdge>
-__global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persistent_kernel(
-    const typename Elem<DT>::T* logits, int64_t row_stride, int vocab, int64_t n_rows,
+// kRows: consecutive rows that a workgroup holds side by side, each by BLK of its threads (see pick_rows).
+template <int DT, int BLK, int NV, int kRows, bool kEntropy, bool kWide, bool kEdge>
+__global__ __launch_bounds__(BLK * kRows, waves_per_simd(NV, kRows)) void fused_sweep_persistent_kernel(
+    const typename Elem<DT>::T* logits, int64_t row_stride, int vocab, uint32_t n_rows,
     const void* __restrict__ labels, int labels_dtype, float inv_t, const float* __restrict__ row_ops, int has_old,
     Params p, float grad_scale, const float* __restrict__ grad_scale_dev, mrl::Again again,
     typename Elem<DT>::T* dlogits, int64_t d_stride, float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ row_terms,
@@ -660,8 +664,9 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     using T = typename E::T;
     static_assert(!kWide || BLK == kWideBlock, "halves of a row are held by workgroups of kWideBlock threads");
     static_assert(!(kWide && kEdge), "a row that two workgroups hold is aligned");
+    static_assert(kRows == 1 || (!kWide && (BLK & (BLK - 1)) == 0), "whole rows side by side");
     // two sets of partials used in turn: a slow wavefront may still read the last row's
-    __shared__ Stats lds[2][BLK / 64];
+    __shared__ Stats lds[2][kRows * BLK / 64];
     int parts = 0;
     // Two slots used in turn, one per BROADCAST: thread 0 may write the next ticket while a slow wavefront
     // has yet to read this one's, and the barrier of the broadcast in between separates a slot's reuse.
@@ -670,7 +675,9 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     int slot = 0;
     __shared__ Inbox inbox;                 // the other half's record (wide rows)
 
-    const int tid = threadIdx.x;
+    // this thread within its row, and the row within the workgroup's unit (the same for a whole wavefront)
+    const int tid = kRows == 1 ? (int)threadIdx.x : (int)threadIdx.x & (BLK - 1);
+    const int lane_row = kRows == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / BLK);
     const bool outputs = tid == 0 && (!kEdge || row_terms != nullptr);
     // as in scale_rows_note_kernel: equal scales are noted by workgroup 0 at once, others by whoever ends last
     bool moved = false;
@@ -678,7 +685,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         const float u = *grad_scale_dev;
         moved = u / again.carried[0] != 1.f;
         if (!moved && !again.always) {
-            if (blockIdx.x == 0 && tid == 0) note_scale(u, again.carried, again.learned);
+            if (blockIdx.x == 0 && threadIdx.x == 0) note_scale(u, again.carried, again.learned);
             return;
         }
     }
@@ -695,7 +702,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     // is never read: its descriptor gets zero bytes, so the (unconditional) loads return zeros
     // without touching memory; the same happens past the last row.
     struct Next {
-        int64_t r;              // >= n_rows: none
+        uint32_t r;             // unit; behind the last: none
         int64_t y;
         const T* zy_ptr;
         RowRef row;
@@ -703,8 +710,9 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         const T* edge_base;
         uint32_t edge_bytes;    // 0: not read
     };
-    int64_t r = (int64_t)blockIdx.x * group;
-    int left = group - 1;                   // rows of the current ticket behind r
+    // 32 bits: at most 2^31 - 2 units, and what tickets add behind them stays far below 2^32 as well
+    uint32_t r = blockIdx.x * (uint32_t)group;
+    int left = group - 1;                   // units of the current ticket behind r
     // the unit behind r: the next of the ticket, or the first of a new ticket (asked for in `mine`)
     auto following = [&](uint32_t mine) {
         if (left > 0) {
@@ -712,25 +720,29 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
             return r + 1;
         }
         left = group - 1;
-        const int64_t t = (int64_t)broadcast_ticket(mine, &next_row[slot]);
+        const uint32_t t = broadcast_ticket(mine, &next_row[slot]);
         slot ^= 1;
-        return row_ticket ? t + (int64_t)gridDim.x * group : n_rows;
+        return row_ticket ? t + gridDim.x * (uint32_t)group : n_rows;
     };
-    auto plan = [&](int64_t r2) {
+    auto plan = [&](uint32_t r2) {
         Next n;
         n.r = r2;
-        const bool has = r2 < n_rows;
-        const int64_t un = has ? r2 : r;                    // unit
-        const int64_t rn = kWide ? (un >> 1) : un;          // row
+        bool has = r2 * kRows < n_rows;
+        const uint32_t un = has ? r2 : r;                   // unit
+        uint32_t rn = kWide ? (un >> 1) : un * kRows + lane_row;    // row
+        if (kRows > 1 && rn >= n_rows) {                    // the last unit may be short of rows
+            has = false;
+            rn = n_rows - 1;
+        }
         const int hn = kWide ? (int)(un & 1) : 0;
-        const bool live = has && (row_ops[rn * MRL_ROW_OPS + MRL_OP_MASK] != 0.f);
-        const T* nrow = logits + rn * row_stride;
+        const bool live = has && (row_ops[(int64_t)rn * MRL_ROW_OPS + MRL_OP_MASK] != 0.f);
+        const T* nrow = logits + (int64_t)rn * row_stride;
         if (kEdge) {
             const RowSpan span = row_span<DT>(nrow, vocab);
             n.row = row_ref(nrow + span.head, live ? (uint32_t)span.n_vec * 16u : 0u);
             n.edge_base = nrow;
             n.edge_bytes = live ? unit_bytes[0] : 0u;
-            n.edge_off = edge_offset<DT>(span, vocab);
+            n.edge_off = edge_offset<DT>(span, vocab, tid);
         } else {
             n.row = row_ref(nrow + (hn ? half_elems : 0), live ? unit_bytes[hn] : 0u);
         }
@@ -752,7 +764,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     auto load_edge = [&](const Next& n) {
         return kEdge ? E::buf_load_bits(mrl::make_rsrc(n.edge_base, n.edge_bytes), n.edge_off) : 0u;
     };
-    if (r < n_rows) {
+    if (r * kRows < n_rows) {
         const Next first = plan(r);
         y = first.y;
         // the same sequence of operations as one turn of the loop leaves behind (with stores that
@@ -760,28 +772,38 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         // the compiler has to assume when it places the waits of the statistics pass - is the same
         // on every path into it
         const RowRef none = row_ref(dlogits, 0u);
-        mrl::buf_atomic_add_u32(mrl::make_rsrc(dlogits, 0u), lane_offset(), 0u);
-        zero_part<BLK, 0, H>(none);
-        load_part<BLK, 0, H>(v, first.row);
-        zero_part<BLK, H, NV>(none);
+        mrl::buf_atomic_add_u32(mrl::make_rsrc(dlogits, 0u), lane_offset(tid), 0u);
+        zero_part<BLK, 0, H>(none, tid);
+        load_part<BLK, 0, H>(v, first.row, tid);
+        zero_part<BLK, H, NV>(none, tid);
         if (kEdge) E::buf_store(mrl::make_rsrc(dlogits, 0u), 0u, 0.f);
         mrl::buf_store_b32(0u, mrl::make_rsrc(dlogits, 0u), 0u);
-        load_part<BLK, H, NV>(v, first.row);
+        load_part<BLK, H, NV>(v, first.row, tid);
         edge_bits = load_edge(first);
         zy_bits = E::load_bits(first.zy_ptr);
     }
-    while (r < n_rows) {
-        const int64_t row = kWide ? (r >> 1) : r;
+    while (r * kRows < n_rows) {
+        const uint32_t place = kWide ? (r >> 1) : r * kRows + lane_row;
+        const bool mine_to_do = kRows == 1 || place < n_rows;   // else a place behind the last row: nothing is written
+        const int64_t row = mine_to_do ? place : n_rows - 1;
         const int half = kWide ? (int)(r & 1) : 0;
         const int my_first = half ? half_elems : 0;         // first entry of this unit within the row
         RowSpan span = {0, (int)(unit_bytes[half] / 16u)};
         if (kEdge) span = row_span<DT>(logits + row * row_stride, vocab);
         const int n_vec = span.n_vec;
         T* const drow = dlogits + row * d_stride + my_first;
-        const RowRef dst = row_ref(drow + span.head, kEdge ? (uint32_t)n_vec * 16u : unit_bytes[half]);
-        const uint32_t edge_off = kEdge ? edge_offset<DT>(span, vocab) : 0u;
+        const RowRef dst = row_ref(drow + span.head, !mine_to_do ? 0u : (kEdge ? (uint32_t)n_vec * 16u : unit_bytes[half]));
+        const uint32_t edge_off = kEdge ? edge_offset<DT>(span, vocab, tid) : 0u;
+        const uint32_t edge_bytes = mine_to_do ? unit_bytes[0] : 0u;
         const float* ops = row_ops + row * MRL_ROW_OPS;
-        const float m = ops[MRL_OP_MASK];
+        const float m = mine_to_do ? ops[MRL_OP_MASK] : 0.f;
+        // the reduction's barrier is for the whole workgroup: it comes where any of its rows counts
+        bool reduced = false;
+#pragma unroll
+        for (int i = 0; i < (kRows > 1 ? kRows : 0); ++i) {
+            const uint32_t ri = r * kRows + i;
+            reduced = reduced || (ri < n_rows && row_ops[(int64_t)ri * MRL_ROW_OPS + MRL_OP_MASK] != 0.f);
+        }
         const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
         // the label's entry gets its one-hot term from the unit that holds it
         const int64_t y_here = y - my_first;
@@ -789,12 +811,51 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
         Next nx;
         uint32_t zy_next = 0, edge_next = 0;
 
+        if constexpr (kRows > 1) {
+            // Rows of all kinds share one path: two paths that load the next rows would leave them in different
+            // registers, and the copies where the paths meet wait for every load.  A row without a gradient is
+            // written as the product of zero coefficients and zeros.
+            float z_y = E::from_bits(zy_bits), z_edge = kEdge ? E::from_bits(edge_bits) : 0.f;
+            RowGrad g = {k, 0.f, 0.f, 0.f, 0.f};
+            bool live = false;
+            if (reduced) {
+                const Stats st = thread_stats<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k, !y_ok, edge_off != 0x80000000u, z_edge, tid);
+                const Stats tot = reduce_row<BLK, kEntropy>(st, k, lds[parts] + lane_row * (BLK / 64), tid);
+                parts ^= 1;
+                float lse;
+                const RowScalars s = row_scalars<kEntropy>(tot, k, inv_t, y_ok, z_y, ops, has_old, p, grad_scale, m, lse);
+                if (m != 0.f) {
+                    if (outputs) write_row_outputs(row, s, m, logp, entropy, row_terms);
+                    live = s.g_lp != 0.f || s.g_h != 0.f;
+                    if (live) g = row_grad<kEntropy>(s, k, inv_t, lse);
+                }
+            }
+            if (m == 0.f && outputs && mine_to_do) write_masked_row_outputs(row, logp, entropy, row_terms);
+            if (!live) {
+#pragma unroll
+                for (int q = 0; q < NV; ++q) v[q] = mrl::make_u32x4(0u, 0u, 0u, 0u);
+                z_y = z_edge = 0.f;
+            }
+            const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset((int)threadIdx.x), (uint32_t)group);
+            grad_part<DT, BLK, kEntropy, 0, H>(v, g, dst, tid);
+            nx = plan(following(mine));
+            load_part<BLK, 0, H>(v, nx.row, tid);
+            grad_part<DT, BLK, kEntropy, H, NV>(v, g, dst, tid);
+            if (kEdge) E::buf_store(mrl::make_rsrc(drow, edge_bytes), edge_off, grad_elem<kEntropy>(g, z_edge));
+            store_label_grad<DT, BLK, kEntropy, kEdge>(drow, unit_bytes[0], span, g, live && y_ok, y, z_y, tid);
+            load_part<BLK, H, NV>(v, nx.row, tid);
+            y = nx.y;
+            zy_bits = E::load_bits(nx.zy_ptr);
+            edge_bits = load_edge(nx);
+            r = nx.r;
+            continue;
+        }
         bool wrote = false;                 // dlogits of row r written and the next row requested
         if (m != 0.f) {
             float z_y = E::from_bits(zy_bits);
             const float z_edge = kEdge ? E::from_bits(edge_bits) : 0.f;
-            const Stats st = thread_stats<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k, !y_ok, edge_off != 0x80000000u, z_edge);
-            Stats tot = reduce_workgroup<BLK, kEntropy>(st, k, lds[parts]);
+            const Stats st = thread_stats<DT, BLK, NV, kEntropy, kEdge>(v, n_vec, k, !y_ok, edge_off != 0x80000000u, z_edge, tid);
+            Stats tot = reduce_row<BLK, kEntropy>(st, k, lds[parts], tid);
             parts ^= 1;
             if (kWide) {
                 // the logit at the label as this unit loaded it counts only if the label lies in this
@@ -812,14 +873,14 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
                 const RowGrad g = row_grad<kEntropy>(s, k, inv_t, lse);
                 // the ticket is asked for ahead of the stores and picked up behind the first H of
                 // them: it is older than every store, so waiting for it does not wait for them
-                const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset(), (uint32_t)group);
-                grad_part<DT, BLK, kEntropy, 0, H>(v, g, dst);
+                const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset((int)threadIdx.x), (uint32_t)group);
+                grad_part<DT, BLK, kEntropy, 0, H>(v, g, dst, tid);
                 nx = plan(following(mine));
-                load_part<BLK, 0, H>(v, nx.row);
-                grad_part<DT, BLK, kEntropy, H, NV>(v, g, dst);
-                if (kEdge) E::buf_store(mrl::make_rsrc(drow, unit_bytes[0]), edge_off, grad_elem<kEntropy>(g, z_edge));
-                store_label_grad<DT, BLK, kEntropy, kEdge>(drow, unit_bytes[half], span, g, y_mine, y_here, z_y);
-                load_part<BLK, H, NV>(v, nx.row);
+                load_part<BLK, 0, H>(v, nx.row, tid);
+                grad_part<DT, BLK, kEntropy, H, NV>(v, g, dst, tid);
+                if (kEdge) E::buf_store(mrl::make_rsrc(drow, edge_bytes), edge_off, grad_elem<kEntropy>(g, z_edge));
+                store_label_grad<DT, BLK, kEntropy, kEdge>(drow, unit_bytes[half], span, g, y_mine, y_here, z_y, tid);
+                load_part<BLK, H, NV>(v, nx.row, tid);
                 edge_next = load_edge(nx);
                 zy_next = E::load_bits(nx.zy_ptr);
                 wrote = true;
@@ -828,14 +889,14 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
             write_masked_row_outputs(row, logp, entropy, row_terms);
         }
         if (!wrote) {                       // no gradient for this row: zeros, same order of operations
-            const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset(), (uint32_t)group);
-            zero_part<BLK, 0, H>(dst);
+            const uint32_t mine = mrl::buf_atomic_add_u32(left > 0 ? no_ticket : ticket, lane_offset((int)threadIdx.x), (uint32_t)group);
+            zero_part<BLK, 0, H>(dst, tid);
             nx = plan(following(mine));
-            load_part<BLK, 0, H>(v, nx.row);
-            zero_part<BLK, H, NV>(dst);
-            if (kEdge) E::buf_store(mrl::make_rsrc(drow, unit_bytes[0]), edge_off, 0.f);
+            load_part<BLK, 0, H>(v, nx.row, tid);
+            zero_part<BLK, H, NV>(dst, tid);
+            if (kEdge) E::buf_store(mrl::make_rsrc(drow, edge_bytes), edge_off, 0.f);
             mrl::buf_store_b32(0u, mrl::make_rsrc(dlogits, 0u), 0u);
-            load_part<BLK, H, NV>(v, nx.row);
+            load_part<BLK, H, NV>(v, nx.row, tid);
             edge_next = load_edge(nx);
             zy_next = E::load_bits(nx.zy_ptr);
         }
@@ -846,7 +907,7 @@ __global__ __launch_bounds__(BLK, waves_per_simd(NV)) void fused_sweep_persisten
     }
     // Every wavefront of a workgroup with rows has read the old scale by now: it has passed the barrier of at
     // least one ticket.  One without rows has nothing to do whatever it reads.
-    if (kEdge && again.carried && tid == 0)
+    if (kEdge && again.carried && threadIdx.x == 0)
         note_scale_last(*grad_scale_dev, again.carried, again.learned, moved ? again.rescales : nullptr);
 }
 
@@ -984,7 +1045,8 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
 //   bf16:  16 KB 1 517 -> 5 467, 32 KB 2 980 -> 5 595, 48 KB 4 197 -> 5 731, 64 KB 5 144 -> 6 139,
 //          80 KB 4 417 -> 5 906, 100 KB 5 199 -> 5 879 (512 x 16; 512 x 12 where both fit within 2 %)
 //   fp32 (half the entries per byte to compute): 32 KB 3 802 -> 5 599, 48 KB 4 859 -> 6 205, 64 KB 5 832 -> 6 083;
-//          96 and 128 KB stay with 1024 x 8 (6 190 and 6 250 against 5 800 and 5 700 with 512 x 16)
+//          96 and 128 KB stay with 1024 x 8 (6 190 and 6 250 against 5 800 and 5 700 with 512 x 16);
+//          34 KB 5 361 with 512 x 12, 39 KB 6 046: up to there 256 x 12, which takes rows side by side
 // The choice depends on the row's length alone, so a row's result does not depend on the other rows' contents.
 // Its place does enter for rows that are not whole 128-byte lines (see RowSpan): which thread adds which entry
 // follows from the row's address modulo 128, so the fp32 sums round differently at another place in the batch.
@@ -995,6 +1057,7 @@ inline Shape pick_shape(int dtype, int64_t n_vec) {
     if (n_vec <= 1024) return k256x4;
     if (n_vec <= 2048) return k256x8;
     if (dtype == MRL_F32) {
+        if (n_vec <= 2496) return k256x12;
         if (n_vec <= 4096) return k512x12;
         if (n_vec <= 8192) return k1024x8;
     } else {
@@ -1005,6 +1068,45 @@ inline Shape pick_shape(int dtype, int64_t n_vec) {
     if (n_vec <= 12288) return k1024x12;
     if (n_vec <= 16384) return k1024x16;
     return n_vec <= kMaxVec ? k1024x19 : kTooLong;
+}
+
+// Rows of 256 threads that a workgroup holds side by side (and with how many vectors a thread: fewer than the row's
+// shape has where that leaves no lane idle; which thread holds what is the same, and with it every bit of the
+// results).  Six or eight small workgroups per CU keep as many bytes in flight as two larger ones, but as many
+// separate bursts of 16 to 48 KiB: the rows of a unit are requested, and written, together.  1 GB of logits, GB/s
+// of a row alone -> side by side (16 bits without and with the entropy's sum; fp32 within 1 % of each other):
+//   16 bits  8 000 entries 5 227 -> 5 733, 5 247 -> 5 675; 11 776 5 522 -> 6 046, 5 497 -> 5 845; 13 824 5 461 ->
+//            6 052, 5 471 -> 5 974; 16 384 5 458 -> 6 116, 5 473 -> 6 069; 17 408 5 399 -> 5 895, 5 383 -> 5 826;
+//            20 480 5 683 -> 5 866, 5 665 -> 5 823.  Not 7 168 (4 846 -> 4 824 with entropy), 9 728 (5 516 -> 5 227)
+//            and 22 528 (5 616 -> 5 700): there the last of a thread's vectors are mostly past the row, and the
+//            arithmetic of a unit, which starts and ends together, shows
+//   fp32     3 328 5 405 -> 5 954, 4 096 5 497 -> 5 849, 4 864 5 604 -> 6 053, 5 888 5 588 -> 6 200, 8 192 5 568 -> 6 190,
+//            8 704 5 361 -> 5 939, 9 728 5 825 -> 6 017
+// Few rows: where all start at once they share tickets and are done sooner (1 024 x 8 000 bf16 13.0 -> 10.8 us,
+// 1 024 x 5 888 fp32 13.9 -> 12.6); in between the last, half empty round of larger units costs more than they gain
+// (2 048 x 16 384 bf16 26.6 -> 29.0 us, 4 096 x 8 000 28.9 -> 30.8; 8 192 x 16 384 100.1 -> 97.6), except where rows
+// are longer than 32 KiB (1 024 x 17 408 21.8 -> 15.7, 3 072 47.0 -> 45.0).
+struct SideBySide {
+    int rows, vectors;          // rows 1: a row to a workgroup
+};
+
+inline SideBySide pick_rows(int dtype, int64_t n_vec, int64_t n_rows) {
+    const SideBySide alone = {1, 0};
+    SideBySide s = alone;
+    int64_t at_once = 0;        // rows that start together on 256 CUs
+    if (dtype == MRL_F32) {
+        if (n_vec > 512 && n_vec <= 1024) s = {4, 4}, at_once = 2048;
+        else if (n_vec > 1024 && n_vec <= 2048) s = {4, 8}, at_once = 1024;
+        else if (n_vec > 2048 && n_vec <= 2496) s = {4, 12};
+    } else {
+        if (n_vec > 928 && n_vec <= 1024) s = {4, 4}, at_once = 2048;
+        else if (n_vec > 1312 && n_vec <= 1792) s = {2, 7}, at_once = 1024;
+        else if (n_vec > 1792 && n_vec <= 2048) s = {2, 8}, at_once = 1024;
+        else if (n_vec > 2048 && n_vec <= 2560) s = {2, 10};
+    }
+    const bool long_rows = n_vec > 2048;
+    const bool pays = n_rows >= (n_vec <= 1024 ? 16384 : 8192) || (n_rows >= 512 && (long_rows || n_rows <= at_once));
+    return pays ? s : alone;
 }
 
 // Number of CUs of the current device (one persistent workgroup each); 0 if the query fails.
@@ -1024,23 +1126,24 @@ constexpr int64_t kWorkspaceHeader = 16;    // the row counter, padded to the al
 // Unaligned rows below this go to the split kernels: a thread then holds less than half of its 4 vectors.
 constexpr int64_t kMinEdgeRowBytes = 8192;
 
-template <int DT, int BLK, int NV, bool kEntropy, bool kWide, bool kEdge>
+template <int DT, int BLK, int NV, int kRows, bool kEntropy, bool kWide, bool kEdge>
 int launch_sweep(const mrl::FusedArgs& a) {
     using T = typename Elem<DT>::T;
     const Params p = {a.clip_lo, a.clip_hi, a.kl_coef, a.entropy_coeff, 1.f, a.kl_penalty, 0};
     unsigned int* counter = reinterpret_cast<unsigned int*>(a.workspace);
-    const int64_t units = kWide ? 2 * a.n_rows : a.n_rows;
+    const int64_t rows = kWide ? 2 * a.n_rows : a.n_rows;       // half rows are counted as such
+    const int64_t units = (rows + kRows - 1) / kRows;
     int64_t grid = units;
     int group = 1;
     if (counter != nullptr) {
         const int cus = cu_count();
         if (cus < 2) return mrl::fail(MRL_ERR_LAUNCH, "mrl_fused_logprob_loss: cannot query the device");
         // half rows: an even number of workgroups, so that the halves of a row start side by side
-        const int64_t cap = kWide ? (cus & ~1) : (int64_t)cus * (waves_per_simd(NV) * 4 / (BLK / 64));
+        const int64_t cap = kWide ? (cus & ~1) : (int64_t)cus * (waves_per_simd(NV, kRows) * 4 / (BLK * kRows / 64));
         // Rows per ticket: the counter serves about 85 tickets per microsecond, rows below 32 KiB go faster
         // than that (8 000 bf16 logits, rows per ticket 1 / 2 / 4: 2 728 / 5 085 / 5 276 GB/s for 155 648 rows,
         // 1 819 / 2 537 / 2 479 for 2 048; 16 384: 5 241 / 5 481 / 5 294; 24 576: 5 681 / 5 466 / 5 253).
-        if (BLK == 256 && NV <= 8 && a.n_rows > 512) group = NV <= 4 && a.n_rows >= 4096 ? 4 : 2;
+        if (BLK * kRows == 256 && NV <= 8 && a.n_rows > 512) group = NV <= 4 && a.n_rows >= 4096 ? 4 : 2;
         grid = (units + group - 1) / group;
         if (cap < grid) grid = cap;
         if (!a.workspace_cleared) {
@@ -1050,39 +1153,47 @@ int launch_sweep(const mrl::FusedArgs& a) {
         }
     }
     HalfRecord* rec = kWide ? reinterpret_cast<HalfRecord*>(reinterpret_cast<char*>(a.workspace) + kWorkspaceHeader) : nullptr;
-    hipLaunchKernelGGL((fused_sweep_persistent_kernel<DT, BLK, NV, kEntropy, kWide, kEdge>), dim3((unsigned)grid), dim3(BLK),
-                       0, a.stream, (const T*)a.logits, a.row_stride, (int)a.vocab, units, a.labels, a.labels_dtype,
+    hipLaunchKernelGGL((fused_sweep_persistent_kernel<DT, BLK, NV, kRows, kEntropy, kWide, kEdge>), dim3((unsigned)grid),
+                       dim3(BLK * kRows), 0, a.stream, (const T*)a.logits, a.row_stride, (int)a.vocab, (uint32_t)rows, a.labels, a.labels_dtype,
                        a.inv_t, a.row_ops, a.has_old, p, a.grad_scale, a.grad_scale_dev, a.again, (T*)a.dlogits, a.d_stride, a.logp,
                        a.entropy, a.row_terms, counter, group, (int)a.half_elems, rec,
                        g_wide_spin_limit.load(std::memory_order_relaxed));
     return mrl::check_launch("mrl_fused_logprob_loss");
 }
 
-template <int DT, int BLK, int NV>
+template <int DT, int BLK, int NV, int kRows = 1>
 int launch_narrow(const mrl::FusedArgs& a) {
     if (a.edge)
-        return a.with_entropy ? launch_sweep<DT, BLK, NV, true, false, true>(a) : launch_sweep<DT, BLK, NV, false, false, true>(a);
-    return a.with_entropy ? launch_sweep<DT, BLK, NV, true, false, false>(a) : launch_sweep<DT, BLK, NV, false, false, false>(a);
+        return a.with_entropy ? launch_sweep<DT, BLK, NV, kRows, true, false, true>(a)
+                              : launch_sweep<DT, BLK, NV, kRows, false, false, true>(a);
+    return a.with_entropy ? launch_sweep<DT, BLK, NV, kRows, true, false, false>(a)
+                          : launch_sweep<DT, BLK, NV, kRows, false, false, false>(a);
 }
 
 template <int DT, int NV>
 int launch_1024(const mrl::FusedArgs& a) {
     if (!a.wide) return launch_narrow<DT, kWideBlock, NV>(a);
-    return a.with_entropy ? launch_sweep<DT, kWideBlock, NV, true, true, false>(a)
-                          : launch_sweep<DT, kWideBlock, NV, false, true, false>(a);
+    return a.with_entropy ? launch_sweep<DT, kWideBlock, NV, 1, true, true, false>(a)
+                          : launch_sweep<DT, kWideBlock, NV, 1, false, true, false>(a);
 }
 
 template <int DT>
-int fused_by_shape(Shape shape, const mrl::FusedArgs& a) {
-    if (shape == k256x4) return launch_narrow<DT, 256, 4>(a);
-    if (shape == k256x8) return launch_narrow<DT, 256, 8>(a);
-    if (shape == k512x12) return launch_narrow<DT, 512, 12>(a);
+int fused_by_shape(Shape shape, SideBySide side, const mrl::FusedArgs& a) {
     if constexpr (DT == MRL_F32) {
+        if (side.rows == 4 && side.vectors == 8) return launch_narrow<DT, 256, 8, 4>(a);
+        if (side.rows == 4 && side.vectors == 12) return launch_narrow<DT, 256, 12, 4>(a);
         if (shape == k1024x8) return launch_narrow<DT, 1024, 8>(a);
     } else {
-        if (shape == k256x12) return launch_narrow<DT, 256, 12>(a);
+        if (side.rows == 2 && side.vectors == 7) return launch_narrow<DT, 256, 7, 2>(a);
+        if (side.rows == 2 && side.vectors == 8) return launch_narrow<DT, 256, 8, 2>(a);
+        if (side.rows == 2) return launch_narrow<DT, 256, 10, 2>(a);
         if (shape == k512x16) return launch_narrow<DT, 512, 16>(a);
     }
+    if (side.rows == 4) return launch_narrow<DT, 256, 4, 4>(a);
+    if (shape == k256x4) return launch_narrow<DT, 256, 4>(a);
+    if (shape == k256x8) return launch_narrow<DT, 256, 8>(a);
+    if (shape == k256x12) return launch_narrow<DT, 256, 12>(a);
+    if (shape == k512x12) return launch_narrow<DT, 512, 12>(a);
     if (shape == k1024x12) return launch_1024<DT, 12>(a);
     if (shape == k1024x16) return launch_1024<DT, 16>(a);
     return launch_1024<DT, 19>(a);
@@ -1231,6 +1342,8 @@ static int run_sweep(const char* fn, mrl::FusedArgs& a, int64_t workspace_bytes)
         a.half_elems = (n_vec + 1) / 2 * (16 / eb);
         shape = pick_shape(a.dtype, (n_vec + 1) / 2);
     }
+    // without a counter every row has a workgroup of its own
+    const SideBySide side = a.workspace != nullptr && !a.wide ? pick_rows(a.dtype, n_vec, a.n_rows) : SideBySide{1, 0};
     if (a.workspace != nullptr || a.wide) {
         const int64_t need = a.wide ? mrl_fused_workspace_bytes(a.dtype, a.n_rows, a.vocab) : kWorkspaceHeader;
         MRL_REQUIRE(a.workspace != nullptr && workspace_bytes >= need, MRL_ERR_INVALID_ARG,
@@ -1238,9 +1351,9 @@ static int run_sweep(const char* fn, mrl::FusedArgs& a, int64_t workspace_bytes)
                     "their statistics through it)", fn, (long long)(a.workspace ? workspace_bytes : 0), (long long)need);
     }
     switch (a.dtype) {
-        case MRL_F32: return fused_by_shape<MRL_F32>(shape, a);
-        case MRL_BF16: return fused_by_shape<MRL_BF16>(shape, a);
-        default: return fused_by_shape<MRL_F16>(shape, a);
+        case MRL_F32: return fused_by_shape<MRL_F32>(shape, side, a);
+        case MRL_BF16: return fused_by_shape<MRL_BF16>(shape, side, a);
+        default: return fused_by_shape<MRL_F16>(shape, side, a);
     }
 }
 

@@ -1472,6 +1472,64 @@ def test_fused_sweep_tickets_of_masked_rows(dev, rows, vocab, runs):
     assert bool(terms[live, 5].all().item())                            # the mask, of every live row
 
 
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 7432), (torch.bfloat16, 8003), (torch.bfloat16, 10505), (torch.float16, 14336),
+                                         (torch.bfloat16, 14347), (torch.bfloat16, 16384), (torch.bfloat16, 16392),
+                                         (torch.float16, 20480), (torch.float32, 2052), (torch.float32, 4096),
+                                         (torch.float32, 4103), (torch.float32, 8192), (torch.float32, 8196),
+                                         (torch.float32, 9984)])
+@pytest.mark.parametrize("rows", [512, 1023, 16386])
+def test_fused_sweep_rows_side_by_side(dev, dtype, vocab, rows):
+    """Rows that a workgroup holds two or four of: every row comes out as a workgroup of its own delivers it, bit for
+    bit - at the ends of each range of lengths, with edges, in units that are short of rows, with masked rows in
+    every place of a unit and runs of them, rows whose gradient is zero, labels outside the vocabulary, in place."""
+    if rows * vocab > 2 ** 28:
+        rows = 8193
+    gen = torch.Generator(device=dev).manual_seed(vocab + rows)
+    z = (torch.randn(rows, vocab, generator=gen, device=dev) * 3).to(dtype)
+    z[5, ::7] = torch.finfo(dtype).min
+    z[6, 3] = float("-inf")
+    z[9] = 2.0                                                          # all alike
+    z[10, vocab // 2:] += 80.0                                          # far above a thread's first vector
+    y = torch.randint(0, vocab, (rows,), generator=gen, device=dev)
+    y[7], y[8], y[11], y[12] = -1, vocab, 0, vocab - 1
+    ops = torch.zeros(rows, 8, device=dev)
+    ops[:, 0] = -torch.rand(rows, generator=gen, device=dev) * 8        # old log-prob
+    ops[:, 1] = -torch.rand(rows, generator=gen, device=dev) * 8        # ref log-prob
+    ops[:, 2] = torch.randn(rows, generator=gen, device=dev)            # advantage
+    r = torch.arange(rows, device=dev)
+    ops[:, 3] = ((r % 5 != 2) & ((r // 37) % 3 != 1)).float()           # mask: single rows, whole units
+    ops[:, 4] = ops[:, 5] = 1.0 / rows
+
+    def sweep(entropy, ticket, out, scale=None):
+        terms = torch.full((rows, 8), 7.0, device=dev)
+        lp, ent = torch.full((rows,), 7.0, device=dev), torch.full((rows,), 7.0, device=dev)
+        z_in = out if out is not None else z
+        dz = out if out is not None else torch.full_like(z, 7.0)
+        _lib.call("mrl_fused_logprob_loss", z_in.data_ptr(), _lib.dtype_code(z), rows, vocab, vocab, y.data_ptr(), _lib.I64,
+                  1.0, ops.data_ptr(), 1, 0.8, 1.2, 3 if entropy else 0, 0.01, 0.002 if entropy else 0.0, 1.0, _lib.ptr(scale),
+                  dz.data_ptr(), vocab, lp.data_ptr(), ent.data_ptr() if entropy else None, terms.data_ptr(),
+                  _lib.ptr(ticket), 0 if ticket is None else 16, 0, _lib.stream(dev))
+        return dz.view(torch.int16 if dtype != torch.float32 else torch.int32), lp, ent, terms
+
+    counter = torch.empty(4, dtype=torch.int32, device=dev)
+    for entropy in (True, False):
+        want = sweep(entropy, None, None)
+        dead = (ops[:, 3] == 0)
+        assert not want[0][dead].any().item() and want[0][~dead].any().item()
+        for got in (sweep(entropy, counter, None), sweep(entropy, counter, z.clone())):
+            for a, b in zip(got, want):
+                assert torch.equal(a.nan_to_num(-5.0) if a.is_floating_point() else a,
+                                   b.nan_to_num(-5.0) if b.is_floating_point() else b)
+    if vocab % (16 // z.element_size()):                # rows with edges: the gradients once more at another scale
+        half = torch.tensor(0.5, device=dev)
+        want = sweep(True, None, None, half)[0]
+        carried, learned, dz = torch.tensor([1.0, 0.0], device=dev), torch.zeros((), device=dev), torch.full_like(z, 7.0)
+        _lib.call("mrl_fused_logprob_regrad", z.data_ptr(), _lib.dtype_code(z), rows, vocab, vocab, y.data_ptr(), _lib.I64, 1.0,
+                  ops.data_ptr(), 1, 0.8, 1.2, 3, 0.01, 0.002, 1.0, half.data_ptr(), carried.data_ptr(), learned.data_ptr(), None,
+                  0, dz.data_ptr(), vocab, counter.data_ptr(), 16, 0, _lib.stream(dev))
+        assert torch.equal(dz.view(want.dtype), want) and carried.tolist() == [0.5, 0.0] and learned.item() == 0.5
+
+
 @pytest.mark.parametrize("dtype,vocab", [(torch.float32, 152064), (torch.bfloat16, 262144)])
 def test_fused_sweep_wide_rows(dev, dtype, vocab):
     """Rows that two workgroups hold: more half rows than workgroups (tickets are recycled, partners
