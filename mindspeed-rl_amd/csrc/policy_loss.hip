@@ -29,27 +29,52 @@ __device__ __forceinline__ double block_sum(double v, double* lds) {
     return r;
 }
 
-// N sums at once, each as block_sum takes it: one pair of barriers for all of them.
-template <int N>
-__device__ __forceinline__ void block_sums(double (&v)[N], double (*lds)[kWaves]) {
+// x of the lane that a step of a reduction inside 16 lanes pairs with this one: quad_perm [1,0,3,2], [2,3,0,1],
+// row_half_mirror, row_mirror, each of which pairs groups that already agree.
+template <int kStep>
+__device__ __forceinline__ double lane_partner(double x) {
+    constexpr int kControl[4] = {0xB1, 0x4E, 0x141, 0x140};
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kControl[kStep], 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kControl[kStep], 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+
+template <int kSteps>
+__device__ __forceinline__ double lanes_sum(double x) {
+    x += lane_partner<0>(x);
+    x += lane_partner<1>(x);
+    if (kSteps > 2) x += lane_partner<2>(x);
+    if (kSteps > 3) x += lane_partner<3>(x);
+    return x;
+}
+
+__device__ __forceinline__ double lane_double(double x, int lane) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+
+// N sums at once over kCount wavefronts (4 or 16), in a fixed order; the FIRST wavefront gets them.  Inside a wavefront
+// by lane operands and scalar registers, not through the LDS crossbar, which took 84 shuffles of 32 bits for seven sums
+// from every wavefront: fused_seq_reduce_kernel with 1024 threads 15.0 -> 8.4 us (20 x 2 048 tokens), with 256 7.2 ->
+// 6.3 (16 x 1 024).
+template <int N, int kCount>
+__device__ __forceinline__ void block_sums(double (&v)[N], double (*lds)[kCount]) {
+    static_assert(kCount == 4 || kCount == 16, "partials of 4 or 16 wavefronts");
+    __syncthreads();                      // lds may still be read from the previous call
+    const int wave = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < N; ++q) {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+        const double x = lanes_sum<4>(v[q]);
+        v[q] = (lane_double(x, 0) + lane_double(x, 16)) + (lane_double(x, 32) + lane_double(x, 48));
+        if ((threadIdx.x & 63) == 0) lds[q][wave] = v[q];
     }
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) {
+    if (wave != 0) return;
 #pragma unroll
-        for (int q = 0; q < N; ++q) lds[q][threadIdx.x >> 6] = v[q];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < N; ++q) {
-        double r = 0.0;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) r += lds[q][w];
-        v[q] = r;
-    }
+    for (int q = 0; q < N; ++q) v[q] = lanes_sum<kCount == 16 ? 4 : 2>(lds[q][threadIdx.x & (kCount - 1)]);
 }
 constexpr int kSums = 7;                // the most that are taken at once
 
@@ -91,15 +116,15 @@ __global__ __launch_bounds__(kBlock) void policy_loss_rows_kernel(
 // Combines the per-sequence sums in a fixed order and writes the eight output scalars (and the loss
 // once more to loss_out, if given: a 0-dim tensor of its own for autograd).  kCoherent: the sums were
 // written by other workgroups of the SAME launch with device-scope stores and are read likewise.
-template <bool kCoherent>
+template <bool kCoherent, int kCount>
 __device__ __forceinline__ void finalize_sums(const float* row_sums, int64_t batch, const Params& p,
                                               float* __restrict__ out, float* __restrict__ loss_out,
-                                              float* __restrict__ host_out, double (*lds)[kWaves]) {
+                                              float* __restrict__ host_out, double (*lds)[kCount]) {
     auto at = [&](int64_t e) {
         return kCoherent ? __hip_atomic_load(row_sums + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : row_sums[e];
     };
     double tot[kSums] = {0, 0, 0, 0, 0, 0, 0};             // the six sums, and the sequences' means
-    for (int64_t i = threadIdx.x; i < batch; i += kBlock) {
+    for (int64_t i = threadIdx.x; i < batch; i += kCount * 64) {
         float v[6];
 #pragma unroll
         for (int q = 0; q < 6; ++q) {
@@ -204,23 +229,57 @@ __device__ __forceinline__ void seq_window(const SeqArgs& a, int64_t i, int64_t&
     if (n > a.width) n = a.width;
 }
 
+// Threads of a sequence's workgroup in the two kernels below, by the width alone.  A sequence is one workgroup's, so
+// few long ones leave the chip idle and what counts is how many of a thread's loads follow each other.  us, mask sums /
+// token sums, 256 threads and one load at a time -> now: 2 sequences x 16 384 tokens 13.0 -> 4.3 / 22.0 -> 11.8,
+// 8 x 4 096 6.3 -> 4.0 / 11.0 -> 8.9, 20 x 2 048 4.6 -> 3.8 / 8.6 -> 7.6, 32 x 512 3.2 -> 3.2 / 6.7 -> 6.0.  Below the
+// lines 1024 threads only add partials to combine (16 x 1 100 token sums 7.0 with 256, 8.2 with 1024).
+constexpr int kLongBlock = 1024;
+constexpr int64_t kLongMask = 1024, kLongTokens = 2048;
+
+// This thread's share of a row of `width` values, added up in the order of the columns, kDeep loads at a time.
+template <int kThreads, typename T>
+__device__ __forceinline__ float strided_sum(const T* __restrict__ row, int64_t width) {
+    constexpr int kDeep = 4;
+    float acc = 0.f;
+    for (int64_t j = threadIdx.x; j < width; j += kDeep * kThreads) {
+        T v[kDeep];
+#pragma unroll
+        for (int q = 0; q < kDeep; ++q) v[q] = j + q * kThreads < width ? row[j + q * kThreads] : T(0);
+#pragma unroll
+        for (int q = 0; q < kDeep; ++q) acc += (float)v[q];
+    }
+    return acc;
+}
+
 // One workgroup per sequence: its window and the sum of its mask row (the general form, for an
 // explicit mask tensor or very many sequences).
-__global__ __launch_bounds__(kBlock) void fused_seq_kernel(SeqArgs a, const void* __restrict__ mask, int mdtype,
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void fused_seq_kernel(SeqArgs a, const void* __restrict__ mask, int mdtype,
                                                            int64_t* __restrict__ row_start,
                                                            int32_t* __restrict__ row_count,
                                                            float* __restrict__ seq_msum) {
-    __shared__ double lds[kWaves];
+    __shared__ double lds[1][kThreads / 64];
     const int64_t i = blockIdx.x;
     float acc = 0.f;
-    for (int64_t j = threadIdx.x; j < a.width; j += kBlock) acc += mask_at(mask, mdtype, a.resp, a.rdtype, i, j, a.width);
-    const double msum = block_sum((double)acc, lds);
+    if (mask == nullptr) {
+        for (int64_t j = threadIdx.x; j < a.width; j += kThreads) acc += mask_at(mask, mdtype, a.resp, a.rdtype, i, j, a.width);
+    } else {
+        switch (mdtype) {
+            case MRL_F32: acc = strided_sum<kThreads>((const float*)mask + i * a.width, a.width); break;
+            case MRL_I32: acc = strided_sum<kThreads>((const int32_t*)mask + i * a.width, a.width); break;
+            case MRL_I64: acc = strided_sum<kThreads>((const int64_t*)mask + i * a.width, a.width); break;
+            default: acc = strided_sum<kThreads>((const uint8_t*)mask + i * a.width, a.width); break;
+        }
+    }
+    double msum[1] = {(double)acc};
+    block_sums(msum, lds);
     if (threadIdx.x == 0) {
         int64_t start, n;
         seq_window(a, i, start, n);
         row_start[i] = start;
         row_count[i] = (int32_t)n;
-        seq_msum[i] = (float)msum;
+        seq_msum[i] = (float)msum[0];
     }
 }
 
@@ -324,24 +383,40 @@ __global__ __launch_bounds__(kBlock) void fused_row_ops_kernel(
 // sequences' sums into the outputs (what policy_loss_finalize_kernel does in a launch of its own)
 // and leaves the counter at zero again.  The sums then travel with device-scope stores and loads,
 // which pass the caches that workgroups of one launch do not share.
-__global__ __launch_bounds__(kBlock) void fused_seq_reduce_kernel(
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void fused_seq_reduce_kernel(
     const float* __restrict__ row_terms, const int64_t* __restrict__ row_start, const int32_t* __restrict__ row_count,
     int64_t width, const float* __restrict__ old, const float* __restrict__ ref, const float* __restrict__ adv,
     const void* __restrict__ mask, int mdtype, const void* __restrict__ resp, int rdtype, Params p,
     float* row_sums, uint32_t* done, float* __restrict__ out, float* __restrict__ loss_out,
     float* __restrict__ host_out) {
-    __shared__ double lds[kSums][kWaves];
+    __shared__ double lds[kSums][kThreads / 64];
     __shared__ uint32_t last;
     const int64_t i = blockIdx.x;
     const int64_t start = row_start[i];
-    const int64_t count = row_count[i];
+    const int64_t count = row_count[i] < width ? row_count[i] : width;
     float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int64_t j = threadIdx.x; j < width; j += kBlock) {
-        if (j < count) {
-            const float* t = row_terms + (start + j) * S_N;
+    // tokens with a row: two 16-byte loads each, kDeep tokens of a thread at a time
+    constexpr int kDeep = 4;
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    const f4* terms = reinterpret_cast<const f4*>(row_terms + start * S_N);
+    const f4 none = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t j = threadIdx.x; j < count; j += kDeep * kThreads) {
+        f4 lo[kDeep], hi[kDeep];
 #pragma unroll
-            for (int q = 0; q < 6; ++q) acc[q] += t[q];
-        } else {
+        for (int u = 0; u < kDeep; ++u) {
+            const bool in = j + u * kThreads < count;
+            lo[u] = in ? terms[(j + u * kThreads) * 2] : none;
+            hi[u] = in ? terms[(j + u * kThreads) * 2 + 1] : none;
+        }
+#pragma unroll
+        for (int u = 0; u < kDeep; ++u) {
+            acc[0] += lo[u].x; acc[1] += lo[u].y; acc[2] += lo[u].z; acc[3] += lo[u].w;
+            acc[4] += hi[u].x; acc[5] += hi[u].y;
+        }
+    }
+    for (int64_t j = threadIdx.x; j < width; j += kThreads) {
+        if (j >= count) {
             const float m = mask_at(mask, mdtype, resp, rdtype, i, j, width);
             if (m == 0.f) continue;
             const int64_t e = i * width + j;
@@ -496,8 +571,12 @@ extern "C" int mrl_fused_loss_prepare(int layout, int64_t batch, int64_t width, 
     // the mask is implied by the response lengths and the sequences are few: one launch does it all
     const bool inline_tables = mask == nullptr && batch <= kInlineSeqs && n_rows > 0;
     if (batch > 0 && !inline_tables) {
-        hipLaunchKernelGGL(fused_seq_kernel, dim3((unsigned)batch), dim3(kBlock), 0, s, sa, mask, mask_dtype, row_start,
-                           row_count, seq_mask_sum);
+        if (width > kLongMask)
+            hipLaunchKernelGGL(fused_seq_kernel<kLongBlock>, dim3((unsigned)batch), dim3(kLongBlock), 0, s, sa, mask, mask_dtype,
+                               row_start, row_count, seq_mask_sum);
+        else
+            hipLaunchKernelGGL(fused_seq_kernel<kBlock>, dim3((unsigned)batch), dim3(kBlock), 0, s, sa, mask, mask_dtype,
+                               row_start, row_count, seq_mask_sum);
         int rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
@@ -548,9 +627,14 @@ extern "C" int mrl_fused_loss_reduce_host(const float* row_terms, const int64_t*
     const Params p = {clip_lo, clip_hi, kl_coef, entropy_coeff, loss_scale, kl_penalty, seq_mean};
     hipStream_t s = mrl::as_stream(stream);
     if (batch > 0) {
-        hipLaunchKernelGGL(fused_seq_reduce_kernel, dim3((unsigned)batch), dim3(kBlock), 0, s, row_terms, row_start,
-                           row_count, width, old_log_prob, ref_log_prob, advantages, mask, mask_dtype, response_length,
-                           response_dtype, p, row_sums, done_counter, out, loss_out, host_out);
+        if (width > kLongTokens)
+            hipLaunchKernelGGL(fused_seq_reduce_kernel<kLongBlock>, dim3((unsigned)batch), dim3(kLongBlock), 0, s, row_terms,
+                               row_start, row_count, width, old_log_prob, ref_log_prob, advantages, mask, mask_dtype,
+                               response_length, response_dtype, p, row_sums, done_counter, out, loss_out, host_out);
+        else
+            hipLaunchKernelGGL(fused_seq_reduce_kernel<kBlock>, dim3((unsigned)batch), dim3(kBlock), 0, s, row_terms,
+                               row_start, row_count, width, old_log_prob, ref_log_prob, advantages, mask, mask_dtype,
+                               response_length, response_dtype, p, row_sums, done_counter, out, loss_out, host_out);
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK || done_counter != nullptr) return rc;
     }

@@ -1530,6 +1530,53 @@ def test_fused_sweep_rows_side_by_side(dev, dtype, vocab, rows):
         assert torch.equal(dz.view(want.dtype), want) and carried.tolist() == [0.5, 0.0] and learned.item() == 0.5
 
 
+@pytest.mark.parametrize("width", [1, 255, 1024, 1025, 2048, 2049, 4097, 16384])
+@pytest.mark.parametrize("mask_dtype", [None, torch.float32, torch.int64, torch.int32, torch.uint8])
+def test_sequence_sums_by_width(dev, width, mask_dtype):
+    """Mask sums and token sums of sequences around the widths at which another workgroup size takes over, with tokens
+    behind the last row, against 64 bits: a thread adds up at most width / 256 + 1 terms in fp32 (64 above 2 048), the
+    rest is fp64 and one rounding."""
+    gen = torch.Generator().manual_seed(width)
+    batch = 3
+    count = torch.tensor([width, max(0, width - 5), width // 2], dtype=torch.int32)
+    start = torch.tensor([0, int(count[0]), int(count[:2].sum())], dtype=torch.int64)
+    terms = torch.rand(int(count.sum()) + 1, 8, generator=gen)
+    old, adv = -torch.rand(batch, width, generator=gen), torch.randn(batch, width, generator=gen)
+    resp = torch.full((batch,), width, dtype=torch.int32)
+    live = torch.ones(batch, width) if mask_dtype is None else (torch.rand(batch, width, generator=gen) < 0.7).float()
+    mask = None if mask_dtype is None else live.to(mask_dtype).to(dev)
+    code = _lib.I64 if mask is None else _lib.dtype_code(mask)
+    want = torch.zeros(batch, 6, dtype=torch.float64)
+    for i in range(batch):
+        n = int(count[i])
+        want[i] = terms[start[i]:start[i] + n, :6].double().sum(0)
+        m, o, a = live[i, n:].double(), old[i, n:].double(), adv[i, n:].double()        # no row: log-prob 0, entropy 0
+        ratio = torch.exp(-o)
+        pg, clipped = -a * ratio, -a * ratio.clamp(0.8, 1.2)
+        want[i] += torch.stack([(torch.maximum(pg, clipped) * m).sum(), ((clipped > pg) * m).sum(), (o * m).sum(),
+                                m.sum() * 0, m.sum() * 0, m.sum()])
+    sums, out = torch.empty(batch, 8, device=dev), torch.empty(8, device=dev)
+    td, sd, cd, od, ad, rd = (t.to(dev) for t in (terms, start, count, old, adv, resp))
+    _lib.call("mrl_fused_loss_reduce", td.data_ptr(), sd.data_ptr(), cd.data_ptr(), batch, width, od.data_ptr(), None,
+              ad.data_ptr(), _lib.ptr(mask), code, rd.data_ptr(), _lib.I32, 0.8, 1.2, 0, 0.0, 0.0, 0, 1.0, sums.data_ptr(),
+              out.data_ptr(), torch.zeros(1, dtype=torch.int32, device=dev).data_ptr(), None, _lib.stream(dev))
+    size = torch.maximum(want.abs(), torch.full_like(want, 1.0)) + 2 * width ** 0.5
+    assert ((sums[:, :6].cpu().double() - want).abs() <= 70 * 2.0 ** -24 * size).all()
+    assert abs(out[6].item() - want[:, 5].sum().item()) <= 70 * 2.0 ** -24 * (3 * width)
+    # the mask sums and windows of the prepare step
+    ones = torch.ones(batch, dtype=torch.int32, device=dev)
+    lens = (resp + 1).to(dev)
+    n_rows = batch * (width + 1)
+    cu = (torch.arange(batch + 1, dtype=torch.int32) * (width + 1)).to(dev)
+    rs, rc, ms = (torch.empty(batch, dtype=d, device=dev) for d in (torch.int64, torch.int32, torch.float32))
+    ops = torch.empty(n_rows, 8, device=dev)
+    _lib.call("mrl_fused_loss_prepare", 0, batch, width, n_rows, lens.data_ptr(), cu.data_ptr(), 0, ones.data_ptr(), _lib.I32,
+              rd.data_ptr(), _lib.I32, od.data_ptr(), None, ad.data_ptr(), _lib.ptr(mask), code, 0, rs.data_ptr(),
+              rc.data_ptr(), ms.data_ptr(), ops.data_ptr(), None, 0, None, 1.0, None, _lib.stream(dev))
+    assert torch.equal(ms.cpu(), live.sum(1)) and rc.tolist() == [width] * batch
+    assert torch.equal(ops.view(batch, width + 1, 8)[:, :width, 3].cpu(), live)
+
+
 @pytest.mark.parametrize("dtype,vocab", [(torch.float32, 152064), (torch.bfloat16, 262144)])
 def test_fused_sweep_wide_rows(dev, dtype, vocab):
     """Rows that two workgroups hold: more half rows than workgroups (tickets are recycled, partners
