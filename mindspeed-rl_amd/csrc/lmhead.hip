@@ -222,13 +222,17 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
     mfma_tile_loop<false, false>(smem, weight, hdim, vocab, hidden, hdim, n_tokens, hdim, seq, tile_stats);
 }
 
-// A workgroup finishes 16 tokens.  16 threads per token merge the leaves (thread q takes leaves q, q + 16,
-// ...; the loads of 16 neighbouring tokens are 64 contiguous bytes), then the 16 partial results are merged
-// in order; and one wavefront per token computes the label logit as an fp32 dot product of the token's
-// hidden row with the label's weight row.
+// A workgroup finishes 16 tokens.  One wavefront per token computes the label logit as an fp32 dot product of the
+// token's hidden row with the label's weight row; 16 threads per token, of the first four wavefronts, merge the leaves
+// (thread q takes leaves q, q + 16, ...; the loads of 16 neighbouring tokens are 64 contiguous bytes), then the 16
+// partial results are merged in order.  Few tokens are bound by the loads that follow each other, many by the rows'
+// bytes: a wavefront to each token up to kFewTokens, 4 tokens to one behind, us, 4 wavefronts and 512 entries at a time
+// -> now: 224 tokens x 3 072 14.2 -> 5.7, 589 x 4 224 17.6 -> 6.4, 4 000 x 1 024 10.6 -> 7.2, 7 100 x 3 776 19.6 -> 15.0,
+// 17 122 x 3 584 34.9 -> 32.8, 20 959 x 768 13.1 -> 13.6 (15.3 with a wavefront to each).
 constexpr int kFinishTokens = 16;
-template <typename LabelT, bool kEntropy>
-__global__ __launch_bounds__(256) void lmhead_finish_kernel(
+constexpr int64_t kFewTokens = 4096;
+template <typename LabelT, bool kEntropy, int kFinishWaves>
+__global__ __launch_bounds__(64 * kFinishWaves) void lmhead_finish_kernel(
     const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ weight, const LabelT* __restrict__ labels,
     const float* __restrict__ partial, int n_tokens, int vocab, int hdim, int n_leaves, float inv_t,
     const int32_t* __restrict__ cells, float* __restrict__ logp, float* __restrict__ entropy,
@@ -237,7 +241,7 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t0 = (int)blockIdx.x * kFinishTokens;
     const float k = inv_t * kLog2e;
-    {
+    if (wave < 4) {
         const int mine = threadIdx.x & 15, q = threadIdx.x >> 4;
         const int t = min(t0 + mine, n_tokens - 1);
         Stats r = {kMaxInit, 0.f, 0.f};
@@ -249,26 +253,46 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(
         }
         part[q][mine] = r;
     }
-    __syncthreads();
-    for (int i = wave; i < kFinishTokens; i += 4) {
-        const int t = t0 + i;
+    auto label_logit = [&](int t, float& dot, bool& y_ok) {
+        dot = 0.f;
+        y_ok = false;
         if (t >= n_tokens) return;
         const int64_t y = (int64_t)labels[t];
-        const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
-        float dot = 0.f;
-        if (y_ok) {
-            const uint16_t* hrow = hidden + (int64_t)t * hdim;
-            const uint16_t* wrow = weight + y * hdim;
-            for (int j = lane * 8; j < hdim; j += 64 * 8) {
-                const u32x4 hv = *reinterpret_cast<const u32x4*>(hrow + j);
-                const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + j);
+        y_ok = (y >= 0) && (y < (int64_t)vocab);
+        if (!y_ok) return;
+        const uint16_t* hrow = hidden + (int64_t)t * hdim;
+        const uint16_t* wrow = weight + y * hdim;
+        constexpr int kDeep = 4;                    // 2 x 4 loads on their way at a time
+        for (int at = 0; at < hdim; at += kDeep * 512) {            // 512 entries a wavefront and load
+            const int j = at + lane * 8;
+            u32x4 hv[kDeep], wv[kDeep];
+#pragma unroll
+            for (int d = 0; d < kDeep; ++d) {
+                if (at + d * 512 >= hdim) continue;                 // uniform
+                const bool in = j + d * 512 < hdim;
+                hv[d] = in ? *reinterpret_cast<const u32x4*>(hrow + j + d * 512) : mrl::make_u32x4(0u, 0u, 0u, 0u);
+                wv[d] = in ? *reinterpret_cast<const u32x4*>(wrow + j + d * 512) : mrl::make_u32x4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (int d = 0; d < kDeep; ++d) {
+                if (at + d * 512 >= hdim) continue;
                 float a[8], b[8];
-                Elem<MRL_BF16>::unpack(hv, a);
-                Elem<MRL_BF16>::unpack(wv, b);
+                Elem<MRL_BF16>::unpack(hv[d], a);
+                Elem<MRL_BF16>::unpack(wv[d], b);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(a[e], b[e], dot);
             }
         }
+    };
+    float dot;
+    bool y_ok;
+    constexpr bool kOne = kFinishWaves == kFinishTokens;        // the product need not wait for the leaves
+    if (kOne) label_logit(t0 + wave, dot, y_ok);
+    __syncthreads();
+    for (int i = wave; i < kFinishTokens; i += kFinishWaves) {
+        const int t = t0 + i;
+        if (t >= n_tokens) return;
+        if (!kOne) label_logit(t, dot, y_ok);
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
         Stats r = part[lane & 15][i];
@@ -354,7 +378,7 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
                            inv_temperature * kLog2e, partial);
         int rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
-        const dim3 fgrid((unsigned)((n + kFinishTokens - 1) / kFinishTokens)), fblock(256);
+        const dim3 fgrid((unsigned)((n + kFinishTokens - 1) / kFinishTokens)), fblock(n <= kFewTokens ? 1024 : 256);
         const int64_t out_lo = cells ? 0 : lo;
         float* ent = entropy ? entropy + out_lo : nullptr;
         float* lse_out = lse ? lse + out_lo : nullptr;
@@ -363,10 +387,17 @@ static int lmhead_forward(const char* fn, const void* hidden, const void* weight
             hipLaunchKernelGGL(kernel, fgrid, fblock, 0, s, h, (const uint16_t*)weight, lab + lo, (const float*)partial, n,
                                (int)vocab, (int)hidden_dim, leaves.n, inv_temperature, to, logp + out_lo, ent, lse_out);
         };
-        if (wide_labels)
-            finish(entropy ? lmhead_finish_kernel<int64_t, true> : lmhead_finish_kernel<int64_t, false>, (const int64_t*)labels);
-        else
-            finish(entropy ? lmhead_finish_kernel<int32_t, true> : lmhead_finish_kernel<int32_t, false>, (const int32_t*)labels);
+        auto finish_by_count = [&](auto* lab, auto with_entropy) {
+            using LabelT = std::remove_cv_t<std::remove_pointer_t<decltype(lab)>>;
+            if (n <= kFewTokens) finish(lmhead_finish_kernel<LabelT, decltype(with_entropy)::value, 16>, lab);
+            else finish(lmhead_finish_kernel<LabelT, decltype(with_entropy)::value, 4>, lab);
+        };
+        auto finish_by_label = [&](auto with_entropy) {
+            if (wide_labels) finish_by_count((const int64_t*)labels, with_entropy);
+            else finish_by_count((const int32_t*)labels, with_entropy);
+        };
+        if (entropy) finish_by_label(std::true_type());
+        else finish_by_label(std::false_type());
         rc = mrl::check_launch(fn);
         if (rc != MRL_OK) return rc;
     }
