@@ -20,7 +20,8 @@
 // groups of 32).
 //
 // dHidden has few tiles and a long K (the vocabulary): 162 tokens x 2 944 is 12 tiles on 256 CUs, 4 000 x 5 120
-// is 1.25 rounds of the chip.  Tiles behind the last whole round may therefore be cut along K into slices
+// is 1.25 rounds of the chip; dWeight of a small model over many tokens likewise.  Tiles behind the last whole round
+// may therefore be cut along K into slices
 // (plan_split); a slice leaves its fp32 sums in the caller's workspace and merge_slices_kernel adds them in
 // the order of the slices.  Units are numbered slice by slice, so the workgroups of an XCD still share operand
 // tiles.  Both backward products, uncut and cut: 300 x 32 000 x 1 024 557 -> 99 us, 1 380 x 152 064 x 3 584
@@ -89,10 +90,11 @@ constexpr int64_t kMaxSlices = 1024;                // of all tiles together: 25
 // through memory to the merge.  dHidden and dWeight together, uncut and in the slices it chooses, ms: 174 of 256
 // tiles (12 356 x 152 064 x 3 584) 20.55 and in 4 19.73 (in 3 20.76, in 5 19.98); 104 (9 000 x 152 064 x 2 560)
 // 12.33 and in 7 10.27; 144 (2 300 x 32 000 x 4 096) 1.118 and in 3 0.978.
-inline SplitPlan plan_split(int64_t total, int grid, int64_t n_ksteps) {
+// worth: the share of the whole product that a cut has to save.
+inline SplitPlan plan_split(int64_t total, int grid, int64_t n_ksteps, double worth) {
     SplitPlan p = {total / grid * grid, (int)(total % grid), 1};
     if (p.rest == 0) return p;
-    double best = (double)n_ksteps;
+    double best = (double)n_ksteps * (1.0 - worth * (double)(total / grid + 1));
     for (int64_t s = 2; s * p.rest <= kMaxSlices && s * 4 <= n_ksteps; ++s) {
         const int64_t rounds = (s * p.rest + grid - 1) / grid;
         const double cost = (double)rounds * ((double)((n_ksteps + s - 1) / s) + 10.0) + 0.1 * (double)(s * p.rest) + 10.0;
@@ -326,7 +328,30 @@ static SplitPlan whole_tiles(const Product& p) { return SplitPlan{make_grid(p.m,
 
 static SplitPlan plan_dhidden(int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
     const int grid = persistent_grid();
-    return plan_split(make_grid(hidden_dim, n_tokens).total, grid < 8 ? 1 : grid, (vocab + BK - 1) / BK);
+    return plan_split(make_grid(hidden_dim, n_tokens).total, grid < 8 ? 1 : grid, (vocab + BK - 1) / BK, 0.0);
+}
+
+// dWeight's last round is cut where that saves a twelfth of the product; else the sums stay those of the fp32
+// accumulation over chunks, rounded once.  us, uncut -> cut with its merge: 26 702 x 20 264 x 1 792 (560 tiles) 2 000
+// -> 1 559; 23 143 x 9 688 x 768 (114) 507 -> 292; 20 959 x 10 736 x 768 (126) 465 -> 274; 28 849 x 35 104 x 704 (414)
+// 1 405 -> 1 218; 13 058 x 8 488 x 512 (68) 291 -> 124; 5 000 x 19 776 x 2 560 (780) 432 -> 403.
+static SplitPlan plan_dweight(int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
+    const int grid = persistent_grid();
+    return plan_split(make_grid(hidden_dim, vocab).total, grid < 8 ? 1 : grid, (n_tokens + BK - 1) / BK, 1.0 / 12);
+}
+
+// The product with a k-major A, cut along k by the plan as far as the workspace reaches.
+template <bool kBTrans>
+static int cut_product(const char* fn, Product p, const SplitPlan& plan, void* workspace, int64_t workspace_bytes) {
+    if (plan.n_slices == 1 || workspace == nullptr || workspace_bytes < slice_bytes(plan))
+        return launch_gemm<kBf16, true, kBTrans, false>(fn, p, whole_tiles(p));
+    p.sums = reinterpret_cast<float*>(workspace);
+    int rc = plan.whole > 0 ? launch_gemm<kBf16, true, kBTrans, false>(fn, p, plan) : MRL_OK;
+    if (rc == MRL_OK) rc = launch_gemm<kF32, true, kBTrans, true>(fn, p, plan);
+    if (rc != MRL_OK) return rc;
+    hipLaunchKernelGGL(merge_slices_kernel, dim3((unsigned)plan.rest, BN / 16), dim3(256), 0, p.stream, p.sums, plan, (int)p.m,
+                       (int)p.n, (uint16_t*)p.out, p.ldo);
+    return check_launch(fn);
 }
 
 // dHidden[t][h] = sum_v W[v][h] * dlogits[t][v]: the weight as it lies is the k-major operand; its rows
@@ -336,24 +361,21 @@ static int dhidden(const char* fn, const void* weight, const void* dlogits, int6
                    int64_t vocab, int64_t hidden_dim, void* d_hidden, void* workspace, int64_t workspace_bytes,
                    hipStream_t s) {
     const Product p = {weight, hidden_dim, hidden_dim, dlogits, dlogits_row_stride, n_tokens, vocab, d_hidden, hidden_dim,
-                       reinterpret_cast<float*>(workspace), s};
-    const SplitPlan plan = plan_dhidden(n_tokens, vocab, hidden_dim);
-    if (plan.n_slices == 1 || workspace == nullptr || workspace_bytes < slice_bytes(plan))
-        return launch_gemm<kBf16, true, false, false>(fn, p, whole_tiles(p));
-    int rc = plan.whole > 0 ? launch_gemm<kBf16, true, false, false>(fn, p, plan) : MRL_OK;
-    if (rc == MRL_OK) rc = launch_gemm<kF32, true, false, true>(fn, p, plan);
-    if (rc != MRL_OK) return rc;
-    hipLaunchKernelGGL(merge_slices_kernel, dim3((unsigned)plan.rest, BN / 16), dim3(256), 0, s, p.sums, plan, (int)p.m,
-                       (int)p.n, (uint16_t*)p.out, p.ldo);
-    return check_launch(fn);
+                       nullptr, s};
+    return cut_product<false>(fn, p, plan_dhidden(n_tokens, vocab, hidden_dim), workspace, workspace_bytes);
 }
 
-// dW[v][h] (+)= sum_t hidden[t][h] * dlogits[t][v]: both operands k-major as they lie, any n_tokens
+// dW[v][h] (+)= sum_t hidden[t][h] * dlogits[t][v]: both operands k-major as they lie, any n_tokens; written as bf16 at
+// once, cut along the tokens as far as the workspace reaches
 template <int kOut>
 static int dweight(const char* fn, const void* hidden, const void* dlogits, int64_t dlogits_row_stride, int64_t n_tokens,
-                   int64_t vocab, int64_t hidden_dim, void* out, float* sums, hipStream_t s) {
+                   int64_t vocab, int64_t hidden_dim, void* out, float* sums, void* workspace, int64_t workspace_bytes,
+                   hipStream_t s) {
     const Product p = {hidden, hidden_dim, hidden_dim, dlogits, dlogits_row_stride, vocab, n_tokens, out, hidden_dim, sums, s};
-    return launch_gemm<kOut, true, true, false>(fn, p, whole_tiles(p));
+    if constexpr (kOut == kBf16)
+        return cut_product<true>(fn, p, plan_dweight(n_tokens, vocab, hidden_dim), workspace, workspace_bytes);
+    else
+        return launch_gemm<kOut, true, true, false>(fn, p, whole_tiles(p));
 }
 
 static int check_bwd(const char* fn, int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
@@ -398,12 +420,15 @@ extern "C" int mrl_lmhead_logprob_bwd(const void* hidden, const void* weight, co
     hipStream_t s = mrl::as_stream(stream);
     rc = mrl::dhidden(fn, weight, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_hidden, nullptr, 0, s);
     if (rc != MRL_OK) return rc;
-    return mrl::dweight<kF32Add>(fn, hidden, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_weight, d_weight, s);
+    return mrl::dweight<kF32Add>(fn, hidden, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_weight, d_weight, nullptr, 0, s);
 }
 
 extern "C" int64_t mrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t hidden_dim) {
     if (n_tokens <= 0 || vocab <= 0 || hidden_dim <= 0) return 0;
-    return mrl::slice_bytes(mrl::plan_dhidden(n_tokens, vocab, hidden_dim));
+    // one after the other
+    const int64_t h = mrl::slice_bytes(mrl::plan_dhidden(n_tokens, vocab, hidden_dim));
+    const int64_t w = mrl::slice_bytes(mrl::plan_dweight(n_tokens, vocab, hidden_dim));
+    return h > w ? h : w;
 }
 
 extern "C" int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weight, const void* dlogits,
@@ -421,7 +446,7 @@ extern "C" int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weig
                       workspace_bytes, s);
     if (rc != MRL_OK) return rc;
 #define MRL_DWEIGHT(OUT, dst) \
-    mrl::dweight<OUT>(fn, hidden, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, dst, d_weight_sums, s)
+    mrl::dweight<OUT>(fn, hidden, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, dst, d_weight_sums, workspace, workspace_bytes, s)
     if (first) return last ? MRL_DWEIGHT(kBf16, d_weight) : MRL_DWEIGHT(kF32, d_weight_sums);
     return last ? MRL_DWEIGHT(kSumToBf16, d_weight) : MRL_DWEIGHT(kF32Add, d_weight_sums);
 #undef MRL_DWEIGHT

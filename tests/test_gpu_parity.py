@@ -3504,6 +3504,38 @@ def test_lmhead_backward_chunk(dev, tokens, vocab, hdim):
         assert torch.equal(again, dh) and torch.equal(dw, dw32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("tokens,vocab,hdim", [(6001, 8200, 512), (9000, 1000, 64), (5040, 19784, 2560), (12345, 8200, 264)])
+def test_lmhead_dweight_cut_along_the_tokens(dev, tokens, vocab, hdim):
+    """dWeight of one chunk whose last round of tiles (or all of them, ragged ones) is cut along the tokens, against 64
+    bits and the uncut call: one rounding to bf16 (2^-8 of the value at most) and fp32 sums of `tokens` products of
+    spread sqrt(tokens); not further from 64 bits than the uncut call; dHidden is the same either way."""
+    g = torch.Generator(device=dev).manual_seed(tokens + vocab)
+    v_pad = (vocab + 63) // 64 * 64
+    h = torch.randn(tokens, hdim, generator=g, device=dev).to(torch.bfloat16)
+    w = torch.randn(vocab, hdim, generator=g, device=dev).to(torch.bfloat16)
+    dz = torch.zeros(tokens, v_pad, dtype=torch.bfloat16, device=dev)
+    dz[:, :vocab] = torch.randn(tokens, vocab, generator=g, device=dev)
+    lib, stream = _lib.load(), _lib.stream(dev)
+    need = lib.mrl_lmhead_bwd_workspace_bytes(tokens, vocab, hdim)
+    assert need > 0 and need % (256 * 256 * 4) == 0
+    ws = torch.full((need + 64,), 0xFF, dtype=torch.uint8, device=dev)      # NaNs, should a slice not be written
+    outs = []
+    for ws_bytes in (need, 0, need):
+        dh, dw = torch.full_like(h, 7.0), torch.full_like(w, 7.0)
+        _lib.call("mrl_lmhead_logprob_bwd_chunk", h.data_ptr(), w.data_ptr(), dz.data_ptr(), v_pad, tokens, vocab, hdim,
+                  dh.data_ptr(), dw.data_ptr(), None, 1, 1, ws.data_ptr() if ws_bytes else None, ws_bytes, stream)
+        outs.append((dh, dw))
+    torch.cuda.synchronize()
+    assert (ws[need:] == 0xFF).all().item()
+    assert torch.equal(outs[0][1], outs[2][1]) and torch.equal(outs[0][0], outs[2][0])
+    cut, uncut = outs[0][1].double(), outs[1][1].double()
+    want = dz[:, :vocab].double().t().contiguous() @ h.double()
+    assert not torch.equal(cut, uncut), "nothing was cut"
+    assert ((cut - want).abs() <= 2 ** -8 * want.abs() + 1e-5 * tokens ** 0.5).all().item()
+    assert (cut - want).norm().item() <= 1.001 * (uncut - want).norm().item()
+    assert ((outs[0][0].float() - outs[1][0].float()).abs() <= 2 ** -7 * outs[1][0].float().abs() + 2e-5 * vocab ** 0.5).all().item()
+
+
 @pytest.mark.parametrize("hdim", [8, 264])
 @pytest.mark.parametrize("tokens", [1, 31, 32, 33, 63, 65, 96, 97, 127, 129, 193])
 def test_lmhead_products_at_the_edges_of_a_slot(dev, tokens, hdim):
