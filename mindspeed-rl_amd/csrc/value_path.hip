@@ -34,9 +34,33 @@ __device__ __forceinline__ double block_sum(double x, double* lds) {
     return lds[kWaves];
 }
 
+// Three of them at once: the same sums in the same order, one pair of barriers (value_loss_finish_kernel 3.7 -> 3.1 us,
+// whiten_moments_kernel 4.6 -> 4.2 with three calls before).
+__device__ __forceinline__ void block_sum3(double (&x)[3], double (*lds)[kReduceBlock / 64 + 1]) {
+    constexpr int kWaves = kReduceBlock / 64;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) x[q] += __shfl_xor(x[q], off, 64);
+        if ((threadIdx.x & 63) == 0) lds[q][threadIdx.x >> 6] = x[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) t += lds[threadIdx.x][w];
+        lds[threadIdx.x][kWaves] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 3; ++q) x[q] = lds[q][kWaves];
+}
+
 // ---------------------------------------------------------------------------- KL-penalised rewards
 // One workgroup per sample: kld = penalty(old, ref) * mask, rewards = onehot(last response token) *
-// score - beta * kld, row_kl = sum(kld * mask) / (sum(mask) + 1e-8).
+// score - beta * kld, row_kl = sum(kld * mask) / (sum(mask) + 1e-8).  A thread has four columns on their way at a time:
+// bound by loads that follow each other, 122 x 4 096 8.4 -> 6.6 us, 128 x 2 048 5.5 -> 4.9.
+constexpr int kColumns = 4;
 __global__ __launch_bounds__(256) void kl_rewards_kernel(const float* __restrict__ old_lp,
                                                          const float* __restrict__ ref_lp,
                                                          const void* __restrict__ lens, int ldtype,
@@ -53,14 +77,25 @@ __global__ __launch_bounds__(256) void kl_rewards_kernel(const float* __restrict
     const float score = scores[i];
     Params p = {0.f, 0.f, 0.f, 0.f, 1.f, penalty, 0};
     double acc = 0.0;
-    for (int64_t j = threadIdx.x; j < width; j += 256) {
-        const int64_t e = i * width + j;
-        const float m = j < n ? 1.f : 0.f;
-        const Token t = token_terms<false>(old_lp[e], 0.f, false, ref_lp[e], 0.f, p);
-        const float kld = t.kl * m;
-        const float r = j == hot ? score : 0.f;
-        rewards[e] = r - beta * kld;
-        if (m != 0.f) acc += (double)(kld * m);
+    for (int64_t j0 = threadIdx.x; j0 < width; j0 += kColumns * 256) {
+        float old_mine[kColumns], ref_mine[kColumns];
+#pragma unroll
+        for (int q = 0; q < kColumns; ++q) {
+            const int64_t e = i * width + (j0 + q * 256 < width ? j0 + q * 256 : j0);
+            old_mine[q] = old_lp[e];
+            ref_mine[q] = ref_lp[e];
+        }
+#pragma unroll
+        for (int q = 0; q < kColumns; ++q) {
+            const int64_t j = j0 + q * 256;
+            if (j >= width) break;
+            const float m = j < n ? 1.f : 0.f;
+            const Token t = token_terms<false>(old_mine[q], 0.f, false, ref_mine[q], 0.f, p);
+            const float kld = t.kl * m;
+            const float r = j == hot ? score : 0.f;
+            rewards[i * width + j] = r - beta * kld;
+            if (m != 0.f) acc += (double)(kld * m);
+        }
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
@@ -278,7 +313,7 @@ __global__ __launch_bounds__(kReduceBlock) void whiten_moments_kernel(float* __r
                                                                      const Moments* __restrict__ moments,
                                                                      int64_t n_moments, int64_t n,
                                                                      double* __restrict__ info) {
-    __shared__ double lds[kReduceBlock / 64 + 1];
+    __shared__ double lds[3][kReduceBlock / 64 + 1];
     Moments mom = {0.0, 0.0, 0.0};
     for (int64_t i = threadIdx.x; i < n_moments; i += kReduceBlock) {
         const Moments o = moments[i];
@@ -286,7 +321,9 @@ __global__ __launch_bounds__(kReduceBlock) void whiten_moments_kernel(float* __r
         mom.x += o.x;
         mom.xx += o.xx;
     }
-    const double count = block_sum(mom.w, lds), total = block_sum(mom.x, lds), squares = block_sum(mom.xx, lds);
+    double sums[3] = {mom.w, mom.x, mom.xx};
+    block_sum3(sums, lds);
+    const double count = sums[0], total = sums[1], squares = sums[2];
     const float fc = (float)count, denom = fc + 1e-8f;
     const float mean = (float)total / denom;
     const double md = (double)mean;
@@ -449,11 +486,12 @@ __global__ __launch_bounds__(kReduceBlock) void value_loss_finish_kernel(const L
                                                                         float loss_scale, float* __restrict__ out,
                                                                         float* __restrict__ loss_out,
                                                                         float* __restrict__ host_out) {
-    __shared__ double lds[kReduceBlock / 64 + 1];
+    __shared__ double lds[3][kReduceBlock / 64 + 1];
     LossSums s = {0.0, 0.0, 0.0};
     if ((int)threadIdx.x < n) s = sums[threadIdx.x];       // n <= kLossRows = kReduceBlock
-    const double ssum = block_sum(s.loss, lds), csum = block_sum(s.clipped, lds), count = block_sum(s.count, lds);
-    if (threadIdx.x == 0) write_value_loss(ssum, csum, count, loss_scale, out, loss_out, host_out);
+    double all[3] = {s.loss, s.clipped, s.count};
+    block_sum3(all, lds);
+    if (threadIdx.x == 0) write_value_loss(all[0], all[1], all[2], loss_scale, out, loss_out, host_out);
 }
 static_assert(kLossRows == kReduceBlock, "the finishing workgroup takes one partial sum per thread");
 
