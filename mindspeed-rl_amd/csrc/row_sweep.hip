@@ -1047,10 +1047,19 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
 //   fp32 (half the entries per byte to compute): 32 KB 3 802 -> 5 599, 48 KB 4 859 -> 6 205, 64 KB 5 832 -> 6 083;
 //          96 and 128 KB stay with 1024 x 8 (6 190 and 6 250 against 5 800 and 5 700 with 512 x 16);
 //          34 KB 5 361 with 512 x 12, 39 KB 6 046: up to there 256 x 12, which takes rows side by side
+// Vectors of a thread that lie past the row are computed on all the same, so that a shape with fewer is the faster one,
+// the more so with the entropy's sum and with few rows, which wait for a single row's chain; which thread holds what is
+// as in the larger shape, and with it every bit.  512 x 12 -> 512 x 8, without and with entropy, GB/s of 1 GB of logits
+// and us of 600 rows: 24 640 bf16 5 680 -> 5 985 and 5 232 -> 5 743, 19.6 -> 17.5 and 20.4 -> 15.9; 32 000 5 910 ->
+// 5 927 and 5 843 -> 5 874, 20.4 -> 19.4; 12 000 fp32 6 090 -> 6 195, 18.0 -> 17.1.  Its registers leave room for three
+// workgroups per CU, which pays where all rows start at once; with more rows three move less than two (32 000 bf16
+// 5 624, 12 000 fp32 5 815), hence the limit in launch_sweep.  1024 x 12 -> 1024 x 10 with entropy: 66 000 bf16 5 427 ->
+// 5 561, 42.2 -> 40.3; 1024 x 16 -> 1024 x 14: 100 352 5 853 -> 5 916, 55.6 -> 53.1.  512 x 10 and 512 x 14 changed
+// nothing but 2 to 3 % of few rows.
 // The choice depends on the row's length alone, so a row's result does not depend on the other rows' contents.
 // Its place does enter for rows that are not whole 128-byte lines (see RowSpan): which thread adds which entry
 // follows from the row's address modulo 128, so the fp32 sums round differently at another place in the batch.
-enum Shape { k256x4, k256x8, k256x12, k512x12, k512x16, k1024x8, k1024x12, k1024x16, k1024x19, kTooLong };
+enum Shape { k256x4, k256x8, k256x12, k512x8, k512x12, k512x16, k1024x8, k1024x10, k1024x12, k1024x14, k1024x16, k1024x19, kTooLong };
 constexpr int64_t kMaxVec = 19 * 1024;              // vectors of the widest row that one workgroup holds
 
 inline Shape pick_shape(int dtype, int64_t n_vec) {
@@ -1058,14 +1067,17 @@ inline Shape pick_shape(int dtype, int64_t n_vec) {
     if (n_vec <= 2048) return k256x8;
     if (dtype == MRL_F32) {
         if (n_vec <= 2496) return k256x12;
-        if (n_vec <= 4096) return k512x12;
+        if (n_vec <= 4096) return k512x8;
         if (n_vec <= 8192) return k1024x8;
     } else {
         if (n_vec <= 3072) return k256x12;
+        if (n_vec <= 4096) return k512x8;
         if (n_vec <= 6144) return k512x12;
         if (n_vec <= 8192) return k512x16;
     }
+    if (n_vec <= 10240) return k1024x10;
     if (n_vec <= 12288) return k1024x12;
+    if (n_vec <= 14336) return k1024x14;
     if (n_vec <= 16384) return k1024x16;
     return n_vec <= kMaxVec ? k1024x19 : kTooLong;
 }
@@ -1139,7 +1151,9 @@ int launch_sweep(const mrl::FusedArgs& a) {
         const int cus = cu_count();
         if (cus < 2) return mrl::fail(MRL_ERR_LAUNCH, "mrl_fused_logprob_loss: cannot query the device");
         // half rows: an even number of workgroups, so that the halves of a row start side by side
-        const int64_t cap = kWide ? (cus & ~1) : (int64_t)cus * (waves_per_simd(NV, kRows) * 4 / (BLK * kRows / 64));
+        int64_t per_cu = waves_per_simd(NV, kRows) * 4 / (BLK * kRows / 64);
+        if (BLK == 512 && NV == 8 && rows > per_cu * cus) per_cu = 2;       // see pick_shape
+        const int64_t cap = kWide ? (cus & ~1) : (int64_t)cus * per_cu;
         // Rows per ticket: the counter serves about 85 tickets per microsecond, rows below 32 KiB go faster
         // than that (8 000 bf16 logits, rows per ticket 1 / 2 / 4: 2 728 / 5 085 / 5 276 GB/s for 155 648 rows,
         // 1 819 / 2 537 / 2 479 for 2 048; 16 384: 5 241 / 5 481 / 5 294; 24 576: 5 681 / 5 466 / 5 253).
@@ -1187,14 +1201,17 @@ int fused_by_shape(Shape shape, SideBySide side, const mrl::FusedArgs& a) {
         if (side.rows == 2 && side.vectors == 7) return launch_narrow<DT, 256, 7, 2>(a);
         if (side.rows == 2 && side.vectors == 8) return launch_narrow<DT, 256, 8, 2>(a);
         if (side.rows == 2) return launch_narrow<DT, 256, 10, 2>(a);
+        if (shape == k512x12) return launch_narrow<DT, 512, 12>(a);
         if (shape == k512x16) return launch_narrow<DT, 512, 16>(a);
     }
     if (side.rows == 4) return launch_narrow<DT, 256, 4, 4>(a);
     if (shape == k256x4) return launch_narrow<DT, 256, 4>(a);
     if (shape == k256x8) return launch_narrow<DT, 256, 8>(a);
     if (shape == k256x12) return launch_narrow<DT, 256, 12>(a);
-    if (shape == k512x12) return launch_narrow<DT, 512, 12>(a);
+    if (shape == k512x8) return launch_narrow<DT, 512, 8>(a);
+    if (shape == k1024x10) return launch_1024<DT, 10>(a);
     if (shape == k1024x12) return launch_1024<DT, 12>(a);
+    if (shape == k1024x14) return launch_1024<DT, 14>(a);
     if (shape == k1024x16) return launch_1024<DT, 16>(a);
     return launch_1024<DT, 19>(a);
 }

@@ -1530,6 +1530,52 @@ def test_fused_sweep_rows_side_by_side(dev, dtype, vocab, rows):
         assert torch.equal(dz.view(want.dtype), want) and carried.tolist() == [0.5, 0.0] and learned.item() == 0.5
 
 
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 24580), (torch.float16, 24584), (torch.bfloat16, 32003), (torch.bfloat16, 32768),
+                                         (torch.float32, 9988), (torch.float32, 14001), (torch.float32, 16384), (torch.bfloat16, 65544),
+                                         (torch.bfloat16, 81920), (torch.float16, 98312), (torch.bfloat16, 114691),
+                                         (torch.float32, 40960), (torch.float32, 57344)])
+@pytest.mark.parametrize("rows", [7, 770, 1300])
+def test_fused_sweep_shapes_that_fit_the_row(dev, dtype, vocab, rows):
+    """The ends of the lengths that 512 x 8, 1024 x 10 and 1024 x 14 hold, with fewer rows than start at once and more:
+    log-probs, entropies and gradients against 64 bits, in place as well, masked rows zero."""
+    gen = torch.Generator(device=dev).manual_seed(vocab + rows)
+    z = (torch.randn(rows, vocab, generator=gen, device=dev) * 3).to(dtype)
+    y = torch.randint(0, vocab, (rows,), generator=gen, device=dev)
+    y[0], y[1] = 0, vocab - 1
+    live = torch.arange(rows, device=dev) % 5 != 3
+    ops = torch.zeros(rows, 8, device=dev)
+    ops[:, 2], ops[:, 3], ops[:, 4], ops[:, 5] = 1.0, live.float(), 1.0, 1.0      # no old log-prob: a ratio of 1
+    counter = torch.empty(4, dtype=torch.int32, device=dev)
+
+    def sweep(out, entropy):
+        z_in, dz = (out, out) if out is not None else (z, torch.full_like(z, 7.0))
+        terms, lp, ent = torch.empty(rows, 8, device=dev), torch.empty(rows, device=dev), torch.empty(rows, device=dev)
+        _lib.call("mrl_fused_logprob_loss", z_in.data_ptr(), _lib.dtype_code(z), rows, vocab, vocab, y.data_ptr(), _lib.I64,
+                  1.0, ops.data_ptr(), 0, 0.8, 1.2, 0, 0.0, 0.01 if entropy else 0.0, 1.0, None, dz.data_ptr(), vocab,
+                  lp.data_ptr(), ent.data_ptr() if entropy else None, terms.data_ptr(), counter.data_ptr(), 16, 0, _lib.stream(dev))
+        return dz, lp, ent
+
+    # fp32 sums of at most 152 terms a thread and 20 steps behind them, and exponents rounded to 2^-19 of themselves
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 4e-5}[dtype]
+    tiny = 2.0 ** -24 if dtype is torch.float16 else 0.0
+    for entropy in (False, True):
+        dz, lp, ent = sweep(None, entropy)
+        again = sweep(z.clone(), entropy)
+        assert torch.equal(again[0], dz) and torch.equal(again[1], lp)
+        assert not dz[~live].any().item()
+        for lo in range(0, rows, 256):
+            part, on = slice(lo, lo + 256), live[lo:lo + 256]
+            logp = torch.log_softmax(z[part][on].double(), -1)
+            p, at = logp.exp(), y[part][on][:, None]
+            assert (lp[part][on].double() - logp.gather(-1, at)[:, 0]).abs().max().item() < 2e-5
+            want = p.scatter_add(-1, at, torch.full_like(at, -1.0, dtype=torch.float64))
+            if entropy:
+                h = -(p * logp).sum(-1, keepdim=True)
+                assert (ent[part][on].double() - h[:, 0]).abs().max().item() < 2e-4
+                want += 0.01 * p * (logp + h)
+            assert ((dz[part][on].double() - want).abs() <= want.abs() * (unit + 4e-5) + 4e-5 * p + tiny + 1e-12).all().item()
+
+
 @pytest.mark.parametrize("width", [1, 255, 1024, 1025, 2048, 2049, 4097, 16384])
 @pytest.mark.parametrize("mask_dtype", [None, torch.float32, torch.int64, torch.int32, torch.uint8])
 def test_sequence_sums_by_width(dev, width, mask_dtype):
