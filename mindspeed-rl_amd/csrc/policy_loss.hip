@@ -627,7 +627,8 @@ extern "C" int mrl_fused_loss_reduce_host(const float* row_terms, const int64_t*
     const Params p = {clip_lo, clip_hi, kl_coef, entropy_coeff, loss_scale, kl_penalty, seq_mean};
     hipStream_t s = mrl::as_stream(stream);
     if (batch > 0) {
-        if (width > kLongTokens)
+        // (a launch has fewer than 2^32 threads)
+        if (width > kLongTokens && batch <= 0xffffffffLL / kLongBlock)
             hipLaunchKernelGGL(fused_seq_reduce_kernel<kLongBlock>, dim3((unsigned)batch), dim3(kLongBlock), 0, s, row_terms,
                                row_start, row_count, width, old_log_prob, ref_log_prob, advantages, mask, mask_dtype,
                                response_length, response_dtype, p, row_sums, done_counter, out, loss_out, host_out);

@@ -75,14 +75,14 @@ struct WindowCells {
 template <int DT, typename LabelT, bool kEntropy, int kBlk, int kDeep, typename Rows>
 __global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
     const typename Elem<DT>::T* __restrict__ logits, int64_t row_stride, int vocab,
-    const LabelT* __restrict__ labels, Rows rows, float inv_t,
+    const LabelT* __restrict__ labels, Rows rows, uint32_t first, float inv_t,
     float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int kVec = E::kVec;
     __shared__ Stats lds[kBlk / 64];
 
-    const int64_t out = blockIdx.x, r = rows.row(out);
+    const int64_t out = first + blockIdx.x, r = rows.row(out);
     if (r < 0) {
         if (threadIdx.x == 0) {
             logp[out] = 0.f;
@@ -345,15 +345,21 @@ struct FwdArgs {
 template <int DT, typename LabelT, int kBlk, int kDeep, typename Rows>
 int launch_fwd_shape(const char* fn, const FwdArgs& a, const Rows& rows) {
     using T = typename Elem<DT>::T;
-    const dim3 grid((unsigned)a.n_out), block(kBlk);
+    // a launch has fewer than 2^32 threads: more rows or cells (of a window mostly empty ones) take several
+    constexpr int64_t kMost = 0xffffffffLL / kBlk;
+    for (int64_t first = 0; first < a.n_out; first += kMost) {
+        const dim3 grid((unsigned)(a.n_out - first < kMost ? a.n_out - first : kMost)), block(kBlk);
 #define MRL_FWD_LAUNCH(ENT)                                                                                           \
     hipLaunchKernelGGL((vocab_fwd_kernel<DT, LabelT, ENT, kBlk, kDeep, Rows>), grid, block, 0, a.stream,              \
-                       (const T*)a.logits, a.row_stride, (int)a.vocab, (const LabelT*)a.labels, rows, a.inv_t, a.logp, \
-                       a.entropy, a.lse)
-    if (a.with_entropy) MRL_FWD_LAUNCH(true);
-    else MRL_FWD_LAUNCH(false);
+                       (const T*)a.logits, a.row_stride, (int)a.vocab, (const LabelT*)a.labels, rows, (uint32_t)first, \
+                       a.inv_t, a.logp, a.entropy, a.lse)
+        if (a.with_entropy) MRL_FWD_LAUNCH(true);
+        else MRL_FWD_LAUNCH(false);
 #undef MRL_FWD_LAUNCH
-    return mrl::check_launch(fn);
+        const int rc = mrl::check_launch(fn);
+        if (rc != MRL_OK) return rc;
+    }
+    return MRL_OK;
 }
 
 // Threads of a row's workgroup and vectors a thread and round, by the row's length alone, so that a row's result
@@ -413,7 +419,7 @@ int check_common(const char* fn, const void* logits, int logits_dtype, int64_t n
                  int64_t row_stride, const void* labels, int labels_dtype, float inv_t) {
     MRL_REQUIRE(n_rows >= 0 && vocab > 0, MRL_ERR_INVALID_ARG, "%s: n_rows=%lld vocab=%lld", fn,
                 (long long)n_rows, (long long)vocab);
-    MRL_REQUIRE(n_rows <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED, "%s: n_rows=%lld exceeds the grid limit", fn,
+    MRL_REQUIRE(n_rows <= 0x7fffffffLL, MRL_ERR_UNSUPPORTED, "%s: n_rows=%lld exceeds 2^31 - 1", fn,
                 (long long)n_rows);
     MRL_REQUIRE(vocab <= (1LL << 30), MRL_ERR_UNSUPPORTED, "%s: vocab=%lld exceeds 2^30", fn, (long long)vocab);
     const int eb = mrl::float_dtype_bytes(logits_dtype);
@@ -464,7 +470,7 @@ extern "C" int mrl_window_logprob(const void* logits, int logits_dtype, int64_t 
                                response_length, response_dtype};
     rc = mrl::check_seq_windows(fn, q, batch, width, n_rows);
     if (rc != MRL_OK || batch == 0 || width == 0) return rc;
-    MRL_REQUIRE(width <= 0x7fffffffLL / batch, MRL_ERR_UNSUPPORTED, "%s: batch=%lld x width=%lld exceeds the grid limit", fn,
+    MRL_REQUIRE(width <= 0x7fffffffLL / batch, MRL_ERR_UNSUPPORTED, "%s: batch=%lld x width=%lld exceeds 2^31 - 1", fn,
                 (long long)batch, (long long)width);
     MRL_REQUIRE(logp && entropy, MRL_ERR_INVALID_ARG, "%s: NULL output", fn);
     MRL_REQUIRE(mrl::aligned(logp, 4) && mrl::aligned(entropy, 4), MRL_ERR_MISALIGNED, "%s: fp32 outputs misaligned", fn);

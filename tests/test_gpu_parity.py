@@ -3317,6 +3317,31 @@ def test_forward_sweep_by_row_length(dev, dtype, vectors):
             assert (got.double() - want).abs().max().item() <= bound * scale, (vocab, stride)
 
 
+@pytest.mark.parametrize("vocab,batch", [(65536, 513), (32000, 1025)])
+def test_scoring_pass_over_more_cells_than_a_launch_holds(dev, vocab, batch):
+    """Windows of 8 192 columns whose cells, at the 1024 or 512 threads that a row of this length takes, are more than
+    2^32 threads (a launch has fewer): the few live ones come out as the flagged rows do, bit for bit, the rest zero."""
+    width, live = 8192, torch.arange(batch, device=dev) % 3                 # 0, 1 or 2 cells of a sequence
+    threads = 1024 if vocab // 8 > 7168 else 512
+    assert (batch - 1) * width * threads == 2 ** 32
+    seqlens = (live + 1).to(torch.int32)                                    # a prompt of one token
+    cu = torch.cat([torch.zeros(1, device=dev), torch.cumsum(seqlens, 0)]).to(torch.int32)
+    n_rows = int(cu[-1])
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    z = torch.randn(n_rows, vocab, generator=gen, device=dev).to(torch.bfloat16)
+    y = torch.randint(0, vocab, (n_rows,), generator=gen, device=dev)
+    ones = torch.ones(batch, dtype=torch.int32, device=dev)
+    got = torch.full((2, batch, width), 7.0, device=dev)
+    _lib.call("mrl_window_logprob", z.data_ptr(), _lib.BF16, n_rows, vocab, vocab, y.data_ptr(), _lib.I64, 1.0, 0, batch,
+              width, seqlens.data_ptr(), cu.data_ptr(), 0, ones.data_ptr(), _lib.I32, None, _lib.I32, 1,
+              got[0].data_ptr(), got[1].data_ptr(), _lib.stream(dev))
+    lp, ent, _ = mrl.vocab_logprob_entropy(z, y)
+    cells = torch.arange(width, device=dev) < live[:, None]
+    rows = (cu[:-1, None] + torch.arange(width, device=dev))[cells].long()
+    assert torch.equal(got[0][cells], lp[rows]) and torch.equal(got[1][cells], ent[rows])
+    assert not got[:, ~cells].any().item()
+
+
 @pytest.mark.parametrize("layout", ["padded", "packed"])
 @pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1000), (torch.bfloat16, 1003), (torch.float32, 4096),
                                          (torch.float32, 77), (torch.float16, 8200)])
