@@ -55,42 +55,77 @@ struct RowSplit {
 // a workgroup that reads.  505 of 1 208 padded rows x 32 000 bf16 48 -> 19 us a pass, 133 rows x 8 000 45 -> 20;
 // 60 779 rows x 8 000 185 -> 175; the sweep itself is bound by memory as before.
 struct FlaggedRows {
+    static constexpr int kCells = 1;
     const uint8_t* active;          // NULL: all
     __device__ __forceinline__ int64_t row(int64_t out) const { return active != nullptr && active[out] == 0 ? -1 : out; }
 };
 
+// The window of a sequence that is the same for the whole workgroup; its lengths are requested together.
+__device__ __forceinline__ void uniform_window(const mrl::SeqWindows& w, uint32_t i, int64_t& start, int64_t& n) {
+    if (!w.packed) return w.window(i, start, n);
+    int32_t first = w.cu[i], length = w.seqlens[i];
+    int64_t prompt = mrl::load_index(w.prompt, w.prompt_dtype, i);
+    asm volatile("" : "+s"(first), "+s"(length), "+s"(prompt));
+    const bool inside = prompt - 1 < length;
+    start = inside ? first + prompt - 1 : first;
+    n = inside ? length - prompt : length;
+}
+
 struct WindowCells {
+    static constexpr int kCells = 1;
     mrl::SeqWindows seqs;
     uint32_t width;
     int64_t n_rows;
     __device__ __forceinline__ int64_t row(int64_t out) const {
         const uint32_t i = (uint32_t)out / width, j = (uint32_t)out - i * width;
         int64_t start, n;
-        seqs.window(i, start, n);
+        uniform_window(seqs, i, start, n);
         const int64_t t = start + j;
         return (int64_t)j < n && t >= 0 && t < n_rows ? t : -1;
     }
 };
 
-template <int DT, typename LabelT, bool kEntropy, int kBlk, int kDeep, typename Rows>
-__global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
+// Many cells (see launch_fwd_shape).  An empty one keeps a workgroup's registers for the microsecond that the loads of
+// its window take, and a CU has room for two workgroups of 1024 threads but eight of 256: a pass over windows with few
+// live cells consists of that.  So a workgroup of 512 or 1024 threads takes kCells = 2 or 4 cells of a sequence, a half
+// or quarter of the width apart: the live ones are the first, and fall to different workgroups.
+template <int kOfUnit>
+struct ManyCells {
+    static constexpr int kCells = kOfUnit;
+    mrl::SeqWindows seqs;
+    uint32_t width, step;           // step: units of a sequence, width / kCells rounded up
+    int64_t n_rows;
+    struct Unit {
+        int64_t first, start, n;    // of the sequence: its first cell, its window
+        uint32_t j;
+    };
+    __device__ __forceinline__ Unit unit(uint32_t u) const {
+        const uint32_t i = u / step;
+        Unit r;
+        r.j = u - i * step;
+        r.first = (int64_t)i * width;
+        uniform_window(seqs, i, r.start, r.n);
+        return r;
+    }
+    // whether there is a cell c of the unit; its place and the row that it reads
+    __device__ __forceinline__ bool cell(const Unit& u, int c, int64_t& out, int64_t& row) const {
+        const uint32_t j = u.j + (uint32_t)c * step;
+        const int64_t t = u.start + j;
+        out = u.first + j;
+        row = (int64_t)j < u.n && t >= 0 && t < n_rows ? t : -1;
+        return j < width;
+    }
+};
+
+// Log-prob, entropy and log-sum-exp of row r, by the whole workgroup.
+template <int DT, typename LabelT, bool kEntropy, int kBlk, int kDeep>
+__device__ __forceinline__ void score_row(
     const typename Elem<DT>::T* __restrict__ logits, int64_t row_stride, int vocab,
-    const LabelT* __restrict__ labels, Rows rows, uint32_t first, float inv_t,
-    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
+    const LabelT* __restrict__ labels, int64_t r, int64_t out, float inv_t,
+    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out, Stats* lds) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int kVec = E::kVec;
-    __shared__ Stats lds[kBlk / 64];
-
-    const int64_t out = first + blockIdx.x, r = rows.row(out);
-    if (r < 0) {
-        if (threadIdx.x == 0) {
-            logp[out] = 0.f;
-            if (entropy) entropy[out] = 0.f;
-            if (lse_out) lse_out[out] = 0.f;
-        }
-        return;
-    }
     const T* row = logits + r * row_stride;
     const float k = inv_t * kLog2e;
 
@@ -181,6 +216,42 @@ __global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
         if (kEntropy) entropy[out] = lse - (tot.u / tot.s) * inv_t;
         else if (entropy) entropy[out] = 0.f;
         if (lse_out) lse_out[out] = lse;
+    }
+}
+
+template <int DT, typename LabelT, bool kEntropy, int kBlk, int kDeep, typename Rows>
+__global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
+    const typename Elem<DT>::T* __restrict__ logits, int64_t row_stride, int vocab,
+    const LabelT* __restrict__ labels, Rows rows, uint32_t first, float inv_t,
+    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out) {
+    __shared__ Stats lds[kBlk / 64];
+    auto no_row = [&](int64_t out) {
+        logp[out] = 0.f;
+        if (entropy) entropy[out] = 0.f;
+        if (lse_out) lse_out[out] = 0.f;
+    };
+    auto score = [&](int64_t r, int64_t out) {
+        score_row<DT, LabelT, kEntropy, kBlk, kDeep>(logits, row_stride, vocab, labels, r, out, inv_t, logp, entropy, lse_out, lds);
+    };
+    if constexpr (Rows::kCells == 1) {
+        const int64_t out = first + blockIdx.x, r = rows.row(out);
+        if (r < 0) {
+            if (threadIdx.x == 0) no_row(out);
+            return;
+        }
+        score(r, out);
+    } else {
+        const auto unit = rows.unit(first + blockIdx.x);
+        int64_t out, r;
+        if (threadIdx.x < Rows::kCells && rows.cell(unit, (int)threadIdx.x, out, r) && r < 0) no_row(out);
+        if (unit.n <= (int64_t)unit.j) return;          // then no later one has a row either
+#pragma unroll 1
+        for (int c = 0; c < Rows::kCells; ++c) {
+            if (!rows.cell(unit, c, out, r)) return;
+            if (r < 0) continue;
+            score(r, out);
+            __syncthreads();                // the partials have been read
+        }
     }
 }
 
@@ -336,19 +407,19 @@ struct FwdArgs {
     const void* logits; int logits_dtype; int64_t vocab, row_stride;
     const void* labels; int labels_dtype;
     float inv_t;
-    int64_t n_out;                  // workgroups: rows or cells
+    int64_t n_out;                  // rows or cells
     bool with_entropy;
     float *logp, *entropy, *lse;
     hipStream_t stream;
 };
 
 template <int DT, typename LabelT, int kBlk, int kDeep, typename Rows>
-int launch_fwd_shape(const char* fn, const FwdArgs& a, const Rows& rows) {
+int launch_fwd_units(const char* fn, const FwdArgs& a, const Rows& rows, int64_t n_units) {
     using T = typename Elem<DT>::T;
     // a launch has fewer than 2^32 threads: more rows or cells (of a window mostly empty ones) take several
     constexpr int64_t kMost = 0xffffffffLL / kBlk;
-    for (int64_t first = 0; first < a.n_out; first += kMost) {
-        const dim3 grid((unsigned)(a.n_out - first < kMost ? a.n_out - first : kMost)), block(kBlk);
+    for (int64_t first = 0; first < n_units; first += kMost) {
+        const dim3 grid((unsigned)(n_units - first < kMost ? n_units - first : kMost)), block(kBlk);
 #define MRL_FWD_LAUNCH(ENT)                                                                                           \
     hipLaunchKernelGGL((vocab_fwd_kernel<DT, LabelT, ENT, kBlk, kDeep, Rows>), grid, block, 0, a.stream,              \
                        (const T*)a.logits, a.row_stride, (int)a.vocab, (const LabelT*)a.labels, rows, (uint32_t)first, \
@@ -360,6 +431,30 @@ int launch_fwd_shape(const char* fn, const FwdArgs& a, const Rows& rows) {
         if (rc != MRL_OK) return rc;
     }
     return MRL_OK;
+}
+
+template <int DT, typename LabelT, int kBlk, int kDeep>
+int launch_fwd_shape(const char* fn, const FwdArgs& a, const FlaggedRows& rows) {
+    return launch_fwd_units<DT, LabelT, kBlk, kDeep>(fn, a, rows, a.n_out);
+}
+
+// A cell to a workgroup, or several: where most of the cells are known to be empty, or so many that their rows, should
+// they all have one, keep the chip busy either way.  us a pass over bf16 windows, with 256 threads and a cell each / 512
+// or 1024 and a cell each / as it is: 256 x 8 192 cells with 7 rows to a sequence, 152 064 logits 1 123 / 4 351 / 1 174,
+// 32 000 1 057 / 2 122 / 990; 16 x 2 048 with 255, 65 536 86 / 135 / 87; all with rows, 16 x 2 048, 152 064 1 425 /
+// 1 408 / 1 409, 32 000 306 / 298 / 298.  Several cells over fewer of them leave CUs idle: 2 500 with rows x 152 064 118 /
+// 112 / 124, 10 000 x 65 536 191 / 187 / 194; with rows for one in ten they do not, 4 x 1 024 x 152 064 32 / 29 / 23.
+template <int DT, typename LabelT, int kBlk, int kDeep>
+int launch_fwd_shape(const char* fn, const FwdArgs& a, const WindowCells& w) {
+    if constexpr (kBlk > 256) {
+        constexpr int kCells = kBlk / 256;
+        if (a.n_out >= 16384 || (a.n_out >= 4096 && a.n_out >= 4 * w.n_rows)) {
+            const uint32_t step = (w.width + kCells - 1) / kCells;
+            const ManyCells<kCells> rows = {w.seqs, w.width, step, w.n_rows};
+            return launch_fwd_units<DT, LabelT, kBlk, kDeep>(fn, a, rows, a.n_out / w.width * step);
+        }
+    }
+    return launch_fwd_units<DT, LabelT, kBlk, kDeep>(fn, a, w, a.n_out);
 }
 
 // Threads of a row's workgroup and vectors a thread and round, by the row's length alone, so that a row's result

@@ -3342,6 +3342,37 @@ def test_scoring_pass_over_more_cells_than_a_launch_holds(dev, vocab, batch):
     assert not got[:, ~cells].any().item()
 
 
+@pytest.mark.parametrize("vocab", [28680, 57352])
+@pytest.mark.parametrize("batch,width", [(7, 2343), (3, 5462), (4, 1021), (5, 1025), (5000, 1), (2100, 3)])
+def test_scoring_pass_over_many_cells(dev, vocab, batch, width):
+    """Windows of so many cells, or so many empty ones, that a workgroup of 512 or 1024 threads takes several of them:
+    every cell as the flagged rows give it, bit for bit, zeros elsewhere - widths that do not divide, empty and full
+    windows beside each other, windows behind the rows, labels outside the vocabulary."""
+    gen = torch.Generator().manual_seed(batch * width + vocab)
+    n = torch.randint(0, max(2, width // 12), (batch,), generator=gen) if width > 3 else torch.randint(0, width + 1, (batch,), generator=gen)
+    n[0], n[-1] = 0, width if width < 1100 else width // 3
+    if width == 1025:
+        n[2] = width                                    # all of it: several rows to a workgroup
+    seqlens = (n + 1).to(torch.int32)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(seqlens, 0)]).to(torch.int32)
+    n_rows = int(cu[-1]) - 3                            # the last window ends behind the rows
+    z = torch.randn(n_rows, vocab, generator=torch.Generator(device=dev).manual_seed(vocab), device=dev).to(torch.bfloat16)
+    y = torch.randint(-1, vocab + 1, (n_rows,), generator=gen).to(dev)
+    ones = torch.ones(batch, dtype=torch.int32, device=dev)
+    seqlens_d, cu_d = seqlens.to(dev), cu.to(dev)
+    for entropy in (0, 1):
+        got = torch.full((2, batch, width), 7.0, device=dev)
+        _lib.call("mrl_window_logprob", z.data_ptr(), _lib.BF16, n_rows, vocab, vocab, y.data_ptr(), _lib.I64, 1.0, 0, batch,
+                  width, seqlens_d.data_ptr(), cu_d.data_ptr(), 0, ones.data_ptr(), _lib.I32, None, _lib.I32, entropy,
+                  got[0].data_ptr(), got[1].data_ptr(), _lib.stream(dev))
+        lp, ent, _ = mrl.vocab_logprob_entropy(z, y, want_entropy=bool(entropy))
+        rows = cu[:-1, None].long() + torch.arange(width)
+        cells = ((torch.arange(width) < n[:, None]) & (rows < n_rows)).to(dev)
+        rows = rows.to(dev)[cells]
+        assert torch.equal(got[0][cells], lp[rows]) and not got[:, ~cells].any().item()
+        assert torch.equal(got[1][cells], ent[rows]) if entropy else not got[1].any().item()
+
+
 @pytest.mark.parametrize("layout", ["padded", "packed"])
 @pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1000), (torch.bfloat16, 1003), (torch.float32, 4096),
                                          (torch.float32, 77), (torch.float16, 8200)])
