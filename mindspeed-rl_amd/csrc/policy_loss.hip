@@ -58,8 +58,7 @@ __device__ __forceinline__ double lane_double(double x, int lane) {
 
 // N sums at once over kCount wavefronts (4 or 16), in a fixed order; the FIRST wavefront gets them.  Inside a wavefront
 // by lane operands and scalar registers, not through the LDS crossbar, which took 84 shuffles of 32 bits for seven sums
-// from every wavefront: fused_seq_reduce_kernel with 1024 threads 15.0 -> 8.4 us (20 x 2 048 tokens), with 256 7.2 ->
-// 6.3 (16 x 1 024).
+// from every wavefront: fused_seq_reduce_kernel of 256 threads 7.2 -> 6.3 us (16 x 1 024 tokens).
 template <int N, int kCount>
 __device__ __forceinline__ void block_sums(double (&v)[N], double (*lds)[kCount]) {
     static_assert(kCount == 4 || kCount == 16, "partials of 4 or 16 wavefronts");
@@ -229,13 +228,17 @@ __device__ __forceinline__ void seq_window(const SeqArgs& a, int64_t i, int64_t&
     if (n > a.width) n = a.width;
 }
 
-// Threads of a sequence's workgroup in the two kernels below, by the width alone.  A sequence is one workgroup's, so
-// few long ones leave the chip idle and what counts is how many of a thread's loads follow each other.  us, mask sums /
-// token sums, 256 threads and one load at a time -> now: 2 sequences x 16 384 tokens 13.0 -> 4.3 / 22.0 -> 11.8,
-// 8 x 4 096 6.3 -> 4.0 / 11.0 -> 8.9, 20 x 2 048 4.6 -> 3.8 / 8.6 -> 7.6, 32 x 512 3.2 -> 3.2 / 6.7 -> 6.0.  Below the
-// lines 1024 threads only add partials to combine (16 x 1 100 token sums 7.0 with 256, 8.2 with 1024).
+// Threads of a sequence's workgroup in the two kernels below.  A sequence is one workgroup's, so few long ones leave the
+// chip idle and what counts is how many of a thread's loads follow each other; of many, and of token sums up to 4 096,
+// 1024 threads only add partials to combine.  us, 256 threads and one load at a time -> as it is (256 threads and four
+// loads where the lines give 1024, or the other way round): mask sums, 2 sequences x 16 384 16.4 -> 4.7, 8 x 4 096 6.5 ->
+// 3.6 (4.8), 20 x 2 048 4.5 -> 3.3 (3.8), 32 x 512 3.2 -> 3.0, 1 024 x 2 049 5.2 -> 4.4 (5.8), 2 048 x 1 100 5.4 -> 4.6
+// (8.5); token sums, 2 x 16 384 16.0 -> 11.2, 64 x 8 192 11.8 -> 10.0, 8 x 4 096 9.1 -> 8.2 (8.8), 256 x 2 049 10.2 -> 9.5
+// (11.0), 20 x 2 048 7.6 -> 6.7.  Token sums go by the width alone, so that a sequence's do not depend on the others; sums
+// of zeros and ones are exact whichever way they are taken.
 constexpr int kLongBlock = 1024;
-constexpr int64_t kLongMask = 1024, kLongTokens = 2048;
+constexpr int64_t kLongSeq = 4096;
+inline bool long_mask_rows(int64_t batch, int64_t width) { return width > (batch <= 512 ? 1024 : kLongSeq); }
 
 // This thread's share of a row of `width` values, added up in the order of the columns, kDeep loads at a time.
 template <int kThreads, typename T>
@@ -571,7 +574,7 @@ extern "C" int mrl_fused_loss_prepare(int layout, int64_t batch, int64_t width, 
     // the mask is implied by the response lengths and the sequences are few: one launch does it all
     const bool inline_tables = mask == nullptr && batch <= kInlineSeqs && n_rows > 0;
     if (batch > 0 && !inline_tables) {
-        if (width > kLongMask)
+        if (long_mask_rows(batch, width))
             hipLaunchKernelGGL(fused_seq_kernel<kLongBlock>, dim3((unsigned)batch), dim3(kLongBlock), 0, s, sa, mask, mask_dtype,
                                row_start, row_count, seq_mask_sum);
         else
@@ -628,7 +631,7 @@ extern "C" int mrl_fused_loss_reduce_host(const float* row_terms, const int64_t*
     hipStream_t s = mrl::as_stream(stream);
     if (batch > 0) {
         // (a launch has fewer than 2^32 threads)
-        if (width > kLongTokens && batch <= 0xffffffffLL / kLongBlock)
+        if (width > kLongSeq && batch <= 0xffffffffLL / kLongBlock)
             hipLaunchKernelGGL(fused_seq_reduce_kernel<kLongBlock>, dim3((unsigned)batch), dim3(kLongBlock), 0, s, row_terms,
                                row_start, row_count, width, old_log_prob, ref_log_prob, advantages, mask, mask_dtype,
                                response_length, response_dtype, p, row_sums, done_counter, out, loss_out, host_out);

@@ -1576,12 +1576,12 @@ def test_fused_sweep_shapes_that_fit_the_row(dev, dtype, vocab, rows):
             assert ((dz[part][on].double() - want).abs() <= want.abs() * (unit + 4e-5) + 4e-5 * p + tiny + 1e-12).all().item()
 
 
-@pytest.mark.parametrize("width", [1, 255, 1024, 1025, 2048, 2049, 4097, 16384])
+@pytest.mark.parametrize("width", [1, 255, 1024, 1025, 2048, 2049, 4096, 4097, 16384])
 @pytest.mark.parametrize("mask_dtype", [None, torch.float32, torch.int64, torch.int32, torch.uint8])
 def test_sequence_sums_by_width(dev, width, mask_dtype):
     """Mask sums and token sums of sequences around the widths at which another workgroup size takes over, with tokens
-    behind the last row, against 64 bits: a thread adds up at most width / 256 + 1 terms in fp32 (64 above 2 048), the
-    rest is fp64 and one rounding."""
+    behind the last row, against 64 bits: a thread adds up at most width / 256 + 1 terms in fp32 (width / 1024 + 1 above
+    4 096), the rest is fp64 and one rounding.  (Without a mask few sequences are counted in fused_row_ops_kernel.)"""
     gen = torch.Generator().manual_seed(width)
     batch = 3
     count = torch.tensor([width, max(0, width - 5), width // 2], dtype=torch.int32)
@@ -1621,6 +1621,56 @@ def test_sequence_sums_by_width(dev, width, mask_dtype):
               rc.data_ptr(), ms.data_ptr(), ops.data_ptr(), None, 0, None, 1.0, None, _lib.stream(dev))
     assert torch.equal(ms.cpu(), live.sum(1)) and rc.tolist() == [width] * batch
     assert torch.equal(ops.view(batch, width + 1, 8)[:, :width, 3].cpu(), live)
+
+
+@pytest.mark.parametrize("batch,width,mask_dtype", [(2049, 1024, None), (2050, 1025, None), (2050, 4096, None), (2051, 4097, None),
+                                                    (512, 1025, torch.int64), (513, 1025, torch.float32),
+                                                    (513, 4097, torch.uint8), (1025, 4097, torch.int64), (1500, 4096, torch.int32)])
+@pytest.mark.parametrize("seq_mean", [0, 1])
+def test_sequence_sums_of_many_sequences(dev, batch, width, mask_dtype, seq_mean):
+    """More sequences than the finishing workgroup has threads, or than are counted in fused_row_ops_kernel without a
+    mask: mask sums and windows exactly, all eight outputs against 64 bits.  All terms are positive: a thread adds up at
+    most width / 256 + 1 = 17 of them in fp32, then one rounding of a sequence's sum, of each mean and of the loss."""
+    gen = torch.Generator(device=dev).manual_seed(batch + width)
+    count = torch.randint(1, 40, (batch,), generator=gen, device=dev)
+    count[torch.randperm(batch, generator=torch.Generator().manual_seed(1))[:40].to(dev)] = width
+    start = torch.cumsum(count, 0) - count
+    terms = torch.rand(int(count.sum()), 8, generator=gen, device=dev)
+    terms[:, 5] = 1.0                                                       # the mask
+    live = torch.arange(width, device=dev) < count[:, None]
+    mask = None if mask_dtype is None else live.to(mask_dtype)
+    code = _lib.I64 if mask is None else _lib.dtype_code(mask)
+    zeros = torch.zeros(batch, width, device=dev)
+    sums, out = torch.empty(batch, 8, device=dev), torch.empty(8, device=dev)
+    counter, loss = torch.zeros(1, dtype=torch.int32, device=dev), torch.empty((), device=dev)
+    rows = count.to(torch.int32)
+    for _ in range(2):                                                      # the counter is zero again
+        _lib.call("mrl_fused_loss_reduce", terms.data_ptr(), start.data_ptr(), rows.data_ptr(), batch, width, zeros.data_ptr(),
+                  zeros.data_ptr(), zeros.data_ptr(), _lib.ptr(mask), code, count.data_ptr(), _lib.I64, 0.8, 1.2,
+                  _lib.KL_KL, 0.25, 0.125, seq_mean, 0.5, sums.data_ptr(), out.data_ptr(), counter.data_ptr(), loss.data_ptr(),
+                  _lib.stream(dev))
+    of_seq = torch.zeros(batch, 6, dtype=torch.float64, device=dev)
+    of_seq.index_add_(0, torch.repeat_interleave(torch.arange(batch, device=dev), count), terms[:, :6].double())
+    assert ((sums[:, :6].double() - of_seq).abs() <= 19 * 2.0 ** -24 * of_seq).all().item()
+    tot = of_seq.sum(0)
+    pg = (of_seq[:, 0] / of_seq[:, 5]).mean() if seq_mean else tot[0] / tot[5]
+    kl, ent = tot[3] / tot[5], tot[4] / tot[5]
+    want = torch.stack([0.5 * (pg + 0.25 * kl - 0.125 * ent), pg + 0.25 * kl - 0.125 * ent, tot[1] / tot[5] * (1 - seq_mean),
+                        tot[2] / tot[5], kl, ent, tot[5], torch.full_like(pg, batch)])
+    size = torch.stack([pg + kl + ent, pg + kl + ent, *want[2:]])
+    assert ((out.double() - want).abs() <= 25 * 2.0 ** -24 * size).all().item() and loss.item() == out[0].item()
+    assert out[6].item() == int(count.sum()) and out[7].item() == batch and counter.item() == 0
+    # the mask sums and windows of the prepare step
+    n_rows = batch * 3
+    lens = torch.full((batch,), 3, dtype=torch.int32, device=dev)
+    cu = torch.arange(batch + 1, dtype=torch.int32, device=dev) * 3
+    ones = torch.ones(batch, dtype=torch.int32, device=dev)
+    rs, rc, ms = (torch.empty(batch, dtype=d, device=dev) for d in (torch.int64, torch.int32, torch.float32))
+    ops = torch.empty(n_rows, 8, device=dev)
+    _lib.call("mrl_fused_loss_prepare", 0, batch, width, n_rows, lens.data_ptr(), cu.data_ptr(), 0, ones.data_ptr(), _lib.I32,
+              count.data_ptr(), _lib.I64, zeros.data_ptr(), None, zeros.data_ptr(), _lib.ptr(mask), code, 0, rs.data_ptr(),
+              rc.data_ptr(), ms.data_ptr(), ops.data_ptr(), None, 0, None, 1.0, None, _lib.stream(dev))
+    assert torch.equal(ms, count.float()) and (rc == 2).all().item() and torch.equal(rs, cu[:-1].long())
 
 
 @pytest.mark.parametrize("dtype,vocab", [(torch.float32, 152064), (torch.bfloat16, 262144)])
