@@ -441,6 +441,8 @@ extern "C" int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weig
     MRL_REQUIRE(n_tokens > 0, MRL_ERR_INVALID_ARG, "%s: an empty chunk", fn);
     MRL_REQUIRE(hidden && weight && dlogits && d_hidden && (d_weight || !last) && (d_weight_sums || (first && last)),
                 MRL_ERR_INVALID_ARG, "%s: NULL pointer", fn);
+    MRL_REQUIRE(mrl::aligned(workspace, 16) && mrl::aligned(d_weight_sums, 16), MRL_ERR_MISALIGNED,
+                "%s: the workspace and d_weight_sums must be 16-byte aligned", fn);
     hipStream_t s = mrl::as_stream(stream);
     rc = mrl::dhidden(fn, weight, dlogits, dlogits_row_stride, n_tokens, vocab, hidden_dim, d_hidden, workspace,
                       workspace_bytes, s);

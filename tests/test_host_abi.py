@@ -205,6 +205,16 @@ def test_argument_validation_launches_nothing():
     assert err.value.code == -1 and "multiple of 16" in str(err.value)
 
 
+@pytest.mark.parametrize("first,last", [(1, 1), (1, 0), (0, 0), (0, 1)])
+def test_lmhead_backward_refuses_misaligned_sums(first, last):
+    """A workspace or sums that are not 16-byte aligned are refused whether or not a product is cut, before any launch."""
+    lib = _lib.load()
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) + 15) // 16 * 16
+    for workspace, n_bytes, sums in ((p + 4, 0, p), (p + 8, 1 << 28, p), (None, 0, p + 4), (p, 1 << 28, p + 8)):
+        assert lib.mrl_lmhead_logprob_bwd_chunk(p, p, p, 128, 4, 128, 64, p, p, sums, first, last, workspace, n_bytes, None) == -3
+
+
 def test_cpu_tensors_are_refused_loudly():
     z = torch.randn(2, 8)
     with pytest.raises(RuntimeError, match="no CPU fallback"):
