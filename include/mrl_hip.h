@@ -557,7 +557,7 @@ int mrl_lmhead_logprob_fwd_cells(const void* hidden, const void* weight, int64_t
  *
  * hidden [n_tokens, hidden_dim] and weight [vocab, hidden_dim] are dense bf16, hidden_dim % 64 == 0,
  * vocab % 8 == 0; logits / dlogits rows are logits_row_stride / dlogits_row_stride apart.  The
- * backward reads hidden, weight and dlogits as they lie (no transposed copies, no workspace); it
+ * backward reads hidden, weight and dlogits as they lie (no transposed copies); it
  * wants dlogits_row_stride a multiple of 64 (and at least vocab) with zeros in the padding columns,
  * since it reads whole steps of 64 columns; n_tokens is arbitrary.  dWeight is accumulated chunk
  * after chunk in stream order, without atomics, so the result does not depend on timing.  Nothing
@@ -571,13 +571,17 @@ int mrl_lmhead_logprob_bwd(const void* hidden, const void* weight, const void* d
 /* The same two products for one chunk of a step whose dWeight ends as bf16 [vocab, hidden_dim]: the first
  * chunk overwrites d_weight_sums (fp32, need not be cleared), the chunks between add to it, the last adds
  * to it and writes the sum to d_weight; a chunk that is both first and last writes d_weight at once
- * (d_weight_sums may be NULL).  Every entry is rounded once, as by mrl_lmhead_logprob_bwd and a conversion.
- * workspace (nullable): mrl_lmhead_bwd_workspace_bytes(n_tokens, vocab, hidden_dim) bytes, 16-byte aligned,
- * for dHidden tiles that are cut along the vocabulary when they do not fill the chip (0 bytes where they
- * do); with NULL or fewer bytes none is cut.  dHidden is the same to rounding either way: cut tiles group
- * their fp32 sums by slices, whose number follows from n_tokens, so a token's dHidden then differs in its
- * rounding with the number of tokens beside it; uncut it depends on neither that nor the chunking.
- * n_tokens > 0. */
+ * (d_weight_sums may be NULL).  Every entry is rounded to bf16 once.
+ * workspace (nullable): mrl_lmhead_bwd_workspace_bytes(n_tokens, vocab, hidden_dim) bytes, at most 256 MiB,
+ * 16-byte aligned, for tiles that are cut when they do not fill the chip: dHidden's along the vocabulary and,
+ * in a chunk that is both first and last and where it saves a twelfth of the product, dWeight's along the
+ * tokens.  The two use it one after the other and the size is what the larger needs, 0 where neither is cut
+ * (the size does not know of first and last: other chunks leave dWeight's part alone); a product for which
+ * the bytes given (0 with NULL) do not suffice is not cut.  Both results are the same to rounding either way:
+ * cut tiles group their fp32 sums by slices, whose number follows from n_tokens, so the last bits depend on
+ * whether a workspace is given and, for a token's dHidden, on the number of tokens beside it; uncut, dHidden
+ * depends on neither that nor the chunking, and dWeight equals that of mrl_lmhead_logprob_bwd into zeros,
+ * converted.  n_tokens > 0. */
 int64_t mrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t hidden_dim);
 int mrl_lmhead_logprob_bwd_chunk(const void* hidden, const void* weight, const void* dlogits,
                                  int64_t dlogits_row_stride, int64_t n_tokens, int64_t vocab,

@@ -246,9 +246,9 @@ class _FusedLmHeadLoss(torch.autograd.Function):
         if v_pad != vocab:
             logits[:, vocab:].zero_()
         d_hidden = torch.empty_like(h2d)
-        # dWeight leaves the last chunk's product as bf16; fp32 sums exist only between chunks.  dHidden of a
-        # step in one chunk may be cut along the vocabulary; in several it never is, so that it does not
-        # depend on the chunking.
+        # dWeight leaves the last chunk's product as bf16; fp32 sums exist only between chunks.  In a step of one
+        # chunk dHidden may be cut along the vocabulary and dWeight along the tokens, which groups their fp32 sums
+        # by the number of rows; in several neither is, so that dHidden does not depend on the chunking.
         one_chunk = n_rows <= chunk
         d_weight = torch.empty((vocab, hdim), dtype=w.dtype, device=dev) if n_rows > 0 else torch.zeros_like(w)
         d_weight32 = None if one_chunk else torch.empty((vocab, hdim), dtype=torch.float32, device=dev)
