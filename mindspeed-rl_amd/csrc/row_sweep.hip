@@ -130,13 +130,67 @@ __device__ __forceinline__ float grad_elem(const RowGrad& g, float z) {
     return e * w;
 }
 
-// Vectors that are complete for every thread of a row that the host gives to a workgroup of BLK threads
-// with NV vectors each (see pick_shape for the shortest such rows); the later ones may be partly or wholly
-// past the end of the row.  A row with edges has up to 8 vectors less than its length suggests.
+// The shapes of a workgroup that holds a row, shortest rows first: threads, vectors a thread, and the longest row
+// that it is taken for in vectors of fp32 and of 16-bit logits (0: none).  Why the lines lie there: see pick_shape.
+struct RowShape {
+    int threads, vectors;
+    int64_t most_f32, most_16;
+    constexpr int64_t most(int dtype) const { return dtype == MRL_F32 ? most_f32 : most_16; }
+};
+constexpr int64_t kMaxVec = 19 * 1024;              // vectors of the widest row that one workgroup holds
+constexpr int64_t kMinHalf = (kMaxVec + 1) / 2;     // of the shorter half of a wider one
+constexpr RowShape kRowShapes[] = {
+    {256, 4, 1024, 1024},      {256, 8, 2048, 2048},      {256, 12, 2496, 3072},     {512, 8, 4096, 4096},
+    {512, 12, 0, 6144},        {512, 16, 0, 8192},        {1024, 8, 8192, 0},        {1024, 10, 10240, 10240},
+    {1024, 12, 12288, 12288},  {1024, 14, 14336, 14336},  {1024, 16, 16384, 16384},  {1024, 19, kMaxVec, kMaxVec},
+};
+constexpr int kShapes = sizeof(kRowShapes) / sizeof(kRowShapes[0]);
+
+// Rows that are held side by side (see pick_rows), each by 256 threads: how many, vectors a thread, and the row lengths in
+// vectors, longer than `above` and up to `most` (0: none).
+struct SideShape {
+    int rows, vectors;
+    int64_t above_f32, most_f32, above_16, most_16;
+    constexpr int64_t above(int dtype) const { return dtype == MRL_F32 ? above_f32 : above_16; }
+    constexpr int64_t most(int dtype) const { return dtype == MRL_F32 ? most_f32 : most_16; }
+};
+constexpr int kSideThreads = 256;
+constexpr SideShape kSideShapes[] = {
+    {4, 4, 512, 1024, 928, 1024}, {2, 7, 0, 0, 1312, 1792},  {4, 8, 1024, 2048, 0, 0},
+    {2, 8, 0, 0, 1792, 2048},     {2, 10, 0, 0, 2048, 2560}, {4, 12, 2048, 2496, 0, 0},
+};
+constexpr int kSides = sizeof(kSideShapes) / sizeof(kSideShapes[0]);
+
+// Vectors of a thread that are complete in every row that the tables give to a workgroup of BLK threads with NV vectors
+// each; the later ones may be partly or wholly past the end of the row.  A row with edges has up to 8 vectors less than
+// its length suggests.
+constexpr int complete_vectors(int threads, int vectors, bool edge) {
+    int64_t least = kMaxVec + 1;
+    for (int dtype : {MRL_F32, MRL_BF16}) {
+        int64_t before = 0;                         // the longest row of a smaller shape
+        for (const RowShape& s : kRowShapes) {
+            const int64_t most = s.most(dtype);
+            if (most == 0) continue;
+            if (s.threads == threads && s.vectors == vectors) {
+                if (before + 1 < least) least = before + 1;
+                // halves of wide rows: the shorter one may be a vector less than the one that the shape follows from
+                const int64_t half = before > kMinHalf ? before : kMinHalf;
+                if (most > kMinHalf && half < least) least = half;
+            }
+            before = most;
+        }
+        for (const SideShape& s : kSideShapes)
+            if (threads == kSideThreads && s.vectors == vectors && s.most(dtype) != 0 && s.above(dtype) + 1 < least)
+                least = s.above(dtype) + 1;
+    }
+    if (edge) least -= 8;
+    return least < threads ? 0 : (int)(least / threads);
+}
+
 template <int BLK, int NV, bool kEdge>
 struct Tail {
-    static constexpr int kRow = NV <= 4 ? 0 : (NV <= 8 || BLK * NV == 512 * 12 ? 4 : (NV == 19 ? 16 : NV - 4));
-    static constexpr int kFull = kRow - (kEdge && kRow > 0 ? 1 : 0);
+    static constexpr int kFull = complete_vectors(BLK, NV, kEdge);
+    static_assert(kFull <= NV, "no row of this many threads and vectors is in the tables");
 };
 
 // Vector q of a row is addressed through a descriptor of its own (the row from byte q * 16 * BLK on,
@@ -1054,7 +1108,10 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
 //          80 KB 4 417 -> 5 906, 100 KB 5 199 -> 5 879 (512 x 16; 512 x 12 where both fit within 2 %)
 //   fp32 (half the entries per byte to compute): 32 KB 3 802 -> 5 599, 48 KB 4 859 -> 6 205, 64 KB 5 832 -> 6 083;
 //          96 and 128 KB stay with 1024 x 8 (6 190 and 6 250 against 5 800 and 5 700 with 512 x 16);
-//          34 KB 5 361 with 512 x 12, 39 KB 6 046: up to there 256 x 12, which takes rows side by side
+//          34 and 39 KB 5 354 and 5 934 with 512 x 8, up to there 256 x 12, which takes rows side by side (5 833 and
+//          5 963; 600 of them 16.3 and 16.7 -> 12.6 and 12.9 us; fewer than 512, a row to a workgroup, within 5 %).  That
+//          one is not as in the larger shape: half the threads add up twice the vectors, which rounds differently
+// 16-bit rows of 40 to 48 KB, 256 x 12 and with 512 x 8: 24 576 entries 5 576 and 6 115 GB/s, 600 of them 15.6 and 17.2 us.
 // Vectors of a thread that lie past the row are computed on all the same, so that a shape with fewer is the faster one,
 // the more so with the entropy's sum and with few rows, which wait for a single row's chain; which thread holds what is
 // as in the larger shape, and with it every bit.  512 x 12 -> 512 x 8, without and with entropy, GB/s of 1 GB of logits
@@ -1067,66 +1124,10 @@ __global__ void grad_scale_note_kernel(const float* __restrict__ upstream, float
 // The choice depends on the row's length alone, so a row's result does not depend on the other rows' contents.
 // Its place does enter for rows that are not whole 128-byte lines (see RowSpan): which thread adds which entry
 // follows from the row's address modulo 128, so the fp32 sums round differently at another place in the batch.
-enum Shape { k256x4, k256x8, k256x12, k512x8, k512x12, k512x16, k1024x8, k1024x10, k1024x12, k1024x14, k1024x16, k1024x19, kTooLong };
-constexpr int64_t kMaxVec = 19 * 1024;              // vectors of the widest row that one workgroup holds
-
-inline Shape pick_shape(int dtype, int64_t n_vec) {
-    if (n_vec <= 1024) return k256x4;
-    if (n_vec <= 2048) return k256x8;
-    if (dtype == MRL_F32) {
-        if (n_vec <= 2496) return k256x12;
-        if (n_vec <= 4096) return k512x8;
-        if (n_vec <= 8192) return k1024x8;
-    } else {
-        if (n_vec <= 3072) return k256x12;
-        if (n_vec <= 4096) return k512x8;
-        if (n_vec <= 6144) return k512x12;
-        if (n_vec <= 8192) return k512x16;
-    }
-    if (n_vec <= 10240) return k1024x10;
-    if (n_vec <= 12288) return k1024x12;
-    if (n_vec <= 14336) return k1024x14;
-    if (n_vec <= 16384) return k1024x16;
-    return n_vec <= kMaxVec ? k1024x19 : kTooLong;
-}
-
-// Rows of 256 threads that a workgroup holds side by side (and with how many vectors a thread: fewer than the row's
-// shape has where that leaves no lane idle; which thread holds what is the same, and with it every bit of the
-// results).  Six or eight small workgroups per CU keep as many bytes in flight as two larger ones, but as many
-// separate bursts of 16 to 48 KiB: the rows of a unit are requested, and written, together.  1 GB of logits, GB/s
-// of a row alone -> side by side (16 bits without and with the entropy's sum; fp32 within 1 % of each other):
-//   16 bits  8 000 entries 5 227 -> 5 733, 5 247 -> 5 675; 11 776 5 522 -> 6 046, 5 497 -> 5 845; 13 824 5 461 ->
-//            6 052, 5 471 -> 5 974; 16 384 5 458 -> 6 116, 5 473 -> 6 069; 17 408 5 399 -> 5 895, 5 383 -> 5 826;
-//            20 480 5 683 -> 5 866, 5 665 -> 5 823.  Not 7 168 (4 846 -> 4 824 with entropy), 9 728 (5 516 -> 5 227)
-//            and 22 528 (5 616 -> 5 700): there the last of a thread's vectors are mostly past the row, and the
-//            arithmetic of a unit, which starts and ends together, shows
-//   fp32     3 328 5 405 -> 5 954, 4 096 5 497 -> 5 849, 4 864 5 604 -> 6 053, 5 888 5 588 -> 6 200, 8 192 5 568 -> 6 190,
-//            8 704 5 361 -> 5 939, 9 728 5 825 -> 6 017
-// Few rows: where all start at once they share tickets and are done sooner (1 024 x 8 000 bf16 13.0 -> 10.8 us,
-// 1 024 x 5 888 fp32 13.9 -> 12.6); in between the last, half empty round of larger units costs more than they gain
-// (2 048 x 16 384 bf16 26.6 -> 29.0 us, 4 096 x 8 000 28.9 -> 30.8; 8 192 x 16 384 100.1 -> 97.6), except where rows
-// are longer than 32 KiB (1 024 x 17 408 21.8 -> 15.7, 3 072 47.0 -> 45.0).
-struct SideBySide {
-    int rows, vectors;          // rows 1: a row to a workgroup
-};
-
-inline SideBySide pick_rows(int dtype, int64_t n_vec, int64_t n_rows) {
-    const SideBySide alone = {1, 0};
-    SideBySide s = alone;
-    int64_t at_once = 0;        // rows that start together on 256 CUs
-    if (dtype == MRL_F32) {
-        if (n_vec > 512 && n_vec <= 1024) s = {4, 4}, at_once = 2048;
-        else if (n_vec > 1024 && n_vec <= 2048) s = {4, 8}, at_once = 1024;
-        else if (n_vec > 2048 && n_vec <= 2496) s = {4, 12};
-    } else {
-        if (n_vec > 928 && n_vec <= 1024) s = {4, 4}, at_once = 2048;
-        else if (n_vec > 1312 && n_vec <= 1792) s = {2, 7}, at_once = 1024;
-        else if (n_vec > 1792 && n_vec <= 2048) s = {2, 8}, at_once = 1024;
-        else if (n_vec > 2048 && n_vec <= 2560) s = {2, 10};
-    }
-    const bool long_rows = n_vec > 2048;
-    const bool pays = n_rows >= (n_vec <= 1024 ? 16384 : 8192) || (n_rows >= 512 && (long_rows || n_rows <= at_once));
-    return pays ? s : alone;
+inline int pick_shape(int dtype, int64_t n_vec) {
+    for (int i = 0; i < kShapes; ++i)
+        if (n_vec <= kRowShapes[i].most(dtype)) return i;
+    return kShapes;                                 // too long: two halves
 }
 
 // Number of CUs of the current device (one persistent workgroup each); 0 if the query fails.
@@ -1135,6 +1136,35 @@ int cu_count() {
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     return n;
+}
+
+// Rows of 256 threads that a workgroup holds side by side (and with how many vectors a thread: fewer than the row's
+// shape has where that leaves no lane idle; which thread holds what is the same, and with it every bit of the
+// results).  A CU holds four to eight such rows either way (six of 256 x 8 alone, four side by side), but alone they are
+// as many separate bursts of 16 to 48 KiB: the rows of a unit are requested, and written, together.  1 GB of logits, GB/s
+// of a row alone -> side by side (16 bits without and with the entropy's sum; fp32 within 1 % of each other):
+//   16 bits  8 000 entries 5 227 -> 5 733, 5 247 -> 5 675; 11 776 5 522 -> 6 046, 5 497 -> 5 845; 13 824 5 461 ->
+//            6 052, 5 471 -> 5 974; 16 384 5 458 -> 6 116, 5 473 -> 6 069; 17 408 5 399 -> 5 895, 5 383 -> 5 826;
+//            20 480 5 683 -> 5 866, 5 665 -> 5 823.  Not 7 168 (4 846 -> 4 824 with entropy), 9 728 (5 516 -> 5 227)
+//            and 22 528 (5 616 -> 5 700): there the last of a thread's vectors are mostly past the row, and the
+//            arithmetic of a unit, which starts and ends together, shows
+//   fp32     3 328 5 405 -> 5 954, 4 096 5 497 -> 5 849, 4 864 5 604 -> 6 053, 5 888 5 588 -> 6 200, 8 192 5 568 -> 6 190,
+//            8 704 5 421 -> 5 854, 9 984 5 683 -> 5 973
+// Few rows: where all start at once they share tickets and are done sooner, also where four of them leave CUs without any
+// (512 rows, us: 8 192 bf16 12.0 -> 9.4, 16 384 12.8 -> 11.2, 2 112 fp32 11.3 -> 8.7, 8 192 12.3 -> 11.1, 8 704 12.6 -> 12.1;
+// 1 024 x 8 000 bf16 13.0 -> 10.8, 1 024 x 5 888 fp32 13.9 -> 12.6); in between the last, half empty round of larger units costs more than they gain
+// (2 048 x 16 384 bf16 26.6 -> 29.0 us, 4 096 x 8 000 28.9 -> 30.8; 8 192 x 16 384 100.1 -> 97.6), except where rows
+// are longer than 32 KiB (1 024 x 17 408 21.8 -> 15.7, 3 072 47.0 -> 45.0).
+// Returns the place in kSideShapes; -1: a row to a workgroup.
+inline int pick_rows(int dtype, int64_t n_vec, int64_t n_rows) {
+    for (int i = 0; i < kSides; ++i) {
+        const SideShape& s = kSideShapes[i];
+        if (n_vec <= s.above(dtype) || n_vec > s.most(dtype)) continue;
+        if (n_rows >= (n_vec <= 1024 ? 16384 : 8192)) return i;
+        const int per_cu = waves_per_simd(s.vectors, s.rows);       // a row is a wavefront on each of a CU's four SIMDs
+        return n_rows >= 512 && (n_vec > 2048 || n_rows <= (int64_t)per_cu * cu_count()) ? i : -1;
+    }
+    return -1;
 }
 
 // Upper bound of the polls a workgroup spends waiting for the other half of a wide row before it
@@ -1192,36 +1222,35 @@ int launch_narrow(const mrl::FusedArgs& a) {
                           : launch_sweep<DT, BLK, NV, kRows, false, false, false>(a);
 }
 
-template <int DT, int NV>
-int launch_1024(const mrl::FusedArgs& a) {
-    if (!a.wide) return launch_narrow<DT, kWideBlock, NV>(a);
-    return a.with_entropy ? launch_sweep<DT, kWideBlock, NV, 1, true, true, false>(a)
-                          : launch_sweep<DT, kWideBlock, NV, 1, false, true, false>(a);
+template <int DT, int I = 0>
+int fused_by_shape(int shape, const mrl::FusedArgs& a) {
+    if constexpr (I < kShapes) {
+        constexpr RowShape s = kRowShapes[I];
+        if (I != shape) return fused_by_shape<DT, I + 1>(shape, a);
+        if constexpr (s.most(DT) > 0) {
+            if constexpr (s.most(DT) > kMinHalf)
+                if (a.wide)
+                    return a.with_entropy ? launch_sweep<DT, s.threads, s.vectors, 1, true, true, false>(a)
+                                          : launch_sweep<DT, s.threads, s.vectors, 1, false, true, false>(a);
+            return launch_narrow<DT, s.threads, s.vectors>(a);
+        }
+    }
+    return mrl::fail(MRL_ERR_LAUNCH, "mrl_fused_logprob_loss: no shape for these rows");
+}
+
+template <int DT, int I = 0>
+int fused_side_by_side(int side, const mrl::FusedArgs& a) {
+    if constexpr (I < kSides) {
+        constexpr SideShape s = kSideShapes[I];
+        if (I != side) return fused_side_by_side<DT, I + 1>(side, a);
+        if constexpr (s.most(DT) > 0) return launch_narrow<DT, kSideThreads, s.vectors, s.rows>(a);
+    }
+    return mrl::fail(MRL_ERR_LAUNCH, "mrl_fused_logprob_loss: no shape for these rows");
 }
 
 template <int DT>
-int fused_by_shape(Shape shape, SideBySide side, const mrl::FusedArgs& a) {
-    if constexpr (DT == MRL_F32) {
-        if (side.rows == 4 && side.vectors == 8) return launch_narrow<DT, 256, 8, 4>(a);
-        if (side.rows == 4 && side.vectors == 12) return launch_narrow<DT, 256, 12, 4>(a);
-        if (shape == k1024x8) return launch_narrow<DT, 1024, 8>(a);
-    } else {
-        if (side.rows == 2 && side.vectors == 7) return launch_narrow<DT, 256, 7, 2>(a);
-        if (side.rows == 2 && side.vectors == 8) return launch_narrow<DT, 256, 8, 2>(a);
-        if (side.rows == 2) return launch_narrow<DT, 256, 10, 2>(a);
-        if (shape == k512x12) return launch_narrow<DT, 512, 12>(a);
-        if (shape == k512x16) return launch_narrow<DT, 512, 16>(a);
-    }
-    if (side.rows == 4) return launch_narrow<DT, 256, 4, 4>(a);
-    if (shape == k256x4) return launch_narrow<DT, 256, 4>(a);
-    if (shape == k256x8) return launch_narrow<DT, 256, 8>(a);
-    if (shape == k256x12) return launch_narrow<DT, 256, 12>(a);
-    if (shape == k512x8) return launch_narrow<DT, 512, 8>(a);
-    if (shape == k1024x10) return launch_1024<DT, 10>(a);
-    if (shape == k1024x12) return launch_1024<DT, 12>(a);
-    if (shape == k1024x14) return launch_1024<DT, 14>(a);
-    if (shape == k1024x16) return launch_1024<DT, 16>(a);
-    return launch_1024<DT, 19>(a);
+int fused_sweep(int shape, int side, const mrl::FusedArgs& a) {
+    return side >= 0 ? fused_side_by_side<DT>(side, a) : fused_by_shape<DT>(shape, a);
 }
 
 }  // namespace
@@ -1360,15 +1389,15 @@ static int run_sweep(const char* fn, mrl::FusedArgs& a, int64_t workspace_bytes)
         MRL_REQUIRE(a.d_stride == a.row_stride, MRL_ERR_INVALID_ARG, "%s: in-place needs identical strides", fn);
     }
     const int64_t n_vec = a.vocab / (16 / eb);
-    Shape shape = pick_shape(a.dtype, n_vec);
-    a.wide = shape == kTooLong;
+    int shape = pick_shape(a.dtype, n_vec);
+    a.wide = shape == kShapes;
     a.half_elems = 0;
     if (a.wide) {
         a.half_elems = (n_vec + 1) / 2 * (16 / eb);
         shape = pick_shape(a.dtype, (n_vec + 1) / 2);
     }
     // without a counter every row has a workgroup of its own
-    const SideBySide side = a.workspace != nullptr && !a.wide ? pick_rows(a.dtype, n_vec, a.n_rows) : SideBySide{1, 0};
+    const int side = a.workspace != nullptr && !a.wide ? pick_rows(a.dtype, n_vec, a.n_rows) : -1;
     if (a.workspace != nullptr || a.wide) {
         const int64_t need = a.wide ? mrl_fused_workspace_bytes(a.dtype, a.n_rows, a.vocab) : kWorkspaceHeader;
         MRL_REQUIRE(a.workspace != nullptr && workspace_bytes >= need, MRL_ERR_INVALID_ARG,
@@ -1376,9 +1405,9 @@ static int run_sweep(const char* fn, mrl::FusedArgs& a, int64_t workspace_bytes)
                     "their statistics through it)", fn, (long long)(a.workspace ? workspace_bytes : 0), (long long)need);
     }
     switch (a.dtype) {
-        case MRL_F32: return fused_by_shape<MRL_F32>(shape, side, a);
-        case MRL_BF16: return fused_by_shape<MRL_BF16>(shape, side, a);
-        default: return fused_by_shape<MRL_F16>(shape, side, a);
+        case MRL_F32: return fused_sweep<MRL_F32>(shape, side, a);
+        case MRL_BF16: return fused_sweep<MRL_BF16>(shape, side, a);
+        default: return fused_sweep<MRL_F16>(shape, side, a);
     }
 }
 
