@@ -1623,6 +1623,51 @@ def test_sequence_sums_by_width(dev, width, mask_dtype):
     assert torch.equal(ops.view(batch, width + 1, 8)[:, :width, 3].cpu(), live)
 
 
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 8000), (torch.bfloat16, 14003), (torch.float16, 16384), (torch.float32, 4100),
+                                         (torch.float32, 9984), (torch.bfloat16, 32000), (torch.bfloat16, 32003),
+                                         (torch.float32, 40960), (torch.bfloat16, 66000), (torch.bfloat16, 114688)])
+def test_sweeps_over_rows_that_are_not_finite(dev, dtype, vocab):
+    """Rows with an infinity, a NaN, or nothing but -inf are not finite in log-prob and log-sum-exp, as in torch, and no
+    row beside them (in the same workgroup for the shorter ones) changes a bit: forward and fused sweep, out of place and
+    in place, with and without entropy."""
+    rows = 514
+    gen = torch.Generator(device=dev).manual_seed(vocab)
+    clean = (torch.randn(rows, vocab, generator=gen, device=dev) * 3).to(dtype)
+    y = torch.randint(0, vocab, (rows,), generator=gen, device=dev)
+    odd = {3: (vocab // 2, float("inf")), 5: (0, float("nan")), 6: (vocab - 1, float("nan")), 9: (slice(None), float("-inf")),
+           17: (vocab // 3, float("inf")), 513: (1, float("nan"))}
+    z = clean.clone()
+    for r, (at, value) in odd.items():
+        z[r, at] = value
+    y[17] = vocab // 3                                              # the label's own logit
+    beside = torch.tensor([r not in odd for r in range(rows)], device=dev)
+    ops = torch.zeros(rows, 8, device=dev)
+    ops[:, 2], ops[:, 3], ops[:, 4], ops[:, 5] = 1.0, (torch.arange(rows, device=dev) % 7 != 4).float(), 1.0, 1.0
+    ops[9, 3] = 1.0
+    counter = torch.empty(4, dtype=torch.int32, device=dev)
+
+    def sweep(z_in, dz, entropy):
+        terms, lp, ent = torch.empty(rows, 8, device=dev), torch.empty(rows, device=dev), torch.zeros(rows, device=dev)
+        _lib.call("mrl_fused_logprob_loss", z_in.data_ptr(), _lib.dtype_code(z), rows, vocab, vocab, y.data_ptr(), _lib.I64,
+                  1.0, ops.data_ptr(), 0, 0.8, 1.2, 0, 0.0, 0.01 if entropy else 0.0, 1.0, None, dz.data_ptr(), vocab,
+                  lp.data_ptr(), ent.data_ptr() if entropy else None, terms.data_ptr(), counter.data_ptr(), 16, 0, _lib.stream(dev))
+        return dz, lp, ent, terms
+
+    for entropy in (False, True):
+        want = sweep(clean, torch.empty_like(z), entropy)
+        got = sweep(z, torch.empty_like(z), entropy)
+        buf = z.clone()
+        for out in (got, sweep(buf, buf, entropy)):
+            for a, b in zip(out, want):
+                assert torch.equal(a[beside], b[beside])
+            assert not out[1][~beside].isfinite().any().item()
+        want = mrl.vocab_logprob_entropy(clean, y, want_entropy=entropy)
+        got = mrl.vocab_logprob_entropy(z, y, want_entropy=entropy)
+        for a, b in zip(got, want):
+            assert a is None or torch.equal(a[beside], b[beside])
+        assert not got[0][~beside].isfinite().any().item() and not got[2][~beside].isfinite().any().item()
+
+
 @pytest.mark.parametrize("batch,width,mask_dtype", [(2049, 1024, None), (2050, 1025, None), (2050, 4096, None), (2051, 4097, None),
                                                     (512, 1025, torch.int64), (513, 1025, torch.float32),
                                                     (513, 4097, torch.uint8), (1025, 4097, torch.int64), (1500, 4096, torch.int32)])
