@@ -173,6 +173,8 @@ __device__ __forceinline__ void score_row(
     // The last whole round, and with it what is left of the row, of which a thread may have fewer vectors or none:
     // range-checked.  A round of its own for the rest, however short, was waited for like any other: us a pass, 2 903
     // rows x 33 024 bf16 (two rounds and 32 vectors) 37.5 -> 34.5, x 30 000 34.3 -> 32.4, 662 x 32 000 14.8 -> 13.5.
+    // Where there is no rest few rows pay for it all the same: 300 x 16 384 fp32 6.1 -> 6.2, 1 000 10.8 -> 11.0, and 11.2
+    // if the rest's tests of a lane's vectors are gone through as well.
     {
         const mrl::rsrc_t rest = mrl::make_rsrc(vec + n_full, (uint32_t)(sp.n_vec - n_full) * 16u);
         u32x4 v[kDeep], w[kDeep];
@@ -180,6 +182,7 @@ __device__ __forceinline__ void score_row(
 #pragma unroll
         for (int q = 0; q < kDeep; ++q) w[q] = mrl::buf_load_nt(rest, (uint32_t)(q * kBlk + tid) * 16u);
         if (n_full > 0) add_round(v);
+        if (n_full != sp.n_vec)
 #pragma unroll
         for (int q = 0; q < kDeep; ++q) {
             if (n_full + q * kBlk + tid < sp.n_vec) {
@@ -460,13 +463,16 @@ int launch_fwd_shape(const char* fn, const FwdArgs& a, const WindowCells& w) {
 // Threads of a row's workgroup and vectors a thread and round, by the row's length alone, so that a row's result
 // does not depend on how many rows there are.  Many rows are bound by memory whatever the shape (within 3 %); few
 // of them, a workgroup to a CU or less, by the rounds that a thread waits for one after the other, which more threads
-// make fewer of, up to where most of a workgroup has nothing to load.  us a pass, 256 x 4 for all rows -> now:
-// 98 x 152 064 bf16 20.2 -> 12.4, 116 x 129 280 18.0 -> 11.9, 49 x 152 064 fp32 29.5 -> 15.6; 2 GB of rows of
-// 152 064 bf16 293 -> 286, 63 712 299 -> 286, 32 000 294 -> 288.
-// The lines: 2 GB of rows of 3 750 vectors (30 000 bf16) 291 with 256 threads and 281 with 512, of 3 250 287 and
-// 298; of 4 096 fp32 vectors 286 and 290; of 6 500 284 with 512 and 285 with 1024, of 7 964 290 and 286.  Rows of 512
-// vectors and less would gain from a wavefront each (4 000 bf16 458 -> 324), but entropies of merged vocabulary
-// shards then differ by up to 2.3e-5 from the whole row's, more than they may.
+// make fewer of, up to where most of a workgroup has nothing to load.  us a pass, 256 x 4 for all rows and a round for
+// their rest -> now: 98 x 152 064 bf16 20.2 -> 12.4, 116 x 129 280 18.0 -> 11.9, 49 x 152 064 fp32 29.5 -> 15.6; 2 GB of
+// rows of 152 064 bf16 293 -> 286, 32 000 294 -> 287.
+// The lines, us for 2 GB of rows without and with entropy: 16 bits, 256 and 512 threads, 3 584 vectors 290 and 288, 294
+// and 284, 3 000 291 and 290, 296 and 287 (they could lie lower; before the rest went with the last round 512 were the
+// slower ones there); fp32 4 096 vectors 287 and 293, 292 and 299, 5 000 287 and 285, 292 and 291; 512 and 1024, 6 500
+// vectors 287 and 283, 291 and 288, 7 168 287 and 282, 288 and 281, 7 964 286 and 286, 289 and 285, 300 rows of 7 168
+// fp32 vectors 7.7 and 8.1.  1024 threads with 4 vectors: 7 964 294, 12 500 and more within 0.5 % of 3.  Rows of 512
+// vectors and less would gain from a wavefront each (4 000 bf16 458 -> 324), but entropies of merged vocabulary shards
+// then differ by up to 2.3e-5 from the whole row's, more than they may.
 template <int DT, typename LabelT, typename Rows>
 int launch_fwd(const char* fn, const FwdArgs& a, const Rows& rows) {
     const int64_t n_vec = a.vocab / Elem<DT>::kVec;
