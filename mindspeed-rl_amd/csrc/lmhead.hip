@@ -226,9 +226,11 @@ __global__ __launch_bounds__(mrl_tile::kThreads, 1) void lmhead_fwd_kernel(
 // token's hidden row with the label's weight row; 16 threads per token, of the first four wavefronts, merge the leaves
 // (thread q takes leaves q, q + 16, ...; the loads of 16 neighbouring tokens are 64 contiguous bytes), then the 16
 // partial results are merged in order.  Few tokens are bound by the loads that follow each other, many by the rows'
-// bytes: a wavefront to each token up to kFewTokens, 4 tokens to one behind, us, 4 wavefronts and 512 entries at a time
-// -> now: 224 tokens x 3 072 14.2 -> 5.7, 589 x 4 224 17.6 -> 6.4, 4 000 x 1 024 10.6 -> 7.2, 7 100 x 3 776 19.6 -> 15.0,
-// 17 122 x 3 584 34.9 -> 32.8, 20 959 x 768 13.1 -> 13.6 (15.3 with a wavefront to each).
+// bytes: a wavefront to each token up to kFewTokens, 4 tokens to one behind.  us, 4 wavefronts and 512 entries at a time
+// -> now, 32 000 logits unless given: 224 tokens x 3 072 14.6 -> 6.3, 589 x 4 224 20.7 -> 8.2, 4 000 x 1 024 10.0 -> 7.2,
+// 7 100 x 3 776 26.4 -> 21.6, 12 000 x 2 048 20.0 -> 19.8.  Beyond that the four loads at a time gain nothing and cost up
+// to 6 % of a few microseconds in passes of milliseconds: 20 959 x 10 736 x 768 14.8 -> 14.9, 9 000 x 512 10.5 -> 11.2,
+// 17 122 x 152 064 x 3 584 49.6 -> 52.1; a wavefront to each there 18.0, 11.9 and 51.6.
 constexpr int kFinishTokens = 16;
 constexpr int64_t kFewTokens = 4096;
 template <typename LabelT, bool kEntropy, int kFinishWaves>
