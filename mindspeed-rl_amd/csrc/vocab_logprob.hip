@@ -60,17 +60,6 @@ struct FlaggedRows {
     __device__ __forceinline__ int64_t row(int64_t out) const { return active != nullptr && active[out] == 0 ? -1 : out; }
 };
 
-// The window of a sequence that is the same for the whole workgroup; its lengths are requested together.
-__device__ __forceinline__ void uniform_window(const mrl::SeqWindows& w, uint32_t i, int64_t& start, int64_t& n) {
-    if (!w.packed) return w.window(i, start, n);
-    int32_t first = w.cu[i], length = w.seqlens[i];
-    int64_t prompt = mrl::load_index(w.prompt, w.prompt_dtype, i);
-    asm volatile("" : "+s"(first), "+s"(length), "+s"(prompt));
-    const bool inside = prompt - 1 < length;
-    start = inside ? first + prompt - 1 : first;
-    n = inside ? length - prompt : length;
-}
-
 struct WindowCells {
     static constexpr int kCells = 1;
     mrl::SeqWindows seqs;
@@ -79,7 +68,7 @@ struct WindowCells {
     __device__ __forceinline__ int64_t row(int64_t out) const {
         const uint32_t i = (uint32_t)out / width, j = (uint32_t)out - i * width;
         int64_t start, n;
-        uniform_window(seqs, i, start, n);
+        seqs.window(i, start, n);
         const int64_t t = start + j;
         return (int64_t)j < n && t >= 0 && t < n_rows ? t : -1;
     }
@@ -104,7 +93,7 @@ struct ManyCells {
         Unit r;
         r.j = u - i * step;
         r.first = (int64_t)i * width;
-        uniform_window(seqs, i, r.start, r.n);
+        seqs.window(i, r.start, r.n);
         return r;
     }
     // whether there is a cell c of the unit; its place and the row that it reads
@@ -122,7 +111,7 @@ template <int DT, typename LabelT, bool kEntropy, int kBlk, int kDeep>
 __device__ __forceinline__ void score_row(
     const typename Elem<DT>::T* __restrict__ logits, int64_t row_stride, int vocab,
     const LabelT* __restrict__ labels, int64_t r, int64_t out, float inv_t,
-    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out, Stats* lds) {
+    float* __restrict__ logp, float* __restrict__ entropy, float* __restrict__ lse_out, Stats* lds, const int tid) {
     using E = Elem<DT>;
     using T = typename E::T;
     constexpr int kVec = E::kVec;
@@ -133,13 +122,12 @@ __device__ __forceinline__ void score_row(
     const int64_t y = (int64_t)labels[r];
     const bool y_ok = (y >= 0) && (y < (int64_t)vocab);
     float z_y = 0.f;
-    if (threadIdx.x == 0 && y_ok) z_y = E::load(row + y);
+    if (tid == 0 && y_ok) z_y = E::load(row + y);
 
     const RowSplit<T, kVec> sp(row, vocab);
     const u32x4* vec = reinterpret_cast<const u32x4*>(row + sp.head);
 
     Stats st = {kMaxInit, 0.f, 0.f};
-    const int tid = threadIdx.x;
 
     // rounds of kDeep vectors a thread, all requested before any is used
     auto request = [&](u32x4 (&v)[kDeep], int base) {
@@ -233,8 +221,9 @@ __global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
         if (entropy) entropy[out] = 0.f;
         if (lse_out) lse_out[out] = 0.f;
     };
-    auto score = [&](int64_t r, int64_t out) {
-        score_row<DT, LabelT, kEntropy, kBlk, kDeep>(logits, row_stride, vocab, labels, r, out, inv_t, logp, entropy, lse_out, lds);
+    auto score = [&](int64_t r, int64_t out, int tid) {
+        score_row<DT, LabelT, kEntropy, kBlk, kDeep>(logits, row_stride, vocab, labels, r, out, inv_t, logp, entropy, lse_out, lds,
+                                                     tid);
     };
     if constexpr (Rows::kCells == 1) {
         const int64_t out = first + blockIdx.x, r = rows.row(out);
@@ -242,7 +231,7 @@ __global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
             if (threadIdx.x == 0) no_row(out);
             return;
         }
-        score(r, out);
+        score(r, out, (int)threadIdx.x);
     } else {
         const auto unit = rows.unit(first + blockIdx.x);
         int64_t out, r;
@@ -252,7 +241,11 @@ __global__ __launch_bounds__(kBlk) void vocab_fwd_kernel(
         for (int c = 0; c < Rows::kCells; ++c) {
             if (!rows.cell(unit, c, out, r)) return;
             if (r < 0) continue;
-            score(r, out);
+            int tid = (int)threadIdx.x;
+            // what follows from it is computed for each cell: kept from cell to cell it would take the registers of a
+            // workgroup on every CU (79 instead of 62 with 512 threads and entropies)
+            asm volatile("" : "+v"(tid));
+            score(r, out, tid);
             __syncthreads();                // the partials have been read
         }
     }
@@ -441,17 +434,18 @@ int launch_fwd_shape(const char* fn, const FwdArgs& a, const FlaggedRows& rows) 
     return launch_fwd_units<DT, LabelT, kBlk, kDeep>(fn, a, rows, a.n_out);
 }
 
-// A cell to a workgroup, or several: where most of the cells are known to be empty, or so many that their rows, should
-// they all have one, keep the chip busy either way.  us a pass over bf16 windows, with 256 threads and a cell each / 512
-// or 1024 and a cell each / as it is: 256 x 8 192 cells with 7 rows to a sequence, 152 064 logits 1 123 / 4 351 / 1 174,
-// 32 000 1 057 / 2 122 / 990; 16 x 2 048 with 255, 65 536 86 / 135 / 87; all with rows, 16 x 2 048, 152 064 1 425 /
-// 1 408 / 1 409, 32 000 306 / 298 / 298.  Several cells over fewer of them leave CUs idle: 2 500 with rows x 152 064 118 /
-// 112 / 124, 10 000 x 65 536 191 / 187 / 194; with rows for one in ten they do not, 4 x 1 024 x 152 064 32 / 29 / 23.
+// A cell to a workgroup, or several: where most of the cells are known to be empty, or so many, in long windows, that
+// their rows keep the chip busy either way.  us a pass over bf16 windows, with 256 threads and a cell each / 512 or 1024
+// and a cell each / as it is: 256 x 8 192 cells with 7 rows to a sequence, 152 064 logits 1 123 / 4 263 / 1 162, 32 000
+// 1 055 / 2 066 / 998; 16 x 2 048 with 255, 57 344 75 / 76 / 73; with entropies, 20 x 2 048 of which two thirds have rows,
+// 152 064 964 / 949 / 938.  Several cells over fewer of them leave CUs idle (2 500 with rows x 152 064 118 / 112 / 124),
+// and in short windows the rows of a workgroup are many (384 of up to 78 x 126 784 785 / 760 / 789); where one in ten has
+// a row neither shows, 4 x 1 024 x 152 064 32 / 29 / 23.
 template <int DT, typename LabelT, int kBlk, int kDeep>
 int launch_fwd_shape(const char* fn, const FwdArgs& a, const WindowCells& w) {
     if constexpr (kBlk > 256) {
         constexpr int kCells = kBlk / 256;
-        if (a.n_out >= 16384 || (a.n_out >= 4096 && a.n_out >= 4 * w.n_rows)) {
+        if ((a.n_out >= 16384 && w.width >= 512) || (a.n_out >= 4096 && a.n_out >= 4 * w.n_rows)) {
             const uint32_t step = (w.width + kCells - 1) / kCells;
             const ManyCells<kCells> rows = {w.seqs, w.width, step, w.n_rows};
             return launch_fwd_units<DT, LabelT, kBlk, kDeep>(fn, a, rows, a.n_out / w.width * step);

@@ -3412,13 +3412,13 @@ def test_forward_sweep_by_row_length(dev, dtype, vectors):
             assert (got.double() - want).abs().max().item() <= bound * scale, (vocab, stride)
 
 
-@pytest.mark.parametrize("vocab,batch", [(65536, 513), (32000, 1025)])
-def test_scoring_pass_over_more_cells_than_a_launch_holds(dev, vocab, batch):
-    """Windows of 8 192 columns whose cells, at the 1024 or 512 threads that a row of this length takes, are more than
-    2^32 threads (a launch has fewer): the few live ones come out as the flagged rows do, bit for bit, the rest zero."""
-    width, live = 8192, torch.arange(batch, device=dev) % 3                 # 0, 1 or 2 cells of a sequence
-    threads = 1024 if vocab // 8 > 7168 else 512
-    assert (batch - 1) * width * threads == 2 ** 32
+@pytest.mark.parametrize("vocab", [8000, 57344, 131072])
+def test_scoring_pass_over_more_cells_than_a_launch_holds(dev, vocab):
+    """Windows whose cells, 256 threads to each or 512 and 1024 to two and four of them, are more than 2^32 threads (a launch
+    has fewer): the few live ones come out as the flagged rows do, bit for bit, the rest zero."""
+    batch, width = 2049, 8192
+    assert (batch - 1) * width * 256 == 2 ** 32
+    live = torch.arange(batch, device=dev) % 3                              # 0, 1 or 2 cells of a sequence
     seqlens = (live + 1).to(torch.int32)                                    # a prompt of one token
     cu = torch.cat([torch.zeros(1, device=dev), torch.cumsum(seqlens, 0)]).to(torch.int32)
     n_rows = int(cu[-1])
@@ -3437,17 +3437,15 @@ def test_scoring_pass_over_more_cells_than_a_launch_holds(dev, vocab, batch):
     assert not got[:, ~cells].any().item()
 
 
-@pytest.mark.parametrize("vocab", [28680, 57352])
-@pytest.mark.parametrize("batch,width", [(7, 2343), (3, 5462), (4, 1021), (5, 1025), (5000, 1), (2100, 3)])
+@pytest.mark.parametrize("vocab", [32776, 57344, 90120])
+@pytest.mark.parametrize("batch,width", [(7, 2343), (3, 5462), (4, 1021), (33, 512), (700, 23), (2100, 3)])
 def test_scoring_pass_over_many_cells(dev, vocab, batch, width):
     """Windows of so many cells, or so many empty ones, that a workgroup of 512 or 1024 threads takes several of them:
-    every cell as the flagged rows give it, bit for bit, zeros elsewhere - widths that do not divide, empty and full
-    windows beside each other, windows behind the rows, labels outside the vocabulary."""
+    every cell as the flagged rows give it, bit for bit, zeros elsewhere - widths that do not divide, long and short ones,
+    empty and full windows beside each other, windows behind the rows, labels outside the vocabulary."""
     gen = torch.Generator().manual_seed(batch * width + vocab)
-    n = torch.randint(0, max(2, width // 12), (batch,), generator=gen) if width > 3 else torch.randint(0, width + 1, (batch,), generator=gen)
-    n[0], n[-1] = 0, width if width < 1100 else width // 3
-    if width == 1025:
-        n[2] = width                                    # all of it: several rows to a workgroup
+    n = torch.randint(0, max(2, width // 12), (batch,), generator=gen)
+    n[0], n[-1] = 0, width if width < 1100 else width // 3          # all of it: several rows to a workgroup
     seqlens = (n + 1).to(torch.int32)
     cu = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(seqlens, 0)]).to(torch.int32)
     n_rows = int(cu[-1]) - 3                            # the last window ends behind the rows
