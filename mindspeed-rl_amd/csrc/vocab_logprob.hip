@@ -455,23 +455,26 @@ int launch_fwd_shape(const char* fn, const FwdArgs& a, const WindowCells& w) {
 }
 
 // Threads of a row's workgroup and vectors a thread and round, by the row's length alone, so that a row's result
-// does not depend on how many rows there are.  Many rows are bound by memory whatever the shape (within 3 %); few
-// of them, a workgroup to a CU or less, by the rounds that a thread waits for one after the other, which more threads
-// make fewer of, up to where most of a workgroup has nothing to load.  us a pass, 256 x 4 for all rows and a round for
-// their rest -> now: 98 x 152 064 bf16 20.2 -> 12.4, 116 x 129 280 18.0 -> 11.9, 49 x 152 064 fp32 29.5 -> 15.6; 2 GB of
-// rows of 152 064 bf16 293 -> 286, 32 000 294 -> 287.
-// The lines, us for 2 GB of rows without and with entropy: 16 bits, 256 and 512 threads, 3 584 vectors 290 and 288, 294
-// and 284, 3 000 291 and 290, 296 and 287 (they could lie lower; before the rest went with the last round 512 were the
-// slower ones there); fp32 4 096 vectors 287 and 293, 292 and 299, 5 000 287 and 285, 292 and 291; 512 and 1024, 6 500
-// vectors 287 and 283, 291 and 288, 7 168 287 and 282, 288 and 281, 7 964 286 and 286, 289 and 285, 300 rows of 7 168
-// fp32 vectors 7.7 and 8.1.  1024 threads with 4 vectors: 7 964 294, 12 500 and more within 0.5 % of 3.  Rows of 512
-// vectors and less would gain from a wavefront each (4 000 bf16 458 -> 324), but entropies of merged vocabulary shards
-// then differ by up to 2.3e-5 from the whole row's, more than they may.
+// does not depend on how many rows there are.  Few rows are bound by the rounds that a thread waits for one after the
+// other, which more threads make fewer of: 98 x 152 064 bf16 20.2 -> 12.4 us with 1024, 116 x 129 280 18.0 -> 11.9, 49 x
+// 152 064 fp32 29.5 -> 15.6.  Many are bound by memory without entropies whatever the shape, and with them by the
+// arithmetic as well, which larger workgroups overlap less: fewer of them are on a CU, and more of a row goes with the
+// rest.  Windows of which four fifths have rows, sigma 3, us without and with entropies, 256 / 512 / 1024 threads:
+//   16 bits  4 000 vectors, 38 069 rows 355 / 350 / 412, 358 / 363 to 375 / 447; 2 022 rows 23 / 22 / 27, 24 / 23 / 28
+//            6 500, 23 417 rows 351 / 346 / 365, 354 / 351 / 400; 2 022 36 / 34 / 34, 38 / 35 / 37; 209 9.7 / 7.0 / 6.6
+//            8 192, 18 583 rows 357 / 347 / 353, 360 / 348 / 373; 2 022 46 / 42 / 41, 48 / 44 / 44; 209 11 / 8.1 / 7.1
+//            11 500, 13 227 rows 352 / 349 / 347, 355 / 349 / 354; 2 022 64 / 58 / 56, 66 / 60 / 58; 209 16 / 10 / 8.6
+//            19 008, 8 002 rows 357 / 353 / 346, 360 / 355 / 346; 2 022 104 / 95 / 92; 209 25 / 16 / 12
+//   fp32     4 096, 37 185 rows 351 / 357 / 373; 8 000, 19 026 rows 353 / 350 / 348, 2 022 41 / 40 / 39, 209 8.5 / 6.4 / 6.2
+// A CU holds two workgroups of 1024 threads: 601 rows of 152 064 bf16, a few more than two to each, take 33 us, and with
+// 512 threads 29.  1024 threads with 4 vectors: 7 964 vectors 294 us for 2 GB (286 with 3), 12 500 and more within 0.5 %.
+// Rows of 512 vectors and less would gain from a wavefront each (4 000 bf16 458 -> 324), but entropies of merged
+// vocabulary shards then differ by up to 2.3e-5 from the whole row's, more than they may.
 template <int DT, typename LabelT, typename Rows>
 int launch_fwd(const char* fn, const FwdArgs& a, const Rows& rows) {
     const int64_t n_vec = a.vocab / Elem<DT>::kVec;
-    if (n_vec <= (DT == MRL_F32 ? 4096 : 3584)) return launch_fwd_shape<DT, LabelT, 256, 4>(fn, a, rows);
-    if (n_vec <= 7168) return launch_fwd_shape<DT, LabelT, 512, 4>(fn, a, rows);
+    if (n_vec <= 4096) return launch_fwd_shape<DT, LabelT, 256, 4>(fn, a, rows);
+    if (n_vec <= (DT == MRL_F32 ? 7168 : 11264)) return launch_fwd_shape<DT, LabelT, 512, 4>(fn, a, rows);
     return launch_fwd_shape<DT, LabelT, 1024, 3>(fn, a, rows);
 }
 

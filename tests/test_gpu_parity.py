@@ -3388,9 +3388,10 @@ def test_response_windows(dev, layout, index):
 
 
 @pytest.mark.parametrize("dtype,vectors", [(torch.bfloat16, n) for n in (1, 63, 511, 512, 513, 1025, 3583, 3584, 3585, 4097, 7167,
-                                                                         7168, 7169, 9215, 9216, 9217, 19008)] +
+                                                                         7168, 7169, 9215, 9216, 9217, 4095, 4096, 11263,
+                                                                         11264, 11265, 12288, 19008)] +
                          [(torch.float32, n) for n in (512, 513, 4095, 4096, 4097, 7168, 7169, 12288, 38016)] +
-                         [(torch.float16, n) for n in (512, 3585, 7169)])
+                         [(torch.float16, n) for n in (512, 3585, 7169, 11265)])
 def test_forward_sweep_by_row_length(dev, dtype, vectors):
     """Rows around the lengths at which another workgroup size takes over, and around whole rounds of it; dense
     rows of whole vectors, and rows with edges at a stride.  A thread adds up vocab / threads entries and two
