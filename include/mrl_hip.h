@@ -184,9 +184,10 @@ int mrl_window_cut(int layout, int64_t batch, int64_t width, int64_t n_rows, con
                    const float* logp_rows, const float* entropy_rows, float* logp, float* entropy,
                    void* stream);
 
-/* mrl_window_logprob: a whole scoring pass in one launch: what mrl_vocab_logprob_fwd over the rows that
- * mrl_window_rows flags, followed by mrl_window_cut, leaves in logp and entropy ([batch, width], both written;
- * entropies are zeros unless want_entropy), bit for bit.  labels: one per row of the logits. */
+/* mrl_window_logprob: a whole scoring pass in one launch (more, where the window has more cells than a
+ * launch has threads for): what mrl_vocab_logprob_fwd over the rows that mrl_window_rows flags, followed by
+ * mrl_window_cut, leaves in logp and entropy ([batch, width], both written; entropies are zeros unless
+ * want_entropy), bit for bit.  labels: one per row of the logits. */
 int mrl_window_logprob(const void* logits, int logits_dtype, int64_t n_rows, int64_t vocab,
                        int64_t row_stride, const void* labels, int labels_dtype, float inv_temperature,
                        int layout, int64_t batch, int64_t width, const int32_t* seqlens,

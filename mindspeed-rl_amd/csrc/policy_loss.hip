@@ -6,6 +6,7 @@
 // order - deterministic, no float atomics - and writes the eight output scalars.  Backward is
 // one element-wise launch that re-derives each token's local gradient from the inputs and the
 // saved denominators.
+#include "lane_ops.h"
 #include "mrl_internal.h"
 #include "policy_terms.h"
 #include "row_sweep.h"
@@ -13,6 +14,8 @@
 namespace {
 
 using namespace mrl_loss;
+using mrl::lane_value;
+using mrl::lanes_sum;
 
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
@@ -29,33 +32,6 @@ __device__ __forceinline__ double block_sum(double v, double* lds) {
     return r;
 }
 
-// x of the lane that a step of a reduction inside 16 lanes pairs with this one: quad_perm [1,0,3,2], [2,3,0,1],
-// row_half_mirror, row_mirror, each of which pairs groups that already agree.
-template <int kStep>
-__device__ __forceinline__ double lane_partner(double x) {
-    constexpr int kControl[4] = {0xB1, 0x4E, 0x141, 0x140};
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kControl[kStep], 0xf, 0xf, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kControl[kStep], 0xf, 0xf, true);
-    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
-}
-
-template <int kSteps>
-__device__ __forceinline__ double lanes_sum(double x) {
-    x += lane_partner<0>(x);
-    x += lane_partner<1>(x);
-    if (kSteps > 2) x += lane_partner<2>(x);
-    if (kSteps > 3) x += lane_partner<3>(x);
-    return x;
-}
-
-__device__ __forceinline__ double lane_double(double x, int lane) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
-}
-
 // N sums at once over kCount wavefronts (4 or 16), in a fixed order; the FIRST wavefront gets them.  Inside a wavefront
 // by lane operands and scalar registers, not through the LDS crossbar, which took 84 shuffles of 32 bits for seven sums
 // from every wavefront: fused_seq_reduce_kernel of 256 threads 7.2 -> 6.3 us (16 x 1 024 tokens).
@@ -67,7 +43,7 @@ __device__ __forceinline__ void block_sums(double (&v)[N], double (*lds)[kCount]
 #pragma unroll
     for (int q = 0; q < N; ++q) {
         const double x = lanes_sum<4>(v[q]);
-        v[q] = (lane_double(x, 0) + lane_double(x, 16)) + (lane_double(x, 32) + lane_double(x, 48));
+        v[q] = (lane_value(x, 0) + lane_value(x, 16)) + (lane_value(x, 32) + lane_value(x, 48));
         if ((threadIdx.x & 63) == 0) lds[q][wave] = v[q];
     }
     __syncthreads();

@@ -15,6 +15,7 @@
 // has to stay on chip): a plain stream of one vector per thread.
 #include <atomic>
 
+#include "lane_ops.h"
 #include "mrl_internal.h"
 #include "policy_terms.h"
 #include "row_sweep.h"
@@ -24,6 +25,9 @@ namespace {
 
 using namespace mrl_vocab;
 using namespace mrl_loss;
+using mrl::lane_value;
+using mrl::lanes_max;
+using mrl::lanes_sum;
 
 // Vectors of the next row that are requested early (see fused_sweep_persistent_kernel); build-time
 // tuning constants, measured on the 152064-entry bf16 row.  The fused sweep gains 4 % from an early
@@ -36,37 +40,6 @@ using namespace mrl_loss;
 #ifndef MRL_BWD_CHUNK_THREADS
 #define MRL_BWD_CHUNK_THREADS 256
 #endif
-
-// One step of a reduction over the 16 lanes of a row: lane i's partner by quad_perm [1,0,3,2], [2,3,0,1],
-// row_half_mirror and row_mirror, each of which pairs groups that already agree.  A VALU operand, no trip through
-// the LDS crossbar as a shuffle.
-template <int kStep>
-__device__ __forceinline__ float row_partner(float x) {
-    constexpr int kControl[4] = {0xB1, 0x4E, 0x141, 0x140};
-    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), kControl[kStep], 0xf, 0xf, true));
-}
-
-template <int kSteps>
-__device__ __forceinline__ float row_max(float x) {
-    x = fmaxf(x, row_partner<0>(x));
-    if (kSteps > 1) x = fmaxf(x, row_partner<1>(x));
-    if (kSteps > 2) x = fmaxf(x, row_partner<2>(x));
-    if (kSteps > 3) x = fmaxf(x, row_partner<3>(x));
-    return x;
-}
-
-template <int kSteps>
-__device__ __forceinline__ float row_sum(float x) {
-    x += row_partner<0>(x);
-    if (kSteps > 1) x += row_partner<1>(x);
-    if (kSteps > 2) x += row_partner<2>(x);
-    if (kSteps > 3) x += row_partner<3>(x);
-    return x;
-}
-
-__device__ __forceinline__ float lane_value(float x, int lane) {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), lane));
-}
 
 // Two-level reduction for the BLK / 64 wavefronts that hold a row: the largest reference first, so that a part is
 // rescaled once and the rest is sums; inside a wavefront over its 4 rows of 16 lanes and these through scalar
@@ -83,15 +56,15 @@ __device__ __forceinline__ Stats reduce_row(Stats st, float k, Stats* lds, int t
     constexpr int kWaves = BLK / 64;
     constexpr int kSteps = kWaves == 16 ? 4 : (kWaves == 8 ? 3 : 2);
     static_assert(kWaves == 4 || kWaves == 8 || kWaves == 16, "partials of 4, 8 or 16 wavefronts");
-    const float m16 = row_max<4>(st.m);
+    const float m16 = lanes_max<4>(st.m);
     Stats t;
     t.m = fmaxf(fmaxf(lane_value(m16, 0), lane_value(m16, 16)), fmaxf(lane_value(m16, 32), lane_value(m16, 48)));
     const float f = fast_exp2((st.m - t.m) * k);
-    const float s16 = row_sum<4>(st.s * f);
+    const float s16 = lanes_sum<4>(st.s * f);
     t.s = (lane_value(s16, 0) + lane_value(s16, 16)) + (lane_value(s16, 32) + lane_value(s16, 48));
     t.u = 0.f;
     if (kEntropy) {
-        const float u16 = row_sum<4>(st.u * f);
+        const float u16 = lanes_sum<4>(st.u * f);
         t.u = (lane_value(u16, 0) + lane_value(u16, 16)) + (lane_value(u16, 32) + lane_value(u16, 48));
     }
     const int wave = tid >> 6, lane = tid & 63;
@@ -101,13 +74,13 @@ __device__ __forceinline__ Stats reduce_row(Stats st, float k, Stats* lds, int t
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     const Stats x = lds[lane & (kWaves - 1)];
-    const float m = row_max<kSteps>(x.m);
+    const float m = lanes_max<kSteps>(x.m);
     const float fx = fast_exp2((x.m - m) * k);
     // the same in every lane, which the branches and addresses that follow from it have to be known to be
     Stats r;
     r.m = lane_value(m, 0);
-    r.s = lane_value(row_sum<kSteps>(x.s * fx), 0);
-    r.u = kEntropy ? lane_value(row_sum<kSteps>(x.u * fx), 0) : 0.f;
+    r.s = lane_value(lanes_sum<kSteps>(x.s * fx), 0);
+    r.u = kEntropy ? lane_value(lanes_sum<kSteps>(x.u * fx), 0) : 0.f;
     return r;
 }
 
